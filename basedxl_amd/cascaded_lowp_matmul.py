@@ -189,7 +189,7 @@ class PreparedWeight:
     kept as MFMA operand slots; ``cascaded_lowp_matmul(a, prepared)`` then splits only ``a``.
     The arithmetic is the same as with the raw weight (same split, same products).  Kernels for
     prepared weights exist for bf16 x 2, bf16 x 3, fp16 x 3 and fp8 x 3 with the 'tri' product set and
-    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4; the
+    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4 (16-bit: K of 8); the
     product with any other combination fails with CascmmError (use the raw weight there).
 
     ``glu=True``: ``w`` is the ``[in, 2 * inner]`` weight of a gated projection (diffusers' GEGLU:
@@ -245,16 +245,14 @@ class PreparedWeight:
         return self
 
     def usable_with(self, a2: torch.Tensor, products: str = "tri") -> bool:
-        """Whether the prepared kernels take this left operand: fp32 (or fp16 / bf16 tensors with a
-        weight of the same dtype kept as one term of that format), K a multiple of 64, rows 16-byte
-        aligned (anything else goes through the raw weight)."""
-        if self.K % 64 != 0 or self.N % 4 != 0 or a2.data_ptr() % 16 != 0:
-            return False
-        if not self.has_kernel(a2.dtype, products):
+        """Whether the prepared kernels take this left operand, rows 16-byte aligned: fp32 with K a multiple
+        of 64 and N of 4, or fp16 / bf16 tensors with a weight of the same dtype kept as one term of that format
+        and K a multiple of 8 (anything else goes through the raw weight)."""
+        if a2.data_ptr() % 16 != 0 or not self.has_kernel(a2.dtype, products):
             return False
         if a2.dtype == torch.float32:
-            return a2.shape[0] <= 1 or a2.stride(0) % 4 == 0
-        return (a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp
+            return self.K % 64 == 0 and self.N % 4 == 0 and (a2.shape[0] <= 1 or a2.stride(0) % 4 == 0)
+        return (self.K % 8 == 0 and a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp
                 and (a2.shape[0] <= 1 or a2.stride(0) % 8 == 0))
 
     def has_kernel(self, dtype: torch.dtype, products: str = "tri") -> bool:
@@ -470,7 +468,8 @@ def cascaded_lowp_matmul_grouped(a_list, b_list, *, outs=None, biases=None, lowp
                     exps[2 * i + 1:2 * i + 2].copy_(kept.reshape(1))
             if kept is None:
                 _activation_exps(b_list[i], max(N, 1), None, exps.data_ptr() + 8 * i + 4, stream)
-    # 16-bit tensors as one term of their own format: room for every right operand re-laid as operand slots
+    # 16-bit tensors as one term of their own format: room for every right operand re-laid as operand slots (rows that are
+    # not whole 16-byte chunks)
     ws = None
     if a_list[0].dtype != torch.float32:
         need = _workspace_bytes(M, N, K, _DTYPES[a_list[0].dtype], fmt, terms, prod)

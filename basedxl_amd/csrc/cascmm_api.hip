@@ -30,6 +30,8 @@ static const std::vector<VariantDesc>& table() {
     v.insert(v.end(), p, p + n);
     p = variants_chain(&n);
     v.insert(v.end(), p, p + n);
+    p = variants_h16(&n);
+    v.insert(v.end(), p, p + n);
     return v;
   }();
   return t;
@@ -58,12 +60,12 @@ static bool prepared_as_k16_slots(int64_t K, int fmt, int terms, bool glu) {
   return fmt == CASCMM_FMT_FP8 && terms == 3 && K > 0 && K % F8K64::BK == 0 && !glu;
 }
 
-// bytes of a prepared weight: planes x ceil(K/8) x N operand slots of 16 bytes
+// bytes of a prepared weight: planes x prepared_kgroups(K) x N operand slots of 16 bytes
 static int64_t prepared_bytes(int64_t K, int64_t N, int fmt, int terms, bool glu = false) {
   if (prepared_as_k16_slots(K, fmt, terms, glu)) return f8k64_slot_bytes(N, K);
   const int planes = fmt == CASCMM_FMT_FP8 ? (terms + 1) / 2 : terms;
   int64_t slots = 0, bytes = 0;   // (saturates instead of overflowing: callers compare the result with limits)
-  if (__builtin_mul_overflow((int64_t)planes * ((K + 7) / 8), N, &slots) || __builtin_mul_overflow(slots, (int64_t)16, &bytes))
+  if (__builtin_mul_overflow((int64_t)planes * prepared_kgroups(K), N, &slots) || __builtin_mul_overflow(slots, (int64_t)16, &bytes))
     return INT64_MAX;
   return bytes;
 }
@@ -79,13 +81,17 @@ static int check_problem(const Problem& q) {
   return CASCMM_OK;
 }
 
+// 16-bit tensors multiplied as one term of their own format: exact operands, nothing to split
+static bool own_format16(const Problem& q) {
+  return q.terms == 1 && ((q.dtype == CASCMM_DT_F16 && q.fmt == CASCMM_FMT_FP16) || (q.dtype == CASCMM_DT_BF16 && q.fmt == CASCMM_FMT_BF16));
+}
+
 // what the fast (buffer-load, 16-byte accesses, no K tail) kernels need apart from K % BK == 0
 static bool fast_ok(const Problem& q, const void* A, const void* B) {
   if (q.dtype != CASCMM_DT_F32) {
-    // 16-bit operands: only with a prepared right operand, as one term of their own format
-    return q.bpre && q.terms == 1 &&
-           ((q.dtype == CASCMM_DT_F16 && q.fmt == CASCMM_FMT_FP16) || (q.dtype == CASCMM_DT_BF16 && q.fmt == CASCMM_FMT_BF16)) &&
-           q.lda % 8 == 0 && (A == nullptr || aligned_to(A, 16)) && q.lda * 2 * 512 < INT32_MAX;
+    // 16-bit operands: only as one term of their own format; a raw right operand with whole 16-byte chunks too
+    return own_format16(q) && q.lda % 8 == 0 && (A == nullptr || aligned_to(A, 16)) && q.lda * 2 * 512 < INT32_MAX &&
+           (q.bpre || (q.ldb % 8 == 0 && q.N % 8 == 0 && (B == nullptr || aligned_to(B, 16))));
   }
   return q.dtype == CASCMM_DT_F32 && q.lda % 4 == 0 && (A == nullptr || aligned_to(A, 16)) &&
          q.ldb % 4 == 0 && q.N % 4 == 0 && (B == nullptr || aligned_to(B, 16)) &&
@@ -96,7 +102,7 @@ static bool fast_ok(const Problem& q, const void* A, const void* B) {
 static bool variant_matches(const VariantDesc& v, const Problem& q, bool fast) {
   const int full = (q.products == CASCMM_PROD_FULL && q.terms > 1) ? 1 : 0;
   if (v.iodt != q.dtype || v.fmt != q.fmt || v.terms != q.terms || v.full != full || v.bpre != q.bpre) return false;
-  if (v.fast && (!fast || q.K % v.BK != 0)) return false;
+  if (v.fast && (!fast || (v.kind != KIND_H16 && q.K % v.BK != 0))) return false;
   if (v.kind == KIND_SPLITK && (q.M > 5 * v.BM || q.K < 4 * v.BK)) return false;  // skinny: few row tiles, deep K
   if (v.kind == KIND_F8K64 && (q.products != CASCMM_PROD_TRI || q.K % v.BK != 0 || q.K == 0 || q.glu ||
                                f8k64_slot_bytes(q.M, q.K) > INT32_MAX || f8k64_slot_bytes(q.N, q.K) > INT32_MAX))
@@ -111,6 +117,9 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, bool fast) {
     return false;
   if (v.kind == KIND_WAVEK && (q.N % v.BN != 0 || q.M * q.lda * 4 > INT32_MAX || q.K == 0)) return false;
   if (v.kind == KIND_SLOTK && (q.K % 32 != 0 || q.K < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
+    return false;
+  // (32-bit byte offsets down A and, where it is raw, B, two stages past the end included; K in whole 16-byte chunks)
+  if (v.kind == KIND_H16 && (q.K % 8 != 0 || q.K == 0 || q.M * q.lda * 2 > INT32_MAX || (!q.bpre && (q.K + 64) * q.ldb * 2 > INT32_MAX)))
     return false;
   if (q.glu && !v.glu) return false;
   if (q.glu_slots && v.kind != KIND_W512) return false;
@@ -213,6 +222,27 @@ static double skinny_estimate_us(const Problem& q) {
   return 8.5 + 160.0 * (double)(q.K / sp) * 4.0 / 70.0e3 + 2.0 * sp * (double)q.M * (double)q.N * 4.0 / 4.0e6;
 }
 
+// The 16-bit kernels (KIND_H16).  A workgroup's k costs s1 with every CU at work (L2 or the board's power is shared)
+// and s0 with few; a round of 256 tiles adds `end` for its store, a launch `start`.  raw: the factor on k of a right
+// operand that the LDS transposes.  Measured on the Linear shapes of a UNet and on squares (graph replay, every tile
+// forced in turn).
+struct H16Cost { int BM, BN; double s0, s1, start, end, raw; };
+static const H16Cost kH16Cost[] = {
+    {256, 320, 0.0205, 0.0315, 3.8, 8.0, 1.06}, {256, 256, 0.0175, 0.0255, 4.0, 6.5, 1.03}, {128, 256, 0.0090, 0.0138, 3.5, 3.5, 1.04},
+    {128, 160, 0.0058, 0.0092, 3.5, 2.4, 1.17}, {128, 128, 0.0056, 0.0077, 3.3, 1.8, 1.16}, {64, 160, 0.0047, 0.0053, 3.7, 2.7, 1.10},
+    {64, 128, 0.0042, 0.0046, 3.3, 1.1, 1.06},  {128, 64, 0.0044, 0.0050, 3.5, 1.1, 1.02},  {64, 64, 0.0026, 0.0033, 3.2, 1.0, 1.20},
+};
+static double h16_estimate_us(const VariantDesc& v, const Problem& q, double tiles) {
+  for (const H16Cost& c : kH16Cost)
+    if (c.BM == v.BM && c.BN == v.BN) {
+      const double full = (double)(int64_t)(tiles / kNumCUs), rem = tiles / kNumCUs - full;
+      const double last = rem > 0 ? (c.s1 * rem > c.s0 ? c.s1 * rem : c.s0) : 0.0;
+      const double k = (double)((q.K + v.BK - 1) / v.BK * v.BK) * (q.bpre ? 1.0 : c.raw);
+      return c.start + (full + (rem > 0 ? 1.0 : 0.0)) * c.end + k * (full * c.s1 + last);
+    }
+  return 1e9;
+}
+
 // ws_bytes: workspace the caller brought; *splits_out: K split the cost was computed for (the
 // LDS-tiled two-term bf16 kernels may split K over up to kMaxTileSplits work items per tile when a
 // single problem has too few tiles to occupy the chip and the workspace holds the partials)
@@ -234,6 +264,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
   if (v.kind == KIND_WAVEK) return wavek_estimate_us(q, count, v.BN);
+  if (v.kind == KIND_H16) return h16_estimate_us(v, q, tiles);
   if (v.kind == KIND_F8K64) {
     // stages of 64 k at ~2.1 us per resident round, the K split the launcher will use, and the passes
     // around the GEMM: the split of A (and of B unless prepared), the reduction of a K split
@@ -486,7 +517,7 @@ __global__ __launch_bounds__(256) void prepare_weight_kernel(const void* B, int 
                                                             const int32_t* tensor_exp, u32x4* out, int flags) {
   typedef typename IoType<IODT>::T T;
   const int glu = flags & 1, chained = flags & 2;
-  const int kgs = (K + 7) / 8;
+  const int kgs = chained ? K / 8 : (int)prepared_kgroups(K);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)kgs * N) return;
   const int kg = (int)(i / N), n = (int)(i - (int64_t)kg * N);
@@ -515,7 +546,7 @@ __global__ __launch_bounds__(256) void prepare_weight_kernel(const void* B, int 
 template <int IODT, int FMT>
 static int launch_prepare(const void* B, int K, int N, int64_t ldb, int terms, const int32_t* e, u32x4* out, hipStream_t s,
                           int glu) {
-  const int64_t total = (int64_t)((K + 7) / 8) * N;
+  const int64_t total = ((glu & 2) ? (int64_t)(K / 8) : prepared_kgroups(K)) * N;
   const unsigned grid = (unsigned)((total + 255) / 256);
   hipError_t err = hipSuccess;
   switch (terms) {
@@ -539,14 +570,16 @@ static int launch_prepare_fmt(const void* B, int K, int N, int64_t ldb, int fmt,
 // 16-bit tensors multiplied as one term of their own format can use the prepared-operand kernels
 // when the caller brought room for the re-laid B
 // (a grouped launch needs `count` such buffers, one behind the other)
+// (where the kernels that read a raw right operand do not take it: rows that are not whole 16-byte chunks)
 static bool onthefly_prepare_ok(const Problem& q, int count, const void* const* A, const void* const* B,
                                 const void* workspace, size_t workspace_bytes) {
-  if (q.bpre || q.dtype == CASCMM_DT_F32 || q.terms != 1 || q.K % 64 != 0) return false;
-  if (!((q.dtype == CASCMM_DT_F16 && q.fmt == CASCMM_FMT_FP16) || (q.dtype == CASCMM_DT_BF16 && q.fmt == CASCMM_FMT_BF16)))
-    return false;
-  if (q.lda % 8 != 0) return false;
-  for (int i = 0; i < count; ++i)
+  if (q.bpre || !own_format16(q) || q.K % 8 != 0 || q.lda % 8 != 0) return false;
+  bool raw = true;   // every right operand can be read where it lies
+  for (int i = 0; i < count; ++i) {
     if (!A[i] || !B[i] || !aligned_to(A[i], 16) || !aligned_to(B[i], 2)) return false;
+    raw = raw && fast_ok(q, A[i], B[i]);
+  }
+  if (raw && select_variant(q, true, count, 0) >= 0) return false;
   const int64_t need = prepared_bytes(q.K, q.N, q.fmt, 1);
   return workspace && aligned_to(workspace, 16) && need <= INT32_MAX && workspace_bytes >= (size_t)need * count;
 }
@@ -901,8 +934,7 @@ size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fm
     need = n > need ? n : need;
   }
   // 16-bit tensors as one term of their own format: room for B re-laid as operand slots
-  if (((dtype == CASCMM_DT_F16 && fmt == CASCMM_FMT_FP16) || (dtype == CASCMM_DT_BF16 && fmt == CASCMM_FMT_BF16)) &&
-      terms == 1 && K % 64 == 0) {
+  if (own_format16(q) && K % 8 == 0) {
     const int64_t n = prepared_bytes(K, N, fmt, 1);
     if (n <= INT32_MAX && (size_t)n > need) need = (size_t)n;
   }

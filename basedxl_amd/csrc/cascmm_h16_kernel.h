@@ -1,0 +1,376 @@
+// Plain 16-bit GEMM (fp16 or bf16 tensors as ONE term of their own format, fp32 accumulation; gfx950).
+//
+// Eight consecutive elements of a row of A already are one lane's MFMA operand, and so is one 16-byte operand
+// slot of a prepared B (cascmm_prepare_weight); a raw B [K][N] is transposed by the LDS itself on the way to the
+// registers (ds_read_b64_tr_b16: sixteen lanes read 4 rows x 16 columns and every lane gets one column's four k).
+// So nothing passes the VALU: every operand byte goes memory -> LDS by `buffer_load ... lds` and LDS -> MFMA.
+//
+// Workgroup: four waves, one per SIMD, WM x WN over the tile (WK = 2: two wave groups take alternate 16-k slices
+// of every stage and meet in LDS at the end).  NS stages of BK k in LDS, one barrier per stage.  It sits in front of
+// a stage's last slice, whose fragments are in registers by then: behind it stage s + 1 has landed, so the last
+// slice's MFMAs hide the first fragment reads of the next stage, and the buffer of stage s is free, so the loads of
+// stage s + NS start at once: NS - 1 stages are in flight (with the barrier at the top of a stage it was one less).
+//
+// What bounds it: one product per element leaves three times fewer MFMA cycles per byte than the two-term
+// cascade, so a tile is as good as its bytes per multiply-add: (BM + BN) x 2 bytes per k through the CU's share
+// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared, graph replay; in brackets the
+// copy-only LDS kernels with producer waves that these replaced): 2048 x 1280 x 10240 on 256 x 320 52.1 us (62.1), its
+// loop at 1320 TFLOP/s, which is the board's power with random operands (zeros: a third faster); 4096^3 on
+// 256 x 256 115 us (135); 8192 x 2560 x 640 on 128 x 160 29.4 us (33.5); 2048^3 on 128 x 128 20.8 us (23.0), its loop
+// at 66 bytes per ns and CU from the L2s; 2048 x 1280 x 1280 12.2 us (14.0); 512 x 1280 x 1280 on 64 x 64 7.6 us (9.5).
+// With B raw (no re-lay pass: 2048^3 28.7 -> 23.5 us) the transposing reads cost 3 - 16 %.
+//
+// The MFMAs take their operands swapped (B first): a lane then holds ONE ROW of C and four consecutive columns
+// per register quad, which are packed to 8 bytes, turned row-wise through LDS and stored 16 bytes per lane.
+#pragma once
+#include <type_traits>
+
+#include "cascmm_tile_kernel.h"
+
+namespace cascmm {
+
+template <int WM_, int WN_, int WK_, int MT_, int NTL_, int BK_, int NS_>
+struct H16 {
+  static constexpr int WM = WM_, WN = WN_, WK = WK_, MT = MT_, NTL = NTL_, BK = BK_, NS = NS_, NT = 256;
+  static constexpr int WTM = 32 * MT, WTN = 32 * NTL, BM = WM * WTM, BN = WN * WTN;
+  static constexpr int KG = BK / 8;                  // 16-byte chunks of a row of A (slot rows of B) per stage
+  static constexpr int SLW = BK / 16 / WK;           // 16-k slices of a stage that a wave multiplies
+  static constexpr int A_STAGE = BM * BK * 2, B_STAGE = BN * BK * 2, STAGE = A_STAGE + B_STAGE;
+  static constexpr int A_LOADS = A_STAGE / 4096, B_LOADS = B_STAGE / 4096, LOADS = A_LOADS + B_LOADS;   // per wave and stage
+  static constexpr int OUT_ROW = WTN * 2 + 16;       // bytes of a row of C in the store's LDS area (padded: banks)
+  static constexpr int SUM_WAVE = WK == 2 ? (NTL + 1) / 2 * 4096 : 0;   // the other wave group's sums of this wave's blocks
+  static constexpr int OUT_WAVE = 32 * OUT_ROW + WTN * 4 > SUM_WAVE ? 32 * OUT_ROW + WTN * 4 : SUM_WAVE;
+  static constexpr int LDS_BYTES = NS * STAGE > 4 * OUT_WAVE ? NS * STAGE : 4 * OUT_WAVE;
+  // tile rows an XCD walks down before moving one tile to the right: about square in bytes
+  static constexpr int GROUP_M = BN >= 2 * BM ? 8 : 4;
+  static_assert(WM * WN * WK == 4 && (BK == 32 || BK == 64) && SLW % 2 == 0 && NS >= 3, "layout");
+  static_assert(A_STAGE % 4096 == 0 && B_STAGE % 4096 == 0, "every wave issues the same number of loads");
+  static_assert((NS - 1) * LOADS <= 63, "the wait counter has six bits");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+};
+
+typedef __attribute__((address_space(3))) void* h16_lds_ptr;
+
+// (functions of their own: in a call whose arguments depend on a template parameter the host pass of the compiler
+// rejects the builtin without a message and then leaves out the kernel's launch stub)
+__device__ __forceinline__ void h16_load_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char* dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (h16_lds_ptr)dst, 16, voffset, soffset, 0, 0);
+}
+// Transposing read, as assembly: in front of the builtin the compiler waits for every `buffer_load ... lds` in
+// flight (it cannot see that they write other buffers), which serialised loads and MFMAs.  The caller waits for the
+// result itself.
+template <int OFF> __device__ __forceinline__ u32x2 h16_read_tr(unsigned lds_addr) {
+  u32x2 v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "n"(OFF));
+  return v;
+}
+
+// MFMA with the accumulator in ordinary vector registers: there are sixteen blocks' worth of accumulation registers,
+// which is where the compiler puts every accumulator of an MFMA that it selects itself
+template <int FMT> __device__ __forceinline__ void h16_mfma_v(u32x4 a, u32x4 b, f32x16& c) {
+  if constexpr (FMT == CASCMM_FMT_BF16) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+
+template <int FMT> struct H16Elem;
+template <> struct H16Elem<CASCMM_FMT_BF16> { typedef __bf16 T; static constexpr int DT = CASCMM_DT_BF16; };
+template <> struct H16Elem<CASCMM_FMT_FP16> { typedef _Float16 T; static constexpr int DT = CASCMM_DT_F16; };
+
+// Host-checked: K % 8 == 0, lda % 8 == 0, A 16-byte aligned, M * lda * 2 below 2 GiB; RAWB = 0: B prepared
+// ([ceil(K / 64) * 8][N] slots, zeros beyond K) below 2 GiB; RAWB = 1: B [K][ldb] with N % 8 == 0, ldb % 8 == 0,
+// 16-byte aligned, K * ldb * 2 below 2 GiB.  Any M and N: rows and columns past the edge are loaded as zeros or as
+// some other column's values and not stored.  grid.y: the problem of a group.
+// GLU: gated store (see GroupParams; RAWB = 0, NTL even: a wave owns whole value / gate pairs of blocks).
+template <class T, int FMT, int RAWB, int GLU>
+__global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams p) {
+  typedef typename H16Elem<FMT>::T E;
+  typedef IoType<H16Elem<FMT>::DT> Io;
+  static_assert(!GLU || (!RAWB && T::NTL % 2 == 0), "the gated store pairs a wave's blocks");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char h16_smem[];
+  unsigned char* smem = h16_smem;
+  const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave / (T::WM * T::WN), wmn = wave % (T::WM * T::WN);
+  const int wm0 = (wmn / T::WN) * T::WTM, wn0 = (wmn % T::WN) * T::WTN;
+  const int prob = blockIdx.y;
+  int tm, tn;
+  tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, T::GROUP_M);
+  const int m0 = tm * T::BM, n0 = tn * T::BN;
+  const int ksteps = (p.K + T::BK - 1) / T::BK;
+
+  // rows past M read as zero (the buffer ends with row M - 1), and so does everything past B's last row or slot row
+  const int kgs = (p.K + 63) / 64 * 8;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + p.K) * 2;
+  const int64_t b_bytes = RAWB ? ((int64_t)(p.K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[prob], 0, (int)b_bytes, 0x00020000);
+
+  // ---- loads: this wave's kilobytes of a stage ----
+  // A: row r of the stage's BM x BK block at r * 2 BK bytes; position pos of a row holds chunk (pos - rot(r)) mod KG,
+  // rot = r / 2 (BK = 64) or r / 4 (BK = 32): the sixteen lanes a 16-byte LDS read serves together hit every bank once
+  constexpr int RSH = T::KG == 8 ? 1 : 2;
+  int a_voff[T::A_LOADS], a_k[T::A_LOADS];
+#pragma unroll
+  for (int j = 0; j < T::A_LOADS; ++j) {
+    const int row = (wave * T::A_LOADS + j) * (64 / T::KG) + lane / T::KG;
+    const int chunk = (lane % T::KG - (row >> RSH)) & (T::KG - 1);
+    a_k[j] = chunk * 8;
+    a_voff[j] = m0 + row < p.M ? (int)(((int64_t)(m0 + row) * p.lda + chunk * 8) * 2) : 0x7FFFFFFF;
+  }
+  // B prepared: slot (k group, column) at (kg * BN + column) * 16.  B raw: row k at 2 BN k bytes, its 16-byte chunks
+  // (8 columns) permuted by an XOR so that the four rows of a transposing read lie on different banks
+  constexpr int CPR = T::BN / 8;   // chunks per row of raw B
+  constexpr int XSH = (T::BN * 2) % 256 == 0 ? 0 : (T::BN * 2) % 256 == 128 ? 1 : 2;
+  auto xor_of = [](int row) { return XSH == 0 ? 4 * (row & 3) : XSH == 1 ? 4 * ((row >> 1) & 1) : 0; };
+  int b_voff[T::B_LOADS];
+#pragma unroll
+  for (int j = 0; j < T::B_LOADS; ++j) {
+    const int s = (wave * T::B_LOADS + j) * 64 + lane;
+    if (RAWB) b_voff[j] = (int)(((int64_t)(s / CPR) * p.ldb + n0 + ((s % CPR) ^ xor_of(s / CPR)) * 8) * 2);
+    else b_voff[j] = ((s / T::BN) * p.N + n0 + s % T::BN) * 16;
+  }
+  const int b_step = RAWB ? (int)(T::BK * p.ldb * 2) : T::KG * p.N * 16;
+  auto issue = [&](int step, int buf, int j) {
+    unsigned char* st = smem + buf * T::STAGE;
+    if (j < T::A_LOADS) {
+      // (past K: beyond the buffer's end, zeros)
+      const int v = a_k[j] < p.K - step * T::BK ? a_voff[j] : 0x7FFFFFFF;
+      h16_load_lds(ra, st + (wave * T::A_LOADS + j) * 1024, v, step * T::BK * 2);
+    } else {
+      const int bs = (step < ksteps ? step : ksteps) * b_step;
+      h16_load_lds(rb, st + T::A_STAGE + (wave * T::B_LOADS + j - T::A_LOADS) * 1024, b_voff[j - T::A_LOADS], bs);
+    }
+  };
+
+  // ---- fragments: slice sl of a stage ----
+  const int a_row = wm0 + l31;
+  int a_frag[T::SLW];
+#pragma unroll
+  for (int x = 0; x < T::SLW; ++x) {
+    const int sl = T::WK == 1 ? x : 2 * x + wk;
+    a_frag[x] = a_row * T::BK * 2 + ((2 * sl + g + (a_row >> RSH)) & (T::KG - 1)) * 16;
+  }
+  // raw B: lane i = lane % 16 of a group of sixteen reads row 8 g + i / 4 (+ 4), columns 16 (lane / 16 % 2) + 4 (i % 4)
+  int b_frag[RAWB ? T::NTL : 1];
+  const int b_slice = RAWB ? 16 * T::BN * 2 : 2 * T::BN * 16;
+  if (RAWB) {
+    const int i = lane & 15, row = 8 * g + (i >> 2);
+#pragma unroll
+    for (int ni = 0; ni < T::NTL; ++ni) {
+      const int chunk = (wn0 + ni * 32) / 8 + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+      b_frag[ni] = T::A_STAGE + wk * b_slice + row * T::BN * 2 + (chunk ^ xor_of(row)) * 16 + (i & 1) * 8;
+    }
+  } else {
+    b_frag[0] = T::A_STAGE + wk * b_slice + (g * T::BN + wn0 + l31) * 16;
+  }
+  u32x4 Af[2][T::MT], Bf[2][T::NTL];
+  auto read = [&](const unsigned char* st, int x, int buf, int r) {   // r: A's blocks, then B's
+    if (r < T::MT) Af[buf][r] = *(const u32x4*)(st + a_frag[x] + r * 32 * T::BK * 2);
+    else if (RAWB) {
+      const unsigned src = (unsigned)(uintptr_t)(h16_lds_ptr)(st + b_frag[r - T::MT] + x * T::WK * b_slice);
+      const u32x2 lo = h16_read_tr<0>(src), hi = h16_read_tr<8 * T::BN>(src);   // (four rows further down)
+      Bf[buf][r - T::MT] = (u32x4){lo[0], lo[1], hi[0], hi[1]};
+    } else {
+      Bf[buf][r - T::MT] = *(const u32x4*)(st + b_frag[0] + x * T::WK * b_slice + (r - T::MT) * 512);
+    }
+  };
+
+#define H16_FENCE() __builtin_amdgcn_sched_barrier(0)
+  f32x16 acc[T::MT][T::NTL];
+  // Loads of a stage: the first P with the last slice of stage s - NS, the others with the first slices of s - NS + 1.
+  constexpr int P = (T::LOADS + T::SLW - 1) / T::SLW;
+#pragma unroll
+  for (int s = 0; s < T::NS; ++s)
+#pragma unroll
+    for (int j = 0; j < (s < T::NS - 1 ? T::LOADS : P); ++j) issue(s, s, j);
+  H16_FENCE();
+  // (cleared while the first loads are in flight; the empty statements make the zeros real here)
+#pragma unroll
+  for (int mi = 0; mi < T::MT; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < T::NTL; ++ni) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[mi][ni][e] = 0.f;
+      if (mi * T::NTL + ni < 16) asm volatile("" : "+a"(acc[mi][ni]));
+      else asm volatile("" : "+v"(acc[mi][ni]));
+    }
+  H16_FENCE();
+  constexpr int W0 = (T::NS - 2) * T::LOADS + P, W1 = (T::NS - 2) * T::LOADS;
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (W0 & 0xF) | ((W0 >> 4) << 14));   // stage 0 has landed
+  __builtin_amdgcn_s_barrier();
+  H16_FENCE();
+#pragma unroll
+  for (int r = 0; r < T::MT + T::NTL; ++r) read(smem, 0, 0, r);
+  if (RAWB) __builtin_amdgcn_s_waitcnt(0xC07F);
+
+  int cur = 0, before = T::NS - 1;   // LDS buffers of this stage and of the one before it
+  for (int s = 0; s < ksteps; ++s) {
+    const int nx = cur == T::NS - 1 ? 0 : cur + 1;
+    const unsigned char* st0 = smem + cur * T::STAGE;
+    const unsigned char* st1 = smem + nx * T::STAGE;
+#pragma unroll
+    for (int x = 0; x < T::SLW; ++x) {
+      const int buf = x & 1;
+      const bool last = x == T::SLW - 1;
+      if (last) {
+        // own loads of stage s + 1 have landed and own reads of stage s are over, then everybody's
+        __builtin_amdgcn_s_waitcnt(0x0070 | (W1 & 0xF) | ((W1 >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        H16_FENCE();
+      }
+      // behind the MFMAs of a slice: first the fragment reads of the next one, then this slice's share of the loads
+      constexpr int READS = T::MT + T::NTL, MF = T::MT * T::NTL;
+      const int l0 = last ? 0 : P + x * (T::LOADS - P) / (T::SLW - 1), l1 = last ? P : P + (x + 1) * (T::LOADS - P) / (T::SLW - 1);
+      constexpr int RG = MF >= READS ? READS : (MF + 1) / 2;   // gaps that take the reads
+#pragma unroll
+      for (int mf = 0; mf < MF; ++mf) {
+        const int ni = mf / T::MT, mi = mf % T::MT;
+        if (mi * T::NTL + ni < 16)
+          acc[mi][ni] = Lowp<FMT>::mfma(Lowp<FMT>::operand(Bf[buf][ni], 0), Lowp<FMT>::operand(Af[buf][mi], 0), acc[mi][ni]);
+        else
+          h16_mfma_v<FMT>(Bf[buf][ni], Af[buf][mi], acc[mi][ni]);
+        H16_FENCE();
+#pragma unroll
+        for (int r = 0; r < READS; ++r) {
+          if (r * RG / READS != mf) continue;
+          if (last) read(st1, 0, buf ^ 1, r);
+          else read(st0, x + 1, buf ^ 1, r);
+        }
+#pragma unroll
+        for (int j = 0; j < T::LOADS; ++j) {
+          if (j < l0 || j >= l1 || (j - l0) * MF / (l1 - l0) != mf) continue;
+          if (last) issue(s + T::NS, cur, j);
+          else issue(s + T::NS - 1, before, j);
+        }
+        H16_FENCE();
+      }
+      if (RAWB) {   // (results of reads written as assembly: the compiler does not wait for them)
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        H16_FENCE();
+      }
+    }
+    before = cur;
+    cur = nx;
+  }
+#undef H16_FENCE
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // the loads past the last stage have landed before LDS is used again
+  // (the MFMAs written as assembly are invisible to the compiler's hazard handling)
+  asm volatile("s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
+  __syncthreads();
+
+  // ---- two wave groups: each finishes its share of the blocks, the other one's sums come through LDS ----
+  constexpr int OB = GLU ? T::NTL / 2 : T::NTL;              // 32-column blocks of C per row block
+  constexpr int HALF = T::WK == 2 ? (OB + 1) / 2 : OB;       // wave group 0: blocks 0 .. HALF - 1, group 1: the others
+  unsigned char* area = smem + wave * T::OUT_WAVE;
+  // (The store is straight-line code that every wave runs once, so its length is time: instructions come from L2 at
+  // some 10 KB per us.  With or without a bias, 16-byte or single stores are therefore separate copies.)
+  auto finish = [&](auto first_tag, auto count_tag, auto bias_tag) {
+    constexpr int B0 = decltype(first_tag)::value, NB = decltype(count_tag)::value;
+    constexpr bool BIAS = decltype(bias_tag)::value != 0;
+    // ---- store: of block (mi, ni) a lane holds row 32 mi + l31, columns 32 ni + 8 q + 4 g + e in register 4 q + e ----
+    const int no = GLU ? p.N >> 1 : p.N;
+    const int oc0 = (GLU ? (n0 + wn0) >> 1 : n0 + wn0) + 32 * B0;
+    float* bl = (float*)(area + 32 * T::OUT_ROW);   // the wave's bias values, in the order of its columns
+    if constexpr (BIAS) {
+      const E* bias = (const E*)p.bias[prob];
+      for (int c = lane; c < NB * (GLU ? 64 : 32); c += 64) {
+        // (gated: blocks alternate value and gate columns)
+        const int col = GLU ? oc0 + (c >> 6) * 32 + (c & 31) : oc0 + c;
+        bl[c] = col < no ? Io::load(bias + (GLU && (c & 32) ? no : 0) + col) : 0.f;
+      }
+    }
+    E* C = (E*)p.C[prob] + (int64_t)(m0 + wm0) * p.ldc + oc0;
+    const bool vec = (p.ldc & 7) == 0 && (no & 7) == 0 && ((uintptr_t)p.C[prob] & 15) == 0;
+    // rows past M fall beyond the end of the buffer and are dropped, columns past the last one are sent there too
+    const int64_t c_bytes = ((int64_t)(p.M - 1 - m0 - wm0) * p.ldc + (no - oc0)) * 2;
+    const i32x4 rc = make_rsrc(C, c_bytes < 0 ? 0 : c_bytes);
+    const int ldc_bytes = (int)p.ldc * 2;
+    constexpr int CHUNKS = 4 * NB, ITS = 2 * NB;   // 16-byte chunks of a row; of 32 rows, per lane
+#pragma unroll
+    for (int mi = 0; mi < T::MT; ++mi) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int at = 8 * q + 4 * g;
+          typedef E e2 __attribute__((ext_vector_type(2)));
+          f32x4 y;
+          if constexpr (GLU) {
+            f32x4 bv = {0.f, 0.f, 0.f, 0.f}, bg = bv;
+            if constexpr (BIAS) {
+              bv = *(const f32x4*)(bl + 64 * b + at);
+              bg = *(const f32x4*)(bl + 64 * b + 32 + at);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = gated_value(acc[mi][2 * b][4 * q + e] + bv[e], acc[mi][2 * b + 1][4 * q + e] + bg[e]);
+          } else {
+            f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (BIAS) bv = *(const f32x4*)(bl + 32 * b + at);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = BIAS ? acc[mi][B0 + b][4 * q + e] + bv[e] : acc[mi][B0 + b][4 * q + e];
+          }
+          const u32x2 out = {__builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){y[0], y[1]}, e2)),
+                             __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){y[2], y[3]}, e2))};
+          *(u32x2*)(area + l31 * T::OUT_ROW + (32 * b + at) * 2) = out;
+        }
+      if (vec) {
+        // (a few at a time: the reads' latency overlaps, the registers last)
+        constexpr int GRP = ITS <= 8 ? ITS : ITS == 10 ? 5 : 4;
+        static_assert(ITS % GRP == 0, "groups");
+#pragma unroll
+        for (int i0 = 0; i0 < ITS; i0 += GRP) {
+          u32x4 v[GRP];
+#pragma unroll
+          for (int it = 0; it < GRP; ++it) {
+            const int i = (i0 + it) * 64 + lane;
+            v[it] = *(const u32x4*)(area + (i / CHUNKS) * T::OUT_ROW + (i % CHUNKS) * 16);
+          }
+#pragma unroll
+          for (int it = 0; it < GRP; ++it) {
+            const int i = (i0 + it) * 64 + lane, c = i % CHUNKS;
+            llvm_raw_buffer_store_v4f32(__builtin_bit_cast(f32x4, v[it]), rc, oc0 + c * 8 < no ? (mi * 32 + i / CHUNKS) * ldc_bytes + c * 16 : 0x7FFFFFFF, 0, 0);
+          }
+        }
+      } else {
+#pragma unroll 1
+        for (int i = lane; i < 32 * NB * 32; i += 64) {
+          const int row = i / (32 * NB), c = i % (32 * NB);
+          const E h = *(const E*)(area + row * T::OUT_ROW + c * 2);
+          if (m0 + wm0 + mi * 32 + row < p.M && oc0 + c < no) C[(int64_t)(mi * 32 + row) * p.ldc + c] = h;
+        }
+      }
+    }
+  };
+  auto with_bias = [&](auto first, auto count) {
+    if (p.bias[prob]) finish(first, count, std::integral_constant<int, 1>{});
+    else finish(first, count, std::integral_constant<int, 0>{});
+  };
+  if constexpr (T::WK == 2) {
+    static_assert(T::MT == 1 && !GLU, "one row block per wave");
+    unsigned char* other = smem + (wave ^ (T::WM * T::WN)) * T::OUT_WAVE;
+#pragma unroll
+    for (int b = 0; b < T::NTL; ++b)
+      if ((b < HALF) == (wk == 1))   // the other group's block
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x16& v = acc[0][b];
+          *(f32x4*)(other + ((b % HALF) * 4 + q) * 1024 + lane * 16) = (f32x4){v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < T::NTL; ++b)
+      if ((b < HALF) == (wk == 0))
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 o = *(const f32x4*)(area + ((b % HALF) * 4 + q) * 1024 + lane * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[0][b][4 * q + e] += o[e];
+        }
+    if (wk == 0) with_bias(std::integral_constant<int, 0>{}, std::integral_constant<int, HALF>{});
+    else with_bias(std::integral_constant<int, HALF>{}, std::integral_constant<int, OB - HALF>{});
+  } else {
+    with_bias(std::integral_constant<int, 0>{}, std::integral_constant<int, OB>{});
+  }
+}
+
+}  // namespace cascmm

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   int tm, tn;
   tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int kgroups = p.K >> 3;
+  const int kgroups = ARAW ? (int)prepared_kgroups(p.K) : p.K >> 3;   // (slots x slots: both buffers end with K)
   const int ksteps = p.K >> 4;
   // Which 16-k stages of the problem a wave owns.  A as slots: every fourth one, own stage i = stage
   // wave + 4 i.  A raw: every fourth PAIR of stages, own stage i = stage 8 (i / 2) + 2 wave + i % 2, so that

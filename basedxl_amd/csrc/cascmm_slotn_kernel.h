@@ -45,7 +45,7 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   int tm, tn;
   tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int kgroups = p.K >> 3;
+  const int kgroups = (int)prepared_kgroups(p.K);
   const int ksteps = p.K >> 5;
   const int n_own = (ksteps - wave + T::NW - 1) / T::NW;   // 0 for the last waves of a very short K: they add zeros
   // The loop runs in trips of two stages without a branch inside; a wave with an odd number of stages runs one

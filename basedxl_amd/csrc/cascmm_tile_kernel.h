@@ -170,9 +170,6 @@ struct TileGemm {
   static constexpr int B_UNITS = TL::KG * TL::BNS;         // 8(k) x 1(n) columns of B
   static constexpr int D = TL::DEPTH;
   static_assert(!BPRE || TL::BNQ == 0, "prepared B is staged column by column");
-  // 16-bit operands on the fast path: A is fp16 (bf16) data multiplied as one fp16 (bf16) term, so
-  // 8 consecutive elements of a row ARE the operand slot: the producers copy 16 bytes, no split
-  static constexpr bool RAW16 = IODT != CASCMM_DT_F32;
   static constexpr int BREGS = BPRE ? 4 * PL : 8;            // registers of one B unit in the ring
   // the gated epilogue needs prepared B (columns in any order at no cost) and a consumer wave that
   // owns whole value / gate pairs of 32-column blocks
@@ -298,7 +295,7 @@ struct TileGemm {
       if constexpr (BPRE) {
         // the descriptor covers the whole prepared buffer; the tile's column goes into the
         // per-lane offsets (the host checked that the buffer is smaller than 2 GiB)
-        const int kgs = (p.K + 7) / 8;
+        const int kgs = (int)prepared_kgroups(p.K);
         c.ldb_bytes = p.N * 16;
         c.plane_bytes = kgs * c.ldb_bytes;
         c.rb = make_rsrc(p.B[prob], (int64_t)PL * c.plane_bytes);
@@ -348,11 +345,9 @@ struct TileGemm {
         const f32x4 v0 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it], soff_a, 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) r.a[it][e] = v0[e];
-        if constexpr (!RAW16) {
-          const f32x4 v1 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it] + 16, soff_a, 0);
+        const f32x4 v1 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it] + 16, soff_a, 0);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) r.a[it][4 + e] = v1[e];
-        }
+        for (int e = 0; e < 4; ++e) r.a[it][4 + e] = v1[e];
       }
       if constexpr (BPRE) {
         load_prepared(c, k0, r);
@@ -436,32 +431,25 @@ struct TileGemm {
     // that unit's registers for K step k_next (ISSUE).  Spreading the loads between the VALU
     // batches keeps the texture-address unit busy while the splits run; issued in one burst
     // they would stall the wave on the full address FIFO with no VALU work to overlap.
-    template <bool ISSUE, bool RAW = false>
+    template <bool ISSUE>
     static __device__ __forceinline__ void restage(const Ctx& c, u32x4* stage, Regs& r, int k_next) {
       u32x4* sb = stage + PL * LL::kATerm;
       const int soff_a = k_next * ES;
 #pragma unroll
       for (int it = 0; it < A_IT; ++it) {
         if (A_ALL || c.lds_a[it] >= 0) {
-          if constexpr (RAW) {
-            const f32x4 v = {r.a[it][0], r.a[it][1], r.a[it][2], r.a[it][3]};
-            stage[c.lds_a[it]] = __builtin_bit_cast(u32x4, v);
-          } else {
-            u32x4 t[PL];
-            split8<FMT, TERMS>(r.a[it], t, c.scale_a);
+          u32x4 t[PL];
+          split8<FMT, TERMS>(r.a[it], t, c.scale_a);
 #pragma unroll
-            for (int i = 0; i < PL; ++i) stage[i * LL::kATerm + c.lds_a[it]] = t[i];
-          }
+          for (int i = 0; i < PL; ++i) stage[i * LL::kATerm + c.lds_a[it]] = t[i];
         }
         if (ISSUE && (!WEIGHTED || c.lds_a[it] >= 0)) {
           const f32x4 v0 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it], soff_a, 0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) r.a[it][e] = v0[e];
-          if constexpr (!RAW) {
-            const f32x4 v1 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it] + 16, soff_a, 0);
+          const f32x4 v1 = llvm_raw_buffer_load_v4f32(c.ra, c.voff_a[it] + 16, soff_a, 0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r.a[it][4 + e] = v1[e];
-          }
+          for (int e = 0; e < 4; ++e) r.a[it][4 + e] = v1[e];
         }
       }
 #pragma unroll
@@ -519,10 +507,6 @@ struct TileGemm {
     template <bool FAST>
     static __device__ __forceinline__ void loop(const GroupParams& p, u32x4* lds, int ktiles, int nitems) {
       static_assert(FAST || !BPRE, "prepared B has no bounds-checked loader");
-      constexpr bool RAW = FAST && RAW16;
-      static_assert(!RAW || (BPRE && TERMS == 1 &&
-                             ((IODT == CASCMM_DT_F16 && FMT == CASCMM_FMT_FP16) || (IODT == CASCMM_DT_BF16 && FMT == CASCMM_FMT_BF16))),
-                    "16-bit operands on the fast path: one term of their own format, prepared B");
       const int rtid = threadIdx.x - TL::NCW * kWave - T0;
       const int tiles = p.tiles_m * p.tiles_n;
       const int gsteps = nitems * ktiles;
@@ -580,9 +564,9 @@ struct TileGemm {
         for (int d = 0; d < D; ++d) {
           if (FAST) {
             const int k_next = target(g + d + D);
-            restage<true, RAW>(ctx, lds + ((g + d) & 1) * LL::kStage, ring[d], k_next);
+            restage<true>(ctx, lds + ((g + d) & 1) * LL::kStage, ring[d], k_next);
           } else {
-            restage<false, RAW>(ctx, lds + ((g + d) & 1) * LL::kStage, ring[d], 0);
+            restage<false>(ctx, lds + ((g + d) & 1) * LL::kStage, ring[d], 0);
             issue(g + d + D, ring[d]);
           }
           __syncthreads();
@@ -595,9 +579,9 @@ struct TileGemm {
         if (g + dd < gsteps) {
           if (FAST && g + dd + D < gsteps) {
             const int k_next = target(g + dd + D);
-            restage<true, RAW>(ctx, lds + ((g + dd) & 1) * LL::kStage, ring[d], k_next);
+            restage<true>(ctx, lds + ((g + dd) & 1) * LL::kStage, ring[d], k_next);
           } else {
-            restage<false, RAW>(ctx, lds + ((g + dd) & 1) * LL::kStage, ring[d], 0);
+            restage<false>(ctx, lds + ((g + dd) & 1) * LL::kStage, ring[d], 0);
             if (g + dd + D < gsteps) issue(g + dd + D, ring[d]);
           }
           __syncthreads();
@@ -803,8 +787,7 @@ struct TileGemm {
               for (int e = 0; e < 4; ++e) {
                 const float y = gated(res[mi][2 * nj][4 * q + e] + bv, res[mi][2 * nj + 1][4 * q + e] + bg);
                 const int soff = (mi * 32 + q * 8 + e) * ldc_bytes;
-                if constexpr (IODT == CASCMM_DT_F32) llvm_raw_buffer_store_f32(y, rc, voff, soff, kResultStoreAux);
-                else llvm_raw_buffer_store_i16(__builtin_bit_cast(short, (IoT)y), rc, voff, soff, kResultStoreAux);
+                llvm_raw_buffer_store_f32(y, rc, voff, soff, kResultStoreAux);
               }
         }
         return;

@@ -16,8 +16,9 @@ namespace cascmm {
 // KIND_F8K64: three fp8 terms on the fp8-rate MFMA; splits its operands into the workspace first
 // KIND_F16K: three fp16 terms on operand slots; finds both scales and splits its operands into the workspace first
 // KIND_WAVEK: skinny problems in one launch, K split over the waves of a workgroup (no workspace)
+// KIND_H16: 16-bit tensors as one term of their own format, right operand prepared or raw (no workspace)
 // KIND_SLOTK: prepared right operand, K split over the waves of a workgroup (64 x 160 tiles, one problem per launch)
-enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6 };
+enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7 };
 constexpr int kNumCUs = 256;  // MI355X: what the cost model's constants were measured on
 constexpr int kMaxDevices = 64;
 
@@ -420,14 +421,6 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
    &launch_tile<Tile<BM, BN, BK, WM, WN, WK, DEPTH, NP, false>, CASCMM_DT_F32, FMT, TERMS, FULL, true, true>, true,    \
    ((BN) / (WN)) % 64 == 0}
 
-// fp16 (bf16) operands in memory multiplied as one fp16 (bf16) term, right operand prepared: the
-// producers only copy
-#define CASCMM_TILE_VARIANT_BPRE16(NAME, BM, BN, BK, WM, WN, WK, DEPTH, NP, IODT, FMT)                       \
-  {NAME, KIND_TILE, IODT, FMT, 1, false, BM, BN, BK, Tile<BM, BN, BK, WM, WN, WK, DEPTH, NP, false>::NT,     \
-   LdsLayout<Tile<BM, BN, BK, WM, WN, WK, DEPTH, NP, false>, 1>::kBytes, true, true,                         \
-   &launch_tile<Tile<BM, BN, BK, WM, WN, WK, DEPTH, NP, false>, IODT, FMT, 1, false, true, true>, true,      \
-   ((BN) / (WN)) % 64 == 0}
-
 // B-direct kernels: fp32 operands, fast path only
 #define CASCMM_BD_VARIANT(NAME, BM, WN, BK, DEPTH, NP, FMT, TERMS, FULL)                                \
   {NAME, KIND_TILE, CASCMM_DT_F32, FMT, TERMS, FULL, BM, 32 * WN, BK, TileBD<BM, WN, BK, DEPTH, NP>::NT, \
@@ -474,5 +467,6 @@ const VariantDesc* variants_fp8(int* n);
 const VariantDesc* variants_io16(int* n);
 const VariantDesc* variants_bpre(int* n);
 const VariantDesc* variants_chain(int* n);
+const VariantDesc* variants_h16(int* n);
 
 }  // namespace cascmm

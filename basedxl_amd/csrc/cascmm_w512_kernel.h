@@ -110,7 +110,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
     if (BPRE) {
       // run inst = (term * 2 + k group) * 5 + run of 64 columns; lane = column inside the run
       const int tk = inst / 5, run = inst % 5;
-      b_voff[j] = (((tk >> 1) * (p.K >> 3) + (tk & 1)) * p.N + n0 + run * 64 + lane) * 16;
+      b_voff[j] = (((tk >> 1) * (int)prepared_kgroups(p.K) + (tk & 1)) * p.N + n0 + run * 64 + lane) * 16;
     } else {
       const int f = inst * 256 + lane * 4;
       const int k = f / T::BN, pos = f % T::BN;

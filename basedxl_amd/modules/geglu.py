@@ -22,7 +22,7 @@ class BasedXLLowPGEGLU(nn.Module):
     ``value * gelu(gate)`` ([..., inner]), gelu in its exact (erf) form.
 
     The fused kernels take fp32 activations (any cascade) or fp16 / bf16 activations (as one term of
-    their own format) on the GPU with ``in % 64 == 0`` and ``inner % 32 == 0`` and read a prepared
+    their own format) on the GPU with ``in % 64 == 0`` (16-bit: ``% 8``) and ``inner % 32 == 0`` and read a prepared
     (pre-split, column-interleaved) copy of the weight, made on first use.  ``prepared=False`` keeps
     no such copy: the large-tile kernel applies the gate on the raw weight where it takes the problem
     (fp32, two bf16 terms, rows % 256 == 0, inner % 160 == 0).  Anything else runs the cascade GEMM on the
@@ -42,14 +42,17 @@ class BasedXLLowPGEGLU(nn.Module):
         self._prepared: Optional[PreparedWeight] = None
 
     def _fusable(self, x: torch.Tensor) -> bool:
-        if not x.is_cuda or x.dtype != self.weight.dtype or self.in_features % 64 != 0 or self.inner % 32 != 0:
+        if not x.is_cuda or x.dtype != self.weight.dtype or not self._preparable():
             return False
         # 16-bit tensors have prepared kernels only for one term of their own format
         return x.dtype == torch.float32 or (self.lowp, self.terms) == default_cascade(x.dtype)
 
+    def _preparable(self) -> bool:
+        return self.in_features % (64 if self.weight.dtype == torch.float32 else 8) == 0 and self.inner % 32 == 0
+
     def prepare(self) -> None:
         """Prepare the gated weight now (needs the weight on the GPU); otherwise on the first eager call."""
-        if self.prepared and self.weight.is_cuda and self.in_features % 64 == 0 and self.inner % 32 == 0 and (
+        if self.prepared and self.weight.is_cuda and self._preparable() and (
                 self._prepared is None or self._prepared.device != self.weight.device):
             self._prepared = PreparedWeight(self.weight, lowp=self.lowp, terms=self.terms, glu=True)
 

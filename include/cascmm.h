@@ -33,9 +33,9 @@ extern "C" {
 /* element type of A, B, C and bias as stored in memory (C has the type of A, like
  * `torch.empty((M, N), dtype=a.dtype)` at cascaded_lowp_matmul.py:161).  The cascade kernels
  * take fp32.  fp16 (bf16) tensors multiplied as ONE fp16 (bf16) term have fast kernels too:
- * through cascmm_gemm_prepared, or through cascmm_gemm when K % 64 == 0, the rows of A are
- * 16-byte aligned and the workspace holds cascmm_workspace_bytes(...) (B is re-laid there
- * first).  Other combinations with 16-bit tensors run on bounds-checked kernels (bf16 or
+ * through cascmm_gemm_prepared, or through cascmm_gemm, when K % 8 == 0 and the rows of A are
+ * 16-byte aligned (a raw B whose rows are not whole 16-byte chunks is re-laid in the workspace
+ * first, cascmm_workspace_bytes(...)).  Other combinations with 16-bit tensors run on bounds-checked kernels (bf16 or
  * fp16 terms, 1 or 2 of them, tri). */
 enum cascmm_dtype { CASCMM_DT_F32 = 0, CASCMM_DT_F16 = 1, CASCMM_DT_BF16 = 2 };
 
@@ -141,7 +141,8 @@ int cascmm_gemm_grouped(int count, const void* const* A, const void* const* B, v
  * Prepared weights.  A Linear layer's weight is constant, so its split can be done once: the
  * counterpart of the one-time `W.T.contiguous().clone()` of basedxl/modules/lowp_linear.py:12.
  * cascmm_prepare_weight writes B[K,N] (leading dimension ldb, element type `dtype`) as MFMA
- * operand slots -- 16 bytes = 8 consecutive k of one column of one plane, [plane][ceil(K/8)][N];
+ * operand slots -- 16 bytes = 8 consecutive k of one column of one plane, [plane][8 ceil(K/64)][N]
+ * (the slots past K are zero);
  * planes = terms (bf16, fp16) or ceil(terms/2) (fp8) -- into `out` (16-byte aligned, at least
  * cascmm_prepared_bytes(K, N, fmt, terms) bytes, allocated by the caller).  fp8: *tensor_exp
  * (device int32, NULL = 0) is the scale exponent applied before the split; pass the same value
@@ -149,8 +150,8 @@ int cascmm_gemm_grouped(int count, const void* const* A, const void* const* B, v
  * cascmm_gemm_prepared runs `count` (1..8) GEMMs C[i] = A[i] . B[i] (+ bias[i]) of one shape whose
  * right operands are prepared buffers; arguments as cascmm_gemm_grouped, without ldb (the
  * workspace, which may be NULL, is used for the K split of under-filled single launches and
- * holds cascmm_workspace_bytes(...)).  Only the fast kernels exist for it: A must be fp32 with 16-byte aligned rows
- * (CASCMM_ERR_ALIGNMENT otherwise), K a multiple of 32 or 64 depending on the kernel
+ * holds cascmm_workspace_bytes(...)).  Only the fast kernels exist for it: A must have 16-byte aligned rows
+ * (CASCMM_ERR_ALIGNMENT otherwise), K be a multiple of 32 or 64 depending on the kernel (16-bit: of 8)
  * (CASCMM_ERR_BAD_FORMAT when no kernel fits), the prepared buffer below 2 GiB
  * (CASCMM_ERR_TOO_LARGE).  The results equal cascmm_gemm's bit for bit when the same kernel
  * tile is used (same split, same order of accumulation).
