@@ -189,7 +189,7 @@ class PreparedWeight:
     kept as MFMA operand slots; ``cascaded_lowp_matmul(a, prepared)`` then splits only ``a``.
     The arithmetic is the same as with the raw weight (same split, same products).  Kernels for
     prepared weights exist for bf16 x 2, bf16 x 3, fp16 x 3 and fp8 x 3 with the 'tri' product set and
-    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4 (16-bit: K of 8); the
+    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4 (two bf16 terms and 16-bit: K of 8); the
     product with any other combination fails with CascmmError (use the raw weight there).
 
     ``glu=True``: ``w`` is the ``[in, 2 * inner]`` weight of a gated projection (diffusers' GEGLU:
@@ -245,15 +245,19 @@ class PreparedWeight:
         return self
 
     def usable_with(self, a2: torch.Tensor, products: str = "tri") -> bool:
-        """Whether the prepared kernels take this left operand, rows 16-byte aligned: fp32 with K a multiple
-        of 64 and N of 4, or fp16 / bf16 tensors with a weight of the same dtype kept as one term of that format
-        and K a multiple of 8 (anything else goes through the raw weight)."""
-        if a2.data_ptr() % 16 != 0 or not self.has_kernel(a2.dtype, products):
+        """Whether the prepared kernels take this left operand: fp32, two bf16 terms: K a multiple of 8; other
+        cascades and gated weights: K a multiple of 64, N of 4, rows 16-byte aligned; fp16 / bf16 tensors with a
+        weight of the same dtype kept as one term of that format: K a multiple of 8, rows on dwords (anything else
+        goes through the raw weight)."""
+        if not self.has_kernel(a2.dtype, products):
             return False
-        if a2.dtype == torch.float32:
-            return self.K % 64 == 0 and self.N % 4 == 0 and (a2.shape[0] <= 1 or a2.stride(0) % 4 == 0)
-        return (self.K % 8 == 0 and a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp
-                and (a2.shape[0] <= 1 or a2.stride(0) % 8 == 0))
+        rows, lda = a2.shape[0], a2.stride(0)
+        if a2.dtype != torch.float32:
+            return (self.K % 8 == 0 and a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp
+                    and a2.data_ptr() % 4 == 0 and (rows <= 1 or lda % 2 == 0))
+        if (self.lowp, self.terms) == ("bf16", 2) and not self.glu and self.K % 8 == 0:
+            return True
+        return self.K % 64 == 0 and self.N % 4 == 0 and a2.data_ptr() % 16 == 0 and (rows <= 1 or lda % 4 == 0)
 
     def has_kernel(self, dtype: torch.dtype, products: str = "tri") -> bool:
         """Whether the library has a prepared-operand kernel for this weight's cascade with left
@@ -293,8 +297,8 @@ def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, pro
         if a.dtype not in _DTYPES:
             raise TypeError(f"unsupported dtype {a.dtype}")
         a2 = _rows(a.reshape(-1, w.K))
-        # the prepared kernels load 16 bytes of a row at a time: rows that do not start on such a
-        # boundary are copied, as basedxl/triton/cascaded_lowp_matmul.py:158 copies every `a`
+        # most prepared kernels want rows that start on 16-byte boundaries: others are copied, as
+        # basedxl/triton/cascaded_lowp_matmul.py:158 copies every `a`
         per16 = 16 // a2.element_size()
         if a2.data_ptr() % 16 != 0 or (a2.shape[0] > 1 and a2.stride(0) % per16 != 0):
             a2 = a2.contiguous()
@@ -468,10 +472,9 @@ def cascaded_lowp_matmul_grouped(a_list, b_list, *, outs=None, biases=None, lowp
                     exps[2 * i + 1:2 * i + 2].copy_(kept.reshape(1))
             if kept is None:
                 _activation_exps(b_list[i], max(N, 1), None, exps.data_ptr() + 8 * i + 4, stream)
-    # 16-bit tensors as one term of their own format: room for every right operand re-laid as operand slots (rows that are
-    # not whole 16-byte chunks)
+    # room for every operand whose rows have to be copied first (rows that are not whole 16-byte chunks)
     ws = None
-    if a_list[0].dtype != torch.float32:
+    if a_list[0].dtype != torch.float32 or K % 4 != 0:
         need = _workspace_bytes(M, N, K, _DTYPES[a_list[0].dtype], fmt, terms, prod)
         ws = _workspace(dev, stream, n * need) if need else None
     st = _lib.lib().cascmm_gemm_grouped(n, pa, pb, pc, pbias, M, N, K, lda, max(N, 1), max(N, 1),

@@ -52,12 +52,25 @@ struct Problem {
   bool bpre = false;  // B is a prepared (already split) weight buffer
   bool glu = false;   // gated epilogue: B prepared by cascmm_prepare_weight_glu, C has N / 2 columns
   bool glu_slots = false;   // ... written as the left operand slots of the next GEMM (large-tile kernel only)
+  // the rows of A are whole 16-byte chunks with zeros between K and the last chunk's end: fp32 with K % 4 == 0, 16-bit
+  // with K % 8 == 0, or rows padded in the workspace (relay)
+  bool chunked = false;
+  // three fp8 / fp16 terms: only the kernels that split both operands into slots first; K is rounded up to whole
+  // stages, of which the operands hold k_valid, and their rows need no alignment
+  bool split_first = false;
+  int64_t k_valid = 0;
 };
 
 // Three fp8 terms with K a multiple of 64 are prepared for the fp8-rate kernel: [term][K/16][N] slots
 // of 16 k each (the gated layout keeps the older form, whose kernels have the gated store)
 static bool prepared_as_k16_slots(int64_t K, int fmt, int terms, bool glu) {
   return fmt == CASCMM_FMT_FP8 && terms == 3 && K > 0 && K % F8K64::BK == 0 && !glu;
+}
+
+// a x b x c > 2^31 - 1, for any non-negative 64-bit factors (the product itself may not fit 64 bits)
+static bool beyond_i32(int64_t a, int64_t b, int64_t c) {
+  int64_t ab = 0, abc = 0;
+  return __builtin_mul_overflow(a, b, &ab) || __builtin_mul_overflow(ab, c, &abc) || abc > INT32_MAX;
 }
 
 // bytes of a prepared weight: planes x prepared_kgroups(K) x N operand slots of 16 bytes
@@ -77,7 +90,7 @@ static int check_problem(const Problem& q) {
   if (q.products != CASCMM_PROD_TRI && q.products != CASCMM_PROD_FULL) return CASCMM_ERR_BAD_FORMAT;
   if (q.M < 0 || q.N < 0 || q.K < 0) return CASCMM_ERR_BAD_SHAPE;
   if (q.M > INT32_MAX || q.N > INT32_MAX || q.K > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
-  if (q.lda < q.K || q.ldb < q.N || q.ldc < (q.glu ? q.N / 2 : q.N)) return CASCMM_ERR_BAD_SHAPE;
+  if (q.lda < (q.split_first ? q.k_valid : q.K) || q.ldb < q.N || q.ldc < (q.glu ? q.N / 2 : q.N)) return CASCMM_ERR_BAD_SHAPE;
   return CASCMM_OK;
 }
 
@@ -86,23 +99,37 @@ static bool own_format16(const Problem& q) {
   return q.terms == 1 && ((q.dtype == CASCMM_DT_F16 && q.fmt == CASCMM_FMT_FP16) || (q.dtype == CASCMM_DT_BF16 && q.fmt == CASCMM_FMT_BF16));
 }
 
-// what the fast (buffer-load, 16-byte accesses, no K tail) kernels need apart from K % BK == 0
-static bool fast_ok(const Problem& q, const void* A, const void* B) {
+// What the rows of the operands allow.  FIT_DWORD: 32-bit byte offsets inside a tile and down a column block of B
+// (buffer offsets are 32-bit): the kernels whose loads are checked against the buffers' ends dword by dword take any
+// alignment and any N.  FIT_FAST: 16-byte aligned rows and N % 4 == 0 too, which the other fast kernels need (K % BK is
+// checked per kernel).  16-bit tensors have one kind of fast kernel: rows on dwords.
+enum RowFit { FIT_NONE = 0, FIT_DWORD = 1, FIT_FAST = 2 };
+static RowFit row_fit(const Problem& q, const void* A, const void* B) {
   if (q.dtype != CASCMM_DT_F32) {
-    // 16-bit operands: only as one term of their own format; a raw right operand with whole 16-byte chunks too
-    return own_format16(q) && q.lda % 8 == 0 && (A == nullptr || aligned_to(A, 16)) && q.lda * 2 * 512 < INT32_MAX &&
-           (q.bpre || (q.ldb % 8 == 0 && q.N % 8 == 0 && (B == nullptr || aligned_to(B, 16))));
+    // 16-bit operands: only as one term of their own format
+    return own_format16(q) && q.lda % 2 == 0 && (A == nullptr || aligned_to(A, 4)) && q.lda * 2 * 512 < INT32_MAX &&
+                   (q.bpre || (q.ldb % 2 == 0 && q.N % 2 == 0 && (B == nullptr || aligned_to(B, 4))))
+               ? FIT_FAST
+               : FIT_NONE;
   }
-  return q.dtype == CASCMM_DT_F32 && q.lda % 4 == 0 && (A == nullptr || aligned_to(A, 16)) &&
-         q.ldb % 4 == 0 && q.N % 4 == 0 && (B == nullptr || aligned_to(B, 16)) &&
-         q.lda * 4 * 512 < INT32_MAX && q.ldb * 4 * 136 < INT32_MAX &&  // 32-bit byte offsets inside a tile
-         (q.bpre || q.K * q.ldb * 4 < INT32_MAX);  // ... and down a column block of B (buffer offsets are 32-bit)
+  if (q.split_first) return FIT_FAST;
+  if (!(q.lda * 4 * 512 < INT32_MAX && (q.bpre || (q.ldb * 4 * 136 < INT32_MAX && q.K * q.ldb * 4 < INT32_MAX)))) return FIT_NONE;
+  return q.lda % 4 == 0 && (A == nullptr || aligned_to(A, 16)) &&
+                 (q.bpre || (q.ldb % 4 == 0 && q.N % 4 == 0 && (B == nullptr || aligned_to(B, 16))))
+             ? FIT_FAST
+             : FIT_DWORD;
 }
 
-static bool variant_matches(const VariantDesc& v, const Problem& q, bool fast) {
+static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) {
   const int full = (q.products == CASCMM_PROD_FULL && q.terms > 1) ? 1 : 0;
   if (v.iodt != q.dtype || v.fmt != q.fmt || v.terms != q.terms || v.full != full || v.bpre != q.bpre) return false;
-  if (v.fast && (!fast || (v.kind != KIND_H16 && q.K % v.BK != 0))) return false;
+  if (q.split_first && v.kind != KIND_F8K64 && v.kind != KIND_F16K) return false;
+  const bool any_rows = v.kind == KIND_WAVEK || v.kind == KIND_SLOTK;
+  if (v.fast && fit < (any_rows ? FIT_DWORD : FIT_FAST)) return false;
+  // K in whole 32-k steps, or a tail of whole 16-byte chunks (a weight less than one 64-k stage deep is not worth keeping
+  // split: such a prepared operand is refused)
+  if (any_rows && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
+  if (v.fast && !any_rows && v.kind != KIND_H16 && q.K % v.BK != 0) return false;
   if (v.kind == KIND_SPLITK && (q.M > 5 * v.BM || q.K < 4 * v.BK)) return false;  // skinny: few row tiles, deep K
   if (v.kind == KIND_F8K64 && (q.products != CASCMM_PROD_TRI || q.K % v.BK != 0 || q.K == 0 || q.glu ||
                                f8k64_slot_bytes(q.M, q.K) > INT32_MAX || f8k64_slot_bytes(q.N, q.K) > INT32_MAX))
@@ -115,11 +142,11 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, bool fast) {
   if (v.kind == KIND_W512 && (q.M % v.BM != 0 || q.N % v.BN != 0 || q.M * q.lda * 4 > INT32_MAX ||
                               (!q.bpre && q.K * q.ldb * 4 > INT32_MAX) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
-  if (v.kind == KIND_WAVEK && (q.N % v.BN != 0 || q.M * q.lda * 4 > INT32_MAX || q.K == 0)) return false;
-  if (v.kind == KIND_SLOTK && (q.K % 32 != 0 || q.K < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
+  if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
+  if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
   // (32-bit byte offsets down A and, where it is raw, B, two stages past the end included; K in whole 16-byte chunks)
-  if (v.kind == KIND_H16 && (q.K % 8 != 0 || q.K == 0 || q.M * q.lda * 2 > INT32_MAX || (!q.bpre && (q.K + 64) * q.ldb * 2 > INT32_MAX)))
+  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || q.M * q.lda * 2 > INT32_MAX || (!q.bpre && beyond_i32(q.K + 64, q.ldb, 2))))
     return false;
   if (q.glu && !v.glu) return false;
   if (q.glu_slots && v.kind != KIND_W512) return false;
@@ -199,11 +226,10 @@ static const std::vector<VariantInfo>& variant_info() {
 // costs 2.5 us, prologue and the meeting of the partial tiles 0.6 us per round of workgroups.
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
-         !q.glu && q.K > 0 && q.K % 32 == 0 && q.N % 32 == 0 && q.M * q.lda * 4 <= INT32_MAX;
+         !q.glu && q.K > 0 && (q.K % 32 == 0 || q.chunked) && q.M * q.lda * 4 <= INT32_MAX;
 }
 static double wavek_estimate_us(const Problem& q, int count, int bn) {
-  if (q.N % bn != 0) return 1e9;
-  const double items = (double)count * (double)((q.M + 31) / 32) * (double)(q.N / bn);
+  const double items = (double)count * (double)((q.M + 31) / 32) * (double)((q.N + bn - 1) / bn);
   const double active = items < kNumCUs ? items : kNumCUs;
   const double per_cu = bn == 32 ? 85.0e3 : 60.0e3;                       // bytes per us
   const double rate = per_cu < 17.0e6 / active ? per_cu : 17.0e6 / active;
@@ -349,8 +375,9 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
 struct SelectKey {
   int64_t M, N, K;
   size_t ws_bytes;
-  // flags: fast | bpre << 1 | glu << 2, and what variant_matches reads of the leading dimensions (the
-  // 32-bit addressing limits of some kernels): M lda, K ldb and 1024 ldc beyond 2^31 bytes << 3, 4, 5
+  // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
+  // some kernels: M lda, K ldb and 1024 ldc beyond 2^31 bytes << 3, 4, 5; lda below 32 << 7), glu_slots << 6,
+  // chunked << 8, split_first << 9, the fit of the rows << 10
   int dtype, fmt, terms, products, count, flags;
   bool operator==(const SelectKey& o) const {
     return M == o.M && N == o.N && K == o.K && ws_bytes == o.ws_bytes && dtype == o.dtype && fmt == o.fmt &&
@@ -369,20 +396,14 @@ struct SelectKeyHash {
 };
 struct SelectHit { int variant, splits; };
 
-static int select_variant_uncached(const Problem& q, bool fast, int count, size_t ws_bytes, int* splits_out);
+static int select_variant_uncached(const Problem& q, RowFit fit, int count, size_t ws_bytes, int* splits_out);
 
-// a x b x c > 2^31 - 1, for any non-negative 64-bit factors (the product itself may not fit 64 bits)
-static bool beyond_i32(int64_t a, int64_t b, int64_t c) {
-  int64_t ab = 0, abc = 0;
-  return __builtin_mul_overflow(a, b, &ab) || __builtin_mul_overflow(ab, c, &abc) || abc > INT32_MAX;
-}
-
-static int select_variant(const Problem& q, bool fast, int count, size_t ws_bytes = (size_t)-1,
+static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_bytes = (size_t)-1,
                           int* splits_out = nullptr) {
   static std::mutex mu;
   static std::unordered_map<SelectKey, SelectHit, SelectKeyHash> memo;
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
-                      (fast ? 1 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
+                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
                           (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0)};
   {
     std::lock_guard<std::mutex> lock(mu);
@@ -393,7 +414,7 @@ static int select_variant(const Problem& q, bool fast, int count, size_t ws_byte
     }
   }
   int splits = 1;
-  const int v = select_variant_uncached(q, fast, count, ws_bytes, &splits);
+  const int v = select_variant_uncached(q, fit, count, ws_bytes, &splits);
   {
     std::lock_guard<std::mutex> lock(mu);
     if (memo.size() >= 4096) memo.clear();
@@ -403,13 +424,13 @@ static int select_variant(const Problem& q, bool fast, int count, size_t ws_byte
   return v;
 }
 
-static int select_variant_uncached(const Problem& q, bool fast, int count, size_t ws_bytes, int* splits_out) {
+static int select_variant_uncached(const Problem& q, RowFit fit, int count, size_t ws_bytes, int* splits_out) {
   const auto& t = table();
   int best = -1;
   double best_cost = 0;
   if (splits_out) *splits_out = 1;
   for (int i = 0; i < (int)t.size(); ++i) {
-    if (!variant_matches(t[i], q, fast)) continue;
+    if (!variant_matches(t[i], q, fit)) continue;
     if (count > 1 && !t[i].grouped) continue;
     if (t[i].kind == KIND_SPLITK &&
         skinny_workspace_bytes(q.M, q.N, q.K, t[i].BM, t[i].BN, t[i].BK) > ws_bytes)
@@ -567,29 +588,193 @@ static int launch_prepare_fmt(const void* B, int K, int N, int64_t ldb, int fmt,
   return CASCMM_ERR_BAD_FORMAT;
 }
 
-// 16-bit tensors multiplied as one term of their own format can use the prepared-operand kernels
-// when the caller brought room for the re-laid B
-// (a grouped launch needs `count` such buffers, one behind the other)
-// (where the kernels that read a raw right operand do not take it: rows that are not whole 16-byte chunks)
-static bool onthefly_prepare_ok(const Problem& q, int count, const void* const* A, const void* const* B,
-                                const void* workspace, size_t workspace_bytes) {
-  if (q.bpre || !own_format16(q) || q.K % 8 != 0 || q.lda % 8 != 0) return false;
-  bool raw = true;   // every right operand can be read where it lies
-  for (int i = 0; i < count; ++i) {
-    if (!A[i] || !B[i] || !aligned_to(A[i], 16) || !aligned_to(B[i], 2)) return false;
-    raw = raw && fast_ok(q, A[i], B[i]);
+// ---------------------------------------------------------------------------------------
+// operands whose rows no fast kernel reads, copied into the workspace first
+// ---------------------------------------------------------------------------------------
+// Workgroups 0 .. a_blocks - 1: rows of A [M][K] (row stride lda) as rows of a_chunks 16-byte chunks, zeros past K; a
+// thread writes one chunk.  The others (16-bit elements as one term of their own format only): B [K][N] as operand
+// slots [8 ceil(K/64)][N], a thread the eight k of a column.  E: an unsigned type of the elements' size; bits are moved.
+template <typename E>
+__global__ __launch_bounds__(256) void relay_kernel(const E* __restrict__ A, int M, int K, int64_t lda, int a_chunks, u32x4* __restrict__ a_out,
+                                                   int a_blocks, const E* __restrict__ B, int N, int64_t ldb, u32x4* __restrict__ b_out) {
+  constexpr int PER = 16 / sizeof(E);
+  typedef E chunk_t __attribute__((ext_vector_type(PER)));
+  chunk_t c;
+  if ((int)blockIdx.x < a_blocks) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)M * a_chunks) return;
+    const int row = (int)(i / a_chunks), k0 = (int)(i - (int64_t)row * a_chunks) * PER;
+    const E* src = A + (int64_t)row * lda + k0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) c[e] = k0 + e < K ? src[e] : (E)0;
+    a_out[i] = __builtin_bit_cast(u32x4, c);
+  } else {
+    const int64_t i = (int64_t)(blockIdx.x - a_blocks) * 256 + threadIdx.x;
+    if (i >= prepared_kgroups(K) * N) return;
+    const int kg = (int)(i / N), n = (int)(i - (int64_t)kg * N);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) c[e] = kg * PER + e < K ? B[(int64_t)(kg * PER + e) * ldb + n] : (E)0;
+    b_out[i] = __builtin_bit_cast(u32x4, c);
   }
-  if (raw && select_variant(q, true, count, 0) >= 0) return false;
-  const int64_t need = prepared_bytes(q.K, q.N, q.fmt, 1);
-  return workspace && aligned_to(workspace, 16) && need <= INT32_MAX && workspace_bytes >= (size_t)need * count;
 }
 
-// One launch for `count` problems of one shape (count == 1: a plain GEMM).
+// What a problem needs copied before the fast kernels take it (nothing: neither flag), and the bytes of one such copy,
+// rounded up to whole 256.  fp32 (two bf16 terms): rows of A whose length is not a multiple of 4; everything else is read
+// where it lies.  16-bit: rows of A that are not whole chunks or do not start on dwords, and a raw B of odd N or ldb.
+// The bounds-checked kernels, which read element by element, stay for callers without a workspace: 7488 x 1061 x 3192
+// fp32 601 us, copied first 248; 37 x 2139 x 6528 fp16 238 against 15; and where nothing is copied, 333 x 456 x 211 18.6
+// against 6.4, 44 x 1124 x 1728 42.5 against 8.7.
+struct Relay { bool a = false, b = false; size_t a_bytes = 0, b_bytes = 0; int a_chunks = 0; };
+static Relay relay_of(const Problem& q, int count, const void* const* A, const void* const* B) {
+  Relay r;
+  if (q.bpre || q.split_first || q.K == 0) return r;
+  const bool f32 = q.dtype == CASCMM_DT_F32;
+  if (f32 ? !(q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && (q.products == CASCMM_PROD_TRI)) : !own_format16(q)) return r;
+  const int64_t es = f32 ? 4 : 2, per = 16 / es;
+  r.a = q.K % per != 0 || (!f32 && q.lda % 2 != 0);
+  r.b = !f32 && (q.N % 2 != 0 || q.ldb % 2 != 0);
+  for (int i = 0; i < count; ++i) {
+    r.a = r.a || (!f32 && A && !aligned_to(A[i], 4));
+    r.b = r.b || (!f32 && B && !aligned_to(B[i], 4));
+  }
+  const int64_t lines = (q.K * es + 127) / 128;   // (rows of whole cache lines)
+  int64_t a_bytes = 0, b_bytes = r.b ? prepared_bytes(q.K, q.N, q.fmt, 1) : 0;
+  if (__builtin_mul_overflow(q.M, lines * 128, &a_bytes) || a_bytes > INT32_MAX || b_bytes > INT32_MAX) return Relay();
+  r.a_chunks = (int)lines * 8;
+  r.a_bytes = r.a ? f8k64_up(a_bytes) : 0;
+  r.b_bytes = f8k64_up(b_bytes);
+  return r;
+}
+static size_t relay_bytes(const Relay& r, int count) { return (size_t)count * (r.a_bytes + r.b_bytes); }
+
+// three fp8 / fp16 terms that the slot kernels take once K is rounded up to their stages: they split both operands in a
+// pass of their own, which fills the rest with zeros and reads rows of any alignment
+static Problem rounded_up(const Problem& q, RowFit fit) {
+  Problem e = q;
+  e.k_valid = q.K;
+  const int64_t step = q.fmt == CASCMM_FMT_FP8 ? 64 : 32;
+  if (q.dtype == CASCMM_DT_F32 && !q.bpre && !q.glu && q.terms == 3 && q.products == CASCMM_PROD_TRI && q.fmt != CASCMM_FMT_BF16 &&
+      (fit != FIT_FAST || q.K % step != 0) && q.K > 0 && !beyond_i32(q.K, q.ldb, 4)) {
+    e.split_first = true;
+    e.K = (q.K + step - 1) / step * step;
+  }
+  return e;
+}
+
+// The slot kernel for such a problem, or a negative status: none, no room, or the bounds-checked kernel, which needs one
+// launch where these need three, is expected to be faster (a 32-k step of its 64 x 64 tiles 1.35 us: 100 x 300 x 200
+// fp16 x 3 16.5 us against 21; 300 x 500 x 1001 25.9 against 24, fp8 x 3 35 against 26, 3740 x 1090 x 992 fp16 x 3 132 against 81)
+static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem* e) {
+  *e = rounded_up(q, fit);
+  if (!e->split_first) return CASCMM_ERR_BAD_FORMAT;
+  const int v = select_variant(*e, FIT_FAST, 1, room);
+  if (v < 0) return v;
+  const double tiles = (double)((q.M + 63) / 64) * (double)((q.N + 63) / 64);
+  const double rounds = (double)(int64_t)((tiles + kNumCUs - 1) / kNumCUs);
+  return variant_cost(v, *e, 1) < 3.5 + 1.35 * rounds * (double)((q.K + 31) / 32) ? v : (int)CASCMM_ERR_BAD_FORMAT;
+}
+
+// The launch itself, on operands as they lie (exps_dyn, b_exp_src: see gemm_impl)
+static int gemm_on_rows(int count, const void* const* A, const void* const* B, void* const* C, const void* const* bias, const Problem& q0,
+                        const int32_t* tensor_exps, void* workspace, size_t workspace_bytes, hipStream_t stream, int variant,
+                        int32_t* exps_dyn = nullptr, const int32_t* b_exp_src = nullptr) {
+  Problem q = q0;
+  const size_t es = dtype_size(q.dtype);
+  RowFit fit = FIT_FAST;
+  for (int i = 0; i < count; ++i) {
+    if (!A[i] || !B[i]) return CASCMM_ERR_NULL_POINTER;
+    if (!aligned_to(A[i], es) || !aligned_to(B[i], q.bpre ? 16 : es)) return CASCMM_ERR_ALIGNMENT;
+    fit = std::min(fit, row_fit(q, A[i], q.bpre ? nullptr : B[i]));
+  }
+  if (q.bpre) {
+    // prepared weights only have the fast kernels: K and the rows of A as the kernel needs them (checked per
+    // variant), and a buffer the 32-bit offsets can span
+    if (fit == FIT_NONE) return CASCMM_ERR_ALIGNMENT;
+    if (prepared_bytes(q.K, q.N, q.fmt, q.terms, q.glu) > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
+  }
+
+  const auto& t = table();
+  int splits = 1;
+  if (variant < 0) {
+    if (count == 1 && !q.split_first) {
+      Problem e;
+      if (select_rounded_up(q, fit, workspace ? workspace_bytes : 0, &e) >= 0) {
+        q = e;
+        fit = FIT_FAST;
+      }
+    }
+    variant = select_variant(q, fit, count, workspace ? workspace_bytes : 0, &splits);
+    if (variant < 0 && count > 1) {
+      // no kernel takes these problems in one launch (the fp8-rate kernel runs one at a time): one
+      // launch each, in order on the stream, sharing the workspace
+      for (int i = 0; i < count; ++i) {
+        const void* bi = bias ? bias[i] : nullptr;
+        const int st1 = gemm_on_rows(1, A + i, B + i, C + i, bias ? &bi : nullptr, q, tensor_exps ? tensor_exps + 2 * i : nullptr,
+                                  workspace, workspace_bytes, stream, -1);
+        if (st1 != CASCMM_OK) return st1;
+      }
+      return CASCMM_OK;
+    }
+    if (variant < 0) return variant;
+  } else {
+    splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
+    variant &= 0xFFFF;
+    if (splits > kMaxTileSplits) return CASCMM_ERR_BAD_VARIANT;
+    if (variant >= (int)t.size()) return CASCMM_ERR_BAD_VARIANT;
+    if (!variant_matches(t[variant], q, fit)) return CASCMM_ERR_BAD_VARIANT;
+  }
+  const VariantDesc& v = t[variant];
+  if (exps_dyn && (v.kind != KIND_F8K64 || count != 1)) return CASCMM_ERR_BAD_VARIANT;
+  if (count > 1 && !v.grouped) {
+    // a forced kernel that runs one problem per launch: one launch each, in order on the stream
+    if (v.kind == KIND_SPLITK) return CASCMM_ERR_BAD_VARIANT;
+    for (int i = 0; i < count; ++i) {
+      const void* bi = bias ? bias[i] : nullptr;
+      const int st1 = gemm_on_rows(1, A + i, B + i, C + i, bias ? &bi : nullptr, q, tensor_exps ? tensor_exps + 2 * i : nullptr,
+                                workspace, workspace_bytes, stream, variant | (splits > 1 ? splits << 16 : 0));
+      if (st1 != CASCMM_OK) return st1;
+    }
+    return CASCMM_OK;
+  }
+  GroupParams p;
+  memset(&p, 0, sizeof(p));
+  p.M = (int)q.M; p.N = (int)q.N; p.K = (int)q.K;
+  p.k_valid = (int)(q.split_first ? q.k_valid : q.K);
+  p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc;
+  const int64_t tm = (q.M + v.BM - 1) / v.BM, tn = (q.N + v.BN - 1) / v.BN;
+  if (tm * tn * count > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
+  p.tiles_m = (int)tm; p.tiles_n = (int)tn;
+  p.count = count;
+  p.workspace = workspace;
+  p.workspace_bytes = workspace_bytes;
+  p.k_splits = v.kind == KIND_TILE ? splits : 1;
+  p.tensor_exps = q.fmt == CASCMM_FMT_FP8 ? tensor_exps : nullptr;
+  p.glu = q.glu_slots ? 2 : (q.glu ? 1 : 0);
+  p.exps_dyn = exps_dyn;
+  p.b_exp_src = b_exp_src;
+  for (int i = 0; i < count; ++i) {
+    p.A[i] = A[i]; p.B[i] = B[i]; p.C[i] = C[i]; p.bias[i] = bias ? bias[i] : nullptr;
+  }
+  return v.launch(p, stream);
+}
+
+// whether the rows of A are whole 16-byte chunks by K alone
+static bool chunked_by_k(const Problem& q) { return q.K % (q.dtype == CASCMM_DT_F32 ? 4 : 8) == 0; }
+
+// the kernel for a shape whose operands lie well (what the selection functions of the ABI answer: the launch may copy
+// rows first and then take another)
+static int select_for_shape(Problem q, int count) {
+  q.chunked = q.K % 8 == 0;
+  return select_variant(q, row_fit(q, nullptr, nullptr), count);
+}
+
+// One launch for `count` problems of one shape (count == 1: a plain GEMM), behind a copy of operands whose rows need one.
 // exps_dyn (fp8-rate kernel only, count == 1): the launch finds the left operand's scale exponent
 // itself and leaves {e_A, *b_exp_src} there; CASCMM_ERR_BAD_VARIANT when another kernel is selected.
 static int gemm_impl(int count, const void* const* A, const void* const* B, void* const* C, const void* const* bias,
-                     const Problem& q, const int32_t* tensor_exps, void* workspace, size_t workspace_bytes,
+                     const Problem& q0, const int32_t* tensor_exps, void* workspace, size_t workspace_bytes,
                      hipStream_t stream, int variant, int32_t* exps_dyn = nullptr, const int32_t* b_exp_src = nullptr) {
+  Problem q = q0;
   int st = check_problem(q);
   if (st != CASCMM_OK) return st;
   if (count < 1 || count > kMaxGroup) return CASCMM_ERR_BAD_SHAPE;
@@ -615,98 +800,49 @@ static int gemm_impl(int count, const void* const* A, const void* const* B, void
     }
     return err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
   }
-  if (onthefly_prepare_ok(q, count, A, B, workspace, workspace_bytes)) {
-    // fp16 x fp16 (bf16 x bf16) tensors as one term: re-lay B as operand slots in the workspace
-    // (one pass over B), then the copy-only kernels
-    const size_t each = (size_t)prepared_bytes(q.K, q.N, q.fmt, 1);
-    const void* bp[kMaxGroup];
-    for (int i = 0; i < count; ++i) {
-      void* dst = (char*)workspace + (size_t)i * each;
-      bp[i] = dst;
-      int same = -1;   // the same weight twice in one group is prepared once
-      for (int j = 0; j < i && same < 0; ++j)
-        if (B[j] == B[i]) same = j;
-      if (same >= 0) {
-        bp[i] = bp[same];
-        continue;
-      }
-      st = cascmm_prepare_weight(B[i], q.K, q.N, q.ldb, q.dtype, q.fmt, 1, nullptr, dst, each, (void*)stream);
-      if (st != CASCMM_OK) return st;
-    }
-    Problem qp = q;
-    qp.bpre = true;
-    qp.ldb = q.N;
-    const int r = gemm_impl(count, A, bp, C, bias, qp, tensor_exps, nullptr, 0, stream, variant < 0 ? -1 : variant);
-    if (r != CASCMM_ERR_BAD_FORMAT && r != CASCMM_ERR_BAD_VARIANT) return r;
-  }
-  bool fast = true;
-  for (int i = 0; i < count; ++i) {
-    if (!A[i] || !B[i]) return CASCMM_ERR_NULL_POINTER;
-    if (!aligned_to(A[i], es) || !aligned_to(B[i], q.bpre ? 16 : es)) return CASCMM_ERR_ALIGNMENT;
-    fast = fast && fast_ok(q, A[i], q.bpre ? nullptr : B[i]);
-  }
-  if (q.bpre) {
-    // prepared weights only have the fast kernels: fp32 A with 16-byte aligned rows, K a multiple
-    // of the kernel's K step (checked per variant), and a buffer the 32-bit offsets can span
-    if (!fast) return CASCMM_ERR_ALIGNMENT;
-    if (prepared_bytes(q.K, q.N, q.fmt, q.terms, q.glu) > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
-  }
-
-  const auto& t = table();
-  int splits = 1;
+  q.chunked = chunked_by_k(q);
   if (variant < 0) {
-    variant = select_variant(q, fast, count, workspace ? workspace_bytes : 0, &splits);
-    if (variant < 0 && count > 1) {
-      // no kernel takes these problems in one launch (the fp8-rate kernel runs one at a time): one
-      // launch each, in order on the stream, sharing the workspace
+    const Relay r = relay_of(q, count, A, B);
+    if ((r.a || r.b) && workspace && aligned_to(workspace, 16) && workspace_bytes >= relay_bytes(r, count)) {
+      const void* ap[kMaxGroup];
+      const void* bp[kMaxGroup];
+      char* ws = (char*)workspace;
       for (int i = 0; i < count; ++i) {
-        const void* bi = bias ? bias[i] : nullptr;
-        const int st1 = gemm_impl(1, A + i, B + i, C + i, bias ? &bi : nullptr, q, tensor_exps ? tensor_exps + 2 * i : nullptr,
-                                  workspace, workspace_bytes, stream, -1);
-        if (st1 != CASCMM_OK) return st1;
+        if (!A[i] || !B[i]) return CASCMM_ERR_NULL_POINTER;
+        if (!aligned_to(A[i], es) || !aligned_to(B[i], es)) return CASCMM_ERR_ALIGNMENT;
+        // (the same operand twice in one group is copied once)
+        bool copy_a = r.a, copy_b = r.b;
+        ap[i] = A[i];
+        bp[i] = B[i];
+        for (int j = 0; j < i; ++j) {
+          if (copy_a && A[j] == A[i]) { ap[i] = ap[j]; copy_a = false; }
+          if (copy_b && B[j] == B[i]) { bp[i] = bp[j]; copy_b = false; }
+        }
+        if (copy_a) { ap[i] = ws; ws += r.a_bytes; }
+        if (copy_b) { bp[i] = ws; ws += r.b_bytes; }
+        const unsigned a_blocks = copy_a ? (unsigned)((q.M * r.a_chunks + 255) / 256) : 0;
+        const unsigned b_blocks = copy_b ? (unsigned)((prepared_kgroups(q.K) * q.N + 255) / 256) : 0;
+        if (a_blocks + b_blocks == 0) continue;
+        hipError_t err = hipSuccess;
+        if (q.dtype == CASCMM_DT_F32)
+          CASCMM_LAUNCH(err, (relay_kernel<unsigned>), dim3(a_blocks), dim3(256), 0, stream, (const unsigned*)A[i], (int)q.M, (int)q.K, q.lda, r.a_chunks,
+                        (u32x4*)ap[i], (int)a_blocks, (const unsigned*)nullptr, 0, (int64_t)0, (u32x4*)nullptr);
+        else
+          CASCMM_LAUNCH(err, (relay_kernel<unsigned short>), dim3(a_blocks + b_blocks), dim3(256), 0, stream, (const unsigned short*)A[i], (int)q.M,
+                        (int)q.K, q.lda, r.a_chunks, (u32x4*)ap[i], (int)a_blocks, (const unsigned short*)B[i], (int)q.N, q.ldb, (u32x4*)bp[i]);
+        if (err != hipSuccess) return CASCMM_ERR_LAUNCH;
       }
-      return CASCMM_OK;
+      A = ap;
+      B = bp;
+      if (r.a) q.lda = r.a_chunks * (16 / (int64_t)es);
+      q.chunked = true;
+      q.bpre = r.b;
+      if (r.b) q.ldb = q.N;
+      // (the kernels behind a copy need no workspace of their own)
+      return gemm_on_rows(count, A, B, C, bias, q, tensor_exps, nullptr, 0, stream, -1);
     }
-    if (variant < 0) return variant;
-  } else {
-    splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
-    variant &= 0xFFFF;
-    if (splits > kMaxTileSplits) return CASCMM_ERR_BAD_VARIANT;
-    if (variant >= (int)t.size()) return CASCMM_ERR_BAD_VARIANT;
-    if (!variant_matches(t[variant], q, fast)) return CASCMM_ERR_BAD_VARIANT;
   }
-  const VariantDesc& v = t[variant];
-  if (exps_dyn && (v.kind != KIND_F8K64 || count != 1)) return CASCMM_ERR_BAD_VARIANT;
-  if (count > 1 && !v.grouped) {
-    // a forced kernel that runs one problem per launch: one launch each, in order on the stream
-    if (v.kind == KIND_SPLITK) return CASCMM_ERR_BAD_VARIANT;
-    for (int i = 0; i < count; ++i) {
-      const void* bi = bias ? bias[i] : nullptr;
-      const int st1 = gemm_impl(1, A + i, B + i, C + i, bias ? &bi : nullptr, q, tensor_exps ? tensor_exps + 2 * i : nullptr,
-                                workspace, workspace_bytes, stream, variant | (splits > 1 ? splits << 16 : 0));
-      if (st1 != CASCMM_OK) return st1;
-    }
-    return CASCMM_OK;
-  }
-  GroupParams p;
-  memset(&p, 0, sizeof(p));
-  p.M = (int)q.M; p.N = (int)q.N; p.K = (int)q.K;
-  p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc;
-  const int64_t tm = (q.M + v.BM - 1) / v.BM, tn = (q.N + v.BN - 1) / v.BN;
-  if (tm * tn * count > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
-  p.tiles_m = (int)tm; p.tiles_n = (int)tn;
-  p.count = count;
-  p.workspace = workspace;
-  p.workspace_bytes = workspace_bytes;
-  p.k_splits = v.kind == KIND_TILE ? splits : 1;
-  p.tensor_exps = q.fmt == CASCMM_FMT_FP8 ? tensor_exps : nullptr;
-  p.glu = q.glu_slots ? 2 : (q.glu ? 1 : 0);
-  p.exps_dyn = exps_dyn;
-  p.b_exp_src = b_exp_src;
-  for (int i = 0; i < count; ++i) {
-    p.A[i] = A[i]; p.B[i] = B[i]; p.C[i] = C[i]; p.bias[i] = bias ? bias[i] : nullptr;
-  }
-  return v.launch(p, stream);
+  return gemm_on_rows(count, A, B, C, bias, q, tensor_exps, workspace, workspace_bytes, stream, variant, exps_dyn, b_exp_src);
 }
 
 }  // namespace cascmm
@@ -744,7 +880,7 @@ int cascmm_init(void) {
 int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K,
                         int64_t lda, int64_t ldb, int64_t ldc, int dtype, int fmt, int terms, int products,
                         const int32_t* tensor_exps, void* stream) {
-  const Problem q{M, N, K, lda, ldb, ldc, dtype, fmt, terms, products};
+  Problem q{M, N, K, lda, ldb, ldc, dtype, fmt, terms, products};
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
   if (M == 0 || N == 0 || K == 0) return cascmm_gemm(A, B, C, bias, M, N, K, lda, ldb, ldc, dtype, fmt, terms, products,
@@ -753,23 +889,32 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
   size_t need = 0;
   const void* const a1[1] = {A};
   const void* const b1[1] = {B};
-  if (onthefly_prepare_ok(q, 1, a1, b1, (void*)16, (size_t)-1)) {
-    need = (size_t)prepared_bytes(K, N, fmt, 1);            // 16-bit tensors: B re-laid as operand slots
+  const Relay relay = relay_of(q, 1, a1, b1);
+  if (relay.a || relay.b) {
+    need = relay_bytes(relay, 1);
+    if (need > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) need = 0;   // (the bounds-checked kernels need no copy)
   } else if (A && B) {
+    const RowFit fit = row_fit(q, A, B);
+    q.chunked = chunked_by_k(q);
+    Problem e;
     int splits = 1;
-    int v = select_variant(q, fast_ok(q, A, B), 1, (size_t)-1, &splits);
+    int v = select_rounded_up(q, fit, (size_t)CASCMM_NOALLOC_SCRATCH_BYTES, &e);
+    if (v < 0) {
+      e = q;
+      v = select_variant(q, fit, 1, (size_t)-1, &splits);
+    }
     if (v < 0) return v;
-    if ((table()[v].kind == KIND_F8K64 && f8k64_workspace_bytes(M, N, K, false, table()[v].BM) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) ||
-        (table()[v].kind == KIND_F16K && f16k_workspace_bytes(M, N, K) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES)) {
+    if ((table()[v].kind == KIND_F8K64 && f8k64_workspace_bytes(M, N, e.K, false, table()[v].BM) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) ||
+        (table()[v].kind == KIND_F16K && f16k_workspace_bytes(M, N, e.K) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES)) {
       // the fp8-rate kernel is a choice, not a need: without room for its operand slots the choice is
       // made among the kernels that split inside the GEMM
-      v = select_variant(q, fast_ok(q, A, B), 1, (size_t)CASCMM_NOALLOC_SCRATCH_BYTES, &splits);
+      v = select_variant(q, fit, 1, (size_t)CASCMM_NOALLOC_SCRATCH_BYTES, &splits);
       if (v < 0) return v;
     }
     const VariantDesc& d = table()[v];
     if (d.kind == KIND_SPLITK) need = skinny_workspace_bytes(M, N, K, d.BM, d.BN, d.BK);
-    else if (d.kind == KIND_F8K64) need = f8k64_workspace_bytes(M, N, K, false, d.BM);
-    else if (d.kind == KIND_F16K) need = f16k_workspace_bytes(M, N, K);
+    else if (d.kind == KIND_F8K64) need = f8k64_workspace_bytes(M, N, e.K, false, d.BM);
+    else if (d.kind == KIND_F16K) need = f16k_workspace_bytes(M, N, e.K);
     else if (splits > 1) need = (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
   }
   if (need > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) return CASCMM_ERR_SCRATCH_LIMIT;
@@ -807,8 +952,9 @@ int cascmm_select_variant_glu(int64_t M, int64_t N, int64_t K, int64_t lda, int6
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
   if (N % 64 != 0 || K == 0) return CASCMM_ERR_BAD_SHAPE;
-  const bool fast = fast_ok(q, nullptr, nullptr);
-  const int v = select_variant(q, fast, 1);
+  q.chunked = chunked_by_k(q);
+  const RowFit fit = row_fit(q, nullptr, nullptr);
+  const int v = select_variant(q, fit, 1);
   if (v < 0) return v;
   // worth it?  The alternative is the best plain kernel for the product plus the caller's gate, which
   // reads M x N values and writes half as many (measured at about 3.5 TB/s, two launches); the kernel
@@ -816,7 +962,7 @@ int cascmm_select_variant_glu(int64_t M, int64_t N, int64_t K, int64_t lda, int6
   Problem plain = q;
   plain.glu = false;
   plain.ldc = N;
-  const int vp = select_variant(plain, fast, 1);
+  const int vp = select_variant(plain, fit, 1);
   if (vp >= 0) {
     const double gate_us = 2.0 + (double)M * (double)N * 6.0 / 3.5e6;
     if (variant_cost(v, q, 1) > variant_cost(vp, plain, 1) + gate_us) return CASCMM_ERR_BAD_FORMAT;
@@ -861,7 +1007,7 @@ static int prepare_weight_impl(const void* B, int64_t K, int64_t N, int64_t ldb,
     if (dtype != CASCMM_DT_F32) return CASCMM_ERR_BAD_DTYPE;
     const int64_t units = (K >> 4) * N;
     return launch_kernel(f8k64_split_cols_kernel<0>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, (const float*)B, (int)K,
-                         (int)N, ldb, tensor_exp, (u32x4*)out) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
+                         (int)K, (int)N, ldb, tensor_exp, (u32x4*)out) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
   }
   if (dtype == CASCMM_DT_F32) return launch_prepare_fmt<CASCMM_DT_F32>(B, (int)K, (int)N, ldb, fmt, terms, tensor_exp, (u32x4*)out, s, glu);
   if (dtype == CASCMM_DT_F16) return launch_prepare_fmt<CASCMM_DT_F16>(B, (int)K, (int)N, ldb, fmt, terms, tensor_exp, (u32x4*)out, s, glu);
@@ -907,43 +1053,37 @@ int cascmm_select_variant_prepared(int count, int64_t M, int64_t N, int64_t K, i
   q.bpre = true;
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
-  return select_variant(q, fast_ok(q, nullptr, nullptr), count);
+  return select_for_shape(q, count);
 }
 
 size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fmt, int terms, int products) {
   // upper bound over the skinny variants that could be selected for this problem (the
   // selection also depends on pointer alignment, which is not known here)
-  const Problem q{M, N, K, K, N, N, dtype, fmt, terms, products};
+  Problem q{M, N, K, K, N, N, dtype, fmt, terms, products};
   if (check_problem(q) != CASCMM_OK) return 0;
-  size_t need = 0;
+  q.chunked = chunked_by_k(q);
+  const RowFit fit = row_fit(q, nullptr, nullptr);
+  // rows of A (and, 16-bit, all of B) copied first
+  const Relay relay = relay_of(q, 1, nullptr, nullptr);
+  size_t need = relay_bytes(relay, 1);
   for (const auto& v : table()) {
-    if (v.kind != KIND_SPLITK || !variant_matches(v, q, fast_ok(q, nullptr, nullptr))) continue;
+    if (v.kind != KIND_SPLITK || !variant_matches(v, q, fit)) continue;
     const size_t n = skinny_workspace_bytes(M, N, K, v.BM, v.BN, v.BK);
     need = n > need ? n : need;
   }
-  // three fp8 terms on the fp8-rate kernel: the operand slots of A and B
+  // three fp8 terms on the fp8-rate kernel, three fp16 terms on operand slots: the slots of A and B
+  const Problem e = rounded_up(q, fit);
   for (const auto& v : table()) {
-    if (v.kind != KIND_F8K64 || v.bpre || !variant_matches(v, q, fast_ok(q, nullptr, nullptr))) continue;
-    const size_t n = f8k64_workspace_bytes(M, N, K, false, v.BM);
+    if ((v.kind != KIND_F8K64 && v.kind != KIND_F16K) || v.bpre || !variant_matches(v, e, e.split_first ? FIT_FAST : fit)) continue;
+    const size_t n = v.kind == KIND_F8K64 ? f8k64_workspace_bytes(M, N, e.K, false, v.BM) : f16k_workspace_bytes(M, N, e.K);
     need = n > need ? n : need;
-  }
-  // three fp16 terms on operand slots: the slots of A and B
-  for (const auto& v : table()) {
-    if (v.kind != KIND_F16K || !variant_matches(v, q, fast_ok(q, nullptr, nullptr))) continue;
-    const size_t n = f16k_workspace_bytes(M, N, K);
-    need = n > need ? n : need;
-  }
-  // 16-bit tensors as one term of their own format: room for B re-laid as operand slots
-  if (own_format16(q) && K % 8 == 0) {
-    const int64_t n = prepared_bytes(K, N, fmt, 1);
-    if (n <= INT32_MAX && (size_t)n > need) need = (size_t)n;
   }
   // K split of the LDS-tiled kernels: up to kMaxTileSplits partial results when some kernel
   // would run the problem with at most half the CUs busy
   if (dtype == CASCMM_DT_F32 && N % 4 == 0) {
     for (int vi = 0; vi < (int)table().size(); ++vi) {
       const VariantDesc& v = table()[vi];
-      if (v.kind != KIND_TILE || !variant_matches(v, q, fast_ok(q, nullptr, nullptr))) continue;
+      if (v.kind != KIND_TILE || !variant_matches(v, q, fit)) continue;
       int sp = 1;
       variant_cost(vi, q, 1, (size_t)-1, &sp);
       const size_t n = sp > 1 ? (size_t)kMaxTileSplits * M * N * sizeof(float) : 0;
@@ -958,7 +1098,7 @@ int cascmm_select_variant(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t 
   const Problem q{M, N, K, lda, ldb, ldc, dtype, fmt, terms, products};
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
-  return select_variant(q, fast_ok(q, nullptr, nullptr), 1);
+  return select_for_shape(q, 1);
 }
 
 int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -967,7 +1107,7 @@ int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, in
   const Problem q{M, N, K, lda, ldb, ldc, dtype, fmt, terms, products};
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
-  return select_variant(q, fast_ok(q, nullptr, nullptr), count);
+  return select_for_shape(q, count);
 }
 
 int cascmm_variant_count(void) { return (int)table().size(); }
@@ -1049,11 +1189,17 @@ int cascmm_gemm_fp8_autoscale(const void* A, const void* B, int b_prepared, void
   const void* bias1 = bias;
   if (M > 0 && N > 0 && K > 0 && A && B) {
     // the fp8-rate kernel splits A in a pass of its own anyway: the search rides on it
-    const bool fast = fast_ok(q, A, q.bpre ? nullptr : B);
-    if (!q.bpre || fast) {
-      const int v = select_variant(q, fast, 1, workspace ? workspace_bytes : 0);
+    const RowFit fit = row_fit(q, A, q.bpre ? nullptr : B);
+    if (!q.bpre || fit == FIT_FAST) {
+      const size_t room = workspace ? workspace_bytes : 0;
+      Problem e;
+      int v = q.bpre ? (int)CASCMM_ERR_BAD_FORMAT : select_rounded_up(q, fit, room, &e);
+      if (v < 0) {
+        e = q;
+        v = select_variant(q, fit, 1, room);
+      }
       if (v >= 0 && table()[v].kind == KIND_F8K64)
-        return gemm_impl(1, &A, &B, &C, bias ? &bias1 : nullptr, q, nullptr, workspace, workspace_bytes, (hipStream_t)stream, v,
+        return gemm_impl(1, &A, &B, &C, bias ? &bias1 : nullptr, e, nullptr, workspace, workspace_bytes, (hipStream_t)stream, v,
                          exps_out, b_exp);
     }
   }

@@ -366,6 +366,9 @@ struct GroupParams {
   // host side only: when set, the variant's launch function stores the handle of its GEMM kernel here
   // and returns without checking or launching anything (the library names its kernels this way)
   const void** kernel_out;
+  // kernels that split their operands into slots first (three fp8 / fp16 terms): K is rounded up to whole stages, the
+  // operands hold k_valid of it and the slots beyond are zeros
+  int k_valid;
 };
 
 }  // namespace cascmm

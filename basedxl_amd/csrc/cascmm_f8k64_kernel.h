@@ -65,6 +65,34 @@ inline __host__ __device__ int64_t f8k64_slot_bytes(int64_t rows, int64_t K) {
   return bytes;
 }
 
+// eight consecutive elements of a row, `left` of which exist (the others are zeros); vec: 16-byte aligned
+__device__ __forceinline__ void load_row8(const float* __restrict__ src, int left, int vec, float (&r)[8]) {
+  if (vec && left >= 8) {
+    const f32x4 v0 = *(const f32x4*)src, v1 = *(const f32x4*)(src + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[e] = v0[e];
+      r[4 + e] = v1[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = e < left ? src[e] : 0.f;
+  }
+}
+
+// KN consecutive elements of a column, `left` of which exist (one test for all of them: a test per element would put
+// the loads one behind the other)
+template <int KN>
+__device__ __forceinline__ void load_column(const float* __restrict__ src, int64_t ld, int left, float (&x)[KN]) {
+  if (left >= KN) {
+#pragma unroll
+    for (int e = 0; e < KN; ++e) x[e] = src[(int64_t)e * ld];
+  } else {
+#pragma unroll
+    for (int e = 0; e < KN; ++e) x[e] = e < left ? src[(int64_t)e * ld] : 0.f;
+  }
+}
+
 // max|a| of this workgroup's share of A [M, K] (bit pattern) -> amax_out[blockIdx.x]; no atomics, no
 // meeting point: the kernel that splits A reduces the gridDim.x values.
 template <int UNUSED>
@@ -87,8 +115,9 @@ __global__ __launch_bounds__(1024) void f8k64_amax_kernel(const float* __restric
 // are the per-workgroup maxima |a| (bit patterns) of a preceding f8k64_amax_kernel; every workgroup
 // reduces them itself (1 KB from L2, behind its loads of A), and the first one leaves {e_A, *b_exp}
 // in exps_out for the GEMM.
+// k_valid <= K: the depth of A; slots beyond it are zeros.  vec: rows of A start on 16-byte boundaries.
 template <int UNUSED>
-__global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __restrict__ A, int M, int K, int64_t lda,
+__global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __restrict__ A, int M, int K, int k_valid, int vec, int64_t lda,
                                                               const int32_t* __restrict__ tensor_exp, u32x4* __restrict__ out,
                                                               const unsigned* __restrict__ amax, int n_amax,
                                                               const int32_t* __restrict__ b_exp, int32_t* __restrict__ exps_out) {
@@ -124,8 +153,10 @@ __global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __re
       u32x4 t[3];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const f32x4 v0 = *(const f32x4*)(src + 8 * h), v1 = *(const f32x4*)(src + 8 * h + 4);
-        float r[8] = {v0[0] * scale, v0[1] * scale, v0[2] * scale, v0[3] * scale, v1[0] * scale, v1[1] * scale, v1[2] * scale, v1[3] * scale};
+        float r[8];
+        load_row8(src + 8 * h, k_valid - (ku0 + ku) * 16 - 8 * h, vec, r);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] *= scale;
         const u32x2 t0 = Lowp<CASCMM_FMT_FP8>::peel<false>(r);
         const u32x2 t1 = Lowp<CASCMM_FMT_FP8>::peel<false>(r);
         const u32x2 t2 = Lowp<CASCMM_FMT_FP8>::peel<true>(r);
@@ -149,7 +180,7 @@ __global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __re
 // Split of the RIGHT operand: B [K, N] fp32 row-major -> slots[term][K/16][N]; thread (ku, n) walks
 // 16 rows of column n (consecutive threads: consecutive columns, coalesced both ways).
 template <int UNUSED>
-__global__ __launch_bounds__(256) void f8k64_split_cols_kernel(const float* __restrict__ B, int K, int N, int64_t ldb,
+__global__ __launch_bounds__(256) void f8k64_split_cols_kernel(const float* __restrict__ B, int K, int k_valid, int N, int64_t ldb,
                                                               const int32_t* __restrict__ tensor_exp, u32x4* __restrict__ out) {
   const int kus = K >> 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -157,12 +188,14 @@ __global__ __launch_bounds__(256) void f8k64_split_cols_kernel(const float* __re
   const int ku = (int)(i / N), n = (int)(i - (int64_t)ku * N);
   const float scale = tensor_exp ? __builtin_ldexpf(1.f, *tensor_exp) : 1.f;
   const float* src = B + (int64_t)ku * 16 * ldb + n;
+  float x[16];
+  load_column<16>(src, ldb, k_valid - ku * 16, x);
   u32x4 t[3];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     float r[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = src[(int64_t)(8 * h + e) * ldb] * scale;
+    for (int e = 0; e < 8; ++e) r[e] = x[8 * h + e] * scale;
     const u32x2 t0 = Lowp<CASCMM_FMT_FP8>::peel<false>(r);
     const u32x2 t1 = Lowp<CASCMM_FMT_FP8>::peel<false>(r);
     const u32x2 t2 = Lowp<CASCMM_FMT_FP8>::peel<true>(r);

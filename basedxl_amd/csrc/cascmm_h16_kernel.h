@@ -76,9 +76,9 @@ template <int FMT> struct H16Elem;
 template <> struct H16Elem<CASCMM_FMT_BF16> { typedef __bf16 T; static constexpr int DT = CASCMM_DT_BF16; };
 template <> struct H16Elem<CASCMM_FMT_FP16> { typedef _Float16 T; static constexpr int DT = CASCMM_DT_F16; };
 
-// Host-checked: K % 8 == 0, lda % 8 == 0, A 16-byte aligned, M * lda * 2 below 2 GiB; RAWB = 0: B prepared
-// ([ceil(K / 64) * 8][N] slots, zeros beyond K) below 2 GiB; RAWB = 1: B [K][ldb] with N % 8 == 0, ldb % 8 == 0,
-// 16-byte aligned, K * ldb * 2 below 2 GiB.  Any M and N: rows and columns past the edge are loaded as zeros or as
+// Host-checked: the rows of A start on dwords and are whole 16-byte chunks, zeros past K (K % 8 == 0, or padded), M * lda * 2
+// below 2 GiB; RAWB = 0: B prepared ([ceil(K / 64) * 8][N] slots, zeros beyond K) below 2 GiB; RAWB = 1: B [K][ldb] with
+// N % 2 == 0 and rows on dwords, K * ldb * 2 below 2 GiB.  Any M and N: rows and columns past the edge are loaded as zeros or as
 // some other column's values and not stored.  grid.y: the problem of a group.
 // GLU: gated store (see GroupParams; RAWB = 0, NTL even: a wave owns whole value / gate pairs of blocks).
 template <class T, int FMT, int RAWB, int GLU>
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 
   // rows past M read as zero (the buffer ends with row M - 1), and so does everything past B's last row or slot row
   const int kgs = (p.K + 63) / 64 * 8;
-  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + p.K) * 2;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + (p.K + 7) / 8 * 8) * 2;
   const int64_t b_bytes = RAWB ? ((int64_t)(p.K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[prob], 0, (int)b_bytes, 0x00020000);

@@ -34,12 +34,12 @@ int launch_prepare_left(const float* A, int M, int K, int64_t lda, void* out, hi
              : CASCMM_ERR_LAUNCH;
 }
 
-const void* slotk_kernel_handle(int araw) { return araw ? (const void*)cascmm_slotk_kernel<1> : (const void*)cascmm_slotk_kernel<0>; }
+const void* slotk_kernel_handle(int araw) { return araw ? (const void*)cascmm_slotk_kernel<1, 0> : (const void*)cascmm_slotk_kernel<0, 0>; }
 
-template <int ARAW>
+template <int ARAW, int TAIL>
 static int launch_slotk_t(const SlotKParams& q, hipStream_t stream) {
   typedef SlotK T;
-  auto kfn = cascmm_slotk_kernel<ARAW>;
+  auto kfn = cascmm_slotk_kernel<ARAW, TAIL>;
   static LdsFlags lds_set;
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
   SlotKParams p = q;
@@ -53,34 +53,34 @@ static int launch_slotk_t(const SlotKParams& q, hipStream_t stream) {
 }
 
 int launch_slotk(const SlotKParams& q, int araw, hipStream_t stream) {
-  return araw ? launch_slotk_t<1>(q, stream) : launch_slotk_t<0>(q, stream);
+  return araw ? launch_slotk_t<1, 0>(q, stream) : launch_slotk_t<0, 0>(q, stream);
 }
 
 // the variant-table face of the kernel: raw fp32 left operand, prepared right operand
 static int launch_slotk_variant(const GroupParams& p, hipStream_t stream) {
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_slotk_kernel<1>; return CASCMM_OK; }
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_slotk_kernel<1, 0>; return CASCMM_OK; }
   if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
-  if (p.K % (2 * SlotK::BK) != 0 || p.K < 2 * SlotK::BK) return CASCMM_ERR_BAD_VARIANT;   // raw A comes in pairs of stages
-  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.N * 4 > 0x7FFFFFFF || p.ldc * (int64_t)(SlotK::BM * 4) > 0x7FFFFFFF)
+  if (p.lda < 2 * SlotK::BK) return CASCMM_ERR_BAD_VARIANT;
+  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || prepared_kgroups(p.K) * p.N * 32 > 0x7FFFFFFF || p.ldc * (int64_t)(SlotK::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   SlotKParams q;
   memset(&q, 0, sizeof(q));
   q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
   q.M = p.M; q.N = p.N; q.K = p.K; q.lda = p.lda; q.ldc = p.ldc;
-  return launch_slotk_t<1>(q, stream);
+  // (raw A comes in pairs of 16-k stages)
+  return p.K % (2 * SlotK::BK) == 0 ? launch_slotk_t<1, 0>(q, stream) : launch_slotk_t<1, 1>(q, stream);
 }
 
 // the 64 x 80 tile of the same design, for problems that make too few 64 x 160 tiles to occupy the chip
 static int launch_slotn_variant(const GroupParams& p, hipStream_t stream) {
   typedef SlotN T;
-  auto kfn = cascmm_slotn_kernel<0>;
+  auto kfn = p.K % T::BK == 0 ? cascmm_slotn_kernel<0> : cascmm_slotn_kernel<1>;
   if (p.kernel_out) { *p.kernel_out = (const void*)kfn; return CASCMM_OK; }
   if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
-  if (p.K % T::BK != 0 || p.K < T::BK) return CASCMM_ERR_BAD_VARIANT;
-  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.N * 4 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
+  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || prepared_kgroups(p.K) * p.N * 32 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
-  static LdsFlags lds_set;
-  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
+  static LdsFlags lds_set[2];
+  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[p.K % T::BK == 0 ? 0 : 1])) return CASCMM_ERR_LAUNCH;
   SlotKParams q;
   memset(&q, 0, sizeof(q));
   q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
@@ -97,14 +97,15 @@ static int launch_slotn_variant(const GroupParams& p, hipStream_t stream) {
 // both operands raw fp32
 static int launch_rawk_variant(const GroupParams& p, hipStream_t stream) {
   typedef SlotK T;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_rawk_kernel; return CASCMM_OK; }
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_rawk_kernel<0>; return CASCMM_OK; }
   if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
-  if (p.K % (2 * T::BK) != 0 || p.K < 2 * T::BK || p.N % 4 != 0) return CASCMM_ERR_BAD_VARIANT;   // raw A comes in pairs of stages
+  if (p.lda < 2 * T::BK) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
-  auto kfn = cascmm_rawk_kernel;
-  static LdsFlags lds_set;
-  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
+  const bool tail = p.K % (2 * T::BK) != 0;   // raw A comes in pairs of stages
+  auto kfn = tail ? cascmm_rawk_kernel<1> : cascmm_rawk_kernel<0>;
+  static LdsFlags lds_set[2];
+  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[tail ? 1 : 0])) return CASCMM_ERR_LAUNCH;
   SlotKParams q;
   memset(&q, 0, sizeof(q));
   q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
@@ -114,7 +115,7 @@ static int launch_rawk_variant(const GroupParams& p, hipStream_t stream) {
   q.group_m = SlotK::GROUP_M;
   const int64_t grid = (int64_t)q.tiles_m * q.tiles_n;
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  const int c_vec = p.ldc % 4 == 0 && (uintptr_t)p.C[0] % 16 == 0;
+  const int c_vec = p.N % 4 == 0 && p.ldc % 4 == 0 && (uintptr_t)p.C[0] % 16 == 0;
   return launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q, c_vec) == hipSuccess ? CASCMM_OK
                                                                                                                      : CASCMM_ERR_LAUNCH;
 }

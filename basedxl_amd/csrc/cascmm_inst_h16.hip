@@ -18,8 +18,8 @@ static int launch_h16_kernel(const GroupParams& p, hipStream_t stream) {
 template <class T, int FMT, int RAWB, int GLU>
 static int launch_h16(const GroupParams& p, hipStream_t stream) {
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_h16_kernel<T, FMT, RAWB, 0>; return CASCMM_OK; }
-  if (p.count < 1 || p.k_splits > 1 || p.K % 8 != 0 || p.lda % 8 != 0 || (p.glu && !GLU)) return CASCMM_ERR_BAD_VARIANT;
-  if (RAWB && (p.N % 8 != 0 || p.ldb % 8 != 0)) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count < 1 || p.k_splits > 1 || p.lda % 2 != 0 || (p.glu && !GLU)) return CASCMM_ERR_BAD_VARIANT;
+  if (RAWB && (p.N % 2 != 0 || p.ldb % 2 != 0)) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 2 > 0x7FFFFFFF || (RAWB ? ((int64_t)p.K + 64) * p.ldb * 2 : prepared_kgroups(p.K) * p.N * 16) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   if constexpr (GLU) {

@@ -32,10 +32,11 @@
 
 namespace cascmm {
 
-// Host-checked: K % 16 == 0, K >= 16 (raw A: K % 32 == 0), the slot buffers 16-byte aligned and below 2 GiB,
-// raw A 16-byte aligned with lda % 4 == 0 and M * lda * 4 below 2 GiB, C rows addressable with 32-bit
-// byte offsets inside a tile.
-template <int ARAW>
+// Host-checked: the slot buffers 16-byte aligned and below 2 GiB, raw A: lda >= 32, M * lda * 4 below 2 GiB (rows need
+// no alignment: see cascmm_wavek_kernel), C rows addressable with 32-bit byte offsets inside a tile.  TAIL = 0:
+// K % 16 == 0, K >= 16 (raw A: K % 32 == 0).  TAIL = 1 (raw A only): any K whose rows of A are whole 16-byte chunks,
+// zeros past K; the chunks past K are fetched from beyond the buffer, as zeros (the slots of B past K are zeros).
+template <int ARAW, int TAIL>
 __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_slotk_kernel(const SlotKParams p) {
   typedef SlotK T;
   extern __shared__ __attribute__((aligned(1024))) unsigned char slotk_smem[];
@@ -48,7 +49,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int kgroups = ARAW ? (int)prepared_kgroups(p.K) : p.K >> 3;   // (slots x slots: both buffers end with K)
-  const int ksteps = p.K >> 4;
+  const int ksteps = TAIL ? (p.K + 31) / 32 * 2 : p.K >> 4;
   // Which 16-k stages of the problem a wave owns.  A as slots: every fourth one, own stage i = stage
   // wave + 4 i.  A raw: every fourth PAIR of stages, own stage i = stage 8 (i / 2) + 2 wave + i % 2, so that
   // what the wave fetches of a row for a pair is one whole 128-byte line (with every fourth stage it was half
@@ -96,11 +97,13 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   // A pair of stages in LDS: 64 rows x 128 bytes (eight 16-byte chunks of 4 k).  Load j of a pair (0 .. 7)
   // brings rows 8 j + lane / 8; position pos of a row holds chunk (pos - row / 2) mod 8, which spreads the
   // fragment reads of 16 consecutive rows over all banks.  (row / 2) mod 8 = (4 j + lane / 16) mod 8: two
-  // offsets per lane, by the parity of j.  K % 32 == 0 (host-checked for raw A), so a wave's pairs are whole.
-  int dma_voff[2];
+  // offsets per lane, by the parity of j.  A wave's pairs are whole: K % 32 == 0, or zeros (TAIL).
+  int dma_voff[2], dma_k[2];
 #pragma unroll
-  for (int jp = 0; jp < 2; ++jp)
-    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + (((lane & 7) - (4 * jp + (lane >> 4))) & 7) * 4) * 4);
+  for (int jp = 0; jp < 2; ++jp) {
+    dma_k[jp] = (((lane & 7) - (4 * jp + (lane >> 4))) & 7) * 4;
+    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + dma_k[jp]) * 4);
+  }
   const int dma_rows8 = (int)p.lda * 32;   // bytes from one load's rows to the next one's
   // the part ni (0 .. 3) of own stage i's share of its pair's loads: load 4 sp + ni of pair i / 2, sp = i % 2
   // (passed separately: a constant where i is not); past the wave's last pair: the problem's first pair
@@ -113,8 +116,9 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   for (int ni = 0; ni < 4; ++ni) dma_v[ni] = dma_voff[ni & 1] + ni * (dma_rows8 - 1024);
   auto dma_a = [&](int i, int ni, int sp) {
     const int q = i >> 1;
-    const int koff = (2 * q < n_own ? stage_of(2 * q) * (T::BK * 4) : 0) + 4 * sp * dma_rows8;
-    wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, dma_v[ni], koff, ni);
+    const int k0 = 2 * q < n_own ? stage_of(2 * q) * T::BK : 0;
+    const int v = !TAIL || dma_k[ni & 1] < p.K - k0 ? dma_v[ni] : 0x7FFFFFFF;
+    wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, v, k0 * 4 + 4 * sp * dma_rows8, ni);
   };
   // fragment of lane (l31, g), row block mi, stage parity s: row 32 mi + l31, chunks 4 s + 2 g and 4 s + 2 g + 1
   // at their rotated places
@@ -320,9 +324,10 @@ struct RawK {
   static constexpr int D = 4, AHEAD = 6;   // B ring in registers; raw A requested this many stages ahead (even: whole pairs)
 };
 
-// Host-checked: fp32 operands, K % 32 == 0, N % 4 == 0, lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
-// aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets inside a
-// tile.  c_vec: ldc % 4 == 0 and C 16-byte aligned (16-byte stores).
+// Host-checked: fp32 operands, lda >= 32, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte
+// offsets inside a tile; any N and any alignment of rows.  TAIL as above (0: K % 32 == 0; the rows of B past K lie
+// beyond its buffer).  c_vec: N % 4 == 0, ldc % 4 == 0 and C 16-byte aligned (16-byte stores).
+template <int TAIL>
 __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_rawk_kernel(const SlotKParams p, int c_vec) {
   typedef SlotK T;
   constexpr int D = RawK::D, AHEAD = RawK::AHEAD;
@@ -332,7 +337,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   int tm, tn;
   tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int ksteps = p.K >> 4;
+  const int ksteps = TAIL ? (p.K + 31) / 32 * 2 : p.K >> 4;
   // a wave owns every fourth PAIR of 16-k stages (see the kernel above): own stage i = stage 8 (i / 2) + 2 wave + i % 2
   const int own_tail = (ksteps & 7) - 2 * wave;
   const int n_own = 2 * (ksteps >> 3) + (own_tail < 0 ? 0 : own_tail > 2 ? 2 : own_tail);   // 0 for the last waves of a very short K: they add zeros
@@ -370,18 +375,21 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   const __amdgpu_buffer_rsrc_t rar =
       __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
   unsigned char* ring = slotk_smem + wave * T::RING;
-  int dma_voff[2];
+  int dma_voff[2], dma_k[2];
 #pragma unroll
-  for (int jp = 0; jp < 2; ++jp)
-    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + (((lane & 7) - (4 * jp + (lane >> 4))) & 7) * 4) * 4);
+  for (int jp = 0; jp < 2; ++jp) {
+    dma_k[jp] = (((lane & 7) - (4 * jp + (lane >> 4))) & 7) * 4;
+    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + dma_k[jp]) * 4);
+  }
   const int dma_rows8 = (int)p.lda * 32;
   int dma_v[4];   // (as in the kernel above: one M0 and one scalar offset for the four loads of a stage)
 #pragma unroll
   for (int ni = 0; ni < 4; ++ni) dma_v[ni] = dma_voff[ni & 1] + ni * (dma_rows8 - 1024);
   auto dma_a = [&](int i, int ni, int sp) {   // sp = i % 2
     const int q = i >> 1;
-    const int koff = (2 * q < n_own ? stage_of(2 * q) * (T::BK * 4) : 0) + 4 * sp * dma_rows8;
-    wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, dma_v[ni], koff, ni);
+    const int k0 = 2 * q < n_own ? stage_of(2 * q) * T::BK : 0;
+    const int v = !TAIL || dma_k[ni & 1] < p.K - k0 ? dma_v[ni] : 0x7FFFFFFF;
+    wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, v, k0 * 4 + 4 * sp * dma_rows8, ni);
   };
   int a_frag[2][2];
 #pragma unroll
@@ -535,12 +543,12 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
     const i32x4 rc = make_rsrc(p.C + (int64_t)m0 * p.ldc + n0, c_bytes);
     // columns past N (a ragged last tile) are sent beyond the end as well
     const int colq = 4 * l31, cols = 128 + l31;
-    const bool inq = n0 + colq < p.N, ins = n0 + cols < p.N;   // (N % 4 == 0: four adjacent columns are inside together)
+    const bool inq = n0 + colq < p.N, ins = n0 + cols < p.N;   // (c_vec: four adjacent columns are inside together)
     f32x4 bq = {0.f, 0.f, 0.f, 0.f};
     float bs = 0.f;
     if (p.bias && inq) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bq[j] = p.bias[n0 + colq + j];
+      for (int j = 0; j < 4; ++j) bq[j] = n0 + colq + j < p.N ? p.bias[n0 + colq + j] : 0.f;
     }
     if (p.bias && ins) bs = p.bias[n0 + cols];
     const int voq = inq ? (g * 4 * ldc_bytes) + colq * 4 : c_bytes;
@@ -555,7 +563,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
           llvm_raw_buffer_store_v4f32(v4, rc, voq, soff, kResultStoreAux);
         } else {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) llvm_raw_buffer_store_f32(v4[j], rc, inq ? voq + 4 * j : c_bytes, soff, kResultStoreAux);
+          for (int j = 0; j < 4; ++j) llvm_raw_buffer_store_f32(v4[j], rc, n0 + colq + j < p.N ? voq + 4 * j : c_bytes, soff, kResultStoreAux);
         }
         llvm_raw_buffer_store_f32(sum[mi][4][e] + bs, rc, vos, soff, kResultStoreAux);
       }

@@ -33,10 +33,10 @@ struct SlotN {
   static constexpr int LDS_BYTES = NW * RING > RED_BYTES ? NW * RING : RED_BYTES;   // 128 KB
 };
 
-// Host-checked: K % 32 == 0, K >= 32, the slot buffer 16-byte aligned and below 2 GiB, A 16-byte aligned with
-// lda % 4 == 0 and M * lda * 4 below 2 GiB, C rows addressable with 32-bit byte offsets inside a tile.
-// (SlotKParams: a = fp32 [M][lda], b_slots = [2][K/8][N] x 16 bytes.)
-template <int UNUSED>
+// Host-checked: the slot buffer 16-byte aligned and below 2 GiB, M * lda * 4 below 2 GiB, C rows addressable with 32-bit
+// byte offsets inside a tile.  TAIL as in cascmm_slotk_kernel (0: K % 32 == 0, K >= 32).
+// (SlotKParams: a = fp32 [M][lda], b_slots = [2][8 ceil(K/64)][N] x 16 bytes.)
+template <int TAIL>
 __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_slotn_kernel(const SlotKParams p) {
   typedef SlotN T;
   extern __shared__ __attribute__((aligned(1024))) unsigned char slotn_smem[];
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int kgroups = (int)prepared_kgroups(p.K);
-  const int ksteps = p.K >> 5;
+  const int ksteps = (p.K + 31) >> 5;
   const int n_own = (ksteps - wave + T::NW - 1) / T::NW;   // 0 for the last waves of a very short K: they add zeros
   // The loop runs in trips of two stages without a branch inside; a wave with an odd number of stages runs one
   // stage past its last: its B loads point beyond the end of the buffer and return zeros, its A loads fetch the
@@ -79,14 +79,17 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   // 5, 7) gives the row pairs 0, 1, 6, 7 the odd rotations and the pairs 2 .. 5 the even ones, so that either sixteen
   // cover every unit once (a rotation by h itself reads every fragment in eight passes instead of four: counted).
   auto rot = [](int h) { return (0x75642031u >> (4 * h)) & 7u; };
-  int dma_voff[2];
+  int dma_voff[2], dma_k[2];
 #pragma unroll
-  for (int jp = 0; jp < 2; ++jp)
-    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + (((lane & 7) - (int)rot(4 * jp + (lane >> 4))) & 7) * 4) * 4);
+  for (int jp = 0; jp < 2; ++jp) {
+    dma_k[jp] = (((lane & 7) - (int)rot(4 * jp + (lane >> 4))) & 7) * 4;
+    dma_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + dma_k[jp]) * 4);
+  }
   const int dma_rows8 = (int)p.lda * 32;
   auto dma_a = [&](int i, int j) {
-    const int koff = i < n_own ? (wave + T::NW * i) * (T::BK * 4) : 0;
-    wavek_load_lds(rar, ring + (i & (T::RA - 1)) * T::A_STAGE + j * 1024, dma_voff[j & 1], koff + j * dma_rows8);
+    const int k0 = i < n_own ? (wave + T::NW * i) * T::BK : 0;
+    const int v = !TAIL || dma_k[j & 1] < p.K - k0 ? dma_voff[j & 1] : 0x7FFFFFFF;
+    wavek_load_lds(rar, ring + (i & (T::RA - 1)) * T::A_STAGE + j * 1024, v, k0 * 4 + j * dma_rows8);
   };
   // fragment of lane (l15, kg), row block mb: row 16 mb + l15, chunks 2 kg and 2 kg + 1 at their rotated places
   int a_frag[2];

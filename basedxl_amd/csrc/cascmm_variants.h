@@ -219,16 +219,16 @@ int launch_w512(const GroupParams& p, hipStream_t stream) {
 template <int NB>
 int launch_wavek(const GroupParams& p, hipStream_t stream) {
   typedef WaveK<NB> T;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<NB>; return CASCMM_OK; }
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<NB, 0>; return CASCMM_OK; }
   if (p.glu || p.k_splits > 1 || p.count < 1) return CASCMM_ERR_BAD_VARIANT;
-  if (p.N % T::BN != 0 || p.K % T::BK != 0) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  auto kfn = cascmm_wavek_kernel<NB>;
-  static LdsFlags lds_set;
-  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
+  const bool tail = p.N % T::BN != 0 || p.K % T::BK != 0;
+  auto kfn = tail ? cascmm_wavek_kernel<NB, 1> : cascmm_wavek_kernel<NB, 0>;
+  static LdsFlags lds_set[2];
+  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[tail ? 1 : 0])) return CASCMM_ERR_LAUNCH;
   GroupParams q = p;
   q.tiles_m = (p.M + T::BM - 1) / T::BM;
-  q.tiles_n = p.N / T::BN;
+  q.tiles_n = (p.N + T::BN - 1) / T::BN;
   const int64_t grid = (int64_t)q.count * q.tiles_m * q.tiles_n;
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
   if (launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q) != hipSuccess) return CASCMM_ERR_LAUNCH;
@@ -244,7 +244,7 @@ inline double f8k64_stage_us(int bm) { return bm == 256 ? 2.1 : 1.15; }
 template <int MT> struct F8Tile { typedef F8K64T<MT> T; };
 template <> struct F8Tile<0> { typedef F8WK T; };
 inline int f8k64_splits(int64_t M, int64_t N, int64_t K, int bm) {
-  if (bm == F8WK::BM) return 1;
+  if (bm == F8WK::BM || N % 4 != 0) return 1;   // (the reduction of a split writes four columns at a time)
   const int64_t tiles = ((M + bm - 1) / bm) * ((N + F8K64::BN - 1) / F8K64::BN);
   const int64_t steps = K / F8K64::BK;
   int best = 1;
@@ -297,16 +297,17 @@ int launch_f8k64(const GroupParams& p, hipStream_t stream) {
     // the scale of A is not known yet: per-workgroup maxima now, reduced by the split of A, which
     // leaves {e_A, e_B} in exps_dyn for the GEMM (no atomics, no pass of its own for the reduction)
     unsigned* am = (unsigned*)((char*)p.workspace + need - kF8K64AmaxGroups * sizeof(unsigned));
-    const int64_t total = (int64_t)p.M * p.K;
+    const int64_t total = (int64_t)p.M * p.k_valid;
     n_amax = (int)std::max<int64_t>(1, std::min<int64_t>((total + 8191) / 8192, kF8K64AmaxGroups));
     if (launch_kernel(f8k64_amax_kernel<0>, dim3((unsigned)n_amax), dim3(1024), 0, stream, (const float*)p.A[0], (int64_t)p.M,
-                      (int64_t)p.K, p.lda, am) != hipSuccess)
+                      (int64_t)p.k_valid, p.lda, am) != hipSuccess)
       return CASCMM_ERR_LAUNCH;
     amax = am;
     exps = p.exps_dyn;
     b_exp = p.b_exp_src;
   }
-  if (launch_kernel(f8k64_split_rows_kernel<0>, dim3(a_grid), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K, p.lda,
+  const int vec = p.lda % 4 == 0 && (uintptr_t)p.A[0] % 16 == 0;
+  if (launch_kernel(f8k64_split_rows_kernel<0>, dim3(a_grid), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K, p.k_valid, vec, p.lda,
                     p.exps_dyn ? (const int32_t*)nullptr : p.tensor_exps, a_slots, amax, n_amax, b_exp, p.exps_dyn) != hipSuccess)
     return CASCMM_ERR_LAUNCH;
   if (!BPRE) {
@@ -314,7 +315,7 @@ int launch_f8k64(const GroupParams& p, hipStream_t stream) {
     ws_next += f8k64_up(f8k64_slot_bytes(p.N, p.K));
     const int64_t units = (int64_t)kus * p.N;
     if (launch_kernel(f8k64_split_cols_kernel<0>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, (const float*)p.B[0],
-                      p.K, p.N, p.ldb, b_exp, bs) != hipSuccess)
+                      p.K, p.k_valid, p.N, p.ldb, b_exp, bs) != hipSuccess)
       return CASCMM_ERR_LAUNCH;
     b_slots = bs;
   }
@@ -366,16 +367,16 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
   unsigned* amax_a = (unsigned*)ws;
   unsigned* amax_b = amax_a + kF8K64AmaxGroups;
   int32_t* exps = (int32_t*)(amax_b + kF8K64AmaxGroups);
-  const int n_a = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)p.M * p.K + 8191) / 8192, kF8K64AmaxGroups));
-  const int n_b = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)p.K * p.N + 8191) / 8192, kF8K64AmaxGroups));
+  const int n_a = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)p.M * p.k_valid + 8191) / 8192, kF8K64AmaxGroups));
+  const int n_b = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)p.k_valid * p.N + 8191) / 8192, kF8K64AmaxGroups));
   if (launch_kernel(f16k_amax_kernel<0>, dim3((unsigned)(n_a + n_b)), dim3(1024), 0, stream, (const float*)p.A[0], (int64_t)p.M,
-                    (int64_t)p.K, p.lda, n_a, (const float*)p.B[0], (int64_t)p.N, p.ldb, amax_a, amax_b) != hipSuccess)
+                    (int64_t)p.k_valid, p.lda, n_a, (const float*)p.B[0], (int64_t)p.N, p.ldb, amax_a, amax_b) != hipSuccess)
     return CASCMM_ERR_LAUNCH;
   const int kus = p.K >> 3;
   const int a_blocks = ((p.M + 63) / 64) * ((kus + 3) / 4);
   const int64_t b_blocks = ((int64_t)kus * p.N + 255) / 256;
   if (launch_kernel(f16k_split_kernel<0>, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K,
-                    p.lda, a_slots, (const unsigned*)amax_a, n_a, a_blocks, (const float*)p.B[0], p.N, p.ldb, b_slots,
+                    p.k_valid, (int)(p.lda % 4 == 0 && (uintptr_t)p.A[0] % 16 == 0), p.lda, a_slots, (const unsigned*)amax_a, n_a, a_blocks, (const float*)p.B[0], p.N, p.ldb, b_slots,
                     (const unsigned*)amax_b, n_b, exps) != hipSuccess)
     return CASCMM_ERR_LAUNCH;
   F8K64Params q;

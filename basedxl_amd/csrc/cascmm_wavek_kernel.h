@@ -53,10 +53,12 @@ __device__ __forceinline__ void wavek_load_lds_kb(__amdgpu_buffer_rsrc_t rsrc, u
   }
 }
 
-// Host-checked: fp32 operands, two bf16 terms, products hi.hi + hi.lo + lo.hi; K % 32 == 0,
-// N % (32 NB) == 0, lda % 4 == 0 and A 16-byte aligned, NB == 2: ldb % 2 == 0 and B 8-byte aligned;
-// M * lda * 4 and K * ldb * 4 below 2 GiB.
-template <int NB>
+// Host-checked: fp32 operands, two bf16 terms, products hi.hi + hi.lo + lo.hi; M * lda * 4 and K * ldb * 4 below
+// 2 GiB.  Rows need no alignment (a 16-byte buffer load wants its address on a dword, and its dwords are checked
+// against the buffer's end one by one).  TAIL = 0: K % 32 == 0 and N % (32 NB) == 0.  TAIL = 1: any N, and any K whose
+// rows of A are whole 16-byte chunks, zeros past K (K % 4 == 0, or rows padded by the caller): the chunks past K are
+// fetched from beyond the buffer, as zeros, and so are the rows of B past K.
+template <int NB, int TAIL>
 __global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const GroupParams p) {
   typedef WaveK<NB> T;
   extern __shared__ __attribute__((aligned(1024))) unsigned char wavek_smem[];
@@ -76,20 +78,21 @@ __global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const Group
   const int t = id - prob * tiles;
   const int tn = t / p.tiles_m, tm = t - tn * p.tiles_m;
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int steps = p.K / T::BK;                              // all of them
+  const int steps = (p.K + T::BK - 1) / T::BK;                // all of them
   const int my_steps = (steps - wave + T::NW - 1) / T::NW;    // those of this wave: wave, wave + 8, ...
   const int trips = (steps + T::NW - 1) / T::NW;              // of wave 0, the longest
   const int ldb_bytes = (int)p.ldb * 4;
 
-  // rows past M read as zero: the buffer ends with row M - 1
+  // rows past M read as zero: the buffer ends with row M - 1 (B: with row K - 1)
   const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)((int64_t)p.M * p.lda * 4), 0x00020000);
-  const i32x4 rb = make_rsrc(p.B[prob], (int)((int64_t)p.K * p.ldb * 4));
-  int a_voff[4];
+      __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)(((int64_t)(p.M - 1) * p.lda + p.K) * 4), 0x00020000);
+  const i32x4 rb = make_rsrc(p.B[prob], ((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
+  int a_voff[4], a_k[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int row = j * 8 + (lane >> 3);
     const int chunk = ((lane & 7) - (row >> 1)) & 7;
+    a_k[j] = chunk * 4;
     a_voff[j] = (int)(((int64_t)(m0 + row) * p.lda + chunk * 4) * 4);
   }
   const int b_voff = 8 * g * ldb_bytes + (n0 + NB * l31) * 4;
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const Group
     const int step = wave + ii * T::NW;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      wavek_load_lds(ra, ring + st * T::A_STAGE + j * 1024, a_voff[j], step * T::BK * 4);
+      wavek_load_lds(ra, ring + st * T::A_STAGE + j * 1024, !TAIL || a_k[j] < p.K - step * T::BK ? a_voff[j] : 0x7FFFFFFF, step * T::BK * 4);
 #pragma unroll
     for (int j2 = 0; j2 < 2; ++j2)
 #pragma unroll
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const Group
     for (int w = 0; w < T::NW; ++w) sum += part[((w * NB + nb) * 16 + e) * 64 + ln];
     const int row = m0 + 8 * (e >> 2) + 4 * (ln >> 5) + (e & 3);
     const int col = n0 + NB * (ln & 31) + nb;
-    if (row < p.M) C[(int64_t)row * p.ldc + col] = sum + (bias ? bias[col] : 0.f);
+    if (row < p.M && (!TAIL || col < p.N)) C[(int64_t)row * p.ldc + col] = sum + (bias ? bias[col] : 0.f);
   }
 }
 

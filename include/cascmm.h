@@ -33,9 +33,10 @@ extern "C" {
 /* element type of A, B, C and bias as stored in memory (C has the type of A, like
  * `torch.empty((M, N), dtype=a.dtype)` at cascaded_lowp_matmul.py:161).  The cascade kernels
  * take fp32.  fp16 (bf16) tensors multiplied as ONE fp16 (bf16) term have fast kernels too:
- * through cascmm_gemm_prepared, or through cascmm_gemm, when K % 8 == 0 and the rows of A are
- * 16-byte aligned (a raw B whose rows are not whole 16-byte chunks is re-laid in the workspace
- * first, cascmm_workspace_bytes(...)).  Other combinations with 16-bit tensors run on bounds-checked kernels (bf16 or
+ * through cascmm_gemm_prepared when K % 8 == 0 and the rows of A start on dwords, and through
+ * cascmm_gemm for any shape (rows of A that are not whole 16-byte chunks and a B of odd N are
+ * copied into the workspace first, cascmm_workspace_bytes(...); without one the bounds-checked
+ * kernels run).  Other combinations with 16-bit tensors run on bounds-checked kernels (bf16 or
  * fp16 terms, 1 or 2 of them, tri). */
 enum cascmm_dtype { CASCMM_DT_F32 = 0, CASCMM_DT_F16 = 1, CASCMM_DT_BF16 = 2 };
 
