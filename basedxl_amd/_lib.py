@@ -101,6 +101,16 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def native():
+    """The extension module that takes ordinary eager calls (imported once, after torch)."""
+    try:
+        from . import _native
+    except ImportError as e:
+        raise ImportError(f"the host extension {os.path.join(_HERE, '_native.so')} is not built or does not load: {e}. "
+                          "Run `python -m basedxl_amd.build`.") from None
+    return _native
+
+
 def check(status: int, where: str) -> None:
     if status != 0:
         raise CascmmError(status, where)

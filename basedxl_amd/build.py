@@ -1,9 +1,10 @@
-"""Builds libcascmm.so (HIP, gfx950 only) in-tree with hipcc.
+"""Builds libcascmm.so (HIP, gfx950 only) and _native.so (host C++) in-tree.
 
     python -m basedxl_amd.build
 
 Every .hip file under csrc/ is one translation unit; they are compiled in parallel and
-linked into basedxl_amd/libcascmm.so, which the ctypes loader in _lib.py opens.
+linked into basedxl_amd/libcascmm.so, which the ctypes loader in _lib.py opens.  csrc/host/native.cpp
+becomes the extension module basedxl_amd._native, which takes ordinary eager calls to that library.
 """
 from __future__ import annotations
 
@@ -16,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libcascmm.so")
+NATIVE = os.path.join(HERE, "_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -42,11 +44,40 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_native() -> str:
+    """The host extension's object (in a folder of its own: what lies beside it is the library's)."""
+    import sysconfig
+
+    import torch
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    obj = os.path.join(OBJ, "host", "native.o")
+    os.makedirs(os.path.dirname(obj), exist_ok=True)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-I", "/opt/rocm/include", "-I", sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, "host", "native.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on native.cpp:\n" + r.stderr[-4000:])
+    return obj
+
+
+def _link_native(obj: str) -> None:
+    import torch
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", NATIVE, obj, "-L", libs, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+           "-L", HERE, "-l:libcascmm.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("link of _native.so failed:\n" + r.stderr)
+
+
 def build(verbose: bool = True, jobs: int = 8) -> str:
     os.makedirs(OBJ, exist_ok=True)
     srcs = sources()
-    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + 1)) as ex:
+        native = ex.submit(_compile_native)
         objs = list(ex.map(_compile, srcs))
+        native_obj = native.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -57,8 +88,9 @@ def build(verbose: bool = True, jobs: int = 8) -> str:
         ctypes.CDLL(LIB)
     except OSError as e:
         raise RuntimeError(f"{LIB} was linked but does not load: {e}") from None
+    _link_native(native_obj)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} translation units")
+        print(f"built {LIB} from {len(srcs)} translation units, and {NATIVE}")
     return LIB
 
 

@@ -21,12 +21,15 @@ import torch
 
 from . import _lib
 
+_native = _lib.native()
+
 _DTYPES = {torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16}
 
 #: persistent split-K / re-lay workspaces (contents need no initialisation), one per (device index,
 #: stream handle) for eager launches and one per device (key "capture") for launches recorded into a
 #: device graph
 _workspaces: Dict[Tuple[int, object], torch.Tensor] = {}
+_native.init(_workspaces)
 _MIN_WORKSPACE = 1 << 20
 
 
@@ -209,7 +212,7 @@ class PreparedWeight:
         self.K, self.N = int(w.shape[0]), int(w.shape[1])
         self.shape = (self.K, self.N)
         self.lowp, self.terms, self.fmt = lowp, int(terms), _lib.FMT_BY_NAME[lowp]
-        self.dtype, self.device = w.dtype, w.device
+        self.dtype, self.device, self.dt = w.dtype, w.device, _DTYPES[w.dtype]
         self.glu = bool(glu)
         if self.glu and self.N % 64 != 0:
             raise ValueError("glu=True needs a weight whose width is a multiple of 64")
@@ -238,7 +241,7 @@ class PreparedWeight:
         self = cls.__new__(cls)
         self.K, self.N, self.shape = int(K), int(N), (int(K), int(N))
         self.lowp, self.terms, self.fmt = lowp, int(terms), _lib.FMT_BY_NAME[lowp]
-        self.dtype, self.device = dtype, slots.device
+        self.dtype, self.device, self.dt = dtype, slots.device, _DTYPES[dtype]
         self.glu = bool(glu)
         self.out_features = self.N // 2 if self.glu else self.N
         self.exp, self.slots = exp, slots
@@ -750,6 +753,14 @@ def cascaded_lowp_matmul(
     b_exp: Optional[torch.Tensor] = None,
     tensor_exps: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
+    if out is None and variant < 0 and not dump_ptx and tensor_exps is None:
+        # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
+        if type(b) is PreparedWeight:
+            y = _native.prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+        else:
+            y = _native.matmul(a, b, bias, lowp, terms, products)
+        if y is not None:
+            return y
     if lowp is None or terms is None:
         d_lowp, d_terms = default_cascade(a.dtype)
         lowp = d_lowp if lowp is None else lowp

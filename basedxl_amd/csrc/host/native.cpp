@@ -1,0 +1,233 @@
+// The host path of an ordinary eager call in one C++ function: checks, result tensor, stream, workspace and the call
+// into libcascmm.so.
+//
+// A UNet step makes some 500 of these calls, most of them on kernels of 5 - 15 us; issued from Python (argument checks,
+// views, torch.empty, a ctypes call of twenty arguments) each took 13 - 21 us of host time, so the GPU waited for the
+// host.  Everything here is a short cut: a function returns None whenever a call is not the ordinary case (another
+// device, unusual strides, a workspace that has to grow, a status other than 0, ...) and the Python code, which holds
+// all rules and raises all errors, takes it from the start.  Nothing is remembered about a tensor.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+#include <tuple>
+#include <unordered_map>
+
+#include "../../../include/cascmm.h"
+
+namespace {
+
+PyObject* g_workspaces = nullptr;   // the dict {(device index, stream handle): uint8 tensor} of the Python wrapper
+
+struct Need {
+  int64_t M, N, K;
+  int dt, fmt, terms, products;
+  bool operator==(const Need& o) const {
+    return M == o.M && N == o.N && K == o.K && dt == o.dt && fmt == o.fmt && terms == o.terms && products == o.products;
+  }
+};
+struct NeedHash {
+  size_t operator()(const Need& n) const {
+    uint64_t h = 1469598103934665603ull;
+    for (uint64_t v : {(uint64_t)n.M, (uint64_t)n.N, (uint64_t)n.K, (uint64_t)(n.dt | n.fmt << 8 | n.terms << 16 | n.products << 24)})
+      h = (h ^ v) * 1099511628211ull;
+    return (size_t)h;
+  }
+};
+// cascmm_workspace_bytes per problem (it walks the whole variant table); guarded by the interpreter lock
+size_t workspace_need(const Need& n) {
+  static std::unordered_map<Need, size_t, NeedHash> memo;
+  auto it = memo.find(n);
+  if (it != memo.end()) return it->second;
+  if (memo.size() >= 4096) memo.clear();
+  return memo[n] = cascmm_workspace_bytes(n.M, n.N, n.K, n.dt, n.fmt, n.terms, n.products);
+}
+
+int dtype_code(const at::Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return CASCMM_DT_F32;
+    case at::kHalf: return CASCMM_DT_F16;
+    case at::kBFloat16: return CASCMM_DT_BF16;
+    default: return -1;
+  }
+}
+int format_code(PyObject* s) {
+  if (!PyUnicode_Check(s)) return -1;
+  if (PyUnicode_CompareWithASCIIString(s, "bf16") == 0) return CASCMM_FMT_BF16;
+  if (PyUnicode_CompareWithASCIIString(s, "fp16") == 0) return CASCMM_FMT_FP16;
+  return -1;   // (fp8 products find scales first: not the ordinary case)
+}
+int products_code(PyObject* s) {
+  if (!PyUnicode_Check(s)) return -1;
+  if (PyUnicode_CompareWithASCIIString(s, "tri") == 0) return CASCMM_PROD_TRI;
+  if (PyUnicode_CompareWithASCIIString(s, "full") == 0) return CASCMM_PROD_FULL;
+  return -1;
+}
+
+// a plain torch.Tensor or Parameter on the current GPU (no subclass: those may not own memory)
+const at::Tensor* gpu_tensor(PyObject* o, int device) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  return t.is_cuda() && t.get_device() == device && t.has_storage() ? &t : nullptr;
+}
+// the left operand as rows of K elements: false where it is not a view of such rows
+bool rows_of(const at::Tensor& a, int64_t& M, int64_t& K, int64_t& lda) {
+  if (a.dim() < 1) return false;
+  K = a.size(-1);
+  if (K <= 0 || a.numel() == 0) return false;
+  M = a.numel() / K;
+  if (a.is_contiguous()) lda = K;
+  else if (a.dim() == 2 && a.stride(1) == 1 && a.stride(0) >= K) lda = a.stride(0);
+  else return false;
+  if (M == 1) lda = K;
+  return true;
+}
+// a bias the kernels can read (None: no bias); false: not the ordinary case
+bool bias_of(PyObject* o, const at::Tensor& a, int64_t n, int device, const void*& ptr) {
+  ptr = nullptr;
+  if (o == Py_None) return true;
+  const at::Tensor* b = gpu_tensor(o, device);
+  if (!b || b->dim() != 1 || b->size(0) != n || b->scalar_type() != a.scalar_type() || !b->is_contiguous()) return false;
+  ptr = b->const_data_ptr();
+  return true;
+}
+// the stream's workspace if it holds `need` bytes already (eager launches: a recorded one takes the Python path)
+bool workspace_of(size_t need, int device, hipStream_t stream, void*& ptr, size_t& bytes) {
+  ptr = nullptr;
+  bytes = 0;
+  if (need == 0) return true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+  PyObject* key = Py_BuildValue("(iK)", device, (unsigned long long)(uintptr_t)stream);
+  if (!key) { PyErr_Clear(); return false; }
+  PyObject* ws = PyDict_GetItem(g_workspaces, key);   // borrowed
+  Py_DECREF(key);
+  if (!ws || !THPVariable_Check(ws)) return false;
+  const at::Tensor& t = THPVariable_Unpack(ws);
+  if ((size_t)t.numel() < need) return false;
+  ptr = t.data_ptr();
+  bytes = (size_t)t.numel();
+  return true;
+}
+at::Tensor result_like(const at::Tensor& a, int64_t n) {
+  c10::SmallVector<int64_t, 6> sizes(a.sizes().begin(), a.sizes().end());
+  sizes.back() = n;
+  return at::empty(sizes, at::TensorOptions().dtype(a.scalar_type()).device(a.device()));
+}
+
+// matmul(a, b, bias | None, lowp | None, terms | None, products) -> Tensor | None: b a raw [K, N] tensor
+PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 6) Py_RETURN_NONE;
+  try {
+    const int device = c10::hip::current_device();
+    const at::Tensor *a = gpu_tensor(args[0], device), *b = gpu_tensor(args[1], device);
+    if (!a || !b || b->dim() != 2 || b->scalar_type() != a->scalar_type() || !b->is_contiguous()) Py_RETURN_NONE;
+    const int dt = dtype_code(*a);
+    // the default cascade: two bf16 terms for fp32, one term of their own format for 16-bit tensors
+    const int fmt = args[3] != Py_None ? format_code(args[3]) : dt == CASCMM_DT_F16 ? CASCMM_FMT_FP16 : CASCMM_FMT_BF16;
+    const int terms = args[4] != Py_None ? (PyLong_Check(args[4]) ? (int)PyLong_AsLong(args[4]) : -1) : dt == CASCMM_DT_F32 ? 2 : 1;
+    const int products = products_code(args[5]);
+    int64_t M, K, lda;
+    const void* bias;
+    if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    if (dt < 0 || fmt < 0 || terms < 1 || products < 0 || !rows_of(*a, M, K, lda) || b->size(0) != K || b->size(1) <= 0) Py_RETURN_NONE;
+    const int64_t N = b->size(1);
+    if (!bias_of(args[2], *a, N, device, bias)) Py_RETURN_NONE;
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    void* ws;
+    size_t ws_bytes;
+    if (!workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, ws, ws_bytes)) Py_RETURN_NONE;
+    at::Tensor out = result_like(*a, N);
+    const void *ap = a->const_data_ptr(), *bp = b->const_data_ptr();
+    void* cp = out.data_ptr();
+    int st;
+    Py_BEGIN_ALLOW_THREADS
+    st = cascmm_gemm_variant(ap, bp, cp, bias, M, N, K, lda, N, N, dt, fmt, terms, products, nullptr, ws, ws_bytes, stream, -1);
+    Py_END_ALLOW_THREADS
+    if (st != CASCMM_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+  } catch (...) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+}
+
+// prepared(a, slots, bias | None, K, N, fmt, terms, products, dtype of the weight, glu, min_rows) -> Tensor | None: the
+// operand slots of a PreparedWeight (not fp8); fp32 problems of fewer than min_rows rows are left to the caller
+PyObject* prepared(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 11) Py_RETURN_NONE;
+  try {
+    const int device = c10::hip::current_device();
+    const at::Tensor *a = gpu_tensor(args[0], device), *slots = gpu_tensor(args[1], device);
+    if (!a || !slots) Py_RETURN_NONE;
+    const int64_t wk = PyLong_AsLongLong(args[3]), N = PyLong_AsLongLong(args[4]);
+    const int fmt = (int)PyLong_AsLong(args[5]), terms = (int)PyLong_AsLong(args[6]), products = products_code(args[7]);
+    const int w_dt = (int)PyLong_AsLong(args[8]), glu = PyObject_IsTrue(args[9]);
+    const int64_t min_rows = PyLong_AsLongLong(args[10]);
+    if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    const int dt = dtype_code(*a);
+    int64_t M, K, lda;
+    const void* bias;
+    if (dt < 0 || fmt == CASCMM_FMT_FP8 || products < 0 || N <= 0 || !rows_of(*a, M, K, lda) || K != wk) Py_RETURN_NONE;
+    if (!bias_of(args[2], *a, N, device, bias)) Py_RETURN_NONE;
+    const uintptr_t at0 = (uintptr_t)a->const_data_ptr();
+    if (at0 % 16 != 0 || (size_t)lda * a->element_size() % 16 != 0) Py_RETURN_NONE;   // (the wrapper copies such rows)
+    if (dt == CASCMM_DT_F32) {
+      const bool any_rows = fmt == CASCMM_FMT_BF16 && terms == 2 && !glu && K % 8 == 0;
+      if (M < min_rows || (!any_rows && (K % 64 != 0 || N % 4 != 0))) Py_RETURN_NONE;
+    } else if (dt != w_dt || terms != 1 || K % 8 != 0) {
+      Py_RETURN_NONE;
+    }
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    void* ws = nullptr;
+    size_t ws_bytes = 0;
+    if (dt == CASCMM_DT_F32 && !glu &&
+        !workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, ws, ws_bytes))
+      Py_RETURN_NONE;
+    const int64_t NO = glu ? N / 2 : N;
+    at::Tensor out = result_like(*a, NO);
+    const void *ap = (const void*)at0, *bp = slots->const_data_ptr();
+    void* cp = out.data_ptr();
+    int st;
+    Py_BEGIN_ALLOW_THREADS
+    st = glu ? cascmm_gemm_prepared_glu(1, &ap, &bp, &cp, bias ? &bias : nullptr, M, N, K, lda, NO, dt, fmt, terms, products, nullptr, stream, -1)
+             : cascmm_gemm_prepared(1, &ap, &bp, &cp, bias ? &bias : nullptr, M, N, K, lda, NO, dt, fmt, terms, products, nullptr, ws, ws_bytes,
+                                    stream, -1);
+    Py_END_ALLOW_THREADS
+    if (st != CASCMM_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+  } catch (...) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+}
+
+// init(workspaces): the dict to look workspaces up in
+PyObject* init(PyObject*, PyObject* d) {
+  if (!PyDict_Check(d)) {
+    PyErr_SetString(PyExc_TypeError, "init takes the dict of workspaces");
+    return nullptr;
+  }
+  Py_INCREF(d);
+  Py_XDECREF(g_workspaces);
+  g_workspaces = d;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = {
+    {"matmul", (PyCFunction)(void (*)(void))matmul, METH_FASTCALL, "raw operands; None: not the ordinary case"},
+    {"prepared", (PyCFunction)(void (*)(void))prepared, METH_FASTCALL, "prepared weight; None: not the ordinary case"},
+    {"init", init, METH_O, "hands over the workspaces' dict"},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "host path of ordinary eager calls", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&kModule); }

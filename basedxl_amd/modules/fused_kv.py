@@ -48,7 +48,7 @@ class BasedXLFusedKV(nn.Module):
             if recompute or self.kv_cache is None:
                 self.kv_cache = self.to_kv(states)
             kv = self.kv_cache
-        return kv[..., : self.out_features], kv[..., self.out_features:]
+        return kv.narrow(-1, 0, self.out_features), kv.narrow(-1, self.out_features, self.out_features)
 
 
 class BasedXLFusedQKV(nn.Module):
@@ -76,5 +76,5 @@ class BasedXLFusedQKV(nn.Module):
         self.to_qkv = BasedXLLowPLinear(fused, **cascade_kwargs)
 
     def forward(self, states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-        q, k, v = self.to_qkv(states).split(self.splits, dim=-1)
+        q, k, v = self.to_qkv(states).split_with_sizes(self.splits, dim=-1)
         return q, k, v

@@ -14,7 +14,10 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import _lib
 from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, cascaded_lowp_matmul_glu, default_cascade, gated_variant
+
+_native = _lib.native()
 
 
 class BasedXLLowPGEGLU(nn.Module):
@@ -66,6 +69,12 @@ class BasedXLLowPGEGLU(nn.Module):
             h = cascade_linear(x, self.weight, None, self.bias, self.lowp, self.terms, self.products, False, None)
             value, gate = h.chunk(2, dim=-1)
             return value * F.gelu(gate)
+        pw = self._prepared
+        if self.prepared and pw is not None and pw.device == self.weight.device:
+            # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
+            y = _native.prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, True, 0)
+            if y is not None:
+                return y
         if not self.prepared and x.is_cuda and x.dtype == self.weight.dtype and gated_variant(
                 x, self.weight, lowp=self.lowp, terms=self.terms, products=self.products) >= 0:
             return cascaded_lowp_matmul_glu(x, self.weight, bias=self.bias, lowp=self.lowp, terms=self.terms, products=self.products)

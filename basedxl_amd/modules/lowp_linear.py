@@ -6,7 +6,10 @@ import torch.nn as nn
 
 from typing import Optional
 
+from .. import _lib
 from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, default_cascade, tensor_scale_exp
+
+_native = _lib.native()
 
 
 class BasedXLLowPLinear(nn.Module):
@@ -50,6 +53,16 @@ class BasedXLLowPLinear(nn.Module):
             pw = self._prepared_weight
             return cascade_linear(x, self.weight, None if pw is None else pw.slots, self.bias, self.lowp, self.terms,
                                   self.products, False, self._weight_exp if pw is None else pw.exp)
+        # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
+        pw = self._prepared_weight
+        if not self.prepared or (x.dtype == torch.float32 and x.numel() < 32 * self.in_features):
+            y = _native.matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
+        elif pw is not None and pw.device == self.weight.device:
+            y = _native.prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 32)
+        else:
+            y = None
+        if y is not None:
+            return y
         if self.prepared and x.is_cuda:
             if self._prepared_weight is None or self._prepared_weight.device != self.weight.device:
                 self._prepared_weight = PreparedWeight(self.weight, lowp=self.lowp, terms=self.terms)

@@ -1,0 +1,69 @@
+"""The native short cut of ordinary eager calls (csrc/host/native.cpp): the same results as the Python wrapper it stands for,
+and None for every call that is not the ordinary case."""
+import pytest
+import torch
+
+from basedxl_amd import BasedXLFusedKV, BasedXLLowPLinear, PreparedWeight, _lib, cascaded_lowp_matmul
+
+_native = _lib.native()
+
+
+def test_what_is_not_ordinary_is_left_to_the_wrapper():
+    a, b = torch.randn(4, 8), torch.randn(8, 4)
+    assert _native.matmul(a, b, None, None, None, "tri") is None                       # no GPU tensors
+    assert _native.matmul(a.numpy(), b, None, None, None, "tri") is None
+    assert _native.matmul(a, b, None, "fp7", 2 ** 80, "tri") is None and _native.matmul(a, b) is None
+    assert _native.prepared(a, b, None, 8, 4, 0, 2, "tri", 0, False, 0) is None
+    with pytest.raises(TypeError):
+        _native.init([])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", [(2, 1280, 320), (154, 320, 200), (512, 640, 640)])
+def test_same_bits_as_the_wrapper(gpu_device, dtype, M, K, N):
+    """`out=` takes the Python path; the result must be the same kernel's, bit for bit, raw and prepared, with and without a
+    bias, batch dimensions, row strides, and inside a device graph."""
+    g = torch.Generator().manual_seed(K)
+    rn = lambda *s: (torch.randn(*s, generator=g) * 0.1).to("cuda:0").to(dtype)
+    a, w, bias, frame = rn(M, K), rn(K, N), rn(N), rn(M, K + 8)
+    pw = PreparedWeight(w)
+    for x in (a, frame[:, :K], a.view(M // 2, 2, K)):
+        for b in (w, pw):
+            for bb in (None, bias):
+                out = torch.empty(M, N, dtype=dtype, device="cuda:0")
+                want = cascaded_lowp_matmul(x, b, bias=bb, out=out)
+                got = cascaded_lowp_matmul(x, b, bias=bb)
+                assert got.shape == (*x.shape[:-1], N) and torch.equal(got, want)
+    assert _native.matmul(a, w, None, None, None, "tri") is not None                     # (the short cut did run)
+    assert _native.matmul(a.t(), w, None, None, None, "tri") is None and _native.matmul(a, w.t(), None, None, None, "tri") is None
+    assert _native.matmul(a, w, bias[:-1], None, None, "tri") is None and _native.matmul(a, w, None, "fp8", 3, "tri") is None
+    want = cascaded_lowp_matmul(a, w)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        got = cascaded_lowp_matmul(a, w)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_modules_take_it_on_another_stream_and_after_a_move_of_shape(gpu_device):
+    torch.manual_seed(3)
+    lin = torch.nn.Linear(640, 320).to("cuda:0")
+    mod, kv = BasedXLLowPLinear(lin, prepared=True), BasedXLFusedKV(lin, torch.nn.Linear(640, 320).to("cuda:0"))
+    for rows in (2, 40, 300, 2):
+        x = torch.randn(rows, 640, device="cuda:0")
+        want = BasedXLLowPLinear(lin)(x)
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            y = mod(x)
+            k, v = kv(x)
+        s.synchronize()
+        torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(k, want, rtol=1e-5, atol=1e-5)
+        assert k.shape == v.shape == (rows, 320)
