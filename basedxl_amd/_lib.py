@@ -6,6 +6,7 @@ import of the operator fails with an error that says how to build it.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 from ctypes import c_char_p, c_int, c_int32, c_int64, c_size_t, c_void_p, POINTER
 
@@ -101,13 +102,24 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+#: persistent split-K / re-lay workspaces, see cascaded_lowp_matmul.py (here because the host extension looks them up as well)
+workspaces: dict = {}
+
+_native = None
+
+
 def native():
-    """The extension module that takes ordinary eager calls (imported once, after torch)."""
-    try:
-        from . import _native
-    except ImportError as e:
-        raise ImportError(f"the host extension {os.path.join(_HERE, '_native.so')} is not built or does not load: {e}. "
-                          "Run `python -m basedxl_amd.build`.") from None
+    """The extension module that takes ordinary eager calls (imported on first use, like the library: the package itself
+    can be imported before anything is built)."""
+    global _native
+    if _native is None:
+        try:
+            module = importlib.import_module("._native", __package__)
+        except ImportError as e:
+            raise ImportError(f"the host extension {os.path.join(_HERE, '_native.so')} is not built or does not load: {e}. "
+                              "Run `python -m basedxl_amd.build`.") from None
+        module.init(workspaces)
+        _native = module
     return _native
 
 

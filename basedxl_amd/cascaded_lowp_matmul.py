@@ -21,15 +21,12 @@ import torch
 
 from . import _lib
 
-_native = _lib.native()
-
 _DTYPES = {torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16}
 
 #: persistent split-K / re-lay workspaces (contents need no initialisation), one per (device index,
 #: stream handle) for eager launches and one per device (key "capture") for launches recorded into a
 #: device graph
-_workspaces: Dict[Tuple[int, object], torch.Tensor] = {}
-_native.init(_workspaces)
+_workspaces: Dict[Tuple[int, object], torch.Tensor] = _lib.workspaces
 _MIN_WORKSPACE = 1 << 20
 
 
@@ -756,9 +753,9 @@ def cascaded_lowp_matmul(
     if out is None and variant < 0 and not dump_ptx and tensor_exps is None:
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         if type(b) is PreparedWeight:
-            y = _native.prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+            y = _lib.native().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
         else:
-            y = _native.matmul(a, b, bias, lowp, terms, products)
+            y = _lib.native().matmul(a, b, bias, lowp, terms, products)
         if y is not None:
             return y
     if lowp is None or terms is None:

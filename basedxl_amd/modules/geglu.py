@@ -17,8 +17,6 @@ import torch.nn.functional as F
 from .. import _lib
 from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, cascaded_lowp_matmul_glu, default_cascade, gated_variant
 
-_native = _lib.native()
-
 
 class BasedXLLowPGEGLU(nn.Module):
     """Wraps the ``proj`` Linear ([in] -> [2 * inner]) of a GEGLU block; ``forward(x)`` returns
@@ -72,7 +70,7 @@ class BasedXLLowPGEGLU(nn.Module):
         pw = self._prepared
         if self.prepared and pw is not None and pw.device == self.weight.device:
             # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
-            y = _native.prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, True, 0)
+            y = _lib.native().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, True, 0)
             if y is not None:
                 return y
         if not self.prepared and x.is_cuda and x.dtype == self.weight.dtype and gated_variant(

@@ -8,6 +8,23 @@ from basedxl_amd import BasedXLFusedKV, BasedXLLowPLinear, PreparedWeight, _lib,
 _native = _lib.native()
 
 
+def test_the_package_imports_before_anything_is_built(tmp_path):
+    """A fresh checkout holds neither library, and the build itself imports the package."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    import basedxl_amd
+    src = os.path.dirname(basedxl_amd.__file__)
+    shutil.copytree(src, tmp_path / "basedxl_amd", ignore=shutil.ignore_patterns("*.so", "build", "__pycache__"))
+    code = ("from basedxl_amd import build, _lib\nassert build.sources()\n"
+            "for load in (_lib.lib, _lib.native):\n    try:\n        load()\n    except ImportError as e:\n"
+            "        assert 'basedxl_amd.build' in str(e), e\n    else:\n        raise SystemExit('loaded what is not there')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, env={**os.environ, "PYTHONPATH": str(tmp_path)}, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
 def test_what_is_not_ordinary_is_left_to_the_wrapper():
     a, b = torch.randn(4, 8), torch.randn(8, 4)
     assert _native.matmul(a, b, None, None, None, "tri") is None                       # no GPU tensors
