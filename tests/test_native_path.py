@@ -3,7 +3,7 @@ and None for every call that is not the ordinary case."""
 import pytest
 import torch
 
-from basedxl_amd import BasedXLFusedKV, BasedXLLowPLinear, PreparedWeight, _lib, cascaded_lowp_matmul
+from basedxl_amd import BasedXLFusedKV, BasedXLLowPGEGLU, BasedXLLowPLinear, PreparedWeight, _lib, cascaded_lowp_matmul
 
 _native = _lib.native()
 
@@ -65,6 +65,15 @@ def test_same_bits_as_the_wrapper(gpu_device, dtype, M, K, N):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_gated_layer_refuses_activations_of_another_dtype(gpu_device):
+    """A 16-bit weight kept as two bf16 terms has fp32 kernels, but the layer's input has its weight's dtype."""
+    mod = BasedXLLowPGEGLU(torch.nn.Linear(64, 128).to("cuda:0", torch.bfloat16), lowp="bf16", terms=2)
+    mod.prepare()
+    with pytest.raises(TypeError):
+        mod(torch.randn(40, 64, device="cuda:0"))
 
 
 @pytest.mark.gpu
