@@ -97,8 +97,10 @@ bool bias_of(PyObject* o, const at::Tensor& a, int64_t n, int device, const void
   ptr = b->const_data_ptr();
   return true;
 }
-// the stream's workspace if it holds `need` bytes already (eager launches: a recorded one takes the Python path)
-bool workspace_of(size_t need, int device, hipStream_t stream, void*& ptr, size_t& bytes) {
+// the stream's workspace if it holds `need` bytes already (eager launches: a recorded one takes the Python path).
+// `hold` keeps it until the launch: another thread may replace the dict's entry while this one has given up the lock, and
+// memory freed before the launch could be written by work that was enqueued in between
+bool workspace_of(size_t need, int device, hipStream_t stream, at::Tensor& hold, void*& ptr, size_t& bytes) {
   ptr = nullptr;
   bytes = 0;
   if (need == 0) return true;
@@ -109,10 +111,10 @@ bool workspace_of(size_t need, int device, hipStream_t stream, void*& ptr, size_
   PyObject* ws = PyDict_GetItem(g_workspaces, key);   // borrowed
   Py_DECREF(key);
   if (!ws || !THPVariable_Check(ws)) return false;
-  const at::Tensor& t = THPVariable_Unpack(ws);
-  if ((size_t)t.numel() < need) return false;
-  ptr = t.data_ptr();
-  bytes = (size_t)t.numel();
+  hold = THPVariable_Unpack(ws);
+  if ((size_t)hold.numel() < need) return false;
+  ptr = hold.data_ptr();
+  bytes = (size_t)hold.numel();
   return true;
 }
 at::Tensor result_like(const at::Tensor& a, int64_t n) {
@@ -140,9 +142,10 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t N = b->size(1);
     if (!bias_of(args[2], *a, N, device, bias)) Py_RETURN_NONE;
     const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    at::Tensor hold;
     void* ws;
     size_t ws_bytes;
-    if (!workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, ws, ws_bytes)) Py_RETURN_NONE;
+    if (!workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, hold, ws, ws_bytes)) Py_RETURN_NONE;
     at::Tensor out = result_like(*a, N);
     const void *ap = a->const_data_ptr(), *bp = b->const_data_ptr();
     void* cp = out.data_ptr();
@@ -185,10 +188,11 @@ PyObject* prepared(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       Py_RETURN_NONE;
     }
     const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    at::Tensor hold;
     void* ws = nullptr;
     size_t ws_bytes = 0;
     if (dt == CASCMM_DT_F32 && !glu &&
-        !workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, ws, ws_bytes))
+        !workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, hold, ws, ws_bytes))
       Py_RETURN_NONE;
     const int64_t NO = glu ? N / 2 : N;
     at::Tensor out = result_like(*a, NO);
