@@ -59,6 +59,7 @@ struct Problem {
   // stages, of which the operands hold k_valid, and their rows need no alignment
   bool split_first = false;
   int64_t k_valid = 0;
+  bool whole_k = false;   // no K split over workgroups (cascmm_ksplit.h)
 };
 
 // Three fp8 terms with K a multiple of 64 are prepared for the fp8-rate kernel: [term][K/16][N] slots
@@ -203,6 +204,8 @@ static const TunedCost kTuned[] = {
 };
 
 constexpr int kMaxTileSplits = 4;
+// kernels that split K over workgroups as cascmm_ksplit.h describes
+static bool ksplit_kind(const VariantDesc& v) { return v.kind == KIND_H16 || v.kind == KIND_SLOTK; }
 // the fp8-rate kernel with K over the waves: us per 64-k stage of a wave, and per round of tiles
 constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {1280, 5120} x 1280, 4096 x {640, 2560} x 640)
 
@@ -223,7 +226,10 @@ static const std::vector<VariantInfo>& variant_info() {
 // The kernel that splits K over the waves of a workgroup (KIND_WAVEK) moves (32 + BN) x K x 4 bytes
 // into every workgroup and is bound by that: a CU pulled in 85 bytes per ns with the 32-wide and
 // 60 with the 64-wide tile, all CUs together 17 KB per ns (154 x 2048 x {640, 1280, 2560}); a launch
-// costs 2.5 us, prologue and the meeting of the partial tiles 0.6 us per round of workgroups.
+// costs 2.5 us, prologue and the meeting of the partial tiles 0.6 us.  A launch of several rounds pays the
+// start of every workgroup (one fits a CU, so nothing hides it) and runs at 48 / 52 bytes per ns and CU: 1425 x 2112 x
+// 528 41 us, 576 x 560 x 7532 74 us, 448 x 592 x 1952 18.3 us; priced as single rounds these kept the kernel on
+// problems that the 64 x 160 tiles run in 25, 33 and 13.6 us.
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
          !q.glu && q.K > 0 && (q.K % 32 == 0 || q.chunked) && q.M * q.lda * 4 <= INT32_MAX;
@@ -233,8 +239,12 @@ static double wavek_estimate_us(const Problem& q, int count, int bn) {
   const double active = items < kNumCUs ? items : kNumCUs;
   const double per_cu = bn == 32 ? 85.0e3 : 60.0e3;                       // bytes per us
   const double rate = per_cu < 17.0e6 / active ? per_cu : 17.0e6 / active;
-  const double rounds = (double)(int64_t)((items + kNumCUs - 1) / kNumCUs);
-  return 2.5 + rounds * (0.6 + (double)(32 + bn) * (double)q.K * 4.0 / rate);
+  const double bytes = (double)(32 + bn) * (double)q.K * 4.0;
+  if (items <= kNumCUs) return 2.5 + 0.6 + bytes / rate;
+  const double start = bn == 32 ? 1.7 : 4.1, full_rate = bn == 32 ? 48.0e3 : 52.0e3;
+  const double full = (double)(int64_t)(items / kNumCUs), rest = items - full * kNumCUs;
+  const double rest_rate = rest * per_cu < kNumCUs * full_rate ? per_cu : kNumCUs * full_rate / rest;
+  return 2.5 + full * (start + bytes / full_rate) + (rest > 0 ? start + bytes / rest_rate : 0.0);
 }
 static double wavek_estimate_us(const Problem& q, int count) {
   const double a = wavek_estimate_us(q, count, 32), b = wavek_estimate_us(q, count, 64);
@@ -258,22 +268,49 @@ static const H16Cost kH16Cost[] = {
     {128, 160, 0.0058, 0.0092, 3.5, 2.4, 1.17}, {128, 128, 0.0056, 0.0077, 3.3, 1.8, 1.16}, {64, 160, 0.0047, 0.0053, 3.7, 2.7, 1.10},
     {64, 128, 0.0042, 0.0046, 3.3, 1.1, 1.06},  {128, 64, 0.0044, 0.0050, 3.5, 1.1, 1.02},  {64, 64, 0.0026, 0.0033, 3.2, 1.0, 1.20},
 };
-static double h16_estimate_us(const VariantDesc& v, const Problem& q, double tiles) {
+static double h16_estimate_us(const VariantDesc& v, const Problem& q, double tiles, int64_t k_per) {
   for (const H16Cost& c : kH16Cost)
     if (c.BM == v.BM && c.BN == v.BN) {
       const double full = (double)(int64_t)(tiles / kNumCUs), rem = tiles / kNumCUs - full;
       const double last = rem > 0 ? (c.s1 * rem > c.s0 ? c.s1 * rem : c.s0) : 0.0;
-      const double k = (double)((q.K + v.BK - 1) / v.BK * v.BK) * (q.bpre ? 1.0 : c.raw);
+      const double k = (double)((k_per + v.BK - 1) / v.BK * v.BK) * (q.bpre ? 1.0 : c.raw);
       return c.start + (full + (rem > 0 ? 1.0 : 0.0)) * c.end + k * (full * c.s1 + last);
     }
   return 1e9;
 }
 
+// The K-over-waves kernels (KIND_SLOTK): whole trips of four stages per wave, K in steps of 256; tiles over the edge of C
+// were 3 - 9 % slower than their whole neighbours (320 x 956 x 1792, 800 x 896 x 2688).
+static double slotk_estimate_us(const TunedCost& t, const VariantDesc& v, const Problem& q, double tiles, int64_t k_per) {
+  const double full = (double)(int64_t)(tiles / kNumCUs), rem = tiles - full * kNumCUs;
+  const double tail = full == 0 ? t.tail_first : t.tail_later;
+  const double rounds = full + (rem > 0 ? tail + (1.0 - tail) * rem / kNumCUs : 0.0);
+  const double edge = (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.05 : 1.0;
+  return edge * rounds * ((double)((k_per + 255) / 256 * 256) / 64.0 * t.step64_us + t.fixed_us);
+}
+
+// K split over workgroups (cascmm_ksplit.h): where the tiles leave CUs idle, `estimate(tiles, k of a split)` with the
+// chip filled against the second launch and the partial results, written and read back.  Measured: 7 x 3264 x 880 fp16
+// 14.8 -> 6.8 us in eight splits, 256 x 5120 x 1280 23.0 -> 14.0 in five, 34 x 2008 x 2176 fp32 prepared 15.5 -> 9.7 in
+// eight, 154 x 2048 x 2560 raw 18.4 -> 15.5 in four.  Below 11 us the second launch, 3 us of the
+// host's time, costs an eager call more than it gives (keys and values 40 x 1664 x 768 fp16 8.4 -> 11.5 us).
+template <class F>
+static double ksplit_best(const Problem& q, int count, double tiles, size_t ws_bytes, double launch_us, double bytes_per_us, int* splits, F estimate) {
+  double best = estimate(tiles, q.K);
+  *splits = 1;
+  if (count != 1 || q.glu || q.whole_k || best < 11.0) return best;
+  for (int sp = 2; sp <= kMaxKSplits && tiles * sp <= kNumCUs; ++sp) {
+    if (!ksplit_valid(q.K, sp) || ksplit_bytes(q.M, q.N, sp) > ws_bytes) continue;
+    const double c = estimate(tiles * sp, ksplit_k(q.K, sp)) + launch_us + (double)ksplit_bytes(q.M, q.N, sp) / bytes_per_us;
+    if (c < best) { best = c; *splits = sp; }
+  }
+  return best;
+}
+
 // ws_bytes: workspace the caller brought; *splits_out: K split the cost was computed for (the
 // LDS-tiled two-term bf16 kernels may split K over up to kMaxTileSplits work items per tile when a
 // single problem has too few tiles to occupy the chip and the workspace holds the partials)
-static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes = 0,
-                           int* splits_out = nullptr) {
+static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes = 0, int* splits_out = nullptr) {
   const VariantDesc& v = table()[vi];
   const VariantInfo& info = variant_info()[vi];
   if (splits_out) *splits_out = 1;
@@ -286,11 +323,22 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
     // smaller row tile was faster wherever both were measured.
     if ((double)((q.M + 63) / 64) * (double)((q.N + 127) / 128) >= kNumCUs / 2) return 1e9;
     // ... unless the one-launch kernel that splits K over its waves is expected to be faster
-    if (wavek_eligible(q) && wavek_estimate_us(q, count) < skinny_estimate_us(q)) return 1e9;
+    const double skinny_us = skinny_estimate_us(q);
+    if (wavek_eligible(q) && wavek_estimate_us(q, count) < skinny_us) return 1e9;
+    // ... or the K-over-waves tiles, K split over workgroups too (64 x 5120 x 1280: 17.1 us here, 15.2 there)
+    for (int i = 0; i < (int)table().size(); ++i)
+      if (table()[i].kind == KIND_SLOTK && variant_matches(table()[i], q, FIT_DWORD) && variant_cost(i, q, count, ws_bytes) < skinny_us) return 1e9;
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
   if (v.kind == KIND_WAVEK) return wavek_estimate_us(q, count, v.BN);
-  if (v.kind == KIND_H16) return h16_estimate_us(v, q, tiles);
+  int ks = 1;
+  if (v.kind == KIND_H16 || (v.kind == KIND_SLOTK && info.tuned)) {
+    const double us = v.kind == KIND_H16
+        ? ksplit_best(q, count, tiles, ws_bytes, 1.6, 3.8e6, &ks, [&](double t, int64_t k) { return h16_estimate_us(v, q, t, k); })
+        : ksplit_best(q, count, tiles, ws_bytes, 2.8, 12.0e6, &ks, [&](double t, int64_t k) { return slotk_estimate_us(*info.tuned, v, q, t, k); });
+    if (splits_out) *splits_out = ks;
+    return us;
+  }
   if (v.kind == KIND_F8K64) {
     // stages of 64 k at ~2.1 us per resident round, the K split the launcher will use, and the passes
     // around the GEMM: the split of A (and of B unless prepared), the reduction of a K split
@@ -322,9 +370,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
     // tiles that hang over the edge of C take the bounds-checked epilogue and load clamped
     // columns: measured about a quarter slower (32768 x 640 x 320 on the 128-wide tile)
     const double edge = (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.25 : 1.0;
-    // (the kernels that split K over their waves run whole trips of four stages per wave: K in steps of 256)
-    const double k_run = v.kind == KIND_SLOTK ? (double)((q.K + 255) / 256 * 256) : (double)q.K;
-    double best = edge * rounds * (k_run / 64.0 * t.step64_us + t.fixed_us);
+    double best = edge * rounds * ((double)q.K / 64.0 * t.step64_us + t.fixed_us);
     if (v.kind == KIND_TILE && count == 1 && q.dtype == CASCMM_DT_F32 && q.N % 4 == 0 && full == 0 && !q.glu) {
       const int64_t ksteps = (q.K + v.BK - 1) / v.BK;
       for (int sp = 2; sp <= kMaxTileSplits; ++sp) {
@@ -377,7 +423,7 @@ struct SelectKey {
   size_t ws_bytes;
   // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
   // some kernels: M lda, K ldb and 1024 ldc beyond 2^31 bytes << 3, 4, 5; lda below 32 << 7), glu_slots << 6,
-  // chunked << 8, split_first << 9, the fit of the rows << 10
+  // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12
   int dtype, fmt, terms, products, count, flags;
   bool operator==(const SelectKey& o) const {
     return M == o.M && N == o.N && K == o.K && ws_bytes == o.ws_bytes && dtype == o.dtype && fmt == o.fmt &&
@@ -403,7 +449,7 @@ static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_byt
   static std::mutex mu;
   static std::unordered_map<SelectKey, SelectHit, SelectKeyHash> memo;
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
-                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
+                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
                           (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0)};
   {
     std::lock_guard<std::mutex> lock(mu);
@@ -646,6 +692,21 @@ static Relay relay_of(const Problem& q, int count, const void* const* A, const v
   return r;
 }
 static size_t relay_bytes(const Relay& r, int count) { return (size_t)count * (r.a_bytes + r.b_bytes); }
+// the problem that is left once its operands are copied
+static Problem relayed(const Problem& q0, const Relay& r) {
+  Problem q = q0;
+  if (r.a) q.lda = r.a_chunks * (16 / (int64_t)dtype_size(q.dtype));
+  q.chunked = true;
+  q.bpre = r.b;
+  if (r.b) q.ldb = q.N;
+  return q;
+}
+// what the partial results of the chosen kernel's K split take, at most `room`
+static size_t ksplit_need(const Problem& q, RowFit fit, size_t room) {
+  int splits = 1;
+  const int v = select_variant(q, fit, 1, room, &splits);
+  return v >= 0 && ksplit_kind(table()[v]) ? ksplit_bytes(q.M, q.N, splits) : 0;
+}
 
 // three fp8 / fp16 terms that the slot kernels take once K is rounded up to their stages: they split both operands in a
 // pass of their own, which fills the rest with zeros and reads rows of any alignment
@@ -719,8 +780,8 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
   } else {
     splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
     variant &= 0xFFFF;
-    if (splits > kMaxTileSplits) return CASCMM_ERR_BAD_VARIANT;
     if (variant >= (int)t.size()) return CASCMM_ERR_BAD_VARIANT;
+    if (splits > (ksplit_kind(t[variant]) ? kMaxKSplits : kMaxTileSplits)) return CASCMM_ERR_BAD_VARIANT;
     if (!variant_matches(t[variant], q, fit)) return CASCMM_ERR_BAD_VARIANT;
   }
   const VariantDesc& v = t[variant];
@@ -748,6 +809,16 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
   p.workspace = workspace;
   p.workspace_bytes = workspace_bytes;
   p.k_splits = v.kind == KIND_TILE ? splits : 1;
+  p.k_per = p.K;
+  if (ksplit_kind(v) && splits > 1 && count == 1 && !q.glu) {
+    // (a forced count of which some would be empty: the others; without room for the partial results: K whole)
+    const int64_t k_per = ksplit_k(q.K, splits);
+    splits = (int)((q.K + k_per - 1) / k_per);
+    if (workspace && aligned_to(workspace, 16) && ksplit_bytes(q.M, q.N, splits) <= workspace_bytes && splits > 1) {
+      p.k_splits = splits;
+      p.k_per = (int)k_per;
+    }
+  }
   p.tensor_exps = q.fmt == CASCMM_FMT_FP8 ? tensor_exps : nullptr;
   p.glu = q.glu_slots ? 2 : (q.glu ? 1 : 0);
   p.exps_dyn = exps_dyn;
@@ -801,6 +872,11 @@ static int gemm_impl(int count, const void* const* A, const void* const* B, void
     return err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
   }
   q.chunked = chunked_by_k(q);
+  // Calls of several launches that meet in the workspace go to the stream as a whole: two threads that share a stream, and
+  // with it the workspace, must not put one call's launches between another's.
+  static std::mutex workspace_mu;
+  std::unique_lock<std::mutex> whole(workspace_mu, std::defer_lock);
+  if (workspace) whole.lock();
   if (variant < 0) {
     const Relay r = relay_of(q, count, A, B);
     if ((r.a || r.b) && workspace && aligned_to(workspace, 16) && workspace_bytes >= relay_bytes(r, count)) {
@@ -832,14 +908,8 @@ static int gemm_impl(int count, const void* const* A, const void* const* B, void
                         (int)q.K, q.lda, r.a_chunks, (u32x4*)ap[i], (int)a_blocks, (const unsigned short*)B[i], (int)q.N, q.ldb, (u32x4*)bp[i]);
         if (err != hipSuccess) return CASCMM_ERR_LAUNCH;
       }
-      A = ap;
-      B = bp;
-      if (r.a) q.lda = r.a_chunks * (16 / (int64_t)es);
-      q.chunked = true;
-      q.bpre = r.b;
-      if (r.b) q.ldb = q.N;
-      // (the kernels behind a copy need no workspace of their own)
-      return gemm_on_rows(count, A, B, C, bias, q, tensor_exps, nullptr, 0, stream, -1);
+      const size_t rest = workspace_bytes - relay_bytes(r, count);
+      return gemm_on_rows(count, ap, bp, C, bias, relayed(q, r), tensor_exps, rest > 0 ? (char*)workspace + relay_bytes(r, count) : nullptr, rest, stream, -1);
     }
   }
   return gemm_on_rows(count, A, B, C, bias, q, tensor_exps, workspace, workspace_bytes, stream, variant, exps_dyn, b_exp_src);
@@ -893,6 +963,7 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
   if (relay.a || relay.b) {
     need = relay_bytes(relay, 1);
     if (need > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) need = 0;   // (the bounds-checked kernels need no copy)
+    else need += ksplit_need(relayed(q, relay), FIT_FAST, (size_t)CASCMM_NOALLOC_SCRATCH_BYTES - need);
   } else if (A && B) {
     const RowFit fit = row_fit(q, A, B);
     q.chunked = chunked_by_k(q);
@@ -904,7 +975,19 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
       v = select_variant(q, fit, 1, (size_t)-1, &splits);
     }
     if (v < 0) return v;
-    if ((table()[v].kind == KIND_F8K64 && f8k64_workspace_bytes(M, N, e.K, false, table()[v].BM) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) ||
+    bool as_chosen = true;
+    if (ksplit_kind(table()[v]) && ksplit_bytes(M, N, splits) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) {
+      // (a K split over workgroups is a choice: without it the call is refused or taken as the other kernels need)
+      e.whole_k = true;
+      v = select_variant(e, fit, 1, (size_t)-1, &splits);
+      if (v < 0) return v;
+      as_chosen = table()[v].kind == KIND_TILE && splits > 1;
+    }
+    // (refused where nothing comes near the tile kernels' own K split: few rows have the one-launch kernel)
+    if (table()[v].kind == KIND_TILE && splits > 1 && (size_t)splits * (size_t)M * (size_t)N * sizeof(float) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES &&
+        wavek_eligible(e) && (M <= 160 || wavek_estimate_us(e, 1) < 1.8 * variant_cost(v, e, 1, (size_t)-1)))
+      as_chosen = false;
+    if (!as_chosen || (table()[v].kind == KIND_F8K64 && f8k64_workspace_bytes(M, N, e.K, false, table()[v].BM) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) ||
         (table()[v].kind == KIND_F16K && f16k_workspace_bytes(M, N, e.K) > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES)) {
       // the fp8-rate kernel is a choice, not a need: without room for its operand slots the choice is
       // made among the kernels that split inside the GEMM
@@ -915,6 +998,7 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
     if (d.kind == KIND_SPLITK) need = skinny_workspace_bytes(M, N, K, d.BM, d.BN, d.BK);
     else if (d.kind == KIND_F8K64) need = f8k64_workspace_bytes(M, N, e.K, false, d.BM);
     else if (d.kind == KIND_F16K) need = f16k_workspace_bytes(M, N, e.K);
+    else if (ksplit_kind(d)) need = ksplit_bytes(M, N, splits);
     else if (splits > 1) need = (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
   }
   if (need > (size_t)CASCMM_NOALLOC_SCRATCH_BYTES) return CASCMM_ERR_SCRATCH_LIMIT;
@@ -1066,6 +1150,19 @@ size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fm
   // rows of A (and, 16-bit, all of B) copied first
   const Relay relay = relay_of(q, 1, nullptr, nullptr);
   size_t need = relay_bytes(relay, 1);
+  // K split over workgroups, behind such a copy or on the operands as they lie, raw or prepared
+  size_t parts = 0;
+  for (int pre = 0; pre < 2; ++pre) {
+    Problem e = relay.a || relay.b ? relayed(q, relay) : q;
+    e.bpre = e.bpre || pre != 0;
+    for (int vi = 0; vi < (int)table().size(); ++vi) {
+      if (!ksplit_kind(table()[vi]) || !variant_matches(table()[vi], e, FIT_FAST)) continue;
+      int sp = 1;
+      variant_cost(vi, e, 1, (size_t)-1, &sp);
+      parts = std::max(parts, ksplit_bytes(M, N, sp));
+    }
+  }
+  need += parts;
   for (const auto& v : table()) {
     if (v.kind != KIND_SPLITK || !variant_matches(v, q, fit)) continue;
     const size_t n = skinny_workspace_bytes(M, N, K, v.BM, v.BN, v.BK);

@@ -350,6 +350,7 @@ struct GroupParams {
   void* workspace;          // split-K partials: fp32 [k_splits][M][N]
   size_t workspace_bytes;
   int k_splits;             // LDS-tiled kernels: work item = (split, problem, tile); 0 or 1 = no split
+  int k_per;                // kernels on cascmm_ksplit.h: k of a split (K: no split)
   const int32_t* tensor_exps;  // fp8: {e_A, e_B} of problem i at [2i], [2i + 1]; NULL = all zero
   // Gated epilogue: C has N/2 columns, C[m][32 j + l] = (v + bias[32 j + l]) * gelu(g + bias[N/2 + 32 j + l])
   // with v and g the entries of A x B in row m whose columns of B are, for a prepared operand (which

@@ -25,7 +25,7 @@
 #pragma once
 #include <type_traits>
 
-#include "cascmm_tile_kernel.h"
+#include "cascmm_ksplit.h"
 
 namespace cascmm {
 
@@ -79,7 +79,8 @@ template <> struct H16Elem<CASCMM_FMT_FP16> { typedef _Float16 T; static constex
 // Host-checked: the rows of A start on dwords and are whole 16-byte chunks, zeros past K (K % 8 == 0, or padded), M * lda * 2
 // below 2 GiB; RAWB = 0: B prepared ([ceil(K / 64) * 8][N] slots, zeros beyond K) below 2 GiB; RAWB = 1: B [K][ldb] with
 // N % 2 == 0 and rows on dwords, K * ldb * 2 below 2 GiB.  Any M and N: rows and columns past the edge are loaded as zeros or as
-// some other column's values and not stored.  grid.y: the problem of a group.
+// some other column's values and not stored.  grid.y: the problem of a group.  k_splits > 1: K in splits of k_per (a
+// multiple of 64), fp32 sums to the workspace instead of a result, see cascmm_ksplit.h.
 // GLU: gated store (see GroupParams; RAWB = 0, NTL even: a wave owns whole value / gate pairs of blocks).
 template <class T, int FMT, int RAWB, int GLU>
 __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams p) {
@@ -94,16 +95,20 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   const int wm0 = (wmn / T::WN) * T::WTM, wn0 = (wmn % T::WN) * T::WTN;
   const int prob = blockIdx.y;
   int tm, tn;
-  tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, T::GROUP_M);
+  tile_coords(blockIdx.x, p.tiles_m * p.k_splits, p.tiles_n, tm, tn, T::GROUP_M < p.tiles_m || p.k_splits == 1 ? T::GROUP_M : p.tiles_m);
+  const int split = ksplit_of_row(tm, p.tiles_m, p.k_per, p.K);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int ksteps = (p.K + T::BK - 1) / T::BK;
+  const int k0 = split * p.k_per;
+  const int K = p.K - k0 < p.k_per ? p.K - k0 : p.k_per;
+  const int ksteps = (K + T::BK - 1) / T::BK;
 
   // rows past M read as zero (the buffer ends with row M - 1), and so does everything past B's last row or slot row
-  const int kgs = (p.K + 63) / 64 * 8;
-  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + (p.K + 7) / 8 * 8) * 2;
-  const int64_t b_bytes = RAWB ? ((int64_t)(p.K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)a_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[prob], 0, (int)b_bytes, 0x00020000);
+  const int kgs = (K + 63) / 64 * 8;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + (K + 7) / 8 * 8) * 2;
+  const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
+  const int64_t b_first = RAWB ? (int64_t)k0 * p.ldb * 2 : (int64_t)(k0 / 8) * p.N * 16;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)p.A[prob] + k0), 0, (int)a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)p.B[prob] + b_first), 0, (int)b_bytes, 0x00020000);
 
   // ---- loads: this wave's kilobytes of a stage ----
   // A: row r of the stage's BM x BK block at r * 2 BK bytes; position pos of a row holds chunk (pos - rot(r)) mod KG,
@@ -134,7 +139,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     unsigned char* st = smem + buf * T::STAGE;
     if (j < T::A_LOADS) {
       // (past K: beyond the buffer's end, zeros)
-      const int v = a_k[j] < p.K - step * T::BK ? a_voff[j] : 0x7FFFFFFF;
+      const int v = a_k[j] < K - step * T::BK ? a_voff[j] : 0x7FFFFFFF;
       h16_load_lds(ra, st + (wave * T::A_LOADS + j) * 1024, v, step * T::BK * 2);
     } else {
       const int bs = (step < ksteps ? step : ksteps) * b_step;
@@ -267,6 +272,26 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   auto finish = [&](auto first_tag, auto count_tag, auto bias_tag) {
     constexpr int B0 = decltype(first_tag)::value, NB = decltype(count_tag)::value;
     constexpr bool BIAS = decltype(bias_tag)::value != 0;
+    if constexpr (!BIAS && !GLU) {
+      if (p.k_splits > 1) {   // (a lane's four consecutive columns of its row; the wave's rows of a block, 32 bytes each)
+        const int row = (p.N + 3) & ~3, col0 = n0 + wn0 + 32 * B0;
+        float* part = (float*)p.workspace + ((int64_t)split * p.M + m0 + wm0) * row + col0;
+        const int64_t bytes = ((int64_t)(p.M - 1 - m0 - wm0) * row + (row - col0)) * 4;
+        const i32x4 rp = make_rsrc(part, bytes < 0 ? 0 : bytes);
+#pragma unroll
+        for (int mi = 0; mi < T::MT; ++mi)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f32x16& v = acc[mi][B0 + b];
+              const int col = 32 * b + 8 * q + 4 * g;
+              llvm_raw_buffer_store_v4f32((f32x4){v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]}, rp,
+                                          col0 + col < row ? ((mi * 32 + l31) * row + col) * 4 : 0x7FFFFFFF, 0, 0);
+            }
+        return;
+      }
+    }
     // ---- store: of block (mi, ni) a lane holds row 32 mi + l31, columns 32 ni + 8 q + 4 g + e in register 4 q + e ----
     const int no = GLU ? p.N >> 1 : p.N;
     const int oc0 = (GLU ? (n0 + wn0) >> 1 : n0 + wn0) + 32 * B0;

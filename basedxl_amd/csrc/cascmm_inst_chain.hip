@@ -36,17 +36,24 @@ int launch_prepare_left(const float* A, int M, int K, int64_t lda, void* out, hi
 
 const void* slotk_kernel_handle(int araw) { return araw ? (const void*)cascmm_slotk_kernel<1, 0> : (const void*)cascmm_slotk_kernel<0, 0>; }
 
+// workgroups of a launch, and what the kernels need to find their tile and split (see cascmm_ksplit.h)
+static int64_t slot_grid(SlotKParams& q, int splits, int group_m) {
+  q.stack_m = q.tiles_m * splits;
+  q.group_m = splits > 1 && q.tiles_m < group_m ? q.tiles_m : group_m;
+  return (int64_t)q.stack_m * q.tiles_n;
+}
+
 template <int ARAW, int TAIL>
-static int launch_slotk_t(const SlotKParams& q, hipStream_t stream) {
+static int launch_slotk_t(const SlotKParams& q, hipStream_t stream, int splits = 1) {
   typedef SlotK T;
   auto kfn = cascmm_slotk_kernel<ARAW, TAIL>;
   static LdsFlags lds_set;
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
   SlotKParams p = q;
+  if (splits == 1) p.k_per = q.K;
   p.tiles_m = (q.M + T::BM - 1) / T::BM;
   p.tiles_n = (q.N + T::BN - 1) / T::BN;
-  p.group_m = SlotK::GROUP_M;
-  const int64_t grid = (int64_t)p.tiles_m * p.tiles_n;
+  const int64_t grid = slot_grid(p, splits, SlotK::GROUP_M);
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
   return launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, p) == hipSuccess ? CASCMM_OK
                                                                                                               : CASCMM_ERR_LAUNCH;
@@ -56,19 +63,37 @@ int launch_slotk(const SlotKParams& q, int araw, hipStream_t stream) {
   return araw ? launch_slotk_t<1, 0>(q, stream) : launch_slotk_t<0, 0>(q, stream);
 }
 
+// the operands of a launch from the variant table, the result or, where K is split over workgroups, the partial ones
+static int slot_params(const GroupParams& p, SlotKParams& q) {
+  memset(&q, 0, sizeof(q));
+  q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
+  q.M = p.M; q.N = p.N; q.K = p.K; q.lda = p.lda; q.ldb = p.ldb; q.ldc = p.ldc;
+  q.k_per = p.k_per;
+  if (p.k_splits > 1) {
+    const int st = ksplit_check(p);
+    if (st != CASCMM_OK) return st;
+    q.C = (float*)p.workspace;
+    q.ldc = ksplit_row(p.N);
+    q.bias = nullptr;
+  }
+  return CASCMM_OK;
+}
+static int slot_finish(const GroupParams& p, int st, hipStream_t stream) {
+  return st == CASCMM_OK && p.k_splits > 1 ? launch_ksplit_reduce<CASCMM_DT_F32>(p, stream) : st;
+}
+
 // the variant-table face of the kernel: raw fp32 left operand, prepared right operand
 static int launch_slotk_variant(const GroupParams& p, hipStream_t stream) {
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_slotk_kernel<1, 0>; return CASCMM_OK; }
-  if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count != 1 || p.glu) return CASCMM_ERR_BAD_VARIANT;
   if (p.lda < 2 * SlotK::BK) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || prepared_kgroups(p.K) * p.N * 32 > 0x7FFFFFFF || p.ldc * (int64_t)(SlotK::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   SlotKParams q;
-  memset(&q, 0, sizeof(q));
-  q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
-  q.M = p.M; q.N = p.N; q.K = p.K; q.lda = p.lda; q.ldc = p.ldc;
+  const int st = slot_params(p, q);
+  if (st != CASCMM_OK) return st;
   // (raw A comes in pairs of 16-k stages)
-  return p.K % (2 * SlotK::BK) == 0 ? launch_slotk_t<1, 0>(q, stream) : launch_slotk_t<1, 1>(q, stream);
+  return slot_finish(p, p.K % (2 * SlotK::BK) == 0 ? launch_slotk_t<1, 0>(q, stream, p.k_splits) : launch_slotk_t<1, 1>(q, stream, p.k_splits), stream);
 }
 
 // the 64 x 80 tile of the same design, for problems that make too few 64 x 160 tiles to occupy the chip
@@ -76,29 +101,27 @@ static int launch_slotn_variant(const GroupParams& p, hipStream_t stream) {
   typedef SlotN T;
   auto kfn = p.K % T::BK == 0 ? cascmm_slotn_kernel<0> : cascmm_slotn_kernel<1>;
   if (p.kernel_out) { *p.kernel_out = (const void*)kfn; return CASCMM_OK; }
-  if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count != 1 || p.glu) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || prepared_kgroups(p.K) * p.N * 32 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   static LdsFlags lds_set[2];
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[p.K % T::BK == 0 ? 0 : 1])) return CASCMM_ERR_LAUNCH;
   SlotKParams q;
-  memset(&q, 0, sizeof(q));
-  q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
-  q.M = p.M; q.N = p.N; q.K = p.K; q.lda = p.lda; q.ldc = p.ldc;
+  const int st = slot_params(p, q);
+  if (st != CASCMM_OK) return st;
   q.tiles_m = (p.M + T::BM - 1) / T::BM;
   q.tiles_n = (p.N + T::BN - 1) / T::BN;
-  q.group_m = T::GROUP_M;
-  const int64_t grid = (int64_t)q.tiles_m * q.tiles_n;
+  const int64_t grid = slot_grid(q, p.k_splits, T::GROUP_M);
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  return launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q) == hipSuccess ? CASCMM_OK
-                                                                                                              : CASCMM_ERR_LAUNCH;
+  const hipError_t err = launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q);
+  return slot_finish(p, err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH, stream);
 }
 
 // both operands raw fp32
 static int launch_rawk_variant(const GroupParams& p, hipStream_t stream) {
   typedef SlotK T;
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_rawk_kernel<0>; return CASCMM_OK; }
-  if (p.count != 1 || p.glu || p.k_splits > 1) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count != 1 || p.glu) return CASCMM_ERR_BAD_VARIANT;
   if (p.lda < 2 * T::BK) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
@@ -107,17 +130,15 @@ static int launch_rawk_variant(const GroupParams& p, hipStream_t stream) {
   static LdsFlags lds_set[2];
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[tail ? 1 : 0])) return CASCMM_ERR_LAUNCH;
   SlotKParams q;
-  memset(&q, 0, sizeof(q));
-  q.a = p.A[0]; q.b_slots = p.B[0]; q.C = (float*)p.C[0]; q.bias = (const float*)p.bias[0];
-  q.M = p.M; q.N = p.N; q.K = p.K; q.lda = p.lda; q.ldb = p.ldb; q.ldc = p.ldc;
+  const int st = slot_params(p, q);
+  if (st != CASCMM_OK) return st;
   q.tiles_m = (p.M + T::BM - 1) / T::BM;
   q.tiles_n = (p.N + T::BN - 1) / T::BN;
-  q.group_m = SlotK::GROUP_M;
-  const int64_t grid = (int64_t)q.tiles_m * q.tiles_n;
+  const int64_t grid = slot_grid(q, p.k_splits, SlotK::GROUP_M);
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  const int c_vec = p.N % 4 == 0 && p.ldc % 4 == 0 && (uintptr_t)p.C[0] % 16 == 0;
-  return launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q, c_vec) == hipSuccess ? CASCMM_OK
-                                                                                                                     : CASCMM_ERR_LAUNCH;
+  const int c_vec = q.N % 4 == 0 && q.ldc % 4 == 0 && (uintptr_t)q.C % 16 == 0;
+  const hipError_t err = launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q, c_vec);
+  return slot_finish(p, err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH, stream);
 }
 
 static const VariantDesc kChainTable[] = {

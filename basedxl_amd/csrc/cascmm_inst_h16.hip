@@ -11,19 +11,27 @@ static int launch_h16_kernel(const GroupParams& p, hipStream_t stream) {
     static LdsFlags lds_set;
     if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
   }
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.count);
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.k_splits), (unsigned)p.count);
   return launch_kernel(kfn, grid, dim3(T::NT), (size_t)T::LDS_BYTES, stream, p) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
 }
 
 template <class T, int FMT, int RAWB, int GLU>
 static int launch_h16(const GroupParams& p, hipStream_t stream) {
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_h16_kernel<T, FMT, RAWB, 0>; return CASCMM_OK; }
-  if (p.count < 1 || p.k_splits > 1 || p.lda % 2 != 0 || (p.glu && !GLU)) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count < 1 || p.lda % 2 != 0 || (p.glu && !GLU)) return CASCMM_ERR_BAD_VARIANT;
   if (RAWB && (p.N % 2 != 0 || p.ldb % 2 != 0)) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 2 > 0x7FFFFFFF || (RAWB ? ((int64_t)p.K + 64) * p.ldb * 2 : prepared_kgroups(p.K) * p.N * 16) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   if constexpr (GLU) {
     if (p.glu) return launch_h16_kernel<T, FMT, 0, 1>(p, stream);
+  }
+  if (p.k_splits > 1) {
+    const int st = ksplit_check(p);
+    if (st != CASCMM_OK) return st;
+    GroupParams q = p;
+    q.bias[0] = nullptr;
+    const int sg = launch_h16_kernel<T, FMT, RAWB, 0>(q, stream);
+    return sg == CASCMM_OK ? launch_ksplit_reduce<H16Elem<FMT>::DT>(p, stream) : sg;
   }
   return launch_h16_kernel<T, FMT, RAWB, 0>(p, stream);
 }

@@ -46,10 +46,13 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   // contiguous range of tile ids, and ids walk GROUP_M tile rows down before moving one tile to the right:
   // a tile's B slots are 2.5 times its A slots, so the block of tiles that share an L2 is taller than wide.
   int tm, tn;
-  tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
+  tile_coords((int)blockIdx.x, p.stack_m, p.tiles_n, tm, tn, p.group_m);
+  const int split = ksplit_of_row(tm, p.tiles_m, p.k_per, p.K);   // (raw A only)
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int kgroups = ARAW ? (int)prepared_kgroups(p.K) : p.K >> 3;   // (slots x slots: both buffers end with K)
-  const int ksteps = TAIL ? (p.K + 31) / 32 * 2 : p.K >> 4;
+  const int k0_split = split * p.k_per, K = p.K - k0_split < p.k_per ? p.K - k0_split : p.k_per;
+  float* C = p.C + (int64_t)split * p.M * p.ldc;
+  const int ksteps = TAIL ? (K + 31) / 32 * 2 : K >> 4;
   // Which 16-k stages of the problem a wave owns.  A as slots: every fourth one, own stage i = stage
   // wave + 4 i.  A raw: every fourth PAIR of stages, own stage i = stage 8 (i / 2) + 2 wave + i % 2, so that
   // what the wave fetches of a row for a pair is one whole 128-byte line (with every fourth stage it was half
@@ -65,12 +68,13 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   // stage, times the zero slots of B).
 
   // ---- right operand: lane (l31, g) reads k group 2 step + g, column block ni 512 bytes further ----
-  const i32x4 rb = make_rsrc(p.b_slots, (int64_t)2 * kgroups * p.N * 16);
+  const int b_first = (k0_split >> 3) * p.N * 16;
+  const i32x4 rb = make_rsrc((const char*)p.b_slots + b_first, (int64_t)2 * kgroups * p.N * 16 - b_first);
   const int vb = (g * p.N + n0 + l31) * 16;
   const int b_term = kgroups * p.N * 16;   // from term 0 to term 1
   const int b_step = 2 * p.N * 16;         // from one 16-k stage to the next
   u32x4 Br[T::D][T::NTL][2];               // [ring buffer][column block][term]
-  const int b_end = 2 * b_term;            // the buffer's size: every offset from there on is outside
+  const int b_end = 2 * b_term - b_first;  // the buffer's size: every offset from there on is outside
   auto issue_b = [&](int i, int buf, int ni) {
     const int base = i < n_own ? stage_of(i) * b_step : b_end;
 #pragma unroll
@@ -90,9 +94,9 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
 
   // ---- left operand raw -----------------------------------------------------------------------------
   // rows past M read as zero: the buffer ends with row M - 1
-  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + p.K) * 4;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + K) * 4;
   const __amdgpu_buffer_rsrc_t rar =
-      __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, ARAW ? (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes) : 0, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)((const float*)p.a + k0_split), 0, ARAW ? (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes) : 0, 0x00020000);
   unsigned char* ring = slotk_smem + wave * T::RING;
   // A pair of stages in LDS: 64 rows x 128 bytes (eight 16-byte chunks of 4 k).  Load j of a pair (0 .. 7)
   // brings rows 8 j + lane / 8; position pos of a row holds chunk (pos - row / 2) mod 8, which spreads the
@@ -117,7 +121,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   auto dma_a = [&](int i, int ni, int sp) {
     const int q = i >> 1;
     const int k0 = 2 * q < n_own ? stage_of(2 * q) * T::BK : 0;
-    const int v = !TAIL || dma_k[ni & 1] < p.K - k0 ? dma_v[ni] : 0x7FFFFFFF;
+    const int v = !TAIL || dma_k[ni & 1] < K - k0 ? dma_v[ni] : 0x7FFFFFFF;
     wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, v, k0 * 4 + 4 * sp * dma_rows8, ni);
   };
   // fragment of lane (l31, g), row block mi, stage parity s: row 32 mi + l31, chunks 4 s + 2 g and 4 s + 2 g + 1
@@ -263,7 +267,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
     const int ldc_bytes = (int)p.ldc * 4;
     // rows past M fall beyond the end of the buffer and are dropped
     const int64_t c_bytes = ((int64_t)(p.M - 1 - m0) * p.ldc + (p.N - n0)) * 4;
-    const i32x4 rc = make_rsrc(p.C + (int64_t)m0 * p.ldc + n0, c_bytes);
+    const i32x4 rc = make_rsrc(C + (int64_t)m0 * p.ldc + n0, c_bytes);
 #pragma unroll
     for (int b = W; b < T::BLOCKS; b += T::NW) {
       const int mi = b / T::NTL, ni = b % T::NTL;
@@ -335,9 +339,12 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int tm, tn;
-  tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
+  tile_coords((int)blockIdx.x, p.stack_m, p.tiles_n, tm, tn, p.group_m);
+  const int split = ksplit_of_row(tm, p.tiles_m, p.k_per, p.K);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int ksteps = TAIL ? (p.K + 31) / 32 * 2 : p.K >> 4;
+  const int k0_split = split * p.k_per, K = p.K - k0_split < p.k_per ? p.K - k0_split : p.k_per;
+  float* C = p.C + (int64_t)split * p.M * p.ldc;
+  const int ksteps = TAIL ? (K + 31) / 32 * 2 : K >> 4;
   // a wave owns every fourth PAIR of 16-k stages (see the kernel above): own stage i = stage 8 (i / 2) + 2 wave + i % 2
   const int own_tail = (ksteps & 7) - 2 * wave;
   const int n_own = 2 * (ksteps >> 3) + (own_tail < 0 ? 0 : own_tail > 2 ? 2 : own_tail);   // 0 for the last waves of a very short K: they add zeros
@@ -346,9 +353,9 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
 
   // ---- B: rows 8 g .. 8 g + 7 of a stage; beyond the last stage the loads point past the end of the
   // buffer and return zeros (see the kernel above) ----
-  const int64_t b_bytes64 = ((int64_t)(p.K - 1) * p.ldb + p.N) * 4;
+  const int64_t b_bytes64 = ((int64_t)(K - 1) * p.ldb + p.N) * 4;
   const int b_bytes = (int)(b_bytes64 > 0x7FFFFFFF ? 0x7FFFFFFF : b_bytes64);
-  const i32x4 rb = make_rsrc(p.b_slots, b_bytes);
+  const i32x4 rb = make_rsrc((const float*)p.b_slots + (int64_t)k0_split * p.ldb, b_bytes);
   const int vbq = 8 * g * ldb_bytes + (n0 + 4 * l31) * 4;
   const int vbs = 8 * g * ldb_bytes + (n0 + 128 + l31) * 4;
   f32x4 Bq[D][8];   // [ring buffer][k]: columns 4 l31 .. 4 l31 + 3
@@ -371,9 +378,9 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   };
 
   // ---- A: as in cascmm_slotk_kernel<1> ----
-  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + p.K) * 4;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + K) * 4;
   const __amdgpu_buffer_rsrc_t rar =
-      __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)((const float*)p.a + k0_split), 0, (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
   unsigned char* ring = slotk_smem + wave * T::RING;
   int dma_voff[2], dma_k[2];
 #pragma unroll
@@ -388,7 +395,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   auto dma_a = [&](int i, int ni, int sp) {   // sp = i % 2
     const int q = i >> 1;
     const int k0 = 2 * q < n_own ? stage_of(2 * q) * T::BK : 0;
-    const int v = !TAIL || dma_k[ni & 1] < p.K - k0 ? dma_v[ni] : 0x7FFFFFFF;
+    const int v = !TAIL || dma_k[ni & 1] < K - k0 ? dma_v[ni] : 0x7FFFFFFF;
     wavek_load_lds_kb(rar, ring + (q & (T::RA / 2 - 1)) * (2 * T::A_STAGE) + sp * 4096, v, k0 * 4 + 4 * sp * dma_rows8, ni);
   };
   int a_frag[2][2];
@@ -540,7 +547,7 @@ __global__ __launch_bounds__(SlotK::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
     const int ldc_bytes = (int)p.ldc * 4;
     const int64_t c_bytes64 = ((int64_t)(p.M - 1 - m0) * p.ldc + (p.N - n0)) * 4;   // rows past M fall beyond the end: dropped
     const int c_bytes = (int)(c_bytes64 > 0x7FFFFFFF ? 0x7FFFFFFF : c_bytes64);
-    const i32x4 rc = make_rsrc(p.C + (int64_t)m0 * p.ldc + n0, c_bytes);
+    const i32x4 rc = make_rsrc(C + (int64_t)m0 * p.ldc + n0, c_bytes);
     // columns past N (a ragged last tile) are sent beyond the end as well
     const int colq = 4 * l31, cols = 128 + l31;
     const bool inq = n0 + colq < p.N, ins = n0 + cols < p.N;   // (c_vec: four adjacent columns are inside together)

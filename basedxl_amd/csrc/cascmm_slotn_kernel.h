@@ -43,18 +43,22 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int tm, tn;
-  tile_coords((int)blockIdx.x, p.tiles_m, p.tiles_n, tm, tn, p.group_m);
+  tile_coords((int)blockIdx.x, p.stack_m, p.tiles_n, tm, tn, p.group_m);
+  const int split = ksplit_of_row(tm, p.tiles_m, p.k_per, p.K);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int kgroups = (int)prepared_kgroups(p.K);
-  const int ksteps = (p.K + 31) >> 5;
+  const int k0_split = split * p.k_per, K = p.K - k0_split < p.k_per ? p.K - k0_split : p.k_per;
+  const float* A = (const float*)p.a + k0_split;
+  float* C = p.C + (int64_t)split * p.M * p.ldc;
+  const int ksteps = (K + 31) >> 5;
   const int n_own = (ksteps - wave + T::NW - 1) / T::NW;   // 0 for the last waves of a very short K: they add zeros
   // The loop runs in trips of two stages without a branch inside; a wave with an odd number of stages runs one
   // stage past its last: its B loads point beyond the end of the buffer and return zeros, its A loads fetch the
   // problem's first stage (finite values for the zeros to multiply).
 
   // ---- B: lane (l15, kg) reads k group 4 stage + kg of column n0 + 16 nb + l15 ----
-  const int b_term = kgroups * p.N * 16, b_end = 2 * b_term;
-  const i32x4 rb = make_rsrc(p.b_slots, (int64_t)b_end);
+  const int b_term = kgroups * p.N * 16, b_first = (k0_split >> 3) * p.N * 16, b_end = 2 * b_term - b_first;
+  const i32x4 rb = make_rsrc((const char*)p.b_slots + b_first, (int64_t)b_end);
   const int vb = (kg * p.N + n0 + l15) * 16;
   const int b_step = 4 * p.N * 16;
   u32x4 Br[T::D][T::NB][2];
@@ -66,9 +70,9 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   };
 
   // ---- A: rows past M read as zero (the buffer ends with row M - 1) ----
-  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + p.K) * 4;
+  const int64_t a_bytes = ((int64_t)(p.M - 1) * p.lda + K) * 4;
   const __amdgpu_buffer_rsrc_t rar =
-      __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
   unsigned char* ring = slotn_smem + wave * T::RING;
   // Load j of a stage (0 .. 7) brings rows 8 j + lane / 8 to LDS bytes j * 1024 + 16 lane, i.e. lane % 8 is the
   // position inside the row's 128 bytes; position pos of row r holds chunk (pos - rot(h)) mod 8 with h = (r / 2) mod 8
@@ -88,7 +92,7 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   const int dma_rows8 = (int)p.lda * 32;
   auto dma_a = [&](int i, int j) {
     const int k0 = i < n_own ? (wave + T::NW * i) * T::BK : 0;
-    const int v = !TAIL || dma_k[j & 1] < p.K - k0 ? dma_voff[j & 1] : 0x7FFFFFFF;
+    const int v = !TAIL || dma_k[j & 1] < K - k0 ? dma_voff[j & 1] : 0x7FFFFFFF;
     wavek_load_lds(rar, ring + (i & (T::RA - 1)) * T::A_STAGE + j * 1024, v, k0 * 4 + j * dma_rows8);
   };
   // fragment of lane (l15, kg), row block mb: row 16 mb + l15, chunks 2 kg and 2 kg + 1 at their rotated places
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1)
   // rows past M fall beyond the end of the buffer and are dropped
   const int64_t c_bytes64 = ((int64_t)(p.M - 1 - m0) * p.ldc + (p.N - n0)) * 4;
   const int c_bytes = (int)(c_bytes64 > 0x7FFFFFFF ? 0x7FFFFFFF : c_bytes64);
-  const i32x4 rc = make_rsrc(p.C + (int64_t)m0 * p.ldc + n0, c_bytes);
+  const i32x4 rc = make_rsrc(C + (int64_t)m0 * p.ldc + n0, c_bytes);
 #pragma unroll
   for (int x = 0; x < T::BLOCKS / T::NW; ++x) {
     const int b = wave + T::NW * x;          // (wave-uniform)

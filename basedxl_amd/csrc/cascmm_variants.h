@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "cascmm_bdirect_kernel.h"
+#include "cascmm_ksplit.h"
 #include "cascmm_w512_kernel.h"
 #include "cascmm_f8k64_kernel.h"
 #include "cascmm_f16k_kernel.h"
@@ -455,6 +456,7 @@ struct SlotKParams {
   int64_t lda, ldb, ldc;   // ldb: cascmm_rawk_kernel only (raw B)
   int tiles_m, tiles_n;
   int group_m;             // tile rows an XCD's range of tiles walks down before moving one tile to the right
+  int stack_m, k_per;      // tiles_m x splits; k of a split (fewer than K: C is the partial results): see cascmm_ksplit.h
 };
 
 int launch_slotk(const SlotKParams& q, int araw, hipStream_t stream);

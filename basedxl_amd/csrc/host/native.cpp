@@ -191,7 +191,7 @@ PyObject* prepared(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor hold;
     void* ws = nullptr;
     size_t ws_bytes = 0;
-    if (dt == CASCMM_DT_F32 && !glu &&
+    if (!glu &&
         !workspace_of(workspace_need({M, N, K, dt, fmt, terms, products}), device, stream, hold, ws, ws_bytes))
       Py_RETURN_NONE;
     const int64_t NO = glu ? N / 2 : N;
