@@ -143,6 +143,9 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_W512 && (q.M % v.BM != 0 || q.N % v.BN != 0 || q.M * q.lda * 4 > INT32_MAX ||
                               (!q.bpre && q.K * q.ldb * 4 > INT32_MAX) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
+  if (v.kind == KIND_W512E && (q.M < W512_EDGE_ROWS || q.N < v.BN || (q.glu && v.BN == W512::BN && q.N % v.BN != 0) || q.K == 0 || q.M * q.lda * 4 > INT32_MAX ||
+                               (!q.bpre && q.K * q.ldb * 4 > INT32_MAX) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
+    return false;
   if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
@@ -172,8 +175,12 @@ static const TunedCost kTuned[] = {
     {"t64x64x64_w2x2x1_d3_bf16x2_tri", 0.671, 2.34, 1.00, 1.00},
     {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 1.064, 4.69, 0.90, 0.80},
     {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 1.224, 6.84, 0.80, 0.70},
-    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 3.250, 5.00, 0.70, 0.50},
-    {"t256x320x32_w512_bf16x2_tri", 5.65, 16.0, 1.00, 1.00},
+    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 3.200, 6.50, 0.70, 0.50},
+    // (the large tiles on every whole or ragged shape of 4992 x 2048 x 2048 to 4096^3 that was swept: partly filled rounds
+    // are faster than full ones, the board's power goes to fewer CUs: 64 of 256 tiles 0.62, 144 tiles 0.7, 192 tiles 0.88)
+    {"t256x320x32_w512_bf16x2_tri", 5.65, 16.0, 0.50, 0.50},
+    {"t256x320x32_w512_edge_bf16x2_tri", 5.65, 17.0, 0.50, 0.50},
+    {"t256x256x32_w512_edge_bf16x2_tri", 4.60, 10.5, 0.45, 0.45},
     // three fp16 / bf16 terms
     {"t128x128x32_w4x2x1_d2_fp16x3_tri", 3.107, 7.22, 0.90, 0.80},
     {"t64x64x32_w2x2x1_d3_fp16x3_tri", 1.088, 2.27, 1.00, 1.00},
@@ -193,7 +200,9 @@ static const TunedCost kTuned[] = {
     {"t64x64x64_w2x2x1_d3_bf16x2_tri_bpre", 0.515, 2.08, 1.00, 1.00},
     {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 1.250, 5.89, 0.80, 0.50},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri_bpre", 2.837, 12.00, 0.60, 0.50},
-    {"t256x320x32_w512_bf16x2_tri_bpre", 5.50, 16.0, 1.00, 1.00},
+    {"t256x320x32_w512_bf16x2_tri_bpre", 5.40, 15.0, 0.50, 0.50},
+    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 5.40, 16.0, 0.50, 0.50},
+    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 4.50, 11.5, 0.45, 0.45},
     // K split over the waves: a round of 256 tiles costs 0.011 us per k + 8 us, and rounds do not overlap
     // (2048 x {1280, 5120} x 1280: 21.7 / 64.3 us; 1024 x 1280 x 1280: 17.4 us -- 7 % less than with raw A fetched
     // in half lines, A/B on one box)
@@ -369,7 +378,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
     const double rounds = full + (rem > 0 ? tail + (1.0 - tail) * rem / kNumCUs : 0.0);
     // tiles that hang over the edge of C take the bounds-checked epilogue and load clamped
     // columns: measured about a quarter slower (32768 x 640 x 320 on the 128-wide tile)
-    const double edge = (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.25 : 1.0;
+    const double edge = v.kind != KIND_W512E && (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.25 : 1.0;
     double best = edge * rounds * ((double)q.K / 64.0 * t.step64_us + t.fixed_us);
     if (v.kind == KIND_TILE && count == 1 && q.dtype == CASCMM_DT_F32 && q.N % 4 == 0 && full == 0 && !q.glu) {
       const int64_t ksteps = (q.K + v.BK - 1) / v.BK;

@@ -13,13 +13,14 @@
 
 namespace cascmm {
 
-// KIND_W512: the large-tile kernel (whole 256 x 320 tiles only, one problem per launch)
+// KIND_W512: the large-tile kernel (whole 256 x 320 tiles only, one problem per launch); KIND_W512E: its instantiations
+// that take tiles over the edges of C
 // KIND_F8K64: three fp8 terms on the fp8-rate MFMA; splits its operands into the workspace first
 // KIND_F16K: three fp16 terms on operand slots; finds both scales and splits its operands into the workspace first
 // KIND_WAVEK: skinny problems in one launch, K split over the waves of a workgroup (no workspace)
 // KIND_H16: 16-bit tensors as one term of their own format, right operand prepared or raw (no workspace)
 // KIND_SLOTK: prepared right operand, K split over the waves of a workgroup (64 x 160 tiles, one problem per launch)
-enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7 };
+enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7, KIND_W512E = 8 };
 constexpr int kNumCUs = 256;  // MI355X: what the cost model's constants were measured on
 constexpr int kMaxDevices = 64;
 
@@ -192,10 +193,10 @@ int launch_bdirect(const GroupParams& gp, hipStream_t stream) {
 }
 
 // the large-tile kernel (BPRE = 1: right operand prepared)
-template <int BPRE, int GLU>
+template <int BPRE, int GLU, int NTL = 5, int EDGE = 0>
 int launch_w512_kernel(const GroupParams& p, hipStream_t stream) {
-  typedef W512 T;
-  auto kfn = cascmm_w512_kernel<BPRE, GLU>;
+  typedef W512Tile<NTL> T;
+  auto kfn = cascmm_w512_kernel<BPRE, GLU, NTL, EDGE>;
   static LdsFlags lds_set;
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set)) return CASCMM_ERR_LAUNCH;
   const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n);
@@ -214,6 +215,22 @@ int launch_w512(const GroupParams& p, hipStream_t stream) {
   // (the gated stores are instantiations of their own; glu == 2: the result leaves as operand slots)
   if (p.glu == 2) return launch_w512_kernel<BPRE, 2>(p, stream);
   return p.glu ? launch_w512_kernel<BPRE, 1>(p, stream) : launch_w512_kernel<BPRE, 0>(p, stream);
+}
+
+// ... whose tiles may hang over the edges of C
+template <int BPRE, int NTL>
+int launch_w512_edge(const GroupParams& p, hipStream_t stream) {
+  typedef W512Tile<NTL> T;
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_w512_kernel<BPRE, 0, NTL, 1>; return CASCMM_OK; }
+  if (p.count != 1 || p.k_splits > 1 || p.glu == 2 || (p.glu && (!BPRE || (NTL == 5 && p.N % T::BN != 0)))) return CASCMM_ERR_BAD_VARIANT;
+  if (p.M < W512_EDGE_ROWS || p.N < T::BN || p.N % 4 != 0 || p.K % 32 != 0 || p.K < 32) return CASCMM_ERR_BAD_VARIANT;
+  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 32 : (int64_t)p.K * p.ldb * 4) > 0x7FFFFFFF ||
+      p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
+    return CASCMM_ERR_TOO_LARGE;
+  if constexpr (BPRE) {
+    if (p.glu) return launch_w512_kernel<BPRE, 1, NTL, 1>(p, stream);
+  }
+  return launch_w512_kernel<BPRE, 0, NTL, 1>(p, stream);
 }
 
 // skinny problems, K split over the waves of a workgroup
@@ -409,6 +426,10 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \
   {NAME, KIND_W512, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512::BM, W512::BN, 32, W512::NT, W512::LDS_BYTES, true, \
    false, &launch_w512<BPRE>, BPRE != 0, true}
+
+#define CASCMM_W512_EDGE_VARIANT(NAME, BPRE, NTL)                                                                         \
+  {NAME, KIND_W512E, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512Tile<NTL>::BM, W512Tile<NTL>::BN, 32, W512Tile<NTL>::NT, \
+   W512Tile<NTL>::LDS_BYTES, true, false, &launch_w512_edge<BPRE, NTL>, BPRE != 0, BPRE != 0}
 
 // eight producer waves, every B column loaded singly (all producer threads share A and B evenly)
 #define CASCMM_TILE_VARIANT_PS(NAME, BM, BN, BK, WM, WN, WK, DEPTH, NP, IODT, FMT, TERMS, FULL, FAST)          \

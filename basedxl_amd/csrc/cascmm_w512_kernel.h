@@ -35,17 +35,35 @@
 
 namespace cascmm {
 
-struct W512 {
-  static constexpr int BM = 256, BN = 320, BK = 16, NS = 4, NT = 256;
-  static constexpr int WTM = 128, WTN = 160, MT = 4, NTL = 5;
+template <int NTL_>
+struct W512Tile {
+  static constexpr int NTL = NTL_;                  // column blocks of a wave
+  static constexpr int BM = 256, BN = 64 * NTL, BK = 16, NS = 4, NT = 256;
+  static constexpr int WTM = 128, WTN = 32 * NTL, MT = 4;
   static constexpr int A_STAGE = BM * BK * 4;       // raw fp32: 64 bytes per row
   static constexpr int B_STAGE = BK * BN * 4;       // raw fp32
-  static constexpr int STAGE = A_STAGE + B_STAGE;   // 36 KB
-  static constexpr int LDS_BYTES = NS * STAGE;      // 144 KB
-  static constexpr int LOADS = 9;                   // direct loads per wave and stage: 4 of A, 5 of B
+  static constexpr int STAGE = A_STAGE + B_STAGE;   // 36 KB (NTL = 4: 32 KB)
+  static constexpr int LDS_BYTES = NS * STAGE;      // 144 KB (128 KB)
+  static constexpr int LOADS = 4 + NTL;             // direct loads per wave and stage: 4 of A, NTL of B
 };
+typedef W512Tile<5> W512;
+constexpr int W512_EDGE_ROWS = 64;   // EDGE: the fewest rows
 
 typedef __attribute__((address_space(3))) void* w512_lds_ptr;
+
+// one wave-wide direct load, j KB behind the LDS address (and the lane offset)
+__device__ __forceinline__ void w512_load0(__amdgpu_buffer_rsrc_t r, w512_lds_ptr dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ void w512_load1(__amdgpu_buffer_rsrc_t r, w512_lds_ptr dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, voff, soff, 1024, 0);
+}
+__device__ __forceinline__ void w512_load2(__amdgpu_buffer_rsrc_t r, w512_lds_ptr dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, voff, soff, 2048, 0);
+}
+__device__ __forceinline__ void w512_load3(__amdgpu_buffer_rsrc_t r, w512_lds_ptr dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, voff, soff, 3072, 0);
+}
 
 // MFMA with the accumulator in ordinary vector registers
 __device__ __forceinline__ void w512_mfma_v(u32x4 a, u32x4 b, f32x16& c) {
@@ -55,7 +73,20 @@ __device__ __forceinline__ f32x16 w512_mfma_a(u32x4 a, u32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Host-checked: M % 256 == 0, N % 320 == 0, K % 32 == 0, lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
+// an empty statement that uses a block where it is kept
+__device__ __forceinline__ void w512_in_acc(f32x16& c) { asm volatile("" : "+a"(c)); }
+__device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(c)); }
+
+// NTL: column blocks of a wave; 5 is the 256 x 320 tile described above, 4 the same on 256 x 256 (sixteen blocks, all in
+// the accumulation registers).
+// EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
+// costs the loop nothing, and the stores past it go beyond the descriptor's end.
+// Measured (graph replay, raw / prepared weight; in brackets the fastest other kernel): 1976 x 1280 x 10240 on 256 x 320
+// 129.6 / 122.4 us (164.8 / 153.6), its gated form 126.1 (158.5); 7800 x 640 x 5120 139 / 134 (155 / 143); 1500 x 1280 x 10240
+// on 256 x 256 104 / 98 (134 / 110); 4096^3 316 / 297 (351 / 326) = 1.30 PFLOP/s of MFMA work, as on the wider tile: what is
+// left is the clock the board's power allows.
+// Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, N % 4 == 0; with the gated store N % 320 == 0 on the wider
+// tile), K % 32 == 0, lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
 // aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets
 // inside a tile.
 // GLU = 1: the gated store (C has N / 2 columns, see GroupParams); a raw operand's gate columns are
@@ -75,9 +106,12 @@ __device__ __forceinline__ f32x16 w512_mfma_a(u32x4 a, u32x4 b, f32x16 c) {
 // 16-byte reads instead of eight 4-byte ones, and the split of B, 55 % of the kernel's VALU work,
 // is gone.  Same terms, same order of products: the results equal the raw kernel's bit for bit.
 // (a template, so that only the translation unit that lists the variant compiles it)
-template <int BPRE, int GLU = 0>
-__global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_w512_kernel(const GroupParams p) {
-  typedef W512 T;
+template <int BPRE, int GLU = 0, int NTL = 5, int EDGE = 0>
+__global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_w512_kernel(const GroupParams p) {
+  typedef W512Tile<NTL> T;
+  static_assert(NTL == 4 || NTL == 5, "");
+  static_assert(!GLU || NTL == 5 || (GLU == 1 && BPRE && EDGE), "");
+  static_assert(GLU != 2 || !EDGE, "");
   extern __shared__ __attribute__((aligned(1024))) unsigned char w512_smem[];
   unsigned char* smem = w512_smem;
   const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, g = lane >> 5;
@@ -94,23 +128,26 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
   // in front of every B load)
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[0], 0, 0x7FFFFFFE, 0x00020000);
   // per wave and stage: 4 loads of A (16 rows x 64 bytes each; LDS position 4 row + pos holds chunk
-  // (pos - row / 4) mod 4 of the row) and 5 loads of B (256 consecutive floats of the stage's [16][320]
-  // area)
-  int a_voff[4], b_voff[5];
+  // (pos - row / 4) mod 4 of the row) and NTL loads of B (256 consecutive floats of the stage's
+  // [16][BN] area)
+  int a_voff[4], b_voff[T::NTL];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int inst = wave * 4 + j;
     const int row = inst * 16 + (lane >> 2);
     const int chunk = ((lane & 3) - (row >> 2)) & 3;
-    a_voff[j] = (int)(((int64_t)(m0 + row) * p.lda + chunk * 4) * 4);
+    const int arow = EDGE && m0 + row >= p.M ? p.M - 1 : m0 + row;
+    a_voff[j] = (int)(((int64_t)arow * p.lda + chunk * 4) * 4);
   }
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    const int inst = wave * 5 + j;
+  for (int j = 0; j < T::NTL; ++j) {
+    const int inst = wave * T::NTL + j;
     if (BPRE) {
-      // run inst = (term * 2 + k group) * 5 + run of 64 columns; lane = column inside the run
-      const int tk = inst / 5, run = inst % 5;
-      b_voff[j] = (((tk >> 1) * (int)prepared_kgroups(p.K) + (tk & 1)) * p.N + n0 + run * 64 + lane) * 16;
+      // run inst = (term * 2 + k group) * NTL + run of 64 columns; lane = column inside the run
+      const int tk = inst / T::NTL, run = inst % T::NTL;
+      int col = n0 + run * 64 + lane;
+      if (EDGE && col >= p.N) col = p.N - 1;
+      b_voff[j] = (((tk >> 1) * (int)prepared_kgroups(p.K) + (tk & 1)) * p.N + col) * 16;
     } else {
       const int f = inst * 256 + lane * 4;
       const int k = f / T::BN, pos = f % T::BN;
@@ -120,6 +157,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
       // gated store: the tile's ten column blocks are value 0, gate 0, value 1, ... of output columns
       // n0 / 2 + 32 j + l; the raw operand keeps its gate columns N / 2 further right
       if (GLU) col = ((n >> 5) & 1) * (p.N >> 1) + (n0 >> 1) + 32 * (n >> 6) + (n & 31);
+      if (EDGE && col >= p.N) col = p.N - 4;   // (four columns at a time, N a multiple of 4)
       b_voff[j] = k * ldb_bytes + col * 4;
     }
   }
@@ -127,7 +165,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
   // The loads of a wave land in consecutive kilobytes of LDS: the LDS address is M0 plus the instruction's immediate
   // offset, so a wave's A loads of a stage share one M0 and differ in the immediate; the immediate moves the memory
   // address too, which the lane offsets make up for (they stay non-negative: load j starts at least j KB into its
-  // operand).  The fifth B load is 4 KB further, beyond the immediate's range, and takes an M0 of its own.
+  // operand, at an edge as well: 64 rows of 32 k and BN columns are more than 3 KB).  The fifth B load is 4 KB further, beyond the immediate's range, and takes an M0 of its own.
 #pragma unroll
   for (int j = 1; j < 4; ++j) {
     a_voff[j] -= j * 1024;
@@ -137,18 +175,20 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int step = step_ < ksteps - 1 ? step_ : ksteps - 1;
     const int st = step_ % T::NS;
     const w512_lds_ptr al = (w512_lds_ptr)(smem + st * T::STAGE + wave * 4096);
-    const w512_lds_ptr bl = (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * 5120);
+    const w512_lds_ptr bl = (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * (T::NTL * 1024));
     const int as = step * T::BK * 4, bs = step * b_step;
     switch (j) {
-      case 0: __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, al, 16, a_voff[0], as, 0, 0); break;
-      case 1: __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, al, 16, a_voff[1], as, 1024, 0); break;
-      case 2: __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, al, 16, a_voff[2], as, 2048, 0); break;
-      case 3: __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, al, 16, a_voff[3], as, 3072, 0); break;
-      case 4: __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, bl, 16, b_voff[0], bs, 0, 0); break;
-      case 5: __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, bl, 16, b_voff[1], bs, 1024, 0); break;
-      case 6: __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, bl, 16, b_voff[2], bs, 2048, 0); break;
-      case 7: __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, bl, 16, b_voff[3], bs, 3072, 0); break;
-      default: __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * 5120 + 4096), 16, b_voff[4], bs, 0, 0); break;
+      case 0: w512_load0(ra, al, a_voff[0], as); break;
+      case 1: w512_load1(ra, al, a_voff[1], as); break;
+      case 2: w512_load2(ra, al, a_voff[2], as); break;
+      case 3: w512_load3(ra, al, a_voff[3], as); break;
+      case 4: w512_load0(rb, bl, b_voff[0], bs); break;
+      case 5: w512_load1(rb, bl, b_voff[1], bs); break;
+      case 6: w512_load2(rb, bl, b_voff[2], bs); break;
+      case 7: w512_load3(rb, bl, b_voff[3], bs); break;
+      default:
+        if constexpr (T::NTL == 5) w512_load0(rb, (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * 5120 + 4096), b_voff[4], bs);
+        break;
     }
   };
 
@@ -169,7 +209,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
   f32x16 acc[T::MT][T::NTL];
 
   // ---- software pipeline ---------------------------------------------------------------------
-  // Blocks are numbered t = stage * 5 + ni.  While the 12 MFMAs of block t issue, the raw B values of
+  // Blocks are numbered t = stage * NTL + ni.  While the 12 MFMAs of block t issue, the raw B values of
   // block t + 2 are read from LDS and those of block t + 1 (read one block earlier) are split; the A
   // values of row block ni of the next stage are read and split during block ni (0 .. 3), two loads of
   // a later stage are issued per block.
@@ -219,11 +259,11 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
   for (int mi = 0; mi < T::MT; ++mi)
 #pragma unroll
     for (int ni = 0; ni < T::NTL; ++ni) {
-      if (ni < 4) asm volatile("" : "+a"(acc[mi][ni]));
-      else asm volatile("" : "+v"(acc[mi][ni]));
+      if (ni < 4) w512_in_acc(acc[mi][ni]);
+      else w512_in_vec(acc[mi][ni]);
     }
   W512_FENCE();
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (18 & 0xF) | ((18 >> 4) << 14));   // vmcnt(18): stage 0 has landed
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * T::LOADS & 0xF) | ((2 * T::LOADS >> 4) << 14));   // vmcnt(2 stages): stage 0 has landed
   __builtin_amdgcn_s_barrier();
   {
 #pragma unroll
@@ -254,7 +294,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       // top of stage s + j: the own loads of stage s + j + 1 have landed, then everybody's
-      __builtin_amdgcn_s_waitcnt(0x0F70 | T::LOADS);                     // vmcnt(9)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | T::LOADS);                     // vmcnt(one stage)
       __builtin_amdgcn_s_barrier();
       const unsigned char* st0 = smem + ((s + j) % T::NS) * T::STAGE;       // this stage
       const unsigned char* st1 = smem + ((s + j + 1) % T::NS) * T::STAGE;   // the next one
@@ -282,7 +322,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
             else w512_mfma_v(a, b, acc[mi][ni]);
           }
         };
-        auto dl = [&](int k) {   // two load slots per block: 10 per stage, 9 used
+        auto dl = [&](int k) {   // two load slots per block: 2 NTL per stage, of which 4 + NTL are used
           const int slot = ni * 2 + k;
           if (slot < T::LOADS) issue1(s + j + T::NS - 1, slot);
         };
@@ -319,7 +359,7 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
           }
           if (BPRE && gi == 4) read_slot_hi(nxt, stn, n1);     // seven MFMAs before the next block's first
           if (BPRE && gi == 8) read_slot_lo(nxt, stn, n1);
-          // the stage's nine loads: two per block, apart from each other and in gaps that hold one half-split
+          // the stage's loads: two per block, apart from each other and in gaps that hold one half-split
           // (several loads in neighbouring gaps of one block cost 30 cycles each: counted)
           if (gi == 9) dl(0);
           if (gi == 10) dl(1);
@@ -408,7 +448,28 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     return;
   }
-  if constexpr (GLU == 1) {
+  if constexpr (GLU == 1 && NTL == 4) {
+    // Gated store of the 256-wide tile: a wave's four blocks are value 0, gate 0, value 1, gate 1 of its own 64 columns.
+    const int half = p.N >> 1, rows = p.M - (m0 + wm0);
+    const i32x4 re = make_rsrc((float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc, rows > 0 ? (int64_t)(rows < T::WTM ? rows : T::WTM) * ldc_bytes : 0);
+#pragma unroll
+    for (int pair = 0; pair < 2; ++pair) {
+      const int col = ((n0 + wn0) >> 1) + 32 * pair + el31, read = col < half ? col : half - 1;
+      const float bv = bias ? bias[read] : 0.f, bg = bias ? bias[half + read] : 0.f;
+      const int voff = col < half ? eg * 4 * ldc_bytes + col * 4 : 0x7FFFFFFF;
+#pragma unroll
+      for (int mi = 0; mi < T::MT; ++mi)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * q + e;
+            llvm_raw_buffer_store_f32((acc[mi][2 * pair][r] + bv) * gelu_value(acc[mi][2 * pair + 1][r] + bg), re,
+                                      (int)((unsigned)voff + (unsigned)((mi * 32 + q * 8 + e) * ldc_bytes)), 0, kLargeTileStoreAux);
+          }
+    }
+    return;
+  } else if constexpr (GLU == 1) {
     // Gated store: C[m][n0 / 2 + 32 j + l] = (value j + bias) x gelu(gate j + bias), j = 0 .. 4.  The
     // left wave of a row pair holds value 0, gate 0, value 1, gate 1, value 2, the right one gate 2,
     // value 3, gate 3, value 4, gate 4: pair 2 is the only one that spans two waves; the right wave
@@ -426,7 +487,9 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     __syncthreads();
     float* C = (float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc + c0;
-    const i32x4 rc = make_rsrc(C, 0x7FFFFFFF);
+    // (EDGE: the descriptor ends with the last row of C, the row offsets are part of the checked lane offset)
+    const int rows = p.M - (m0 + wm0);
+    const i32x4 rc = make_rsrc(C, !EDGE ? 0x7FFFFFFF : rows > 0 ? (int64_t)(rows < T::WTM ? rows : T::WTM) * ldc_bytes - c0 * 4 : 0);
     auto out_pair = [&](int pair, int vb, int gb, bool gate_in_lds) {
       const float bv = bias ? bias[c0 + 32 * pair + el31] : 0.f;
       const float bg = (bias && !gate_in_lds) ? bias[half + c0 + 32 * pair + el31] : 0.f;
@@ -439,7 +502,8 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * q + e;
             const float gl = gate_in_lds ? xbuf[(mi * 16 + r) * 64 + elane] : gelu_value(acc[mi][gb][r] + bg);
-            llvm_raw_buffer_store_f32((acc[mi][vb][r] + bv) * gl, rc, voff, (mi * 32 + q * 8 + e) * ldc_bytes, kLargeTileStoreAux);
+            const int roff = (mi * 32 + q * 8 + e) * ldc_bytes;
+            llvm_raw_buffer_store_f32((acc[mi][vb][r] + bv) * gl, rc, EDGE ? voff + roff : voff, EDGE ? 0 : roff, kLargeTileStoreAux);
           }
     };
     if ((wave & 1) == 0) {
@@ -454,6 +518,27 @@ __global__ __launch_bounds__(W512::NT) __attribute__((amdgpu_waves_per_eu(1, 1))
   }
   float* C = (float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc + n0 + wn0;
   const i32x4 rc = make_rsrc(C, 0x7FFFFFFF);
+  if (EDGE && (m0 + T::BM > p.M || n0 + T::BN > p.N)) {
+    // The descriptor ends with the last row of C and a lane past the last column points beyond any descriptor, so the
+    // stores need no branches (with a test per store such a tile took 28 us longer, and the launch with it).
+    const int rows = p.M - (m0 + wm0);
+    const i32x4 re = make_rsrc((float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc, rows > 0 ? (int64_t)(rows < T::WTM ? rows : T::WTM) * ldc_bytes : 0);
+#pragma unroll
+    for (int ni = 0; ni < T::NTL; ++ni) {
+      const int col = n0 + wn0 + ni * 32 + el31;
+      const float bv = bias ? bias[col < p.N ? col : p.N - 1] : 0.f;
+      const int voff = col < p.N ? eg * 4 * ldc_bytes + col * 4 : 0x7FFFFFFF;
+#pragma unroll
+      for (int mi = 0; mi < T::MT; ++mi)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            llvm_raw_buffer_store_f32(acc[mi][ni][4 * q + e] + bv, re, (int)((unsigned)voff + (unsigned)((mi * 32 + q * 8 + e) * ldc_bytes)), 0,
+                                      kLargeTileStoreAux);
+    }
+    return;
+  }
 #pragma unroll
   for (int ni = 0; ni < T::NTL; ++ni) {
     const float bv = bias ? bias[n0 + wn0 + ni * 32 + el31] : 0.f;

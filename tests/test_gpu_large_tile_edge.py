@@ -1,0 +1,64 @@
+"""The large-tile kernels whose tiles may hang over the edges of C (EDGE in csrc/cascmm_w512_kernel.h): plain and gated stores."""
+import pytest
+import torch
+
+from basedxl_amd import PreparedWeight, _lib, cascaded_lowp_matmul
+
+pytestmark = pytest.mark.gpu
+
+
+def _kernels(suffix=""):
+    names = [(vi, n) for vi, n in enumerate(_lib.variant_names()) if "_w512_edge_" in n and n.endswith(suffix)]
+    assert names
+    return names
+
+
+# (M, K, N): the fewest rows, one tile and a row or four columns more, a wave's half of the tile missing, several tiles;
+# the gaps between the rows of both sides, the rows and columns past the ends: NaNs that no result may see, 777 that stay
+@pytest.mark.parametrize("M, K, N", [(64, 32, 320), (256, 64, 320), (257, 64, 324), (385, 96, 460), (128, 32, 576), (1000, 160, 1284), (515, 64, 640)])
+def test_exact_on_integers_over_the_edges(gpu_device, M, K, N):
+    gen = torch.Generator().manual_seed(M + N)
+    ints = lambda *s: torch.randint(-90, 91, s, generator=gen)
+    A, B, bias = ints(M, K), ints(K, N), ints(N)
+    want = A @ B + bias
+    for vi, name in _kernels():
+        frame = torch.full((M + 4, K + 8), float("nan"), device="cuda")
+        frame[:M, :K] = A
+        a, b, biasd = frame[:M, :K], B.float().cuda(), bias.float().cuda()
+        prepared = name.endswith("_bpre")
+        w = PreparedWeight(b) if prepared else b
+        out = torch.full((M + 4, N if prepared else N + 8), 777.0, device="cuda")   # (a prepared weight's result is contiguous)
+        print(name, M, K, N, flush=True)
+        cascaded_lowp_matmul(a, w, bias=biasd, out=out[:M, :N], variant=vi)
+        assert torch.equal(out[:M, :N].cpu().long(), want), name
+        assert (out[M:] == 777.0).all() and (out[:, N:] == 777.0).all(), name
+
+
+# N: value and gate columns together; the 256 x 320 tile has the gated store where its columns are whole
+@pytest.mark.parametrize("M, K, N", [(64, 64, 320), (300, 64, 640), (257, 128, 448), (1000, 192, 1280)])
+def test_gated_store_over_the_edges(gpu_device, M, K, N):
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    a = torch.randn(M, K, device="cuda", generator=gen)
+    b, bias = torch.randn(K, N, device="cuda", generator=gen) * 0.2, torch.randn(N, device="cuda", generator=gen)
+    value, gate = (a.cpu().double() @ b.cpu().double() + bias.cpu().double()).chunk(2, dim=-1)
+    want = value * torch.nn.functional.gelu(gate)
+    w = PreparedWeight(b, glu=True)
+    ran = 0
+    for vi, name in _kernels("_bpre"):
+        if "320" in name and N % 320 != 0:
+            continue
+        out = torch.full((M + 4, N // 2), 777.0, device="cuda")
+        print(name, M, K, N, flush=True)
+        cascaded_lowp_matmul(a, w, bias=bias, out=out[:M], variant=vi)
+        # two bf16 terms drop lo.lo, 2^-18 of a product; value and gate each: 2^-16 of the result at most
+        assert ((out[:M].cpu().double() - want).norm() / want.norm()).item() < 2.0 ** -16, name
+        assert (out[M:] == 777.0).all(), name
+        ran += 1
+    assert ran
+
+
+def test_ragged_rows_of_a_wide_layer_take_the_large_tile():
+    l, names = _lib.lib(), _lib.variant_names()
+    pick = lambda M, K, N: names[l.cascmm_select_variant(M, N, K, K, N, N, 0, 0, 2, 0) & 0xFFFF]
+    assert pick(1976, 1280, 10240) == "t256x320x32_w512_edge_bf16x2_tri" and pick(4096, 4096, 4096) == "t256x256x32_w512_edge_bf16x2_tri"
+    assert pick(2048, 1280, 10240) == "t256x320x32_w512_bf16x2_tri" and "w512" not in pick(2048, 2048, 2048)
