@@ -228,6 +228,15 @@ def test_fast_kernels_are_not_chosen_when_offsets_would_overflow():
     assert big >= 0 and "generic" in names[big]
 
 
+def test_remembered_selection_tells_row_strides_at_the_limit_apart():
+    """Selections are remembered per problem: two row strides on either side of a kernel's 32-bit limit are two problems."""
+    l, names = _lib.lib(), _lib.variant_names()
+    pick = lambda lda, ldb: names[l.cascmm_select_variant(64, 64, 4096, lda, ldb, 64, 1, 1, 1, 0) & 0xFFFF]
+    assert "_h16_" in pick(4096, 150000)                  # 4096 rows of B span less than 2^31 bytes
+    assert "_h16_" not in pick(4096, 1 << 18)             # ... exactly 2^31
+    assert "_h16_" in pick(4096, 150000)
+
+
 def test_slot_kernels_of_the_three_term_fp16_cascade_are_sized_and_bounded():
     """The fp16 kernels that split both operands into operand slots first: the workspace the library asks for holds
     both operands' slots (6 bytes per element); they are offered only where a slot buffer stays below 2 GiB (32-bit
