@@ -129,8 +129,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.fast && fit < (any_rows ? FIT_DWORD : FIT_FAST)) return false;
   // K in whole 32-k steps, or a tail of whole 16-byte chunks (a weight less than one 64-k stage deep is not worth keeping
   // split: such a prepared operand is refused)
-  if (any_rows && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
-  if (v.fast && !any_rows && v.kind != KIND_H16 && q.K % v.BK != 0) return false;
+  if ((any_rows || v.kind == KIND_W512E) && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
+  if (v.fast && !any_rows && v.kind != KIND_H16 && (v.kind != KIND_W512E || q.glu) && q.K % v.BK != 0) return false;
   if (v.kind == KIND_SPLITK && (q.M > 5 * v.BM || q.K < 4 * v.BK)) return false;  // skinny: few row tiles, deep K
   if (v.kind == KIND_F8K64 && (q.products != CASCMM_PROD_TRI || q.K % v.BK != 0 || q.K == 0 || q.glu ||
                                f8k64_slot_bytes(q.M, q.K) > INT32_MAX || f8k64_slot_bytes(q.N, q.K) > INT32_MAX))
@@ -143,8 +143,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_W512 && (q.M % v.BM != 0 || q.N % v.BN != 0 || q.M * q.lda * 4 > INT32_MAX ||
                               (!q.bpre && q.K * q.ldb * 4 > INT32_MAX) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
-  if (v.kind == KIND_W512E && (q.M < W512_EDGE_ROWS || q.N < v.BN || (q.glu && v.BN == W512::BN && q.N % v.BN != 0) || q.K == 0 || q.M * q.lda * 4 > INT32_MAX ||
-                               (!q.bpre && q.K * q.ldb * 4 > INT32_MAX) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
+  if (v.kind == KIND_W512E && (q.M < W512_EDGE_ROWS || q.N < v.BN || (q.glu && v.BN == W512::BN && q.N % v.BN != 0) || q.lda < 32 || q.M * q.lda * 4 > INT32_MAX ||
+                               (!q.bpre && beyond_i32(q.K + 32, q.ldb, 4)) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
   if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
@@ -176,8 +176,8 @@ static const TunedCost kTuned[] = {
     {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 1.064, 4.69, 0.90, 0.80},
     {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 1.224, 6.84, 0.80, 0.70},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri", 3.200, 6.50, 0.70, 0.50},
-    // (the large tiles on every whole or ragged shape of 4992 x 2048 x 2048 to 4096^3 that was swept: partly filled rounds
-    // are faster than full ones, the board's power goes to fewer CUs: 64 of 256 tiles 0.62, 144 tiles 0.7, 192 tiles 0.88)
+    // (the large tiles: partly filled rounds are faster than full ones, the board's power goes to fewer CUs: 64 of 256
+    // tiles 0.62 of a round, 144 tiles 0.7, 192 tiles 0.88)
     {"t256x320x32_w512_bf16x2_tri", 5.65, 16.0, 0.50, 0.50},
     {"t256x320x32_w512_edge_bf16x2_tri", 5.65, 17.0, 0.50, 0.50},
     {"t256x256x32_w512_edge_bf16x2_tri", 4.60, 10.5, 0.45, 0.45},
@@ -289,12 +289,14 @@ static double h16_estimate_us(const VariantDesc& v, const Problem& q, double til
 }
 
 // The K-over-waves kernels (KIND_SLOTK): whole trips of four stages per wave, K in steps of 256; tiles over the edge of C
-// were 3 - 9 % slower than their whole neighbours (320 x 956 x 1792, 800 x 896 x 2688).
+// were 3 - 9 % slower than their whole neighbours (320 x 956 x 1792, 800 x 896 x 2688); over several rounds of
+// raw operands that is lost in the rest (2500^3 119 us, 131 on the tile it would leave it to), not with the weight prepared
+// (3000 x 2048 x 2048 85 us, 78 there).
 static double slotk_estimate_us(const TunedCost& t, const VariantDesc& v, const Problem& q, double tiles, int64_t k_per) {
   const double full = (double)(int64_t)(tiles / kNumCUs), rem = tiles - full * kNumCUs;
   const double tail = full == 0 ? t.tail_first : t.tail_later;
   const double rounds = full + (rem > 0 ? tail + (1.0 - tail) * rem / kNumCUs : 0.0);
-  const double edge = (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.05 : 1.0;
+  const double edge = (full == 0 || q.bpre) && (q.N % v.BN != 0 || q.M % v.BM != 0) ? 1.05 : 1.0;
   return edge * rounds * ((double)((k_per + 255) / 256 * 256) / 64.0 * t.step64_us + t.fixed_us);
 }
 

@@ -80,13 +80,15 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // NTL: column blocks of a wave; 5 is the 256 x 320 tile described above, 4 the same on 256 x 256 (sixteen blocks, all in
 // the accumulation registers).
 // EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
-// costs the loop nothing, and the stores past it go beyond the descriptor's end.
+// costs the loop nothing, and the stores past it go beyond the descriptor's end; the last stages may hang over K.
 // Measured (graph replay, raw / prepared weight; in brackets the fastest other kernel): 1976 x 1280 x 10240 on 256 x 320
 // 129.6 / 122.4 us (164.8 / 153.6), its gated form 126.1 (158.5); 7800 x 640 x 5120 139 / 134 (155 / 143); 1500 x 1280 x 10240
 // on 256 x 256 104 / 98 (134 / 110); 4096^3 316 / 297 (351 / 326) = 1.30 PFLOP/s of MFMA work, as on the wider tile: what is
-// left is the clock the board's power allows.
+// left is the clock the board's power allows.  K off its steps (in brackets the K-over-waves kernel, the only other one that
+// takes it): 3700^3 270 / 253 us (350 / 314), 8192 x 328 x 2560 47.5 / 45.3 (84 / 82), 3000 x 1100 x 9000 175 / 165 (239 / 219);
+// the test per load of A costs whole K nothing that can be measured (2048 x 1280 x 10240 131.4 / 123.7, without EDGE 130.0 / 123.2).
 // Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, N % 4 == 0; with the gated store N % 320 == 0 on the wider
-// tile), K % 32 == 0, lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
+// tile), K % 32 == 0 (EDGE: rows of A of whole 16-byte chunks, zeros between K and the last one's end), lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
 // aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets
 // inside a tile.
 // GLU = 1: the gated store (C has N / 2 columns, see GroupParams); a raw operand's gate columns are
@@ -120,24 +122,24 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   int tm, tn;
   tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int ksteps = p.K / T::BK;
+  const int ksteps = EDGE ? (p.K + 31) / 32 * 2 : p.K / T::BK;
   const int ldb_bytes = (int)p.ldb * 4;
 
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A[0], 0, 0x7FFFFFFF, 0x00020000);
   // (one record fewer than A's: with equal words the compiler keeps one copy of them and rebuilds this descriptor from it
   // in front of every B load)
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[0], 0, 0x7FFFFFFE, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[0], 0, EDGE && !BPRE ? (int)((((int64_t)p.K - 1) * p.ldb + p.N) * 4) : 0x7FFFFFFE, 0x00020000);
   // per wave and stage: 4 loads of A (16 rows x 64 bytes each; LDS position 4 row + pos holds chunk
   // (pos - row / 4) mod 4 of the row) and NTL loads of B (256 consecutive floats of the stage's
   // [16][BN] area)
+  const int a_chunk = ((lane & 3) - (lane >> 4)) & 3;   // (the same for every load: its first row is a multiple of 16)
   int a_voff[4], b_voff[T::NTL];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int inst = wave * 4 + j;
     const int row = inst * 16 + (lane >> 2);
-    const int chunk = ((lane & 3) - (row >> 2)) & 3;
     const int arow = EDGE && m0 + row >= p.M ? p.M - 1 : m0 + row;
-    a_voff[j] = (int)(((int64_t)arow * p.lda + chunk * 4) * 4);
+    a_voff[j] = (int)(((int64_t)arow * p.lda + a_chunk * 4) * 4);
   }
 #pragma unroll
   for (int j = 0; j < T::NTL; ++j) {
@@ -177,11 +179,14 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
     const w512_lds_ptr al = (w512_lds_ptr)(smem + st * T::STAGE + wave * 4096);
     const w512_lds_ptr bl = (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * (T::NTL * 1024));
     const int as = step * T::BK * 4, bs = step * b_step;
+    // EDGE: chunks past K come from beyond the buffer, as zeros (B's rows past K do by themselves: its buffer ends there, or
+    // its slots hold zeros)
+    auto av = [&](int jj) { return EDGE && a_chunk * 4 >= p.K - step * T::BK ? 0x7FFFFFFF : a_voff[jj]; };
     switch (j) {
-      case 0: w512_load0(ra, al, a_voff[0], as); break;
-      case 1: w512_load1(ra, al, a_voff[1], as); break;
-      case 2: w512_load2(ra, al, a_voff[2], as); break;
-      case 3: w512_load3(ra, al, a_voff[3], as); break;
+      case 0: w512_load0(ra, al, av(0), as); break;
+      case 1: w512_load1(ra, al, av(1), as); break;
+      case 2: w512_load2(ra, al, av(2), as); break;
+      case 3: w512_load3(ra, al, av(3), as); break;
       case 4: w512_load0(rb, bl, b_voff[0], bs); break;
       case 5: w512_load1(rb, bl, b_voff[1], bs); break;
       case 6: w512_load2(rb, bl, b_voff[2], bs); break;
