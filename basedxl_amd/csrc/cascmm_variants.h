@@ -217,13 +217,14 @@ int launch_w512(const GroupParams& p, hipStream_t stream) {
   return p.glu ? launch_w512_kernel<BPRE, 1>(p, stream) : launch_w512_kernel<BPRE, 0>(p, stream);
 }
 
-// ... whose tiles may hang over the edges of C
+// ... whose tiles may hang over the edges of C.  A raw B is loaded four columns at a time (N % 4 == 0); a prepared one column by
+// column, and so are all stores, so its N is anything.
 template <int BPRE, int NTL>
 int launch_w512_edge(const GroupParams& p, hipStream_t stream) {
   typedef W512Tile<NTL> T;
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_w512_kernel<BPRE, 0, NTL, 1>; return CASCMM_OK; }
   if (p.count != 1 || p.k_splits > 1 || p.glu == 2 || (p.glu && (!BPRE || (NTL == 5 && p.N % T::BN != 0)))) return CASCMM_ERR_BAD_VARIANT;
-  if (p.M < W512_EDGE_ROWS || p.N < T::BN || p.N % 4 != 0 || p.lda % 4 != 0 || p.lda < 32) return CASCMM_ERR_BAD_VARIANT;
+  if (p.M < W512_EDGE_ROWS || p.N < T::BN || (!BPRE && p.N % 4 != 0) || p.lda % 4 != 0 || p.lda < 32) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 32 : ((int64_t)p.K + 32) * p.ldb * 4) > 0x7FFFFFFF ||
       p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;

@@ -87,7 +87,7 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // left is the clock the board's power allows.  K off its steps (in brackets the K-over-waves kernel, the only other one that
 // takes it): 3700^3 270 / 253 us (350 / 314), 8192 x 328 x 2560 47.5 / 45.3 (84 / 82), 3000 x 1100 x 9000 175 / 165 (239 / 219);
 // the test per load of A costs whole K nothing that can be measured (2048 x 1280 x 10240 131.4 / 123.7, without EDGE 130.0 / 123.2).
-// Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, N % 4 == 0; with the gated store N % 320 == 0 on the wider
+// Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, raw B: N % 4 == 0; with the gated store N % 320 == 0 on the wider
 // tile), K % 32 == 0 (EDGE: rows of A of whole 16-byte chunks, zeros between K and the last one's end), lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
 // aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets
 // inside a tile.

@@ -1,0 +1,65 @@
+"""The automatic choice of a kernel and the kernels' own launch checks have to agree: a problem that the library selects a
+kernel for must not be refused by that kernel's launcher.
+
+The calls run in a child process that sees no GPU, on addresses that are never read: arguments are checked, a kernel is
+selected, its launcher checks them again, and then the launch itself fails for want of a device.  That status (LAUNCH) is what
+a call has to reach."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LAUNCH, BAD_FORMAT, ALIGNMENT, TOO_LARGE = -7, -4, -6, -9
+F32_BF16X2, FP16, BF16 = (0, 0, 2), (1, 1, 1), (2, 0, 1)          # (dtype, format, terms)
+
+CHILD = """
+import ctypes, json, sys
+from basedxl_amd import _lib
+l = _lib.lib()
+if l.cascmm_init() == 0:
+    raise SystemExit("a GPU is visible")
+A, B, C, WS = 1 << 40, 2 << 40, 3 << 40, 4 << 40
+out = []
+for c in json.load(sys.stdin):
+    M, K, N, (dt, fmt, terms) = c["M"], c["K"], c["N"], c["cascade"]
+    glu, n = c.get("glu", False), c.get("count", 1)
+    lda, ldb, ldc = c.get("lda", K), c.get("ldb", N), c.get("ldc", N // 2 if glu else N)
+    a = A + c.get("a_offset", 0)
+    need = l.cascmm_workspace_bytes(M, N, K, dt, fmt, terms, 0) * n if c.get("workspace", True) else 0
+    ws = (WS if need else None, need, None)
+    arr = lambda p: (ctypes.c_void_p * n)(*[p] * n)
+    if glu:
+        st = l.cascmm_gemm_prepared_glu(n, arr(a), arr(B), arr(C), None, M, N, K, lda, ldc, dt, fmt, terms, 0, None, None, -1)
+    elif c.get("prepared"):
+        st = l.cascmm_gemm_prepared(n, arr(a), arr(B), arr(C), None, M, N, K, lda, ldc, dt, fmt, terms, 0, None, *ws, -1)
+    elif n > 1:
+        st = l.cascmm_gemm_grouped(n, arr(a), arr(B), arr(C), None, M, N, K, lda, ldb, ldc, dt, fmt, terms, 0, None, *ws, -1)
+    else:
+        st = l.cascmm_gemm(a, B, C, None, M, N, K, lda, ldb, ldc, dt, fmt, terms, 0, None, *ws)
+    out.append(st)
+json.dump(out, sys.stdout)
+"""
+
+
+def statuses(cases):
+    env = dict(os.environ, PYTHONPATH=ROOT, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="")
+    r = subprocess.run([sys.executable, "-c", CHILD], input=json.dumps(cases), cwd=ROOT, env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout)
+
+
+def refused(cases):
+    """The cases that do not reach the launch, with their statuses."""
+    return [(c, st) for c, st in zip(cases, statuses(cases)) if st != LAUNCH]
+
+
+@pytest.mark.parametrize("step", [1, 2, 3])
+def test_prepared_widths_off_four(step):
+    """Weights kept split, two bf16 terms: any width, from a few rows to those that the large tiles are chosen for."""
+    cases = [dict(M=M, K=K, N=N + step, cascade=F32_BF16X2, prepared=True)
+             for M in (1, 40, 64, 200, 333, 1000, 2466, 4096, 8192) for K in (64, 72, 336, 640, 1280, 3712)
+             for N in (4, 256, 316, 320, 636, 1280, 2016, 3000, 5100, 10240)]
+    assert not refused(cases)

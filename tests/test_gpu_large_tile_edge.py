@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from basedxl_amd import PreparedWeight, _lib, cascaded_lowp_matmul
+from basedxl_amd import BasedXLLowPLinear, PreparedWeight, _lib, cascaded_lowp_matmul
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +36,33 @@ def test_exact_on_integers_over_the_edges(gpu_device, M, K, N):
         cascaded_lowp_matmul(a, w, bias=biasd, out=out[:M, :N], variant=vi)
         assert torch.equal(out[:M, :N].cpu().long(), want), name
         assert (out[M:] == 777.0).all() and (out[:, N:] == 777.0).all(), name
+
+
+# a prepared weight's width is anything: one column more than whole tiles, than a wave's half, one short of a tile; rows whole and not
+@pytest.mark.parametrize("M, K, N", [(256, 64, 641), (300, 72, 322), (64, 336, 1283), (513, 64, 481), (256, 96, 639)])
+def test_prepared_widths_off_four_are_exact_on_integers(gpu_device, M, K, N):
+    gen = torch.Generator().manual_seed(M + N)
+    ints = lambda *s: torch.randint(-90, 91, s, generator=gen)
+    A, B, bias = ints(M, K), ints(K, N), ints(N)
+    want = A @ B + bias
+    w = PreparedWeight(B.float().cuda())
+    for vi, name in _kernels("_bpre"):
+        out = torch.full((M + 4, N), 777.0, device="cuda")
+        print(name, M, K, N, flush=True)
+        cascaded_lowp_matmul(A.float().cuda(), w, bias=bias.float().cuda(), out=out[:M], variant=vi)
+        assert torch.equal(out[:M].cpu().long(), want), name
+        assert (out[M:] == 777.0).all(), name
+
+
+@pytest.mark.parametrize("M, K, N", [(2466, 336, 2019), (1000, 640, 2562)])
+def test_prepared_layer_of_odd_width(gpu_device, M, K, N):
+    """The layer on the kernel that is chosen for it.  Two bf16 terms of each factor drop lo.lo: 2^-18 of a product, 2^-16 of the
+    result at most."""
+    lin = torch.nn.Linear(K, N).to("cuda")
+    x = torch.randn(M, K, device="cuda")
+    want = torch.nn.functional.linear(x.double(), lin.weight.double(), lin.bias.double())
+    got = BasedXLLowPLinear(lin, prepared=True)(x)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2.0 ** -16
 
 
 # N: value and gate columns together; the 256 x 320 tile has the gated store where its columns are whole
