@@ -149,8 +149,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
-  // (32-bit byte offsets down A and, where it is raw, B, two stages past the end included; K in whole 16-byte chunks)
-  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || q.M * q.lda * 2 > INT32_MAX || (!q.bpre && beyond_i32(q.K + 64, q.ldb, 2))))
+  // (32-bit byte offsets down a raw B, two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
+  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (!q.bpre && beyond_i32(q.K + 64, q.ldb, 2))))
     return false;
   if (q.glu && !v.glu) return false;
   if (q.glu_slots && v.kind != KIND_W512) return false;
@@ -434,8 +434,8 @@ struct SelectKey {
   size_t ws_bytes;
   // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
   // some kernels: M lda, K ldb and 1024 ldc beyond 2^31 bytes << 3, 4, 5; lda below 32 << 7), glu_slots << 6,
-  // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12, the same limits as the kernels state them with
-  // stages past K or two-byte elements << 13, 14, 15
+  // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12, K ldb as the kernels state it with
+  // stages past K, of four-byte and two-byte elements << 13, 14
   int dtype, fmt, terms, products, count, flags;
   bool operator==(const SelectKey& o) const {
     return M == o.M && N == o.N && K == o.K && ws_bytes == o.ws_bytes && dtype == o.dtype && fmt == o.fmt &&
@@ -463,7 +463,7 @@ static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_byt
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
                       (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
                           (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0) | (beyond_i32(q.K + 32, q.ldb, 4) ? 8192 : 0) |
-                          (beyond_i32(q.M, q.lda, 2) ? 16384 : 0) | (beyond_i32(q.K + 64, q.ldb, 2) ? 32768 : 0)};
+                          (beyond_i32(q.K + 64, q.ldb, 2) ? 16384 : 0)};
   {
     std::lock_guard<std::mutex> lock(mu);
     auto it = memo.find(key);

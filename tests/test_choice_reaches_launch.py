@@ -63,3 +63,12 @@ def test_prepared_widths_off_four(step):
              for M in (1, 40, 64, 200, 333, 1000, 2466, 4096, 8192) for K in (64, 72, 336, 640, 1280, 3712)
              for N in (4, 256, 316, 320, 636, 1280, 2016, 3000, 5100, 10240)]
     assert not refused(cases)
+
+
+@pytest.mark.parametrize("cascade", [FP16, BF16])
+def test_sixteen_bit_activations_beyond_two_gib(cascade):
+    """16-bit layers with prepared weights, plain and gated, one problem and several: activations of any size."""
+    cases = [dict(M=M, K=K, N=N, cascade=cascade, prepared=True, glu=glu, count=count, lda=K + pad)
+             for M, K in ((4194304, 320), (9105865, 384), (26000000, 64), (1100000, 1000)) for N in (64, 640, 10240) for glu in (False, True)
+             for count in (1, 3) for pad in (0, 64)]
+    assert not refused(cases)

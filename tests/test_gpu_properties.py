@@ -350,6 +350,29 @@ def test_operands_beyond_two_gib_are_addressed_correctly(gpu_device):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_sixteen_bit_activations_beyond_two_gib(gpu_device, dtype):
+    """16-bit tensors of more than 2 GiB: weight raw, prepared and gated.  Integers whose sums stay below 2^8 (|a| <= 1, |b| <= 1, 64
+    products), so the plain results are exact; a gated one is the one of a copy of the rows, which the same kernel computes."""
+    dev, M, K, N = "cuda:0", 16777216 + 3, 72, 64
+    a = torch.zeros(M, K, dtype=dtype, device=dev)
+    assert a.numel() * 2 > 2 ** 31
+    rows = torch.tensor([0, 1, 255, 256, 14913080, 14913081, 15000000, M - 260, M - 2, M - 1], device=dev)   # (2 GiB: row 14913080)
+    a[rows] = torch.randint(-1, 2, (len(rows), K), device=dev).to(dtype)
+    b = torch.randint(-1, 2, (K, N), device=dev).to(dtype)
+    want = (a[rows].cpu().float() @ b.cpu().float()).to(dev)
+    for w in (b, PreparedWeight(b)):
+        got = cascaded_lowp_matmul(a, w)
+        assert torch.equal(got[rows].float(), want)
+        got[rows] = 0
+        assert not got.any()
+        del got
+    gated = PreparedWeight(b, glu=True)
+    assert torch.equal(cascaded_lowp_matmul(a, gated)[rows], cascaded_lowp_matmul(a[rows], gated))
+    del a
+    torch.cuda.empty_cache()
+
+
 def test_two_streams_do_not_share_scratch(gpu_device):
     """The library keeps no state; the Python operator keeps one workspace (K-split partials, re-laid
     16-bit weights) and one scale-search scratch PER STREAM.  Launches that need them, issued
