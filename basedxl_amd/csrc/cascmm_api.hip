@@ -149,8 +149,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
-  // (32-bit byte offsets down a raw B, two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
-  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (!q.bpre && beyond_i32(q.K + 64, q.ldb, 2))))
+  // (32-bit byte offsets down B, a raw one's two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
+  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (q.bpre ? beyond_i32((q.K + 63) / 64, q.N, 128) : beyond_i32(q.K + 64, q.ldb, 2))))
     return false;
   if (q.glu && !v.glu) return false;
   if (q.glu_slots && v.kind != KIND_W512) return false;
@@ -652,7 +652,7 @@ static int launch_prepare_fmt(const void* B, int K, int N, int64_t ldb, int fmt,
 // ---------------------------------------------------------------------------------------
 // Workgroups 0 .. a_blocks - 1: rows of A [M][K] (row stride lda) as rows of a_chunks 16-byte chunks, zeros past K; a
 // thread writes one chunk.  The others (16-bit elements as one term of their own format only): B [K][N] as operand
-// slots [8 ceil(K/64)][N], a thread the eight k of a column.  E: an unsigned type of the elements' size; bits are moved.
+// slots [4 ceil(K/32)][N], a thread the eight k of a column.  E: an unsigned type of the elements' size; bits are moved.
 template <typename E>
 __global__ __launch_bounds__(256) void relay_kernel(const E* __restrict__ A, int M, int K, int64_t lda, int a_chunks, u32x4* __restrict__ a_out,
                                                    int a_blocks, const E* __restrict__ B, int N, int64_t ldb, u32x4* __restrict__ b_out) {

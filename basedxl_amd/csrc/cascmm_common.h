@@ -291,9 +291,10 @@ __device__ __forceinline__ int exp_of_amax(unsigned bits) {
   return e;
 }
 
-// slot rows ([K/8][N] x 16 bytes) of one plane of a prepared right operand: K rounded up to whole 64-k stages, the
-// slots beyond K zero, so that a kernel's last stage reads zeros there whatever the left operand holds past K
-__host__ __device__ inline int64_t prepared_kgroups(int64_t K) { return (K / 64 + (K % 64 != 0 ? 1 : 0)) * 8; }
+// slot rows ([K/8][N] x 16 bytes) of one plane of a prepared right operand: K rounded up to whole 32-k stages, the
+// slots beyond K zero, so that the last stage of a kernel that reads two planes finds zeros there whatever the left
+// operand holds past K (of one plane, what lies beyond reads as zeros too: the buffer ends there)
+__host__ __device__ inline int64_t prepared_kgroups(int64_t K) { return (K / 32 + (K % 32 != 0 ? 1 : 0)) * 4; }
 
 struct GemmParams {
   const void* A;

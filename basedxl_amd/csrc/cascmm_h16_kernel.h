@@ -77,7 +77,7 @@ template <> struct H16Elem<CASCMM_FMT_BF16> { typedef __bf16 T; static constexpr
 template <> struct H16Elem<CASCMM_FMT_FP16> { typedef _Float16 T; static constexpr int DT = CASCMM_DT_F16; };
 
 // Host-checked: the rows of A start on dwords and are whole 16-byte chunks, zeros past K (K % 8 == 0, or padded), 512 of
-// them below 2 GiB; RAWB = 0: B prepared ([ceil(K / 64) * 8][N] slots, zeros beyond K) below 2 GiB; RAWB = 1: B [K][ldb] with
+// them below 2 GiB; RAWB = 0: B prepared (prepared_kgroups(K) x N slots, zeros beyond K), 2 GiB not reached with K rounded up to 64; RAWB = 1: B [K][ldb] with
 // N % 2 == 0 and rows on dwords, K * ldb * 2 below 2 GiB.  Any M and N: rows and columns past the edge are loaded as zeros or as
 // some other column's values and not stored.  grid.y: the problem of a group.  k_splits > 1: K in splits of k_per (a
 // multiple of 64), fp32 sums to the workspace instead of a result, see cascmm_ksplit.h.
@@ -104,9 +104,9 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 
   // A's buffer starts with the tile's first row, so A itself may be of any size: the offsets inside a tile stay below
   // 512 rows.  Rows past M read as zero (it ends with row M - 1), and so does everything past B's last row or slot row
-  const int kgs = (K + 63) / 64 * 8;
+  const int64_t kgs = prepared_kgroups(K);
   const int64_t a_bytes = ((int64_t)(p.M - 1 - m0) * p.lda + (K + 7) / 8 * 8) * 2;
-  const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
+  const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : kgs * p.N * 16;
   const int64_t b_first = RAWB ? (int64_t)k0 * p.ldb * 2 : (int64_t)(k0 / 8) * p.N * 16;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)p.A[prob] + (int64_t)m0 * p.lda + k0), 0,
                                                                      (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);

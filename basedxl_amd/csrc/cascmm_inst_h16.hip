@@ -20,7 +20,7 @@ static int launch_h16(const GroupParams& p, hipStream_t stream) {
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_h16_kernel<T, FMT, RAWB, 0>; return CASCMM_OK; }
   if (p.count < 1 || p.lda % 2 != 0 || (p.glu && !GLU)) return CASCMM_ERR_BAD_VARIANT;
   if (RAWB && (p.N % 2 != 0 || p.ldb % 2 != 0)) return CASCMM_ERR_BAD_VARIANT;
-  if (p.lda * 2 * 512 >= 0x7FFFFFFF || (RAWB ? ((int64_t)p.K + 64) * p.ldb * 2 : prepared_kgroups(p.K) * p.N * 16) > 0x7FFFFFFF)
+  if (p.lda * 2 * 512 >= 0x7FFFFFFF || (RAWB ? ((int64_t)p.K + 64) * p.ldb * 2 : ((int64_t)p.K + 63) / 64 * 128 * p.N) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
   if constexpr (GLU) {
     if (p.glu) return launch_h16_kernel<T, FMT, 0, 1>(p, stream);

@@ -35,7 +35,7 @@ struct SlotN {
 
 // Host-checked: the slot buffer 16-byte aligned and below 2 GiB, M * lda * 4 below 2 GiB, C rows addressable with 32-bit
 // byte offsets inside a tile.  TAIL as in cascmm_slotk_kernel (0: K % 32 == 0, K >= 32).
-// (SlotKParams: a = fp32 [M][lda], b_slots = [2][8 ceil(K/64)][N] x 16 bytes.)
+// (SlotKParams: a = fp32 [M][lda], b_slots = [2][4 ceil(K/32)][N] x 16 bytes.)
 template <int TAIL>
 __global__ __launch_bounds__(SlotN::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_slotn_kernel(const SlotKParams p) {
   typedef SlotN T;

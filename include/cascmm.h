@@ -142,7 +142,7 @@ int cascmm_gemm_grouped(int count, const void* const* A, const void* const* B, v
  * Prepared weights.  A Linear layer's weight is constant, so its split can be done once: the
  * counterpart of the one-time `W.T.contiguous().clone()` of basedxl/modules/lowp_linear.py:12.
  * cascmm_prepare_weight writes B[K,N] (leading dimension ldb, element type `dtype`) as MFMA
- * operand slots -- 16 bytes = 8 consecutive k of one column of one plane, [plane][8 ceil(K/64)][N]
+ * operand slots -- 16 bytes = 8 consecutive k of one column of one plane, [plane][4 ceil(K/32)][N]
  * (the slots past K are zero);
  * planes = terms (bf16, fp16) or ceil(terms/2) (fp8) -- into `out` (16-byte aligned, at least
  * cascmm_prepared_bytes(K, N, fmt, terms) bytes, allocated by the caller).  fp8: *tensor_exp

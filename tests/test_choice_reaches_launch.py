@@ -72,3 +72,14 @@ def test_sixteen_bit_activations_beyond_two_gib(cascade):
              for M, K in ((4194304, 320), (9105865, 384), (26000000, 64), (1100000, 1000)) for N in (64, 640, 10240) for glu in (False, True)
              for count in (1, 3) for pad in (0, 64)]
     assert not refused(cases)
+
+
+def test_prepared_buffers_of_whole_32_k_stages():
+    """A prepared weight whose K is a multiple of 32 holds its own slots and no more, so buffers kept from before any rounding fit, and
+    one just below 2 GiB is taken."""
+    from basedxl_amd import _lib
+    for K in (32, 96, 1056, 1280):
+        for fmt, terms, planes in ((0, 2, 2), (1, 3, 3), (0, 1, 1), (1, 1, 1)):
+            assert _lib.lib().cascmm_prepared_bytes(K, 332, fmt, terms) == planes * K * 332 * 2
+    assert not refused([dict(M=M, K=K, N=N, cascade=c, prepared=True) for M in (1, 300) for K, N, c in
+                        ((1056, 500368, F32_BF16X2), (224, 2166220, F32_BF16X2), (160, 2217588, (0, 0, 3)), (352, 1414720, (0, 2, 3)), (1056, 500369, F32_BF16X2))])

@@ -57,3 +57,32 @@ def test_each_kernel_with_a_tail_is_exact_on_integers(gpu_device, name, M, K, N)
     print("tail", name, (M, K, N), flush=True)
     got = cascaded_lowp_matmul(ad, PreparedWeight(bd) if name.endswith("_bpre") else bd, variant=_lib.variant_names().index(name))
     assert torch.equal(got.cpu().long(), a @ b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", [(70, 96, 163), (300, 72, 644), (129, 360, 1003), (65, 104, 64)])
+def test_nothing_past_a_prepared_buffer_is_read_into_the_result(gpu_device, dtype, M, K, N):
+    """Slots in the middle of a buffer of NaNs, K off the 64-k stages: every kernel for such a weight, exact on integers (16-bit
+    results: |x| <= 1, sums of at most 360 products below 2^8)."""
+    hi = 100 if dtype == torch.float32 else 1
+    g = torch.Generator().manual_seed(K + N)
+    a, b = (torch.randint(-hi, hi + 1, s, generator=g) for s in ((M, K), (K, N)))
+    w = PreparedWeight(b.to(dtype).to("cuda:0"))
+    frame = torch.full((w.slots.numel() + 2 * 128 * N * 16,), 0xFF, dtype=torch.uint8, device="cuda:0")
+    inner = frame[128 * N * 16:][:w.slots.numel()]
+    inner.copy_(w.slots)
+    moved = PreparedWeight.from_slots(inner, K, N, dtype, w.lowp, w.terms)
+    frame_a = torch.full((M, K + 8), float("nan"), dtype=dtype, device="cuda:0")
+    frame_a[:, :K] = a.to(dtype).to("cuda:0")
+    tag = {torch.float32: ("bf16x2_tri_bpre",), torch.float16: ("_h16_fp16x1_bpre_ioh",), torch.bfloat16: ("_h16_bf16x1_bpre_iob",)}[dtype]
+    ran = 0
+    for vi, name in [(-1, "automatic")] + [(vi, n) for vi, n in enumerate(_lib.variant_names()) if n.endswith(tag)]:
+        print("slots", dtype, (M, K, N), name, flush=True)
+        try:
+            got = cascaded_lowp_matmul(frame_a[:, :K], moved, variant=vi)
+        except _lib.CascmmError as e:
+            assert vi >= 0 and e.status == -8      # (that kernel takes whole stages or tiles only: refused on the host)
+            continue
+        assert torch.equal(got.cpu().double(), (a @ b).to(dtype).double()), name
+        ran += 1
+    assert ran >= 3                                # (of the fp32 ones the two K-over-waves kernels take any shape)
