@@ -244,6 +244,14 @@ class PreparedWeight:
         self.exp, self.slots = exp, slots
         return self
 
+    def check_slots(self) -> None:
+        """Raises where the buffer is not one of this weight's layout (one kept in a file from another layout, say): a
+        kernel reads what K, N and the cascade say."""
+        need = max(_lib.lib().cascmm_prepared_bytes(self.K, self.N, self.fmt, self.terms), 16)
+        have = self.slots.numel() * self.slots.element_size()
+        if have != need:
+            raise ValueError(f"the operand slots of a {self.K} x {self.N} weight of this cascade are {need} bytes, got {have}: prepare it again")
+
     def usable_with(self, a2: torch.Tensor, products: str = "tri") -> bool:
         """Whether the prepared kernels take this left operand: fp32, two bf16 terms: K a multiple of 8; other
         cascades and gated weights: K a multiple of 64, N of 4, rows 16-byte aligned; fp16 / bf16 tensors with a
@@ -294,6 +302,7 @@ def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, pro
         _check_device_tensor(a, "a")
         if (w.K, w.N, w.fmt, w.terms, w.glu) != (w0.K, w0.N, w0.fmt, w0.terms, w0.glu) or a.dtype != a_list[0].dtype:
             raise ValueError("grouped problems must share one shape, cascade and activation dtype")
+        w.check_slots()
         if a.dtype not in _DTYPES:
             raise TypeError(f"unsupported dtype {a.dtype}")
         a2 = _rows(a.reshape(-1, w.K))
@@ -695,6 +704,7 @@ def cascaded_lowp_matmul_glu_chained(a: torch.Tensor, w, *, bias: Optional[torch
     if prepared:
         if not w.glu or (w.lowp, w.terms) != ("bf16", 2):
             raise ValueError("the prepared weight must be a gated one of two bf16 terms")
+        w.check_slots()
         K, N, wptr = w.K, w.N, w.slots.data_ptr()
     else:
         _check_device_tensor(w, "w")

@@ -179,6 +179,8 @@ PyObject* prepared(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const void* bias;
     if (dt < 0 || fmt == CASCMM_FMT_FP8 || products < 0 || N <= 0 || !rows_of(*a, M, K, lda) || K != wk) Py_RETURN_NONE;
     if (!bias_of(args[2], *a, N, device, bias)) Py_RETURN_NONE;
+    const size_t slot_bytes = cascmm_prepared_bytes(wk, N, fmt, terms);
+    if (slots->nbytes() != (slot_bytes > 16 ? slot_bytes : 16)) Py_RETURN_NONE;   // (not this layout: the wrapper raises)
     const uintptr_t at0 = (uintptr_t)a->const_data_ptr();
     if (at0 % 16 != 0 || (size_t)lda * a->element_size() % 16 != 0) Py_RETURN_NONE;   // (the wrapper copies such rows)
     if (dt == CASCMM_DT_F32) {

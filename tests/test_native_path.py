@@ -35,6 +35,15 @@ def test_what_is_not_ordinary_is_left_to_the_wrapper():
         _native.init([])
 
 
+def test_slots_are_checked_against_the_layout():
+    w = PreparedWeight.from_slots(torch.zeros(2 * 12 * 64 * 16, dtype=torch.uint8), 96, 64, torch.float32, "bf16", 2)
+    w.check_slots()
+    for n in (16, 2 * 12 * 64 * 16 - 16, 2 * 16 * 64 * 16):
+        w.slots = torch.zeros(n, dtype=torch.uint8)
+        with pytest.raises(ValueError, match="slots"):
+            w.check_slots()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K,N", [(2, 1280, 320), (154, 320, 200), (512, 640, 640)])
@@ -65,6 +74,20 @@ def test_same_bits_as_the_wrapper(gpu_device, dtype, M, K, N):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_slots_of_another_layout_are_refused(gpu_device):
+    """A buffer that is shorter or longer than the weight's slots, as one kept in a file from another layout would be."""
+    w, x = PreparedWeight(torch.randn(96, 64, device="cuda:0")), torch.randn(40, 96, device="cuda:0")
+    want = cascaded_lowp_matmul(x, w)
+    for n in (-16, 16, 2 * 4 * 64 * 16):
+        slots = torch.zeros(w.slots.numel() + n, dtype=torch.uint8, device="cuda:0")
+        other = PreparedWeight.from_slots(slots, 96, 64, torch.float32, "bf16", 2)
+        assert _native.prepared(x, slots, None, 96, 64, other.fmt, 2, "tri", other.dt, False, 0) is None
+        with pytest.raises(ValueError, match="slots"):
+            cascaded_lowp_matmul(x, other)
+    assert torch.equal(cascaded_lowp_matmul(x, PreparedWeight.from_slots(w.slots, 96, 64, torch.float32, "bf16", 2)), want)
 
 
 @pytest.mark.gpu
