@@ -307,7 +307,6 @@ def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, pro
         _check_device_tensor(a, "a")
         if (w.K, w.N, w.fmt, w.terms, w.glu) != (w0.K, w0.N, w0.fmt, w0.terms, w0.glu) or a.dtype != a_list[0].dtype:
             raise ValueError("grouped problems must share one shape, cascade and activation dtype")
-        w.check_slots()
         if a.dtype not in _DTYPES:
             raise TypeError(f"unsupported dtype {a.dtype}")
         a2 = _rows(a.reshape(-1, w.K))
@@ -337,6 +336,8 @@ def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, pro
         biases = [_check_bias(bb, a2s[0], N) for bb in biases]   # (a gated weight takes all N = 2 * inner entries)
     if w0.fmt == _lib.FMT_FP8 and any(w.exp is None for w in w_list):
         raise ValueError("an fp8 PreparedWeight needs its tensor-scale exponent (exp)")
+    for w in w_list:
+        w.check_slots()
     arr = ctypes.c_void_p * n
     pa = arr(*[t.data_ptr() for t in a2s])
     pb = arr(*[w.slots.data_ptr() for w in w_list])
