@@ -258,19 +258,27 @@ class PreparedWeight:
             raise ValueError(f"the operand slots of a {self.K} x {self.N} weight of this cascade are {need} bytes, got {have}: prepare it again")
 
     def usable_with(self, a2: torch.Tensor, products: str = "tri") -> bool:
-        """Whether the prepared kernels take this left operand: fp32, two bf16 terms: K a multiple of 8; other
-        cascades and gated weights: K a multiple of 64, N of 4, rows 16-byte aligned; fp16 / bf16 tensors with a
-        weight of the same dtype kept as one term of that format: K a multiple of 8, rows on dwords (anything else
-        goes through the raw weight)."""
+        """Whether the prepared kernels take this left operand: K a multiple of 64, N of 4 and rows on 16-byte boundaries;
+        fp32 with two bf16 terms also K a multiple of 8, any N and any rows, fp16 / bf16 tensors with a weight of the same
+        dtype kept as one term of that format also K a multiple of 8, any N and rows on dwords (anything else goes through
+        the raw weight).  Most kernels for what lies off the first rule have 32-bit offsets, so there the library is asked about
+        this very shape: fp32 rows that span 2 GiB, say, or slots of that size may have none."""
         if not self.has_kernel(a2.dtype, products):
             return False
-        rows, lda = a2.shape[0], a2.stride(0)
-        if a2.dtype != torch.float32:
-            return (self.K % 8 == 0 and a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp
-                    and a2.data_ptr() % 4 == 0 and (rows <= 1 or lda % 2 == 0))
-        if (self.lowp, self.terms) == ("bf16", 2) and not self.glu and self.K % 8 == 0:
+        rows, lda, f32 = a2.shape[0], a2.stride(0), a2.dtype == torch.float32
+        if not f32 and not (a2.dtype == self.dtype and self.terms == 1 and default_cascade(a2.dtype)[0] == self.lowp):
+            return False
+        aligned = a2.data_ptr() % 16 == 0 and (rows <= 1 or lda % (4 if f32 else 8) == 0)
+        if self.K % 64 == 0 and self.N % 4 == 0 and aligned:
             return True
-        return self.K % 64 == 0 and self.N % 4 == 0 and a2.data_ptr() % 16 == 0 and (rows <= 1 or lda % 4 == 0)
+        if self.K % 8 != 0 or (f32 and (self.glu or (self.lowp, self.terms) != ("bf16", 2))):
+            return False
+        if not f32 and (a2.data_ptr() % 4 != 0 or (rows > 1 and lda % 2 != 0)):
+            return False
+        l = _lib.lib()
+        st = l.cascmm_select_variant_prepared(1, rows, self.N, self.K, lda if aligned and rows > 1 else self.K, self.N, _DTYPES[a2.dtype],
+                                              self.fmt, self.terms, _lib.PROD_BY_NAME[products])
+        return st >= 0 and l.cascmm_prepared_bytes(self.K, self.N, self.fmt, self.terms) < 2 ** 31
 
     def has_kernel(self, dtype: torch.dtype, products: str = "tri") -> bool:
         """Whether the library has a prepared-operand kernel for this weight's cascade with left

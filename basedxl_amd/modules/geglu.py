@@ -49,7 +49,10 @@ class BasedXLLowPGEGLU(nn.Module):
         return x.dtype == torch.float32 or (self.lowp, self.terms) == default_cascade(x.dtype)
 
     def _preparable(self) -> bool:
-        return self.in_features % (64 if self.weight.dtype == torch.float32 else 8) == 0 and self.inner % 32 == 0
+        if self.inner % 32 != 0:
+            return False
+        return self.in_features % 64 == 0 or (self.weight.dtype != torch.float32 and self.in_features % 8 == 0
+                                              and (self.in_features + 63) // 64 * 256 * self.inner < 2 ** 31)   # (slots in 64-k stages: 32-bit offsets)
 
     def prepare(self) -> None:
         """Prepare the gated weight now (needs the weight on the GPU); otherwise on the first eager call."""

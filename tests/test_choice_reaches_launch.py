@@ -83,3 +83,30 @@ def test_prepared_buffers_of_whole_32_k_stages():
             assert _lib.lib().cascmm_prepared_bytes(K, 332, fmt, terms) == planes * K * 332 * 2
     assert not refused([dict(M=M, K=K, N=N, cascade=c, prepared=True) for M in (1, 300) for K, N, c in
                         ((1056, 500368, F32_BF16X2), (224, 2166220, F32_BF16X2), (160, 2217588, (0, 0, 3)), (352, 1414720, (0, 2, 3)), (1056, 500369, F32_BF16X2))])
+
+
+def test_what_a_prepared_weight_says_it_takes_reaches_the_launch():
+    """``usable_with`` decides between the prepared and the raw weight of a layer: it must say no to what no prepared kernel
+    takes (fp32 activations of 2 GiB off the 64-k stages or of odd width, slots of 2 GiB), and go on saying yes to what one does."""
+    import torch
+    from basedxl_amd import PreparedWeight
+    names = {F32_BF16X2: (torch.float32, "bf16", 2), FP16: (torch.float16, "fp16", 1), BF16: (torch.bfloat16, "bf16", 1)}
+    taken, said_no = [], []
+    for cascade, (dtype, lowp, terms) in names.items():
+        for K, N in ((64, 64), (72, 64), (72, 63), (1280, 1282), (328, 640), (640, 640), (96, 3), (1056, 508402), (1048, 508402), (72, 7456540), (32, 16000000)):
+            w = PreparedWeight.from_slots(torch.empty(1, dtype=torch.uint8, device="meta"), K, N, dtype, lowp, terms)
+            for M in (1, 33, 4096, 500000, 1700000, 2000000, 9000000):
+                if M * N > 2 ** 42:
+                    continue                 # (more tiles than a launch has)
+                for pad in (0, 4, 8, 1 << 20):
+                    a = torch.empty_strided((M, K), (K + pad, 1), dtype=dtype, device="meta")
+                    c = dict(M=M, K=K, N=N, cascade=cascade, prepared=True, lda=K + pad if M > 1 else K)
+                    if (K + pad) % (4 if dtype == torch.float32 else 8) != 0:
+                        c["lda"] = K             # (such rows are copied)
+                    (taken if w.usable_with(a) else said_no).append(c)
+    assert len(taken) > 300
+    aligned = [c for c in taken if c["K"] % 64 == 0 and c["N"] % 4 == 0]      # (the rule of always; rows of a MiB apart had no kernel then either)
+    assert not [r for r in refused([c for c in taken if c not in aligned])]
+    assert not [r for r in refused(aligned) if r[0]["lda"] * 2048 < 2 ** 31 - 1]
+    # and no kernel goes unused: what it says no to has none
+    assert len(refused(said_no)) == len(said_no) > 20
