@@ -684,6 +684,15 @@ __global__ __launch_bounds__(256) void relay_kernel(const E* __restrict__ A, int
 // fp32 601 us, copied first 248; 37 x 2139 x 6528 fp16 238 against 15; and where nothing is copied, 333 x 456 x 211 18.6
 // against 6.4, 44 x 1124 x 1728 42.5 against 8.7.
 struct Relay { bool a = false, b = false; size_t a_bytes = 0, b_bytes = 0; int a_chunks = 0; };
+// the problem that is left once its operands are copied
+static Problem relayed(const Problem& q0, const Relay& r) {
+  Problem q = q0;
+  if (r.a) q.lda = r.a_chunks * (16 / (int64_t)dtype_size(q.dtype));
+  q.chunked = true;
+  q.bpre = r.b;
+  if (r.b) q.ldb = q.N;
+  return q;
+}
 static Relay relay_of(const Problem& q, int count, const void* const* A, const void* const* B) {
   Relay r;
   if (q.bpre || q.split_first || q.K == 0) return r;
@@ -702,18 +711,15 @@ static Relay relay_of(const Problem& q, int count, const void* const* A, const v
   r.a_chunks = (int)lines * 8;
   r.a_bytes = r.a ? f8k64_up(a_bytes) : 0;
   r.b_bytes = f8k64_up(b_bytes);
+  // (a copied B is a prepared one, which the bounds-checked kernels do not take: without a kernel for what is left, rows of A
+  // too far apart for 32-bit offsets for instance, nothing is copied and the operands are read where they lie)
+  if (r.b) {
+    const Problem e = relayed(q, r);
+    if (select_variant(e, row_fit(e, nullptr, nullptr), count) < 0) return Relay();
+  }
   return r;
 }
 static size_t relay_bytes(const Relay& r, int count) { return (size_t)count * (r.a_bytes + r.b_bytes); }
-// the problem that is left once its operands are copied
-static Problem relayed(const Problem& q0, const Relay& r) {
-  Problem q = q0;
-  if (r.a) q.lda = r.a_chunks * (16 / (int64_t)dtype_size(q.dtype));
-  q.chunked = true;
-  q.bpre = r.b;
-  if (r.b) q.ldb = q.N;
-  return q;
-}
 // what the partial results of the chosen kernel's K split take, at most `room`
 static size_t ksplit_need(const Problem& q, RowFit fit, size_t room) {
   int splits = 1;

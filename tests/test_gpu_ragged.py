@@ -86,3 +86,19 @@ def test_nothing_past_a_prepared_buffer_is_read_into_the_result(gpu_device, dtyp
         assert torch.equal(got.cpu().double(), (a @ b).to(dtype).double()), name
         ran += 1
     assert ran >= 3                                # (of the fp32 ones the two K-over-waves kernels take any shape)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N,lda", [(300, 64, 33, 1 << 21), (70, 72, 641, (1 << 21) + 2), (5, 100, 65, 1 << 22)])
+def test_rows_far_apart_next_to_a_weight_of_odd_width(gpu_device, dtype, M, K, N, lda):
+    """A raw 16-bit weight of odd width is copied into slots first, and slots have the kernels with 32-bit offsets only; rows of A
+    2^21 elements apart are beyond those (exact on integers)."""
+    g = torch.Generator().manual_seed(K + N)
+    a, b = (torch.randint(-1, 2, s, generator=g) for s in ((M, K), (K, N)))
+    wide = torch.empty(M * lda, dtype=dtype, device="cuda:0").as_strided((M, K), (lda, 1))
+    wide.copy_(a.to(dtype))
+    bd = b.to(dtype).to("cuda:0")
+    print("far apart", dtype, (M, K, N, lda), flush=True)
+    assert torch.equal(cascaded_lowp_matmul(wide, bd).cpu().long(), a @ b)
+    for o in cascaded_lowp_matmul_grouped([wide, wide], [bd, bd]):
+        assert torch.equal(o.cpu().long(), a @ b)
