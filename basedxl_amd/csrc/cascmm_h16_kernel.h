@@ -307,7 +307,8 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
       }
     }
     E* C = (E*)p.C[prob] + (int64_t)(m0 + wm0) * p.ldc + oc0;
-    const bool vec = (p.ldc & 7) == 0 && (no & 7) == 0 && ((uintptr_t)p.C[prob] & 15) == 0;
+    // (16-byte stores: 32-bit offsets over the wave's rows; others are addressed one by one)
+    const bool vec = (p.ldc & 7) == 0 && (no & 7) == 0 && ((uintptr_t)p.C[prob] & 15) == 0 && p.ldc * (2 * T::WTM) <= 0x7FFFFFFF;
     // rows past M fall beyond the end of the buffer and are dropped, columns past the last one are sent there too
     const int64_t c_bytes = ((int64_t)(p.M - 1 - m0 - wm0) * p.ldc + (no - oc0)) * 2;
     const i32x4 rc = make_rsrc(C, c_bytes < 0 ? 0 : c_bytes);

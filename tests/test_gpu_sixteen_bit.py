@@ -68,3 +68,21 @@ def test_the_gated_store_of_every_tile(gpu_device, dtype, M, K, N):
         assert bool(((got - want).abs() <= half_ulp * 1.001 * want.abs() + 256 * 4e-7).all()), name
         ran += 1
     assert ran >= 5
+
+
+@pytest.mark.parametrize("ldc", [9000000, 17000008])
+def test_rows_of_the_result_far_apart(gpu_device, ldc):
+    """A result that is a view into something wide: 128 rows of 9 million elements, 64 rows of 17 million, span more than 2 GiB."""
+    M, K, N, dtype = 257, 64, 72, torch.float16
+    g = torch.Generator().manual_seed(ldc)
+    a, b = _integers(g, M, K), _integers(g, K, N)
+    ad, bd = a.to(dtype).to("cuda:0"), b.to(dtype).to("cuda:0")
+    out = torch.empty(M * ldc, dtype=dtype, device="cuda:0").as_strided((M, N + 8), (ldc, 1))
+    for vi, name in _variants("_fp16x1_io16h") + [(-1, "automatic")]:
+        out.fill_(-77.0)
+        print("far apart", ldc, name, flush=True)
+        cascaded_lowp_matmul(ad, bd, out=out[:, :N], variant=vi)
+        assert torch.equal(out[:, :N].cpu().long(), a @ b), name
+        assert bool((out[:, N:] == -77.0).all()), name
+    del out
+    torch.cuda.empty_cache()
