@@ -433,7 +433,7 @@ struct SelectKey {
   int64_t M, N, K;
   size_t ws_bytes;
   // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
-  // some kernels: M lda, K ldb and 1024 ldc beyond 2^31 bytes << 3, 4, 5; lda below 32 << 7), glu_slots << 6,
+  // some kernels: M lda, K ldb, 1024 ldc and 256 ldc beyond 2^31 bytes << 3, 4, 5, 15; lda below 32 << 7), glu_slots << 6,
   // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12, K ldb as the kernels state it with
   // stages past K, of four-byte and two-byte elements << 13, 14
   int dtype, fmt, terms, products, count, flags;
@@ -462,7 +462,7 @@ static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_byt
   static std::unordered_map<SelectKey, SelectHit, SelectKeyHash> memo;
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
                       (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
-                          (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0) | (beyond_i32(q.K + 32, q.ldb, 4) ? 8192 : 0) |
+                          (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0) | (beyond_i32(q.ldc, 256, 1) ? 32768 : 0) | (beyond_i32(q.K + 32, q.ldb, 4) ? 8192 : 0) |
                           (beyond_i32(q.K + 64, q.ldb, 2) ? 16384 : 0)};
   {
     std::lock_guard<std::mutex> lock(mu);

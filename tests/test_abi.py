@@ -237,6 +237,16 @@ def test_remembered_selection_tells_row_strides_at_the_limit_apart():
     assert "_h16_" in pick(4096, 150000)
 
 
+def test_remembered_selection_tells_result_strides_at_the_limits_apart():
+    """... and so are two row strides of the result: the large tiles span 256 rows with 32 bits, the K-over-waves kernels 64."""
+    l, names = _lib.lib(), _lib.variant_names()
+    pick = lambda ldc: names[l.cascmm_select_variant_prepared(1, 200, 640, 1288, 1288, ldc, 0, 0, 2, 0) & 0xFFFF]
+    assert pick(3000000).startswith("k64x")               # 64 x 3000000 x 4 bytes: below 2^31
+    l2 = l.cascmm_select_variant_prepared(1, 200, 640, 1288, 1288, 9000000, 0, 0, 2, 0)
+    assert l2 < 0 or not names[l2 & 0xFFFF].startswith("k64x")
+    assert pick(3000000).startswith("k64x")
+
+
 def test_slot_kernels_of_the_three_term_fp16_cascade_are_sized_and_bounded():
     """The fp16 kernels that split both operands into operand slots first: the workspace the library asks for holds
     both operands' slots (6 bytes per element); they are offered only where a slot buffer stays below 2 GiB (32-bit
