@@ -772,6 +772,11 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
     if (fit == FIT_NONE) return CASCMM_ERR_ALIGNMENT;
     if (prepared_bytes(q.K, q.N, q.fmt, q.terms, q.glu) > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
   }
+  // (a prepared weight that no kernel takes with these rows: ALIGNMENT where they are off 16-byte boundaries, which all of
+  // the kernels take)
+  bool off16 = false;
+  for (int i = 0; i < count; ++i) off16 = off16 || !aligned_to(A[i], 16) || q.lda * (int64_t)es % 16 != 0;
+  const auto none = [&](int status) { return q.bpre && off16 ? (int)CASCMM_ERR_ALIGNMENT : status; };
 
   const auto& t = table();
   int splits = 1;
@@ -795,13 +800,13 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
       }
       return CASCMM_OK;
     }
-    if (variant < 0) return variant;
+    if (variant < 0) return none(variant);
   } else {
     splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
     variant &= 0xFFFF;
     if (variant >= (int)t.size()) return CASCMM_ERR_BAD_VARIANT;
     if (splits > (ksplit_kind(t[variant]) ? kMaxKSplits : kMaxTileSplits)) return CASCMM_ERR_BAD_VARIANT;
-    if (!variant_matches(t[variant], q, fit)) return CASCMM_ERR_BAD_VARIANT;
+    if (!variant_matches(t[variant], q, fit)) return none(CASCMM_ERR_BAD_VARIANT);
   }
   const VariantDesc& v = t[variant];
   if (exps_dyn && (v.kind != KIND_F8K64 || count != 1)) return CASCMM_ERR_BAD_VARIANT;

@@ -151,9 +151,10 @@ int cascmm_gemm_grouped(int count, const void* const* A, const void* const* B, v
  * cascmm_gemm_prepared runs `count` (1..8) GEMMs C[i] = A[i] . B[i] (+ bias[i]) of one shape whose
  * right operands are prepared buffers; arguments as cascmm_gemm_grouped, without ldb (the
  * workspace, which may be NULL, is used for the K split of under-filled single launches and
- * holds cascmm_workspace_bytes(...)).  Only the fast kernels exist for it: A must have 16-byte aligned rows
- * (CASCMM_ERR_ALIGNMENT otherwise), K be a multiple of 32 or 64 depending on the kernel (16-bit: of 8)
- * (CASCMM_ERR_BAD_FORMAT when no kernel fits), the prepared buffer below 2 GiB
+ * holds cascmm_workspace_bytes(...)).  Only the fast kernels exist for it: K a multiple of 32 or 64
+ * depending on the kernel (two bf16 terms: of 4, from 64 on; 16-bit: of 8) (CASCMM_ERR_BAD_FORMAT when
+ * no kernel fits), the rows of A on 16-byte boundaries (two bf16 terms and 16-bit: on dwords)
+ * (CASCMM_ERR_ALIGNMENT when no kernel takes others), the prepared buffer below 2 GiB
  * (CASCMM_ERR_TOO_LARGE).  The results equal cascmm_gemm's bit for bit when the same kernel
  * tile is used (same split, same order of accumulation).
  */

@@ -110,3 +110,14 @@ def test_what_a_prepared_weight_says_it_takes_reaches_the_launch():
     assert not [r for r in refused(aligned) if r[0]["lda"] * 2048 < 2 ** 31 - 1]
     # and no kernel goes unused: what it says no to has none
     assert len(refused(said_no)) == len(said_no) > 20
+
+
+def test_prepared_calls_say_what_is_wrong_with_the_rows():
+    """Rows off 16-byte boundaries that no prepared kernel takes are an alignment error, whatever else would be wrong with K."""
+    F32X3, FP16X3, FP8X3 = (0, 0, 3), (0, 1, 3), (0, 2, 3)
+    off = [dict(M=M, K=K, N=64, cascade=c, prepared=True, glu=glu, **rows) for M in (1, 200) for glu in (False, True)
+           for c, K in ((F32X3, 320), (F32X3, 24), (FP16X3, 64), (FP8X3, 44), (F32_BF16X2, 33))
+           for rows in (dict(lda=K + 4 - K % 4 + 2), dict(a_offset=4, lda=K + 4 - K % 4))]
+    off += [dict(M=200, K=K, N=64, cascade=c, prepared=True, **rows) for c in (FP16, BF16) for K in (64, 66) for rows in (dict(lda=71), dict(lda=72, a_offset=2))]
+    assert {st for st in statuses(off)} == {ALIGNMENT}
+    assert {st for st in statuses([dict(M=200, K=K, N=64, cascade=c, prepared=True, lda=64) for c in (F32X3, FP16X3, FP16) for K in (12, 60)])} == {BAD_FORMAT}
