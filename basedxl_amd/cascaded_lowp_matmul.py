@@ -25,7 +25,7 @@ _DTYPES = {torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16, torch.bfloat1
 
 #: persistent split-K / re-lay workspaces (contents need no initialisation), one per (device index,
 #: stream handle) for eager launches and one per device (key "capture") for launches recorded into a
-#: device graph
+#: device graph whose memory torch's allocator does not manage (:func:`_capture_workspace`)
 _workspaces: Dict[Tuple[int, object], torch.Tensor] = _lib.workspaces
 _MIN_WORKSPACE = 1 << 20
 
@@ -48,9 +48,9 @@ def _grow_capture_workspace(index: int, dev: torch.device, nbytes: int) -> torch
 
 
 def reserve_workspace(nbytes: int, device=None) -> None:
-    """Make sure the workspace that launches recorded into a device graph use holds ``nbytes``, so
-    that a capture allocates nothing.  Every eager launch does this for its own need, so a capture
-    that follows the usual eager warm-up of the same calls finds its workspace already there.  A
+    """Make sure the workspace that launches recorded into a device graph use where torch's allocator has no
+    pool for it (:func:`_capture_workspace`) holds ``nbytes``.  Every eager launch does this for its own need, so
+    a capture that follows the usual eager warm-up of the same calls finds its workspace already there.  A
     buffer that has to grow is replaced, never freed: graphs recorded against it keep replaying into
     memory that nothing else can own."""
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
@@ -60,19 +60,37 @@ def reserve_workspace(nbytes: int, device=None) -> None:
         _grow_capture_workspace(index, dev, nbytes)
 
 
+def _in_graph_pool(t: torch.Tensor) -> bool:
+    """Whether the memory of ``t``, allocated under capture, belongs to a graph's own pool."""
+    at, index = t.data_ptr(), t.device.index
+    for segment in torch.cuda.memory_snapshot():
+        if segment["device"] == index and segment["address"] <= at < segment["address"] + segment["total_size"]:
+            return tuple(segment.get("segment_pool_id", (0, 0))) != (0, 0)
+    return False
+
+
+def _capture_workspace(index: int, device: torch.device, nbytes: int) -> torch.Tensor:
+    """The workspace of a launch that is being recorded: a tensor of the graph's pool, taken and given back within the
+    call as the temporaries of any operator are.  The pool hands a block on to later calls of the same stream only, so
+    the branches of a graph, and graphs that are replayed side by side, never meet in one.  A capture that was not begun
+    through torch has no pool, its blocks would go on to eager tensors: there all launches share the one buffer of the
+    device that the eager warm-up has sized, and such graphs (and their branches) must not run concurrently."""
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if _in_graph_pool(ws):
+        return ws
+    ws = _workspaces.get((index, "capture"))
+    if ws is None or ws.numel() < nbytes:
+        ws = _grow_capture_workspace(index, device, nbytes)
+    return ws
+
+
 def _workspace(device: torch.device, stream: int, nbytes: int) -> Optional[torch.Tensor]:
-    """Launches on one stream are ordered, so they can share one buffer; launches replayed from
-    graphs share the per-device capture buffer (graphs that use it must not replay concurrently)."""
+    """Launches on one stream are ordered, so they can share one buffer.  Hold the result until the launch."""
     if nbytes == 0:
         return None
     index = device.index if device.index is not None else torch.cuda.current_device()
     if torch.cuda.is_current_stream_capturing():
-        ws = _workspaces.get((index, "capture"))
-        if ws is None or ws.numel() < nbytes:
-            # no eager warm-up came first: the buffer comes from the graph's own pool (an
-            # allocation inside the capture, but no fill: nothing is recorded for it)
-            ws = _grow_capture_workspace(index, device, nbytes)
-        return ws
+        return _capture_workspace(index, device, nbytes)
     reserve_workspace(nbytes, device)
     key = (index, stream)
     ws = _workspaces.get(key)

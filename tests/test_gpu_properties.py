@@ -312,6 +312,95 @@ def test_a_captured_graph_keeps_its_workspace_when_a_later_call_needs_a_larger_o
     assert _retired_capture_buffers
 
 
+def test_branches_and_graphs_do_not_meet_in_a_workspace(gpu_device, monkeypatch):
+    """Two branches of one captured graph, and two graphs replayed on two streams, run at the same time.  Whatever needs a
+    workspace (K splits of 16-bit and fp32 layers, raw and prepared; copied rows; slots) has to have one per branch and graph."""
+    from basedxl_amd import cascaded_lowp_matmul as fn
+    import sys
+    op = sys.modules[fn.__module__]
+    dev = "cuda:0"
+    g = torch.Generator(device=dev).manual_seed(11)
+    rn = lambda *s, dtype=torch.float32: torch.randn(*s, device=dev, generator=g).to(dtype)
+    w16x3 = rn(2008, 320) * 0.02
+    weights = [rn(3264, 880, dtype=torch.float16) * 0.02, rn(2008, 2176) * 0.02, rn(5117, 1281) * 0.02, rn(456, 211) * 0.02]
+    weights[0], weights[1] = PreparedWeight(weights[0]), PreparedWeight(weights[1])
+    inputs = lambda: [rn(7, 3264, dtype=torch.float16), rn(34, 2008), rn(30, 5117), rn(333, 456)]
+    run = lambda xs: [cascaded_lowp_matmul(x, w) for x, w in zip(xs, weights)] + [cascaded_lowp_matmul(xs[1], w16x3, lowp="fp16", terms=3)]
+    taken, real = [], op._workspace
+
+    def logged(device, stream, nbytes):
+        ws = real(device, stream, nbytes)
+        if ws is not None and torch.cuda.is_current_stream_capturing():
+            taken.append((label[0], stream, ws.data_ptr(), nbytes))
+        return ws
+
+    monkeypatch.setattr(op, "_workspace", logged)
+    label, graphs, branches = [None], [], []
+    side = torch.cuda.Stream()
+    for n in range(2):
+        xs = [inputs(), inputs()]
+        want = [run(x) for x in xs]                        # eager warm-up
+        torch.cuda.synchronize()
+        graph, label[0] = torch.cuda.CUDAGraph(), n
+        with torch.cuda.graph(graph):
+            side.wait_stream(torch.cuda.current_stream())
+            outs = [run(xs[0]), None]
+            with torch.cuda.stream(side):
+                outs[1] = run(xs[1])
+            torch.cuda.current_stream().wait_stream(side)
+        graphs.append(graph)
+        branches.append((xs, outs))
+    assert len({t[:2] for t in taken}) == 4 and len(taken) >= 12
+    for a in taken:
+        for b in taken:
+            assert a[:2] == b[:2] or a[2] + a[3] <= b[2] or b[2] + b[3] <= a[2], (a, b)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for rep in range(6):
+        for xs, _ in branches:
+            for x in xs[0] + xs[1]:
+                x.copy_(torch.randn(x.shape, device=dev, generator=g))
+        torch.cuda.synchronize()
+        for graph, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                graph.replay()
+        torch.cuda.synchronize()
+        for xs, outs in branches:
+            for x, out in zip(xs, outs):
+                for got, want in zip(out, run(x)):
+                    assert torch.equal(got, want), rep
+
+
+def test_a_capture_that_torch_did_not_begin_uses_the_kept_buffer(gpu_device):
+    """Begun through the runtime, a capture has no pool of its own: a temporary's block would go to the next eager tensor while
+    the graph goes on writing to it."""
+    import ctypes
+    from basedxl_amd.cascaded_lowp_matmul import _workspaces
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    x, w = torch.randn(7, 3264, device="cuda:0").half(), PreparedWeight(torch.randn(3264, 880, device="cuda:0").half())
+    out = torch.empty(7, 880, dtype=torch.float16, device="cuda:0")
+    want = cascaded_lowp_matmul(x, w)
+    torch.cuda.synchronize()
+    kept = _workspaces[(0, "capture")].data_ptr()
+    stream, graph, exe = torch.cuda.Stream(), ctypes.c_void_p(), ctypes.c_void_p()
+    handle = ctypes.c_void_p(stream.cuda_stream)
+    with torch.cuda.stream(stream):
+        assert hip.hipStreamBeginCapture(handle, 2) == 0                       # (relaxed)
+        try:
+            cascaded_lowp_matmul(x, w, out=out)
+        finally:
+            assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+        assert _workspaces[(0, "capture")].data_ptr() == kept
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for _ in range(3):
+            torch.cuda.synchronize()
+            canaries = [torch.full((8 << 20,), 0x5A, dtype=torch.uint8, device="cuda:0") for _ in range(4)]
+            out.fill_(float("nan"))
+            assert hip.hipGraphLaunch(exe, handle) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and all(bool((c == 0x5A).all()) for c in canaries)
+        assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 def test_operands_beyond_two_gib_are_addressed_correctly(gpu_device):
     """The fast kernels address rows through 32-bit offsets from a per-tile buffer descriptor, the
     bounds-checked ones through 64-bit pointers: a left operand and a result of 2.3 GB each (row offsets
