@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import importlib
 import os
+import warnings
 from ctypes import c_char_p, c_int, c_int32, c_int64, c_size_t, c_void_p, POINTER
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -121,6 +122,32 @@ def native():
         module.init(workspaces)
         _native = module
     return _native
+
+
+class _NoShortCut:
+    """What stands in for the extension where it does not load: takes no call."""
+
+    @staticmethod
+    def matmul(*_args):
+        return None
+
+    prepared = matmul
+
+
+_short_cut = None
+
+
+def short_cut():
+    """:func:`native`, or where it does not load (built against another torch, say) a stand-in that leaves every call to the
+    Python code, which needs libcascmm.so only: the same results, more host time per call."""
+    global _short_cut
+    if _short_cut is None:
+        try:
+            _short_cut = native()
+        except ImportError as e:
+            warnings.warn(f"eager calls take the Python path: {e}", RuntimeWarning, stacklevel=3)
+            _short_cut = _NoShortCut
+    return _short_cut
 
 
 def check(status: int, where: str) -> None:

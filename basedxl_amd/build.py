@@ -52,12 +52,14 @@ def _compile_native() -> str:
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
     obj = os.path.join(OBJ, "host", "native.o")
     os.makedirs(os.path.dirname(obj), exist_ok=True)
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
-           "-I", "/opt/rocm/include", "-I", sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, "host", "native.cpp"), "-o", obj]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, "host", "native.cpp"), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed on native.cpp:\n" + r.stderr[-4000:])
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
     return obj
 
 
@@ -77,7 +79,6 @@ def build(verbose: bool = True, jobs: int = 8) -> str:
     with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + 1)) as ex:
         native = ex.submit(_compile_native)
         objs = list(ex.map(_compile, srcs))
-        native_obj = native.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -88,7 +89,7 @@ def build(verbose: bool = True, jobs: int = 8) -> str:
         ctypes.CDLL(LIB)
     except OSError as e:
         raise RuntimeError(f"{LIB} was linked but does not load: {e}") from None
-    _link_native(native_obj)
+    _link_native(native.result())   # (behind the library, which also works without it)
     if verbose:
         print(f"built {LIB} from {len(srcs)} translation units, and {NATIVE}")
     return LIB

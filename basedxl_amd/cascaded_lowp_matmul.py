@@ -795,9 +795,9 @@ def cascaded_lowp_matmul(
     if out is None and variant < 0 and not dump_ptx and tensor_exps is None:
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         if type(b) is PreparedWeight:
-            y = _lib.native().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+            y = _lib.short_cut().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
         else:
-            y = _lib.native().matmul(a, b, bias, lowp, terms, products)
+            y = _lib.short_cut().matmul(a, b, bias, lowp, terms, products)
         if y is not None:
             return y
     if lowp is None or terms is None:

@@ -73,7 +73,7 @@ class BasedXLLowPGEGLU(nn.Module):
         pw = self._prepared
         if self.prepared and pw is not None and pw.device == self.weight.device and x.dtype == self.weight.dtype:
             # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
-            y = _lib.native().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, True, 0)
+            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, True, 0)
             if y is not None:
                 return y
         if not self.prepared and x.is_cuda and x.dtype == self.weight.dtype and gated_variant(

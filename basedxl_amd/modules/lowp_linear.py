@@ -54,9 +54,9 @@ class BasedXLLowPLinear(nn.Module):
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         pw = self._prepared_weight
         if not self.prepared or (x.dtype == torch.float32 and x.numel() < 32 * self.in_features):
-            y = _lib.native().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
+            y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
         elif pw is not None and pw.device == self.weight.device:
-            y = _lib.native().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 32)
+            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 32)
         else:
             y = None
         if y is not None:

@@ -25,6 +25,38 @@ def test_the_package_imports_before_anything_is_built(tmp_path):
     assert r.returncode == 0, r.stderr
 
 
+def test_without_the_extension_calls_take_the_python_path(tmp_path):
+    """An extension that does not load (a changed torch: here an empty file in its place) costs host time and a warning, no call."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    import basedxl_amd
+    src = os.path.dirname(basedxl_amd.__file__)
+    shutil.copytree(src, tmp_path / "basedxl_amd", ignore=shutil.ignore_patterns("_native.so", "build", "__pycache__"))
+    (tmp_path / "basedxl_amd" / "_native.so").write_bytes(b"")
+    code = """
+import warnings, torch, basedxl_amd as b
+from basedxl_amd import _lib
+op = lambda: b.cascaded_lowp_matmul(torch.randn(2, 64), torch.randn(64, 8))
+lin, glu = b.BasedXLLowPLinear(torch.nn.Linear(64, 8)), b.BasedXLLowPGEGLU(torch.nn.Linear(64, 64))
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    for call in (op, lambda: lin(torch.randn(2, 64)), lambda: glu(torch.randn(2, 64)), op):
+        try:
+            call()
+        except RuntimeError as e:
+            assert "no CPU fallback" in str(e), e       # (the wrapper's own words: it was reached)
+        else:
+            raise SystemExit("ran on the CPU")
+assert [w.category for w in seen] == [RuntimeWarning], [str(w.message) for w in seen]
+assert _lib.short_cut().prepared(1, 2, 3) is None and _lib.lib().cascmm_version() == 100
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, env={**os.environ, "PYTHONPATH": str(tmp_path)}, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
 def test_what_is_not_ordinary_is_left_to_the_wrapper():
     a, b = torch.randn(4, 8), torch.randn(8, 4)
     assert _native.matmul(a, b, None, None, None, "tri") is None                       # no GPU tensors
