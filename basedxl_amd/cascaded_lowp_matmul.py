@@ -227,7 +227,7 @@ class PreparedWeight:
         self.K, self.N = int(w.shape[0]), int(w.shape[1])
         self.shape = (self.K, self.N)
         self.lowp, self.terms, self.fmt = lowp, int(terms), _lib.FMT_BY_NAME[lowp]
-        self.dtype, self.device = w.dtype, w.device
+        self.dtype, self.device, self.dt = w.dtype, w.device, _DTYPES[w.dtype]
         self.glu = bool(glu)
         if self.glu and self.N % 64 != 0:
             raise ValueError("glu=True needs a weight whose width is a multiple of 64")
@@ -256,16 +256,18 @@ class PreparedWeight:
         self = cls.__new__(cls)
         self.K, self.N, self.shape = int(K), int(N), (int(K), int(N))
         self.lowp, self.terms, self.fmt = lowp, int(terms), _lib.FMT_BY_NAME[lowp]
-        self.dtype, self.device = dtype, slots.device
+        self.dtype, self.device, self.dt = dtype, slots.device, _DTYPES[dtype]
         self.glu = bool(glu)
         self.out_features = self.N // 2 if self.glu else self.N
         self.exp, self.slots = exp, slots
         return self
 
-    @property
-    def dt(self) -> int:
-        """The library's code of the weight's dtype (derived, so that objects pickled without it have it too)."""
-        return _DTYPES[self.dtype]
+    def __getattr__(self, name: str):
+        # (only asked for what is missing: objects pickled before they held the code of their dtype)
+        if name == "dt":
+            self.dt = _DTYPES[self.dtype]
+            return self.dt
+        raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
 
     def check_slots(self) -> None:
         """Raises where the buffer is not one of this weight's layout (one kept in a file from another layout, say): a

@@ -104,12 +104,12 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 
   // A's buffer starts with the tile's first row, so A itself may be of any size: the offsets inside a tile stay below
   // 512 rows.  Rows past M read as zero (it ends with row M - 1), and so does everything past B's last row or slot row
-  const int64_t kgs = prepared_kgroups(K);
-  const int64_t a_bytes = ((int64_t)(p.M - 1 - m0) * p.lda + (K + 7) / 8 * 8) * 2;
-  const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : kgs * p.N * 16;
+  const int kgs = (K + 31) / 32 * 4;   // prepared_kgroups
+  const int lda = (int)p.lda, rows = p.M - m0 < T::BM ? p.M - m0 : T::BM;
+  const int a_bytes = ((rows - 1) * lda + (K + 7) / 8 * 8) * 2;
+  const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
   const int64_t b_first = RAWB ? (int64_t)k0 * p.ldb * 2 : (int64_t)(k0 / 8) * p.N * 16;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)p.A[prob] + (int64_t)m0 * p.lda + k0), 0,
-                                                                     (int)(a_bytes > 0x7FFFFFFF ? 0x7FFFFFFF : a_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)p.A[prob] + (int64_t)m0 * lda + k0), 0, a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)p.B[prob] + b_first), 0, (int)b_bytes, 0x00020000);
 
   // ---- loads: this wave's kilobytes of a stage ----
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     const int row = (wave * T::A_LOADS + j) * (64 / T::KG) + lane / T::KG;
     const int chunk = (lane % T::KG - (row >> RSH)) & (T::KG - 1);
     a_k[j] = chunk * 8;
-    a_voff[j] = m0 + row < p.M ? (int)(((int64_t)row * p.lda + chunk * 8) * 2) : 0x7FFFFFFF;
+    a_voff[j] = row < rows ? (row * lda + chunk * 8) * 2 : 0x7FFFFFFF;
   }
   // B prepared: slot (k group, column) at (kg * BN + column) * 16.  B raw: row k at 2 BN k bytes, its 16-byte chunks
   // (8 columns) permuted by an XOR so that the four rows of a transposing read lie on different banks
