@@ -867,8 +867,10 @@ def cascaded_lowp_matmul(
         # the reference writes the PTX of the kernel it launched (cascaded_lowp_matmul.py:170-171);
         # here the file holds the gfx950 assembly of the GEMM kernel that ran
         l = _lib.lib()
-        v = variant if variant >= 0 else l.cascmm_select_variant(
-            M, N, K, a2.stride(0), b.stride(0), out2.stride(0), _DTYPES[a.dtype], fmt, terms, prod)
+        dt = _DTYPES[a.dtype]
+        v = variant if variant >= 0 else l.cascmm_call_variant(
+            a2.data_ptr(), b.data_ptr(), M, N, K, a2.stride(0) if M > 1 else max(K, 1), b.stride(0) if K > 1 else max(N, 1),
+            out2.stride(0) if M > 1 else max(N, 1), dt, fmt, terms, prod, _workspace_bytes(M, N, K, dt, fmt, terms, prod))
         with open("dump.ptx", "w") as f:
             f.write(kernel_listing(v & 0xFFFF))
 

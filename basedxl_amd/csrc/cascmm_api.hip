@@ -1222,6 +1222,24 @@ int cascmm_select_variant(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t 
   return select_for_shape(q, 1);
 }
 
+int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                        int dtype, int fmt, int terms, int products, size_t workspace_bytes) {
+  Problem q{M, N, K, lda, ldb, ldc, dtype, fmt, terms, products};
+  const int st = check_problem(q);
+  if (st != CASCMM_OK) return st;
+  q.chunked = chunked_by_k(q);
+  // (as gemm_impl and gemm_on_rows go about it)
+  const Relay r = relay_of(q, 1, &A, &B);
+  if ((r.a || r.b) && workspace_bytes >= relay_bytes(r, 1)) {
+    const Problem e = relayed(q, r);
+    return select_variant(e, row_fit(e, r.a ? nullptr : A, r.b ? nullptr : B), 1, workspace_bytes - relay_bytes(r, 1));
+  }
+  const RowFit fit = row_fit(q, A, B);
+  Problem e;
+  const int v = select_rounded_up(q, fit, workspace_bytes, &e);
+  return v >= 0 ? v : select_variant(q, fit, 1, workspace_bytes);
+}
+
 int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                                   int dtype, int fmt, int terms, int products) {
   if (count < 1 || count > kMaxGroup) return CASCMM_ERR_BAD_SHAPE;

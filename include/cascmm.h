@@ -249,10 +249,16 @@ int cascmm_gemm_chained(const void* Aslots, const void* Bslots, void* C, const v
 size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fmt, int terms,
                               int products);
 
-/* Variant the automatic selection would run for this problem (index), or a negative status. */
+/* Variant the automatic selection would run for this problem (index), or a negative status: on rows of whole
+ * 16-byte chunks that start on 16-byte boundaries, without what a call does to others first (rows copied into
+ * the workspace, K of the three-term fp8 / fp16 cascades rounded up to whole stages). */
 int cascmm_select_variant(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                           int dtype, int fmt, int terms, int products);
-/* Same for a grouped launch of `count` problems (the choice depends on how many tiles the
+/* Variant that cascmm_gemm launches for these very operands with this much workspace (0: none), or a negative status:
+ * the GEMM kernel itself, where copies, splits or a reduction go with it.  Nothing is read or launched. */
+int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                        int64_t ldc, int dtype, int fmt, int terms, int products, size_t workspace_bytes);
+/* Same as cascmm_select_variant for a grouped launch of `count` problems (the choice depends on how many tiles the
  * group has in total). */
 int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                   int64_t ldc, int dtype, int fmt, int terms, int products);

@@ -187,6 +187,28 @@ def test_scale_search_argument_validation():
     assert l.cascmm_tensor_exps(ok, 2 ** 31, 4, 4, 0, None, ok, ok, None) == -9
 
 
+def test_the_kernel_of_a_call_is_the_one_that_is_launched():
+    """What `dump_ptx=True` lists: the kernel behind copies of rows, a rounded-up K and rows on dwords, or the bounds-checked one where
+    a call brings no workspace for them."""
+    l, names = _lib.lib(), _lib.variant_names()
+    A, B = 1 << 40, 2 << 40
+
+    def kernel(M, K, N, cascade=(0, 0, 2), a=0, b=0, lda=0, ldb=0, workspace=True):
+        args = (M, N, K, lda or K, ldb or N, N, *cascade, 0)
+        return names[l.cascmm_call_variant(A + a, B + b, *args, l.cascmm_workspace_bytes(M, N, K, *cascade, 0) if workspace else 0) & 0xFFFF]
+
+    for shape in ((2048, 1280, 1280), (154, 2048, 1280), (2048, 1280, 10240)):                   # nothing special: the selection's answer
+        v = l.cascmm_select_variant(shape[0], shape[2], shape[1], shape[1], shape[2], shape[2], 0, 0, 2, 0)
+        assert kernel(*shape) == names[v & 0xFFFF]
+    assert "_wavek_" in kernel(333, 456, 211) and "_wavek_" in kernel(333, 456, 211, a=4, b=4, lda=457)
+    assert "generic" not in kernel(44, 1124, 1728)                                               # K in whole 16-byte chunks
+    assert "generic" not in kernel(7488, 1061, 3192) and "generic" in kernel(7488, 1061, 3192, workspace=False)   # rows copied first
+    assert "_f16" in kernel(3740, 1090, 992, (0, 1, 3)) and "_f8" in kernel(2048, 1300, 1280, (0, 2, 3))   # K rounded up
+    assert "_h16_" in kernel(37, 2139, 6528, (1, 1, 1)) and "_bpre_" in kernel(64, 640, 641, (1, 1, 1))     # rows, or B, copied
+    assert "generic" in kernel(64, 640, 641, (1, 1, 1), workspace=False)
+    assert l.cascmm_call_variant(A, B, 4, 4, 4, 3, 4, 4, 0, 0, 2, 0, 0) == -2
+
+
 def test_cpu_tensors_are_rejected_without_fallback():
     import torch
     from basedxl_amd import cascaded_lowp_matmul
