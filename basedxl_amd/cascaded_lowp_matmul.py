@@ -262,12 +262,10 @@ class PreparedWeight:
         self.exp, self.slots = exp, slots
         return self
 
-    def __getattr__(self, name: str):
-        # (only asked for what is missing: objects pickled before they held the code of their dtype)
-        if name == "dt":
-            self.dt = _DTYPES[self.dtype]
-            return self.dt
-        raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
+    def __setstate__(self, state: dict) -> None:
+        # (objects pickled before they held the library's code of their dtype)
+        self.__dict__.update(state)
+        self.dt = _DTYPES[self.dtype]
 
     def check_slots(self) -> None:
         """Raises where the buffer is not one of this weight's layout (one kept in a file from another layout, say): a

@@ -71,13 +71,12 @@ def test_prepared_weights_pickled_before_the_short_cut_still_load():
     """A pickled model holds its layers' PreparedWeight objects as plain attributes: those of before have no dtype code."""
     import pickle
     w = PreparedWeight.from_slots(torch.zeros(2 * 8 * 16 * 16, dtype=torch.uint8), 64, 16, torch.float32, "bf16", 2)
-    old = {k: v for k, v in w.__dict__.items() if k != "dt"}
-    assert set(old) == {"K", "N", "shape", "lowp", "terms", "fmt", "dtype", "device", "glu", "out_features", "exp", "slots"}
-    again = PreparedWeight.__new__(PreparedWeight)
-    again.__dict__.update(pickle.loads(pickle.dumps(old)))
+    del w.__dict__["dt"]
+    assert set(w.__dict__) == {"K", "N", "shape", "lowp", "terms", "fmt", "dtype", "device", "glu", "out_features", "exp", "slots"}
+    again = pickle.loads(pickle.dumps(w))
     with pytest.raises(RuntimeError, match="no CPU fallback"):          # (as far as a CPU tensor comes: the short cut has read its arguments)
         cascaded_lowp_matmul(torch.randn(2, 64), again)
-    assert pickle.loads(pickle.dumps(w)).dt == w.dt == _lib.DT_F32
+    assert pickle.loads(pickle.dumps(again)).dt == again.dt == _lib.DT_F32
 
 
 def test_slots_are_checked_against_the_layout():
