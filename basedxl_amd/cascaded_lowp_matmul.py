@@ -207,8 +207,8 @@ class PreparedWeight:
     kept as MFMA operand slots; ``cascaded_lowp_matmul(a, prepared)`` then splits only ``a``.
     The arithmetic is the same as with the raw weight (same split, same products).  Kernels for
     prepared weights exist for bf16 x 2, bf16 x 3, fp16 x 3 and fp8 x 3 with the 'tri' product set and
-    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4 (two bf16 terms and 16-bit: K of 8); the
-    product with any other combination fails with CascmmError (use the raw weight there).
+    for fp16 / bf16 tensors as one term of their own format, K a multiple of 64 and N of 4 (two bf16 terms and 16-bit:
+    K of 8, any N); the product with any other combination may fail with CascmmError (use the raw weight there).
 
     ``glu=True``: ``w`` is the ``[in, 2 * inner]`` weight of a gated projection (diffusers' GEGLU:
     ``h = x @ w + b; y = h[:, :inner] * gelu(h[:, inner:])``); its columns are stored so that a

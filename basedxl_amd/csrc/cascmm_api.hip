@@ -301,9 +301,9 @@ static double slotk_estimate_us(const TunedCost& t, const VariantDesc& v, const 
 }
 
 // K split over workgroups (cascmm_ksplit.h): where the tiles leave CUs idle, `estimate(tiles, k of a split)` with the
-// chip filled against the second launch and the partial results, written and read back.  Measured: 7 x 3264 x 880 fp16
-// 14.8 -> 6.8 us in eight splits, 256 x 5120 x 1280 23.0 -> 14.0 in five, 34 x 2008 x 2176 fp32 prepared 15.5 -> 9.7 in
-// eight, 154 x 2048 x 2560 raw 18.4 -> 15.5 in four.  Below 11 us the second launch, 3 us of the
+// chip filled against the second launch and the partial results, written and read back.  Measured (graph replay): 7 x 3264 x 880
+// fp16 14.8 -> 6.2 us in thirteen splits, 256 x 5120 x 1280 23.0 -> 14.0 in six, 34 x 2008 x 2176 fp32 prepared 15.5 -> 9.5 in
+// eight, 154 x 2048 x 2560 raw 18.4 -> 15.6 in four.  Below 11 us the second launch, 3 us of the
 // host's time, costs an eager call more than it gives (keys and values 40 x 1664 x 768 fp16 8.4 -> 11.5 us).
 template <class F>
 static double ksplit_best(const Problem& q, int count, double tiles, size_t ws_bytes, double launch_us, double bytes_per_us, int* splits, F estimate) {

@@ -13,12 +13,13 @@
 //
 // What bounds it: one product per element leaves three times fewer MFMA cycles per byte than the two-term
 // cascade, so a tile is as good as its bytes per multiply-add: (BM + BN) x 2 bytes per k through the CU's share
-// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared, graph replay; in brackets the
-// copy-only LDS kernels with producer waves that these replaced): 2048 x 1280 x 10240 on 256 x 320 52.1 us (62.1), its
-// loop at 1320 TFLOP/s, which is the board's power with random operands (zeros: a third faster); 4096^3 on
-// 256 x 256 115 us (135); 8192 x 2560 x 640 on 128 x 160 29.4 us (33.5); 2048^3 on 128 x 128 20.8 us (23.0), its loop
-// at 66 bytes per ns and CU from the L2s; 2048 x 1280 x 1280 12.2 us (14.0); 512 x 1280 x 1280 on 64 x 64 7.6 us (9.5).
-// With B raw (no re-lay pass: 2048^3 28.7 -> 23.5 us) the transposing reads cost 3 - 16 %.
+// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared, graph replay in the steady state, two boxes;
+// in brackets the copy-only LDS kernels with producer waves that these replaced, on another one): 2048 x 1280 x 10240 on
+// 256 x 320 57.4 and 59.5 us (62.1; 52.1 here on that box), its loop at the board's power with random operands (zeros: a
+// third faster); 4096^3 on 256 x 256 115 and 119 us (135); 8192 x 2560 x 640 on 128 x 160 27.8 and 29.4 us (33.5); 2048^3 on
+// 128 x 128 18.8 and 21.2 us (23.0), its loop at 66 bytes per ns and CU from the L2s; 2048 x 1280 x 1280 11.2 us (14.0);
+// 512 x 1280 x 1280 on 64 x 64 6.5 us (9.5).  With B raw (no re-lay pass: 2048^3 20.7 and 21.8 us, 28.7 with it) the transposing
+// reads cost 3 - 16 %.  Kernel times and counters: profiles/cascmm_h16_kernel_fp16.txt.
 //
 // The MFMAs take their operands swapped (B first): a lane then holds ONE ROW of C and four consecutive columns
 // per register quad, which are packed to 8 bytes, turned row-wise through LDS and stored 16 bytes per lane.
@@ -94,23 +95,29 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   const int wk = wave / (T::WM * T::WN), wmn = wave % (T::WM * T::WN);
   const int wm0 = (wmn / T::WN) * T::WTM, wn0 = (wmn % T::WN) * T::WTN;
   const int prob = blockIdx.y;
+  // The arguments that A's first loads need, all requested here: left to themselves the reads sink to their uses and wait one
+  // behind the other, which with a descriptor per tile was 0.2 us of a call with new operands (2048 x 1280 x 1280, three
+  // weights in turn: 12.52 us, so 12.26; 512 x 1280 x 1280 6.9 and 6.7).  N among them too: 12.13 and 7.0.
+  int tiles_m = p.tiles_m, tiles_n = p.tiles_n, k_splits = p.k_splits, M = p.M, K_all = p.K, k_per = p.k_per, lda = (int)p.lda;
+  const void *A = p.A[prob], *B = p.B[prob];
+  asm volatile("" : "+s"(tiles_m), "+s"(tiles_n), "+s"(k_splits), "+s"(M), "+s"(K_all), "+s"(k_per), "+s"(lda), "+s"(A), "+s"(B));
   int tm, tn;
-  tile_coords(blockIdx.x, p.tiles_m * p.k_splits, p.tiles_n, tm, tn, T::GROUP_M < p.tiles_m || p.k_splits == 1 ? T::GROUP_M : p.tiles_m);
-  const int split = ksplit_of_row(tm, p.tiles_m, p.k_per, p.K);
+  tile_coords(blockIdx.x, tiles_m * k_splits, tiles_n, tm, tn, T::GROUP_M < tiles_m || k_splits == 1 ? T::GROUP_M : tiles_m);
+  const int split = ksplit_of_row(tm, tiles_m, k_per, K_all);
   const int m0 = tm * T::BM, n0 = tn * T::BN;
-  const int k0 = split * p.k_per;
-  const int K = p.K - k0 < p.k_per ? p.K - k0 : p.k_per;
+  const int k0 = split * k_per;
+  const int K = K_all - k0 < k_per ? K_all - k0 : k_per;
   const int ksteps = (K + T::BK - 1) / T::BK;
 
   // A's buffer starts with the tile's first row, so A itself may be of any size: the offsets inside a tile stay below
   // 512 rows.  Rows past M read as zero (it ends with row M - 1), and so does everything past B's last row or slot row
   const int kgs = (K + 31) / 32 * 4;   // prepared_kgroups
-  const int lda = (int)p.lda, rows = p.M - m0 < T::BM ? p.M - m0 : T::BM;
+  const int rows = M - m0 < T::BM ? M - m0 : T::BM;
   const int a_bytes = ((rows - 1) * lda + (K + 7) / 8 * 8) * 2;
   const int64_t b_bytes = RAWB ? ((int64_t)(K - 1) * p.ldb + p.N) * 2 : (int64_t)kgs * p.N * 16;
   const int64_t b_first = RAWB ? (int64_t)k0 * p.ldb * 2 : (int64_t)(k0 / 8) * p.N * 16;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)p.A[prob] + (int64_t)m0 * lda + k0), 0, a_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)p.B[prob] + b_first), 0, (int)b_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)((const E*)A + (int64_t)m0 * lda + k0), 0, a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)B + b_first), 0, (int)b_bytes, 0x00020000);
 
   // ---- loads: this wave's kilobytes of a stage ----
   // A: row r of the stage's BM x BK block at r * 2 BK bytes; position pos of a row holds chunk (pos - rot(r)) mod KG,

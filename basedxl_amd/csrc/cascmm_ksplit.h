@@ -27,7 +27,8 @@ inline int64_t ksplit_row(int64_t N) { return (N + 3) / 4 * 4; }
 inline size_t ksplit_bytes(int64_t M, int64_t N, int splits) { return splits > 1 ? (size_t)splits * (size_t)M * (size_t)ksplit_row(N) * sizeof(float) : 0; }
 
 // A thread adds four consecutive columns of one row; the loads of up to eight splits are in flight.  Bound by its
-// latency, not by bytes: 2 - 2.5 us for anything up to some 2 MB of partial results.
+// latency, not by bytes: 2.5 - 4.2 us (kernel trace, medians) for 0.3 to 10 MB of partial results alike
+// (profiles/cascmm_ksplit_kernels.txt).
 template <int IODT>
 __global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restrict__ parts, int splits, int M, int N, const void* __restrict__ bias,
                                                            void* __restrict__ C, int64_t ldc, int vec_out) {

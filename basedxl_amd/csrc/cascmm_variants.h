@@ -18,8 +18,10 @@ namespace cascmm {
 // KIND_F8K64: three fp8 terms on the fp8-rate MFMA; splits its operands into the workspace first
 // KIND_F16K: three fp16 terms on operand slots; finds both scales and splits its operands into the workspace first
 // KIND_WAVEK: skinny problems in one launch, K split over the waves of a workgroup (no workspace)
-// KIND_H16: 16-bit tensors as one term of their own format, right operand prepared or raw (no workspace)
-// KIND_SLOTK: prepared right operand, K split over the waves of a workgroup (64 x 160 tiles, one problem per launch)
+// KIND_H16: 16-bit tensors as one term of their own format, right operand prepared or raw (workspace: only for a K split
+// over workgroups, cascmm_ksplit.h)
+// KIND_SLOTK: K split over the waves of a workgroup, right operand prepared (64 x 160 and 64 x 80 tiles) or raw (64 x 160),
+// one problem per launch (workspace as KIND_H16)
 enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7, KIND_W512E = 8 };
 constexpr int kNumCUs = 256;  // MI355X: what the cost model's constants were measured on
 constexpr int kMaxDevices = 64;

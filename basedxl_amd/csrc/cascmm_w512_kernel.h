@@ -81,7 +81,8 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // the accumulation registers).
 // EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
 // costs the loop nothing, and the stores past it go beyond the descriptor's end; the last stages may hang over K.
-// Measured (graph replay, raw / prepared weight; in brackets the fastest other kernel): 1976 x 1280 x 10240 on 256 x 320
+// Measured (graph replay, raw / prepared weight, everything on one box: others are up to 6 % slower, see
+// profiles/cascmm_w512_edge_kernels.txt; in brackets the fastest other kernel): 1976 x 1280 x 10240 on 256 x 320
 // 129.6 / 122.4 us (164.8 / 153.6), its gated form 126.1 (158.5); 7800 x 640 x 5120 139 / 134 (155 / 143); 1500 x 1280 x 10240
 // on 256 x 256 104 / 98 (134 / 110); 4096^3 316 / 297 (351 / 326) = 1.30 PFLOP/s of MFMA work, as on the wider tile: what is
 // left is the clock the board's power allows.  K off its steps (in brackets the K-over-waves kernel, the only other one that

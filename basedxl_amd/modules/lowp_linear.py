@@ -26,10 +26,10 @@ class BasedXLLowPLinear(nn.Module):
         self.lowp, self.terms, self.products = d_lowp if lowp is None else lowp, d_terms if terms is None else terms, products
         self._weight_exp = None   # fp8: tensor-scale exponent of the weight, found on first use
         # prepared=True: the weight is also kept split (once, on first use on the GPU); inputs
-        # the prepared kernels do not take (K not a multiple of 64, ...) use the raw weight.
-        # Default: on for fp16 / bf16 weights multiplied as one term of their own format (there
-        # "prepared" is only a re-layout of the weight, which the raw path would redo in every
-        # call), off for fp32 weights (both operands are then split inside every GEMM)
+        # the prepared kernels do not take (K not a multiple of 8, ...: PreparedWeight.usable_with)
+        # use the raw weight.  Default: on for fp16 / bf16 weights multiplied as one term of their
+        # own format (there "prepared" is only a re-layout of the weight, which saves the raw
+        # path's transposing reads), off for fp32 weights (both operands are then split inside every GEMM)
         if prepared is None:
             prepared = self.weight.dtype != torch.float32 and (self.lowp, self.terms) == (d_lowp, d_terms)
         self.prepared = prepared
