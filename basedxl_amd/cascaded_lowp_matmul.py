@@ -270,8 +270,10 @@ class PreparedWeight:
     def check_slots(self) -> None:
         """Raises where the buffer is not one of this weight's layout (one kept in a file from another layout, say): a
         kernel reads what K, N and the cascade say."""
-        need = max(_lib.lib().cascmm_prepared_bytes(self.K, self.N, self.fmt, self.terms), 16)
-        have = self.slots.numel() * self.slots.element_size()
+        need = self.__dict__.get("_slot_bytes")      # (asked for once: the shape and the cascade do not change)
+        if need is None:
+            need = self._slot_bytes = max(_lib.lib().cascmm_prepared_bytes(self.K, self.N, self.fmt, self.terms), 16)
+        have = self.slots.nbytes
         if have != need:
             raise ValueError(f"the operand slots of a {self.K} x {self.N} weight of this cascade are {need} bytes, got {have}: prepare it again")
 

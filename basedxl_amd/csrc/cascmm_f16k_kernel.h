@@ -134,6 +134,7 @@ __device__ __forceinline__ int f16k_find_exp(const unsigned* __restrict__ amax, 
 // Split of the LEFT operand: A [M, K] fp32 row-major -> slots[term][K/8][M].  A workgroup converts 64 rows x 32 k
 // (a thread: 8 consecutive k of a row) and transposes through LDS so that the slots leave as 1 KB runs along M.
 // (k_valid <= K: the depth of A, slots beyond it are zeros; vec: rows of A start on 16-byte boundaries)
+template <int TAIL>
 __device__ __forceinline__ void f16k_split_rows(int block, const float* __restrict__ A, int M, int K, int k_valid, int vec, int64_t lda, u32x4* __restrict__ out,
                                                 float scale, u32x4 (*slots)[4][64]) {
   const int kus = K >> 3;
@@ -144,7 +145,7 @@ __device__ __forceinline__ void f16k_split_rows(int block, const float* __restri
     if (m0 + row < M && ku0 + ku < kus) {
       const float* src = A + (int64_t)(m0 + row) * lda + (ku0 + ku) * 8;
       float r[8];
-      load_row8(src, k_valid - (ku0 + ku) * 8, vec, r);
+      load_row8<TAIL>(src, k_valid - (ku0 + ku) * 8, vec, r);
       u32x4 t[3];
       f16k_split8(r, scale, t);
 #pragma unroll
@@ -162,6 +163,7 @@ __device__ __forceinline__ void f16k_split_rows(int block, const float* __restri
 
 // Split of the RIGHT operand: B [K, N] fp32 row-major -> slots[term][K/8][N]; thread (ku, n) walks 8 rows of
 // column n (consecutive threads: consecutive columns, coalesced both ways).
+template <int TAIL>
 __device__ __forceinline__ void f16k_split_cols(int block, const float* __restrict__ B, int K, int k_valid, int N, int64_t ldb, u32x4* __restrict__ out,
                                                 float scale) {
   const int kus = K >> 3;
@@ -170,7 +172,7 @@ __device__ __forceinline__ void f16k_split_cols(int block, const float* __restri
   const int ku = (int)(i / N), n = (int)(i - (int64_t)ku * N);
   const float* src = B + (int64_t)ku * 8 * ldb + n;
   float r[8];
-  load_column<8>(src, ldb, k_valid - ku * 8, r);
+  load_column<8, TAIL>(src, ldb, k_valid - ku * 8, r);
   u32x4 t[3];
   f16k_split8(r, scale, t);
 #pragma unroll
@@ -179,7 +181,7 @@ __device__ __forceinline__ void f16k_split_cols(int block, const float* __restri
 
 // Both splits in one launch: workgroups 0 .. a_blocks - 1 split A, the others B.  Every workgroup first reduces its
 // operand's per-workgroup maxima; exps_out[0] = e_A, exps_out[1] = e_B are left by the first workgroup of either part.
-template <int UNUSED>
+template <int TAIL>
 __global__ __launch_bounds__(256) void f16k_split_kernel(const float* __restrict__ A, int M, int K, int k_valid, int vec, int64_t lda, u32x4* __restrict__ a_out,
                                                         const unsigned* __restrict__ amax_a, int n_a, int a_blocks,
                                                         const float* __restrict__ B, int N, int64_t ldb, u32x4* __restrict__ b_out,
@@ -189,8 +191,8 @@ __global__ __launch_bounds__(256) void f16k_split_kernel(const float* __restrict
   const bool left = (int)blockIdx.x < a_blocks;
   const int block = left ? (int)blockIdx.x : (int)blockIdx.x - a_blocks;
   const float scale = __builtin_ldexpf(1.f, f16k_find_exp(left ? amax_a : amax_b, left ? n_a : n_b, exps_out + (left ? 0 : 1), &e_found, block == 0));
-  if (left) f16k_split_rows(block, A, M, K, k_valid, vec, lda, a_out, scale, slots);
-  else f16k_split_cols(block, B, K, k_valid, N, ldb, b_out, scale);
+  if (left) f16k_split_rows<TAIL>(block, A, M, K, k_valid, vec, lda, a_out, scale, slots);
+  else f16k_split_cols<TAIL>(block, B, K, k_valid, N, ldb, b_out, scale);
 }
 
 __device__ __forceinline__ f16x8 f16k_half(const i32x8& v, int s) {

@@ -65,9 +65,12 @@ inline __host__ __device__ int64_t f8k64_slot_bytes(int64_t rows, int64_t K) {
   return bytes;
 }
 
-// eight consecutive elements of a row, `left` of which exist (the others are zeros); vec: 16-byte aligned
+// The operand splits' loads.  TAIL = 0: whole units on 16-byte boundaries (the tests of TAIL = 1 cost 2048 x 1280 x 1280 in
+// three fp8 terms 0.35 us of 32.2).
+// Eight consecutive elements of a row; TAIL = 1: `left` of them exist (the others are zeros), vec: 16-byte aligned.
+template <int TAIL>
 __device__ __forceinline__ void load_row8(const float* __restrict__ src, int left, int vec, float (&r)[8]) {
-  if (vec && left >= 8) {
+  if (!TAIL || (vec && left >= 8)) {
     const f32x4 v0 = *(const f32x4*)src, v1 = *(const f32x4*)(src + 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -80,11 +83,11 @@ __device__ __forceinline__ void load_row8(const float* __restrict__ src, int lef
   }
 }
 
-// KN consecutive elements of a column, `left` of which exist (one test for all of them: a test per element would put
+// KN consecutive elements of a column; TAIL = 1: `left` of them exist (one test for all of them: a test per element would put
 // the loads one behind the other)
-template <int KN>
+template <int KN, int TAIL>
 __device__ __forceinline__ void load_column(const float* __restrict__ src, int64_t ld, int left, float (&x)[KN]) {
-  if (left >= KN) {
+  if (!TAIL || left >= KN) {
 #pragma unroll
     for (int e = 0; e < KN; ++e) x[e] = src[(int64_t)e * ld];
   } else {
@@ -115,8 +118,8 @@ __global__ __launch_bounds__(1024) void f8k64_amax_kernel(const float* __restric
 // are the per-workgroup maxima |a| (bit patterns) of a preceding f8k64_amax_kernel; every workgroup
 // reduces them itself (1 KB from L2, behind its loads of A), and the first one leaves {e_A, *b_exp}
 // in exps_out for the GEMM.
-// k_valid <= K: the depth of A; slots beyond it are zeros.  vec: rows of A start on 16-byte boundaries.
-template <int UNUSED>
+// TAIL = 1: k_valid <= K is the depth of A, slots beyond it are zeros; vec: rows of A start on 16-byte boundaries.
+template <int TAIL>
 __global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __restrict__ A, int M, int K, int k_valid, int vec, int64_t lda,
                                                               const int32_t* __restrict__ tensor_exp, u32x4* __restrict__ out,
                                                               const unsigned* __restrict__ amax, int n_amax,
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __re
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         float r[8];
-        load_row8(src + 8 * h, k_valid - (ku0 + ku) * 16 - 8 * h, vec, r);
+        load_row8<TAIL>(src + 8 * h, k_valid - (ku0 + ku) * 16 - 8 * h, vec, r);
 #pragma unroll
         for (int e = 0; e < 8; ++e) r[e] *= scale;
         const u32x2 t0 = Lowp<CASCMM_FMT_FP8>::peel<false>(r);
@@ -179,7 +182,7 @@ __global__ __launch_bounds__(256) void f8k64_split_rows_kernel(const float* __re
 
 // Split of the RIGHT operand: B [K, N] fp32 row-major -> slots[term][K/16][N]; thread (ku, n) walks
 // 16 rows of column n (consecutive threads: consecutive columns, coalesced both ways).
-template <int UNUSED>
+template <int TAIL>
 __global__ __launch_bounds__(256) void f8k64_split_cols_kernel(const float* __restrict__ B, int K, int k_valid, int N, int64_t ldb,
                                                               const int32_t* __restrict__ tensor_exp, u32x4* __restrict__ out) {
   const int kus = K >> 4;
@@ -189,7 +192,7 @@ __global__ __launch_bounds__(256) void f8k64_split_cols_kernel(const float* __re
   const float scale = tensor_exp ? __builtin_ldexpf(1.f, *tensor_exp) : 1.f;
   const float* src = B + (int64_t)ku * 16 * ldb + n;
   float x[16];
-  load_column<16>(src, ldb, k_valid - ku * 16, x);
+  load_column<16, TAIL>(src, ldb, k_valid - ku * 16, x);
   u32x4 t[3];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {

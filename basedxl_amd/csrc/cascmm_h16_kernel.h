@@ -97,7 +97,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   const int prob = blockIdx.y;
   // The arguments that A's first loads need, all requested here: left to themselves the reads sink to their uses and wait one
   // behind the other, which with a descriptor per tile was 0.2 us of a call with new operands (2048 x 1280 x 1280, three
-  // weights in turn: 12.52 us, so 12.26; 512 x 1280 x 1280 6.9 and 6.7).  N among them too: 12.13 and 7.0.
+  // weights in turn: 12.52 us, so 12.26; 512 x 1280 x 1280 6.7 us, with N among them 7.0).
   int tiles_m = p.tiles_m, tiles_n = p.tiles_n, k_splits = p.k_splits, M = p.M, K_all = p.K, k_per = p.k_per, lda = (int)p.lda;
   const void *A = p.A[prob], *B = p.B[prob];
   asm volatile("" : "+s"(tiles_m), "+s"(tiles_n), "+s"(k_splits), "+s"(M), "+s"(K_all), "+s"(k_per), "+s"(lda), "+s"(A), "+s"(B));

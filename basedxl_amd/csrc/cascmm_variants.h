@@ -328,14 +328,15 @@ int launch_f8k64(const GroupParams& p, hipStream_t stream) {
     b_exp = p.b_exp_src;
   }
   const int vec = p.lda % 4 == 0 && (uintptr_t)p.A[0] % 16 == 0;
-  if (launch_kernel(f8k64_split_rows_kernel<0>, dim3(a_grid), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K, p.k_valid, vec, p.lda,
+  const bool tail = !vec || p.k_valid != p.K;
+  if (launch_kernel(tail ? f8k64_split_rows_kernel<1> : f8k64_split_rows_kernel<0>, dim3(a_grid), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K, p.k_valid, vec, p.lda,
                     p.exps_dyn ? (const int32_t*)nullptr : p.tensor_exps, a_slots, amax, n_amax, b_exp, p.exps_dyn) != hipSuccess)
     return CASCMM_ERR_LAUNCH;
   if (!BPRE) {
     u32x4* bs = (u32x4*)ws_next;
     ws_next += f8k64_up(f8k64_slot_bytes(p.N, p.K));
     const int64_t units = (int64_t)kus * p.N;
-    if (launch_kernel(f8k64_split_cols_kernel<0>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, (const float*)p.B[0],
+    if (launch_kernel(p.k_valid != p.K ? f8k64_split_cols_kernel<1> : f8k64_split_cols_kernel<0>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, (const float*)p.B[0],
                       p.K, p.k_valid, p.N, p.ldb, b_exp, bs) != hipSuccess)
       return CASCMM_ERR_LAUNCH;
     b_slots = bs;
@@ -396,8 +397,9 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
   const int kus = p.K >> 3;
   const int a_blocks = ((p.M + 63) / 64) * ((kus + 3) / 4);
   const int64_t b_blocks = ((int64_t)kus * p.N + 255) / 256;
-  if (launch_kernel(f16k_split_kernel<0>, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K,
-                    p.k_valid, (int)(p.lda % 4 == 0 && (uintptr_t)p.A[0] % 16 == 0), p.lda, a_slots, (const unsigned*)amax_a, n_a, a_blocks, (const float*)p.B[0], p.N, p.ldb, b_slots,
+  const int vec = p.lda % 4 == 0 && (uintptr_t)p.A[0] % 16 == 0;
+  if (launch_kernel(!vec || p.k_valid != p.K ? f16k_split_kernel<1> : f16k_split_kernel<0>, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, (const float*)p.A[0], p.M, p.K,
+                    p.k_valid, vec, p.lda, a_slots, (const unsigned*)amax_a, n_a, a_blocks, (const float*)p.B[0], p.N, p.ldb, b_slots,
                     (const unsigned*)amax_b, n_b, exps) != hipSuccess)
     return CASCMM_ERR_LAUNCH;
   F8K64Params q;
