@@ -314,13 +314,38 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
       }
     }
     E* C = (E*)p.C[prob] + (int64_t)(m0 + wm0) * p.ldc + oc0;
-    // (16-byte stores: 32-bit offsets over the wave's rows; others are addressed one by one)
-    const bool vec = (p.ldc & 7) == 0 && (no & 7) == 0 && ((uintptr_t)p.C[prob] & 15) == 0 && p.ldc * (2 * T::WTM) <= 0x7FFFFFFF;
+    // Stores of 16 bytes, of two elements or of one, as width and alignment of the rows allow, with 32-bit offsets over the wave's
+    // rows; rows too far apart for those are addressed one by one.
+    const bool near_rows = p.ldc * (2 * T::WTM) <= 0x7FFFFFFF;
+    const bool vec = near_rows && (p.ldc & 7) == 0 && (no & 7) == 0 && ((uintptr_t)p.C[prob] & 15) == 0;
+    const bool pairs = (p.ldc & 1) == 0 && (no & 1) == 0 && ((uintptr_t)p.C[prob] & 3) == 0;
     // rows past M fall beyond the end of the buffer and are dropped, columns past the last one are sent there too
     const int64_t c_bytes = ((int64_t)(p.M - 1 - m0 - wm0) * p.ldc + (no - oc0)) * 2;
     const i32x4 rc = make_rsrc(C, c_bytes < 0 ? 0 : c_bytes);
     const int ldc_bytes = (int)p.ldc * 2;
     constexpr int CHUNKS = 4 * NB, ITS = 2 * NB;   // 16-byte chunks of a row; of 32 rows, per lane
+    // 32 rows in W elements a lane, eight reads and then eight stores at a time.  (One element behind the other, each store waiting for
+    // its read, a width off 8 took 6016 x 2240 x 754 from the 27.6 us of 752 to 40, 4096 x 640 x 639 from 7.7 to 13.6.)
+    auto narrow = [&](int mi, auto width_tag) {
+      constexpr int W = decltype(width_tag)::value, PER_ROW = 32 * NB / W;
+      typedef typename std::conditional<W == 2, unsigned, unsigned short>::type U;
+#pragma unroll 1
+      for (int i0 = lane; i0 < 32 * PER_ROW; i0 += 8 * 64) {
+        U v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int i = i0 + 64 * u;
+          v[u] = *(const U*)(area + (i / PER_ROW) * T::OUT_ROW + (i % PER_ROW) * (2 * W));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int i = i0 + 64 * u, c = (i % PER_ROW) * W;
+          const int voff = oc0 + c < no ? (mi * 32 + i / PER_ROW) * ldc_bytes + c * 2 : 0x7FFFFFFF;
+          if constexpr (W == 2) llvm_raw_buffer_store_f32(__builtin_bit_cast(float, v[u]), rc, voff, 0, 0);
+          else llvm_raw_buffer_store_i16(__builtin_bit_cast(short, v[u]), rc, voff, 0, 0);
+        }
+      }
+    };
 #pragma unroll
     for (int mi = 0; mi < T::MT; ++mi) {
 #pragma unroll
@@ -366,6 +391,9 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
             llvm_raw_buffer_store_v4f32(__builtin_bit_cast(f32x4, v[it]), rc, oc0 + c * 8 < no ? (mi * 32 + i / CHUNKS) * ldc_bytes + c * 16 : 0x7FFFFFFF, 0, 0);
           }
         }
+      } else if (near_rows) {
+        if (pairs) narrow(mi, std::integral_constant<int, 2>{});
+        else narrow(mi, std::integral_constant<int, 1>{});
       } else {
 #pragma unroll 1
         for (int i = lane; i < 32 * NB * 32; i += 64) {
