@@ -794,10 +794,10 @@ def cascaded_lowp_matmul(
     b_exp: Optional[torch.Tensor] = None,
     tensor_exps: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    if out is None and variant < 0 and not dump_ptx and tensor_exps is None:
+    if out is None and variant < 0 and not dump_ptx and tensor_exps is None and lowp != "fp8":
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         if type(b) is PreparedWeight:
-            y = _lib.short_cut().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+            y = None if b.fmt == _lib.FMT_FP8 else _lib.short_cut().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
         else:
             y = _lib.short_cut().matmul(a, b, bias, lowp, terms, products)
         if y is not None:

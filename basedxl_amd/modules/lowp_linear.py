@@ -53,7 +53,9 @@ class BasedXLLowPLinear(nn.Module):
                                   self.products, False, self._weight_exp if pw is None else pw.exp)
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         pw = self._prepared_weight
-        if not self.prepared or (x.dtype == torch.float32 and x.numel() < 32 * self.in_features):
+        if self.lowp == "fp8":
+            y = None
+        elif not self.prepared or (x.dtype == torch.float32 and x.numel() < 32 * self.in_features):
             y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
         elif pw is not None and pw.device == self.weight.device:
             y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 32)
