@@ -176,8 +176,8 @@ static const TunedCost kTuned[] = {
     {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 1.064, 4.69, 0.90, 0.80},
     {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 1.224, 6.84, 0.80, 0.70},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri", 3.200, 6.50, 0.70, 0.50},
-    // (the large tiles: partly filled rounds are faster than full ones, the board's power goes to fewer CUs: 64 of 256
-    // tiles 0.62 of a round, 144 tiles 0.7, 192 tiles 0.88)
+    // (the large tiles on raw weights: partly filled rounds are faster than full ones, the board's power goes to fewer CUs: 64 of 256
+    // tiles 0.62 of a round, 144 tiles 0.7, 192 tiles 0.88; on prepared ones: kLargeTileCost)
     {"t256x320x32_w512_bf16x2_tri", 5.65, 16.0, 0.50, 0.50},
     {"t256x320x32_w512_edge_bf16x2_tri", 5.65, 17.0, 0.50, 0.50},
     {"t256x256x32_w512_edge_bf16x2_tri", 4.60, 10.5, 0.45, 0.45},
@@ -200,9 +200,6 @@ static const TunedCost kTuned[] = {
     {"t64x64x64_w2x2x1_d3_bf16x2_tri_bpre", 0.515, 2.08, 1.00, 1.00},
     {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 1.250, 5.89, 0.80, 0.50},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri_bpre", 2.837, 12.00, 0.60, 0.50},
-    {"t256x320x32_w512_bf16x2_tri_bpre", 5.40, 15.0, 0.50, 0.50},
-    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 5.40, 16.0, 0.50, 0.50},
-    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 4.50, 11.5, 0.45, 0.45},
     // K split over the waves: a round of 256 tiles costs 0.011 us per k + 8 us, and rounds do not overlap
     // (2048 x {1280, 5120} x 1280: 21.7 / 64.3 us; 1024 x 1280 x 1280: 17.4 us -- 7 % less than with raw A fetched
     // in half lines, A/B on one box)
@@ -300,6 +297,28 @@ static double slotk_estimate_us(const TunedCost& t, const VariantDesc& v, const 
   return edge * rounds * ((double)((k_per + 255) / 256 * 256) / 64.0 * t.step64_us + t.fixed_us);
 }
 
+// The large tiles on prepared weights.  A round of a few tiles takes a us per 64 k and b; one that fills the chip A and B, for the
+// clock that the board's power leaves; in between by the cube of what is filled, and a round behind another starts c earlier.  Fitted
+// to 128 shapes each of 64 - 8192 rows, K and widths from 320 (gated: 66 and 44), within 5 %: 256 x 256, us: 4928 x 384 x 1152 29.4, 6976 x
+// 320 x 960 26.2, 4096^3 300; gated 1709 x 448 x 3584 33.6, 1500 x 1280 x 10240 99.4.  (With a partly filled round as 0.45 of a full one
+// and a share of the rest the small ones were priced at 18 - 26 us and came here from tiles that run them in 20 - 25: 3072 x 576 x
+// 1728 36 us, 25 on 256 x 128; 4928 x 384 x 1152 28, 22.  Raw weights keep that rule: the other tiles' entries for them lie as far off.)
+struct LargeTileCost { int BN; bool glu; double a, b, A, B, c; };
+static const LargeTileCost kLargeTileCost[] = {
+    {256, false, 2.845, 10.34, 4.415, 12.13, 3.0}, {320, false, 3.438, 12.08, 5.382, 13.81, 3.7},
+    {256, true, 2.830, 12.33, 4.507, 13.15, 6.0},  {320, true, 3.470, 16.43, 5.254, 18.72, 6.6},
+};
+static double large_tile_us(const VariantDesc& v, const Problem& q, double tiles) {
+  for (const LargeTileCost& t : kLargeTileCost)
+    if (t.BN == v.BN && t.glu == q.glu) {
+      const double k = (double)((q.K + 31) / 32) * 0.5, full = (double)(int64_t)(tiles / kNumCUs), part = tiles / kNumCUs - full;
+      const double few = t.a * k + t.b, all = t.A * k + t.B;
+      const double us = full * all + (part > 0 ? few - (full > 0 ? t.c : 0.0) + part * part * part * (all - few) : 0.0);
+      return v.kind == KIND_W512 ? 0.99 * us : us;   // (whole tiles: no test per load of A)
+    }
+  return 1e9;
+}
+
 // K split over workgroups (cascmm_ksplit.h): where the tiles leave CUs idle, `estimate(tiles, k of a split)` with the
 // chip filled against the second launch and the partial results, written and read back.  Measured (graph replay): 7 x 3264 x 880
 // fp16 14.8 -> 6.2 us in thirteen splits, 256 x 5120 x 1280 23.0 -> 14.0 in six, 34 x 2008 x 2176 fp32 prepared 15.5 -> 9.5 in
@@ -342,6 +361,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
   if (v.kind == KIND_WAVEK) return wavek_estimate_us(q, count, v.BN);
+  if ((v.kind == KIND_W512E || v.kind == KIND_W512) && q.bpre) return large_tile_us(v, q, tiles);
   int ks = 1;
   if (v.kind == KIND_H16 || (v.kind == KIND_SLOTK && info.tuned)) {
     const double us = v.kind == KIND_H16

@@ -209,6 +209,15 @@ def test_the_kernel_of_a_call_is_the_one_that_is_launched():
     assert l.cascmm_call_variant(A, B, 4, 4, 4, 3, 4, 4, 0, 0, 2, 0, 0) == -2
 
 
+@pytest.mark.parametrize("M,K,N,large", [(3072, 576, 1728, False), (4928, 384, 1152, False), (6976, 320, 960, False),
+                                         (1500, 1280, 10240, True), (4096, 4096, 4096, True), (7800, 640, 5120, True)])
+def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):
+    """Few tiles and a short K cost the 256-row tiles more than their share of a full round (25, 22 and 21 us on 256 x 128 there, 36, 28 and
+    26 on 256 x 256)."""
+    names = _lib.variant_names()
+    assert ("_w512_" in names[_lib.lib().cascmm_select_variant_prepared(1, M, N, K, K, N, 0, 0, 2, 0) & 0xFFFF]) == large
+
+
 def test_cpu_tensors_are_rejected_without_fallback():
     import torch
     from basedxl_amd import cascaded_lowp_matmul
