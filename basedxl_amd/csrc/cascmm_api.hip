@@ -763,7 +763,11 @@ static Problem rounded_up(const Problem& q, RowFit fit) {
 
 // The slot kernel for such a problem, or a negative status: none, no room, or the bounds-checked kernel, which needs one
 // launch where these need three, is expected to be faster (a 32-k step of its 64 x 64 tiles 1.35 us: 100 x 300 x 200
-// fp16 x 3 16.5 us against 21; 300 x 500 x 1001 25.9 against 24, fp8 x 3 35 against 26, 3740 x 1090 x 992 fp16 x 3 132 against 81)
+// fp16 x 3 16.5 us against 21; 300 x 500 x 1001 25.9 against 24, fp8 x 3 35 against 26, 3740 x 1090 x 992 fp16 x 3 132 against 81).
+// Three fp8 terms need three launches more, of 3 us of the host's time each, behind a scale search that keeps the host
+// busy already: eager calls take 36 us in slots however small they are, so what the bounds-checked kernel runs in less stays
+// there (8 x 632 x 576: 31 us; graph replay 30 and 23), and the launches count as 5 us.  A step of the bounds-checked fp8
+// tiles takes 1.1 us where there are few and 1.9 on 130 CUs (640 x 768 x 814: 49 us).
 static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem* e) {
   *e = rounded_up(q, fit);
   if (!e->split_first) return CASCMM_ERR_BAD_FORMAT;
@@ -771,7 +775,9 @@ static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem*
   if (v < 0) return v;
   const double tiles = (double)((q.M + 63) / 64) * (double)((q.N + 63) / 64);
   const double rounds = (double)(int64_t)((tiles + kNumCUs - 1) / kNumCUs);
-  return variant_cost(v, *e, 1) < 3.5 + 1.35 * rounds * (double)((q.K + 31) / 32) ? v : (int)CASCMM_ERR_BAD_FORMAT;
+  const bool fp8 = q.fmt == CASCMM_FMT_FP8;
+  const double step = fp8 ? std::min(1.2 + 0.006 * tiles, 2.7) : 1.35, slots = variant_cost(v, *e, 1);
+  return (fp8 ? std::max(slots + 5.0, 32.0) : slots) < 3.5 + step * rounds * (double)((q.K + 31) / 32) ? v : (int)CASCMM_ERR_BAD_FORMAT;
 }
 
 // The launch itself, on operands as they lie (exps_dyn, b_exp_src: see gemm_impl)

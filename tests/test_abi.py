@@ -218,6 +218,14 @@ def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):
     assert ("_w512_" in names[_lib.lib().cascmm_select_variant_prepared(1, M, N, K, K, N, 0, 0, 2, 0) & 0xFFFF]) == large
 
 
+@pytest.mark.parametrize("M,K,N,slots", [(8, 632, 576, False), (276, 276, 276, False), (640, 768, 814, True), (704, 584, 617, True), (5, 656, 5248, True)])
+def test_small_fp8_products_off_the_stages_stay_on_one_launch(M, K, N, slots):
+    """Splitting both operands first costs three launches of the host's time: worth it from some 32 us of the one-launch kernel on."""
+    l, names = _lib.lib(), _lib.variant_names()
+    v = l.cascmm_call_variant(1 << 40, 2 << 40, M, N, K, K, N, N, 0, 2, 3, 0, l.cascmm_workspace_bytes(M, N, K, 0, 2, 3, 0))
+    assert ("_f8k64" in names[v & 0xFFFF]) == slots
+
+
 def test_cpu_tensors_are_rejected_without_fallback():
     import torch
     from basedxl_amd import cascaded_lowp_matmul
