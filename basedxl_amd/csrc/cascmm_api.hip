@@ -1,5 +1,6 @@
 // extern "C" entry points: argument checks, kernel selection, small utility kernels.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <dlfcn.h>
@@ -38,9 +39,10 @@ static const std::vector<VariantDesc>& table() {
 }
 
 struct TunedCost;
+struct CallCost;
 // per variant, resolved once when the table is built: its measured cost constants (or none) and what
 // kind of kernel its name says it is
-struct VariantInfo { const TunedCost* tuned; bool p8; bool bdirect; };
+struct VariantInfo { const TunedCost* tuned; const CallCost* call; bool p8; bool bdirect; };
 static const std::vector<VariantInfo>& variant_info();
 
 static bool aligned_to(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
@@ -55,6 +57,9 @@ struct Problem {
   // the rows of A are whole 16-byte chunks with zeros between K and the last chunk's end: fp32 with K % 4 == 0, 16-bit
   // with K % 8 == 0, or rows padded in the workspace (relay)
   bool chunked = false;
+  // a call (not the selection functions, which answer for a shape): the small tiles of KIND_WAVEK are open too, and rows that
+  // are not chunked, which these kernels read where they lie (what lies past K is masked)
+  bool call = false;
   // three fp8 / fp16 terms: only the kernels that split both operands into slots first; K is rounded up to whole
   // stages, of which the operands hold k_valid, and their rows need no alignment
   bool split_first = false;
@@ -129,7 +134,7 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.fast && fit < (any_rows ? FIT_DWORD : FIT_FAST)) return false;
   // K in whole 32-k steps, or a tail of whole 16-byte chunks (a weight less than one 64-k stage deep is not worth keeping
   // split: such a prepared operand is refused)
-  if ((any_rows || v.kind == KIND_W512E) && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
+  if ((v.kind == KIND_SLOTK || v.kind == KIND_W512E) && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
   if (v.fast && !any_rows && v.kind != KIND_H16 && (v.kind != KIND_W512E || q.glu) && q.K % v.BK != 0) return false;
   if (v.kind == KIND_SPLITK && (q.M > 5 * v.BM || q.K < 4 * v.BK)) return false;  // skinny: few row tiles, deep K
   if (v.kind == KIND_F8K64 && (q.products != CASCMM_PROD_TRI || q.K % v.BK != 0 || q.K == 0 || q.glu ||
@@ -146,7 +151,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_W512E && (q.M < W512_EDGE_ROWS || q.N < v.BN || (q.glu && v.BN == W512::BN && q.N % v.BN != 0) || q.lda < 32 || q.M * q.lda * 4 > INT32_MAX ||
                                (!q.bpre && beyond_i32(q.K + 32, q.ldb, 4)) || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
-  if (v.kind == KIND_WAVEK && q.M * q.lda * 4 > INT32_MAX) return false;
+  // (rows that are not chunked: up to four rounds of tiles, larger problems are worth a copy of A)
+  if (v.kind == KIND_WAVEK && (q.K == 0 || (q.K % 32 != 0 && !q.chunked && (!q.call || ((q.M + v.BM - 1) / v.BM) * ((q.N + v.BN - 1) / v.BN) > 4 * kNumCUs)) || (v.call_only && !q.call) || beyond_i32(q.M, q.lda, 4))) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
   // (32-bit byte offsets down B, a raw one's two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
@@ -215,46 +221,71 @@ static bool ksplit_kind(const VariantDesc& v) { return v.kind == KIND_H16 || v.k
 // the fp8-rate kernel with K over the waves: us per 64-k stage of a wave, and per round of tiles
 constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {1280, 5120} x 1280, 4096 x {640, 2560} x 640)
 
+
+// Calls with raw operands and two bf16 terms.  A launch of `tiles` tiles on 256 CUs, k in units of the kernel's loop (KIND_WAVEK:
+// steps per wave; K over four waves: trips of 256 k, in 64s; else 64 k):  c0 + full (c1 + k r1) + |k s0, fill k s1 + MB of B / bw|_x  (the
+// x-norm), where full rounds of 256 tiles go before one that is `fill` full; 16 x 16 and 16 x 32 tiles, of which several fit a CU, have
+// no rounds.  deep: what a step past the straight code's adds; edge: tiles over the edge of C.  Fitted to 1150 shapes (those of a
+// UNet step and of its image sizes, squares, small ones; graph replay, every kernel forced in turn), mean error 0.02 - 0.09: the
+// kernel chosen is 2.2 % behind the fastest of all on average, 7.4 % with the constants above (649 x 320 x 2496 17.1 us, 10.0 on the
+// B-direct kernel; 12 x 3392 x 7104 42.8, 17.7 on a 16 x 32 tile; 1024^3 16.6, 14.2).  The selection functions, which answer for shapes,
+// keep the constants above but for KIND_WAVEK.
+struct CallCost { const char* name; double c0, s0, s1, c1, bw, x, r1, deep, edge; };
+static const CallCost kCallCost[] = {
+    {"t16x16x32_wavek_bf16x2_tri", 1.79, 0.413, 0.493, 0, 24.3, 1.26, 0, 0.0881, 0},
+    {"t16x32x32_wavek_bf16x2_tri", 1.88, 0.636, 0.667, 0, 40, 1.26, 0, 0, 0},
+    {"t16x64x32_wavek_bf16x2_tri", 1.97, 1.05, 0.732, 0.678, 15.6, 1.67, 1.2, 0, 0},
+    {"t32x32x32_wavek_bf16x2_tri", 1.98, 1, 1.02, 0.468, 37.6, 2.39, 1.23, 0, 0},
+    {"t32x64x32_wavek_bf16x2_tri", 2.68, 1.22, 0.589, 0.662, 40, 1.12, 1.77, 0, 0},
+    {"t64x64x32_wavek_bf16x2_tri", 4.64, 1.43, 1.5, 1.78, 40, 1.53, 2.5, 0, 0},
+    {"k64x160x16_wk4_bf16x2_tri", 5.89, 0.622, 0.789, 4.3, 40, 2.93, 0.882, 0, 0.0243},
+    {"bd64x128x64_d3_p4_bf16x2_tri", 4.45, 0.993, 0.111, 1.57, 33.2, 1, 1.11, 0, 0.0431},
+    {"bd96x128x64_d3_p4_bf16x2_tri", 5.99, 1.2, 1.12, 3.16, 40, 4.94, 1.29, 0, 0.058},
+    {"bd128x128x32_d3_p4_bf16x2_tri", 5.71, 1.43, 1.36, 1.74, 5.17, 3.92, 1.65, 0, 0.0717},
+    {"t64x64x64_w2x2x1_d3_bf16x2_tri", 4.46, 0.674, 0.149, 0.798, 40, 1.23, 0.686, 0, 0.0424},
+    {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 5.9, 0.899, 1.02, 2.35, 10.1, 8, 0.972, 0, 0.29},
+    {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 8.68, 0.897, 1.3, 1.49, 8.53, 3.67, 1.37, 0, 0.193},
+    {"t256x128x32_w4x1x1_d2_bf16x2_tri", 9.48, 1.79, 2.2, 6.57, 3.09, 4.83, 2.22, 0, 0.254},
+    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 11.5, 2.05, 3.13, 11.7, 40, 7.77, 2.36, 0, 0.231},
+    {"t256x256x32_w512_edge_bf16x2_tri", 11.1, 2.98, 4.74, 10.2, 40, 4.25, 4.83, 0, 0.00177},
+    {"t256x320x32_w512_edge_bf16x2_tri", 12, 3.38, 5, 13.4, 19, 2.39, 5.8, 0, 0.013},
+    {"t256x320x32_w512_bf16x2_tri", 11.9, 3.21, 5, 6.51, 40, 2.24, 6.86, 0, 0.02},
+};
 static const std::vector<VariantInfo>& variant_info() {
   static const std::vector<VariantInfo> info = [] {
     std::vector<VariantInfo> v;
     for (const VariantDesc& d : table()) {
-      VariantInfo i{nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
+      VariantInfo i{nullptr, nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
       for (const TunedCost& t : kTuned)
         if (strcmp(t.name, d.name) == 0) i.tuned = &t;
+      for (const CallCost& t : kCallCost)
+        if (strcmp(t.name, d.name) == 0) i.call = &t;
       v.push_back(i);
     }
     return v;
   }();
   return info;
 }
-
-// The kernel that splits K over the waves of a workgroup (KIND_WAVEK) moves (32 + BN) x K x 4 bytes
-// into every workgroup and is bound by that: a CU pulled in 85 bytes per ns with the 32-wide and
-// 60 with the 64-wide tile, all CUs together 17 KB per ns (154 x 2048 x {640, 1280, 2560}); a launch
-// costs 2.5 us, prologue and the meeting of the partial tiles 0.6 us.  A launch of several rounds pays the
-// start of every workgroup (one fits a CU, so nothing hides it) and runs at 48 / 52 bytes per ns and CU: 1425 x 2112 x
-// 528 41 us, 576 x 560 x 7532 74 us, 448 x 592 x 1952 18.3 us; priced as single rounds these kept the kernel on
-// problems that the 64 x 160 tiles run in 25, 33 and 13.6 us.
+static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Problem& q, int count, double tiles, int64_t k_per) {
+  const double k = v.kind == KIND_WAVEK ? (double)(((k_per + 31) / 32 + 7) / 8) : v.kind == KIND_SLOTK ? (double)((k_per + 255) / 256 * 4) : (double)k_per / 64.0;
+  const double per = tiles / kNumCUs, mb = (double)count * (double)q.K * (double)q.N * 4.0e-6;
+  const double full = v.BM * v.BN <= 512 ? 0.0 : std::ceil(per) - 1.0, fill = per - full;
+  const double lone = k * t.s0 + (k > 8 ? t.deep * (k - 8) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
+  const double us = t.c0 + full * (t.c1 + k * t.r1) + std::pow(std::pow(lone, t.x) + std::pow(shared, t.x), 1.0 / t.x);
+  return q.N % v.BN != 0 || q.M % v.BM != 0 ? us * (1.0 + t.edge) : us;
+}
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
-         !q.glu && q.K > 0 && (q.K % 32 == 0 || q.chunked) && q.M * q.lda * 4 <= INT32_MAX;
-}
-static double wavek_estimate_us(const Problem& q, int count, int bn) {
-  const double items = (double)count * (double)((q.M + 31) / 32) * (double)((q.N + bn - 1) / bn);
-  const double active = items < kNumCUs ? items : kNumCUs;
-  const double per_cu = bn == 32 ? 85.0e3 : 60.0e3;                       // bytes per us
-  const double rate = per_cu < 17.0e6 / active ? per_cu : 17.0e6 / active;
-  const double bytes = (double)(32 + bn) * (double)q.K * 4.0;
-  if (items <= kNumCUs) return 2.5 + 0.6 + bytes / rate;
-  const double start = bn == 32 ? 1.7 : 4.1, full_rate = bn == 32 ? 48.0e3 : 52.0e3;
-  const double full = (double)(int64_t)(items / kNumCUs), rest = items - full * kNumCUs;
-  const double rest_rate = rest * per_cu < kNumCUs * full_rate ? per_cu : kNumCUs * full_rate / rest;
-  return 2.5 + full * (start + bytes / full_rate) + (rest > 0 ? start + bytes / rest_rate : 0.0);
+         !q.glu && q.K > 0 && !beyond_i32(q.M, q.lda, 4);
 }
 static double wavek_estimate_us(const Problem& q, int count) {
-  const double a = wavek_estimate_us(q, count, 32), b = wavek_estimate_us(q, count, 64);
-  return a < b ? a : b;
+  double best = 1e9;
+  for (size_t i = 0; i < table().size(); ++i) {
+    const VariantDesc& v = table()[i];
+    if (v.kind != KIND_WAVEK || !variant_info()[i].call || (v.call_only && !q.call)) continue;
+    best = std::min(best, call_estimate_us(*variant_info()[i].call, v, q, count, (double)count * (double)((q.M + v.BM - 1) / v.BM) * (double)((q.N + v.BN - 1) / v.BN), q.K));
+  }
+  return best;
 }
 // The skinny split-K path for comparison (its 32-row variant, the one preferred among them): two
 // launches, a workgroup's (32 + 128) x K / splits x 4 bytes at 70 bytes per ns, the partial results
@@ -348,6 +379,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   const double full = (double)(int64_t)(tiles / kNumCUs);
   const double rem = tiles - full * kNumCUs;
   if (v.kind == KIND_SPLITK) {
+    if (q.call) return 1e9;   // (the small tiles of KIND_WAVEK and the K-over-waves tiles: 3 x 4416 x 2752 18 us here, 12.1 there)
     // Problems with too few tiles to occupy the chip: splitting K wins whenever the plain tile
     // kernels would leave more than half of the CUs idle; among the split-K variants the
     // smaller row tile was faster wherever both were measured.
@@ -360,7 +392,15 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
       if (table()[i].kind == KIND_SLOTK && variant_matches(table()[i], q, FIT_DWORD) && variant_cost(i, q, count, ws_bytes) < skinny_us) return 1e9;
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
-  if (v.kind == KIND_WAVEK) return wavek_estimate_us(q, count, v.BN);
+  if (q.call && count == 1 && !info.call && v.fast && wavek_eligible(q) && v.kind != KIND_SPLITK) return 1e9;   // (nowhere the fastest)
+  if (info.call && ((q.call && count == 1) || v.kind == KIND_WAVEK)) {
+    const CallCost& t = *info.call;
+    if (v.kind != KIND_SLOTK) return call_estimate_us(t, v, q, count, tiles, q.K);
+    int ks = 1;
+    const double us = ksplit_best(q, count, tiles, ws_bytes, 2.8, 12.0e6, &ks, [&](double n, int64_t k) { return call_estimate_us(t, v, q, count, n, k); });
+    if (splits_out) *splits_out = ks;
+    return us;
+  }
   if ((v.kind == KIND_W512E || v.kind == KIND_W512) && q.bpre) return large_tile_us(v, q, tiles);
   int ks = 1;
   if (v.kind == KIND_H16 || (v.kind == KIND_SLOTK && info.tuned)) {
@@ -455,7 +495,7 @@ struct SelectKey {
   // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
   // some kernels: M lda, K ldb, 1024 ldc and 256 ldc beyond 2^31 bytes << 3, 4, 5, 15; lda below 32 << 7), glu_slots << 6,
   // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12, K ldb as the kernels state it with
-  // stages past K, of four-byte and two-byte elements << 13, 14
+  // stages past K, of four-byte and two-byte elements << 13, 14, call << 16
   int dtype, fmt, terms, products, count, flags;
   bool operator==(const SelectKey& o) const {
     return M == o.M && N == o.N && K == o.K && ws_bytes == o.ws_bytes && dtype == o.dtype && fmt == o.fmt &&
@@ -481,7 +521,7 @@ static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_byt
   static std::mutex mu;
   static std::unordered_map<SelectKey, SelectHit, SelectKeyHash> memo;
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
-                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
+                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.call ? 65536 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
                           (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0) | (beyond_i32(q.ldc, 256, 1) ? 32768 : 0) | (beyond_i32(q.K + 32, q.ldb, 4) ? 8192 : 0) |
                           (beyond_i32(q.K + 64, q.ldb, 2) ? 16384 : 0)};
   {
@@ -713,7 +753,10 @@ static Problem relayed(const Problem& q0, const Relay& r) {
   if (r.b) q.ldb = q.N;
   return q;
 }
-static Relay relay_of(const Problem& q, int count, const void* const* A, const void* const* B) {
+// where_it_lies: nothing is copied for the kernels that need no copy where they are expected to be faster
+static Relay relay_of(const Problem& q0, int count, const void* const* A, const void* const* B, bool where_it_lies = true) {
+  Problem q = q0;
+  q.call = true;
   Relay r;
   if (q.bpre || q.split_first || q.K == 0) return r;
   const bool f32 = q.dtype == CASCMM_DT_F32;
@@ -731,6 +774,17 @@ static Relay relay_of(const Problem& q, int count, const void* const* A, const v
   r.a_chunks = (int)lines * 8;
   r.a_bytes = r.a ? f8k64_up(a_bytes) : 0;
   r.b_bytes = f8k64_up(b_bytes);
+  // (small problems have a kernel that reads rows of any length where they lie; the copy is a launch of 4 us: 122 x 2382 x 1480
+  // 17.3 us with it)
+  if (f32 && r.a && where_it_lies) {
+    RowFit fit = FIT_FAST;
+    for (int i = 0; i < count; ++i) fit = std::min(fit, row_fit(q, A ? A[i] : nullptr, B ? B[i] : nullptr));
+    const Problem e = relayed(q, r);
+    const int direct = select_variant(q, fit, count), copied = select_variant(e, row_fit(e, nullptr, nullptr), count);
+    if (direct >= 0 && table()[direct].kind == KIND_WAVEK &&
+        (copied < 0 || variant_cost(direct, q, count) < variant_cost(copied, e, count) + 3.5 + (double)a_bytes * 2.0 / 4.0e6))
+      return Relay();
+  }
   // (a copied B is a prepared one, which the bounds-checked kernels do not take: without a kernel for what is left, rows of A
   // too far apart for 32-bit offsets for instance, nothing is copied and the operands are read where they lie)
   if (r.b) {
@@ -922,6 +976,7 @@ static int gemm_impl(int count, const void* const* A, const void* const* B, void
     return err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
   }
   q.chunked = chunked_by_k(q);
+  q.call = true;
   // Calls of several launches that meet in the workspace go to the stream as a whole: two threads that share a stream, and
   // with it the workspace, must not put one call's launches between another's.
   static std::mutex workspace_mu;
@@ -1016,6 +1071,7 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
     else need += ksplit_need(relayed(q, relay), FIT_FAST, (size_t)CASCMM_NOALLOC_SCRATCH_BYTES - need);
   } else if (A && B) {
     const RowFit fit = row_fit(q, A, B);
+    // (what the kernels known to the selection functions would need: the call itself may take a small tile that needs none)
     q.chunked = chunked_by_k(q);
     Problem e;
     int splits = 1;
@@ -1198,7 +1254,7 @@ size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fm
   q.chunked = chunked_by_k(q);
   const RowFit fit = row_fit(q, nullptr, nullptr);
   // rows of A (and, 16-bit, all of B) copied first
-  const Relay relay = relay_of(q, 1, nullptr, nullptr);
+  const Relay relay = relay_of(q, 1, nullptr, nullptr, false);
   size_t need = relay_bytes(relay, 1);
   // K split over workgroups, behind such a copy or on the operands as they lie, raw or prepared
   size_t parts = 0;
@@ -1254,6 +1310,7 @@ int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int6
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
   q.chunked = chunked_by_k(q);
+  q.call = true;
   // (as gemm_impl and gemm_on_rows go about it)
   const Relay r = relay_of(q, 1, &A, &B);
   if ((r.a || r.b) && workspace_bytes >= relay_bytes(r, 1)) {
@@ -1414,6 +1471,11 @@ int cascmm_selftest(void) {
   int bad = 0;
   const auto& t = table();
   for (const TunedCost& c : kTuned) {
+    int hits = 0;
+    for (const VariantDesc& d : t) hits += strcmp(c.name, d.name) == 0 ? 1 : 0;
+    bad += hits == 1 ? 0 : 1;
+  }
+  for (const CallCost& c : kCallCost) {
     int hits = 0;
     for (const VariantDesc& d : t) hits += strcmp(c.name, d.name) == 0 ? 1 : 0;
     bad += hits == 1 ? 0 : 1;

@@ -23,8 +23,12 @@ static const VariantDesc kTable[] = {
     CASCMM_W512_EDGE_VARIANT("t256x320x32_w512_edge_bf16x2_tri", 0, 5),
     CASCMM_W512_EDGE_VARIANT("t256x256x32_w512_edge_bf16x2_tri", 0, 4),
     // K split over the eight waves of a workgroup: one launch, no workspace
-    CASCMM_WAVEK_VARIANT("t32x32x32_wavek_bf16x2_tri", 1),
-    CASCMM_WAVEK_VARIANT("t32x64x32_wavek_bf16x2_tri", 2),
+    CASCMM_WAVEK_VARIANT("t32x32x32_wavek_bf16x2_tri", 32, 1, 1, BF, 2),
+    CASCMM_WAVEK_VARIANT("t32x64x32_wavek_bf16x2_tri", 16, 2, 4, BF, 2),
+    CASCMM_WAVEK_VARIANT("t64x64x32_wavek_bf16x2_tri", 16, 4, 4, BF, 2),
+    CASCMM_WAVEK_VARIANT("t16x16x32_wavek_bf16x2_tri", 16, 1, 1, BF, 2),
+    CASCMM_WAVEK_VARIANT("t16x32x32_wavek_bf16x2_tri", 16, 1, 2, BF, 2),
+    CASCMM_WAVEK_VARIANT("t16x64x32_wavek_bf16x2_tri", 16, 1, 4, BF, 2),
     CASCMM_SKINNY_VARIANT("skinny64x128x64_bf16x2_tri", 64, 4, 64, 2, 4, BF, 2, false),
     CASCMM_SKINNY_VARIANT("skinny32x128x64_bf16x2_tri", 32, 4, 64, 2, 4, BF, 2, false),
     CASCMM_BD_VARIANT("bd128x128x64_d3_p4_bf16x2_tri", 128, 4, 64, 3, 4, BF, 2, false),

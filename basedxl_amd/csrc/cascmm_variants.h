@@ -72,6 +72,7 @@ struct VariantDesc {
   int (*launch)(const GroupParams&, hipStream_t);
   bool bpre = false;  // takes the right operand already split (cascmm_prepare_weight)
   bool glu = false;   // has the gated epilogue
+  bool call_only = false;   // chosen for calls only: the selection functions, which answer for a shape, leave it out
 };
 
 template <class TL, int IODT, int FMT, int TERMS, bool FULL, bool FAST, bool BPRE = false>
@@ -236,23 +237,28 @@ int launch_w512_edge(const GroupParams& p, hipStream_t stream) {
   return launch_w512_kernel<BPRE, 0, NTL, 1>(p, stream);
 }
 
-// skinny problems, K split over the waves of a workgroup
-template <int NB>
+// the tiles of KIND_WAVEK that the selection functions know
+constexpr bool wavek_for_shapes(int bm, int bn) { return bm == 32 && bn >= 32; }
+// skinny and small problems, K split over the waves of a workgroup
+template <int W, int MB, int NB, int FMT, int TERMS>
 int launch_wavek(const GroupParams& p, hipStream_t stream) {
-  typedef WaveK<NB> T;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<NB, 0>; return CASCMM_OK; }
+  typedef WaveK<W, MB, NB> T;
+  constexpr int ALL = T::BM / 8, FEW = T::BM == 16 ? 1 : ALL;
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS>; return CASCMM_OK; }
   if (p.glu || p.k_splits > 1 || p.count < 1) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  const bool tail = p.N % T::BN != 0 || p.K % T::BK != 0;
-  auto kfn = tail ? cascmm_wavek_kernel<NB, 1> : cascmm_wavek_kernel<NB, 0>;
-  static LdsFlags lds_set[2];
-  if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[tail ? 1 : 0])) return CASCMM_ERR_LAUNCH;
+  const bool tail = p.N % T::BN != 0 || p.K % T::BK != 0, few = T::BM == 16 && p.M <= 8;
+  void (*kfn)(const GroupParams) = few ? (tail ? cascmm_wavek_kernel<W, MB, NB, FEW, 1, FMT, TERMS> : cascmm_wavek_kernel<W, MB, NB, FEW, 0, FMT, TERMS>)
+                                       : (tail ? cascmm_wavek_kernel<W, MB, NB, ALL, 1, FMT, TERMS> : cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS>);
+  const int lds = few ? WaveK<W, MB, NB, FEW>::LDS_BYTES : T::LDS_BYTES;
+  static LdsFlags lds_set[4];
+  if (!ensure_lds((const void*)kfn, lds, lds_set[(tail ? 1 : 0) + (few ? 2 : 0)])) return CASCMM_ERR_LAUNCH;
   GroupParams q = p;
   q.tiles_m = (p.M + T::BM - 1) / T::BM;
   q.tiles_n = (p.N + T::BN - 1) / T::BN;
   const int64_t grid = (int64_t)q.count * q.tiles_m * q.tiles_n;
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  if (launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)T::LDS_BYTES, stream, q) != hipSuccess) return CASCMM_ERR_LAUNCH;
+  if (launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)lds, stream, q) != hipSuccess) return CASCMM_ERR_LAUNCH;
   return CASCMM_OK;
 }
 
@@ -424,9 +430,10 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
   {NAME, KIND_F8K64, CASCMM_DT_F32, CASCMM_FMT_FP8, 3, false, F8Tile<MT>::T::BM, F8Tile<MT>::T::BN, F8Tile<MT>::T::BK, \
    F8Tile<MT>::T::NT, F8Tile<MT>::T::LDS_BYTES, true, false, &launch_f8k64<BPRE, MT>, BPRE}
 
-#define CASCMM_WAVEK_VARIANT(NAME, NB)                                                                                \
-  {NAME, KIND_WAVEK, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, WaveK<NB>::BM, WaveK<NB>::BN, WaveK<NB>::BK, WaveK<NB>::NT, \
-   WaveK<NB>::LDS_BYTES, true, true, &launch_wavek<NB>}
+#define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS)                                                                   \
+  {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, WaveK<W, MB, NB>::BM, WaveK<W, MB, NB>::BN, WaveK<W, MB, NB>::BK,   \
+   WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS>, false, false,   \
+   !wavek_for_shapes(W * MB, W * NB)}
 
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \
   {NAME, KIND_W512, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512::BM, W512::BN, 32, W512::NT, W512::LDS_BYTES, true, \

@@ -1,36 +1,49 @@
-// Skinny problems (few rows, e.g. the 77 or 154 text tokens of a cross-attention K/V projection) in
-// ONE launch and without a workspace: K is split over the eight waves of a workgroup instead of
-// over workgroups, so the partial sums meet in LDS and never travel through memory.
+// Skinny problems (few rows, e.g. the two rows of a time embedding, the 77 or 154 text tokens of a cross-attention K/V
+// projection) and small ones in ONE launch and without partial results in memory: K is split over the eight waves of a
+// workgroup instead of over workgroups, so the partial sums meet in LDS.
 //
-// One workgroup computes a 32 x (32 NB) tile of C over the whole K.  Wave w takes the 32-wide K
-// steps w, w + 8, w + 16, ...; it streams its own operands and shares nothing with the other waves
+// One workgroup computes a (W MB) x (W NB) tile of C over the whole K, in blocks of the 16 x 16 x 32 (W = 16) or
+// 32 x 32 x 16 (W = 32) MFMA.  Wave w takes
+// the 32-wide K steps w, w + 8, w + 16, ...; it streams its own operands and shares nothing with the other waves
 // until the end, so the main loop has no barrier:
-//   * A (32 rows x 32 k fp32 per step, 4 KB) goes to the wave's private LDS ring without passing
-//     registers (four `buffer_load ... lds` of 1 KB; eight consecutive lanes fetch the eight
-//     16-byte chunks of one row's 128 bytes, a whole cache line, rotated by row / 2 inside the row
-//     so that the fragment reads spread over all banks);
-//   * B needs no transposition: lane (c, g) of an MFMA wants B[k0 + 8 g + e][column c], e = 0..7,
-//     which is one coalesced 4-byte (NB = 2: 8-byte, the wave's two column blocks are the even
-//     and the odd columns) load per e straight into registers.
-// Three steps beyond the current one are in flight (60 loads, the limit of the wave's load
-// counter), 24 KB per wave.  The values are split in registers right before their MFMAs, like in
-// the large-tile kernel.  At the end the eight partial tiles are added in wave order through LDS
-// (deterministic) and written with the bias.
+//   * A (32 k fp32 of a row are one 128-byte line) goes to the wave's private LDS ring without passing registers
+//     (AL `buffer_load ... lds` of 1 KB, eight rows each: eight consecutive lanes fetch the eight 16-byte chunks
+//     of one row, rotated inside the row so that the fragment reads spread over all banks);
+//   * B needs no transposition: lane (c, g) of an MFMA wants B[k0 + 8 g + e][column c], e = 0..7, which is one
+//     4-, 8- or 16-byte load per e straight into registers: the wave's NB column blocks are the columns NB c + nb.
+// NS - 1 steps beyond the current one are in flight.  The values are split in registers right before their MFMAs, like
+// in the large-tile kernel.  At the end the eight partial tiles are added in wave order through LDS (deterministic)
+// and written with the bias.
 //
-// The shape is bound by what one CU can pull in, (32 + 32 NB) x K x 4 bytes, at the 64 bytes per
-// clock of its vector memory path, not by HBM (the weights are 10 MB) and not by the MFMAs.
+// The shape is bound by what one CU can pull in, W (MB + NB) x K x 4 bytes, at the 64 bytes per clock of its vector
+// memory path, by the instructions of the split (three per element with two bf16 terms, about eight with three fp16 or fp8
+// terms) and by latencies, not by HBM (the weights are 10 MB) and not by the MFMAs.  A CU keeps about 0.4 requests per ns going,
+// whatever it asks for (26 bytes per ns in 64-byte pieces of a row, 42 in 128-byte ones, 71 in 256-byte ones; more steps in
+// flight change nothing), so few columns are spread over as many CUs as there are 16-wide tiles, and 64 x 64 tiles serve the
+// problems of some 256 of them.  Measured (graph replay, us; in brackets the one 32 x 32 / 32 x 64 kernel before, whose steps stood
+// behind branches): 2 x 1280 x 1280 4.2 (7.6), 2 x 320 x 1280 2.6 (4.9), 32 x 1024 x 384 3.6 (7.1), 128 x 1952 x 448 6.5 (10.3),
+// 333 x 456 x 211 3.6 (5.7), 640^3 7.4 (10.6), 768^3 10.7 and 1024^3 13.6 (12.5 and 15.9 on the LDS-tiled kernel), 154 x 2048 x 1280
+// 11.7 (11.4).
 #pragma once
+#include <type_traits>
+
 #include "cascmm_tile_kernel.h"
 
 namespace cascmm {
 
-template <int NB>
+template <int W, int MB, int NB, int AL = W * MB / 8>
 struct WaveK {
-  static constexpr int BM = 32, BN = 32 * NB, BK = 32, NW = 8, NT = 512, NS = 4;
-  static constexpr int A_STAGE = BM * BK * 4;           // 4 KB
-  static constexpr int RING = NS * A_STAGE;             // 16 KB per wave
-  static constexpr int LDS_BYTES = NW * RING;           // 128 KB
-  static constexpr int LOADS = 4 + 16;                  // per wave and step
+  static constexpr int BM = W * MB, BN = W * NB, BK = 32, NW = 8, NT = 512;
+  static constexpr int KM = 512 / W, HALVES = BK / KM;     // k of an MFMA, MFMAs per step
+  static constexpr int REGS = W * W / 64;                  // accumulator registers of a block
+  static constexpr int LOADS = AL + 8 * HALVES;            // per wave and step
+  static constexpr int NS = BM == 16 ? 5 : BM == 32 ? 4 : 2;               // steps in LDS and registers
+  static constexpr int STRAIGHT = BM * BN == 256 ? 8 : BM * BN == 512 ? 6 : BM * BN <= 2048 ? 4 : 2;   // steps of a wave that have straight code
+  static constexpr int A_STAGE = AL * 1024;
+  static constexpr int RING = NS * A_STAGE;                // per wave
+  static constexpr int PART = BM * BN * 4;                 // a wave's partial tile
+  static constexpr int LDS_BYTES = NW * (RING > PART ? RING : PART);
+  static_assert((NS - 1) * LOADS <= 60, "the wait counter has six bits");
 };
 
 typedef __attribute__((address_space(3))) void* wavek_lds_ptr;
@@ -52,17 +65,52 @@ __device__ __forceinline__ void wavek_load_lds_kb(__amdgpu_buffer_rsrc_t rsrc, u
     default: __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (wavek_lds_ptr)dst, 16, voffset, soffset, 3072, 0); break;
   }
 }
+// waits until at most N of the wave's loads are outstanding
+template <int N>
+__device__ __forceinline__ void wavek_wait_loads() {
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | ((N >> 4) << 14));
+}
+// f(0), f(1), ... f(N - 1) with the number as a constant; the second form as long as cond(number) holds, in nested branches
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void wavek_each(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    wavek_each<N, I + 1>(f);
+  }
+}
+template <int N, int I = 0, class C, class F>
+__device__ __forceinline__ void wavek_each_while(C&& cond, F&& f) {
+  if constexpr (I < N) {
+    if (cond(std::integral_constant<int, I>{})) {
+      f(std::integral_constant<int, I>{});
+      wavek_each_while<N, I + 1>(cond, f);
+    }
+  }
+}
+template <int FMT, int W, class ACC>
+__device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lowp<FMT>::Vec b, ACC c) {
+  if constexpr (W == 32) return Lowp<FMT>::mfma(a, b, c);
+  else if constexpr (FMT == CASCMM_FMT_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  else if constexpr (FMT == CASCMM_FMT_FP16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
+}
 
-// Host-checked: fp32 operands, two bf16 terms, products hi.hi + hi.lo + lo.hi; M * lda * 4 and K * ldb * 4 below
-// 2 GiB.  Rows need no alignment (a 16-byte buffer load wants its address on a dword, and its dwords are checked
-// against the buffer's end one by one).  TAIL = 0: K % 32 == 0 and N % (32 NB) == 0.  TAIL = 1: any N, and any K whose
-// rows of A are whole 16-byte chunks, zeros past K (K % 4 == 0, or rows padded by the caller): the chunks past K are
-// fetched from beyond the buffer, as zeros, and so are the rows of B past K.
-template <int NB, int TAIL>
-__global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const GroupParams p) {
-  typedef WaveK<NB> T;
+// Host-checked: fp32 operands, 'tri' products; M * lda * 4 and K * ldb * 4 below 2 GiB.  Rows need no alignment (a 16-byte
+// buffer load wants its address on a dword, and its dwords are checked against the buffer's end one by one).
+// TAIL = 0: K % 32 == 0 and N % (W NB) == 0.  TAIL = 1: any N and K: the rows of B past K lie beyond its buffer (zeros),
+// chunks of A past K are fetched from beyond the buffer, what a row's last chunk holds past K is masked.
+// AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL; what the others hold spoils rows that are not stored).
+template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS>
+__global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
+  typedef WaveK<W, MB, NB, AL> T;
+  typedef Lowp<FMT> L;
+  constexpr int KM = T::KM, HALVES = T::HALVES, REGS = T::REGS;
+  typedef float acc_t __attribute__((ext_vector_type(REGS)));
+  constexpr int PL = L::planes(TERMS);
+  constexpr int CL = AccClasses<FMT, TERMS, false>::kCount;
+  constexpr bool kFold = AccClasses<FMT, TERMS, false>::kChunked;   // the class-0 sum in blocks of NS steps
   extern __shared__ __attribute__((aligned(1024))) unsigned char wavek_smem[];
-  const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, lw = lane & (W - 1), kg = lane / W;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char* ring = wavek_smem + wave * T::RING;
 
@@ -74,122 +122,201 @@ __global__ __launch_bounds__(WaveK<NB>::NT) void cascmm_wavek_kernel(const Group
   const int per = total >> 3;
   int id = blockIdx.x;
   if (id < (per << 3)) id = (id & 7) * per + (id >> 3);
-  const int prob = id / tiles;
+  const void *pa = p.A[0], *pb = p.B[0], *pbias = p.bias[0];
+  void* pc = p.C[0];
+  int prob = 0;
+  if (p.count > 1) {
+    prob = id / tiles;
+    pa = p.A[prob]; pb = p.B[prob]; pbias = p.bias[prob]; pc = p.C[prob];
+  }
   const int t = id - prob * tiles;
   const int tn = t / p.tiles_m, tm = t - tn * p.tiles_m;
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int steps = (p.K + T::BK - 1) / T::BK;                // all of them
   const int my_steps = (steps - wave + T::NW - 1) / T::NW;    // those of this wave: wave, wave + 8, ...
-  const int trips = (steps + T::NW - 1) / T::NW;              // of wave 0, the longest
   const int ldb_bytes = (int)p.ldb * 4;
 
   // rows past M read as zero: the buffer ends with row M - 1 (B: with row K - 1)
-  const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc((void*)p.A[prob], 0, (int)(((int64_t)(p.M - 1) * p.lda + p.K) * 4), 0x00020000);
-  const i32x4 rb = make_rsrc(p.B[prob], ((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
-  int a_voff[4], a_k[4];
+  const int a_end = (int)(((int64_t)(p.M - 1) * p.lda + p.K) * 4), b_end = (int)(((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)pa, 0, a_end, 0x00020000);
+  const i32x4 rb = make_rsrc(pb, b_end);
+  // load j of a step brings rows 8 j + lane / 8 to LDS bytes 1024 j + 16 lane; position pos of row r holds chunk
+  // (pos - rot((r / 2) mod 8)) mod 8 (16-row blocks: the rotations of cascmm_slotn_kernel.h, which explains them)
+  auto rot = [](int h) { return W == 32 ? (h & 7) : (int)((0x75642031u >> (4 * (h & 7))) & 7u); };
+  int a_voff[2], a_k[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = j * 8 + (lane >> 3);
-    const int chunk = ((lane & 7) - (row >> 1)) & 7;
-    a_k[j] = chunk * 4;
-    a_voff[j] = (int)(((int64_t)(m0 + row) * p.lda + chunk * 4) * 4);
+  for (int jp = 0; jp < 2; ++jp) {
+    const int chunk = ((lane & 7) - rot(4 * jp + (lane >> 4))) & 7;
+    a_k[jp] = chunk * 4;
+    a_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + chunk * 4) * 4);
   }
-  const int b_voff = 8 * g * ldb_bytes + (n0 + NB * l31) * 4;
-  // fragment addresses inside a stage: row l31, chunks 4 j2 + 2 g and + 1 at their rotated places
-  int a_frag[2][2];
+  const int rows8 = (int)p.lda * 32;
+  const int b_voff = 8 * kg * ldb_bytes + (n0 + NB * lw) * 4;
+  // fragment of a block of rows: row lw, the chunks of k group kg of MFMA h at their rotated places
+  int a_frag[HALVES][2];
 #pragma unroll
-  for (int j2 = 0; j2 < 2; ++j2)
+  for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) a_frag[j2][h] = l31 * 128 + (((4 * j2 + 2 * g + h) + (l31 >> 1)) & 7) * 16;
+    for (int x = 0; x < 2; ++x) a_frag[h][x] = lw * 128 + ((h * (KM / 4) + 2 * kg + x + rot(lw >> 1)) & 7) * 16;
 
   typedef float bvec __attribute__((ext_vector_type(NB)));
-  bvec Bv[T::NS][2][8];   // raw B of the steps in flight: [stage][k half][e]
+  bvec Bv[T::NS][HALVES][8];   // raw B of the steps in flight
 
-  // the loads of this wave's i-th step (clamped: past its last step a wave fetches that step again
-  // into a stage nobody reads any more)
+  // the loads of this wave's i-th step; past its last step they name places beyond the buffers (zeros, nothing is fetched)
   auto issue = [&](int i, int st) {
-    const int ii = i < my_steps ? i : my_steps - 1;
-    const int step = wave + ii * T::NW;
+    const int k0 = (wave + i * T::NW) * T::BK;
+    const bool real = i < my_steps;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      wavek_load_lds(ra, ring + st * T::A_STAGE + j * 1024, !TAIL || a_k[j] < p.K - step * T::BK ? a_voff[j] : 0x7FFFFFFF, step * T::BK * 4);
+    for (int j = 0; j < AL; ++j)
+      wavek_load_lds(ra, ring + st * T::A_STAGE + j * 1024, !TAIL || a_k[j & 1] < p.K - k0 ? a_voff[j & 1] : 0x7FFFFFFF,
+                     real ? k0 * 4 + j * rows8 : a_end);
 #pragma unroll
-    for (int j2 = 0; j2 < 2; ++j2)
+    for (int h = 0; h < HALVES; ++h)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int soff = (step * T::BK + 16 * j2 + e) * ldb_bytes;
-        if constexpr (NB == 1) Bv[st][j2][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
-        else Bv[st][j2][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0));
+        const int soff = real ? (k0 + KM * h + e) * ldb_bytes : b_end;
+        if constexpr (NB == 1) Bv[st][h][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
+        else if constexpr (NB == 2) Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0));
+        else Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v4f32(rb, b_voff, soff, 0));
       }
+    __builtin_amdgcn_sched_barrier(0);   // (steps in this order: the waits count the loads of younger ones)
   };
 
-  f32x16 acc[NB];
+  acc_t acc[CL][MB][NB], master[kFold ? MB : 1][kFold ? NB : 1];
+  const acc_t zero = {};
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[nb][e] = 0.f;
+    for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+      for (int c = 0; c < CL; ++c) acc[c][mb][nb] = zero;
+      if constexpr (kFold) master[mb][nb] = zero;
+    }
 
-  if (my_steps > 0) {
+  auto step = [&](int i, auto U) {
+    constexpr int u = decltype(U)::value;
+    const unsigned char* stp = ring + u * T::A_STAGE;
 #pragma unroll
-    for (int s = 0; s < T::NS - 1; ++s) issue(s, s);
-  }
-  // `trips` is the same for every wave of the workgroup; a wave with fewer steps idles through
-  // its last trip (the trip count is wave-uniform, so the tests below are scalar branches)
-  for (int i0 = 0; i0 < trips; i0 += T::NS) {
+    for (int h = 0; h < HALVES; ++h) {
+      const int left = p.K - (wave + i * T::NW) * T::BK - KM * h - 8 * kg;   // elements of this lane's k group that exist
+      u32x4 ta[MB][PL];
 #pragma unroll
-    for (int u = 0; u < T::NS; ++u) {
-      const int i = i0 + u;
-      if (i < my_steps) {
-        issue(i + T::NS - 1, (u + T::NS - 1) % T::NS);
-        __builtin_amdgcn_s_waitcnt(0x0F70 | ((3 * T::LOADS) & 0xF) | (((3 * T::LOADS) >> 4) << 14));   // vmcnt(60)
-        const unsigned char* stp = ring + u * T::A_STAGE;
+      for (int mb = 0; mb < MB; ++mb) {
+        const unsigned char* src = stp + mb * (W * 128);
+        const f32x4 x0 = *(const f32x4*)(src + a_frag[h][0]), x1 = *(const f32x4*)(src + a_frag[h][1]);
+        float xa[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+        if constexpr (TAIL) {
 #pragma unroll
-        for (int j2 = 0; j2 < 2; ++j2) {
-          const f32x4 x0 = *(const f32x4*)(stp + a_frag[j2][0]), x1 = *(const f32x4*)(stp + a_frag[j2][1]);
-          float xa[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-          u32x4 ta[2];
-          split8<CASCMM_FMT_BF16, 2>(xa, ta);
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            float xb[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) xb[e] = Bv[u][j2][e][nb];
-            u32x4 tb[2];
-            split8<CASCMM_FMT_BF16, 2>(xb, tb);
-            typedef Lowp<CASCMM_FMT_BF16> L;
-            // smallest products first
-            acc[nb] = L::mfma(L::operand(ta[1], 1), L::operand(tb[0], 0), acc[nb]);
-            acc[nb] = L::mfma(L::operand(ta[0], 0), L::operand(tb[1], 1), acc[nb]);
-            acc[nb] = L::mfma(L::operand(ta[0], 0), L::operand(tb[0], 0), acc[nb]);
-          }
+          for (int e = 0; e < 8; ++e) xa[e] = e < left ? xa[e] : 0.f;
         }
+        split8<FMT, TERMS>(xa, ta[mb]);
+      }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        float xb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
+        u32x4 tb[PL];
+        split8<FMT, TERMS>(xb, tb);
+        // smallest products first
+#pragma unroll
+        for (int s = TERMS - 1; s >= 0; --s)
+#pragma unroll
+          for (int ia = s; ia >= 0; --ia)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+              acc_t& c = acc[AccClasses<FMT, TERMS, false>::index(s)][mb][nb];
+              c = wavek_mfma<FMT, W>(L::operand(ta[mb][L::plane(ia)], ia), L::operand(tb[L::plane(s - ia)], s - ia), c);
+            }
       }
     }
+  };
+  auto fold = [&]() {
+    if constexpr (kFold) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          master[mb][nb] += acc[0][mb][nb];
+          acc[0][mb][nb] = zero;
+        }
+    }
+  };
+  // Up to T::STRAIGHT steps: straight code for their number, which issues no load that nobody needs (a step's loads past the
+  // end of the buffers cost 0.25 us).  More: trips of NS steps without a branch inside, then those that are left, whose loads
+  // are under way already.  In both every path into a step has issued the same loads, so the compiler knows how many are
+  // younger than the ones it waits for.  (With steps skipped by branches it assumed the fewest, and the waits in front of the
+  // splits of B left half the steps in flight.)
+  constexpr int NS = T::NS, L1 = T::LOADS;
+  wavek_each<T::STRAIGHT>([&](auto Z) {
+    constexpr int S = decltype(Z)::value + 1;
+    if (my_steps == S) {
+      wavek_each<(S < NS - 1 ? S : NS - 1)>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+      wavek_each<S>([&](auto U) {
+        constexpr int u = decltype(U)::value, younger = S - 1 - u < NS - 1 ? S - 1 - u : NS - 1;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (u + NS - 1 < S) issue(u + NS - 1, (u + NS - 1) % NS);
+        wavek_wait_loads<younger * L1>();
+        step(u, std::integral_constant<int, u % NS>{});
+      });
+    }
+  });
+  if (my_steps > T::STRAIGHT) {
+    wavek_each<NS - 1>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+    int i = 0;
+    for (; i + NS <= my_steps; i += NS) {
+      wavek_each<NS>([&](auto U) {
+        constexpr int u = decltype(U)::value;
+        issue(i + u + NS - 1, (u + NS - 1) % NS);
+        wavek_wait_loads<(NS - 1) * L1>();
+        step(i + u, U);
+      });
+      fold();
+    }
+    wavek_each_while<NS - 1>([&](auto U) { return i + decltype(U)::value < my_steps; },
+                             [&](auto U) {
+                               constexpr int u = decltype(U)::value;
+                               __builtin_amdgcn_sched_barrier(0);
+                               wavek_wait_loads<(NS - 2 - u) * L1>();
+                               step(i + u, U);
+                             });
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // the redundant loads land before the ring is reused
+  fold();
+  wavek_wait_loads<0>();   // the loads past the last step land before the ring is reused
   __syncthreads();
 
-  // ---- the eight partial tiles meet in LDS: [wave][nb][reg][lane] fp32 -------------------------
+  // ---- the eight partial tiles meet in LDS: [wave][mb][nb][reg][lane] fp32 -------------------------
   float* part = (float*)wavek_smem;
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) part[((wave * NB + nb) * 16 + e) * 64 + lane] = acc[nb][e];
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) {
+        float v = acc[CL - 1][mb][nb][e];
+        if constexpr (CL > 1) {
+#pragma unroll
+          for (int c = CL - 2; c >= 0; --c) v = __builtin_fmaf(v, AccClasses<FMT, TERMS, false>::kFoldScale, acc[c][mb][nb][e]);
+        }
+        if constexpr (kFold) v += master[mb][nb][e];
+        part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
+      }
   __syncthreads();
-  // thread -> (nb, reg, lane) positions tid, tid + 512, ...; of a block a lane holds column l31,
-  // rows 8 (reg / 4) + 4 g + reg % 4
-  float* C = (float*)p.C[prob];
-  const float* bias = (const float*)p.bias[prob];
+  // thread -> (mb, nb, reg, lane) positions tid, tid + 512, ...; of a block a lane holds column lw, rows 4 kg + reg (of 32
+  // rows: 8 (reg / 4) + 4 kg + reg % 4)
+  float* C = (float*)pc;
+  const float* bias = (const float*)pbias;
+  constexpr int OUT = T::BM * T::BN;
 #pragma unroll
-  for (int q = 0; q < NB * 16 * 64 / T::NT; ++q) {
+  for (int q = 0; q < (OUT + T::NT - 1) / T::NT; ++q) {
     const int pos = q * T::NT + tid;
-    const int nb = pos / (16 * 64), e = (pos / 64) % 16, ln = pos % 64;
+    if (OUT % T::NT != 0 && pos >= OUT) break;
+    const int blk = pos / (W * W), e = (pos / 64) % REGS, ln = pos % 64;
+    const int row = m0 + W * (blk / NB) + 8 * (e >> 2) + 4 * (ln / W) + (e & 3);
+    const int col = n0 + NB * (ln & (W - 1)) + blk % NB;
     float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < T::NW; ++w) sum += part[((w * NB + nb) * 16 + e) * 64 + ln];
-    const int row = m0 + 8 * (e >> 2) + 4 * (ln >> 5) + (e & 3);
-    const int col = n0 + NB * (ln & 31) + nb;
+    for (int w = 0; w < T::NW; ++w) sum += part[((w * MB * NB + blk) * REGS + e) * 64 + ln];
     if (row < p.M && (!TAIL || col < p.N)) C[(int64_t)row * p.ldc + col] = sum + (bias ? bias[col] : 0.f);
   }
 }

@@ -1,0 +1,46 @@
+"""The kernels that split K over the eight waves of a workgroup (cascmm_wavek_kernel.h): every tile, at the edges of its tile, of a
+32-k step, of the straight code's numbers of steps and of the ring."""
+import pytest
+import torch
+
+from basedxl_amd import _lib, cascaded_lowp_matmul
+
+pytestmark = pytest.mark.gpu
+
+_TILES = [n for n in _lib.variant_names() if "_wavek_" in n]
+
+
+@pytest.mark.parametrize("name", _TILES)
+@pytest.mark.parametrize("K", [1, 3, 32, 33, 255, 257, 511, 1023, 1280, 1310, 2081, 2565, 3333])
+def test_every_number_of_steps_is_exact_on_integers(name, K):
+    """One, two, ... steps per wave and the trips behind the straight code; K off the steps and off 16-byte chunks, NaNs between the rows
+    of A and beside B's columns, columns and rows past the edge of C untouched."""
+    bm, bn = (int(x) for x in name.split("_")[0][1:].split("x")[:2])
+    lowp, terms = name.split("_")[2].split("x")
+    g = torch.Generator().manual_seed(K)
+    for M, N in ((bm, bn), (7, 2 * bn + 1), (bm + 9, bn - 3)):
+        a, b = (torch.randint(-60, 61, s, generator=g) for s in ((M, K), (K, N)))
+        frame = torch.full((M, K + 3), float("nan"), device="cuda:0")
+        frame[:, :K] = a.float().to("cuda:0")
+        out = torch.full((M + 1, N + 1), -77.0, device="cuda:0")
+        print("wavek", name, (M, K, N), flush=True)
+        got = out[:M, :N]
+        cascaded_lowp_matmul(frame[:, :K], b.float().to("cuda:0"), out=got, lowp=lowp, terms=int(terms), variant=_lib.variant_names().index(name))
+        assert torch.equal(got.cpu().long(), a @ b), (M, N)
+        assert bool((out[M] == -77.0).all()) and bool((out[:, N] == -77.0).all())
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 1280, 1280), (16, 2047, 477), (130, 1281, 448), (600, 600, 600), (1024, 1024, 1024), (3, 5120, 40)])
+def test_a_call_repeats_its_bits_and_keeps_non_finite_values_to_their_rows(M, K, N):
+    a, b = torch.randn(M, K, device="cuda:0"), torch.randn(K, N, device="cuda:0")
+    a[M // 2, K - 1] = float("inf")
+    b[0, N // 3] = float("nan")
+    print("wavek", (M, K, N), flush=True)
+    first = cascaded_lowp_matmul(a, b)
+    for _ in range(3):
+        assert torch.equal(cascaded_lowp_matmul(a, b).nan_to_num(7.0), first.nan_to_num(7.0))
+    bad = ~torch.isfinite(first)
+    assert bool(bad[M // 2].all()) and bool(bad[:, N // 3].all()) and int(bad.sum()) == M + N - 1
+    want = a.double() @ b.double()
+    ok = ~bad
+    assert float((first.double() - want)[ok].norm() / want[ok].norm()) < 1.8e-5
