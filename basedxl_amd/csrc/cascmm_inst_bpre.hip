@@ -21,6 +21,13 @@ static const VariantDesc kTable[] = {
     CASCMM_W512_VARIANT("t256x320x32_w512_bf16x2_tri_bpre", 1),
     CASCMM_W512_EDGE_VARIANT("t256x320x32_w512_edge_bf16x2_tri_bpre", 1, 5),
     CASCMM_W512_EDGE_VARIANT("t256x256x32_w512_edge_bf16x2_tri_bpre", 1, 4),
+    // K split over the eight waves of a workgroup: small problems
+    CASCMM_WAVEK_VARIANT_B("t16x16x32_wavek_bf16x2_tri_bpre", 16, 1, 1, BF, 2, 1),
+    CASCMM_WAVEK_VARIANT_B("t16x32x32_wavek_bf16x2_tri_bpre", 16, 1, 2, BF, 2, 1),
+    CASCMM_WAVEK_VARIANT_B("t16x64x32_wavek_bf16x2_tri_bpre", 16, 1, 4, BF, 2, 1),
+    CASCMM_WAVEK_VARIANT_B("t32x32x32_wavek_bf16x2_tri_bpre", 32, 1, 1, BF, 2, 1),
+    CASCMM_WAVEK_VARIANT_B("t32x64x32_wavek_bf16x2_tri_bpre", 16, 2, 4, BF, 2, 1),
+    CASCMM_WAVEK_VARIANT_B("t64x64x32_wavek_bf16x2_tri_bpre", 16, 4, 4, BF, 2, 1),
     CASCMM_TILE_VARIANT_BPRE("t128x128x32_w4x2x1_d2_bf16x3_tri_bpre", 128, 128, 32, 4, 2, 1, 2, 4, BF, 3, false),
     CASCMM_TILE_VARIANT_BPRE("t128x128x32_w4x2x1_d2_fp16x3_tri_bpre", 128, 128, 32, 4, 2, 1, 2, 4, FP, 3, false),
     CASCMM_TILE_VARIANT_BPRE("t128x128x32_w4x2x1_d2_fp8x3_tri_bpre", 128, 128, 32, 4, 2, 1, 2, 4, F8, 3, false),

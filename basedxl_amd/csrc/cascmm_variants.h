@@ -240,26 +240,33 @@ int launch_w512_edge(const GroupParams& p, hipStream_t stream) {
 // the tiles of KIND_WAVEK that the selection functions know
 constexpr bool wavek_for_shapes(int bm, int bn) { return bm == 32 && bn >= 32; }
 // skinny and small problems, K split over the waves of a workgroup
-template <int W, int MB, int NB, int FMT, int TERMS>
-int launch_wavek(const GroupParams& p, hipStream_t stream) {
-  typedef WaveK<W, MB, NB> T;
-  constexpr int ALL = T::BM / 8, FEW = T::BM == 16 ? 1 : ALL;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS>; return CASCMM_OK; }
-  if (p.glu || p.k_splits > 1 || p.count < 1) return CASCMM_ERR_BAD_VARIANT;
-  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  const bool tail = p.N % T::BN != 0 || p.K % T::BK != 0, few = T::BM == 16 && p.M <= 8;
-  void (*kfn)(const GroupParams) = few ? (tail ? cascmm_wavek_kernel<W, MB, NB, FEW, 1, FMT, TERMS> : cascmm_wavek_kernel<W, MB, NB, FEW, 0, FMT, TERMS>)
-                                       : (tail ? cascmm_wavek_kernel<W, MB, NB, ALL, 1, FMT, TERMS> : cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS>);
-  const int lds = few ? WaveK<W, MB, NB, FEW>::LDS_BYTES : T::LDS_BYTES;
+template <int W, int MB, int NB, int FMT, int TERMS, int BPRE, int GLU>
+int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
+  constexpr int ALL = W * MB / 8, FEW = W * MB == 16 ? 1 : ALL;
+  const bool tail = (!GLU && p.N % (W * NB) != 0) || p.K % 32 != 0, few = FEW != ALL && p.M <= 8;
+  void (*kfn)(const GroupParams) = few ? (tail ? cascmm_wavek_kernel<W, MB, NB, FEW, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, FEW, 0, FMT, TERMS, BPRE, GLU>)
+                                       : (tail ? cascmm_wavek_kernel<W, MB, NB, ALL, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS, BPRE, GLU>);
+  const int lds = few ? WaveK<W, MB, NB, FEW>::LDS_BYTES : WaveK<W, MB, NB, ALL>::LDS_BYTES;
   static LdsFlags lds_set[4];
   if (!ensure_lds((const void*)kfn, lds, lds_set[(tail ? 1 : 0) + (few ? 2 : 0)])) return CASCMM_ERR_LAUNCH;
   GroupParams q = p;
-  q.tiles_m = (p.M + T::BM - 1) / T::BM;
-  q.tiles_n = (p.N + T::BN - 1) / T::BN;
+  q.tiles_m = (p.M + W * MB - 1) / (W * MB);
+  q.tiles_n = (p.N + W * NB - 1) / (W * NB);
   const int64_t grid = (int64_t)q.count * q.tiles_m * q.tiles_n;
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
-  if (launch_kernel(kfn, dim3((unsigned)grid), dim3(T::NT), (size_t)lds, stream, q) != hipSuccess) return CASCMM_ERR_LAUNCH;
-  return CASCMM_OK;
+  return launch_kernel(kfn, dim3((unsigned)grid), dim3(512), (size_t)lds, stream, q) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
+}
+template <int W, int MB, int NB, int FMT, int TERMS, int BPRE>
+int launch_wavek(const GroupParams& p, hipStream_t stream) {
+  constexpr bool kGlu = W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16;
+  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<W, MB, NB, W * MB / 8, 0, FMT, TERMS, BPRE>; return CASCMM_OK; }
+  if ((p.glu && (!kGlu || p.glu != 1 || p.N % 64 != 0)) || p.k_splits > 1 || p.count < 1 || p.K <= 0) return CASCMM_ERR_BAD_VARIANT;
+  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 16 * Lowp<FMT>::planes(TERMS) : (int64_t)p.K * p.ldb * 4) > 0x7FFFFFFF)
+    return CASCMM_ERR_TOO_LARGE;
+  if constexpr (kGlu) {
+    if (p.glu) return launch_wavek_kernel<W, MB, NB, FMT, TERMS, BPRE, 1>(p, stream);
+  }
+  return launch_wavek_kernel<W, MB, NB, FMT, TERMS, BPRE, 0>(p, stream);
 }
 
 // K split of the fp8-rate kernel (row tile bm = 256 or 128) for problems with fewer tiles than CUs:
@@ -430,10 +437,11 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
   {NAME, KIND_F8K64, CASCMM_DT_F32, CASCMM_FMT_FP8, 3, false, F8Tile<MT>::T::BM, F8Tile<MT>::T::BN, F8Tile<MT>::T::BK, \
    F8Tile<MT>::T::NT, F8Tile<MT>::T::LDS_BYTES, true, false, &launch_f8k64<BPRE, MT>, BPRE}
 
-#define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS)                                                                   \
+#define CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, BPRE)                                                        \
   {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, WaveK<W, MB, NB>::BM, WaveK<W, MB, NB>::BN, WaveK<W, MB, NB>::BK,   \
-   WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS>, false, false,   \
-   !wavek_for_shapes(W * MB, W * NB)}
+   WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0,   \
+   W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16, BPRE || !wavek_for_shapes(W * MB, W * NB)}
+#define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS) CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, 0)
 
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \
   {NAME, KIND_W512, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512::BM, W512::BN, 32, W512::NT, W512::LDS_BYTES, true, \

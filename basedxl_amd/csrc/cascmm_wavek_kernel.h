@@ -23,7 +23,8 @@
 // problems of some 256 of them.  Measured (graph replay, us; in brackets the one 32 x 32 / 32 x 64 kernel before, whose steps stood
 // behind branches): 2 x 1280 x 1280 4.2 (7.6), 2 x 320 x 1280 2.6 (4.9), 32 x 1024 x 384 3.6 (7.1), 128 x 1952 x 448 6.5 (10.3),
 // 333 x 456 x 211 3.6 (5.7), 640^3 7.4 (10.6), 768^3 10.7 and 1024^3 13.6 (12.5 and 15.9 on the LDS-tiled kernel), 154 x 2048 x 1280
-// 11.7 (11.4).
+// 11.7 (11.4).  With the weight prepared, two 16-byte loads per step and 16 columns and half the instructions: 2 x 2816 x 1280 5.7 (9.3
+// raw), 154 x 2048 x 1280 9.5, x 640 7.6, 77 x 2048 x 2560 9.5, 108 x 592 x 3155 6.3 (10.0 on the 64 x 80 tile, eager).
 #pragma once
 #include <type_traits>
 
@@ -31,13 +32,14 @@
 
 namespace cascmm {
 
-template <int W, int MB, int NB, int AL = W * MB / 8>
+// B_LOADS: loads of B per step and wave
+template <int W, int MB, int NB, int AL = W * MB / 8, int B_LOADS = W / 2>
 struct WaveK {
   static constexpr int BM = W * MB, BN = W * NB, BK = 32, NW = 8, NT = 512;
   static constexpr int KM = 512 / W, HALVES = BK / KM;     // k of an MFMA, MFMAs per step
   static constexpr int REGS = W * W / 64;                  // accumulator registers of a block
-  static constexpr int LOADS = AL + 8 * HALVES;            // per wave and step
-  static constexpr int NS = BM == 16 ? 5 : BM == 32 ? 4 : 2;               // steps in LDS and registers
+  static constexpr int LOADS = AL + B_LOADS;               // per wave and step
+  static constexpr int NS = BM == 16 && LOADS <= 15 ? 5 : BM <= 32 ? (LOADS <= 20 ? 4 : 3) : 2;               // steps in LDS and registers
   static constexpr int STRAIGHT = BM * BN == 256 ? 8 : BM * BN == 512 ? 6 : BM * BN <= 2048 ? 4 : 2;   // steps of a wave that have straight code
   static constexpr int A_STAGE = AL * 1024;
   static constexpr int RING = NS * A_STAGE;                // per wave
@@ -95,14 +97,23 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
   else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
 }
 
+template <int W, int NB, int FMT, int TERMS, int BPRE, int GLU>
+constexpr int wavek_b_loads() {
+  return BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : (W / 2) * (GLU ? 2 : 1);
+}
+
 // Host-checked: fp32 operands, 'tri' products; M * lda * 4 and K * ldb * 4 below 2 GiB.  Rows need no alignment (a 16-byte
 // buffer load wants its address on a dword, and its dwords are checked against the buffer's end one by one).
 // TAIL = 0: K % 32 == 0 and N % (W NB) == 0.  TAIL = 1: any N and K: the rows of B past K lie beyond its buffer (zeros),
 // chunks of A past K are fetched from beyond the buffer, what a row's last chunk holds past K is masked.
 // AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL; what the others hold spoils rows that are not stored).
-template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS>
+// BPRE = 1: B is a prepared weight, [plane][4 ceil(K/32)][N] operand slots, a load per plane and column block (block nb: columns
+// W nb + c).  GLU = 1 (64-wide tiles): the gated store, C has N / 2 columns; a prepared weight alternates 32 value and 32 gate columns, of a
+// raw one blocks 0 and 1 are value columns 2 c + nb, blocks 2 and 3 their gates from the second half.
+template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
-  typedef WaveK<W, MB, NB, AL> T;
+  static_assert(!GLU || (W == 16 && NB == 4), "a value block and its gate block in one tile");
+  typedef WaveK<W, MB, NB, AL, wavek_b_loads<W, NB, FMT, TERMS, BPRE, GLU>()> T;
   typedef Lowp<FMT> L;
   constexpr int KM = T::KM, HALVES = T::HALVES, REGS = T::REGS;
   typedef float acc_t __attribute__((ext_vector_type(REGS)));
@@ -137,7 +148,8 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   const int ldb_bytes = (int)p.ldb * 4;
 
   // rows past M read as zero: the buffer ends with row M - 1 (B: with row K - 1)
-  const int a_end = (int)(((int64_t)(p.M - 1) * p.lda + p.K) * 4), b_end = (int)(((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
+  const int a_end = (int)(((int64_t)(p.M - 1) * p.lda + p.K) * 4), b_plane = BPRE ? (int)prepared_kgroups(p.K) * p.N * 16 : 0,
+            b_end = BPRE ? PL * b_plane : (int)(((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)pa, 0, a_end, 0x00020000);
   const i32x4 rb = make_rsrc(pb, b_end);
   // load j of a step brings rows 8 j + lane / 8 to LDS bytes 1024 j + 16 lane; position pos of row r holds chunk
@@ -151,7 +163,8 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     a_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + chunk * 4) * 4);
   }
   const int rows8 = (int)p.lda * 32;
-  const int b_voff = 8 * kg * ldb_bytes + (n0 + NB * lw) * 4;
+  // (GLU, raw: two value columns and, `gates` bytes further, their gates)
+  const int b_voff = BPRE ? (kg * p.N + n0 + lw) * 16 : 8 * kg * ldb_bytes + (GLU ? (n0 >> 1) + 2 * lw : n0 + NB * lw) * 4, gates = p.N * 2;
   // fragment of a block of rows: row lw, the chunks of k group kg of MFMA h at their rotated places
   int a_frag[HALVES][2];
 #pragma unroll
@@ -160,7 +173,9 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     for (int x = 0; x < 2; ++x) a_frag[h][x] = lw * 128 + ((h * (KM / 4) + 2 * kg + x + rot(lw >> 1)) & 7) * 16;
 
   typedef float bvec __attribute__((ext_vector_type(NB)));
-  bvec Bv[T::NS][HALVES][8];   // raw B of the steps in flight
+  // B of the steps in flight, raw or as slots
+  bvec Bv[BPRE ? 1 : T::NS][HALVES][8];
+  u32x4 Bp[BPRE ? T::NS : 1][HALVES][NB][PL];
 
   // the loads of this wave's i-th step; past its last step they name places beyond the buffers (zeros, nothing is fetched)
   auto issue = [&](int i, int st) {
@@ -173,12 +188,24 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 #pragma unroll
     for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < (BPRE ? 0 : 8); ++e) {
         const int soff = real ? (k0 + KM * h + e) * ldb_bytes : b_end;
-        if constexpr (NB == 1) Bv[st][h][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
+        if constexpr (GLU) {
+          const f32x2_ld v = llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0), g = llvm_raw_buffer_load_v2f32(rb, b_voff + gates, soff, 0);
+          Bv[st][h][e] = (bvec){v[0], v[1], g[0], g[1]};
+        } else if constexpr (NB == 1) Bv[st][h][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
         else if constexpr (NB == 2) Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0));
         else Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v4f32(rb, b_voff, soff, 0));
       }
+    if constexpr (BPRE) {
+#pragma unroll
+      for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int pl = 0; pl < PL; ++pl)
+            Bp[st][h][nb][pl] = __builtin_bit_cast(u32x4, llvm_raw_buffer_load_v4f32(rb, b_voff + nb * (W * 16), real ? ((k0 + KM * h) >> 3) * p.N * 16 + pl * b_plane : b_end, 0));
+    }
     __builtin_amdgcn_sched_barrier(0);   // (steps in this order: the waits count the loads of younger ones)
   };
 
@@ -213,11 +240,16 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
-        float xb[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
         u32x4 tb[PL];
-        split8<FMT, TERMS>(xb, tb);
+        if constexpr (BPRE) {
+#pragma unroll
+          for (int pl = 0; pl < PL; ++pl) tb[pl] = Bp[u][h][nb][pl];
+        } else {
+          float xb[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
+          split8<FMT, TERMS>(xb, tb);
+        }
         // smallest products first
 #pragma unroll
         for (int s = TERMS - 1; s >= 0; --s)
@@ -306,6 +338,26 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   // rows: 8 (reg / 4) + 4 kg + reg % 4)
   float* C = (float*)pc;
   const float* bias = (const float*)pbias;
+  if constexpr (GLU) {
+    // the gate blocks are two further on
+    const int half = p.N >> 1;
+#pragma unroll
+    for (int q = 0; q < T::BM * 32 / T::NT; ++q) {
+      const int pos = q * T::NT + tid;
+      const int blk = pos / 256, e = (pos / 64) % 4, ln = pos % 64;
+      const int row = m0 + 16 * (blk >> 1) + 4 * (ln >> 4) + e, pair = blk & 1;
+      const int col = (n0 >> 1) + (BPRE ? 16 * pair + (ln & 15) : 2 * (ln & 15) + pair);
+      const int at = (((blk >> 1) * 4 + pair) * 4 + e) * 64 + ln;
+      float v = 0.f, g = 0.f;
+#pragma unroll
+      for (int w = 0; w < T::NW; ++w) {
+        v += part[w * (MB * 4 * 256) + at];
+        g += part[w * (MB * 4 * 256) + at + 2 * 256];
+      }
+      if (row < p.M) C[(int64_t)row * p.ldc + col] = gated_value(v + (bias ? bias[col] : 0.f), g + (bias ? bias[half + col] : 0.f));
+    }
+    return;
+  }
   constexpr int OUT = T::BM * T::BN;
 #pragma unroll
   for (int q = 0; q < (OUT + T::NT - 1) / T::NT; ++q) {
@@ -313,7 +365,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     if (OUT % T::NT != 0 && pos >= OUT) break;
     const int blk = pos / (W * W), e = (pos / 64) % REGS, ln = pos % 64;
     const int row = m0 + W * (blk / NB) + 8 * (e >> 2) + 4 * (ln / W) + (e & 3);
-    const int col = n0 + NB * (ln & (W - 1)) + blk % NB;
+    const int col = n0 + (BPRE ? W * (blk % NB) + (ln & (W - 1)) : NB * (ln & (W - 1)) + blk % NB);
     float sum = 0.f;
 #pragma unroll
     for (int w = 0; w < T::NW; ++w) sum += part[((w * MB * NB + blk) * REGS + e) * 64 + ln];

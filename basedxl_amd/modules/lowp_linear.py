@@ -55,10 +55,10 @@ class BasedXLLowPLinear(nn.Module):
         pw = self._prepared_weight
         if self.lowp == "fp8":
             y = None
-        elif not self.prepared or (x.dtype == torch.float32 and x.numel() < 32 * self.in_features):
+        elif not self.prepared:
             y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
         elif pw is not None and pw.device == self.weight.device:
-            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 32)
+            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
         else:
             y = None
         if y is not None:
@@ -67,9 +67,9 @@ class BasedXLLowPLinear(nn.Module):
             if self._prepared_weight is None or self._prepared_weight.device != self.weight.device:
                 self._prepared_weight = PreparedWeight(self.weight, lowp=self.lowp, terms=self.terms)
             x2 = x.reshape(-1, self.in_features)
-            # a handful of rows (time embeddings): the raw fp32 weight has split-K kernels that stream
-            # it with every CU, the prepared path has none
-            few_rows = x2.shape[0] < 32 and x2.dtype == torch.float32
+            # a handful of rows: three terms and K off 8 have kernels for the raw weight only (two bf16 terms and K of 8: 2 x 2816 x 1280
+            # 9.4 us raw, 5.7 prepared)
+            few_rows = x2.shape[0] < 32 and x2.dtype == torch.float32 and ((self.lowp, self.terms) != ("bf16", 2) or self.in_features % 8 != 0)
             if not few_rows and self._prepared_weight.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), self.products):
                 return cascaded_lowp_matmul(x, self._prepared_weight, bias=self.bias, products=self.products)
         if self.lowp == "fp8" and (self._weight_exp is None or self._weight_exp.device != self.weight.device):

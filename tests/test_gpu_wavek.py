@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from basedxl_amd import _lib, cascaded_lowp_matmul
+from basedxl_amd import PreparedWeight, _lib, cascaded_lowp_matmul
 
 pytestmark = pytest.mark.gpu
 
@@ -11,7 +11,7 @@ _TILES = [n for n in _lib.variant_names() if "_wavek_" in n]
 
 
 @pytest.mark.parametrize("name", _TILES)
-@pytest.mark.parametrize("K", [1, 3, 32, 33, 255, 257, 511, 1023, 1280, 1310, 2081, 2565, 3333])
+@pytest.mark.parametrize("K", [1, 3, 32, 33, 72, 255, 264, 511, 1016, 1280, 1310, 2081, 2568, 3333])
 def test_every_number_of_steps_is_exact_on_integers(name, K):
     """One, two, ... steps per wave and the trips behind the straight code; K off the steps and off 16-byte chunks, NaNs between the rows
     of A and beside B's columns, columns and rows past the edge of C untouched."""
@@ -24,8 +24,15 @@ def test_every_number_of_steps_is_exact_on_integers(name, K):
         frame[:, :K] = a.float().to("cuda:0")
         out = torch.full((M + 1, N + 1), -77.0, device="cuda:0")
         print("wavek", name, (M, K, N), flush=True)
-        got = out[:M, :N]
-        cascaded_lowp_matmul(frame[:, :K], b.float().to("cuda:0"), out=got, lowp=lowp, terms=int(terms), variant=_lib.variant_names().index(name))
+        got, w, variant = out[:M, :N], b.float().to("cuda:0"), _lib.variant_names().index(name)
+        if name.endswith("_bpre"):
+            if K % 8 != 0 or (K < 64 and K % 32 != 0):
+                with pytest.raises(_lib.CascmmError):
+                    cascaded_lowp_matmul(frame[:, :K], PreparedWeight(w, lowp=lowp, terms=int(terms)), variant=variant)
+                continue
+            assert torch.equal(cascaded_lowp_matmul(frame[:, :K], PreparedWeight(w, lowp=lowp, terms=int(terms)), variant=variant).cpu().long(), a @ b), (M, N)
+            continue
+        cascaded_lowp_matmul(frame[:, :K], w, out=got, lowp=lowp, terms=int(terms), variant=variant)
         assert torch.equal(got.cpu().long(), a @ b), (M, N)
         assert bool((out[M] == -77.0).all()) and bool((out[:, N] == -77.0).all())
 
