@@ -33,6 +33,8 @@ static const std::vector<VariantDesc>& table() {
     v.insert(v.end(), p, p + n);
     p = variants_h16(&n);
     v.insert(v.end(), p, p + n);
+    p = variants_hwk(&n);
+    v.insert(v.end(), p, p + n);
     return v;
   }();
   return t;
@@ -136,7 +138,7 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   // K in whole 32-k steps, or a tail of whole 16-byte chunks (a weight less than one 64-k stage deep is not worth keeping
   // split: such a prepared operand is refused)
   if ((v.kind == KIND_SLOTK || v.kind == KIND_W512E) && (q.K == 0 || (q.K % 32 != 0 && !(q.chunked && (!q.bpre || q.K >= 64))))) return false;
-  if (v.fast && !any_rows && v.kind != KIND_H16 && (v.kind != KIND_W512E || q.glu) && q.K % v.BK != 0) return false;
+  if (v.fast && !any_rows && v.kind != KIND_H16 && v.kind != KIND_HWK && (v.kind != KIND_W512E || q.glu) && q.K % v.BK != 0) return false;
   if (v.kind == KIND_SPLITK && (q.M > 5 * v.BM || q.K < 4 * v.BK)) return false;  // skinny: few row tiles, deep K
   if (v.kind == KIND_F8K64 && (q.products != CASCMM_PROD_TRI || q.K % v.BK != 0 || q.K == 0 || q.glu ||
                                f8k64_slot_bytes(q.M, q.K) > INT32_MAX || f8k64_slot_bytes(q.N, q.K) > INT32_MAX))
@@ -159,7 +161,8 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
   // (32-bit byte offsets down B, a raw one's two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
-  if (v.kind == KIND_H16 && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (q.bpre ? beyond_i32((q.K + 63) / 64, q.N, 128) : beyond_i32(q.K + 64, q.ldb, 2))))
+  if (v.kind == KIND_HWK && v.call_only && !q.call) return false;
+  if ((v.kind == KIND_H16 || v.kind == KIND_HWK) && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (q.bpre ? beyond_i32((q.K + 63) / 64, q.N, 128) : beyond_i32(q.K + 64, q.ldb, 2))))
     return false;
   if (q.glu && !v.glu) return false;
   if (q.glu_slots && v.kind != KIND_W512) return false;
@@ -289,10 +292,11 @@ static const std::vector<VariantInfo>& variant_info() {
   return info;
 }
 static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Problem& q, int count, double tiles, int64_t k_per) {
-  const double k = v.kind == KIND_WAVEK ? (double)(((k_per + 31) / 32 + 7) / 8) : v.kind == KIND_SLOTK ? (double)((k_per + 255) / 256 * 4) : (double)k_per / 64.0;
-  const double per = tiles / kNumCUs, mb = (double)count * (double)q.K * (double)q.N * 4.0e-6;
+  const double k = v.kind == KIND_WAVEK || v.kind == KIND_HWK ? (double)(((k_per + v.BK - 1) / v.BK + 7) / 8) : v.kind == KIND_SLOTK ? (double)((k_per + 255) / 256 * 4) : (double)k_per / 64.0;
+  const double per = tiles / kNumCUs, mb = (double)count * (double)q.K * (double)q.N * (double)dtype_size(q.dtype) * 1.0e-6;
+  const double few = v.kind == KIND_HWK ? 4 : 8;   // steps of a wave's straight code
   const double full = v.BM * v.BN <= 512 ? 0.0 : std::ceil(per) - 1.0, fill = per - full;
-  const double lone = k * t.s0 + (k > 8 ? t.deep * (k - 8) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
+  const double lone = k * t.s0 + (k > few ? t.deep * (k - few) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
   const double us = t.c0 + full * (t.c1 + k * t.r1) + std::pow(std::pow(lone, t.x) + std::pow(shared, t.x), 1.0 / t.x);
   return q.N % v.BN != 0 || q.M % v.BM != 0 ? us * (1.0 + t.edge) : us;
 }
@@ -339,6 +343,35 @@ static double h16_estimate_us(const VariantDesc& v, const Problem& q, double til
       const double k = (double)((k_per + v.BK - 1) / v.BK * v.BK) * (q.bpre ? 1.0 : c.raw);
       return c.start + (full + (rem > 0 ? 1.0 : 0.0)) * c.end + k * (full * c.s1 + last);
     }
+  return 1e9;
+}
+
+// The same problems with K over eight waves (KIND_HWK), with a launch's constants of kCallCost (`form`: 0 prepared, 1 raw, 2 gated).
+// Fitted to 326 shapes of 2 - 2600 rows, K and widths 256 - 10240 (fp16, graph replay over three sets of operands, every tile forced
+// in turn), mean error 0.03 - 0.08.  They win where the tiles about fit the CUs at once (2 x 1280 x 1280 prepared 3.2 us, 6.9 on the four-wave kernels;
+// 154 x 2048 x 1280 5.6, 10.3), and lose behind that, where every tile pays its launch and its meeting in LDS (2048 x 640 x 640 raw
+// 12.0 us, 7.3).  The estimates decide, and within 4 % of each other (their error) the four-wave kernels stay: 0.76 (prepared), 0.82 (raw) and 0.90
+// (gated) of the time without these kernels over the shapes, 2 % behind the fastest of all.
+struct HwkCost { int BM, BN, form; CallCost c; };
+static const HwkCost kHwkCost[] = {
+    {16, 16, 0, {nullptr, 2.7, 0.143, 0.345, 0, 20.2, 2.37, 0, 0.197, 0}},
+    {16, 32, 0, {nullptr, 2.61, 0.289, 0.51, 0, 15.7, 2.01, 0, 0.281, 0}},
+    {16, 64, 0, {nullptr, 2.72, 0.492, 0.214, 0.388, 14.9, 1.18, 0.902, 0.383, 0}},
+    {32, 32, 0, {nullptr, 2.8, 0.395, 0.411, 1.12, 12, 1.98, 0.735, 0.184, 0}},
+    {32, 64, 0, {nullptr, 2.91, 0.604, 0.484, 1.06, 19.6, 1.13, 1.19, 0.244, 0}},
+    {64, 64, 0, {nullptr, 3.33, 0.867, 0.773, 1.74, 40, 1.08, 1.81, 0.134, 0}},
+    {16, 32, 1, {nullptr, 2.43, 0.472, 0.805, 0, 30.3, 2.04, 0, 0.5, 0.0752}},
+    {16, 64, 1, {nullptr, 2.58, 0.861, 0.328, 1.32, 40, 1.03, 1.1, 0.5, 0.0352}},
+    {32, 32, 1, {nullptr, 2.68, 0.509, 0.39, 1.31, 40, 1, 0.934, 0.5, 0.0326}},
+    {32, 64, 1, {nullptr, 2.87, 0.978, 0.485, 1.74, 40, 1.05, 1.23, 0.443, 0.0123}},
+    {64, 64, 1, {nullptr, 3.46, 1.28, 1.02, 2.33, 40, 1.6, 1.99, 0.5, 0}},
+    {16, 64, 2, {nullptr, 3.14, 0.0359, 0.141, 0.86, 6.09, 7.35, 0.455, 0.05, 0.0069}},
+    {32, 64, 2, {nullptr, 3.6, 0.264, 0.0524, 1.97, 6.36, 8, 0.586, 0.0225, 0.00763}},
+    {64, 64, 2, {nullptr, 4.08, 0.02, 0.312, 2.82, 6.07, 7.47, 0.839, 0.0025, 0.007}},
+};
+static double hwk_estimate_us(const VariantDesc& v, const Problem& q, int count, double tiles) {
+  for (const HwkCost& t : kHwkCost)
+    if (t.BM == v.BM && t.BN == v.BN && t.form == (q.glu ? 2 : q.bpre ? 0 : 1)) return 1.04 * call_estimate_us(t.c, v, q, count, tiles, q.K);
   return 1e9;
 }
 
@@ -404,6 +437,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   const double tiles = (double)count * (double)((q.M + v.BM - 1) / v.BM) * (double)((q.N + v.BN - 1) / v.BN);
   const double full = (double)(int64_t)(tiles / kNumCUs);
   const double rem = tiles - full * kNumCUs;
+  if (v.kind == KIND_HWK) return hwk_estimate_us(v, q, count, tiles);
   if (v.kind == KIND_SPLITK) {
     if (q.call) return 1e9;   // (the small tiles of KIND_WAVEK and the K-over-waves tiles: 3 x 4416 x 2752 18 us here, 12.1 there)
     // Problems with too few tiles to occupy the chip: splitting K wins whenever the plain tile

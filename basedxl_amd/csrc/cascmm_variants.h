@@ -22,7 +22,8 @@ namespace cascmm {
 // over workgroups, cascmm_ksplit.h)
 // KIND_SLOTK: K split over the waves of a workgroup, right operand prepared (64 x 160 and 64 x 80 tiles) or raw (64 x 160),
 // one problem per launch (workspace as KIND_H16)
-enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7, KIND_W512E = 8 };
+// KIND_HWK: KIND_H16's problems in one launch, K split over the waves of a workgroup (no workspace)
+enum VariantKind { KIND_TILE = 0, KIND_SPLITK = 1, KIND_W512 = 2, KIND_F8K64 = 3, KIND_WAVEK = 4, KIND_SLOTK = 5, KIND_F16K = 6, KIND_H16 = 7, KIND_W512E = 8, KIND_HWK = 9 };
 constexpr int kNumCUs = 256;  // MI355X: what the cost model's constants were measured on
 constexpr int kMaxDevices = 64;
 
@@ -512,5 +513,6 @@ const VariantDesc* variants_io16(int* n);
 const VariantDesc* variants_bpre(int* n);
 const VariantDesc* variants_chain(int* n);
 const VariantDesc* variants_h16(int* n);
+const VariantDesc* variants_hwk(int* n);
 
 }  // namespace cascmm
