@@ -256,6 +256,10 @@ static const CallCost kCallCost[] = {
     {"t256x256x32_w512_edge_bf16x2_tri", 11.1, 2.98, 4.74, 10.2, 40, 4.25, 4.83, 0, 0.00177},
     {"t256x320x32_w512_edge_bf16x2_tri", 12, 3.38, 5, 13.4, 19, 2.39, 5.8, 0, 0.013},
     {"t256x320x32_w512_bf16x2_tri", 11.9, 3.21, 5, 6.51, 40, 2.24, 6.86, 0, 0.02},
+    // three fp16 terms (150 shapes, mean error 0.06 - 0.09)
+    {"t16x16x32_wavek_fp16x3_tri", 2.38, 0.675, 0.768, 0, 19.6, 1.61, 0, 0.0438, 0},
+    {"t16x32x32_wavek_fp16x3_tri", 2.54, 1.12, 1.57, 0, 16.2, 6.97, 0, 0.0319, 0},
+    {"t32x32x32_wavek_fp16x3_tri", 2.75, 1.46, 0.223, 1.49, 35.4, 1, 1.66, 0, 0},
     // prepared weights (460 shapes, mean error 0.01 - 0.05; the kernel chosen is 1 % behind the fastest, 8.6 % with the constants above)
     {"t16x16x32_wavek_bf16x2_tri_bpre", 2.09, 0.244, 0.389, 0, 40, 1.62, 0, 0.217, 0},
     {"t16x32x32_wavek_bf16x2_tri_bpre", 1.86, 0.448, 0.564, 0, 40, 1.52, 0, 0, 0},
@@ -546,6 +550,16 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   return best;
 }
 
+// Three fp16 terms on K over eight waves: only in the place of the tile kernels, which split the operands as they are too (the slot
+// kernels scale both first and so take values beyond fp16's range: their calls stay theirs), up to three tiles of 32 x 32 per CU, of deep
+// K up to one.  150 shapes of 2 - 1500 rows (graph replay): 0.47 of the tile kernels' time (2 x 1280 x 1280 12.8 us, here 6.1; 38 x 256 x 448
+// 9.9, 3.3; 222 x 4352 x 704 32.9, 28.6), 2 % behind the fastest of all; beyond: 391 x 384 x 1984 13.6, here 16.7; 1136 x 3200 x 256 42.8, 44.9.
+static bool wavek_three_terms(const VariantDesc& v) { return v.kind == KIND_WAVEK && v.terms == 3; }
+static bool few_tiles_three_terms(const Problem& q, int count) {
+  const int64_t tiles = (int64_t)count * ((q.M + 31) / 32) * ((q.N + 31) / 32);
+  return tiles <= (q.K <= 2048 ? 3 : 1) * kNumCUs;
+}
+
 // ws_bytes: workspace the caller brought (split-K variants that need more are skipped)
 // The selection walks the whole table and costs every candidate; a model calls the same few dozen
 // problems over and over (eagerly, ~750 Linear calls per UNet step), so the answers are remembered.
@@ -609,7 +623,7 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
   double best_cost = 0;
   if (splits_out) *splits_out = 1;
   for (int i = 0; i < (int)t.size(); ++i) {
-    if (!variant_matches(t[i], q, fit)) continue;
+    if (wavek_three_terms(t[i]) || !variant_matches(t[i], q, fit)) continue;
     if (count > 1 && !t[i].grouped) continue;
     if (t[i].kind == KIND_SPLITK &&
         skinny_workspace_bytes(q.M, q.N, q.K, t[i].BM, t[i].BN, t[i].BK) > ws_bytes)
@@ -622,6 +636,15 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
       best = i;
       best_cost = c;
       if (splits_out) *splits_out = sp;
+    }
+  }
+  if (best >= 0 && t[best].kind == KIND_TILE && few_tiles_three_terms(q, count)) {
+    best_cost = 1e9;
+    for (int i = 0; i < (int)t.size(); ++i) {
+      if (!wavek_three_terms(t[i]) || !variant_matches(t[i], q, fit) || variant_cost(i, q, count) >= best_cost) continue;
+      best = i;
+      best_cost = variant_cost(i, q, count);
+      if (splits_out) *splits_out = 1;
     }
   }
   return best < 0 ? (int)CASCMM_ERR_BAD_FORMAT : best;

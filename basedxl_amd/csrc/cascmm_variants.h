@@ -441,7 +441,7 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
 #define CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, BPRE)                                                        \
   {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, WaveK<W, MB, NB>::BM, WaveK<W, MB, NB>::BN, WaveK<W, MB, NB>::BK,   \
    WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0,   \
-   W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16, BPRE || !wavek_for_shapes(W * MB, W * NB)}
+   W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16, BPRE || FMT != CASCMM_FMT_BF16 || !wavek_for_shapes(W * MB, W * NB)}
 #define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS) CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, 0)
 
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \

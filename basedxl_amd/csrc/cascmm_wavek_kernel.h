@@ -23,7 +23,9 @@
 // problems of some 256 of them.  Measured (graph replay, us; in brackets the one 32 x 32 / 32 x 64 kernel before, whose steps stood
 // behind branches): 2 x 1280 x 1280 4.2 (7.6), 2 x 320 x 1280 2.6 (4.9), 32 x 1024 x 384 3.6 (7.1), 128 x 1952 x 448 6.5 (10.3),
 // 333 x 456 x 211 3.6 (5.7), 640^3 7.4 (10.6), 768^3 10.7 and 1024^3 13.6 (12.5 and 15.9 on the LDS-tiled kernel), 154 x 2048 x 1280
-// 11.7 (11.4).  With the weight prepared, two 16-byte loads per step and 16 columns and half the instructions: 2 x 2816 x 1280 5.7 (9.3
+// 11.7 (11.4).  Three fp16 terms: 2 x 1280 x 1280 6.1 (12.8 on the 64 x 64 tile kernel with its K split), 38 x 256 x 448 3.3 (9.9), 154 x
+// 2048 x 1280 17.3 (20.8), 333 x 456 x 211 5.1 (23.3 on the bounds-checked kernel); their accumulators fill the registers on tiles beyond
+// 32 x 32.  With the weight prepared, two 16-byte loads per step and 16 columns and half the instructions: 2 x 2816 x 1280 5.7 (9.3
 // raw), 154 x 2048 x 1280 9.5, x 640 7.6, 77 x 2048 x 2560 9.5, 108 x 592 x 3155 6.3 (10.0 on the 64 x 80 tile, eager).
 #pragma once
 #include <type_traits>
