@@ -106,6 +106,8 @@ def lib() -> ctypes.CDLL:
 
 #: persistent split-K / re-lay workspaces, see cascaded_lowp_matmul.py (here because the host extension looks them up as well)
 workspaces: dict = {}
+#: the scale searches' scratch of the fp8 cascades (as above)
+scale_scratch: dict = {}
 
 _native = None
 
@@ -121,6 +123,7 @@ def native():
             raise ImportError(f"the host extension {os.path.join(_HERE, '_native.so')} is not built or does not load: {e}. "
                               "Run `python -m basedxl_amd.build`.") from None
         module.init(workspaces)
+        module.init_scales(scale_scratch)
         _native = module
     return _native
 
@@ -132,7 +135,7 @@ class _NoShortCut:
     def matmul(*_args):
         return None
 
-    prepared = matmul
+    prepared = fp8 = matmul
 
 
 _short_cut = None

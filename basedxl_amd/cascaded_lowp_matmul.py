@@ -126,7 +126,7 @@ def _check_bias(bias: Optional[torch.Tensor], like: torch.Tensor, n: int) -> Opt
     return bias.contiguous()
 
 
-_exp_scratch: Dict[Tuple[int, int], torch.Tensor] = {}
+_exp_scratch: Dict[Tuple[int, object], torch.Tensor] = _lib.scale_scratch
 
 
 def _scale_scratch(dev: torch.device, stream: int) -> torch.Tensor:
@@ -794,10 +794,14 @@ def cascaded_lowp_matmul(
     b_exp: Optional[torch.Tensor] = None,
     tensor_exps: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    if out is None and variant < 0 and not dump_ptx and tensor_exps is None and lowp != "fp8":
+    if out is None and variant < 0 and not dump_ptx and tensor_exps is None:
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
-        if type(b) is PreparedWeight:
-            y = None if b.fmt == _lib.FMT_FP8 else _lib.short_cut().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+        if type(b) is PreparedWeight and b.fmt != _lib.FMT_FP8:
+            y = _lib.short_cut().prepared(a, b.slots, bias, b.K, b.N, b.fmt, b.terms, products, b.dt, b.glu, 0)
+        elif type(b) is PreparedWeight:
+            y = None if b.glu else _lib.short_cut().fp8(a, b.slots, bias, b.exp, b.K, b.N, b.terms, products, True)
+        elif lowp == "fp8":
+            y = _lib.short_cut().fp8(a, b, bias, b_exp, 0, 0, terms, products, False)
         else:
             y = _lib.short_cut().matmul(a, b, bias, lowp, terms, products)
         if y is not None:

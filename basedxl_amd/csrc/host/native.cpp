@@ -23,6 +23,7 @@
 
 namespace {
 
+PyObject* g_scales = nullptr;       // the dict {(device index, stream handle): int32[2] tensor} of the fp8 scale searches' scratch
 PyObject* g_workspaces = nullptr;   // the dict {(device index, stream handle): uint8 tensor} of the Python wrapper
 
 struct Need {
@@ -61,7 +62,7 @@ int format_code(PyObject* s) {
   if (!PyUnicode_Check(s)) return -1;
   if (PyUnicode_CompareWithASCIIString(s, "bf16") == 0) return CASCMM_FMT_BF16;
   if (PyUnicode_CompareWithASCIIString(s, "fp16") == 0) return CASCMM_FMT_FP16;
-  return -1;   // (fp8 products find scales first: not the ordinary case)
+  return -1;   // (fp8 products find scales first: a function of their own)
 }
 int products_code(PyObject* s) {
   if (!PyUnicode_Check(s)) return -1;
@@ -115,6 +116,20 @@ bool workspace_of(size_t need, int device, hipStream_t stream, at::Tensor& hold,
   if ((size_t)hold.numel() < need) return false;
   ptr = hold.data_ptr();
   bytes = (size_t)hold.numel();
+  return true;
+}
+// the stream's scratch of the scale searches, if it exists already and nothing is being recorded; `hold` as above
+bool scale_scratch_of(int device, hipStream_t stream, at::Tensor& hold, int32_t*& ptr) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (!g_scales || hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+  PyObject* key = Py_BuildValue("(iK)", device, (unsigned long long)(uintptr_t)stream);
+  if (!key) { PyErr_Clear(); return false; }
+  PyObject* t = PyDict_GetItem(g_scales, key);   // borrowed
+  Py_DECREF(key);
+  if (!t || !THPVariable_Check(t)) return false;
+  hold = THPVariable_Unpack(t);
+  if (hold.numel() != 2 || hold.scalar_type() != at::kInt) return false;
+  ptr = (int32_t*)hold.data_ptr();
   return true;
 }
 at::Tensor result_like(const at::Tensor& a, int64_t n) {
@@ -214,6 +229,77 @@ PyObject* prepared(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
 }
 
+// fp8(a, b, bias | None, b_exp | None, K, N, terms, products, b is slots) -> Tensor | None: fp8 terms of fp32 tensors, the scale of a found
+// in the call; b a raw [K, N] tensor or the operand slots of a PreparedWeight, b_exp its scale exponent (None, raw only: found too)
+PyObject* fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 9) Py_RETURN_NONE;
+  try {
+    const int device = c10::hip::current_device();
+    const at::Tensor *a = gpu_tensor(args[0], device), *b = gpu_tensor(args[1], device);
+    if (!a || !b) Py_RETURN_NONE;
+    int64_t wk = PyLong_AsLongLong(args[4]), N = PyLong_AsLongLong(args[5]);   // (of slots)
+    const int terms = PyLong_Check(args[6]) ? (int)PyLong_AsLong(args[6]) : -1, products = products_code(args[7]), slots = PyObject_IsTrue(args[8]);
+    if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+    if (!slots) {
+      if (b->dim() != 2 || b->scalar_type() != at::kFloat || !b->is_contiguous()) Py_RETURN_NONE;
+      wk = b->size(0);
+      N = b->size(1);
+    }
+    const at::Tensor* exp = args[3] == Py_None ? nullptr : gpu_tensor(args[3], device);
+    if ((args[3] != Py_None || slots) && (!exp || exp->scalar_type() != at::kInt || exp->numel() != 1)) Py_RETURN_NONE;
+    int64_t M, K, lda;
+    const void* bias;
+    if (a->scalar_type() != at::kFloat || terms < 1 || products < 0 || N <= 0 || !rows_of(*a, M, K, lda) || K != wk) Py_RETURN_NONE;
+    if (!bias_of(args[2], *a, N, device, bias)) Py_RETURN_NONE;
+    if (slots) {
+      const size_t bytes = cascmm_prepared_bytes(wk, N, CASCMM_FMT_FP8, terms);
+      if (b->nbytes() != (bytes > 16 ? bytes : 16)) Py_RETURN_NONE;                                    // (not this layout: the wrapper raises)
+      if ((uintptr_t)a->const_data_ptr() % 16 != 0 || lda % 4 != 0 || K % 64 != 0 || N % 4 != 0) Py_RETURN_NONE;   // (the wrapper copies such rows)
+    }
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    at::Tensor hold, hold_scratch;
+    void* ws;
+    size_t ws_bytes;
+    int32_t* scratch;
+    if (!scale_scratch_of(device, stream, hold_scratch, scratch) ||
+        !workspace_of(workspace_need({M, N, K, CASCMM_DT_F32, CASCMM_FMT_FP8, terms, products}), device, stream, hold, ws, ws_bytes))
+      Py_RETURN_NONE;
+    at::Tensor out = result_like(*a, N);
+    at::Tensor exps = at::empty({2}, at::TensorOptions().dtype(at::kInt).device(a->device()));
+    const void *ap = a->const_data_ptr(), *bp = b->const_data_ptr();
+    const int32_t* b_exp = exp ? (const int32_t*)exp->const_data_ptr() : nullptr;
+    void* cp = out.data_ptr();
+    int32_t* ep = (int32_t*)exps.data_ptr();
+    int st;
+    Py_BEGIN_ALLOW_THREADS
+    if (b_exp) {
+      st = cascmm_gemm_fp8_autoscale(ap, bp, slots, cp, bias, M, N, K, lda, N, N, terms, products, b_exp, ep, scratch, ws, ws_bytes, stream);
+    } else {
+      st = cascmm_tensor_exps(ap, M, K, lda, CASCMM_DT_F32, nullptr, ep, scratch, stream);
+      if (st == CASCMM_OK) st = cascmm_tensor_exps(bp, K, N, N, CASCMM_DT_F32, nullptr, ep + 1, scratch, stream);
+      if (st == CASCMM_OK) st = cascmm_gemm_variant(ap, bp, cp, bias, M, N, K, lda, N, N, CASCMM_DT_F32, CASCMM_FMT_FP8, terms, products, ep, ws, ws_bytes, stream, -1);
+    }
+    Py_END_ALLOW_THREADS
+    if (st != CASCMM_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+  } catch (...) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+}
+
+// init_scales(scratch): the dict to look the scale searches' scratch up in
+PyObject* init_scales(PyObject*, PyObject* d) {
+  if (!PyDict_Check(d)) {
+    PyErr_SetString(PyExc_TypeError, "init_scales takes the dict of scale scratch");
+    return nullptr;
+  }
+  Py_INCREF(d);
+  Py_XDECREF(g_scales);
+  g_scales = d;
+  Py_RETURN_NONE;
+}
+
 // init(workspaces): the dict to look workspaces up in
 PyObject* init(PyObject*, PyObject* d) {
   if (!PyDict_Check(d)) {
@@ -229,6 +315,8 @@ PyObject* init(PyObject*, PyObject* d) {
 PyMethodDef kMethods[] = {
     {"matmul", (PyCFunction)(void (*)(void))matmul, METH_FASTCALL, "raw operands; None: not the ordinary case"},
     {"prepared", (PyCFunction)(void (*)(void))prepared, METH_FASTCALL, "prepared weight; None: not the ordinary case"},
+    {"fp8", (PyCFunction)(void (*)(void))fp8, METH_FASTCALL, "fp8 terms, scale found in the call; None: not the ordinary case"},
+    {"init_scales", init_scales, METH_O, "hands over the dict of the scale searches' scratch"},
     {"init", init, METH_O, "hands over the workspaces' dict"},
     {nullptr, nullptr, 0, nullptr},
 };

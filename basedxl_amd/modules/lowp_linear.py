@@ -54,7 +54,13 @@ class BasedXLLowPLinear(nn.Module):
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         pw = self._prepared_weight
         if self.lowp == "fp8":
-            y = None
+            # (a handful of rows: the raw weight, as below)
+            if self.prepared and not x.numel() < 32 * self.in_features:
+                y = None if pw is None or pw.device != self.weight.device else _lib.short_cut().fp8(
+                    x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
+            else:
+                y = None if self._weight_exp is None else _lib.short_cut().fp8(
+                    x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
         elif not self.prepared:
             y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
         elif pw is not None and pw.device == self.weight.device:

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from basedxl_amd import BasedXLFusedKV, BasedXLLowPGEGLU, BasedXLLowPLinear, PreparedWeight, _lib, cascaded_lowp_matmul
+from basedxl_amd.cascaded_lowp_matmul import tensor_scale_exp
 
 _native = _lib.native()
 
@@ -116,6 +117,41 @@ def test_same_bits_as_the_wrapper(gpu_device, dtype, M, K, N):
     for _ in range(3):
         got.zero_()
         graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(64, 128, 64), (300, 456, 212), (2, 1280, 640), (40, 1280, 1281)])
+def test_fp8_calls_are_those_of_the_python_path(gpu_device, M, K, N):
+    """Raw and prepared, scale of the weight kept or found, bit for bit against `out=`, and inside a device graph."""
+    g = torch.Generator().manual_seed(K)
+    rn = lambda *s: torch.randn(*s, generator=g).to("cuda:0")
+    a, w, bias, frame = rn(M, K), rn(K, N) * 0.02, rn(N), rn(M, K + 8)
+    weights = [w] + ([PreparedWeight(w, lowp="fp8", terms=3)] if K % 64 == 0 and N % 4 == 0 else [])
+    exp = tensor_scale_exp(w)
+    for x in (a, frame[:, :K], a.view(M // 2, 2, K)):
+        for b in weights:
+            for bb, e in ((None, None), (bias, None), (bias, exp)):
+                kw = dict(bias=bb) if isinstance(b, PreparedWeight) else dict(bias=bb, lowp="fp8", terms=3, b_exp=e)
+                want = cascaded_lowp_matmul(x, b, out=torch.empty(M, N, device="cuda:0"), **kw)
+                got = cascaded_lowp_matmul(x, b, **kw)
+                assert got.shape == (*x.shape[:-1], N) and torch.equal(got, want.view(got.shape))
+    assert _native.fp8(a, w, bias, exp, 0, 0, 3, "tri", False) is not None and _native.fp8(a, w, None, None, 0, 0, 3, "tri", False) is not None
+    for args in ((a.half(), w, None, exp, 0, 0, 3, "tri", False), (a, w.t(), None, exp, 0, 0, 3, "tri", False), (a, w, bias[:-1], exp, 0, 0, 3, "tri", False),
+                 (a, w, None, exp.float(), 0, 0, 3, "tri", False), (a, w, None, exp, 0, 0, None, "tri", False), (a, w, None, exp, 0, 0, 3, "all", False),
+                 (a, torch.zeros(64, dtype=torch.uint8, device="cuda:0"), None, exp, K, N, 3, "tri", True), (a, w, None)):
+        assert _native.fp8(*args) is None
+    want = cascaded_lowp_matmul(a, w, lowp="fp8", terms=3)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        assert _native.fp8(a, w, None, exp, 0, 0, 3, "tri", False) is None         # (a recorded call: its own scratch, kept by the Python path)
+        got = cascaded_lowp_matmul(a, w, lowp="fp8", terms=3)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(cascaded_lowp_matmul(a, w, lowp="fp8", terms=3), want)
         torch.cuda.synchronize()
         assert torch.equal(got, want)
 
