@@ -260,6 +260,10 @@ static const CallCost kCallCost[] = {
     {"t16x16x32_wavek_fp16x3_tri", 2.38, 0.675, 0.768, 0, 19.6, 1.61, 0, 0.0438, 0},
     {"t16x32x32_wavek_fp16x3_tri", 2.54, 1.12, 1.57, 0, 16.2, 6.97, 0, 0.0319, 0},
     {"t32x32x32_wavek_fp16x3_tri", 2.75, 1.46, 0.223, 1.49, 35.4, 1, 1.66, 0, 0},
+    // three fp8 terms (as three fp16 ones)
+    {"t16x16x32_wavek_fp8x3_tri", 2.52, 0.655, 0.749, 0, 17.9, 1.54, 0, 0, 0},
+    {"t16x32x32_wavek_fp8x3_tri", 2.65, 1.11, 1.6, 0, 16.1, 7.35, 0, 0, 0},
+    {"t32x32x32_wavek_fp8x3_tri", 2.82, 1.44, 0.245, 1.52, 34.4, 1, 1.67, 0, 0},
     // prepared weights (460 shapes, mean error 0.01 - 0.05; the kernel chosen is 1 % behind the fastest, 8.6 % with the constants above)
     {"t16x16x32_wavek_bf16x2_tri_bpre", 2.09, 0.244, 0.389, 0, 40, 1.62, 0, 0.217, 0},
     {"t16x32x32_wavek_bf16x2_tri_bpre", 1.86, 0.448, 0.564, 0, 40, 1.52, 0, 0, 0},
@@ -550,13 +554,18 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   return best;
 }
 
-// Three fp16 terms on K over eight waves: only in the place of the tile kernels, which split the operands as they are too (the slot
-// kernels scale both first and so take values beyond fp16's range: their calls stay theirs), up to three tiles of 32 x 32 per CU, of deep
-// K up to one.  150 shapes of 2 - 1500 rows (graph replay): 0.47 of the tile kernels' time (2 x 1280 x 1280 12.8 us, here 6.1; 38 x 256 x 448
-// 9.9, 3.3; 222 x 4352 x 704 32.9, 28.6), 2 % behind the fastest of all; beyond: 391 x 384 x 1984 13.6, here 16.7; 1136 x 3200 x 256 42.8, 44.9.
+// Three terms on K over eight waves, by the tiles of 32 x 32 (graph replay, 150 shapes of 2 - 1500 rows each).
+// fp16: only in the place of the tile kernels, which split the operands as they are too (the slot kernels scale both first and so take
+// values beyond fp16's range: their calls stay theirs), up to three tiles per CU, of deep K up to one.  0.47 of the tile kernels' time (2 x 1280 x
+// 1280 12.8 us, here 6.1; 38 x 256 x 448 9.9, 3.3; 222 x 4352 x 704 32.9, 28.6), 2 % behind the fastest of all; beyond: 391 x 384 x 1984
+// 13.6, here 16.7; 1136 x 3200 x 256 42.8, 44.9.
+// fp8: in the place of the slot kernels too (all scale by the same exponents), whose passes it does without, up to one tile per CU: 0.56 of the
+// time (2 x 1280 x 1280 11.7, here 6.3; 18 x 2688 x 384 20.4, 10.3); beyond, the fp8-rate instruction wins: 391 x 384 x 1984 11.8, here 17.3; 222 x 4352 x
+// 704 27.4, 28.1.
 static bool wavek_three_terms(const VariantDesc& v) { return v.kind == KIND_WAVEK && v.terms == 3; }
 static bool few_tiles_three_terms(const Problem& q, int count) {
   const int64_t tiles = (int64_t)count * ((q.M + 31) / 32) * ((q.N + 31) / 32);
+  if (q.fmt == CASCMM_FMT_FP8) return tiles <= kNumCUs && q.K <= 4096;
   return tiles <= (q.K <= 2048 ? 3 : 1) * kNumCUs;
 }
 
@@ -638,7 +647,7 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
       if (splits_out) *splits_out = sp;
     }
   }
-  if (best >= 0 && t[best].kind == KIND_TILE && few_tiles_three_terms(q, count)) {
+  if (best >= 0 && (t[best].kind == KIND_TILE || t[best].kind == KIND_F8K64) && few_tiles_three_terms(q, count)) {
     best_cost = 1e9;
     for (int i = 0; i < (int)t.size(); ++i) {
       if (!wavek_three_terms(t[i]) || !variant_matches(t[i], q, fit) || variant_cost(i, q, count) >= best_cost) continue;
@@ -908,6 +917,8 @@ static Problem rounded_up(const Problem& q, RowFit fit) {
 static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem* e) {
   *e = rounded_up(q, fit);
   if (!e->split_first) return CASCMM_ERR_BAD_FORMAT;
+  // (few tiles: K over eight waves on the rows as they lie)
+  if (q.call && q.fmt == CASCMM_FMT_FP8 && fit != FIT_NONE && few_tiles_three_terms(q, 1) && !beyond_i32(q.M, q.lda, 4)) return CASCMM_ERR_BAD_FORMAT;
   const int v = select_variant(*e, FIT_FAST, 1, room);
   if (v < 0) return v;
   const double tiles = (double)((q.M + 63) / 64) * (double)((q.N + 63) / 64);
@@ -1491,6 +1502,8 @@ int cascmm_gemm_fp8_autoscale(const void* A, const void* B, int b_prepared, void
   q.bpre = b_prepared != 0;
   const int st = check_problem(q);
   if (st != CASCMM_OK) return st;
+  q.chunked = chunked_by_k(q);
+  q.call = true;
   const void* bias1 = bias;
   if (M > 0 && N > 0 && K > 0 && A && B) {
     // the fp8-rate kernel splits A in a pass of its own anyway: the search rides on it

@@ -14,6 +14,10 @@ static const VariantDesc kTable[] = {
     CASCMM_F8K64_VARIANT("t128x160x64_f8k64_fp8x3_tri_bpre", true, 1),
     CASCMM_F8K64_VARIANT("k64x160x64_f8k64wk4_fp8x3_tri", false, 0),
     CASCMM_F8K64_VARIANT("k64x160x64_f8k64wk4_fp8x3_tri_bpre", true, 0),
+    // few rows and small problems (cascmm_wavek_kernel.h)
+    CASCMM_WAVEK_VARIANT("t16x16x32_wavek_fp8x3_tri", 16, 1, 1, F8, 3),
+    CASCMM_WAVEK_VARIANT("t16x32x32_wavek_fp8x3_tri", 16, 1, 2, F8, 3),
+    CASCMM_WAVEK_VARIANT("t32x32x32_wavek_fp8x3_tri", 16, 2, 2, F8, 3),
     // three terms (12 significand bits), six products.  name, BM, BN, BK, WM, WN, WK, DEPTH
     CASCMM_TILE_VARIANT("t128x128x32_w4x2x1_d2_fp8x3_tri", 128, 128, 32, 4, 2, 1, 2, F32, F8, 3, false, true),
     CASCMM_TILE_VARIANT("t64x64x64_w2x2x1_d2_fp8x3_tri", 64, 64, 64, 2, 2, 1, 2, F32, F8, 3, false, true),

@@ -25,7 +25,7 @@
 // 333 x 456 x 211 3.6 (5.7), 640^3 7.4 (10.6), 768^3 10.7 and 1024^3 13.6 (12.5 and 15.9 on the LDS-tiled kernel), 154 x 2048 x 1280
 // 11.7 (11.4).  Three fp16 terms: 2 x 1280 x 1280 6.1 (12.8 on the 64 x 64 tile kernel with its K split), 38 x 256 x 448 3.3 (9.9), 154 x
 // 2048 x 1280 17.3 (20.8), 333 x 456 x 211 5.1 (23.3 on the bounds-checked kernel); their accumulators fill the registers on tiles beyond
-// 32 x 32.  With the weight prepared, two 16-byte loads per step and 16 columns and half the instructions: 2 x 2816 x 1280 5.7 (9.3
+// 32 x 32.  Three fp8 terms, scales given: 2 x 1280 x 1280 6.3 (11.7), 18 x 2688 x 384 10.3 (20.4).  With the weight prepared, two 16-byte loads per step and 16 columns and half the instructions: 2 x 2816 x 1280 5.7 (9.3
 // raw), 154 x 2048 x 1280 9.5, x 640 7.6, 77 x 2048 x 2560 9.5, 108 x 592 x 3155 6.3 (10.0 on the 64 x 80 tile, eager).
 #pragma once
 #include <type_traits>
@@ -222,6 +222,17 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       if constexpr (kFold) master[mb][nb] = zero;
     }
 
+  // fp8 terms: the tensors' scales, powers of two
+  constexpr bool kScaled8 = FMT == CASCMM_FMT_FP8;
+  float scale_a = 1.f, scale_b = 1.f, scale_out = 1.f;
+  if constexpr (kScaled8) {
+    if (p.tensor_exps) {
+      const int ea = p.tensor_exps[2 * prob], eb = p.tensor_exps[2 * prob + 1];
+      scale_a = __builtin_ldexpf(1.f, ea);
+      scale_b = __builtin_ldexpf(1.f, eb);
+      scale_out = __builtin_ldexpf(1.f, -(ea + eb));
+    }
+  }
   auto step = [&](int i, auto U) {
     constexpr int u = decltype(U)::value;
     const unsigned char* stp = ring + u * T::A_STAGE;
@@ -238,7 +249,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 #pragma unroll
           for (int e = 0; e < 8; ++e) xa[e] = e < left ? xa[e] : 0.f;
         }
-        split8<FMT, TERMS>(xa, ta[mb]);
+        split8<FMT, TERMS>(xa, ta[mb], scale_a);
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -250,7 +261,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           float xb[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
-          split8<FMT, TERMS>(xb, tb);
+          split8<FMT, TERMS>(xb, tb, scale_b);
         }
         // smallest products first
 #pragma unroll
@@ -371,6 +382,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     float sum = 0.f;
 #pragma unroll
     for (int w = 0; w < T::NW; ++w) sum += part[((w * MB * NB + blk) * REGS + e) * 64 + ln];
+    if constexpr (kScaled8) sum *= scale_out;
     if (row < p.M && (!TAIL || col < p.N)) C[(int64_t)row * p.ldc + col] = sum + (bias ? bias[col] : 0.f);
   }
 }
