@@ -316,6 +316,16 @@ class PreparedWeight:
         return hit
 
 
+def raw_is_faster(rows: int, K: int, N: int, dtype: torch.dtype, lowp: str, terms: int) -> bool:
+    """fp32 activations for which the raw weight's kernels are the faster ones though the weight is kept split too: a handful of rows where
+    three terms and K off 8 have small kernels for the raw weight only (two bf16 terms and K of 8: 2 x 2816 x 1280 9.4 us raw, 5.7
+    prepared), and with three fp8 terms up to a tile of 32 x 32 per CU (64 x 640 x 1280: 9.9 us raw, 19.9 prepared, whose activations
+    are written as slots first; 154 x 2048 x 1280 20.6 and 28.0; beyond, 512 x 1280 x 1280, 30.6 and 25.8)."""
+    if dtype != torch.float32 or ((lowp, terms) == ("bf16", 2) and K % 8 == 0):
+        return False
+    return rows < 32 or ((lowp, terms) == ("fp8", 3) and K <= 4096 and -(-rows // 32) * -(-N // 32) <= 256)
+
+
 def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, products: str = "tri", variant: int = -1):
     """``a_list[i]`` ([..., K] fp32) times the prepared weight ``w_list[i]`` in ONE launch (1..8
     problems of one shape and one cascade); returns the list of results."""

@@ -11,7 +11,7 @@ from typing import Optional
 
 import torch
 
-from .cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul
+from .cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, raw_is_faster
 
 
 @torch.library.custom_op("basedxl_amd::cascade_linear", mutates_args=(), device_types="cuda")
@@ -24,7 +24,7 @@ def cascade_linear(x: torch.Tensor, weight: torch.Tensor, slots: Optional[torch.
     if slots is not None:
         pw = PreparedWeight.from_slots(slots, K, N, weight.dtype, lowp, terms, glu, b_exp)
         x2 = x.reshape(-1, K)
-        few_rows = x2.shape[0] < 32 and x2.dtype == torch.float32 and ((lowp, terms) != ("bf16", 2) or K % 8 != 0)
+        few_rows = raw_is_faster(x2.shape[0], K, N, x2.dtype, lowp, terms)
         if glu or (not few_rows and pw.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), products)):
             return cascaded_lowp_matmul(x, pw, bias=bias, products=products)
     return cascaded_lowp_matmul(x, weight, bias=bias, lowp=lowp, terms=terms, products=products, b_exp=b_exp)

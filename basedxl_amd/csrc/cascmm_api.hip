@@ -917,8 +917,13 @@ static Problem rounded_up(const Problem& q, RowFit fit) {
 static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem* e) {
   *e = rounded_up(q, fit);
   if (!e->split_first) return CASCMM_ERR_BAD_FORMAT;
-  // (few tiles: K over eight waves on the rows as they lie)
-  if (q.call && q.fmt == CASCMM_FMT_FP8 && fit != FIT_NONE && few_tiles_three_terms(q, 1) && !beyond_i32(q.M, q.lda, 4)) return CASCMM_ERR_BAD_FORMAT;
+  // (up to one tile per CU, of 16 columns for 16 rows and fewer, K over eight waves on the rows as they lie: 6 x 2455 x 1079 12.2 us, 33.3
+  // in slots; 153 x 1368 x 728 11.5, 23.5.  Wider results of few rows are left to the comparison below, as before: 5 x 939 x 5189 24.7 in
+  // slots, 8.8 here)
+  const int64_t wide = q.M <= 16 ? 16 : 32;
+  if (q.call && q.fmt == CASCMM_FMT_FP8 && fit != FIT_NONE && ((q.M + wide - 1) / wide) * ((q.N + wide - 1) / wide) <= kNumCUs &&
+      few_tiles_three_terms(q, 1) && !beyond_i32(q.M, q.lda, 4))
+    return CASCMM_ERR_BAD_FORMAT;
   const int v = select_variant(*e, FIT_FAST, 1, room);
   if (v < 0) return v;
   const double tiles = (double)((q.M + 63) / 64) * (double)((q.N + 63) / 64);

@@ -7,7 +7,7 @@ import torch.nn as nn
 from typing import Optional
 
 from .. import _lib
-from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, default_cascade, tensor_scale_exp
+from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, default_cascade, raw_is_faster, tensor_scale_exp
 
 
 class BasedXLLowPLinear(nn.Module):
@@ -54,8 +54,7 @@ class BasedXLLowPLinear(nn.Module):
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         pw = self._prepared_weight
         if self.lowp == "fp8":
-            # (a handful of rows: the raw weight, as below)
-            if self.prepared and not x.numel() < 32 * self.in_features:
+            if self.prepared and not raw_is_faster(x.numel() // max(self.in_features, 1), self.in_features, self.out_features, x.dtype, self.lowp, self.terms):
                 y = None if pw is None or pw.device != self.weight.device else _lib.short_cut().fp8(
                     x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
             else:
@@ -73,9 +72,7 @@ class BasedXLLowPLinear(nn.Module):
             if self._prepared_weight is None or self._prepared_weight.device != self.weight.device:
                 self._prepared_weight = PreparedWeight(self.weight, lowp=self.lowp, terms=self.terms)
             x2 = x.reshape(-1, self.in_features)
-            # a handful of rows: three terms and K off 8 have kernels for the raw weight only (two bf16 terms and K of 8: 2 x 2816 x 1280
-            # 9.4 us raw, 5.7 prepared)
-            few_rows = x2.shape[0] < 32 and x2.dtype == torch.float32 and ((self.lowp, self.terms) != ("bf16", 2) or self.in_features % 8 != 0)
+            few_rows = raw_is_faster(x2.shape[0], self.in_features, self.out_features, x2.dtype, self.lowp, self.terms)
             if not few_rows and self._prepared_weight.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), self.products):
                 return cascaded_lowp_matmul(x, self._prepared_weight, bias=self.bias, products=self.products)
         if self.lowp == "fp8" and (self._weight_exp is None or self._weight_exp.device != self.weight.device):

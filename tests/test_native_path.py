@@ -157,6 +157,21 @@ def test_fp8_calls_are_those_of_the_python_path(gpu_device, M, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,N", [(1, 640, 1280), (33, 640, 1280), (204, 1280, 1280), (205, 1280, 1312), (257, 4160, 320)])
+def test_fp8_layers_on_either_side_of_the_raw_weight_s_rule(gpu_device, rows, K, N):
+    """Prepared and not, before and after prepare(), few tiles and more: the same products, added in another order."""
+    torch.manual_seed(rows)
+    lin, x = torch.nn.Linear(K, N).to("cuda:0").requires_grad_(False), torch.randn(rows, K, device="cuda:0")
+    want = x.double() @ lin.weight.double().t() + lin.bias.double()
+    for prepared in (False, True):
+        mod = BasedXLLowPLinear(lin, lowp="fp8", terms=3, prepared=prepared)
+        first = mod(x)
+        mod.prepare()
+        assert torch.equal(mod(x), first)
+        assert float((first.double() - want).norm() / want.norm()) < 1.4e-4       # (four times the cascade's own error, 3.5e-5)
+
+
+@pytest.mark.gpu
 def test_slots_of_another_layout_are_refused(gpu_device):
     """A buffer that is shorter or longer than the weight's slots, as one kept in a file from another layout would be."""
     w, x = PreparedWeight(torch.randn(96, 64, device="cuda:0")), torch.randn(40, 96, device="cuda:0")
