@@ -358,8 +358,10 @@ static double h16_estimate_us(const VariantDesc& v, const Problem& q, double til
 // Fitted to 326 shapes of 2 - 2600 rows, K and widths 256 - 10240 (fp16, graph replay over three sets of operands, every tile forced
 // in turn), mean error 0.03 - 0.08.  They win where the tiles about fit the CUs at once (2 x 1280 x 1280 prepared 3.2 us, 6.9 on the four-wave kernels;
 // 154 x 2048 x 1280 5.6, 10.3), and lose behind that, where every tile pays its launch and its meeting in LDS (2048 x 640 x 640 raw
-// 12.0 us, 7.3).  The estimates decide, and within 4 % of each other (their error) the four-wave kernels stay: 0.76 (prepared), 0.82 (raw) and 0.90
-// (gated) of the time without these kernels over the shapes, 2 % behind the fastest of all.
+// 12.0 us, 7.3).  The estimates decide, and within 10 % of each other (their error) the four-wave kernels stay; raw weights deeper than
+// the straight code's four steps a wave stay with them too (10 x 2496 x 760 6.4 us, here 7.4): 0.77 (prepared), 0.83 (raw) and 0.90 (gated) of the
+// time without these kernels over the shapes, one of them slower (41 x 4000 x 1624 prepared 8.4 us, here 9.2; 9.2 and 8.9 eager).  64 x 64 tiles
+// gained only with the gated store (plain, by index only: 976 x 2048 x 640 9.1 us on the four-wave kernels, 10.6 on them).
 struct HwkCost { int BM, BN, form; CallCost c; };
 static const HwkCost kHwkCost[] = {
     {16, 16, 0, {nullptr, 2.7, 0.143, 0.345, 0, 20.2, 2.37, 0, 0.197, 0}},
@@ -367,19 +369,18 @@ static const HwkCost kHwkCost[] = {
     {16, 64, 0, {nullptr, 2.72, 0.492, 0.214, 0.388, 14.9, 1.18, 0.902, 0.383, 0}},
     {32, 32, 0, {nullptr, 2.8, 0.395, 0.411, 1.12, 12, 1.98, 0.735, 0.184, 0}},
     {32, 64, 0, {nullptr, 2.91, 0.604, 0.484, 1.06, 19.6, 1.13, 1.19, 0.244, 0}},
-    {64, 64, 0, {nullptr, 3.33, 0.867, 0.773, 1.74, 40, 1.08, 1.81, 0.134, 0}},
     {16, 32, 1, {nullptr, 2.43, 0.472, 0.805, 0, 30.3, 2.04, 0, 0.5, 0.0752}},
     {16, 64, 1, {nullptr, 2.58, 0.861, 0.328, 1.32, 40, 1.03, 1.1, 0.5, 0.0352}},
     {32, 32, 1, {nullptr, 2.68, 0.509, 0.39, 1.31, 40, 1, 0.934, 0.5, 0.0326}},
     {32, 64, 1, {nullptr, 2.87, 0.978, 0.485, 1.74, 40, 1.05, 1.23, 0.443, 0.0123}},
-    {64, 64, 1, {nullptr, 3.46, 1.28, 1.02, 2.33, 40, 1.6, 1.99, 0.5, 0}},
     {16, 64, 2, {nullptr, 3.14, 0.0359, 0.141, 0.86, 6.09, 7.35, 0.455, 0.05, 0.0069}},
     {32, 64, 2, {nullptr, 3.6, 0.264, 0.0524, 1.97, 6.36, 8, 0.586, 0.0225, 0.00763}},
     {64, 64, 2, {nullptr, 4.08, 0.02, 0.312, 2.82, 6.07, 7.47, 0.839, 0.0025, 0.007}},
 };
 static double hwk_estimate_us(const VariantDesc& v, const Problem& q, int count, double tiles) {
+  if (!q.bpre && q.K > 2048) return 1e9;
   for (const HwkCost& t : kHwkCost)
-    if (t.BM == v.BM && t.BN == v.BN && t.form == (q.glu ? 2 : q.bpre ? 0 : 1)) return 1.04 * call_estimate_us(t.c, v, q, count, tiles, q.K);
+    if (t.BM == v.BM && t.BN == v.BN && t.form == (q.glu ? 2 : q.bpre ? 0 : 1)) return 1.1 * call_estimate_us(t.c, v, q, count, tiles, q.K);
   return 1e9;
 }
 
