@@ -557,17 +557,18 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
 
 // Three terms on K over eight waves, by the tiles of 32 x 32 (graph replay, 150 shapes of 2 - 1500 rows each).
 // fp16: only in the place of the tile kernels, which split the operands as they are too (the slot kernels scale both first and so take
-// values beyond fp16's range: their calls stay theirs), up to three tiles per CU, of deep K up to one.  0.47 of the tile kernels' time (2 x 1280 x
-// 1280 12.8 us, here 6.1; 38 x 256 x 448 9.9, 3.3; 222 x 4352 x 704 32.9, 28.6), 2 % behind the fastest of all; beyond: 391 x 384 x 1984
-// 13.6, here 16.7; 1136 x 3200 x 256 42.8, 44.9.
+// values beyond fp16's range: their calls stay theirs), up to two tiles per CU, of deep K up to one, and up to three where the other kernel is
+// the bounds-checked one.  0.47 of the tile kernels' time (2 x 1280 x 1280 12.8 us, here 6.1; 38 x 256 x 448 9.9, 3.3; 222 x 4352 x 704 32.9,
+// 28.6; 788 x 659 x 818 bounds-checked 35.0, 23.0), 2 % behind the fastest of all; beyond: 391 x 384 x 1984 13.6, here 16.7; 96 x 2048 x 8192
+// 41.0, 45.3 (eager); 1136 x 3200 x 256 42.8, 44.9.
 // fp8: in the place of the slot kernels too (all scale by the same exponents), whose passes it does without, up to one tile per CU: 0.56 of the
 // time (2 x 1280 x 1280 11.7, here 6.3; 18 x 2688 x 384 20.4, 10.3); beyond, the fp8-rate instruction wins: 391 x 384 x 1984 11.8, here 17.3; 222 x 4352 x
 // 704 27.4, 28.1.
 static bool wavek_three_terms(const VariantDesc& v) { return v.kind == KIND_WAVEK && v.terms == 3; }
-static bool few_tiles_three_terms(const Problem& q, int count) {
+static bool few_tiles_three_terms(const Problem& q, int count, bool bounds_checked) {
   const int64_t tiles = (int64_t)count * ((q.M + 31) / 32) * ((q.N + 31) / 32);
   if (q.fmt == CASCMM_FMT_FP8) return tiles <= kNumCUs && q.K <= 4096;
-  return tiles <= (q.K <= 2048 ? 3 : 1) * kNumCUs;
+  return tiles <= (bounds_checked ? 3 : q.K <= 2048 ? 2 : 1) * kNumCUs;
 }
 
 // ws_bytes: workspace the caller brought (split-K variants that need more are skipped)
@@ -648,7 +649,7 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
       if (splits_out) *splits_out = sp;
     }
   }
-  if (best >= 0 && (t[best].kind == KIND_TILE || t[best].kind == KIND_F8K64) && few_tiles_three_terms(q, count)) {
+  if (best >= 0 && (t[best].kind == KIND_TILE || t[best].kind == KIND_F8K64) && few_tiles_three_terms(q, count, !t[best].fast)) {
     best_cost = 1e9;
     for (int i = 0; i < (int)t.size(); ++i) {
       if (!wavek_three_terms(t[i]) || !variant_matches(t[i], q, fit) || variant_cost(i, q, count) >= best_cost) continue;
@@ -923,7 +924,7 @@ static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem*
   // slots, 8.8 here)
   const int64_t wide = q.M <= 16 ? 16 : 32;
   if (q.call && q.fmt == CASCMM_FMT_FP8 && fit != FIT_NONE && ((q.M + wide - 1) / wide) * ((q.N + wide - 1) / wide) <= kNumCUs &&
-      few_tiles_three_terms(q, 1) && !beyond_i32(q.M, q.lda, 4))
+      few_tiles_three_terms(q, 1, false) && !beyond_i32(q.M, q.lda, 4))
     return CASCMM_ERR_BAD_FORMAT;
   const int v = select_variant(*e, FIT_FAST, 1, room);
   if (v < 0) return v;
