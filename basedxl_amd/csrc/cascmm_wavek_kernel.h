@@ -99,6 +99,28 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
   else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
 }
 
+// A's rows in a stage: position pos of row r holds chunk (pos - wavek_rot(r / 2)) mod 8 (16-row blocks: the rotations of
+// cascmm_slotn_kernel.h, which explains them)
+template <int W>
+__host__ __device__ constexpr int wavek_rot(int h) {
+  return W == 32 ? (h & 7) : (int)((0x75642031u >> (4 * (h & 7))) & 7u);
+}
+// Byte, in a block of rows of a stage, of half x (16 bytes) of what a lane hands to MFMA h.  With fewer than W rows in the stage the
+// other lanes read rows 0 .. 8 AL - 1 again: what they compute is not stored.
+template <int W, int AL>
+__host__ __device__ constexpr int wavek_fragment(int lane, int h, int x) {
+  const int row = lane & (W - 1) & (8 * AL - 1), kg = lane / W;
+  return row * 128 + ((h * (128 / W) + 2 * kg + x + wavek_rot<W>(row >> 1)) & 7) * 16;
+}
+template <int W, int MB, int AL>
+constexpr bool wavek_fragments_inside() {
+  for (int lane = 0; lane < 64; ++lane)
+    for (int h = 0; h < W / 16; ++h)
+      for (int x = 0; x < 2; ++x)
+        if (wavek_fragment<W, AL>(lane, h, x) + (MB - 1) * W * 128 + 16 > AL * 1024) return false;
+  return true;
+}
+
 template <int W, int NB, int FMT, int TERMS, int BPRE, int GLU>
 constexpr int wavek_b_loads() {
   return BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : (W / 2) * (GLU ? 2 : 1);
@@ -108,7 +130,7 @@ constexpr int wavek_b_loads() {
 // buffer load wants its address on a dword, and its dwords are checked against the buffer's end one by one).
 // TAIL = 0: K % 32 == 0 and N % (W NB) == 0.  TAIL = 1: any N and K: the rows of B past K lie beyond its buffer (zeros),
 // chunks of A past K are fetched from beyond the buffer, what a row's last chunk holds past K is masked.
-// AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL; what the others hold spoils rows that are not stored).
+// AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL), the lanes of the others read those again.
 // BPRE = 1: B is a prepared weight, [plane][4 ceil(K/32)][N] operand slots, a load per plane and column block (block nb: columns
 // W nb + c).  GLU = 1 (64-wide tiles): the gated store, C has N / 2 columns; a prepared weight alternates 32 value and 32 gate columns, of a
 // raw one blocks 0 and 1 are value columns 2 c + nb, blocks 2 and 3 their gates from the second half.
@@ -154,13 +176,11 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
             b_end = BPRE ? PL * b_plane : (int)(((int64_t)(p.K - 1) * p.ldb + p.N) * 4);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)pa, 0, a_end, 0x00020000);
   const i32x4 rb = make_rsrc(pb, b_end);
-  // load j of a step brings rows 8 j + lane / 8 to LDS bytes 1024 j + 16 lane; position pos of row r holds chunk
-  // (pos - rot((r / 2) mod 8)) mod 8 (16-row blocks: the rotations of cascmm_slotn_kernel.h, which explains them)
-  auto rot = [](int h) { return W == 32 ? (h & 7) : (int)((0x75642031u >> (4 * (h & 7))) & 7u); };
+  // load j of a step brings rows 8 j + lane / 8 to LDS bytes 1024 j + 16 lane, their chunks rotated (wavek_rot)
   int a_voff[2], a_k[2];
 #pragma unroll
   for (int jp = 0; jp < 2; ++jp) {
-    const int chunk = ((lane & 7) - rot(4 * jp + (lane >> 4))) & 7;
+    const int chunk = ((lane & 7) - wavek_rot<W>(4 * jp + (lane >> 4))) & 7;
     a_k[jp] = chunk * 4;
     a_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + chunk * 4) * 4);
   }
@@ -168,11 +188,12 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   // (GLU, raw: two value columns and, `gates` bytes further, their gates)
   const int b_voff = BPRE ? (kg * p.N + n0 + lw) * 16 : 8 * kg * ldb_bytes + (GLU ? (n0 >> 1) + 2 * lw : n0 + NB * lw) * 4, gates = p.N * 2;
   // fragment of a block of rows: row lw, the chunks of k group kg of MFMA h at their rotated places
+  static_assert(wavek_fragments_inside<W, MB, AL>(), "a fragment is read from the stage that was waited for");
   int a_frag[HALVES][2];
 #pragma unroll
   for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-    for (int x = 0; x < 2; ++x) a_frag[h][x] = lw * 128 + ((h * (KM / 4) + 2 * kg + x + rot(lw >> 1)) & 7) * 16;
+    for (int x = 0; x < 2; ++x) a_frag[h][x] = wavek_fragment<W, AL>(lane, h, x);
 
   typedef float bvec __attribute__((ext_vector_type(NB)));
   // B of the steps in flight, raw or as slots

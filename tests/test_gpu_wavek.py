@@ -37,6 +37,21 @@ def test_every_number_of_steps_is_exact_on_integers(name, K):
         assert bool((out[M] == -77.0).all()) and bool((out[:, N] == -77.0).all())
 
 
+@pytest.mark.parametrize("name", [n for n in _TILES if n.startswith("t16x")])
+@pytest.mark.parametrize("M", [1, 2, 8, 9])
+def test_few_rows_on_either_side_of_the_half_filled_stage(name, M):
+    """Up to eight rows are half a stage of a 16-row tile, which is all that is fetched and read: up to every stage of the ring and past it."""
+    lowp, terms = name.split("_")[2].split("x")
+    g = torch.Generator().manual_seed(M)
+    for K in (256, 1280, 1536, 2816):
+        a, b = (torch.randint(-60, 61, s, generator=g) for s in ((M, K), (K, 96)))
+        w = b.float().to("cuda:0")
+        print("wavek rows", name, M, K, flush=True)
+        got = cascaded_lowp_matmul(a.float().to("cuda:0"), PreparedWeight(w, lowp=lowp, terms=int(terms)) if name.endswith("_bpre") else w,
+                                   **({} if name.endswith("_bpre") else dict(lowp=lowp, terms=int(terms))), variant=_lib.variant_names().index(name))
+        assert torch.equal(got.cpu().long(), a @ b), K
+
+
 @pytest.mark.parametrize("M,K,N", [(2, 1280, 1280), (16, 2047, 477), (130, 1281, 448), (600, 600, 600), (1024, 1024, 1024), (3, 5120, 40)])
 def test_a_call_repeats_its_bits_and_keeps_non_finite_values_to_their_rows(M, K, N):
     a, b = torch.randn(M, K, device="cuda:0"), torch.randn(K, N, device="cuda:0")
