@@ -316,12 +316,13 @@ class PreparedWeight:
         return hit
 
 
-def raw_is_faster(rows: int, K: int, N: int, dtype: torch.dtype, lowp: str, terms: int) -> bool:
+def raw_is_faster(rows: int, K: int, N: int, dtype: torch.dtype, lowp: str, terms: int, products: str = "tri") -> bool:
     """fp32 activations for which the raw weight's kernels are the faster ones though the weight is kept split too: a handful of rows where
-    three terms and K off 8 have small kernels for the raw weight only (two bf16 terms and K of 8: 2 x 2816 x 1280 9.4 us raw, 5.7
-    prepared), and with three fp8 terms up to a tile of 32 x 32 per CU (64 x 640 x 1280: 9.9 us raw, 19.9 prepared, whose activations
+    three terms, the 'full' products and K off 8 have small kernels for the raw weight only (2 x 1280 x 1280: three fp16 terms 6.2 us raw,
+    39.3 prepared, on ten 128 x 128 tiles, three bf16 terms 11.8 and 38.2; two bf16 terms, 'tri' and K of 8: 2 x 2816 x 1280 9.4 us raw, 5.7 prepared), and with three fp8
+    terms up to a tile of 32 x 32 per CU (64 x 640 x 1280: 9.9 us raw, 19.9 prepared, whose activations
     are written as slots first; 154 x 2048 x 1280 20.6 and 28.0; beyond, 512 x 1280 x 1280, 30.6 and 25.8)."""
-    if dtype != torch.float32 or ((lowp, terms) == ("bf16", 2) and K % 8 == 0):
+    if dtype != torch.float32 or ((lowp, terms, products) == ("bf16", 2, "tri") and K % 8 == 0):
         return False
     return rows < 32 or ((lowp, terms) == ("fp8", 3) and K <= 4096 and -(-rows // 32) * -(-N // 32) <= 256)
 

@@ -24,7 +24,7 @@ def cascade_linear(x: torch.Tensor, weight: torch.Tensor, slots: Optional[torch.
     if slots is not None:
         pw = PreparedWeight.from_slots(slots, K, N, weight.dtype, lowp, terms, glu, b_exp)
         x2 = x.reshape(-1, K)
-        few_rows = raw_is_faster(x2.shape[0], K, N, x2.dtype, lowp, terms)
+        few_rows = raw_is_faster(x2.shape[0], K, N, x2.dtype, lowp, terms, products)
         if glu or (not few_rows and pw.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), products)):
             return cascaded_lowp_matmul(x, pw, bias=bias, products=products)
     return cascaded_lowp_matmul(x, weight, bias=bias, lowp=lowp, terms=terms, products=products, b_exp=b_exp)

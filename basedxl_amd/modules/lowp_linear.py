@@ -52,28 +52,26 @@ class BasedXLLowPLinear(nn.Module):
             return cascade_linear(x, self.weight, None if pw is None else pw.slots, self.bias, self.lowp, self.terms,
                                   self.products, False, self._weight_exp if pw is None else pw.exp)
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
-        pw = self._prepared_weight
-        if self.lowp == "fp8":
-            if self.prepared and not raw_is_faster(x.numel() // max(self.in_features, 1), self.in_features, self.out_features, x.dtype, self.lowp, self.terms):
-                y = None if pw is None or pw.device != self.weight.device else _lib.short_cut().fp8(
-                    x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
-            else:
-                y = None if self._weight_exp is None else _lib.short_cut().fp8(
-                    x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
-        elif not self.prepared:
-            y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
-        elif pw is not None and pw.device == self.weight.device:
-            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
-        else:
+        pw, rows = self._prepared_weight, x.numel() // max(self.in_features, 1)
+        raw = not self.prepared or raw_is_faster(rows, self.in_features, self.out_features, x.dtype, self.lowp, self.terms, self.products)
+        if not raw and (pw is None or pw.device != self.weight.device):
             y = None
+        elif self.lowp == "fp8" and raw:
+            y = None if self._weight_exp is None else _lib.short_cut().fp8(
+                x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
+        elif self.lowp == "fp8":
+            y = _lib.short_cut().fp8(x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
+        elif raw:
+            y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
+        else:
+            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
         if y is not None:
             return y
         if self.prepared and x.is_cuda:
             if self._prepared_weight is None or self._prepared_weight.device != self.weight.device:
                 self._prepared_weight = PreparedWeight(self.weight, lowp=self.lowp, terms=self.terms)
             x2 = x.reshape(-1, self.in_features)
-            few_rows = raw_is_faster(x2.shape[0], self.in_features, self.out_features, x2.dtype, self.lowp, self.terms)
-            if not few_rows and self._prepared_weight.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), self.products):
+            if not raw and self._prepared_weight.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), self.products):
                 return cascaded_lowp_matmul(x, self._prepared_weight, bias=self.bias, products=self.products)
         if self.lowp == "fp8" and (self._weight_exp is None or self._weight_exp.device != self.weight.device):
             self._weight_exp = tensor_scale_exp(self.weight)

@@ -80,6 +80,41 @@ def test_prepared_weights_pickled_before_the_short_cut_still_load():
     assert pickle.loads(pickle.dumps(again)).dt == again.dt == _lib.DT_F32
 
 
+@pytest.mark.parametrize("lowp,terms,products,rows,raw", [("fp16", 3, "tri", 2, True), ("fp16", 3, "tri", 31, True), ("fp16", 3, "tri", 32, False),
+                                                         ("bf16", 3, "tri", 16, True), ("bf16", 2, "full", 2, True), ("bf16", 2, "tri", 2, False),
+                                                         ("fp8", 3, "tri", 2, True), ("fp8", 3, "tri", 4100, False)])
+def test_eager_and_traced_layers_choose_the_same_weight(monkeypatch, lowp, terms, products, rows, raw):
+    """A prepared layer asks one rule whether few rows take the raw weight, whichever way it is called."""
+    from basedxl_amd import compiled
+    from basedxl_amd.modules import lowp_linear
+    taken, exp = [], torch.zeros(1, dtype=torch.int32) if lowp == "fp8" else None
+
+    class Recorder:
+        def matmul(*args):
+            taken.append("raw")
+            return args[0]
+
+        def prepared(*args):
+            taken.append("slots")
+            return args[0]
+
+        def fp8(*args):
+            taken.append("slots" if args[8] else "raw")
+            return args[0]
+
+    layer = BasedXLLowPLinear(torch.nn.Linear(128, 64), lowp=lowp, terms=terms, products=products, prepared=True)
+    layer._prepared_weight = PreparedWeight.from_slots(torch.zeros(16, dtype=torch.uint8), 128, 64, torch.float32, lowp, terms, exp=exp)
+    layer._weight_exp = exp
+    monkeypatch.setattr(lowp_linear._lib, "short_cut", lambda: Recorder)
+    x = torch.zeros(rows, 128)
+    layer(x)
+    monkeypatch.undo()
+    monkeypatch.setattr(PreparedWeight, "usable_with", lambda self, a2, products: True)
+    monkeypatch.setattr(compiled, "cascaded_lowp_matmul", lambda a, b, **_: taken.append("slots" if isinstance(b, PreparedWeight) else "raw") or a.new_empty(rows, 64))
+    compiled.cascade_linear._init_fn(x, layer.weight, layer._prepared_weight.slots, None, lowp, terms, products, False, exp)
+    assert taken == ["raw" if raw else "slots"] * 2
+
+
 def test_slots_are_checked_against_the_layout():
     w = PreparedWeight.from_slots(torch.zeros(2 * 12 * 64 * 16, dtype=torch.uint8), 96, 64, torch.float32, "bf16", 2)
     w.check_slots()
@@ -169,6 +204,22 @@ def test_fp8_layers_on_either_side_of_the_raw_weight_s_rule(gpu_device, rows, K,
         mod.prepare()
         assert torch.equal(mod(x), first)
         assert float((first.double() - want).norm() / want.norm()) < 1.4e-4       # (four times the cascade's own error, 3.5e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lowp,terms,products", [("fp16", 3, "tri"), ("bf16", 3, "tri"), ("bf16", 2, "full"), ("bf16", 2, "tri")])
+@pytest.mark.parametrize("rows", [2, 31, 33])
+def test_first_later_and_traced_calls_of_a_prepared_layer_have_the_same_bits(gpu_device, lowp, terms, products, rows):
+    from basedxl_amd.compiled import cascade_linear
+    torch.manual_seed(rows)
+    lin, x = torch.nn.Linear(1280, 640).to("cuda:0").requires_grad_(False), torch.randn(rows, 1280, device="cuda:0")
+    mod = BasedXLLowPLinear(lin, lowp=lowp, terms=terms, products=products, prepared=True)
+    first = mod(x)
+    mod.prepare()
+    assert torch.equal(mod(x), first)
+    assert torch.equal(cascade_linear(x, mod.weight, mod._prepared_weight.slots, mod.bias, lowp, terms, products, False, None), first)
+    if rows < 32 and (lowp, terms, products) != ("bf16", 2, "tri"):
+        assert torch.equal(BasedXLLowPLinear(lin, lowp=lowp, terms=terms, products=products)(x), first)
 
 
 @pytest.mark.gpu
