@@ -119,11 +119,13 @@ def native():
     if _native is None:
         try:
             module = importlib.import_module("._native", __package__)
-        except ImportError as e:
+            module.init(workspaces)
+            module.init_scales(scale_scratch)
+            if any(not hasattr(module, name) for name in ("matmul", "prepared", "fp8")):
+                raise AttributeError("a function is missing")
+        except (ImportError, AttributeError) as e:      # (AttributeError: the extension of an earlier build)
             raise ImportError(f"the host extension {os.path.join(_HERE, '_native.so')} is not built or does not load: {e}. "
                               "Run `python -m basedxl_amd.build`.") from None
-        module.init(workspaces)
-        module.init_scales(scale_scratch)
         _native = module
     return _native
 

@@ -26,8 +26,12 @@ def test_the_package_imports_before_anything_is_built(tmp_path):
     assert r.returncode == 0, r.stderr
 
 
-def test_without_the_extension_calls_take_the_python_path(tmp_path):
-    """An extension that does not load (a changed torch: here an empty file in its place) costs host time and a warning, no call."""
+@pytest.mark.parametrize("in_its_place", [("_native.so", ""), ("_native.py", "matmul = prepared = init = lambda *_: None\n"),
+                                          ("_native.py", "matmul = prepared = init = init_scales = lambda *_: None\n")],
+                         ids=["no extension", "of a build before the fp8 calls", "half of one"])
+def test_without_the_extension_calls_take_the_python_path(tmp_path, in_its_place):
+    """An extension that does not load (a changed torch: here an empty file in its place), or one that an earlier build left, costs
+    host time and a warning, no call."""
     import os
     import shutil
     import subprocess
@@ -36,7 +40,7 @@ def test_without_the_extension_calls_take_the_python_path(tmp_path):
     import basedxl_amd
     src = os.path.dirname(basedxl_amd.__file__)
     shutil.copytree(src, tmp_path / "basedxl_amd", ignore=shutil.ignore_patterns("_native.so", "build", "__pycache__"))
-    (tmp_path / "basedxl_amd" / "_native.so").write_bytes(b"")
+    (tmp_path / "basedxl_amd" / in_its_place[0]).write_text(in_its_place[1])
     code = """
 import warnings, torch, basedxl_amd as b
 from basedxl_amd import _lib
