@@ -62,7 +62,6 @@ struct Problem {
   // a call (not the selection functions, which answer for a shape): the small tiles of KIND_WAVEK are open too, and rows that
   // are not chunked, which these kernels read where they lie (what lies past K is masked)
   bool call = false;
-  bool gated_any = false;   // cascmm_gemm_gated: the gated stores on the raw weight that the selection and cascmm_gemm_glu leave out
   // three fp8 / fp16 terms: only the kernels that split both operands into slots first; K is rounded up to whole
   // stages, of which the operands hold k_valid, and their rows need no alignment
   bool split_first = false;
@@ -156,7 +155,6 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
     return false;
   // (rows that are not chunked: up to four rounds of tiles, larger problems are worth a copy of A)
   if (v.kind == KIND_WAVEK && q.bpre && q.K % 32 != 0 && !(q.chunked && q.K >= 64)) return false;   // (as KIND_SLOTK)
-  if (v.kind == KIND_WAVEK && q.glu && (!q.bpre && !q.gated_any)) return false;
   if (v.kind == KIND_WAVEK && (q.K == 0 || (q.K % 32 != 0 && !q.chunked && (!q.call || ((q.M + v.BM - 1) / v.BM) * ((q.N + v.BN - 1) / v.BN) > 4 * kNumCUs)) || (v.call_only && !q.call) || beyond_i32(q.M, q.lda, 4))) return false;
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
@@ -580,7 +578,7 @@ struct SelectKey {
   // flags: bpre << 1 | glu << 2, what variant_matches reads of the leading dimensions (the 32-bit addressing limits of
   // some kernels: M lda, K ldb, 1024 ldc and 256 ldc beyond 2^31 bytes << 3, 4, 5, 15; lda below 32 << 7), glu_slots << 6,
   // chunked << 8, split_first << 9, the fit of the rows << 10, whole_k << 12, K ldb as the kernels state it with
-  // stages past K, of four-byte and two-byte elements << 13, 14, call << 16, gated_any << 17
+  // stages past K, of four-byte and two-byte elements << 13, 14, call << 16
   int dtype, fmt, terms, products, count, flags;
   bool operator==(const SelectKey& o) const {
     return M == o.M && N == o.N && K == o.K && ws_bytes == o.ws_bytes && dtype == o.dtype && fmt == o.fmt &&
@@ -606,7 +604,7 @@ static int select_variant(const Problem& q, RowFit fit, int count, size_t ws_byt
   static std::mutex mu;
   static std::unordered_map<SelectKey, SelectHit, SelectKeyHash> memo;
   const SelectKey key{q.M, q.N, q.K, ws_bytes, q.dtype, q.fmt, q.terms, q.products, count,
-                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.call ? 65536 : 0) | (q.gated_any ? 131072 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
+                      (q.lda < 32 ? 128 : 0) | (q.chunked ? 256 : 0) | (q.split_first ? 512 : 0) | ((int)fit << 10) | (q.whole_k ? 4096 : 0) | (q.call ? 65536 : 0) | (q.bpre ? 2 : 0) | (q.glu ? 4 : 0) | (q.glu_slots ? 64 : 0) | (beyond_i32(q.M, q.lda, 4) ? 8 : 0) |
                           (beyond_i32(q.K, q.ldb, 4) ? 16 : 0) | (beyond_i32(q.ldc, 1024, 1) ? 32 : 0) | (beyond_i32(q.ldc, 256, 1) ? 32768 : 0) | (beyond_i32(q.K + 32, q.ldb, 4) ? 8192 : 0) |
                           (beyond_i32(q.K + 64, q.ldb, 2) ? 16384 : 0)};
   {

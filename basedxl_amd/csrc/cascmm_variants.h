@@ -259,7 +259,7 @@ int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
 }
 template <int W, int MB, int NB, int FMT, int TERMS, int BPRE>
 int launch_wavek(const GroupParams& p, hipStream_t stream) {
-  constexpr bool kGlu = W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16;
+  constexpr bool kGlu = BPRE && W == 16 && NB == 4;
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<W, MB, NB, W * MB / 8, 0, FMT, TERMS, BPRE>; return CASCMM_OK; }
   if ((p.glu && (!kGlu || p.glu != 1 || p.N % 64 != 0)) || p.k_splits > 1 || p.count < 1 || p.K <= 0) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 16 * Lowp<FMT>::planes(TERMS) : (int64_t)p.K * p.ldb * 4) > 0x7FFFFFFF)
@@ -441,7 +441,7 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
 #define CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, BPRE)                                                        \
   {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, WaveK<W, MB, NB>::BM, WaveK<W, MB, NB>::BN, WaveK<W, MB, NB>::BK,   \
    WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0,   \
-   W == 16 && NB == 4 && FMT == CASCMM_FMT_BF16, BPRE || FMT != CASCMM_FMT_BF16 || !wavek_for_shapes(W * MB, W * NB)}
+   BPRE && W == 16 && NB == 4, BPRE || FMT != CASCMM_FMT_BF16 || !wavek_for_shapes(W * MB, W * NB)}
 #define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS) CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, 0)
 
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \

@@ -121,9 +121,9 @@ constexpr bool wavek_fragments_inside() {
   return true;
 }
 
-template <int W, int NB, int FMT, int TERMS, int BPRE, int GLU>
+template <int W, int NB, int FMT, int TERMS, int BPRE>
 constexpr int wavek_b_loads() {
-  return BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : (W / 2) * (GLU ? 2 : 1);
+  return BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : W / 2;
 }
 
 // Host-checked: fp32 operands, 'tri' products; M * lda * 4 and K * ldb * 4 below 2 GiB.  Rows need no alignment (a 16-byte
@@ -132,12 +132,11 @@ constexpr int wavek_b_loads() {
 // chunks of A past K are fetched from beyond the buffer, what a row's last chunk holds past K is masked.
 // AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL), the lanes of the others read those again.
 // BPRE = 1: B is a prepared weight, [plane][4 ceil(K/32)][N] operand slots, a load per plane and column block (block nb: columns
-// W nb + c).  GLU = 1 (64-wide tiles): the gated store, C has N / 2 columns; a prepared weight alternates 32 value and 32 gate columns, of a
-// raw one blocks 0 and 1 are value columns 2 c + nb, blocks 2 and 3 their gates from the second half.
+// W nb + c).  GLU = 1 (prepared, 64-wide tiles): the gated store, C has N / 2 columns, B alternates 32 value and 32 gate columns.
 template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
-  static_assert(!GLU || (W == 16 && NB == 4), "a value block and its gate block in one tile");
-  typedef WaveK<W, MB, NB, AL, wavek_b_loads<W, NB, FMT, TERMS, BPRE, GLU>()> T;
+  static_assert(!GLU || (BPRE && W == 16 && NB == 4), "a value block and its gate block in one tile");
+  typedef WaveK<W, MB, NB, AL, wavek_b_loads<W, NB, FMT, TERMS, BPRE>()> T;
   typedef Lowp<FMT> L;
   constexpr int KM = T::KM, HALVES = T::HALVES, REGS = T::REGS;
   typedef float acc_t __attribute__((ext_vector_type(REGS)));
@@ -185,8 +184,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     a_voff[jp] = (int)(((int64_t)(m0 + (lane >> 3)) * p.lda + chunk * 4) * 4);
   }
   const int rows8 = (int)p.lda * 32;
-  // (GLU, raw: two value columns and, `gates` bytes further, their gates)
-  const int b_voff = BPRE ? (kg * p.N + n0 + lw) * 16 : 8 * kg * ldb_bytes + (GLU ? (n0 >> 1) + 2 * lw : n0 + NB * lw) * 4, gates = p.N * 2;
+  const int b_voff = BPRE ? (kg * p.N + n0 + lw) * 16 : 8 * kg * ldb_bytes + (n0 + NB * lw) * 4;
   // fragment of a block of rows: row lw, the chunks of k group kg of MFMA h at their rotated places
   static_assert(wavek_fragments_inside<W, MB, AL>(), "a fragment is read from the stage that was waited for");
   int a_frag[HALVES][2];
@@ -213,10 +211,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 #pragma unroll
       for (int e = 0; e < (BPRE ? 0 : 8); ++e) {
         const int soff = real ? (k0 + KM * h + e) * ldb_bytes : b_end;
-        if constexpr (GLU) {
-          const f32x2_ld v = llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0), g = llvm_raw_buffer_load_v2f32(rb, b_voff + gates, soff, 0);
-          Bv[st][h][e] = (bvec){v[0], v[1], g[0], g[1]};
-        } else if constexpr (NB == 1) Bv[st][h][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
+        if constexpr (NB == 1) Bv[st][h][e] = (bvec){llvm_raw_buffer_load_f32(rb, b_voff, soff, 0)};
         else if constexpr (NB == 2) Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v2f32(rb, b_voff, soff, 0));
         else Bv[st][h][e] = __builtin_bit_cast(bvec, llvm_raw_buffer_load_v4f32(rb, b_voff, soff, 0));
       }
@@ -380,7 +375,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       const int pos = q * T::NT + tid;
       const int blk = pos / 256, e = (pos / 64) % 4, ln = pos % 64;
       const int row = m0 + 16 * (blk >> 1) + 4 * (ln >> 4) + e, pair = blk & 1;
-      const int col = (n0 >> 1) + (BPRE ? 16 * pair + (ln & 15) : 2 * (ln & 15) + pair);
+      const int col = (n0 >> 1) + 16 * pair + (ln & 15);
       const int at = (((blk >> 1) * 4 + pair) * 4 + e) * 64 + ln;
       float v = 0.f, g = 0.f;
 #pragma unroll

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from basedxl_amd import PreparedWeight, _lib, cascaded_lowp_matmul
+from basedxl_amd.cascaded_lowp_matmul import cascaded_lowp_matmul_glu
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +36,31 @@ def test_every_number_of_steps_is_exact_on_integers(name, K):
         cascaded_lowp_matmul(frame[:, :K], w, out=got, lowp=lowp, terms=int(terms), variant=variant)
         assert torch.equal(got.cpu().long(), a @ b), (M, N)
         assert bool((out[M] == -77.0).all()) and bool((out[:, N] == -77.0).all())
+
+
+@pytest.mark.parametrize("name", [n for n in _TILES if n.endswith("_bpre") and n.split("x")[1] == "64"])
+@pytest.mark.parametrize("M,K,N", [(7, 72, 64), (8, 1280, 128), (9, 264, 192), (17, 520, 320), (81, 2568, 704)])
+def test_the_gated_store(name, M, K, N):
+    """value * gelu(gate) of integers below 2^18: sums exact, the gate within an fp32 ulp of the exact one (4e-7 + 2e-7 |gate|), the product
+    rounded once (2^-24 of it)."""
+    g = torch.Generator().manual_seed(M + K + N)
+    a, b, bias = (torch.randint(-9, 10, s, generator=g) for s in ((M, K), (K, N), (N,)))
+    value, gate = (a @ b + bias).double().chunk(2, -1)
+    want = value * torch.nn.functional.gelu(gate)
+    print("wavek gated", name, (M, K, N), flush=True)
+    frame = torch.full((M, K + 4), float("nan"), device="cuda:0")
+    frame[:, :K] = a.float().to("cuda:0")
+    got = cascaded_lowp_matmul(frame[:, :K], PreparedWeight(b.float().to("cuda:0"), glu=True), bias=bias.float().to("cuda:0"),
+                               variant=_lib.variant_names().index(name)).cpu().double()
+    assert bool(((got - want).abs() <= value.abs() * (4e-7 + 2e-7 * gate.abs()) + 2.0 ** -24 * want.abs()).all())
+
+
+def test_the_gated_store_is_on_prepared_weights_only():
+    for name in _TILES:
+        if not name.endswith("_bpre"):
+            a, b = torch.randn(8, 64, device="cuda:0"), torch.randn(64, 64, device="cuda:0")
+            with pytest.raises(_lib.CascmmError):
+                cascaded_lowp_matmul_glu(a, b, variant=_lib.variant_names().index(name))
 
 
 @pytest.mark.parametrize("name", [n for n in _TILES if n.startswith("t16x")])
