@@ -247,7 +247,7 @@ int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
   const bool tail = (!GLU && p.N % (W * NB) != 0) || p.K % 32 != 0, few = FEW != ALL && p.M <= 8;
   void (*kfn)(const GroupParams) = few ? (tail ? cascmm_wavek_kernel<W, MB, NB, FEW, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, FEW, 0, FMT, TERMS, BPRE, GLU>)
                                        : (tail ? cascmm_wavek_kernel<W, MB, NB, ALL, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS, BPRE, GLU>);
-  const int lds = few ? WaveK<W, MB, NB, FEW>::LDS_BYTES : WaveK<W, MB, NB, ALL>::LDS_BYTES;
+  const int lds = few ? WaveKOf<W, MB, NB, FEW, FMT, TERMS, BPRE>::LDS_BYTES : WaveKOf<W, MB, NB, ALL, FMT, TERMS, BPRE>::LDS_BYTES;
   static LdsFlags lds_set[4];
   if (!ensure_lds((const void*)kfn, lds, lds_set[(tail ? 1 : 0) + (few ? 2 : 0)])) return CASCMM_ERR_LAUNCH;
   GroupParams q = p;
@@ -439,8 +439,8 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
    F8Tile<MT>::T::NT, F8Tile<MT>::T::LDS_BYTES, true, false, &launch_f8k64<BPRE, MT>, BPRE}
 
 #define CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, BPRE)                                                        \
-  {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, WaveK<W, MB, NB>::BM, WaveK<W, MB, NB>::BN, WaveK<W, MB, NB>::BK,   \
-   WaveK<W, MB, NB>::NT, WaveK<W, MB, NB>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0,   \
+  {NAME, KIND_WAVEK, CASCMM_DT_F32, FMT, TERMS, false, W * MB, W * NB, 32, 512,                                            \
+   WaveKOf<W, MB, NB, W * MB / 8, FMT, TERMS, BPRE>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0, \
    BPRE && W == 16 && NB == 4, BPRE || FMT != CASCMM_FMT_BF16 || !wavek_for_shapes(W * MB, W * NB)}
 #define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS) CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, 0)
 

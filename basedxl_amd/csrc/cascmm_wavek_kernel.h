@@ -34,8 +34,8 @@
 
 namespace cascmm {
 
-// B_LOADS: loads of B per step and wave
-template <int W, int MB, int NB, int AL = W * MB / 8, int B_LOADS = W / 2>
+// AL: loads of A per step and wave (W MB / 8: all rows of the tile); B_LOADS: those of B
+template <int W, int MB, int NB, int AL, int B_LOADS>
 struct WaveK {
   static constexpr int BM = W * MB, BN = W * NB, BK = 32, NW = 8, NT = 512;
   static constexpr int KM = 512 / W, HALVES = BK / KM;     // k of an MFMA, MFMAs per step
@@ -121,10 +121,9 @@ constexpr bool wavek_fragments_inside() {
   return true;
 }
 
-template <int W, int NB, int FMT, int TERMS, int BPRE>
-constexpr int wavek_b_loads() {
-  return BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : W / 2;
-}
+// The sizes of one kernel: its launch has to bring the LDS that these stages take, and their number depends on the loads
+template <int W, int MB, int NB, int AL, int FMT, int TERMS, int BPRE>
+using WaveKOf = WaveK<W, MB, NB, AL, BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W / 16) : W / 2>;
 
 // Host-checked: fp32 operands, 'tri' products; M * lda * 4 and K * ldb * 4 below 2 GiB.  Rows need no alignment (a 16-byte
 // buffer load wants its address on a dword, and its dwords are checked against the buffer's end one by one).
@@ -136,7 +135,7 @@ constexpr int wavek_b_loads() {
 template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
   static_assert(!GLU || (BPRE && W == 16 && NB == 4), "a value block and its gate block in one tile");
-  typedef WaveK<W, MB, NB, AL, wavek_b_loads<W, NB, FMT, TERMS, BPRE>()> T;
+  typedef WaveKOf<W, MB, NB, AL, FMT, TERMS, BPRE> T;
   typedef Lowp<FMT> L;
   constexpr int KM = T::KM, HALVES = T::HALVES, REGS = T::REGS;
   typedef float acc_t __attribute__((ext_vector_type(REGS)));
