@@ -61,6 +61,7 @@ SIGNATURES = {
     "cascmm_variant_count": (c_int, []),
     "cascmm_variant_name": (c_char_p, [c_int]),
     "cascmm_variant_kernel": (c_char_p, [c_int]),
+    "cascmm_launched_kernel": (c_char_p, [c_int] + [c_int64] * 3),
     "cascmm_probe_mfma": (c_int, [c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "cascmm_probe_stream": (c_int, [c_void_p, c_void_p, c_size_t, c_int, c_void_p, c_size_t, c_void_p]),
     "cascmm_tensor_exp": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p]),

@@ -116,7 +116,7 @@ def _listing(src: str) -> str:
 def kernel_isa(symbol: str, jobs: int = 8) -> str:
     """gfx950 assembly of one kernel of the library, from its label to the end of its
     `.amdhsa_kernel` block (register counts, LDS and scratch sizes), compiled from the sources under
-    csrc/ with the flags of the build.  `symbol` is what `cascmm_variant_kernel` returns."""
+    csrc/ with the flags of the build.  `symbol` is what `cascmm_variant_kernel` or `cascmm_launched_kernel` returns."""
     srcs = [f for f in sources() if f.startswith("cascmm_inst_")] + [f for f in sources() if not f.startswith("cascmm_inst_")]
     with ThreadPoolExecutor(max_workers=min(jobs, len(srcs))) as ex:
         listings = list(ex.map(_listing, srcs))

@@ -775,12 +775,13 @@ def cascaded_lowp_matmul_glu_chained(a: torch.Tensor, w, *, bias: Optional[torch
     return out
 
 
-def kernel_listing(variant: int) -> str:
-    """What `dump_ptx=True` writes: the variant's name, its kernel's symbol and the kernel's gfx950
-    assembly (compiled from the library's sources on first use; without a compiler the two header
+def kernel_listing(variant: int, shape: Optional[Tuple[int, int, int]] = None) -> str:
+    """What `dump_ptx=True` writes: the variant's name, the symbol of its kernel (for ``shape`` = (M, N, K): of the form of it that such
+    a product runs) and the kernel's gfx950 assembly (compiled from the library's sources on first use; without a compiler the two header
     lines and the reason)."""
     l = _lib.lib()
-    name, sym = l.cascmm_variant_name(variant), l.cascmm_variant_kernel(variant)
+    name = l.cascmm_variant_name(variant)
+    sym = l.cascmm_variant_kernel(variant) if shape is None else l.cascmm_launched_kernel(variant, *shape)
     head = f"// gfx950 kernel variant: {name.decode() if name else variant}\n// kernel: {sym.decode() if sym else '?'}\n"
     if not sym:
         return head
@@ -887,6 +888,6 @@ def cascaded_lowp_matmul(
             a2.data_ptr(), b.data_ptr(), M, N, K, a2.stride(0) if M > 1 else max(K, 1), b.stride(0) if K > 1 else max(N, 1),
             out2.stride(0) if M > 1 else max(N, 1), dt, fmt, terms, prod, _workspace_bytes(M, N, K, dt, fmt, terms, prod))
         with open("dump.ptx", "w") as f:
-            f.write(kernel_listing(v & 0xFFFF))
+            f.write(kernel_listing(v & 0xFFFF, (M, N, K)))
 
     return out.reshape(*batch_dims, N)

@@ -1439,10 +1439,15 @@ const char* cascmm_variant_name(int variant) {
 }
 
 const char* cascmm_variant_kernel(int variant) {
-  if (variant < 0 || variant >= (int)table().size()) return nullptr;
+  return cascmm_launched_kernel(variant, 40960, 40960, 40960);   // (a multiple of every tile and stage)
+}
+
+const char* cascmm_launched_kernel(int variant, int64_t M, int64_t N, int64_t K) {
+  if (variant < 0 || variant >= (int)table().size() || M < 0 || N < 0 || K < 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return nullptr;
   const void* handle = nullptr;
   GroupParams p;
   memset(&p, 0, sizeof(p));
+  p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.kernel_out = &handle;
   if (table()[variant].launch(p, nullptr) != CASCMM_OK || !handle) return nullptr;
   // the handle of a kernel is an exported object of this library that carries the kernel's name

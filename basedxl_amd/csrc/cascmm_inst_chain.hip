@@ -84,7 +84,8 @@ static int slot_finish(const GroupParams& p, int st, hipStream_t stream) {
 
 // the variant-table face of the kernel: raw fp32 left operand, prepared right operand
 static int launch_slotk_variant(const GroupParams& p, hipStream_t stream) {
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_slotk_kernel<1, 0>; return CASCMM_OK; }
+  const bool tail = p.K % (2 * SlotK::BK) != 0;   // raw A comes in pairs of 16-k stages
+  if (p.kernel_out) { *p.kernel_out = tail ? (const void*)cascmm_slotk_kernel<1, 1> : (const void*)cascmm_slotk_kernel<1, 0>; return CASCMM_OK; }
   if (p.count != 1 || p.glu) return CASCMM_ERR_BAD_VARIANT;
   if (p.lda < 2 * SlotK::BK) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || prepared_kgroups(p.K) * p.N * 32 > 0x7FFFFFFF || p.ldc * (int64_t)(SlotK::BM * 4) > 0x7FFFFFFF)
@@ -92,8 +93,7 @@ static int launch_slotk_variant(const GroupParams& p, hipStream_t stream) {
   SlotKParams q;
   const int st = slot_params(p, q);
   if (st != CASCMM_OK) return st;
-  // (raw A comes in pairs of 16-k stages)
-  return slot_finish(p, p.K % (2 * SlotK::BK) == 0 ? launch_slotk_t<1, 0>(q, stream, p.k_splits) : launch_slotk_t<1, 1>(q, stream, p.k_splits), stream);
+  return slot_finish(p, tail ? launch_slotk_t<1, 1>(q, stream, p.k_splits) : launch_slotk_t<1, 0>(q, stream, p.k_splits), stream);
 }
 
 // the 64 x 80 tile of the same design, for problems that make too few 64 x 160 tiles to occupy the chip
@@ -120,13 +120,13 @@ static int launch_slotn_variant(const GroupParams& p, hipStream_t stream) {
 // both operands raw fp32
 static int launch_rawk_variant(const GroupParams& p, hipStream_t stream) {
   typedef SlotK T;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_rawk_kernel<0>; return CASCMM_OK; }
+  const bool tail = p.K % (2 * T::BK) != 0;   // raw A comes in pairs of stages
+  auto kfn = tail ? cascmm_rawk_kernel<1> : cascmm_rawk_kernel<0>;
+  if (p.kernel_out) { *p.kernel_out = (const void*)kfn; return CASCMM_OK; }
   if (p.count != 1 || p.glu) return CASCMM_ERR_BAD_VARIANT;
   if (p.lda < 2 * T::BK) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF || p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
-  const bool tail = p.K % (2 * T::BK) != 0;   // raw A comes in pairs of stages
-  auto kfn = tail ? cascmm_rawk_kernel<1> : cascmm_rawk_kernel<0>;
   static LdsFlags lds_set[2];
   if (!ensure_lds((const void*)kfn, T::LDS_BYTES, lds_set[tail ? 1 : 0])) return CASCMM_ERR_LAUNCH;
   SlotKParams q;

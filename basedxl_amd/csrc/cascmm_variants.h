@@ -247,6 +247,7 @@ int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
   const bool tail = (!GLU && p.N % (W * NB) != 0) || p.K % 32 != 0, few = FEW != ALL && p.M <= 8;
   void (*kfn)(const GroupParams) = few ? (tail ? cascmm_wavek_kernel<W, MB, NB, FEW, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, FEW, 0, FMT, TERMS, BPRE, GLU>)
                                        : (tail ? cascmm_wavek_kernel<W, MB, NB, ALL, 1, FMT, TERMS, BPRE, GLU> : cascmm_wavek_kernel<W, MB, NB, ALL, 0, FMT, TERMS, BPRE, GLU>);
+  if (p.kernel_out) { *p.kernel_out = (const void*)kfn; return CASCMM_OK; }
   const int lds = few ? WaveKOf<W, MB, NB, FEW, FMT, TERMS, BPRE>::LDS_BYTES : WaveKOf<W, MB, NB, ALL, FMT, TERMS, BPRE>::LDS_BYTES;
   static LdsFlags lds_set[4];
   if (!ensure_lds((const void*)kfn, lds, lds_set[(tail ? 1 : 0) + (few ? 2 : 0)])) return CASCMM_ERR_LAUNCH;
@@ -260,7 +261,7 @@ int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
 template <int W, int MB, int NB, int FMT, int TERMS, int BPRE>
 int launch_wavek(const GroupParams& p, hipStream_t stream) {
   constexpr bool kGlu = BPRE && W == 16 && NB == 4;
-  if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_wavek_kernel<W, MB, NB, W * MB / 8, 0, FMT, TERMS, BPRE>; return CASCMM_OK; }
+  if (p.kernel_out) return launch_wavek_kernel<W, MB, NB, FMT, TERMS, BPRE, 0>(p, stream);
   if ((p.glu && (!kGlu || p.glu != 1 || p.N % 64 != 0)) || p.k_splits > 1 || p.count < 1 || p.K <= 0) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 16 * Lowp<FMT>::planes(TERMS) : (int64_t)p.K * p.ldb * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;

@@ -271,8 +271,11 @@ const char* cascmm_variant_name(int variant);
  * code object, a profiler's kernel trace and an assembly listing of the library's sources spell it;
  * static string, NULL for an index outside the table.  Works without a GPU.  Stands where the
  * reference reads its compiled kernel back from the launch (`kernel.asm["ptx"]`,
- * basedxl/triton/cascaded_lowp_matmul.py:163-171): the wrapper's `dump_ptx` looks this symbol up. */
+ * basedxl/triton/cascaded_lowp_matmul.py:163-171): the wrapper's `dump_ptx` looks the symbol up.  Several variants have
+ * forms of their kernel for the end of K, columns past the edge or few rows: cascmm_launched_kernel gives the one that
+ * a plain product of this size runs, cascmm_variant_kernel the one for whole tiles. */
 const char* cascmm_variant_kernel(int variant);
+const char* cascmm_launched_kernel(int variant, int64_t M, int64_t N, int64_t K);
 
 /* fp8 tensor scale: writes to *exp_out (device int32) the exponent e with
  * max|x| * 2^e in (224, 448] (0 for an all-zero tensor).  x is [rows, cols] with leading

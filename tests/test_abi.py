@@ -69,6 +69,21 @@ def test_every_variant_names_its_kernel_and_the_kernel_has_a_listing():
     assert ".amdhsa_private_segment_fixed_size 0\n" in text          # and nothing spilled to scratch memory
 
 
+def test_the_listed_kernel_is_the_form_that_a_size_runs():
+    """Few rows, columns past the last tile's edge and the end of K have forms of their own; whole tiles are what the index alone names."""
+    l, names = _lib.lib(), _lib.variant_names()
+    form = lambda name, *shape: l.cascmm_launched_kernel(names.index(name), *shape).decode()
+    tile = "t16x16x32_wavek_bf16x2_tri"
+    for shape, want in (((2, 1280, 1280), (1, 0)), ((2, 1281, 1280), (1, 1)), ((8, 64, 33), (1, 1)), ((9, 1280, 1280), (2, 0)), ((9, 1280, 1270), (2, 1))):
+        assert f"cascmm_wavek_kernelILi16ELi1ELi1ELi{want[0]}ELi{want[1]}E" in form(tile, *shape), shape
+    assert form(tile, 4096, 4096, 4096).encode() == l.cascmm_variant_kernel(names.index(tile))
+    for name in ("k64x160x16_wk4_bf16x2_tri", "k64x160x16_wk4_bf16x2_tri_bpre", "k64x80x32_wk4_bf16x2_tri_bpre"):
+        assert form(name, 64, 160, 1288) != form(name, 64, 160, 1280) == l.cascmm_variant_kernel(names.index(name)).decode(), name
+    for i, name in enumerate(names):
+        assert l.cascmm_launched_kernel(i, 333, 211, 456).decode().startswith("_ZN6cascmm"), name
+    assert l.cascmm_launched_kernel(len(names), 1, 1, 1) is None and l.cascmm_launched_kernel(0, -1, 1, 1) is None
+
+
 def _gemm(M, N, K, lda=None, ldb=None, ldc=None, dtype=0, fmt=0, terms=2, products=0, A=8, B=8, C=8):
     l = _lib.lib()
     return l.cascmm_gemm(A, B, C, None, M, N, K, lda if lda is not None else K, ldb if ldb is not None else N,
