@@ -57,6 +57,7 @@ SIGNATURES = {
     "cascmm_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int]),
     "cascmm_select_variant": (c_int, [c_int64] * 6 + [c_int] * 4),
     "cascmm_call_variant": (c_int, [c_void_p, c_void_p] + [c_int64] * 6 + [c_int] * 4 + [c_size_t]),
+    "cascmm_call_variant_prepared": (c_int, [c_void_p, c_int] + [c_int64] * 5 + [c_int] * 4 + [c_size_t]),
     "cascmm_select_variant_grouped": (c_int, [c_int] + [c_int64] * 6 + [c_int] * 4),
     "cascmm_variant_count": (c_int, []),
     "cascmm_variant_name": (c_char_p, [c_int]),

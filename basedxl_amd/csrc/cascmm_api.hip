@@ -1422,6 +1422,20 @@ int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int6
   return v >= 0 ? v : select_variant(q, fit, 1, workspace_bytes);
 }
 
+int cascmm_call_variant_prepared(const void* A, int glu, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int dtype, int fmt,
+                                 int terms, int products, size_t workspace_bytes) {
+  Problem q{M, N, K, lda, N, ldc, dtype, fmt, terms, products};
+  q.bpre = true;
+  q.glu = glu != 0;
+  const int st = check_problem(q);
+  if (st != CASCMM_OK) return st;
+  if (q.glu && (N % 64 != 0 || K == 0)) return CASCMM_ERR_BAD_SHAPE;
+  if (prepared_bytes(K, N, fmt, terms, q.glu) > INT32_MAX) return CASCMM_ERR_TOO_LARGE;
+  q.chunked = chunked_by_k(q);
+  q.call = true;
+  return select_variant(q, row_fit(q, A, nullptr), 1, q.glu ? 0 : workspace_bytes);
+}
+
 int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                                   int dtype, int fmt, int terms, int products) {
   if (count < 1 || count > kMaxGroup) return CASCMM_ERR_BAD_SHAPE;

@@ -13,7 +13,7 @@ One "step" is one pass of the hot path over one batch of synthetic input:
   to_v from X in one grouped launch, to_out from a second activation tensor).
 
 * ``--workload kv``: the cross-attention key / value projections of the 77 text tokens, X fp32 [154, 2048] x W fp32
-  [2048, 1280] and [2048, 640]: the skinny split-K path, reported in HBM GB/s over the algorithmic bytes;
+  [2048, 1280] and [2048, 640]: one launch with K split over the waves of a workgroup, reported in HBM GB/s over the algorithmic bytes;
 * ``--workload unet``: every Linear layer and 1x1 convolution of one SDXL UNet denoising step (batch 2, 128x128
   latent, random weights), as the patched module tree of basedxl_amd.unet_skeleton calls them, full latent and
   one GPU's half-latent share, 2-term bf16 and 3-term fp8 cascades.
@@ -226,6 +226,13 @@ def measured_peaks(dev):
                    "events around 5 launches after 0.2 s of the same launches"}
 
 
+def _kernel_of_call(l, a, b):
+    """Name of the kernel that an eager call on these two fp32 tensors launches (two bf16 terms)."""
+    (m, k), n = a.shape, b.shape[1]
+    v = l.cascmm_call_variant(a.data_ptr(), b.data_ptr(), m, n, k, k, n, n, 0, 0, 2, 0, l.cascmm_workspace_bytes(m, n, k, 0, 0, 2, 0))
+    return l.cascmm_variant_name(v).decode()
+
+
 def bench_kv(dev, check=True):
     """cfg4: the two cross-attention K/V projections of the text tokens; bandwidth-style figures
     over the algorithmic bytes 4 (MK + KN + MN)."""
@@ -250,7 +257,7 @@ def bench_kv(dev, check=True):
         rec = {"M": 154, "K": 2048, "N": n, "launch_us": round(us, 2), "algorithmic_bytes": algo,
                "hbm_gbs": round(algo / us * 1e-3, 1), "frac_of_8TBs": round(algo / us * 1e-3 / 8000.0, 4),
                "fp32_equiv_tflops": round(2.0 * 154 * 2048 * n / us * 1e-6, 1),
-               "kernel": l.cascmm_variant_name(l.cascmm_select_variant(154, n, 2048, 2048, n, n, 0, 0, 2, 0)).decode()}
+               "kernel": _kernel_of_call(l, x, w)}
         if check:
             exp = oc.fp64_matmul(x_cpu, w_cpu)
             ek, eo = oc.error_metrics(res.cpu(), exp), oc.error_metrics(oc.cascade_matmul_ref(x_cpu, w_cpu), exp)
@@ -368,7 +375,7 @@ def bench_attn(dev, check=True):
     flop = 2.0 * 4096 * 640 * 640
     names = _lib.variant_names()
     k_qkv = names[l.cascmm_select_variant_grouped(3, 4096, 640, 640, 640, 640, 640, 0, 0, 2, 0) & 0xFFFF]
-    k_o = names[l.cascmm_select_variant(4096, 640, 640, 640, 640, 640, 0, 0, 2, 0) & 0xFFFF]
+    k_o = _kernel_of_call(l, x2, w[3])
     rec = {"workload": "cfg2: SDXL 64x64-stage self-attention projections on one GPU's patch share: X fp32 [4096,640] ~N(0,1) x W fp32 "
                        "[640,640] ~N(0,0.02), to_q/to_k/to_v as one grouped launch + to_out; 2-term bf16 cascade (3 products), both "
                        "operands split inside the kernels",
@@ -479,7 +486,7 @@ def bench_sweep(dev, sizes=(256, 512, 1024, 2048, 4096, 8192)):
         ref = a.double() @ b.double()
         err = lambda x: float((x.double() - ref).norm() / ref.norm())   # noqa: E731
         e_c, e_32, e_16 = err(cascaded_lowp_matmul(a, b)), err(torch.matmul(a, b)), err(torch.matmul(a16, b16))
-        rows.append({"n": n, "kernel": l.cascmm_variant_name(l.cascmm_select_variant(n, n, n, n, n, n, 0, 0, 2, 0)).decode(),
+        rows.append({"n": n, "kernel": _kernel_of_call(l, a, b),
                      "cascade_bf16x2_us": round(us, 2), "cascade_fp32_equiv_tflops": round(flop / us * 1e-6, 1),
                      "cascade_mfma_tflops": round(3 * flop / us * 1e-6, 1), "cascade_rel_fro": e_c,
                      "torch_fp32_us": round(us32, 2), "torch_fp32_tflops": round(flop / us32 * 1e-6, 1), "torch_fp32_rel_fro": e_32,

@@ -244,21 +244,28 @@ int cascmm_chained_supported(int64_t M, int64_t N, int64_t K);
 int cascmm_gemm_chained(const void* Aslots, const void* Bslots, void* C, const void* bias,
                         int64_t M, int64_t N, int64_t K, int64_t ldc, void* stream);
 
-/* Bytes of device workspace cascmm_gemm can use for this problem (0 for most shapes).
+/* Bytes of device workspace that some kernel can use for this problem, by choice or by index (0 for most shapes; of few
+ * rows the partial results of kernels that only an index selects: no call needs them, and none fails without).
  * Counterpart of nothing in the reference (its small-M shapes fall back to torch.matmul,
  * cascaded_lowp_matmul.py:155-156); the caller allocates, as it allocates `out` (:161). */
 size_t cascmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int fmt, int terms,
                               int products);
 
-/* Variant the automatic selection would run for this problem (index), or a negative status: on rows of whole
- * 16-byte chunks that start on 16-byte boundaries, without what a call does to others first (rows copied into
- * the workspace, K of the three-term fp8 / fp16 cascades rounded up to whole stages). */
+/* Variant that the selection has for a shape (index), or a negative status: on rows of whole 16-byte chunks that
+ * start on 16-byte boundaries.  What a call launches may be another one: calls have more kernels (small problems on the
+ * tiles that split K over eight waves; the kernels that split K over workgroups on few rows are in the place of those
+ * here, and run in no call), estimates of their own, copy rows into the workspace first and round K of the three-term
+ * fp8 / fp16 cascades up to whole stages.  cascmm_call_variant and cascmm_call_variant_prepared answer for a call. */
 int cascmm_select_variant(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                           int dtype, int fmt, int terms, int products);
 /* Variant that cascmm_gemm launches for these very operands with this much workspace (0: none), or a negative status:
  * the GEMM kernel itself, where copies, splits or a reduction go with it.  Nothing is read or launched. */
 int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                         int64_t ldc, int dtype, int fmt, int terms, int products, size_t workspace_bytes);
+/* The same for cascmm_gemm_prepared (glu == 0) and cascmm_gemm_prepared_glu (glu != 0, N the projection's width; takes
+ * no workspace) with one problem. */
+int cascmm_call_variant_prepared(const void* A, int glu, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int dtype,
+                                 int fmt, int terms, int products, size_t workspace_bytes);
 /* Same as cascmm_select_variant for a grouped launch of `count` problems (the choice depends on how many tiles the
  * group has in total). */
 int cascmm_select_variant_grouped(int count, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

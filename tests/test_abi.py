@@ -224,6 +224,23 @@ def test_the_kernel_of_a_call_is_the_one_that_is_launched():
     assert l.cascmm_call_variant(A, B, 4, 4, 4, 3, 4, 4, 0, 0, 2, 0, 0) == -2
 
 
+def test_the_kernel_of_a_prepared_call_is_asked_for_the_call():
+    """Calls have the small tiles, which the selection for a shape leaves out; of large problems both say the same."""
+    l, names = _lib.lib(), _lib.variant_names()
+
+    def kernel(M, K, N, glu=0, a=0, lda=0):
+        return names[l.cascmm_call_variant_prepared((1 << 40) + a, glu, M, N, K, lda or K, N // 2 if glu else N, 0, 0, 2, 0, 1 << 30) & 0xFFFF]
+
+    for M, K, N in ((2000, 1280, 10240), (4096, 4096, 4096)):
+        assert kernel(M, K, N) == names[l.cascmm_select_variant_prepared(1, M, N, K, K, N, 0, 0, 2, 0) & 0xFFFF]
+    for glu in (0, 1):
+        assert "_wavek_" in kernel(2, 1280, 1280, glu) and kernel(2, 1280, 1280, glu).endswith("_bpre")
+        assert "_wavek_" in kernel(64, 520, 640, glu, a=4, lda=523)
+    assert "_wavek_" not in names[l.cascmm_select_variant_prepared(1, 2, 1280, 1280, 1280, 1280, 0, 0, 2, 0) & 0xFFFF]
+    call = lambda glu, M, N, K, lda, ldc: l.cascmm_call_variant_prepared(1 << 40, glu, M, N, K, lda, ldc, 0, 0, 2, 0, 0)   # noqa: E731
+    assert call(0, 4, 4, 64, 63, 4) == -2 and call(1, 4, 96, 64, 64, 48) == -2 and call(0, 64, 1 << 20, 65536, 65536, 1 << 20) == -9
+
+
 @pytest.mark.parametrize("M,K,N,large", [(3072, 576, 1728, False), (4928, 384, 1152, False), (6976, 320, 960, False),
                                          (1500, 1280, 10240, True), (4096, 4096, 4096, True), (7800, 640, 5120, True)])
 def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):

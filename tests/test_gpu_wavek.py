@@ -92,3 +92,16 @@ def test_a_call_repeats_its_bits_and_keeps_non_finite_values_to_their_rows(M, K,
     want = a.double() @ b.double()
     ok = ~bad
     assert float((first.double() - want)[ok].norm() / want[ok].norm()) < 1.8e-5
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 1280, 1280), (64, 520, 640), (200, 2560, 640), (640, 1280, 1280)])
+@pytest.mark.parametrize("glu", [False, True])
+def test_the_kernel_that_a_prepared_call_is_said_to_launch(M, K, N, glu):
+    """Its bits are those of that kernel by index."""
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    a, w = torch.randn(M, K, device="cuda:0", generator=g), PreparedWeight(torch.randn(K, N, device="cuda:0", generator=g), glu=glu)
+    v = _lib.lib().cascmm_call_variant_prepared(a.data_ptr(), int(glu), M, N, K, K, N // 2 if glu else N, 0, 0, 2, 0,
+                                                _lib.lib().cascmm_workspace_bytes(M, N, K, 0, 0, 2, 0))
+    print("wavek call", (M, K, N), glu, _lib.variant_names()[v & 0xFFFF], flush=True)
+    if "_wavek_" in _lib.variant_names()[v]:      # (the others may split K over workgroups, which the index alone does not)
+        assert torch.equal(cascaded_lowp_matmul(a, w), cascaded_lowp_matmul(a, w, variant=v))
