@@ -44,7 +44,11 @@ struct TunedCost;
 struct CallCost;
 // per variant, resolved once when the table is built: its measured cost constants (or none) and what
 // kind of kernel its name says it is
-struct VariantInfo { const TunedCost* tuned; const CallCost* call; bool p8; bool bdirect; };
+struct VariantInfo {
+  const TunedCost* tuned;
+  const CallCost *call, *shape;   // (shape: for the selection functions)
+  bool p8, bdirect;
+};
 static const std::vector<VariantInfo>& variant_info();
 
 static bool aligned_to(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
@@ -226,71 +230,87 @@ static bool ksplit_kind(const VariantDesc& v) { return v.kind == KIND_H16 || v.k
 constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {1280, 5120} x 1280, 4096 x {640, 2560} x 640)
 
 
-// Calls with two bf16 terms, plain products.  A launch of `tiles` tiles on 256 CUs, k in units of the kernel's loop (KIND_WAVEK:
-// steps per wave; K over four waves: trips of 256 k, in 64s; else 64 k):  c0 + full (c1 + k r1) + |k s0, fill k s1 + MB of B / bw|_x  (the
-// x-norm), where full rounds of 256 tiles go before one that is `fill` full; 16 x 16 and 16 x 32 tiles, of which several fit a CU, have
-// no rounds.  deep: what a step past the straight code's adds; edge: tiles over the edge of C.  Fitted to 1150 shapes (those of a
-// UNet step and of its image sizes, squares, small ones; graph replay, every kernel forced in turn), mean error 0.02 - 0.09: the
-// kernel chosen is 2.2 % behind the fastest of all on average, 7.4 % with the constants above (649 x 320 x 2496 17.1 us, 10.0 on the
-// B-direct kernel; 12 x 3392 x 7104 42.8, 17.7 on a 16 x 32 tile; 1024^3 16.6, 14.2).  The selection functions, which answer for shapes,
-// keep the constants above but for KIND_WAVEK.
+// Calls with two bf16 terms, plain products.  A launch of `tiles` tiles on 256 CUs, k in units of the kernel's loop (KIND_WAVEK and
+// KIND_HWK: steps per wave; K over four waves: trips of 256 k, in 64s; else 64 k):  c0 + full (c1 + k r1) + |k s0, fill k s1 + MB of B / bw|_x
+// (the x-norm), where full rounds of 256 tiles go before one that is `fill` full.  The small tiles have rounds like the others, though several fit
+// a CU: the one CU that gets a second tile runs both at once, and each takes longer (200 x 2560 x 640 prepared: 260 tiles of 16 x 32 14.8 us,
+// 200 of them for 154 rows 9.8; 70 of 32 x 32 10.9).  deep: what a step past the straight code's adds; for the
+// kernels without any, us per 1e9 multiply-adds (tiles filled up) at the board's power, which deep products of many tiles run into.  edge: tiles over
+// an edge of C, us per round (their store is the checked one); of the small ones the share that the form for the right edge costs.
+// MB: both operands.  Fitted to 1633 prepared and 1526 raw shapes of 2 - 9000 rows, K 256 - 5120, widths 256 - 10240, a fifth of them the sizes that
+// models have and squares (graph replay over three sets of operands, every kernel forced in turn), mean error 0.02 - 0.09.  The kernel chosen
+// is behind the fastest of all, on average and in one of twenty: 2 - 2048 rows 0.5 and 3.0 % (prepared), 0.5 and 1.8 % (raw); 600 - 9000 rows 1.0 and 5.7 %,
+// 1.1 and 7.1 %; products beyond 1.2e10 multiply-adds 0.2 and 1.0 %, 0.1 and 0 %; sizes of models 0.4 and 3.0 %, 0.7 and 5.3 %.  (With constants fitted to one set of
+// operands, which the L2s kept, small tiles without rounds and B's bytes alone: 1.5 and 9.9 %, 1.3 and 11 %; 1.7 and 10 %, 2.2 and 16 %; 0.5 and 2.6 %, 0.9 and 8.3 %;
+// 1.3 and 9.6 %, 1.5 and 11 %: 7296 x 1198 x 283 52.6 us, 43.0 with the constants above.)  The eight-wave tiles' errors are on the low side behind a full round
+// (7 %) and with more than 5 MB of A (10 %; rows off 16 bytes of 20 MB and more 25 %, where a copy of A is the alternative), which their estimates are
+// raised by.
+// The selection functions, which answer for shapes, keep the constants above but for KIND_WAVEK.
 struct CallCost { const char* name; double c0, s0, s1, c1, bw, x, r1, deep, edge; };
 static const CallCost kCallCost[] = {
-    {"t16x16x32_wavek_bf16x2_tri", 1.79, 0.413, 0.493, 0, 24.3, 1.26, 0, 0.0881, 0},
-    {"t16x32x32_wavek_bf16x2_tri", 1.88, 0.636, 0.667, 0, 40, 1.26, 0, 0, 0},
-    {"t16x64x32_wavek_bf16x2_tri", 1.97, 1.05, 0.732, 0.678, 15.6, 1.67, 1.2, 0, 0},
+    {"t16x16x32_wavek_bf16x2_tri", 2.45, 0.392, 0.199, 0, 26, 1, 0.477, 0.125, 0.0733},
+    {"t16x32x32_wavek_bf16x2_tri", 2.43, 0.679, 0.376, 0, 19.2, 1.44, 0.656, 0.0251, 0.0805},
+    {"t16x64x32_wavek_bf16x2_tri", 2.5, 0.887, 0.404, 1.12, 25.1, 1, 1.06, 0, 0.0803},
+    {"t32x32x32_wavek_bf16x2_tri", 2.48, 0.877, 0.553, 0.589, 60, 1.29, 1.2, 0, 0.0976},
+    {"t32x64x32_wavek_bf16x2_tri", 3.09, 1.09, 0.626, 1.69, 60, 1, 1.44, 0, 0.0651},
+    {"t64x64x32_wavek_bf16x2_tri", 5.14, 1.28, 1.23, 2.43, 60, 1.23, 2.22, 0, 0.037},
+    {"k64x160x16_wk4_bf16x2_tri", 6.72, 0.592, 0.608, 5.22, 19.3, 2.07, 0.82, 5.46, 0.162},
+    {"bd64x128x64_d3_p4_bf16x2_tri", 4.37, 1.09, 0.917, 1.9, 16.7, 3.99, 1.09, 0.0779, 0.772},
+    {"bd96x128x64_d3_p4_bf16x2_tri", 5.76, 1.25, 1.03, 3.14, 6.56, 4.48, 1.28, 6.18, 1.47},
+    {"bd128x128x32_d3_p4_bf16x2_tri", 5.1, 1.49, 1.21, 3.11, 17, 2.76, 1.53, 6.22, 1.88},
+    {"bd192x128x64_d2_p4_bf16x2_tri", 7.67, 1.87, 1.47, 4.33, 5, 3.57, 2.05, 5.59, 3.17},
+    {"t64x64x64_w2x2x1_d3_bf16x2_tri", 4.88, 0.671, 0.104, 0.691, 60, 1, 0.7, 0, 0.618},
+    {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 6.45, 0.892, 0.615, 2.27, 22.4, 2.09, 0.892, 7.16, 4.2},
+    {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 8.12, 0.968, 1.11, 2.25, 11.9, 2.48, 1.24, 5.43, 4.48},
+    {"t256x128x32_w4x1x1_d2_bf16x2_tri", 9.38, 1.84, 2, 2.77, 7.14, 3.36, 2.32, 4.93, 11.1},
+    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 11.5, 2.09, 2.02, 0.699, 5, 2.59, 2.71, 4.86, 12.8},
+    {"t256x256x32_w512_edge_bf16x2_tri", 10.7, 2.93, 4.73, 9.7, 25.5, 3.7, 4.83, 0.105, 1.47},
+    {"t256x320x32_w512_edge_bf16x2_tri", 12.4, 3.48, 5.78, 13.7, 60, 3.27, 5.71, 0.0162, 1.61},
+    {"t256x320x32_w512_bf16x2_tri", 12.3, 3.45, 5.72, 13.6, 60, 3.27, 5.65, 0.016, 0},
+    // three fp16 terms (448 shapes; the tile chosen is 0.06 % behind the fastest of the three, without rounds 0.4 %, at most 26 %)
+    {"t16x16x32_wavek_fp16x3_tri", 2.47, 0.728, 0.176, 0.125, 28.6, 1, 0.664, 0.051, 0},
+    {"t16x32x32_wavek_fp16x3_tri", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
+    {"t32x32x32_wavek_fp16x3_tri", 2.79, 1.5, 0.319, 1.57, 60, 1, 1.62, 0, 0},
+    // three fp8 terms (493 shapes, hardly ever behind the fastest; without rounds 0.6 %, at most 33 %)
+    {"t16x16x32_wavek_fp8x3_tri", 2.54, 0.713, 0.229, 0.147, 28.1, 1, 0.655, 0.00446, 0},
+    {"t16x32x32_wavek_fp8x3_tri", 2.57, 1.1, 0.207, 1.1, 26.9, 1, 1.24, 0, 0},
+    {"t32x32x32_wavek_fp8x3_tri", 2.91, 1.4, 0.425, 2.04, 60, 1, 4.23, 0.0301, 0},
+    // prepared weights
+    {"t16x16x32_wavek_bf16x2_tri_bpre", 2.63, 0.241, 0.211, 0.112, 20.1, 1.25, 0.347, 0.0308, 0.0554},
+    {"t16x32x32_wavek_bf16x2_tri_bpre", 2.6, 0.367, 0.314, 0, 19.2, 1.27, 0.547, 0.0707, 0.036},
+    {"t16x64x32_wavek_bf16x2_tri_bpre", 2.69, 0.604, 0.365, 0.906, 26.6, 1, 0.986, 0.155, 0.0211},
+    {"t32x32x32_wavek_bf16x2_tri_bpre", 2.67, 0.592, 0.597, 0.772, 29, 1.53, 0.986, 0, 0.0563},
+    {"t32x64x32_wavek_bf16x2_tri_bpre", 2.97, 0.872, 0.585, 1.22, 60, 1, 1.32, 0, 0.0249},
+    {"t64x64x32_wavek_bf16x2_tri_bpre", 4.59, 1.13, 0.884, 1.99, 60, 1.04, 2.03, 0, 0.0331},
+    {"k64x80x32_wk4_bf16x2_tri_bpre", 5.85, 0.322, 0.13, 4.01, 60, 1, 0.433, 5.65, 0},
+    {"k64x160x16_wk4_bf16x2_tri_bpre", 7.2, 0.561, 0.597, 5.11, 18.8, 3.01, 0.738, 4.98, 0.181},
+    {"t64x64x64_w2x2x1_d3_bf16x2_tri_bpre", 4.84, 0.42, 0.155, 0.696, 60, 1.04, 0.515, 7.64, 0.667},
+    {"t64x160x64_w2x1x2_d2_bf16x2_tri_bpre", 7.56, 0.676, 0.654, 2.64, 11.4, 2.59, 0.847, 6.02, 1.9},
+    {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 7.06, 0.989, 1.13, 1.76, 60, 2.59, 1.29, 5.41, 2.23},
+    {"t128x128x64_w2x2x1_d2_bf16x2_tri_bpre", 8.38, 0.911, 1.17, 1.53, 11.9, 3.15, 1.25, 4.85, 2.13},
+    {"t128x160x32_w2x1x2_d3_bf16x2_tri_bpre", 8.7, 1.09, 1.2, 2.33, 6.04, 2.66, 1.48, 4.52, 5.43},
+    {"t256x128x32_w4x1x1_d2_bf16x2_tri_bpre", 8.58, 1.54, 1.81, 3.81, 13.7, 2.3, 2.26, 4.32, 3.23},
+    {"t256x160x32_w4x1x1_d2_bf16x2_tri_bpre", 9.46, 1.98, 2.55, 1.51, 9.49, 4.62, 2.69, 4.44, 8.45},
+    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 11.4, 2.77, 4.31, 9.8, 14.7, 3.83, 4.45, 3.63, 0.921},
+    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 12, 3.27, 5.17, 11, 22.9, 2.97, 5.43, 0.301, 2.16},
+    {"t256x320x32_w512_bf16x2_tri_bpre", 11.9, 3.24, 5.12, 10.9, 22.9, 2.97, 5.38, 0.298, 0},
+};
+// What the selection functions, and with them the limits of cascmm_gemm_noalloc, price the two tiles of KIND_WAVEK by that they know
+static const CallCost kShapeCost[] = {
     {"t32x32x32_wavek_bf16x2_tri", 1.98, 1, 1.02, 0.468, 37.6, 2.39, 1.23, 0, 0},
     {"t32x64x32_wavek_bf16x2_tri", 2.68, 1.22, 0.589, 0.662, 40, 1.12, 1.77, 0, 0},
-    {"t64x64x32_wavek_bf16x2_tri", 4.64, 1.43, 1.5, 1.78, 40, 1.53, 2.5, 0, 0},
-    {"k64x160x16_wk4_bf16x2_tri", 5.89, 0.622, 0.789, 4.3, 40, 2.93, 0.882, 0, 0.0243},
-    {"bd64x128x64_d3_p4_bf16x2_tri", 4.45, 0.993, 0.111, 1.57, 33.2, 1, 1.11, 0, 0.0431},
-    {"bd96x128x64_d3_p4_bf16x2_tri", 5.99, 1.2, 1.12, 3.16, 40, 4.94, 1.29, 0, 0.058},
-    {"bd128x128x32_d3_p4_bf16x2_tri", 5.71, 1.43, 1.36, 1.74, 5.17, 3.92, 1.65, 0, 0.0717},
-    {"t64x64x64_w2x2x1_d3_bf16x2_tri", 4.46, 0.674, 0.149, 0.798, 40, 1.23, 0.686, 0, 0.0424},
-    {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 5.9, 0.899, 1.02, 2.35, 10.1, 8, 0.972, 0, 0.29},
-    {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 8.68, 0.897, 1.3, 1.49, 8.53, 3.67, 1.37, 0, 0.193},
-    {"t256x128x32_w4x1x1_d2_bf16x2_tri", 9.48, 1.79, 2.2, 6.57, 3.09, 4.83, 2.22, 0, 0.254},
-    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 11.5, 2.05, 3.13, 11.7, 40, 7.77, 2.36, 0, 0.231},
-    {"t256x256x32_w512_edge_bf16x2_tri", 11.1, 2.98, 4.74, 10.2, 40, 4.25, 4.83, 0, 0.00177},
-    {"t256x320x32_w512_edge_bf16x2_tri", 12, 3.38, 5, 13.4, 19, 2.39, 5.8, 0, 0.013},
-    {"t256x320x32_w512_bf16x2_tri", 11.9, 3.21, 5, 6.51, 40, 2.24, 6.86, 0, 0.02},
-    // three fp16 terms (150 shapes, mean error 0.06 - 0.09)
-    {"t16x16x32_wavek_fp16x3_tri", 2.38, 0.675, 0.768, 0, 19.6, 1.61, 0, 0.0438, 0},
-    {"t16x32x32_wavek_fp16x3_tri", 2.54, 1.12, 1.57, 0, 16.2, 6.97, 0, 0.0319, 0},
-    {"t32x32x32_wavek_fp16x3_tri", 2.75, 1.46, 0.223, 1.49, 35.4, 1, 1.66, 0, 0},
-    // three fp8 terms (as three fp16 ones)
-    {"t16x16x32_wavek_fp8x3_tri", 2.52, 0.655, 0.749, 0, 17.9, 1.54, 0, 0, 0},
-    {"t16x32x32_wavek_fp8x3_tri", 2.65, 1.11, 1.6, 0, 16.1, 7.35, 0, 0, 0},
-    {"t32x32x32_wavek_fp8x3_tri", 2.82, 1.44, 0.245, 1.52, 34.4, 1, 1.67, 0, 0},
-    // prepared weights (460 shapes, mean error 0.01 - 0.05; the kernel chosen is 1 % behind the fastest, 8.6 % with the constants above)
-    {"t16x16x32_wavek_bf16x2_tri_bpre", 2.09, 0.244, 0.389, 0, 40, 1.62, 0, 0.217, 0},
-    {"t16x32x32_wavek_bf16x2_tri_bpre", 1.86, 0.448, 0.564, 0, 40, 1.52, 0, 0, 0},
-    {"t16x64x32_wavek_bf16x2_tri_bpre", 1.83, 1.02, 1.17, 0.568, 40, 5.19, 1.01, 0, 0},
-    {"t32x32x32_wavek_bf16x2_tri_bpre", 2.03, 0.766, 0.681, 0.327, 40, 2.09, 1.04, 0, 0},
-    {"t32x64x32_wavek_bf16x2_tri_bpre", 2.08, 1.21, 0.761, 1.1, 40, 1.73, 1.37, 0, 0},
-    {"t64x64x32_wavek_bf16x2_tri_bpre", 3.41, 1.5, 1.63, 2.34, 40, 1.96, 2.03, 0, 0},
-    {"k64x80x32_wk4_bf16x2_tri_bpre", 5.19, 0.37, 0.3, 3.44, 40, 1.92, 0.462, 0, 0},
-    {"k64x160x16_wk4_bf16x2_tri_bpre", 6.41, 0.569, 0.744, 3.8, 40, 3.31, 0.829, 0, 0.00316},
-    {"t64x64x64_w2x2x1_d3_bf16x2_tri_bpre", 4.49, 0.438, 0.315, 0.682, 40, 1.63, 0.523, 0, 0.0601},
-    {"t64x160x64_w2x1x2_d2_bf16x2_tri_bpre", 7.34, 0.687, 0.872, 2.96, 14.5, 4.04, 0.912, 0, 0.079},
-    {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 7.04, 0.955, 1.33, 2.27, 40, 4.22, 1.35, 0, 0.0662},
-    {"t128x128x64_w2x2x1_d2_bf16x2_tri_bpre", 8.06, 0.89, 1.26, 2.09, 26, 3.42, 1.29, 0, 0.0649},
-    {"t128x160x32_w2x1x2_d3_bf16x2_tri_bpre", 8.89, 1.05, 1.37, 7.27, 10.3, 2.87, 1.34, 0, 0.136},
-    {"t256x128x32_w4x1x1_d2_bf16x2_tri_bpre", 8.5, 1.55, 2.15, 4.93, 16.8, 3.28, 2.31, 0, 0.0704},
-    {"t256x160x32_w4x1x1_d2_bf16x2_tri_bpre", 9.96, 1.86, 2.98, 9.1, 40, 7.28, 2.45, 0, 0.168},
-    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 10.9, 2.79, 4.39, 8.94, 40, 4.13, 4.51, 0, 0.0112},
-    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 12, 3.31, 5, 11.3, 40, 2.94, 5.34, 0, 0.016},
-    {"t256x320x32_w512_bf16x2_tri_bpre", 12, 3.21, 5, 16, 40, 2.8, 5.18, 0, 0.02},
 };
 static const std::vector<VariantInfo>& variant_info() {
   static const std::vector<VariantInfo> info = [] {
     std::vector<VariantInfo> v;
     for (const VariantDesc& d : table()) {
-      VariantInfo i{nullptr, nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
+      VariantInfo i{nullptr, nullptr, nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
       for (const TunedCost& t : kTuned)
         if (strcmp(t.name, d.name) == 0) i.tuned = &t;
       for (const CallCost& t : kCallCost)
         if (strcmp(t.name, d.name) == 0) i.call = &t;
+      for (const CallCost& t : kShapeCost)
+        if (strcmp(t.name, d.name) == 0) i.shape = &t;
       v.push_back(i);
     }
     return v;
@@ -299,12 +319,19 @@ static const std::vector<VariantInfo>& variant_info() {
 }
 static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Problem& q, int count, double tiles, int64_t k_per) {
   const double k = v.kind == KIND_WAVEK || v.kind == KIND_HWK ? (double)(((k_per + v.BK - 1) / v.BK + 7) / 8) : v.kind == KIND_SLOTK ? (double)((k_per + 255) / 256 * 4) : (double)k_per / 64.0;
-  const double per = tiles / kNumCUs, mb = (double)count * (double)q.K * (double)q.N * (double)dtype_size(q.dtype) * 1.0e-6;
-  const double few = v.kind == KIND_HWK ? 4 : 8;   // steps of a wave's straight code
-  const double full = v.BM * v.BN <= 512 ? 0.0 : std::ceil(per) - 1.0, fill = per - full;
-  const double lone = k * t.s0 + (k > few ? t.deep * (k - few) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
+  const double per = tiles / kNumCUs, mb = (double)count * (double)q.K * (double)(q.call ? q.M + q.N : q.N) * (double)dtype_size(q.dtype) * 1.0e-6;
+  const double few = v.kind == KIND_HWK ? kHwkStraight : wavek_straight(v.BM * v.BN);
+  const double full = std::ceil(per) - 1.0, fill = per - full;
+  const bool small = v.kind == KIND_WAVEK || v.kind == KIND_HWK;
+  const double lone = k * t.s0 + (small && k > few ? t.deep * (k - few) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
   const double us = t.c0 + full * (t.c1 + k * t.r1) + std::pow(std::pow(lone, t.x) + std::pow(shared, t.x), 1.0 / t.x);
-  return q.N % v.BN != 0 || q.M % v.BM != 0 ? us * (1.0 + t.edge) : us;
+  if (small) {
+    const double late = v.kind != KIND_WAVEK || !q.call ? 1.0 : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
+    return late * (q.N % v.BN != 0 ? us * (1.0 + t.edge) : us);
+  }
+  const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * (full + 1.0) : us;
+  const double power = t.deep * tiles * v.BM * v.BN * (double)k_per * 1.0e-9;
+  return std::pow(std::pow(edged, 8.0) + std::pow(power, 8.0), 0.125);
 }
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
@@ -318,8 +345,9 @@ static double wavek_estimate_us(const Problem& q, int count) {
   double best = 1e9;
   for (size_t i = 0; i < table().size(); ++i) {
     const VariantDesc& v = table()[i];
-    if (v.kind != KIND_WAVEK || v.bpre || !variant_info()[i].call || (v.call_only && !q.call)) continue;
-    best = std::min(best, call_estimate_us(*variant_info()[i].call, v, q, count, (double)count * (double)((q.M + v.BM - 1) / v.BM) * (double)((q.N + v.BN - 1) / v.BN), q.K));
+    const VariantInfo& info = variant_info()[i];
+    if (v.kind != KIND_WAVEK || v.bpre || !(q.call ? info.call : info.shape)) continue;
+    best = std::min(best, call_estimate_us(q.call ? *info.call : *info.shape, v, q, count, (double)count * (double)((q.M + v.BM - 1) / v.BM) * (double)((q.N + v.BN - 1) / v.BN), q.K));
   }
   return best;
 }
@@ -353,32 +381,32 @@ static double h16_estimate_us(const VariantDesc& v, const Problem& q, double til
 }
 
 // The same problems with K over eight waves (KIND_HWK), with a launch's constants of kCallCost (`form`: 0 prepared, 1 raw, 2 gated).
-// Fitted to 326 shapes of 2 - 2600 rows, K and widths 256 - 10240 (fp16, graph replay over three sets of operands, every tile forced
-// in turn), mean error 0.03 - 0.08.  They win where the tiles about fit the CUs at once (2 x 1280 x 1280 prepared 3.2 us, 6.9 on the four-wave kernels;
-// 154 x 2048 x 1280 5.6, 10.3), and lose behind that, where every tile pays its launch and its meeting in LDS (2048 x 640 x 640 raw
-// 12.0 us, 7.3).  The estimates decide, and within 10 % of each other (their error) the four-wave kernels stay; raw weights deeper than
-// the straight code's four steps a wave stay with them too (10 x 2496 x 760 6.4 us, here 7.4): 0.77 (prepared), 0.83 (raw) and 0.90 (gated) of the
-// time without these kernels over the shapes, one of them slower (41 x 4000 x 1624 prepared 8.4 us, here 9.2; 9.2 and 8.9 eager).  64 x 64 tiles
+// Fitted as those to 642 prepared and 383 raw shapes of 2 - 2048 rows (fp16), and 262 gated ones.  They win where the tiles about fit the CUs at once
+// (2 x 1280 x 1280 prepared 3.2 us, 6.9 on the four-wave kernels; 154 x 2048 x 1280 5.6, 10.3), and lose behind that, where every tile pays its launch and
+// its meeting in LDS (2048 x 640 x 640 raw 12.0 us, 7.3).  The estimates decide; raw weights deeper than the straight
+// code's four steps a wave stay with the four-wave kernels (10 x 2496 x 760 6.4 us, here 7.4).  The kernel chosen is 0.3 % (prepared) and 0.6 % (raw) behind the
+// fastest of all on average, 2.0 and 3.9 % in one of twenty; prepared 1.2 and 9.0 % with the small tiles priced without rounds
+// (41 x 4000 x 1624: 104 tiles of 32 x 32 9.2 us, 153 of 16 x 32 8.0; 8.5 on the four-wave kernels).  64 x 64 tiles
 // gained only with the gated store (plain, by index only: 976 x 2048 x 640 9.1 us on the four-wave kernels, 10.6 on them).
 struct HwkCost { int BM, BN, form; CallCost c; };
 static const HwkCost kHwkCost[] = {
-    {16, 16, 0, {nullptr, 2.7, 0.143, 0.345, 0, 20.2, 2.37, 0, 0.197, 0}},
-    {16, 32, 0, {nullptr, 2.61, 0.289, 0.51, 0, 15.7, 2.01, 0, 0.281, 0}},
-    {16, 64, 0, {nullptr, 2.72, 0.492, 0.214, 0.388, 14.9, 1.18, 0.902, 0.383, 0}},
-    {32, 32, 0, {nullptr, 2.8, 0.395, 0.411, 1.12, 12, 1.98, 0.735, 0.184, 0}},
-    {32, 64, 0, {nullptr, 2.91, 0.604, 0.484, 1.06, 19.6, 1.13, 1.19, 0.244, 0}},
-    {16, 32, 1, {nullptr, 2.43, 0.472, 0.805, 0, 30.3, 2.04, 0, 0.5, 0.0752}},
-    {16, 64, 1, {nullptr, 2.58, 0.861, 0.328, 1.32, 40, 1.03, 1.1, 0.5, 0.0352}},
-    {32, 32, 1, {nullptr, 2.68, 0.509, 0.39, 1.31, 40, 1, 0.934, 0.5, 0.0326}},
-    {32, 64, 1, {nullptr, 2.87, 0.978, 0.485, 1.74, 40, 1.05, 1.23, 0.443, 0.0123}},
-    {16, 64, 2, {nullptr, 3.14, 0.0359, 0.141, 0.86, 6.09, 7.35, 0.455, 0.05, 0.0069}},
-    {32, 64, 2, {nullptr, 3.6, 0.264, 0.0524, 1.97, 6.36, 8, 0.586, 0.0225, 0.00763}},
-    {64, 64, 2, {nullptr, 4.08, 0.02, 0.312, 2.82, 6.07, 7.47, 0.839, 0.0025, 0.007}},
+    {16, 16, 0, {nullptr, 3.13, 0.0911, 0.117, 0.239, 19.1, 1, 0.286, 0.237, 0}},
+    {16, 32, 0, {nullptr, 3.04, 0.221, 0.18, 0.249, 18.8, 1, 0.409, 0.294, 0}},
+    {16, 64, 0, {nullptr, 3.07, 0.471, 0.246, 0.59, 19.2, 1, 0.831, 0.444, 0}},
+    {32, 32, 0, {nullptr, 3.16, 0.344, 0.328, 1.06, 33.6, 1, 0.75, 0.215, 0}},
+    {32, 64, 0, {nullptr, 3.22, 0.608, 0.561, 1.44, 43.3, 1, 1.07, 0.3, 0}},
+    {16, 32, 1, {nullptr, 2.99, 0.459, 0.308, 0.135, 17.3, 1.23, 0.679, 0.614, 0}},
+    {16, 64, 1, {nullptr, 3.04, 0.843, 0.221, 0.966, 23.6, 1, 1.18, 0.607, 0}},
+    {32, 32, 1, {nullptr, 3.1, 0.52, 0.535, 0.895, 30.1, 1.2, 1.03, 0.561, 0}},
+    {32, 64, 1, {nullptr, 3.25, 0.935, 0.471, 1.38, 27.2, 1, 1.36, 0.509, 0}},
+    {16, 64, 2, {nullptr, 3.32, 0.463, 0.236, 0.562, 16.3, 1, 0.778, 0.427, 0}},
+    {32, 64, 2, {nullptr, 3.53, 0.594, 0.474, 1.27, 33.8, 1, 1.23, 0.353, 0}},
+    {64, 64, 2, {nullptr, 3.84, 0.862, 0.823, 1.92, 60, 1, 1.61, 0.195, 0}},
 };
 static double hwk_estimate_us(const VariantDesc& v, const Problem& q, int count, double tiles) {
   if (!q.bpre && q.K > 2048) return 1e9;
   for (const HwkCost& t : kHwkCost)
-    if (t.BM == v.BM && t.BN == v.BN && t.form == (q.glu ? 2 : q.bpre ? 0 : 1)) return 1.1 * call_estimate_us(t.c, v, q, count, tiles, q.K);
+    if (t.BM == v.BM && t.BN == v.BN && t.form == (q.glu ? 2 : q.bpre ? 0 : 1)) return call_estimate_us(t.c, v, q, count, tiles, q.K);
   return 1e9;
 }
 
@@ -461,10 +489,10 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   }
   if (costed_call(q, count) && !info.call && v.fast && v.kind != KIND_SPLITK) return 1e9;   // (nowhere the fastest)
   if (info.call && (costed_call(q, count) || v.kind == KIND_WAVEK)) {
-    const CallCost& t = *info.call;
+    const CallCost& t = !q.call && info.shape ? *info.shape : *info.call;
     if (v.kind != KIND_SLOTK) return call_estimate_us(t, v, q, count, tiles, q.K);
     int ks = 1;
-    const double us = ksplit_best(q, count, tiles, ws_bytes, 2.8, 12.0e6, &ks, [&](double n, int64_t k) { return call_estimate_us(t, v, q, count, n, k); });
+    const double us = ksplit_best(q, count, tiles, ws_bytes, 2.85, 9.0e6, &ks, [&](double n, int64_t k) { return call_estimate_us(t, v, q, count, n, k); });
     if (splits_out) *splits_out = ks;
     return us;
   }
@@ -472,7 +500,8 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
   int ks = 1;
   if (v.kind == KIND_H16 || (v.kind == KIND_SLOTK && info.tuned)) {
     const double us = v.kind == KIND_H16
-        ? ksplit_best(q, count, tiles, ws_bytes, 1.6, 3.8e6, &ks, [&](double t, int64_t k) { return h16_estimate_us(v, q, t, k); })
+        // (calls on prepared weights, 255 shapes: 2 x 4928 x 2880 in eleven splits 10.2 us, not the 8.0 of the constants before)
+        ? ksplit_best(q, count, tiles, ws_bytes, q.call && q.bpre ? 1.65 : 1.6, q.call && q.bpre ? 1.5e6 : 3.8e6, &ks, [&](double t, int64_t k) { return h16_estimate_us(v, q, t, k); })
         : ksplit_best(q, count, tiles, ws_bytes, 2.8, 12.0e6, &ks, [&](double t, int64_t k) { return slotk_estimate_us(*info.tuned, v, q, t, k); });
     if (splits_out) *splits_out = ks;
     return us;

@@ -27,7 +27,7 @@ struct HWK {
   static constexpr int MB = MB_, NB = NB_, BM = 16 * MB, BN = 16 * NB, BK = 64, NW = 8, NT = 512;
   static constexpr int A_LOADS = 2 * MB, B_LOADS = RAWB ? 16 : 2 * NB, LOADS = A_LOADS + B_LOADS;   // per wave and step
   static constexpr int NS = MB == 1 ? 4 : MB == 2 ? 3 : 2;   // steps in LDS and registers
-  static constexpr int STRAIGHT = 4;                         // steps of a wave that have straight code
+  static constexpr int STRAIGHT = kHwkStraight;
   static constexpr int A_STAGE = A_LOADS * 1024, RING = NS * A_STAGE, PART = BM * BN * 4;
   static constexpr int LDS_BYTES = NW * (RING > PART ? RING : PART);
   static_assert((NS - 1) * LOADS <= 60, "the wait counter has six bits");

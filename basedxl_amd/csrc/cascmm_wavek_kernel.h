@@ -34,6 +34,10 @@
 
 namespace cascmm {
 
+// steps of a wave that have straight code, by the tile's size, and in cascmm_hwk_kernel.h
+constexpr int wavek_straight(int area) { return area == 256 ? 8 : area == 512 ? 6 : area <= 2048 ? 4 : 2; }
+constexpr int kHwkStraight = 4;
+
 // AL: loads of A per step and wave (W MB / 8: all rows of the tile); B_LOADS: those of B
 template <int W, int MB, int NB, int AL, int B_LOADS>
 struct WaveK {
@@ -42,7 +46,7 @@ struct WaveK {
   static constexpr int REGS = W * W / 64;                  // accumulator registers of a block
   static constexpr int LOADS = AL + B_LOADS;               // per wave and step
   static constexpr int NS = BM == 16 && LOADS <= 15 ? 5 : BM <= 32 ? (LOADS <= 20 ? 4 : 3) : 2;               // steps in LDS and registers
-  static constexpr int STRAIGHT = BM * BN == 256 ? 8 : BM * BN == 512 ? 6 : BM * BN <= 2048 ? 4 : 2;   // steps of a wave that have straight code
+  static constexpr int STRAIGHT = wavek_straight(BM * BN);
   static constexpr int A_STAGE = AL * 1024;
   static constexpr int RING = NS * A_STAGE;                // per wave
   static constexpr int PART = BM * BN * 4;                 // a wave's partial tile

@@ -241,6 +241,24 @@ def test_the_kernel_of_a_prepared_call_is_asked_for_the_call():
     assert call(0, 4, 4, 64, 63, 4) == -2 and call(1, 4, 96, 64, 64, 48) == -2 and call(0, 64, 1 << 20, 65536, 65536, 1 << 20) == -9
 
 
+@pytest.mark.parametrize("cascade,prepared,M,K,N,slower", [
+    ((0, 0, 2), True, 200, 2560, 640, "t16x32x32_wavek"),       # 260 tiles on 256 CUs 14.8 us, 70 of 32 x 32 10.9
+    ((0, 0, 2), True, 70, 2752, 1728, "t16x32x32_wavek"),       # 270 tiles 15.3, 162 of 32 x 32 11.2
+    ((0, 0, 2), True, 3392, 960, 256, "t64x64x32_wavek"),       # 13 MB of rows 14.0, K over four waves 11.4
+    ((0, 0, 2), False, 51, 2792, 1152, "t16x16x32_wavek"),      # 288 tiles 15.1, 13.2
+    ((0, 0, 2), False, 7296, 1198, 283, "t64x64x32_wavek"),     # 570 tiles on the rows as they lie 52.6, copied first 43.0
+    ((0, 0, 2), False, 5504, 512, 832, "t256x128x32"),          # 38.2, on a kernel that was left out 28.7
+    ((1, 1, 1), True, 12, 2680, 4544, "t16x16x64_hwk"),         # 284 tiles 10.6, 142 of 16 x 32 8.7
+])
+def test_the_small_tiles_have_rounds_and_their_rows_bytes(cascade, prepared, M, K, N, slower):
+    """A CU that gets a second tile takes longer for both, and operands come from further away than the L2s where a model has several: the
+    estimates behind a call's choice say so.  (us, graph replay over three sets of operands)"""
+    l, names = _lib.lib(), _lib.variant_names()
+    A, B, room = 1 << 40, 2 << 40, 1 << 30
+    v = l.cascmm_call_variant_prepared(A, 0, M, N, K, K, N, *cascade, 0, room) if prepared else l.cascmm_call_variant(A, B, M, N, K, K, N, N, *cascade, 0, room)
+    assert v >= 0 and not names[v & 0xFFFF].startswith(slower)
+
+
 @pytest.mark.parametrize("M,K,N,large", [(3072, 576, 1728, False), (4928, 384, 1152, False), (6976, 320, 960, False),
                                          (1500, 1280, 10240, True), (4096, 4096, 4096, True), (7800, 640, 5120, True)])
 def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):
