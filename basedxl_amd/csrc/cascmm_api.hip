@@ -46,7 +46,7 @@ struct CallCost;
 // kind of kernel its name says it is
 struct VariantInfo {
   const TunedCost* tuned;
-  const CallCost *call, *shape;   // (shape: for the selection functions)
+  const CallCost *call, *gated, *shape;   // (shape: for the selection functions)
   bool p8, bdirect;
 };
 static const std::vector<VariantInfo>& variant_info();
@@ -295,6 +295,20 @@ static const CallCost kCallCost[] = {
     {"t256x320x32_w512_edge_bf16x2_tri_bpre", 12, 3.27, 5.17, 11, 22.9, 2.97, 5.43, 0.301, 2.16},
     {"t256x320x32_w512_bf16x2_tri_bpre", 11.9, 3.24, 5.12, 10.9, 22.9, 2.97, 5.38, 0.298, 0},
 };
+// Gated calls on prepared weights (N: the projection's width; 1096 shapes, fitted in the same way: 0.2 - 0.7 % behind the fastest on average, 5 % in one of
+// twenty; with the eight-wave tiles priced by the plain products' constants and the others by the ones above 1.5 and 9 %: 893 x 320 x 2240 16.6 us,
+// 12.3 on 64 x 64 tiles; 4736 x 4256 x 256 84 and 73)
+static const CallCost kGatedCost[] = {
+    {"t16x64x32_wavek_bf16x2_tri_bpre", 2.56, 0.634, 0.372, 0.75, 19.8, 1, 0.976, 0.0835, 0},
+    {"t32x64x32_wavek_bf16x2_tri_bpre", 2.89, 0.876, 0.596, 0.944, 60, 1, 1.38, 0, 0},
+    {"t64x64x32_wavek_bf16x2_tri_bpre", 4.74, 0.71, 1.13, 1.92, 60, 1.12, 2.1, 0.426, 0},
+    {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 7.36, 0.951, 0.377, 0.872, 60, 1.26, 1.32, 5.89, 2.34},
+    {"t128x128x64_w2x2x1_d2_bf16x2_tri_bpre", 8.87, 0.909, 1.03, 0.863, 18.9, 3.8, 1.29, 5.41, 2.07},
+    {"t256x128x32_w4x1x1_d2_bf16x2_tri_bpre", 9.06, 1.51, 1.84, 2.77, 60, 2.29, 2.4, 4.47, 4.59},
+    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 12.8, 2.79, 4.18, 8.81, 55.8, 3.41, 4.54, 4.19, 0},
+    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 17.3, 3.38, 5.37, 14.6, 60, 4.03, 5.44, 3.56, 0},
+    {"t256x320x32_w512_bf16x2_tri_bpre", 17.1, 3.35, 5.32, 14.5, 60, 4.03, 5.39, 3.52, 0},
+};
 // What the selection functions, and with them the limits of cascmm_gemm_noalloc, price the two tiles of KIND_WAVEK by that they know
 static const CallCost kShapeCost[] = {
     {"t32x32x32_wavek_bf16x2_tri", 1.98, 1, 1.02, 0.468, 37.6, 2.39, 1.23, 0, 0},
@@ -304,11 +318,13 @@ static const std::vector<VariantInfo>& variant_info() {
   static const std::vector<VariantInfo> info = [] {
     std::vector<VariantInfo> v;
     for (const VariantDesc& d : table()) {
-      VariantInfo i{nullptr, nullptr, nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
+      VariantInfo i{nullptr, nullptr, nullptr, nullptr, strstr(d.name, "_p8_") != nullptr, d.name[0] == 'b' && d.name[1] == 'd'};
       for (const TunedCost& t : kTuned)
         if (strcmp(t.name, d.name) == 0) i.tuned = &t;
       for (const CallCost& t : kCallCost)
         if (strcmp(t.name, d.name) == 0) i.call = &t;
+      for (const CallCost& t : kGatedCost)
+        if (strcmp(t.name, d.name) == 0) i.gated = &t;
       for (const CallCost& t : kShapeCost)
         if (strcmp(t.name, d.name) == 0) i.shape = &t;
       v.push_back(i);
@@ -326,7 +342,7 @@ static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Pr
   const double lone = k * t.s0 + (small && k > few ? t.deep * (k - few) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
   const double us = t.c0 + full * (t.c1 + k * t.r1) + std::pow(std::pow(lone, t.x) + std::pow(shared, t.x), 1.0 / t.x);
   if (small) {
-    const double late = v.kind != KIND_WAVEK || !q.call ? 1.0 : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
+    const double late = v.kind != KIND_WAVEK || !q.call || q.glu ? 1.0 : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
     return late * (q.N % v.BN != 0 ? us * (1.0 + t.edge) : us);
   }
   const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * (full + 1.0) : us;
@@ -337,9 +353,9 @@ static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
          !q.glu && q.K > 0 && !beyond_i32(q.M, q.lda, 4);
 }
-// a call whose kernels all have such constants
+// a call whose kernels all have such constants (plain groups too: the tiles of all problems, 0.99 of the time with the constants above over 400 groups of three)
 static bool costed_call(const Problem& q, int count) {
-  return q.call && count == 1 && q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.glu;
+  return q.call && (count == 1 || !q.glu) && q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && (!q.glu || q.bpre);
 }
 static double wavek_estimate_us(const Problem& q, int count) {
   double best = 1e9;
@@ -487,12 +503,13 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
       if (table()[i].kind == KIND_SLOTK && variant_matches(table()[i], q, FIT_DWORD) && variant_cost(i, q, count, ws_bytes) < skinny_us) return 1e9;
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
-  if (costed_call(q, count) && !info.call && v.fast && v.kind != KIND_SPLITK) return 1e9;   // (nowhere the fastest)
-  if (info.call && (costed_call(q, count) || v.kind == KIND_WAVEK)) {
-    const CallCost& t = !q.call && info.shape ? *info.shape : *info.call;
-    if (v.kind != KIND_SLOTK) return call_estimate_us(t, v, q, count, tiles, q.K);
+  const bool costed = costed_call(q, count);
+  const CallCost* c = costed && q.glu ? info.gated : !q.call && info.shape ? info.shape : info.call;
+  if (costed && !c && v.fast) return 1e9;   // (nowhere the fastest)
+  if (c && (costed || v.kind == KIND_WAVEK)) {
+    if (v.kind != KIND_SLOTK) return call_estimate_us(*c, v, q, count, tiles, q.K);
     int ks = 1;
-    const double us = ksplit_best(q, count, tiles, ws_bytes, 2.85, 9.0e6, &ks, [&](double n, int64_t k) { return call_estimate_us(t, v, q, count, n, k); });
+    const double us = ksplit_best(q, count, tiles, ws_bytes, 2.85, 9.0e6, &ks, [&](double n, int64_t k) { return call_estimate_us(*c, v, q, count, n, k); });
     if (splits_out) *splits_out = ks;
     return us;
   }
@@ -1624,7 +1641,9 @@ int cascmm_selftest(void) {
     for (const VariantDesc& d : t) hits += strcmp(c.name, d.name) == 0 ? 1 : 0;
     bad += hits == 1 ? 0 : 1;
   }
-  for (const CallCost& c : kCallCost) {
+  std::vector<CallCost> calls(std::begin(kCallCost), std::end(kCallCost));
+  calls.insert(calls.end(), std::begin(kGatedCost), std::end(kGatedCost));
+  for (const CallCost& c : calls) {
     int hits = 0;
     for (const VariantDesc& d : t) hits += strcmp(c.name, d.name) == 0 ? 1 : 0;
     bad += hits == 1 ? 0 : 1;

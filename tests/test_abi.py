@@ -259,6 +259,14 @@ def test_the_small_tiles_have_rounds_and_their_rows_bytes(cascade, prepared, M, 
     assert v >= 0 and not names[v & 0xFFFF].startswith(slower)
 
 
+@pytest.mark.parametrize("M,K,N,kernel", [(893, 320, 2240, "t64x64x32_wavek"), (824, 320, 2368, "t64x64x32_wavek"),    # 16.6 and 16.1 us on 64 x 256, 12.3 and 12.2
+                                          (1024, 640, 640, "t64x64x32_wavek"), (2, 1280, 10240, "t16x64x32_wavek"), (4096, 1280, 10240, "t256x")])
+def test_gated_calls_compare_their_kernels_by_one_scale(M, K, N, kernel):
+    l = _lib.lib()
+    v = l.cascmm_call_variant_prepared(1 << 40, 1, M, N, K, K, N // 2, 0, 0, 2, 0, 0)
+    assert _lib.variant_names()[v].startswith(kernel)
+
+
 @pytest.mark.parametrize("M,K,N,large", [(3072, 576, 1728, False), (4928, 384, 1152, False), (6976, 320, 960, False),
                                          (1500, 1280, 10240, True), (4096, 4096, 4096, True), (7800, 640, 5120, True)])
 def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):
