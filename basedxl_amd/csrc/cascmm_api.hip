@@ -240,7 +240,7 @@ constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {128
 // MB: both operands.  Fitted to 1633 prepared and 1526 raw shapes of 2 - 9000 rows, K 256 - 5120, widths 256 - 10240, a fifth of them the sizes that
 // models have and squares (graph replay over three sets of operands, every kernel forced in turn), mean error 0.02 - 0.09.  The kernel chosen
 // is behind the fastest of all, on average and in one of twenty: 2 - 2048 rows 0.5 and 3.0 % (prepared), 0.5 and 1.8 % (raw); 600 - 9000 rows 1.0 and 5.7 %,
-// 1.1 and 7.1 %; products beyond 1.2e10 multiply-adds 0.2 and 1.0 %, 0.1 and 0 %; sizes of models 0.4 and 3.0 %, 0.7 and 5.3 %.  (With constants fitted to one set of
+// 1.0 and 6.8 %; products beyond 1.2e10 multiply-adds 0.2 and 1.0 %, 0.1 and 0 %; sizes of models 0.4 and 3.0 %, 0.7 and 4.6 %.  (With constants fitted to one set of
 // operands, which the L2s kept, small tiles without rounds and B's bytes alone: 1.5 and 9.9 %, 1.3 and 11 %; 1.7 and 10 %, 2.2 and 16 %; 0.5 and 2.6 %, 0.9 and 8.3 %;
 // 1.3 and 9.6 %, 1.5 and 11 %: 7296 x 1198 x 283 52.6 us, 43.0 with the constants above.)  The eight-wave tiles' errors are on the low side behind a full round
 // (7 %) and with more than 5 MB of A (10 %; rows off 16 bytes of 20 MB and more 25 %, where a copy of A is the alternative), which their estimates are
@@ -254,19 +254,19 @@ static const CallCost kCallCost[] = {
     {"t32x32x32_wavek_bf16x2_tri", 2.48, 0.877, 0.553, 0.589, 60, 1.29, 1.2, 0, 0.0976},
     {"t32x64x32_wavek_bf16x2_tri", 3.09, 1.09, 0.626, 1.69, 60, 1, 1.44, 0, 0.0651},
     {"t64x64x32_wavek_bf16x2_tri", 5.14, 1.28, 1.23, 2.43, 60, 1.23, 2.22, 0, 0.037},
-    {"k64x160x16_wk4_bf16x2_tri", 6.72, 0.592, 0.608, 5.22, 19.3, 2.07, 0.82, 5.46, 0.162},
-    {"bd64x128x64_d3_p4_bf16x2_tri", 4.37, 1.09, 0.917, 1.9, 16.7, 3.99, 1.09, 0.0779, 0.772},
-    {"bd96x128x64_d3_p4_bf16x2_tri", 5.76, 1.25, 1.03, 3.14, 6.56, 4.48, 1.28, 6.18, 1.47},
-    {"bd128x128x32_d3_p4_bf16x2_tri", 5.1, 1.49, 1.21, 3.11, 17, 2.76, 1.53, 6.22, 1.88},
-    {"bd192x128x64_d2_p4_bf16x2_tri", 7.67, 1.87, 1.47, 4.33, 5, 3.57, 2.05, 5.59, 3.17},
-    {"t64x64x64_w2x2x1_d3_bf16x2_tri", 4.88, 0.671, 0.104, 0.691, 60, 1, 0.7, 0, 0.618},
-    {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 6.45, 0.892, 0.615, 2.27, 22.4, 2.09, 0.892, 7.16, 4.2},
-    {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 8.12, 0.968, 1.11, 2.25, 11.9, 2.48, 1.24, 5.43, 4.48},
-    {"t256x128x32_w4x1x1_d2_bf16x2_tri", 9.38, 1.84, 2, 2.77, 7.14, 3.36, 2.32, 4.93, 11.1},
-    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 11.5, 2.09, 2.02, 0.699, 5, 2.59, 2.71, 4.86, 12.8},
-    {"t256x256x32_w512_edge_bf16x2_tri", 10.7, 2.93, 4.73, 9.7, 25.5, 3.7, 4.83, 0.105, 1.47},
-    {"t256x320x32_w512_edge_bf16x2_tri", 12.4, 3.48, 5.78, 13.7, 60, 3.27, 5.71, 0.0162, 1.61},
-    {"t256x320x32_w512_bf16x2_tri", 12.3, 3.45, 5.72, 13.6, 60, 3.27, 5.65, 0.016, 0},
+    {"k64x160x16_wk4_bf16x2_tri", 6.72, 0.598, 0.632, 5.15, 19.2, 2.19, 0.817, 5.44, 0.178},
+    {"bd64x128x64_d3_p4_bf16x2_tri", 4.36, 1.08, 0.735, 1.88, 15.8, 2.88, 1.1, 5.63, 0.77},
+    {"bd96x128x64_d3_p4_bf16x2_tri", 5.62, 1.23, 0.828, 3.35, 7.45, 2.89, 1.28, 6.21, 1.54},
+    {"bd128x128x32_d3_p4_bf16x2_tri", 5.03, 1.49, 1.22, 3.44, 60, 2.71, 1.53, 6.29, 1.88},
+    {"bd192x128x64_d2_p4_bf16x2_tri", 7.19, 1.87, 1.37, 4.95, 5, 3.33, 2.03, 5.64, 3.33},
+    {"t64x64x64_w2x2x1_d3_bf16x2_tri", 4.77, 0.691, 0.166, 0.732, 60, 1.21, 0.704, 0.0299, 0.612},
+    {"t64x160x64_w2x1x2_d2_p8_bf16x2_tri", 6.13, 0.882, 0.448, 2.91, 60, 1.56, 0.914, 7.15, 3.83},
+    {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 7.79, 0.949, 1.03, 3.05, 14.8, 2.11, 1.24, 5.44, 4.31},
+    {"t256x128x32_w4x1x1_d2_bf16x2_tri", 8.14, 1.84, 1.92, 4.28, 5.15, 3.21, 2.37, 4.76, 10.8},
+    {"t256x160x32_w4x1x1_d2_bf16x2_tri", 10.6, 2.12, 2.43, 5.46, 7.3, 3.16, 2.67, 4.77, 12.2},
+    {"t256x256x32_w512_edge_bf16x2_tri", 10.8, 2.93, 4.76, 9.03, 51.2, 3.72, 4.87, 0, 1.43},
+    {"t256x320x32_w512_edge_bf16x2_tri", 12.5, 3.48, 5.85, 13.5, 60, 3.47, 5.71, 0.153, 1.61},
+    {"t256x320x32_w512_bf16x2_tri", 12.4, 3.45, 5.79, 13.4, 60, 3.47, 5.65, 0.151, 0},
     // three fp16 terms (448 shapes; the tile chosen is 0.06 % behind the fastest of the three, without rounds 0.4 %, at most 26 %)
     {"t16x16x32_wavek_fp16x3_tri", 2.47, 0.728, 0.176, 0.125, 28.6, 1, 0.664, 0.051, 0},
     {"t16x32x32_wavek_fp16x3_tri", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
