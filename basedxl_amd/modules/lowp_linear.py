@@ -52,17 +52,18 @@ class BasedXLLowPLinear(nn.Module):
             return cascade_linear(x, self.weight, None if pw is None else pw.slots, self.bias, self.lowp, self.terms,
                                   self.products, False, self._weight_exp if pw is None else pw.exp)
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
-        pw, rows = self._prepared_weight, x.numel() // max(self.in_features, 1)
-        raw = not self.prepared or raw_is_faster(rows, self.in_features, self.out_features, x.dtype, self.lowp, self.terms, self.products)
-        if not raw and (pw is None or pw.device != self.weight.device):
-            y = None
-        elif self.lowp == "fp8" and raw:
+        pw, raw = self._prepared_weight, not self.prepared
+        if not raw and x.dtype == torch.float32:
+            raw = raw_is_faster(x.numel() // max(self.in_features, 1), self.in_features, self.out_features, x.dtype, self.lowp, self.terms, self.products)
+        if raw and self.lowp != "fp8":
+            y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
+        elif raw:
             y = None if self._weight_exp is None else _lib.short_cut().fp8(
                 x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
+        elif pw is None or pw.device != self.weight.device:
+            y = None
         elif self.lowp == "fp8":
             y = _lib.short_cut().fp8(x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
-        elif raw:
-            y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
         else:
             y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
         if y is not None:
