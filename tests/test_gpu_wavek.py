@@ -38,6 +38,33 @@ def test_every_number_of_steps_is_exact_on_integers(name, K):
         assert bool((out[M] == -77.0).all()) and bool((out[:, N] == -77.0).all())
 
 
+@pytest.mark.parametrize("name", _TILES)
+@pytest.mark.parametrize("side", ["A", "B"])
+def test_every_term_of_either_operand_reaches_the_result(name, side):
+    """The other operand picks one k for each row or column (one +-1, zeros): the result is the picked values with their signs, exact where
+    the terms hold all their bits.  Two bf16 terms hold integers below 2^16, three fp8 terms below 2^12, three fp16 terms 23 bits."""
+    bm, bn = (int(x) for x in name.split("_")[0][1:].split("x")[:2])
+    lowp, terms = name.split("_")[2].split("x")
+    bits, unit = {"bf16": (16, 1.0), "fp8": (12, 1.0), "fp16": (23, 2.0 ** -8)}[lowp]
+    g = torch.Generator().manual_seed(bits)
+    for M, K, N in ((7, 1304, 2 * bn + 1), (bm + 9, 264, bn), (2 * bm, 2568, bn + 8)):
+        rows, cols = (M, K) if side == "A" else (K, N)
+        values = torch.randint(-2 ** bits + 1, 2 ** bits, (rows, cols), generator=g).double() * unit
+        count = N if side == "A" else M
+        k, sign = torch.randint(0, K, (count,), generator=g), torch.randint(0, 2, (count,), generator=g) * 2.0 - 1
+        k[0], k[-1] = K - 1, 0
+        pick = torch.zeros(count, K, dtype=torch.double)
+        pick[torch.arange(count), k] = sign.double()
+        a, b = (values, pick.T.contiguous()) if side == "A" else (pick, values)
+        want = values[:, k] * sign if side == "A" else values[k] * sign[:, None]
+        w = b.float().to("cuda:0")
+        print("wavek terms", name, side, (M, K, N), flush=True)
+        options = {} if name.endswith("_bpre") else dict(lowp=lowp, terms=int(terms))
+        got = cascaded_lowp_matmul(a.float().to("cuda:0"), PreparedWeight(w, lowp=lowp, terms=int(terms)) if name.endswith("_bpre") else w,
+                                   variant=_lib.variant_names().index(name), **options)
+        assert torch.equal(got.cpu().double(), want), (M, K, N)
+
+
 @pytest.mark.parametrize("name", [n for n in _TILES if n.endswith("_bpre") and n.split("x")[1] == "64"])
 @pytest.mark.parametrize("M,K,N", [(7, 72, 64), (8, 1280, 128), (9, 264, 192), (17, 520, 320), (81, 2568, 704)])
 def test_the_gated_store(name, M, K, N):
