@@ -244,7 +244,8 @@ constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {128
 // operands, which the L2s kept, small tiles without rounds and B's bytes alone: 1.5 and 9.9 %, 1.3 and 11 %; 1.7 and 10 %, 2.2 and 16 %; 0.5 and 2.6 %, 0.9 and 8.3 %;
 // 1.3 and 9.6 %, 1.5 and 11 %: 7296 x 1198 x 283 52.6 us, 43.0 with the constants above.)  The eight-wave tiles' errors are on the low side behind a full round
 // (7 %) and with more than 5 MB of A (10 %; rows off 16 bytes of 20 MB and more 25 %, where a copy of A is the alternative), which their estimates are
-// raised by.
+// raised by.  Groups: the tiles of all their problems; there the eight-wave tiles are 5 - 8 % faster than that and the prepared 64 x 160 one 8 % slower (305 groups
+// of two and three, 0.6 and 0.8 % behind the fastest on average, 2.5 and 3.5 % in one of twenty).
 // The selection functions, which answer for shapes, keep the constants above but for KIND_WAVEK.
 struct CallCost { const char* name; double c0, s0, s1, c1, bw, x, r1, deep, edge; };
 static const CallCost kCallCost[] = {
@@ -342,20 +343,22 @@ static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Pr
   const double lone = k * t.s0 + (small && k > few ? t.deep * (k - few) : 0.0), shared = fill * k * t.s1 + mb / t.bw;
   const double us = t.c0 + full * (t.c1 + k * t.r1) + std::pow(std::pow(lone, t.x) + std::pow(shared, t.x), 1.0 / t.x);
   if (small) {
-    const double late = v.kind != KIND_WAVEK || !q.call || q.glu ? 1.0 : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
+    const double late = v.kind != KIND_WAVEK || !q.call || q.glu ? 1.0
+                        : count > 1 ? (v.BM * v.BN == 4096 ? 0.92 : 0.95)
+                        : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
     return late * (q.N % v.BN != 0 ? us * (1.0 + t.edge) : us);
   }
   const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * (full + 1.0) : us;
   const double power = t.deep * tiles * v.BM * v.BN * (double)k_per * 1.0e-9;
-  return std::pow(std::pow(edged, 8.0) + std::pow(power, 8.0), 0.125);
+  return std::pow(std::pow(edged, 8.0) + std::pow(power, 8.0), 0.125) * (count > 1 && q.bpre && v.BM == 64 && v.BN == 160 ? 1.08 : 1.0);
 }
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&
          !q.glu && q.K > 0 && !beyond_i32(q.M, q.lda, 4);
 }
-// a call whose kernels all have such constants (plain groups too: the tiles of all problems, 0.99 of the time with the constants above over 400 groups of three)
-static bool costed_call(const Problem& q, int count) {
-  return q.call && (count == 1 || !q.glu) && q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && (!q.glu || q.bpre);
+// a call whose kernels all have such constants
+static bool costed_call(const Problem& q) {
+  return q.call && q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && (!q.glu || q.bpre);
 }
 static double wavek_estimate_us(const Problem& q, int count) {
   double best = 1e9;
@@ -503,7 +506,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
       if (table()[i].kind == KIND_SLOTK && variant_matches(table()[i], q, FIT_DWORD) && variant_cost(i, q, count, ws_bytes) < skinny_us) return 1e9;
     return 1e-6 * (double)(((q.M + v.BM - 1) / v.BM) * v.BM) + 1e-8 * v.BM;
   }
-  const bool costed = costed_call(q, count);
+  const bool costed = costed_call(q);
   const CallCost* c = costed && q.glu ? info.gated : !q.call && info.shape ? info.shape : info.call;
   if (costed && !c && v.fast) return 1e9;   // (nowhere the fastest)
   if (c && (costed || v.kind == KIND_WAVEK)) {
@@ -702,7 +705,20 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
       if (splits_out) *splits_out = 1;
     }
   }
+  // A group in one launch has fewer kernels to choose from than its problems one behind the other (the large tiles on prepared weights with K off 32, K over
+  // four waves): 3 x (2592 x 552 x 3840) prepared 240 us in one launch, 121 in three.  From 10 us a problem on: an eager launch is 3 us of the
+  // host's time.  (No kernel: the launch then takes the problems one by one.)
+  if (best >= 0 && count > 1 && costed_call(q)) {
+    const int one = select_variant_uncached(q, fit, 1, ws_bytes, nullptr);
+    const double us = one < 0 ? 1e9 : variant_cost(one, q, 1, ws_bytes);
+    if (us >= 10.0 && 1.03 * count * us < best_cost) return CASCMM_ERR_BAD_FORMAT;
+  }
   return best < 0 ? (int)CASCMM_ERR_BAD_FORMAT : best;
+}
+// what such a call is expected to take
+static double call_cost_us(const Problem& q, RowFit fit, int count) {
+  const int v = select_variant(q, fit, count), one = v < 0 && count > 1 ? select_variant(q, fit, 1) : -1;
+  return v >= 0 ? variant_cost(v, q, count) : one >= 0 ? count * variant_cost(one, q, 1) : 1e9;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -918,9 +934,9 @@ static Relay relay_of(const Problem& q0, int count, const void* const* A, const 
     RowFit fit = FIT_FAST;
     for (int i = 0; i < count; ++i) fit = std::min(fit, row_fit(q, A ? A[i] : nullptr, B ? B[i] : nullptr));
     const Problem e = relayed(q, r);
-    const int direct = select_variant(q, fit, count), copied = select_variant(e, row_fit(e, nullptr, nullptr), count);
+    const int direct = select_variant(q, fit, count);
     if (direct >= 0 && table()[direct].kind == KIND_WAVEK &&
-        (copied < 0 || variant_cost(direct, q, count) < variant_cost(copied, e, count) + 3.5 + (double)a_bytes * 2.0 / 4.0e6))
+        variant_cost(direct, q, count) < call_cost_us(e, row_fit(e, nullptr, nullptr), count) + 3.5 + (double)a_bytes * 2.0 / 4.0e6)
       return Relay();
   }
   // (a copied B is a prepared one, which the bounds-checked kernels do not take: without a kernel for what is left, rows of A

@@ -94,3 +94,18 @@ def test_ragged_rows_of_a_wide_layer_take_the_large_tile():
     assert pick(1976, 1280, 10240) == "t256x320x32_w512_edge_bf16x2_tri" and pick(4096, 4096, 4096) == "t256x256x32_w512_edge_bf16x2_tri"
     assert pick(8192, 328, 2560) == "t256x320x32_w512_edge_bf16x2_tri" and "w512" not in pick(2496, 2504, 2500)
     assert pick(2048, 1280, 10240) == "t256x320x32_w512_bf16x2_tri" and "w512" not in pick(2048, 2048, 2048)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(1330, 1768, 1856), (1775, 2408, 1088)])
+def test_a_group_runs_problem_by_problem_where_that_is_faster(M, K, N):
+    """K off 32: one launch has the eight-wave tiles only (138 and 155 us for three), three launches the kernels of single calls (89 and
+    104), whose bits the results have."""
+    from basedxl_amd import PreparedWeight, cascaded_lowp_matmul, cascaded_lowp_matmul_prepared
+    g = torch.Generator(device="cuda:0").manual_seed(N)
+    a = [torch.randn(M, K, device="cuda:0", generator=g) for _ in range(3)]
+    w = [PreparedWeight(torch.randn(K, N, device="cuda:0", generator=g) * 0.02) for _ in range(3)]
+    bias = [torch.randn(N, device="cuda:0", generator=g) for _ in range(3)]
+    print("group", (M, K, N), flush=True)
+    for got, x, p, b in zip(cascaded_lowp_matmul_prepared(a, w, biases=bias), a, w, bias):
+        assert torch.equal(got, cascaded_lowp_matmul(x, p, bias=b))
