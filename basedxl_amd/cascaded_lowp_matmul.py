@@ -328,8 +328,8 @@ def raw_is_faster(rows: int, K: int, N: int, dtype: torch.dtype, lowp: str, term
 
 
 def cascaded_lowp_matmul_prepared(a_list, w_list, *, outs=None, biases=None, products: str = "tri", variant: int = -1):
-    """``a_list[i]`` ([..., K] fp32) times the prepared weight ``w_list[i]`` in ONE launch (1..8
-    problems of one shape and one cascade); returns the list of results."""
+    """``a_list[i]`` ([..., K] fp32) times the prepared weight ``w_list[i]``, in one launch unless their own kernels
+    are expected to be faster (1..8 problems of one shape and one cascade); returns the list of results."""
     import ctypes
 
     n = len(a_list)
@@ -454,7 +454,7 @@ def _gemm_2d(a2: torch.Tensor, b2: torch.Tensor, out2: torch.Tensor, bias: Optio
 def cascaded_lowp_matmul_grouped(a_list, b_list, *, outs=None, biases=None, lowp: Optional[str] = None,
                                  terms: Optional[int] = None,
                                  products: str = "tri", variant: int = -1, b_exps=None):
-    """Several independent cascade GEMMs of one shape in ONE kernel launch.
+    """Several independent cascade GEMMs of one shape in one kernel launch (unless their own kernels are expected to be faster).
 
     ``a_list[i]`` ([..., K], the same tensor may appear several times) times ``b_list[i]``
     ([K, N], contiguous) -> ``outs[i]``.  This is what the reference gets for to_k / to_v by

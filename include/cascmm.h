@@ -121,7 +121,8 @@ int cascmm_gemm_noalloc(const void* A, const void* B, void* C, const void* bias,
                         int dtype, int fmt, int terms, int products,
                         const int32_t* tensor_exps, void* stream);
 
-/* `count` (1..8) independent GEMMs of one shape, layout and cascade in ONE launch: problem i
+/* `count` (1..8) independent GEMMs of one shape, layout and cascade in ONE launch (or one behind the other, where
+ * no kernel takes them together or their own kernels are expected to be faster): problem i
  * computes C[i] = A[i] . B[i] (+ bias[i]); A, B, C, bias are HOST arrays of device pointers
  * (bias may be NULL, or hold NULL entries).  Pointers may repeat (the same activations times
  * several weights).  The kernels are persistent, so the launch gap and the cold first loads of
