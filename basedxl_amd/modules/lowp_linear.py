@@ -53,19 +53,25 @@ class BasedXLLowPLinear(nn.Module):
                                   self.products, False, self._weight_exp if pw is None else pw.exp)
         # the ordinary eager call in one native function; None: whatever is not ordinary about it is decided below
         pw, raw = self._prepared_weight, not self.prepared
-        if not raw and x.dtype == torch.float32:
-            raw = raw_is_faster(x.numel() // max(self.in_features, 1), self.in_features, self.out_features, x.dtype, self.lowp, self.terms, self.products)
-        if raw and self.lowp != "fp8":
+        if not raw and pw is not None and (pw.dt or not (pw.fmt or pw.terms != 2 or pw.K & 7 or self.products != "tri")):
+            # (a 16-bit weight or two bf16 terms: never the raw weight, the rule need not be asked)
+            y = None if pw.device != self.weight.device else _lib.short_cut().prepared(
+                x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
+        elif raw and self.lowp != "fp8":
             y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
-        elif raw:
-            y = None if self._weight_exp is None else _lib.short_cut().fp8(
-                x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
-        elif pw is None or pw.device != self.weight.device:
-            y = None
-        elif self.lowp == "fp8":
-            y = _lib.short_cut().fp8(x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
         else:
-            y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
+            raw = raw or raw_is_faster(x.numel() // max(self.in_features, 1), self.in_features, self.out_features, x.dtype, self.lowp, self.terms, self.products)
+            if raw and self.lowp != "fp8":
+                y = _lib.short_cut().matmul(x, self.weight, self.bias, self.lowp, self.terms, self.products)
+            elif raw:
+                y = None if self._weight_exp is None else _lib.short_cut().fp8(
+                    x, self.weight, self.bias, self._weight_exp, 0, 0, self.terms, self.products, False)
+            elif pw is None or pw.device != self.weight.device:
+                y = None
+            elif self.lowp == "fp8":
+                y = _lib.short_cut().fp8(x, pw.slots, self.bias, pw.exp, pw.K, pw.N, pw.terms, self.products, True)
+            else:
+                y = _lib.short_cut().prepared(x, pw.slots, self.bias, pw.K, pw.N, pw.fmt, pw.terms, self.products, pw.dt, False, 0)
         if y is not None:
             return y
         if self.prepared and x.is_cuda:
