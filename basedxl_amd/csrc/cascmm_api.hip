@@ -242,7 +242,7 @@ constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {128
 // is behind the fastest of all, on average and in one of twenty: 2 - 2048 rows 0.5 and 3.0 % (prepared), 0.5 and 1.8 % (raw); 600 - 9000 rows 1.0 and 5.7 %,
 // 1.0 and 6.8 %; products beyond 1.2e10 multiply-adds 0.2 and 1.0 %, 0.1 and 0 %; sizes of models 0.4 and 3.0 %, 0.7 and 4.6 %.  (With constants fitted to one set of
 // operands, which the L2s kept, small tiles without rounds and B's bytes alone: 1.5 and 9.9 %, 1.3 and 11 %; 1.7 and 10 %, 2.2 and 16 %; 0.5 and 2.6 %, 0.9 and 8.3 %;
-// 1.3 and 9.6 %, 1.5 and 11 %: 7296 x 1198 x 283 52.6 us, 43.0 with the constants above.)  The eight-wave tiles' errors are on the low side behind a full round
+// 1.3 and 9.6 %, 1.5 and 11 %: 7296 x 1198 x 283 54.7 us, 43.9 with these.)  The eight-wave tiles' errors are on the low side behind a full round
 // (7 %) and with more than 5 MB of A (10 %; rows off 16 bytes of 20 MB and more 25 %, where a copy of A is the alternative), which their estimates are
 // raised by.  Groups: the tiles of all their problems; there the eight-wave tiles are 5 - 8 % faster than that and the prepared 64 x 160 one 8 % slower (305 groups
 // of two and three, 0.6 and 0.8 % behind the fastest on average, 2.5 and 3.5 % in one of twenty).
@@ -706,7 +706,7 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
     }
   }
   // A group in one launch has fewer kernels to choose from than its problems one behind the other (the large tiles on prepared weights with K off 32, K over
-  // four waves): 3 x (2592 x 552 x 3840) prepared 240 us in one launch, 121 in three.  From 10 us a problem on: an eager launch is 3 us of the
+  // four waves): 3 x (2592 x 552 x 3840) prepared 238 us in one launch, 126 in three.  From 10 us a problem on: an eager launch is 3 us of the
   // host's time.  (No kernel: the launch then takes the problems one by one.)
   if (best >= 0 && count > 1 && costed_call(q)) {
     const int one = select_variant_uncached(q, fit, 1, ws_bytes, nullptr);
