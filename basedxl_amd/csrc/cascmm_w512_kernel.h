@@ -40,11 +40,11 @@ struct W512Tile {
   static constexpr int NTL = NTL_;                  // column blocks of a wave
   static constexpr int BM = 256, BN = 64 * NTL, BK = 16, NS = 4, NT = 256;
   static constexpr int WTM = 128, WTN = 32 * NTL, MT = 4;
-  static constexpr int A_STAGE = BM * BK * 4;       // raw fp32: 64 bytes per row
+  static constexpr int A_PAIR = BM * 2 * BK * 4;    // raw fp32, two stages: 128 bytes per row
   static constexpr int B_STAGE = BK * BN * 4;       // raw fp32
-  static constexpr int STAGE = A_STAGE + B_STAGE;   // 36 KB (NTL = 4: 32 KB)
-  static constexpr int LDS_BYTES = NS * STAGE;      // 144 KB (128 KB)
-  static constexpr int LOADS = 4 + NTL;             // direct loads per wave and stage: 4 of A, NTL of B
+  static constexpr int B_AREA = 2 * A_PAIR;         // two pairs of A, then NS stages of B
+  static constexpr int LDS_BYTES = B_AREA + NS * B_STAGE;   // 144 KB (NTL = 4: 128 KB)
+  static constexpr int A_LOADS = 8;                 // direct loads per wave: a pair of A; a stage of B has NTL
 };
 typedef W512Tile<5> W512;
 constexpr int W512_EDGE_ROWS = 64;   // EDGE: the fewest rows
@@ -130,17 +130,16 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   // (one record fewer than A's: with equal words the compiler keeps one copy of them and rebuilds this descriptor from it
   // in front of every B load)
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.B[0], 0, EDGE && !BPRE ? (int)((((int64_t)p.K - 1) * p.ldb + p.N) * 4) : 0x7FFFFFFE, 0x00020000);
-  // per wave and stage: 4 loads of A (16 rows x 64 bytes each; LDS position 4 row + pos holds chunk
-  // (pos - row / 4) mod 4 of the row) and NTL loads of B (256 consecutive floats of the stage's
+  // per wave: 8 loads of A for two stages (8 rows x 128 bytes each; LDS position 8 row + pos holds chunk
+  // (pos - row / 2) mod 8 of the row) and NTL loads of B for every stage (256 consecutive floats of the stage's
   // [16][BN] area)
-  const int a_chunk = ((lane & 3) - (lane >> 4)) & 3;   // (the same for every load: its first row is a multiple of 16)
-  int a_voff[4], b_voff[T::NTL];
+  const int a_chunk = ((lane & 7) - (lane >> 4)) & 7;   // of the even loads (their first row is a multiple of 16); the odd ones': ^ 4
+  int a_voff[T::A_LOADS], b_voff[T::NTL];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int inst = wave * 4 + j;
-    const int row = inst * 16 + (lane >> 2);
+  for (int j = 0; j < T::A_LOADS; ++j) {
+    const int row = (wave * T::A_LOADS + j) * 8 + (lane >> 3);
     const int arow = EDGE && m0 + row >= p.M ? p.M - 1 : m0 + row;
-    a_voff[j] = (int)(((int64_t)arow * p.lda + a_chunk * 4) * 4);
+    a_voff[j] = (int)(((int64_t)arow * p.lda + (a_chunk ^ 4 * (j & 1)) * 4) * 4) - (j & 3) * 1024;
   }
 #pragma unroll
   for (int j = 0; j < T::NTL; ++j) {
@@ -168,48 +167,49 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   // The loads of a wave land in consecutive kilobytes of LDS: the LDS address is M0 plus the instruction's immediate
   // offset, so a wave's A loads of a stage share one M0 and differ in the immediate; the immediate moves the memory
   // address too, which the lane offsets make up for (they stay non-negative: load j starts at least j KB into its
-  // operand, at an edge as well: 64 rows of 32 k and BN columns are more than 3 KB).  The fifth B load is 4 KB further, beyond the immediate's range, and takes an M0 of its own.
+  // operand, at an edge as well: 64 rows of 32 k and BN columns are more than 3 KB).  The second four of A and the fifth of B are
+  // 4 KB further, beyond the immediate's range, and take an M0 of their own.
 #pragma unroll
-  for (int j = 1; j < 4; ++j) {
-    a_voff[j] -= j * 1024;
-    b_voff[j] -= j * 1024;
-  }
-  auto issue1 = [&](int step_, int j) {
-    const int step = step_ < ksteps - 1 ? step_ : ksteps - 1;
-    const int st = step_ % T::NS;
-    const w512_lds_ptr al = (w512_lds_ptr)(smem + st * T::STAGE + wave * 4096);
-    const w512_lds_ptr bl = (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * (T::NTL * 1024));
-    const int as = step * T::BK * 4, bs = step * b_step;
+  for (int j = 1; j < 4; ++j) b_voff[j] -= j * 1024;
+  // load j of the pair of stages that starts with stage `first` (even)
+  auto issue_a = [&](int first, int j) {
+    const int step = first < ksteps - 2 ? first : ksteps - 2;
+    const w512_lds_ptr al = (w512_lds_ptr)(smem + (first & 2) * (T::A_PAIR / 2) + wave * (T::A_LOADS * 1024) + (j >> 2) * 4096);
+    const int as = step * T::BK * 4;
     // EDGE: chunks past K come from beyond the buffer, as zeros (B's rows past K do by themselves: its buffer ends there, or
     // its slots hold zeros)
-    auto av = [&](int jj) { return EDGE && a_chunk * 4 >= p.K - step * T::BK ? 0x7FFFFFFF : a_voff[jj]; };
+    const int av = EDGE && (a_chunk ^ 4 * (j & 1)) * 4 >= p.K - step * T::BK ? 0x7FFFFFFF : a_voff[j];
+    switch (j & 3) {
+      case 0: w512_load0(ra, al, av, as); break;
+      case 1: w512_load1(ra, al, av, as); break;
+      case 2: w512_load2(ra, al, av, as); break;
+      default: w512_load3(ra, al, av, as); break;
+    }
+  };
+  auto issue_b = [&](int step_, int j) {
+    const int step = step_ < ksteps - 1 ? step_ : ksteps - 1;
+    const w512_lds_ptr bl = (w512_lds_ptr)(smem + T::B_AREA + step_ % T::NS * T::B_STAGE + wave * (T::NTL * 1024) + (j >> 2) * 4096);
+    const int bs = step * b_step;
     switch (j) {
-      case 0: w512_load0(ra, al, av(0), as); break;
-      case 1: w512_load1(ra, al, av(1), as); break;
-      case 2: w512_load2(ra, al, av(2), as); break;
-      case 3: w512_load3(ra, al, av(3), as); break;
-      case 4: w512_load0(rb, bl, b_voff[0], bs); break;
-      case 5: w512_load1(rb, bl, b_voff[1], bs); break;
-      case 6: w512_load2(rb, bl, b_voff[2], bs); break;
-      case 7: w512_load3(rb, bl, b_voff[3], bs); break;
-      default:
-        if constexpr (T::NTL == 5) w512_load0(rb, (w512_lds_ptr)(smem + st * T::STAGE + T::A_STAGE + wave * 5120 + 4096), b_voff[4], bs);
-        break;
+      case 1: w512_load1(rb, bl, b_voff[1], bs); break;
+      case 2: w512_load2(rb, bl, b_voff[2], bs); break;
+      case 3: w512_load3(rb, bl, b_voff[3], bs); break;
+      default: w512_load0(rb, bl, b_voff[j], bs); break;
     }
   };
 
-  // fragment addresses (bytes inside a stage)
-  const int a_row = wm0 + l31;                          // + mi * 32 rows = mi * 2048 bytes (same rotation: 32 / 4 = 8)
-  const int a_frag0 = a_row * 64 + ((2 * g + (a_row >> 2)) & 3) * 16;
-  const int a_frag1 = a_row * 64 + ((2 * g + 1 + (a_row >> 2)) & 3) * 16;
+  // fragment addresses: of A inside a pair, the second stage's chunks are four further (^ 64 bytes); of B inside a stage
+  const int a_row = wm0 + l31;                          // + mi * 32 rows = mi * 4096 bytes (same rotation: 32 / 2 = 2 x 8)
+  const int a_frag0 = a_row * 128 + ((2 * g + (a_row >> 1)) & 7) * 16;
+  const int a_frag1 = a_row * 128 + ((2 * g + 1 + (a_row >> 1)) & 7) * 16;
   int b_frag[T::NTL];
 #pragma unroll
   for (int ni = 0; ni < T::NTL; ++ni) {
     int pos = wn0 + ni * 32 + l31 + 32 * g;
     pos = pos >= T::BN ? pos - T::BN : pos;
-    b_frag[ni] = T::A_STAGE + (8 * g * T::BN + pos) * 4;   // + e * BN * 4
+    b_frag[ni] = (8 * g * T::BN + pos) * 4;   // + e * BN * 4
     // prepared: slot (term 0, k group g, column) -- term 1 is 2 * BN slots further
-    if (BPRE) b_frag[ni] = T::A_STAGE + (g * T::BN + wn0 + ni * 32 + l31) * 16;
+    if (BPRE) b_frag[ni] = (g * T::BN + wn0 + ni * 32 + l31) * 16;
   }
 
   f32x16 acc[T::MT][T::NTL];
@@ -246,10 +246,15 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
     lo[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
   };
 
+  // in the order in which the loop waits for them: pair 0 of A, stages 0 and 1 of B, pair 1, stage 2
 #pragma unroll
-  for (int s = 0; s < T::NS - 1; ++s)
+  for (int j = 0; j < T::A_LOADS; ++j) issue_a(0, j);
 #pragma unroll
-    for (int j = 0; j < T::LOADS; ++j) issue1(s, j);
+  for (int j = 0; j < 2 * T::NTL; ++j) issue_b(j / T::NTL, j % T::NTL);
+#pragma unroll
+  for (int j = 0; j < T::A_LOADS; ++j) issue_a(2, j);
+#pragma unroll
+  for (int j = 0; j < T::NTL; ++j) issue_b(2, j);
   // the accumulators are cleared while the first loads are in flight: not before them, which would hold
   // the loads back, and not after the barrier, where the first MFMA would wait for it
   W512_FENCE();
@@ -269,12 +274,14 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
       else w512_in_vec(acc[mi][ni]);
     }
   W512_FENCE();
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * T::LOADS & 0xF) | ((2 * T::LOADS >> 4) << 14));   // vmcnt(2 stages): stage 0 has landed
+  constexpr int W0 = T::A_LOADS + 2 * T::NTL, WEVEN = T::A_LOADS + T::NTL, WODD = T::NTL;
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (W0 & 0xF) | ((W0 >> 4) << 14));   // pair 0 and stage 0 have landed
   __builtin_amdgcn_s_barrier();
   {
+    const unsigned char* b0 = smem + T::B_AREA;
 #pragma unroll
     for (int mi = 0; mi < T::MT; ++mi) {
-      const f32x4 x0 = *(const f32x4*)(smem + a_frag0 + mi * 2048), x1 = *(const f32x4*)(smem + a_frag1 + mi * 2048);
+      const f32x4 x0 = *(const f32x4*)(smem + a_frag0 + mi * 4096), x1 = *(const f32x4*)(smem + a_frag1 + mi * 4096);
       float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -283,11 +290,11 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
       }
     }
     if (BPRE) {
-      read_slot_hi(0, smem, 0);
-      read_slot_lo(0, smem, 0);
+      read_slot_hi(0, b0, 0);
+      read_slot_lo(0, b0, 0);
     } else {
-      read_raw(R[0], smem, 0, 0, 8);
-      read_raw(R[1], smem, 1, 0, 8);
+      read_raw(R[0], b0, 0, 0, 8);
+      read_raw(R[1], b0, 1, 0, 8);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         split_1(R[0], H[0], e);
@@ -299,11 +306,14 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   for (int s = 0; s < ksteps; s += 2) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      // top of stage s + j: the own loads of stage s + j + 1 have landed, then everybody's
-      __builtin_amdgcn_s_waitcnt(0x0F70 | T::LOADS);                     // vmcnt(one stage)
+      // top of stage s + j: the own loads of stage s + j + 1 have landed, then everybody's.  In flight: what the stage before
+      // issued, which is a stage of B (odd stages: and before it the pair of A that is read two stages later)
+      if (j == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (WEVEN & 0xF) | ((WEVEN >> 4) << 14));
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | WODD);
       __builtin_amdgcn_s_barrier();
-      const unsigned char* st0 = smem + ((s + j) % T::NS) * T::STAGE;       // this stage
-      const unsigned char* st1 = smem + ((s + j + 1) % T::NS) * T::STAGE;   // the next one
+      const unsigned char* st0 = smem + T::B_AREA + ((s + j) % T::NS) * T::B_STAGE;       // this stage of B
+      const unsigned char* st1 = smem + T::B_AREA + ((s + j + 1) % T::NS) * T::B_STAGE;   // the next one
+      const unsigned char* an = smem + ((s + 2 * j) & 2) * (T::A_PAIR / 2);               // the pair of A that the next stage lies in
 #pragma unroll
       for (int ni = 0; ni < T::NTL; ++ni) {
         const int t = j * T::NTL + ni;        // block number inside the trip: its parity is static
@@ -328,9 +338,14 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
             else w512_mfma_v(a, b, acc[mi][ni]);
           }
         };
-        auto dl = [&](int k) {   // two load slots per block: 2 NTL per stage, of which 4 + NTL are used
-          const int slot = ni * 2 + k;
-          if (slot < T::LOADS) issue1(s + j + T::NS - 1, slot);
+        // loads of a stage: NTL of B, one behind each block; the odd stages' blocks have two more slots, for the pair of A whose
+        // buffer the even stage has read last
+        auto dl = [&](int k) {
+          if (k == 1 && j == 0) issue_b(s + T::NS - 1, ni);
+          if (j == 0) return;
+          const int slot = ni * 3 + k;
+          if (slot < T::A_LOADS) issue_a(s + 4, slot);
+          else if (slot < T::A_LOADS + T::NTL) issue_b(s + 1 + T::NS - 1, slot - T::A_LOADS);
         };
         // What goes between MFMA g and MFMA g + 1 of the block.  A wave alone on its SIMD issues one instruction
         // every four cycles or so, whatever its kind, and an MFMA holds the matrix pipe for 32: more than six
@@ -345,7 +360,8 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
           if (gi == 0) { __builtin_amdgcn_s_waitcnt(0xC07F); W512_FENCE(); }                          // lgkmcnt(0)
           if (gi == 4 && ni < 4) { __builtin_amdgcn_s_waitcnt(BPRE ? 0xC07F : 0xC47F); W512_FENCE(); }   // lgkmcnt(0) / lgkmcnt(4)
           if (gi == 0 && ni < 4) {   // row block ni of the next stage
-            const f32x4 x0 = *(const f32x4*)(st1 + a_frag0 + ni * 2048), x1 = *(const f32x4*)(st1 + a_frag1 + ni * 2048);
+            const int half = j == 0 ? 64 : 0;
+            const f32x4 x0 = *(const f32x4*)(an + (a_frag0 ^ half) + ni * 4096), x1 = *(const f32x4*)(an + (a_frag1 ^ half) + ni * 4096);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               RA[e] = x0[e];
@@ -367,8 +383,9 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
           if (BPRE && gi == 8) read_slot_lo(nxt, stn, n1);
           // the stage's loads: two per block, apart from each other and in gaps that hold one half-split
           // (several loads in neighbouring gaps of one block cost 30 cycles each: counted)
-          if (gi == 9) dl(0);
-          if (gi == 10) dl(1);
+          if (gi == 3) dl(0);
+          if (gi == 9) dl(1);
+          if (gi == 11) dl(2);
         };
 #pragma unroll
         for (int gi = 0; gi < 12; ++gi) {
