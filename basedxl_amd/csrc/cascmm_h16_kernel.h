@@ -34,18 +34,25 @@ template <int WM_, int WN_, int WK_, int MT_, int NTL_, int BK_, int NS_>
 struct H16 {
   static constexpr int WM = WM_, WN = WN_, WK = WK_, MT = MT_, NTL = NTL_, BK = BK_, NS = NS_, NT = 256;
   static constexpr int WTM = 32 * MT, WTN = 32 * NTL, BM = WM * WTM, BN = WN * WTN;
-  static constexpr int KG = BK / 8;                  // 16-byte chunks of a row of A (slot rows of B) per stage
+  // 32-k stages take half a 128-byte line of a row of A: its rows are loaded for two stages at once
+  static constexpr bool PAIR = BK == 32;
+  static constexpr int AK = PAIR ? 2 * BK : BK;      // k of a row of A that are loaded together
+  static constexpr int KG = AK / 8;                  // 16-byte chunks of that
   static constexpr int SLW = BK / 16 / WK;           // 16-k slices of a stage that a wave multiplies
-  static constexpr int A_STAGE = BM * BK * 2, B_STAGE = BN * BK * 2, STAGE = A_STAGE + B_STAGE;
-  static constexpr int A_LOADS = A_STAGE / 4096, B_LOADS = B_STAGE / 4096, LOADS = A_LOADS + B_LOADS;   // per wave and stage
+  static constexpr int A_BUF = BM * AK * 2, B_STAGE = BN * BK * 2;
+  static constexpr int A_STEP = PAIR ? 0 : A_BUF + B_STAGE, B_STEP = PAIR ? B_STAGE : A_STEP;   // from one stage's LDS to the next one's
+  static constexpr int B_AREA = PAIR ? 2 * A_BUF : A_BUF;   // (pairs: two of A, then the stages of B)
+  static constexpr int A_LOADS = A_BUF / 4096, B_LOADS = B_STAGE / 4096, LOADS = A_LOADS + B_LOADS;   // per wave: A (pairs: of two stages), B of a stage
   static constexpr int OUT_ROW = WTN * 2 + 16;       // bytes of a row of C in the store's LDS area (padded: banks)
   static constexpr int SUM_WAVE = WK == 2 ? (NTL + 1) / 2 * 4096 : 0;   // the other wave group's sums of this wave's blocks
   static constexpr int OUT_WAVE = 32 * OUT_ROW + WTN * 4 > SUM_WAVE ? 32 * OUT_ROW + WTN * 4 : SUM_WAVE;
-  static constexpr int LDS_BYTES = NS * STAGE > 4 * OUT_WAVE ? NS * STAGE : 4 * OUT_WAVE;
+  static constexpr int RING_BYTES = PAIR ? B_AREA + NS * B_STAGE : NS * B_STEP;
+  static constexpr int LDS_BYTES = RING_BYTES > 4 * OUT_WAVE ? RING_BYTES : 4 * OUT_WAVE;
   // tile rows an XCD walks down before moving one tile to the right: about square in bytes
   static constexpr int GROUP_M = BN >= 2 * BM ? 8 : 4;
   static_assert(WM * WN * WK == 4 && (BK == 32 || BK == 64) && SLW % 2 == 0 && NS >= 3, "layout");
-  static_assert(A_STAGE % 4096 == 0 && B_STAGE % 4096 == 0, "every wave issues the same number of loads");
+  static_assert(!PAIR || (WK == 1 && NS >= 4 && A_LOADS % 2 == 0), "pairs");
+  static_assert(A_BUF % 4096 == 0 && B_STAGE % 4096 == 0, "every wave issues the same number of loads");
   static_assert((NS - 1) * LOADS <= 63, "the wait counter has six bits");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 };
@@ -107,7 +114,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   const int m0 = tm * T::BM, n0 = tn * T::BN;
   const int k0 = split * k_per;
   const int K = K_all - k0 < k_per ? K_all - k0 : k_per;
-  const int ksteps = (K + T::BK - 1) / T::BK;
+  const int ksteps = T::PAIR ? (K + 63) / 64 * 2 : (K + T::BK - 1) / T::BK;
 
   // A's buffer starts with the tile's first row, so A itself may be of any size: the offsets inside a tile stay below
   // 512 rows.  Rows past M read as zero (it ends with row M - 1), and so does everything past B's last row or slot row
@@ -120,14 +127,15 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)B + b_first), 0, (int)b_bytes, 0x00020000);
 
   // ---- loads: this wave's kilobytes of a stage ----
-  // A: row r of the stage's BM x BK block at r * 2 BK bytes; position pos of a row holds chunk (pos - rot(r)) mod KG,
-  // rot = r / 2 (BK = 64) or r / 4 (BK = 32): the sixteen lanes a 16-byte LDS read serves together hit every bank once
-  constexpr int RSH = T::KG == 8 ? 1 : 2;
-  int a_voff[T::A_LOADS], a_k[T::A_LOADS];
+  // A: row r of the BM x 64 block at r * 128 bytes; position pos of a row holds chunk (pos - r / 2) mod 8: the sixteen
+  // lanes a 16-byte LDS read serves together hit every bank once
+  static_assert(T::KG == 8, "rotation");
+  constexpr int RSH = 1;
+  int a_voff[T::A_LOADS], a_k[T::A_LOADS];   // (a_k: pairs have two values only, even and odd loads)
 #pragma unroll
   for (int j = 0; j < T::A_LOADS; ++j) {
     const int row = (wave * T::A_LOADS + j) * (64 / T::KG) + lane / T::KG;
-    const int chunk = (lane % T::KG - (row >> RSH)) & (T::KG - 1);
+    const int chunk = (lane % T::KG - (row >> RSH)) & (T::KG - 1);   // (rows / 2 mod 8: load j's lanes as load j + 2's)
     a_k[j] = chunk * 8;
     a_voff[j] = row < rows ? (row * lda + chunk * 8) * 2 : 0x7FFFFFFF;
   }
@@ -143,26 +151,33 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     if (RAWB) b_voff[j] = (int)(((int64_t)(s / CPR) * p.ldb + n0 + ((s % CPR) ^ xor_of(s / CPR)) * 8) * 2);
     else b_voff[j] = ((s / T::BN) * p.N + n0 + s % T::BN) * 16;
   }
-  const int b_step = RAWB ? (int)(T::BK * p.ldb * 2) : T::KG * p.N * 16;
-  auto issue = [&](int step, int buf, int j) {
-    unsigned char* st = smem + buf * T::STAGE;
-    if (j < T::A_LOADS) {
-      // (past K: beyond the buffer's end, zeros)
-      const int v = a_k[j] < K - step * T::BK ? a_voff[j] : 0x7FFFFFFF;
-      h16_load_lds(ra, st + (wave * T::A_LOADS + j) * 1024, v, step * T::BK * 2);
-    } else {
-      const int bs = (step < ksteps ? step : ksteps) * b_step;
-      h16_load_lds(rb, st + T::A_STAGE + (wave * T::B_LOADS + j - T::A_LOADS) * 1024, b_voff[j - T::A_LOADS], bs);
-    }
+  const int b_step = RAWB ? (int)(T::BK * p.ldb * 2) : T::BK / 8 * p.N * 16;
+  // load j of A's rows from stage `step` on (pairs: an even one)
+  auto issue_a = [&](int step, int buf, int j) {
+    // (past K: beyond the buffer's end, zeros)
+    const int v = a_k[T::PAIR ? j & 1 : j] < K - step * T::BK ? a_voff[j] : 0x7FFFFFFF;
+    h16_load_lds(ra, smem + (T::PAIR ? (step & 2) * (T::A_BUF / 2) : buf * T::A_STEP) + (wave * T::A_LOADS + j) * 1024, v, step * T::BK * 2);
+  };
+  auto issue_b = [&](int step, int buf, int j) {
+    const int bs = (step < ksteps ? step : ksteps) * b_step;
+    h16_load_lds(rb, smem + T::B_AREA + buf * T::B_STEP + (wave * T::B_LOADS + j) * 1024, b_voff[j], bs);
+  };
+  // load j of the window that stage `s` opens (its buffers are free then): A and B of stage s + NS; pairs: B of that stage,
+  // and, odd stages before it, the rows of A of the pair after the next
+  auto issue = [&](int s, int buf, auto odd_tag, int j) {
+    constexpr bool A = !T::PAIR || decltype(odd_tag)::value != 0;
+    if (A && j < T::A_LOADS) issue_a(T::PAIR ? s + 3 : s + T::NS, buf, j);
+    else issue_b(s + T::NS, buf, A ? j - T::A_LOADS : j);
   };
 
   // ---- fragments: slice sl of a stage ----
   const int a_row = wm0 + l31;
-  int a_frag[T::SLW];
+  constexpr int SLICES = T::PAIR ? 2 * T::SLW : T::SLW;
+  int a_frag[SLICES];
 #pragma unroll
-  for (int x = 0; x < T::SLW; ++x) {
+  for (int x = 0; x < SLICES; ++x) {
     const int sl = T::WK == 1 ? x : 2 * x + wk;
-    a_frag[x] = a_row * T::BK * 2 + ((2 * sl + g + (a_row >> RSH)) & (T::KG - 1)) * 16;
+    a_frag[x] = a_row * T::AK * 2 + ((2 * sl + g + (a_row >> RSH)) & (T::KG - 1)) * 16;
   }
   // raw B: lane i = lane % 16 of a group of sixteen reads row 8 g + i / 4 (+ 4), columns 16 (lane / 16 % 2) + 4 (i % 4)
   int b_frag[RAWB ? T::NTL : 1];
@@ -172,14 +187,14 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 #pragma unroll
     for (int ni = 0; ni < T::NTL; ++ni) {
       const int chunk = (wn0 + ni * 32) / 8 + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
-      b_frag[ni] = T::A_STAGE + wk * b_slice + row * T::BN * 2 + (chunk ^ xor_of(row)) * 16 + (i & 1) * 8;
+      b_frag[ni] = T::B_AREA + wk * b_slice + row * T::BN * 2 + (chunk ^ xor_of(row)) * 16 + (i & 1) * 8;
     }
   } else {
-    b_frag[0] = T::A_STAGE + wk * b_slice + (g * T::BN + wn0 + l31) * 16;
+    b_frag[0] = T::B_AREA + wk * b_slice + (g * T::BN + wn0 + l31) * 16;
   }
   u32x4 Af[2][T::MT], Bf[2][T::NTL];
-  auto read = [&](const unsigned char* st, int x, int buf, int r) {   // r: A's blocks, then B's
-    if (r < T::MT) Af[buf][r] = *(const u32x4*)(st + a_frag[x] + r * 32 * T::BK * 2);
+  auto read = [&](const unsigned char* sa, int xa, const unsigned char* st, int x, int buf, int r) {   // r: A's blocks, then B's
+    if (r < T::MT) Af[buf][r] = *(const u32x4*)(sa + a_frag[xa] + r * 32 * T::AK * 2);
     else if (RAWB) {
       const unsigned src = (unsigned)(uintptr_t)(h16_lds_ptr)(st + b_frag[r - T::MT] + x * T::WK * b_slice);
       const u32x2 lo = h16_read_tr<0>(src), hi = h16_read_tr<8 * T::BN>(src);   // (four rows further down)
@@ -191,12 +206,22 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 
 #define H16_FENCE() __builtin_amdgcn_sched_barrier(0)
   f32x16 acc[T::MT][T::NTL];
-  // Loads of a stage: the first P with the last slice of stage s - NS, the others with the first slices of s - NS + 1.
-  constexpr int P = (T::LOADS + T::SLW - 1) / T::SLW;
+  // Loads of a window: the first P with the last slice of its stage, the others with the first slices of the next one.
+  typedef std::integral_constant<int, 0> Even;
+  typedef std::integral_constant<int, 1> Odd;
+  constexpr int WIN[2] = {T::PAIR ? T::B_LOADS : T::LOADS, T::LOADS};   // of an even stage, of an odd one
+  constexpr int P[2] = {(WIN[0] + T::SLW - 1) / T::SLW, (WIN[1] + T::SLW - 1) / T::SLW};
+  // (as if stages -NS ... -1 had opened their windows)
+  if constexpr (T::PAIR) {
 #pragma unroll
-  for (int s = 0; s < T::NS; ++s)
+    for (int j = 0; j < T::A_LOADS; ++j) issue_a(0, 0, j);
+  }
 #pragma unroll
-    for (int j = 0; j < (s < T::NS - 1 ? T::LOADS : P); ++j) issue(s, s, j);
+  for (int s = 0; s < T::NS - 1; ++s)
+#pragma unroll
+    for (int j = 0; j < WIN[0]; ++j) issue(s - T::NS, s, Even(), j);
+#pragma unroll
+  for (int j = 0; j < P[1]; ++j) issue(-1, T::NS - 1, Odd(), j);
   H16_FENCE();
   // (cleared while the first loads are in flight; the empty statements make the zeros real here)
 #pragma unroll
@@ -209,32 +234,42 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
       else asm volatile("" : "+v"(acc[mi][ni]));
     }
   H16_FENCE();
-  constexpr int W0 = (T::NS - 2) * T::LOADS + P, W1 = (T::NS - 2) * T::LOADS;
+  // What may be in flight: while stage 0 is waited for, and at the barrier of an even and of an odd stage for the next one (pairs:
+  // an odd one waits for the pair of A too, which only two stages of B are younger than)
+  constexpr int W0 = (T::NS - 2) * WIN[0] + P[1];
+  constexpr int W1[2] = {(T::NS - 2) * WIN[0] + (T::PAIR ? (T::NS - 1) / 2 * T::A_LOADS : 0), (T::PAIR ? 2 : T::NS - 2) * WIN[0]};
+  static_assert(W0 <= 63 && W1[0] <= 63, "the wait counter has six bits");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (W0 & 0xF) | ((W0 >> 4) << 14));   // stage 0 has landed
   __builtin_amdgcn_s_barrier();
   H16_FENCE();
 #pragma unroll
-  for (int r = 0; r < T::MT + T::NTL; ++r) read(smem, 0, 0, r);
+  for (int r = 0; r < T::MT + T::NTL; ++r) read(smem, 0, smem, 0, 0, r);
   if (RAWB) __builtin_amdgcn_s_waitcnt(0xC07F);
 
   int cur = 0, before = T::NS - 1;   // LDS buffers of this stage and of the one before it
-  for (int s = 0; s < ksteps; ++s) {
+  // one stage; odd_tag: pairs' second
+  auto stage = [&](int s, auto odd_tag) {
+    constexpr int ODD = decltype(odd_tag)::value;
+    typedef std::integral_constant<int, T::PAIR ? 1 - ODD : 0> Before;   // the stage before it
     const int nx = cur == T::NS - 1 ? 0 : cur + 1;
-    const unsigned char* st0 = smem + cur * T::STAGE;
-    const unsigned char* st1 = smem + nx * T::STAGE;
+    const unsigned char* st0 = smem + cur * T::B_STEP;
+    const unsigned char* st1 = smem + nx * T::B_STEP;
+    const unsigned char* sa0 = T::PAIR ? smem + (s & 2) * (T::A_BUF / 2) : st0;
+    const unsigned char* sa1 = !T::PAIR ? st1 : ODD ? smem + ((s + 1) & 2) * (T::A_BUF / 2) : sa0;
+    constexpr int XA = ODD * T::SLW, XN = T::PAIR && !ODD ? T::SLW : 0;   // A's first slice of this stage, of the next one
 #pragma unroll
     for (int x = 0; x < T::SLW; ++x) {
       const int buf = x & 1;
       const bool last = x == T::SLW - 1;
       if (last) {
         // own loads of stage s + 1 have landed and own reads of stage s are over, then everybody's
-        __builtin_amdgcn_s_waitcnt(0x0070 | (W1 & 0xF) | ((W1 >> 4) << 14));
+        __builtin_amdgcn_s_waitcnt(0x0070 | (W1[ODD] & 0xF) | ((W1[ODD] >> 4) << 14));
         __builtin_amdgcn_s_barrier();
         H16_FENCE();
       }
       // behind the MFMAs of a slice: first the fragment reads of the next one, then this slice's share of the loads
-      constexpr int READS = T::MT + T::NTL, MF = T::MT * T::NTL;
-      const int l0 = last ? 0 : P + x * (T::LOADS - P) / (T::SLW - 1), l1 = last ? P : P + (x + 1) * (T::LOADS - P) / (T::SLW - 1);
+      constexpr int READS = T::MT + T::NTL, MF = T::MT * T::NTL, PB = P[Before::value], WB = WIN[Before::value];
+      const int l0 = last ? 0 : PB + x * (WB - PB) / (T::SLW - 1), l1 = last ? P[ODD] : PB + (x + 1) * (WB - PB) / (T::SLW - 1);
       constexpr int RG = MF >= READS ? READS : (MF + 1) / 2;   // gaps that take the reads
 #pragma unroll
       for (int mf = 0; mf < MF; ++mf) {
@@ -247,14 +282,14 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 #pragma unroll
         for (int r = 0; r < READS; ++r) {
           if (r * RG / READS != mf) continue;
-          if (last) read(st1, 0, buf ^ 1, r);
-          else read(st0, x + 1, buf ^ 1, r);
+          if (last) read(sa1, XN, st1, 0, buf ^ 1, r);
+          else read(sa0, XA + x + 1, st0, x + 1, buf ^ 1, r);
         }
 #pragma unroll
         for (int j = 0; j < T::LOADS; ++j) {
           if (j < l0 || j >= l1 || (j - l0) * MF / (l1 - l0) != mf) continue;
-          if (last) issue(s + T::NS, cur, j);
-          else issue(s + T::NS - 1, before, j);
+          if (last) issue(s, cur, odd_tag, j);
+          else issue(s - 1, before, Before(), j);
         }
         H16_FENCE();
       }
@@ -265,6 +300,10 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     }
     before = cur;
     cur = nx;
+  };
+  for (int s = 0; s < ksteps; s += T::PAIR ? 2 : 1) {
+    stage(s, Even());
+    if constexpr (T::PAIR) stage(s + 1, Odd());
   }
 #undef H16_FENCE
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the loads past the last stage have landed before LDS is used again

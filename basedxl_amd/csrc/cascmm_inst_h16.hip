@@ -50,7 +50,7 @@ static int launch_h16(const GroupParams& p, hipStream_t stream) {
 static const VariantDesc kTable[] = {
     // (stages in LDS: with more than these the first MFMA waits behind the loads of stages that are needed late:
     // 2048 x 2048 x 2048 on 128 x 128: 20.8 us with three, 22.0 with four, 23.5 with five)
-    H16_TILE("t256x320x32", 4, 1, 1, 2, 10, 32, 3),
+    H16_TILE("t256x320x32", 4, 1, 1, 2, 10, 32, 4),
     H16_TILE("t256x256x32", 2, 2, 1, 4, 4, 32, 4),
     H16_TILE("t128x256x64", 2, 2, 1, 2, 4, 64, 3),
     H16_TILE("t128x160x64", 4, 1, 1, 1, 5, 64, 3),
