@@ -388,30 +388,36 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 #pragma unroll
     for (int mi = 0; mi < T::MT; ++mi) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
+      for (int b = 0; b < NB; ++b) {
+        // (a block's bias values at once: quad by quad, every quad waits for its own)
+        f32x4 bv[4], bg[4];
+        if constexpr (BIAS) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            bv[q] = *(const f32x4*)(bl + (GLU ? 64 : 32) * b + 8 * q + 4 * g);
+            if constexpr (GLU) bg[q] = *(const f32x4*)(bl + 64 * b + 32 + 8 * q + 4 * g);
+          }
+        }
+        auto sum = [&](int block, const f32x4* bias4, int q, int x) { return BIAS ? acc[mi][block][4 * q + x] + bias4[q][x] : acc[mi][block][4 * q + x]; };
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int at = 8 * q + 4 * g;
           typedef E e2 __attribute__((ext_vector_type(2)));
-          f32x4 y;
+          float y[4];
           if constexpr (GLU) {
-            f32x4 bv = {0.f, 0.f, 0.f, 0.f}, bg = bv;
-            if constexpr (BIAS) {
-              bv = *(const f32x4*)(bl + 64 * b + at);
-              bg = *(const f32x4*)(bl + 64 * b + 32 + at);
-            }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = gated_value(acc[mi][2 * b][4 * q + e] + bv[e], acc[mi][2 * b + 1][4 * q + e] + bg[e]);
+            for (int x = 0; x < 4; ++x) y[x] = sum(2 * b + 1, bg, q, x);
+            gelu_values(y);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) y[x] *= sum(2 * b, bv, q, x);
           } else {
-            f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (BIAS) bv = *(const f32x4*)(bl + 32 * b + at);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = BIAS ? acc[mi][B0 + b][4 * q + e] + bv[e] : acc[mi][B0 + b][4 * q + e];
+            for (int x = 0; x < 4; ++x) y[x] = sum(B0 + b, bv, q, x);
           }
           const u32x2 out = {__builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){y[0], y[1]}, e2)),
                              __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){y[2], y[3]}, e2))};
-          *(u32x2*)(area + l31 * T::OUT_ROW + (32 * b + at) * 2) = out;
+          *(u32x2*)(area + l31 * T::OUT_ROW + (32 * b + 8 * q + 4 * g) * 2) = out;
         }
+      }
       if (vec) {
         // (a few at a time: the reads' latency overlaps, the registers last)
         constexpr int GRP = ITS <= 8 ? ITS : ITS == 10 ? 5 : 4;

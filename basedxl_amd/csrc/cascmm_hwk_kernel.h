@@ -232,8 +232,10 @@ __global__ __launch_bounds__(512) void cascmm_hwk_kernel(const GroupParams p) {
         }
     }
     if constexpr (GLU) {
+      float gate[4] = {g[0], g[1], g[2], g[3]};
+      gelu_values(gate);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = gated_value(s[e], g[e]);
+      for (int e = 0; e < 4; ++e) s[e] *= gate[e];
     }
     E* c = C + (int64_t)row * p.ldc + col;
     if (vec) *(e4*)c = __builtin_convertvector(s, e4);

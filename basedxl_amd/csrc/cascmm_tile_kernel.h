@@ -174,7 +174,6 @@ struct TileGemm {
   // the gated epilogue needs prepared B (columns in any order at no cost) and a consumer wave that
   // owns whole value / gate pairs of 32-column blocks
   static constexpr bool kGluCapable = BPRE && TL::BNQ == 0 && TL::NTL % 2 == 0;
-  static __device__ __forceinline__ float gated(float v, float g) { return gated_value(v, g); }
   static constexpr int QN = TL::QN;
   static constexpr int QW = TL::BNQ > 0 ? TL::BNQ / QN : 1;   // blocks per row of the permuted part
   static constexpr int SW = TL::BNS > 0 ? TL::BNS : 1;       // columns of the unpermuted part
@@ -782,13 +781,17 @@ struct TileGemm {
 #pragma unroll
           for (int mi = 0; mi < TL::MT; ++mi)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 4; ++q) {
+              float gate[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) gate[e] = res[mi][2 * nj + 1][4 * q + e] + bg;
+              gelu_values(gate);
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const float y = gated(res[mi][2 * nj][4 * q + e] + bv, res[mi][2 * nj + 1][4 * q + e] + bg);
                 const int soff = (mi * 32 + q * 8 + e) * ldc_bytes;
-                llvm_raw_buffer_store_f32(y, rc, voff, soff, kResultStoreAux);
+                llvm_raw_buffer_store_f32((res[mi][2 * nj][4 * q + e] + bv) * gate[e], rc, voff, soff, kResultStoreAux);
               }
+            }
         }
         return;
       }
@@ -802,12 +805,16 @@ struct TileGemm {
           const int row0 = m0 + wm0 + mi * 32 + g * 4;
           IoT* dst = C + (int64_t)row0 * ldc + col;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
+          for (int q = 0; q < 4; ++q) {
+            float gate[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gate[e] = res[mi][2 * nj + 1][4 * q + e] + bg;
+            gelu_values(gate);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (row0 + q * 8 + e < p.M)
-                IoType<IODT>::store(dst + (int64_t)(q * 8 + e) * ldc,
-                                    gated(res[mi][2 * nj][4 * q + e] + bv, res[mi][2 * nj + 1][4 * q + e] + bg));
+                IoType<IODT>::store(dst + (int64_t)(q * 8 + e) * ldc, (res[mi][2 * nj][4 * q + e] + bv) * gate[e]);
+          }
         }
       }
       return;

@@ -420,8 +420,12 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float bg = bias_at(half + c0 + 64 + 8 * (r >> 2) + 4 * eg + (r & 3));
+        float gate[T::MT];
 #pragma unroll
-        for (int mi = 0; mi < T::MT; ++mi) xbuf[(mi * 16 + r) * 64 + elane] = gelu_value(acc[mi][0][r] + bg);
+        for (int mi = 0; mi < T::MT; ++mi) gate[mi] = acc[mi][0][r] + bg;
+        gelu_values(gate);
+#pragma unroll
+        for (int mi = 0; mi < T::MT; ++mi) xbuf[(mi * 16 + r) * 64 + elane] = gate[mi];
       }
     }
     __syncthreads();
@@ -443,12 +447,16 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
         const int soff = ((col0 >> 3) + 2 * s2) * p.M * 16;
 #pragma unroll
         for (int mi = 0; mi < T::MT; ++mi) {
-          float r8[8];
+          float r8[8], gl[8];
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
             const int r = 8 * s2 + x;                               // register 4 q + e with q = 2 s2 + x / 4
-            const float gl = gate_in_lds ? xbuf[(mi * 16 + r) * 64 + elane] : gelu_value(acc[mi][gb][r] + bgt[x]);
-            r8[x] = (acc[mi][vb][r] + bv[x]) * gl;
+            gl[x] = gate_in_lds ? xbuf[(mi * 16 + r) * 64 + elane] : acc[mi][gb][r] + bgt[x];
+          }
+          if (!gate_in_lds) gelu_values(gl);
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            r8[x] = (acc[mi][vb][8 * s2 + x] + bv[x]) * gl[x];
             // the slots are the split of this product ROUNDED to fp32, as a separate pass over the fp32
             // result would split it: keep the compiler from folding the multiplication into the split's
             // subtraction (a fused multiply-subtract would take the residual of the unrounded product)
@@ -483,13 +491,16 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
 #pragma unroll
       for (int mi = 0; mi < T::MT; ++mi)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+          float gate[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * q + e;
-            llvm_raw_buffer_store_f32((acc[mi][2 * pair][r] + bv) * gelu_value(acc[mi][2 * pair + 1][r] + bg), re,
+          for (int e = 0; e < 4; ++e) gate[e] = acc[mi][2 * pair + 1][4 * q + e] + bg;
+          gelu_values(gate);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            llvm_raw_buffer_store_f32((acc[mi][2 * pair][4 * q + e] + bv) * gate[e], re,
                                       (int)((unsigned)voff + (unsigned)((mi * 32 + q * 8 + e) * ldc_bytes)), 0, kLargeTileStoreAux);
-          }
+        }
     }
     return;
   } else if constexpr (GLU == 1) {
@@ -506,7 +517,14 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
 #pragma unroll
       for (int mi = 0; mi < T::MT; ++mi)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) xbuf[(mi * 16 + r) * 64 + elane] = gelu_value(acc[mi][0][r] + bg);
+        for (int q = 0; q < 4; ++q) {
+          float gate[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) gate[e] = acc[mi][0][4 * q + e] + bg;
+          gelu_values(gate);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) xbuf[(mi * 16 + 4 * q + e) * 64 + elane] = gate[e];
+        }
     }
     __syncthreads();
     float* C = (float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc + c0;
@@ -520,14 +538,17 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
 #pragma unroll
       for (int mi = 0; mi < T::MT; ++mi)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+          float gl[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) gl[e] = gate_in_lds ? xbuf[(mi * 16 + 4 * q + e) * 64 + elane] : acc[mi][gb][4 * q + e] + bg;
+          if (!gate_in_lds) gelu_values(gl);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int r = 4 * q + e;
-            const float gl = gate_in_lds ? xbuf[(mi * 16 + r) * 64 + elane] : gelu_value(acc[mi][gb][r] + bg);
             const int roff = (mi * 32 + q * 8 + e) * ldc_bytes;
-            llvm_raw_buffer_store_f32((acc[mi][vb][r] + bv) * gl, rc, EDGE ? voff + roff : voff, EDGE ? 0 : roff, kLargeTileStoreAux);
+            llvm_raw_buffer_store_f32((acc[mi][vb][4 * q + e] + bv) * gl[e], rc, EDGE ? voff + roff : voff, EDGE ? 0 : roff, kLargeTileStoreAux);
           }
+        }
     };
     if ((wave & 1) == 0) {
       out_pair(0, 0, 1, false);
