@@ -389,6 +389,10 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     for (int mi = 0; mi < T::MT; ++mi) {
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
+        // (The large tiles' sums stay in the accumulation registers up to here.  Left alone the compiler moves all of them to ordinary ones
+        // behind the loop, through scratch memory what does not fit: 26 k cycles of store in place of 16 k on 256 x 320, 16 k in place of
+        // 10 k on 256 x 256; gated, and of smaller tiles, its own order is the better one.)
+        if (!GLU && T::MT * T::NTL >= 16 && mi * T::NTL + B0 + b < 16) asm volatile("" : "+a"(acc[mi][B0 + b]));
         // (a block's bias values at once: quad by quad, every quad waits for its own)
         f32x4 bv[4], bg[4];
         if constexpr (BIAS) {
