@@ -506,57 +506,56 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   } else if constexpr (GLU == 1) {
     // Gated store: C[m][n0 / 2 + 32 j + l] = (value j + bias) x gelu(gate j + bias), j = 0 .. 4.  The
     // left wave of a row pair holds value 0, gate 0, value 1, gate 1, value 2, the right one gate 2,
-    // value 3, gate 3, value 4, gate 4: pair 2 is the only one that spans two waves; the right wave
-    // evaluates its gate (which evens out the two waves' arithmetic) and hands gelu(gate), same lanes and
-    // registers, over through the LDS the main loop has given up.
+    // value 3, gate 3, value 4, gate 4: pair 2 is the only one that spans two waves.  Each evaluates half of its gates: the
+    // left wave hands its values of the upper two row blocks over, the right one its gates of the lower two, same lanes and
+    // registers, through the LDS the main loop has given up.  (The gates are what this store takes: with all of pair 2's on the
+    // right wave, and the left one waiting for them, 192 a lane one behind the other in place of 160.)
     const int half = p.N >> 1, c0 = n0 >> 1;
-    float* xbuf = (float*)smem + (wave >> 1) * (T::MT * 16 * 64);   // 16 KB per row pair of waves
+    float* xbuf = (float*)smem + (wave >> 1) * (4 * 16 * 64);        // 16 KB per row pair of waves: 32 values, 32 gates a lane
     __builtin_amdgcn_s_barrier();                                    // every wave has read its last fragments
+    const float b2 = bias ? bias[(wave & 1 ? half : 0) + c0 + 64 + el31] : 0.f;   // of pair 2's columns that this wave holds
     if (wave & 1) {
-      const float bg = bias ? bias[half + c0 + 64 + el31] : 0.f;
 #pragma unroll
-      for (int mi = 0; mi < T::MT; ++mi)
+      for (int r = 0; r < 32; ++r) xbuf[(32 + r) * 64 + elane] = acc[2 + r / 16][0][r & 15] + b2;
+    } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float gate[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) gate[e] = acc[mi][0][4 * q + e] + bg;
-          gelu_values(gate);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) xbuf[(mi * 16 + 4 * q + e) * 64 + elane] = gate[e];
-        }
+      for (int r = 0; r < 32; ++r) xbuf[r * 64 + elane] = acc[r / 16][4][r & 15] + b2;
     }
     __syncthreads();
     float* C = (float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc + c0;
     // (EDGE: the descriptor ends with the last row of C, the row offsets are part of the checked lane offset)
     const int rows = p.M - (m0 + wm0);
     const i32x4 rc = make_rsrc(C, !EDGE ? 0x7FFFFFFF : rows > 0 ? (int64_t)(rows < T::WTM ? rows : T::WTM) * ldc_bytes - c0 * 4 : 0);
-    auto out_pair = [&](int pair, int vb, int gb, bool gate_in_lds) {
-      const float bv = bias ? bias[c0 + 32 * pair + el31] : 0.f;
-      const float bg = (bias && !gate_in_lds) ? bias[half + c0 + 32 * pair + el31] : 0.f;
+    // row blocks first .. last - 1 of a pair; value and gate: its sums with the bias
+    auto out_pair = [&](int pair, int first, int last, auto value, auto gate) {
       const int voff = eg * 4 * ldc_bytes + (pair * 32 + el31) * 4;
 #pragma unroll
-      for (int mi = 0; mi < T::MT; ++mi)
+      for (int mi = first; mi < last; ++mi)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float gl[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) gl[e] = gate_in_lds ? xbuf[(mi * 16 + 4 * q + e) * 64 + elane] : acc[mi][gb][4 * q + e] + bg;
-          if (!gate_in_lds) gelu_values(gl);
+          for (int e = 0; e < 4; ++e) gl[e] = gate(mi, 4 * q + e);
+          gelu_values(gl);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int roff = (mi * 32 + q * 8 + e) * ldc_bytes;
-            llvm_raw_buffer_store_f32((acc[mi][vb][4 * q + e] + bv) * gl[e], rc, EDGE ? voff + roff : voff, EDGE ? 0 : roff, kLargeTileStoreAux);
+            llvm_raw_buffer_store_f32(value(mi, 4 * q + e) * gl[e], rc, EDGE ? voff + roff : voff, EDGE ? 0 : roff, kLargeTileStoreAux);
           }
         }
     };
+    auto own_pair = [&](int pair, int vb, int gb) {
+      const float bv = bias ? bias[c0 + 32 * pair + el31] : 0.f, bg = bias ? bias[half + c0 + 32 * pair + el31] : 0.f;
+      out_pair(pair, 0, T::MT, [&](int mi, int r) { return acc[mi][vb][r] + bv; }, [&](int mi, int r) { return acc[mi][gb][r] + bg; });
+    };
     if ((wave & 1) == 0) {
-      out_pair(0, 0, 1, false);
-      out_pair(1, 2, 3, false);
-      out_pair(2, 4, 0, true);
+      own_pair(0, 0, 1);
+      own_pair(1, 2, 3);
+      out_pair(2, 2, 4, [&](int mi, int r) { return acc[mi][4][r] + b2; }, [&](int mi, int r) { return xbuf[(mi * 16 + r) * 64 + elane]; });
     } else {
-      out_pair(3, 1, 2, false);
-      out_pair(4, 3, 4, false);
+      out_pair(2, 0, 2, [&](int mi, int r) { return xbuf[(mi * 16 + r) * 64 + elane]; }, [&](int mi, int r) { return acc[mi][0][r] + b2; });
+      own_pair(3, 1, 2);
+      own_pair(4, 3, 4);
     }
     return;
   }
