@@ -192,7 +192,11 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   } else {
     b_frag[0] = T::B_AREA + wk * b_slice + (g * T::BN + wn0 + l31) * 16;
   }
-  u32x4 Af[2][T::MT], Bf[2][T::NTL];
+  // How many slices ahead fragments are read: a slice of few MFMAs is over before the next one's are there.  Two on 128 x 128 (loop of 2048^3
+  // 23.7 -> 23.0 k cycles); the smaller tiles gained nothing (512 x 1280 x 1280 on 64 x 64 8.4 -> 8.6 us), the larger ones have MFMAs
+  // enough, and raw, the reads written as assembly must not be in flight where the loop closes.
+  constexpr int PF = !T::PAIR && T::WK == 1 && !RAWB && T::MT * T::NTL == 4 ? 2 : 1;
+  u32x4 Af[2 * PF][T::MT], Bf[2 * PF][T::NTL];
   auto read = [&](const unsigned char* sa, int xa, const unsigned char* st, int x, int buf, int r) {   // r: A's blocks, then B's
     if (r < T::MT) Af[buf][r] = *(const u32x4*)(sa + a_frag[xa] + r * 32 * T::AK * 2);
     else if (RAWB) {
@@ -206,11 +210,13 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 
 #define H16_FENCE() __builtin_amdgcn_sched_barrier(0)
   f32x16 acc[T::MT][T::NTL];
-  // Loads of a window: the first P with the last slice of its stage, the others with the first slices of the next one.
+  // Loads of a window: the first P with the last PF slices of its stage, the others with the first slices of the next one.
   typedef std::integral_constant<int, 0> Even;
   typedef std::integral_constant<int, 1> Odd;
   constexpr int WIN[2] = {T::PAIR ? T::B_LOADS : T::LOADS, T::LOADS};   // of an even stage, of an odd one
-  constexpr int P[2] = {(WIN[0] + T::SLW - 1) / T::SLW, (WIN[1] + T::SLW - 1) / T::SLW};
+  constexpr int P[2] = {(PF * WIN[0] + T::SLW - 1) / T::SLW, (PF * WIN[1] + T::SLW - 1) / T::SLW};
+  constexpr int FIRST = T::SLW - PF;   // the slice that a stage's barrier stands in front of
+  static_assert(PF == 1 || (T::SLW == 2 * PF && !T::PAIR), "a slice's fragments have their buffer");
   // (as if stages -NS ... -1 had opened their windows)
   if constexpr (T::PAIR) {
 #pragma unroll
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
   __builtin_amdgcn_s_barrier();
   H16_FENCE();
 #pragma unroll
-  for (int r = 0; r < T::MT + T::NTL; ++r) read(smem, 0, smem, 0, 0, r);
+  for (int r = 0; r < PF * (T::MT + T::NTL); ++r) read(smem, r / (T::MT + T::NTL), smem, r / (T::MT + T::NTL), r / (T::MT + T::NTL), r % (T::MT + T::NTL));
   if (RAWB) __builtin_amdgcn_s_waitcnt(0xC07F);
 
   int cur = 0, before = T::NS - 1;   // LDS buffers of this stage and of the one before it
@@ -259,9 +265,9 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     constexpr int XA = ODD * T::SLW, XN = T::PAIR && !ODD ? T::SLW : 0;   // A's first slice of this stage, of the next one
 #pragma unroll
     for (int x = 0; x < T::SLW; ++x) {
-      const int buf = x & 1;
-      const bool last = x == T::SLW - 1;
-      if (last) {
+      const int buf = x % (2 * PF), to = (x + PF) % (2 * PF);
+      const bool late = x >= FIRST;
+      if (x == FIRST) {
         // own loads of stage s + 1 have landed and own reads of stage s are over, then everybody's
         __builtin_amdgcn_s_waitcnt(0x0070 | (W1[ODD] & 0xF) | ((W1[ODD] >> 4) << 14));
         __builtin_amdgcn_s_barrier();
@@ -269,8 +275,10 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
       }
       // behind the MFMAs of a slice: first the fragment reads of the next one, then this slice's share of the loads
       constexpr int READS = T::MT + T::NTL, MF = T::MT * T::NTL, PB = P[Before::value], WB = WIN[Before::value];
-      const int l0 = last ? 0 : PB + x * (WB - PB) / (T::SLW - 1), l1 = last ? P[ODD] : PB + (x + 1) * (WB - PB) / (T::SLW - 1);
-      constexpr int RG = MF >= READS ? READS : (MF + 1) / 2;   // gaps that take the reads
+      const int l0 = late ? (x - FIRST) * P[ODD] / PF : PB + x * (WB - PB) / FIRST, l1 = late ? (x - FIRST + 1) * P[ODD] / PF : PB + (x + 1) * (WB - PB) / FIRST;
+      // gaps that take the reads.  Of four, the first two: spread over all of them the last one is waited for (loop of 2048^3 on 128 x 128
+      // raw 32.4 -> 28.2 k cycles, prepared 25.4 -> 23.7; with two reads a gap 64 x 160 raw lost 7 %, 128 x 160 4 %)
+      constexpr int RG = MF == 4 ? 2 : MF >= READS ? READS : (MF + 1) / 2;
 #pragma unroll
       for (int mf = 0; mf < MF; ++mf) {
         const int ni = mf / T::MT, mi = mf % T::MT;
@@ -282,13 +290,13 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 #pragma unroll
         for (int r = 0; r < READS; ++r) {
           if (r * RG / READS != mf) continue;
-          if (last) read(sa1, XN, st1, 0, buf ^ 1, r);
-          else read(sa0, XA + x + 1, st0, x + 1, buf ^ 1, r);
+          if (late) read(sa1, XN + x - FIRST, st1, x - FIRST, to, r);
+          else read(sa0, XA + x + PF, st0, x + PF, to, r);
         }
 #pragma unroll
         for (int j = 0; j < T::LOADS; ++j) {
           if (j < l0 || j >= l1 || (j - l0) * MF / (l1 - l0) != mf) continue;
-          if (last) issue(s, cur, odd_tag, j);
+          if (late) issue(s, cur, odd_tag, j);
           else issue(s - 1, before, Before(), j);
         }
         H16_FENCE();
