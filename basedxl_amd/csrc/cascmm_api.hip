@@ -163,7 +163,7 @@ static bool variant_matches(const VariantDesc& v, const Problem& q, RowFit fit) 
   if (v.kind == KIND_SLOTK && (q.lda < 32 || q.glu || q.M * q.lda * 4 > INT32_MAX || q.ldc * (int64_t)(v.BM * 4) > INT32_MAX))
     return false;
   // (32-bit byte offsets down B, a raw one's two stages past the end included, and inside a tile of A, see row_fit; K in whole 16-byte chunks)
-  if (v.kind == KIND_HWK && v.call_only && !q.call) return false;
+  if ((v.kind == KIND_HWK || v.kind == KIND_W512E) && v.call_only && !q.call) return false;
   if ((v.kind == KIND_H16 || v.kind == KIND_HWK) && ((q.K % 8 != 0 && !q.chunked) || q.K == 0 || (q.bpre ? beyond_i32((q.K + 63) / 64, q.N, 128) : beyond_i32(q.K + 64, q.ldb, 2))))
     return false;
   if (q.glu && !v.glu) return false;
@@ -246,6 +246,9 @@ constexpr double kF8WKStageUs = 2.25, kF8WKFixedUs = 6.0;   // (fit: 2048 x {128
 // (7 %) and with more than 5 MB of A (10 %; rows off 16 bytes of 20 MB and more 25 %, where a copy of A is the alternative), which their estimates are
 // raised by.  Groups: the tiles of all their problems; there the eight-wave tiles are 5 - 8 % faster than that and the prepared 64 x 160 one 8 % slower (305 groups
 // of two and three, 0.6 and 0.8 % behind the fastest on average, 2.5 and 3.5 % in one of twenty).
+// The large tiles of 192 and 128 columns, and all gated large tiles, are fitted to 230 shapes each (raw, prepared, gated; 300 - 9000 rows).  On 376 raw,
+// 380 prepared and 380 gated others they are chosen for 38, 35 and 23, which take 0.92, 0.91 and 0.87 of the time of what was chosen before
+// (one of them more than 3 % longer: gated 1289 x 576 x 4608 28.5 us, 26.5); the kernel chosen is 0.3 - 0.6 % behind the fastest of all on average.
 // The selection functions, which answer for shapes, keep the constants above but for KIND_WAVEK.
 struct CallCost { const char* name; double c0, s0, s1, c1, bw, x, r1, deep, edge; };
 static const CallCost kCallCost[] = {
@@ -265,6 +268,8 @@ static const CallCost kCallCost[] = {
     {"t128x128x64_w4x1x1_d2_p8_bf16x2_tri", 7.79, 0.949, 1.03, 3.05, 14.8, 2.11, 1.24, 5.44, 4.31},
     {"t256x128x32_w4x1x1_d2_bf16x2_tri", 8.14, 1.84, 1.92, 4.28, 5.15, 3.21, 2.37, 4.76, 10.8},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri", 10.6, 2.12, 2.43, 5.46, 7.3, 3.16, 2.67, 4.77, 12.2},
+    {"t256x128x32_w512_narrow_bf16x2_tri", 10, 1.97, 1.97, 6.25, 7.12, 3.15, 2.7, 5.3, 0},
+    {"t256x192x32_w512_narrow_bf16x2_tri", 11.6, 2.48, 3.1, 8.09, 5, 3.95, 3.66, 4.74, 0.115},
     {"t256x256x32_w512_edge_bf16x2_tri", 10.8, 2.93, 4.76, 9.03, 51.2, 3.72, 4.87, 0, 1.43},
     {"t256x320x32_w512_edge_bf16x2_tri", 12.5, 3.48, 5.85, 13.5, 60, 3.47, 5.71, 0.153, 1.61},
     {"t256x320x32_w512_bf16x2_tri", 12.4, 3.45, 5.79, 13.4, 60, 3.47, 5.65, 0.151, 0},
@@ -292,6 +297,8 @@ static const CallCost kCallCost[] = {
     {"t128x160x32_w2x1x2_d3_bf16x2_tri_bpre", 8.7, 1.09, 1.2, 2.33, 6.04, 2.66, 1.48, 4.52, 5.43},
     {"t256x128x32_w4x1x1_d2_bf16x2_tri_bpre", 8.58, 1.54, 1.81, 3.81, 13.7, 2.3, 2.26, 4.32, 3.23},
     {"t256x160x32_w4x1x1_d2_bf16x2_tri_bpre", 9.46, 1.98, 2.55, 1.51, 9.49, 4.62, 2.69, 4.44, 8.45},
+    {"t256x128x32_w512_narrow_bf16x2_tri_bpre", 8.82, 1.83, 2.08, 5.36, 5.45, 4.23, 2.57, 4.58, 0.358},
+    {"t256x192x32_w512_narrow_bf16x2_tri_bpre", 11.6, 2.25, 2.83, 6.84, 5.08, 4.16, 3.5, 4.59, 0.0827},
     {"t256x256x32_w512_edge_bf16x2_tri_bpre", 11.4, 2.77, 4.31, 9.8, 14.7, 3.83, 4.45, 3.63, 0.921},
     {"t256x320x32_w512_edge_bf16x2_tri_bpre", 12, 3.27, 5.17, 11, 22.9, 2.97, 5.43, 0.301, 2.16},
     {"t256x320x32_w512_bf16x2_tri_bpre", 11.9, 3.24, 5.12, 10.9, 22.9, 2.97, 5.38, 0.298, 0},
@@ -306,9 +313,10 @@ static const CallCost kGatedCost[] = {
     {"t64x256x32_w1x4x1_d3_bf16x2_tri_bpre", 7.36, 0.951, 0.377, 0.872, 60, 1.26, 1.32, 5.89, 2.34},
     {"t128x128x64_w2x2x1_d2_bf16x2_tri_bpre", 8.87, 0.909, 1.03, 0.863, 18.9, 3.8, 1.29, 5.41, 2.07},
     {"t256x128x32_w4x1x1_d2_bf16x2_tri_bpre", 9.06, 1.51, 1.84, 2.77, 60, 2.29, 2.4, 4.47, 4.59},
-    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 12.8, 2.79, 4.18, 8.81, 55.8, 3.41, 4.54, 4.19, 0},
-    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 17.3, 3.38, 5.37, 14.6, 60, 4.03, 5.44, 3.56, 0},
-    {"t256x320x32_w512_bf16x2_tri_bpre", 17.1, 3.35, 5.32, 14.5, 60, 4.03, 5.39, 3.52, 0},
+    {"t256x128x32_w512_narrow_bf16x2_tri_bpre", 9.33, 1.72, 1.89, 6.09, 60, 2.35, 2.47, 4.94, 0},
+    {"t256x256x32_w512_edge_bf16x2_tri_bpre", 13.4, 2.63, 3.27, 8.56, 5.22, 2.67, 4.26, 3.78, 0.127},
+    {"t256x320x32_w512_edge_bf16x2_tri_bpre", 16.2, 3.08, 4.34, 10, 60, 2.08, 5.34, 3.48, 1.52},
+    {"t256x320x32_w512_bf16x2_tri_bpre", 16, 3.05, 4.3, 9.9, 60, 2.08, 5.29, 3.44, 0},
 };
 // What the selection functions, and with them the limits of cascmm_gemm_noalloc, price the two tiles of KIND_WAVEK by that they know
 static const CallCost kShapeCost[] = {
@@ -350,7 +358,9 @@ static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Pr
   }
   const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * (full + 1.0) : us;
   const double power = t.deep * tiles * v.BM * v.BN * (double)k_per * 1.0e-9;
-  return std::pow(std::pow(edged, 8.0) + std::pow(power, 8.0), 0.125) * (count > 1 && q.bpre && v.BM == 64 && v.BN == 160 ? 1.08 : 1.0);
+  // (the large tiles of 192 and 128 columns, prepared: with a margin; without one 3072^3 took 153 us on 192, 138 on 256 x 160)
+  const double margin = count > 1 && q.bpre && v.BM == 64 && v.BN == 160 ? 1.08 : q.bpre && v.kind == KIND_W512E && v.call_only ? 1.03 : 1.0;
+  return std::pow(std::pow(edged, 8.0) + std::pow(power, 8.0), 0.125) * margin;
 }
 static bool wavek_eligible(const Problem& q) {
   return q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_BF16 && q.terms == 2 && q.products == CASCMM_PROD_TRI && !q.bpre &&

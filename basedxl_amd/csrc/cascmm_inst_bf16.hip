@@ -22,6 +22,8 @@ static const VariantDesc kTable[] = {
     CASCMM_W512_VARIANT("t256x320x32_w512_bf16x2_tri", 0),
     CASCMM_W512_EDGE_VARIANT("t256x320x32_w512_edge_bf16x2_tri", 0, 5),
     CASCMM_W512_EDGE_VARIANT("t256x256x32_w512_edge_bf16x2_tri", 0, 4),
+    CASCMM_W512_EDGE_VARIANT("t256x192x32_w512_narrow_bf16x2_tri", 0, 3),
+    CASCMM_W512_EDGE_VARIANT("t256x128x32_w512_narrow_bf16x2_tri", 0, 2),
     // K split over the eight waves of a workgroup: one launch, no workspace
     CASCMM_WAVEK_VARIANT("t32x32x32_wavek_bf16x2_tri", 32, 1, 1, BF, 2),
     CASCMM_WAVEK_VARIANT("t32x64x32_wavek_bf16x2_tri", 16, 2, 4, BF, 2),

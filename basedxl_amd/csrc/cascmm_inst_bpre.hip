@@ -21,6 +21,8 @@ static const VariantDesc kTable[] = {
     CASCMM_W512_VARIANT("t256x320x32_w512_bf16x2_tri_bpre", 1),
     CASCMM_W512_EDGE_VARIANT("t256x320x32_w512_edge_bf16x2_tri_bpre", 1, 5),
     CASCMM_W512_EDGE_VARIANT("t256x256x32_w512_edge_bf16x2_tri_bpre", 1, 4),
+    CASCMM_W512_EDGE_VARIANT("t256x192x32_w512_narrow_bf16x2_tri_bpre", 1, 3),
+    CASCMM_W512_EDGE_VARIANT("t256x128x32_w512_narrow_bf16x2_tri_bpre", 1, 2),
     // K split over the eight waves of a workgroup: small problems
     CASCMM_WAVEK_VARIANT_B("t16x16x32_wavek_bf16x2_tri_bpre", 16, 1, 1, BF, 2, 1),
     CASCMM_WAVEK_VARIANT_B("t16x32x32_wavek_bf16x2_tri_bpre", 16, 1, 2, BF, 2, 1),

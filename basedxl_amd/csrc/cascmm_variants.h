@@ -227,12 +227,12 @@ template <int BPRE, int NTL>
 int launch_w512_edge(const GroupParams& p, hipStream_t stream) {
   typedef W512Tile<NTL> T;
   if (p.kernel_out) { *p.kernel_out = (const void*)cascmm_w512_kernel<BPRE, 0, NTL, 1>; return CASCMM_OK; }
-  if (p.count != 1 || p.k_splits > 1 || p.glu == 2 || (p.glu && (!BPRE || (NTL == 5 && p.N % T::BN != 0)))) return CASCMM_ERR_BAD_VARIANT;
+  if (p.count != 1 || p.k_splits > 1 || p.glu == 2 || (p.glu && (!BPRE || NTL == 3 || (NTL == 5 && p.N % T::BN != 0)))) return CASCMM_ERR_BAD_VARIANT;
   if (p.M < W512_EDGE_ROWS || p.N < T::BN || (!BPRE && p.N % 4 != 0) || p.lda % 4 != 0 || p.lda < 32) return CASCMM_ERR_BAD_VARIANT;
   if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (BPRE ? prepared_kgroups(p.K) * p.N * 32 : ((int64_t)p.K + 32) * p.ldb * 4) > 0x7FFFFFFF ||
       p.ldc * (int64_t)(T::BM * 4) > 0x7FFFFFFF)
     return CASCMM_ERR_TOO_LARGE;
-  if constexpr (BPRE) {
+  if constexpr (BPRE && NTL != 3) {
     if (p.glu) return launch_w512_kernel<BPRE, 1, NTL, 1>(p, stream);
   }
   return launch_w512_kernel<BPRE, 0, NTL, 1>(p, stream);
@@ -451,7 +451,7 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
 
 #define CASCMM_W512_EDGE_VARIANT(NAME, BPRE, NTL)                                                                         \
   {NAME, KIND_W512E, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512Tile<NTL>::BM, W512Tile<NTL>::BN, 32, W512Tile<NTL>::NT, \
-   W512Tile<NTL>::LDS_BYTES, true, false, &launch_w512_edge<BPRE, NTL>, BPRE != 0, BPRE != 0}
+   W512Tile<NTL>::LDS_BYTES, true, false, &launch_w512_edge<BPRE, NTL>, BPRE != 0, BPRE != 0 && NTL != 3, NTL <= 3}
 
 // eight producer waves, every B column loaded singly (all producer threads share A and B evenly)
 #define CASCMM_TILE_VARIANT_PS(NAME, BM, BN, BK, WM, WN, WK, DEPTH, NP, IODT, FMT, TERMS, FULL, FAST)          \

@@ -38,12 +38,15 @@ namespace cascmm {
 template <int NTL_>
 struct W512Tile {
   static constexpr int NTL = NTL_;                  // column blocks of a wave
-  static constexpr int BM = 256, BN = 64 * NTL, BK = 16, NS = 4, NT = 256;
+  static constexpr int BM = 256, BN = 64 * NTL, BK = 16, NT = 256;
+  // stages of B and pairs of stages of A in LDS: the narrower tiles' stages are shorter (24 and 36 MFMAs), so more of them are in flight
+  static constexpr int NS = NTL == 2 ? 6 : NTL == 3 ? 5 : 4, NPA = NTL <= 3 ? 3 : 2;
   static constexpr int WTM = 128, WTN = 32 * NTL, MT = 4;
   static constexpr int A_PAIR = BM * 2 * BK * 4;    // raw fp32, two stages: 128 bytes per row
   static constexpr int B_STAGE = BK * BN * 4;       // raw fp32
-  static constexpr int B_AREA = 2 * A_PAIR;         // two pairs of A, then NS stages of B
-  static constexpr int LDS_BYTES = B_AREA + NS * B_STAGE;   // 144 KB (NTL = 4: 128 KB)
+  static constexpr int B_AREA = NPA * A_PAIR;       // the pairs of A, then NS stages of B
+  static constexpr int LDS_BYTES = B_AREA + NS * B_STAGE;   // 144 KB (NTL = 4: 128 KB, 3: 156 KB)
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS");
   static constexpr int A_LOADS = 8;                 // direct loads per wave: a pair of A; a stage of B has NTL
 };
 typedef W512Tile<5> W512;
@@ -78,7 +81,11 @@ __device__ __forceinline__ void w512_in_acc(f32x16& c) { asm volatile("" : "+a"(
 __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(c)); }
 
 // NTL: column blocks of a wave; 5 is the 256 x 320 tile described above, 4 the same on 256 x 256 (sixteen blocks, all in
-// the accumulation registers).
+// the accumulation registers), 3 and 2 on 256 x 192 and 256 x 128, for problems that the wider ones leave CUs idle with: a stage has
+// 36 and 24 MFMAs, more stages are in flight, and a block splits up to two row blocks of A.  In brackets the fastest other kernel, us:
+// raw 1971 x 440 x 2624 24.8 (33.7), 7986 x 320 x 832 21.3 (26.6), 5494 x 448 x 3648 67.3 (76.8), prepared 63.8 (69.5); gated 2028 x 384 x 2432
+// 20.2 (27.0).  The loop keeps the pace of the wider tiles where the chip is full (raw 1976 x 1280 x 3840 67.1, 72.9 on the 256 x 128
+// tile of the kernels with producer waves; with the weight prepared that one stays the faster, 61 against 68).
 // EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
 // costs the loop nothing, and the stores past it go beyond the descriptor's end; the last stages may hang over K.
 // Measured (graph replay, raw / prepared weight, everything on one box: others are up to 6 % slower, see
@@ -112,8 +119,8 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 template <int BPRE, int GLU = 0, int NTL = 5, int EDGE = 0>
 __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void cascmm_w512_kernel(const GroupParams p) {
   typedef W512Tile<NTL> T;
-  static_assert(NTL == 4 || NTL == 5, "");
-  static_assert(!GLU || NTL == 5 || (GLU == 1 && BPRE && EDGE), "");
+  static_assert(NTL >= 2 && NTL <= 5, "");
+  static_assert(!GLU || NTL == 5 || (GLU == 1 && BPRE && EDGE && NTL != 3), "");
   static_assert(GLU != 2 || !EDGE, "");
   extern __shared__ __attribute__((aligned(1024))) unsigned char w512_smem[];
   unsigned char* smem = w512_smem;
@@ -170,11 +177,11 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   // operand, at an edge as well: 64 rows of 32 k and BN columns are more than 3 KB).  The second four of A and the fifth of B are
   // 4 KB further, beyond the immediate's range, and take an M0 of their own.
 #pragma unroll
-  for (int j = 1; j < 4; ++j) b_voff[j] -= j * 1024;
-  // load j of the pair of stages that starts with stage `first` (even)
-  auto issue_a = [&](int first, int j) {
+  for (int j = 1; j < (T::NTL < 4 ? T::NTL : 4); ++j) b_voff[j] -= j * 1024;
+  // load j of the pair of stages that starts with stage `first` (even), into buffer `buf`
+  auto issue_a = [&](int first, int buf, int j) {
     const int step = first < ksteps - 2 ? first : ksteps - 2;
-    const w512_lds_ptr al = (w512_lds_ptr)(smem + (first & 2) * (T::A_PAIR / 2) + wave * (T::A_LOADS * 1024) + (j >> 2) * 4096);
+    const w512_lds_ptr al = (w512_lds_ptr)(smem + buf * T::A_PAIR + wave * (T::A_LOADS * 1024) + (j >> 2) * 4096);
     const int as = step * T::BK * 4;
     // EDGE: chunks past K come from beyond the buffer, as zeros (B's rows past K do by themselves: its buffer ends there, or
     // its slots hold zeros)
@@ -186,15 +193,15 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
       default: w512_load3(ra, al, av, as); break;
     }
   };
-  auto issue_b = [&](int step_, int j) {
+  auto issue_b = [&](int step_, int buf, int j) {
     const int step = step_ < ksteps - 1 ? step_ : ksteps - 1;
-    const w512_lds_ptr bl = (w512_lds_ptr)(smem + T::B_AREA + step_ % T::NS * T::B_STAGE + wave * (T::NTL * 1024) + (j >> 2) * 4096);
+    const w512_lds_ptr bl = (w512_lds_ptr)(smem + T::B_AREA + buf * T::B_STAGE + wave * (T::NTL * 1024) + (j >> 2) * 4096);
     const int bs = step * b_step;
-    switch (j) {
-      case 1: w512_load1(rb, bl, b_voff[1], bs); break;
-      case 2: w512_load2(rb, bl, b_voff[2], bs); break;
-      case 3: w512_load3(rb, bl, b_voff[3], bs); break;
-      default: w512_load0(rb, bl, b_voff[j], bs); break;
+    switch (j & 3) {
+      case 0: w512_load0(rb, bl, b_voff[j], bs); break;
+      case 1: w512_load1(rb, bl, b_voff[j], bs); break;
+      case 2: w512_load2(rb, bl, b_voff[j], bs); break;
+      default: w512_load3(rb, bl, b_voff[j], bs); break;
     }
   };
 
@@ -222,7 +229,8 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
 #define W512_FENCE() __builtin_amdgcn_sched_barrier(0)
   u32x4 Af[2][2][T::MT];   // [buffer][hi / lo][mi]
   float R[2][8];           // raw B values of two blocks in flight
-  float RA[8];             // raw A values of one row block of the next stage
+  constexpr int RBS = T::NTL < 4 ? 2 : 1;   // row blocks of A that a block takes care of, at most
+  float RA[RBS][8];        // their raw values, of the next stage
   u32x4 H[2], L[2];        // split B of the current / next block
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   typedef float f32x2v __attribute__((ext_vector_type(2)));
@@ -246,15 +254,20 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
     lo[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
   };
 
-  // in the order in which the loop waits for them: pair 0 of A, stages 0 and 1 of B, pair 1, stage 2
+  // Stage v issues stage v + NS - 1 of B, an odd one before that the pair (v - 1) / 2 + NPA of A, whose buffer the stage before it has
+  // read last.  Here: what the stages before the first one would have issued.
 #pragma unroll
-  for (int j = 0; j < T::A_LOADS; ++j) issue_a(0, j);
+  for (int v = -2 * T::NPA; v < 0; ++v) {
+    const int pair = (v - 1) / 2 + T::NPA, sb = v + T::NS - 1;   // (v odd: v - 1 is even)
+    if (v & 1) {
 #pragma unroll
-  for (int j = 0; j < 2 * T::NTL; ++j) issue_b(j / T::NTL, j % T::NTL);
+      for (int j = 0; j < T::A_LOADS; ++j)
+        if (pair >= 0) issue_a(2 * pair, pair, j);
+    }
 #pragma unroll
-  for (int j = 0; j < T::A_LOADS; ++j) issue_a(2, j);
-#pragma unroll
-  for (int j = 0; j < T::NTL; ++j) issue_b(2, j);
+    for (int j = 0; j < T::NTL; ++j)
+      if (sb >= 0) issue_b(sb, sb, j);
+  }
   // the accumulators are cleared while the first loads are in flight: not before them, which would hold
   // the loads back, and not after the barrier, where the first MFMA would wait for it
   W512_FENCE();
@@ -274,7 +287,10 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
       else w512_in_vec(acc[mi][ni]);
     }
   W512_FENCE();
-  constexpr int W0 = T::A_LOADS + 2 * T::NTL, WEVEN = T::A_LOADS + T::NTL, WODD = T::NTL;
+  // Loads that may be in flight: what the last NS - 3 stages have issued (W0: all but pair 0 and stage 0)
+  constexpr int WEVEN = (T::NS - 3) * T::NTL + (T::NS - 2) / 2 * T::A_LOADS, WODD = (T::NS - 3) * T::NTL + (T::NS - 3) / 2 * T::A_LOADS;
+  constexpr int W0 = (T::NPA - 1) * T::A_LOADS + (T::NS - 2) * T::NTL;
+  static_assert(2 * T::NPA - 2 >= T::NS - 2, "an odd stage finds the pair of A that it waits for among the older loads");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (W0 & 0xF) | ((W0 >> 4) << 14));   // pair 0 and stage 0 have landed
   __builtin_amdgcn_s_barrier();
   {
@@ -303,17 +319,19 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
     }
   }
 
+  int sbuf = 0, pbuf = 0;   // the buffers of stage s of B and of its pair of A
+  auto stage_buf = [&](int k) { return T::NS == 4 ? (sbuf + k) & 3 : sbuf + k >= T::NS ? sbuf + k - T::NS : sbuf + k; };   // of stage s + k
   for (int s = 0; s < ksteps; s += 2) {
+    const int pnext = T::NPA == 2 ? pbuf ^ 1 : pbuf == T::NPA - 1 ? 0 : pbuf + 1;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      // top of stage s + j: the own loads of stage s + j + 1 have landed, then everybody's.  In flight: what the stage before
-      // issued, which is a stage of B (odd stages: and before it the pair of A that is read two stages later)
+      // top of stage s + j: the own loads of stage s + j + 1 have landed, then everybody's
       if (j == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (WEVEN & 0xF) | ((WEVEN >> 4) << 14));
-      else __builtin_amdgcn_s_waitcnt(0x0F70 | WODD);
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | (WODD & 0xF) | ((WODD >> 4) << 14));
       __builtin_amdgcn_s_barrier();
-      const unsigned char* st0 = smem + T::B_AREA + ((s + j) % T::NS) * T::B_STAGE;       // this stage of B
-      const unsigned char* st1 = smem + T::B_AREA + ((s + j + 1) % T::NS) * T::B_STAGE;   // the next one
-      const unsigned char* an = smem + ((s + 2 * j) & 2) * (T::A_PAIR / 2);               // the pair of A that the next stage lies in
+      const unsigned char* st0 = smem + T::B_AREA + stage_buf(j) * T::B_STAGE;       // this stage of B
+      const unsigned char* st1 = smem + T::B_AREA + stage_buf(j + 1) * T::B_STAGE;   // the next one
+      const unsigned char* an = smem + (j == 0 ? pbuf : pnext) * T::A_PAIR;          // the pair of A that the next stage lies in
 #pragma unroll
       for (int ni = 0; ni < T::NTL; ++ni) {
         const int t = j * T::NTL + ni;        // block number inside the trip: its parity is static
@@ -338,15 +356,18 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
             else w512_mfma_v(a, b, acc[mi][ni]);
           }
         };
-        // loads of a stage: NTL of B, one behind each block; the odd stages' blocks have two more slots, for the pair of A whose
-        // buffer the even stage has read last
+        // loads of a stage: NTL of B, one behind each block; the odd stages' blocks have more slots, for the pair of A
+        constexpr int SLOTS = (T::A_LOADS + 2 * T::NTL - 1) / T::NTL;   // of a block of an odd stage
         auto dl = [&](int k) {
-          if (k == 1 && j == 0) issue_b(s + T::NS - 1, ni);
-          if (j == 0) return;
-          const int slot = ni * 3 + k;
-          if (slot < T::A_LOADS) issue_a(s + 4, slot);
-          else if (slot < T::A_LOADS + T::NTL) issue_b(s + 1 + T::NS - 1, slot - T::A_LOADS);
+          if (k == 1 && j == 0) issue_b(s + T::NS - 1, stage_buf(T::NS - 1), ni);
+          if (j == 0 || k >= SLOTS) return;
+          const int slot = ni * SLOTS + k;
+          if (slot < T::A_LOADS) issue_a(s + 2 * T::NPA, pbuf, slot);
+          else if (slot < T::A_LOADS + T::NTL) issue_b(s + T::NS, stage_buf(0), slot - T::A_LOADS);
         };
+        // row blocks of A that the block reads and splits for the next stage
+        constexpr int RB_OF[4][6] = {{0, 2, 4}, {0, 2, 3, 4}, {0, 1, 2, 3, 4}, {0, 1, 2, 3, 4, 4}};
+        const int rb0 = RB_OF[T::NTL - 2][ni], rbs = RB_OF[T::NTL - 2][ni + 1] - rb0;
         // What goes between MFMA g and MFMA g + 1 of the block.  A wave alone on its SIMD issues one instruction
         // every four cycles or so, whatever its kind, and an MFMA holds the matrix pipe for 32: more than six
         // instructions in a gap leave the pipe waiting.  The sixteen half-splits of the block (three VALU
@@ -358,26 +379,38 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
         // a second one in gap 4 the block's A fragments (younger than them: the raw B reads of gaps 1 and 2)
         auto gap = [&](int gi) {
           if (gi == 0) { __builtin_amdgcn_s_waitcnt(0xC07F); W512_FENCE(); }                          // lgkmcnt(0)
-          if (gi == 4 && ni < 4) { __builtin_amdgcn_s_waitcnt(BPRE ? 0xC07F : 0xC47F); W512_FENCE(); }   // lgkmcnt(0) / lgkmcnt(4)
-          if (gi == 0 && ni < 4) {   // row block ni of the next stage
+          if (gi == 4 && rbs > 0) { __builtin_amdgcn_s_waitcnt(BPRE ? 0xC07F : 0xC47F); W512_FENCE(); }   // lgkmcnt(0) / lgkmcnt(4)
+          if (gi == 0) {   // row blocks of the next stage
             const int half = j == 0 ? 64 : 0;
-            const f32x4 x0 = *(const f32x4*)(an + (a_frag0 ^ half) + ni * 4096), x1 = *(const f32x4*)(an + (a_frag1 ^ half) + ni * 4096);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              RA[e] = x0[e];
-              RA[4 + e] = x1[e];
+            for (int x = 0; x < RBS; ++x) {
+              if (x >= rbs) continue;
+              const f32x4 x0 = *(const f32x4*)(an + (a_frag0 ^ half) + (rb0 + x) * 4096), x1 = *(const f32x4*)(an + (a_frag1 ^ half) + (rb0 + x) * 4096);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                RA[x][e] = x0[e];
+                RA[x][4 + e] = x1[e];
+              }
             }
           }
           if (!BPRE && gi == 1) read_raw(R[cur], st2, n2, 0, 4);
           if (!BPRE && gi == 2) read_raw(R[cur], st2, n2, 4, 8);
-          if (!BPRE && gi < 8) {
-            if (gi & 1) split_2(R[nxt], H[nxt], L[nxt], gi >> 1);
-            else split_1(R[nxt], H[nxt], gi >> 1);
+          if (!BPRE) {   // (two row blocks of A: both halves of a pair in each of the gaps in front of theirs)
+#pragma unroll
+            for (int h = 0; h < 8; ++h) {
+              if ((rbs == 2 ? h >> 1 : h) != gi) continue;
+              if (h & 1) split_2(R[nxt], H[nxt], L[nxt], h >> 1);
+              else split_1(R[nxt], H[nxt], h >> 1);
+            }
           }
-          if (ni < 4 && gi >= 4) {
+          if (gi >= 4) {
             const int h = gi - 4;
-            if (h & 1) split_2(RA, Af[j ^ 1][0][ni], Af[j ^ 1][1][ni], h >> 1);
-            else split_1(RA, Af[j ^ 1][0][ni], h >> 1);
+#pragma unroll
+            for (int x = 0; x < RBS; ++x) {
+              if (x >= rbs) continue;
+              if (h & 1) split_2(RA[x], Af[j ^ 1][0][rb0 + x], Af[j ^ 1][1][rb0 + x], h >> 1);
+              else split_1(RA[x], Af[j ^ 1][0][rb0 + x], h >> 1);
+            }
           }
           if (BPRE && gi == 4) read_slot_hi(nxt, stn, n1);     // seven MFMAs before the next block's first
           if (BPRE && gi == 8) read_slot_lo(nxt, stn, n1);
@@ -386,6 +419,8 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
           if (gi == 3) dl(0);
           if (gi == 9) dl(1);
           if (gi == 11) dl(2);
+          if (gi == 7) dl(3);
+          if (gi == 5) dl(4);
         };
 #pragma unroll
         for (int gi = 0; gi < 12; ++gi) {
@@ -394,6 +429,8 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
         }
       }
     }
+    sbuf = stage_buf(2);
+    pbuf = pnext;
   }
 #undef W512_FENCE
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the redundant loads of the last stages land before LDS is given up
@@ -479,12 +516,12 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
     }
     return;
   }
-  if constexpr (GLU == 1 && NTL == 4) {
-    // Gated store of the 256-wide tile: a wave's four blocks are value 0, gate 0, value 1, gate 1 of its own 64 columns.
+  if constexpr (GLU == 1 && NTL != 5) {
+    // Gated store of the 256 and 128 wide tiles: a wave's blocks are value 0, gate 0, value 1, ... of its own columns.
     const int half = p.N >> 1, rows = p.M - (m0 + wm0);
     const i32x4 re = make_rsrc((float*)p.C[0] + (int64_t)(m0 + wm0) * p.ldc, rows > 0 ? (int64_t)(rows < T::WTM ? rows : T::WTM) * ldc_bytes : 0);
 #pragma unroll
-    for (int pair = 0; pair < 2; ++pair) {
+    for (int pair = 0; pair < NTL / 2; ++pair) {
       const int col = ((n0 + wn0) >> 1) + 32 * pair + el31, read = col < half ? col : half - 1;
       const float bv = bias ? bias[read] : 0.f, bg = bias ? bias[half + read] : 0.f;
       const int voff = col < half ? eg * 4 * ldc_bytes + col * 4 : 0x7FFFFFFF;
