@@ -278,6 +278,9 @@ static const CallCost kCallCost[] = {
     {"t16x32x32_wavek_fp16x3_tri", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
     {"t32x32x32_wavek_fp16x3_tri", 2.79, 1.5, 0.319, 1.57, 60, 1, 1.62, 0, 0},
     // three fp8 terms (493 shapes, hardly ever behind the fastest; without rounds 0.6 %, at most 33 %)
+    {"t16x16x32_wavek_fp16x3_tri_scaled", 2.47, 0.728, 0.176, 0.125, 28.6, 1, 0.664, 0.051, 0},
+    {"t16x32x32_wavek_fp16x3_tri_scaled", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
+    {"t32x32x32_wavek_fp16x3_tri_scaled", 2.79, 1.5, 0.319, 1.57, 60, 1, 1.62, 0, 0},
     {"t16x16x32_wavek_fp8x3_tri", 2.54, 0.713, 0.229, 0.147, 28.1, 1, 0.655, 0.00446, 0},
     {"t16x32x32_wavek_fp8x3_tri", 2.57, 1.1, 0.207, 1.1, 26.9, 1, 1.24, 0, 0},
     {"t32x32x32_wavek_fp8x3_tri", 2.91, 1.4, 0.425, 2.04, 60, 1, 4.23, 0.0301, 0},
@@ -709,7 +712,7 @@ static int select_variant_uncached(const Problem& q, RowFit fit, int count, size
   if (best >= 0 && (t[best].kind == KIND_TILE || t[best].kind == KIND_F8K64) && few_tiles_three_terms(q, count, !t[best].fast)) {
     best_cost = 1e9;
     for (int i = 0; i < (int)t.size(); ++i) {
-      if (!wavek_three_terms(t[i]) || !variant_matches(t[i], q, fit) || variant_cost(i, q, count) >= best_cost) continue;
+      if (!wavek_three_terms(t[i]) || t[i].scaled || !variant_matches(t[i], q, fit) || variant_cost(i, q, count) >= best_cost) continue;
       best = i;
       best_cost = variant_cost(i, q, count);
       if (splits_out) *splits_out = 1;
@@ -1005,6 +1008,24 @@ static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem*
   return (fp8 ? std::max(slots + 5.0, 32.0) : slots) < 3.5 + step * rounds * (double)((q.K + 31) / 32) ? v : (int)CASCMM_ERR_BAD_FORMAT;
 }
 
+// A call that the fp16 slot kernel v would take, as e: K over eight waves on the rows as they lie, which scales its tiles itself, or -1.  (A
+// tile costs 1.15 of the unscaled kernels' time in the median of 119 shapes.)  Up to two tiles of 32 x 32 per CU: 330 tiles of 71 x 3800 x 3520
+// 97.9 us in slots, here 57.6; 286 of 341 x 3576 x 832 77.1, 55.7; beyond 389 x 1152 x 2175 41.3, 47.7; 421 x 760 x 2496 32.8, 41.3.
+static int select_scaled_rows(const Problem& q, RowFit fit, int v, const Problem& e) {
+  const auto& t = table();
+  if (v < 0 || t[v].kind != KIND_F16K || !q.call || ((q.M + 31) / 32) * ((q.N + 31) / 32) > 2 * kNumCUs) return -1;
+  int best = -1;
+  double best_cost = variant_cost(v, e, 1);
+  for (int i = 0; i < (int)t.size(); ++i) {
+    if (!t[i].scaled || !variant_matches(t[i], q, fit)) continue;
+    const double cost = 1.15 * variant_cost(i, q, 1);
+    if (cost >= best_cost) continue;
+    best = i;
+    best_cost = cost;
+  }
+  return best;
+}
+
 // The launch itself, on operands as they lie (exps_dyn, b_exp_src: see gemm_impl)
 static int gemm_on_rows(int count, const void* const* A, const void* const* B, void* const* C, const void* const* bias, const Problem& q0,
                         const int32_t* tensor_exps, void* workspace, size_t workspace_bytes, hipStream_t stream, int variant,
@@ -1032,6 +1053,7 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
   const auto& t = table();
   int splits = 1;
   if (variant < 0) {
+    const RowFit rows_fit = fit;
     if (count == 1 && !q.split_first) {
       Problem e;
       if (select_rounded_up(q, fit, workspace ? workspace_bytes : 0, &e) >= 0) {
@@ -1052,6 +1074,13 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
       return CASCMM_OK;
     }
     if (variant < 0) return none(variant);
+    if (count == 1) {
+      const int rows = select_scaled_rows(q0, rows_fit, variant, q);
+      if (rows >= 0) {
+        variant = rows;
+        q = q0;
+      }
+    }
   } else {
     splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
     variant &= 0xFFFF;
@@ -1490,8 +1519,13 @@ int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int6
   }
   const RowFit fit = row_fit(q, A, B);
   Problem e;
-  const int v = select_rounded_up(q, fit, workspace_bytes, &e);
-  return v >= 0 ? v : select_variant(q, fit, 1, workspace_bytes);
+  int v = select_rounded_up(q, fit, workspace_bytes, &e);
+  if (v < 0) {
+    e = q;
+    v = select_variant(q, fit, 1, workspace_bytes);
+  }
+  const int rows = select_scaled_rows(q, fit, v, e);
+  return rows >= 0 ? rows : v;
 }
 
 int cascmm_call_variant_prepared(const void* A, int glu, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int dtype, int fmt,

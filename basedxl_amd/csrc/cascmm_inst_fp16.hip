@@ -21,6 +21,10 @@ static const VariantDesc kTable[] = {
     CASCMM_WAVEK_VARIANT("t16x16x32_wavek_fp16x3_tri", 16, 1, 1, FP, 3),
     CASCMM_WAVEK_VARIANT("t16x32x32_wavek_fp16x3_tri", 16, 1, 2, FP, 3),
     CASCMM_WAVEK_VARIANT("t32x32x32_wavek_fp16x3_tri", 16, 2, 2, FP, 3),
+    // the same in the place of the kernels below
+    CASCMM_WAVEK_SCALED_VARIANT("t16x16x32_wavek_fp16x3_tri_scaled", 16, 1, 1),
+    CASCMM_WAVEK_SCALED_VARIANT("t16x32x32_wavek_fp16x3_tri_scaled", 16, 1, 2),
+    CASCMM_WAVEK_SCALED_VARIANT("t32x32x32_wavek_fp16x3_tri_scaled", 16, 2, 2),
     // both operands split into pre-scaled operand slots first (cascmm_f16k_kernel.h)
     CASCMM_F16K_VARIANT("t256x160x32_f16k_fp16x3_tri", false),
     CASCMM_F16K_VARIANT("k64x160x32_f16wk4_fp16x3_tri", true),

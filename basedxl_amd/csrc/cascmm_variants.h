@@ -74,6 +74,7 @@ struct VariantDesc {
   bool bpre = false;  // takes the right operand already split (cascmm_prepare_weight)
   bool glu = false;   // has the gated epilogue
   bool call_only = false;   // chosen for calls only: the selection functions, which answer for a shape, leave it out
+  bool scaled = false;      // takes the calls of the slot kernels (cascmm_wavek_kernel.h, SCALED)
 };
 
 template <class TL, int IODT, int FMT, int TERMS, bool FULL, bool FAST, bool BPRE = false>
@@ -257,6 +258,20 @@ int launch_wavek_kernel(const GroupParams& p, hipStream_t stream) {
   const int64_t grid = (int64_t)q.count * q.tiles_m * q.tiles_n;
   if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
   return launch_kernel(kfn, dim3((unsigned)grid), dim3(512), (size_t)lds, stream, q) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
+}
+// (SCALED: the bounds-checked form only, and eight words more of LDS)
+template <int W, int MB, int NB>
+int launch_wavek_scaled(const GroupParams& p, hipStream_t stream) {
+  auto kfn = cascmm_wavek_kernel<W, MB, NB, W * MB / 8, 1, CASCMM_FMT_FP16, 3, 0, 0, 1>;
+  if (p.kernel_out) { *p.kernel_out = (const void*)kfn; return CASCMM_OK; }
+  if (p.glu || p.k_splits > 1 || p.count < 1 || p.K <= 0) return CASCMM_ERR_BAD_VARIANT;
+  if ((int64_t)p.M * p.lda * 4 > 0x7FFFFFFF || (int64_t)p.K * p.ldb * 4 > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
+  constexpr int lds = WaveKOf<W, MB, NB, W * MB / 8, CASCMM_FMT_FP16, 3, 0>::LDS_BYTES + 32;
+  static LdsFlags lds_set;
+  if (!ensure_lds((const void*)kfn, lds, lds_set)) return CASCMM_ERR_LAUNCH;
+  const int64_t grid = (int64_t)p.count * p.tiles_m * p.tiles_n;
+  if (grid <= 0 || grid > 0x7FFFFFFF) return CASCMM_ERR_TOO_LARGE;
+  return launch_kernel(kfn, dim3((unsigned)grid), dim3(512), (size_t)lds, stream, p) == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
 }
 template <int W, int MB, int NB, int FMT, int TERMS, int BPRE>
 int launch_wavek(const GroupParams& p, hipStream_t stream) {
@@ -444,6 +459,9 @@ int launch_f16k(const GroupParams& p, hipStream_t stream) {
    WaveKOf<W, MB, NB, W * MB / 8, FMT, TERMS, BPRE>::LDS_BYTES, true, true, &launch_wavek<W, MB, NB, FMT, TERMS, BPRE>, BPRE != 0, \
    BPRE && W == 16 && NB == 4, BPRE || FMT != CASCMM_FMT_BF16 || !wavek_for_shapes(W * MB, W * NB)}
 #define CASCMM_WAVEK_VARIANT(NAME, W, MB, NB, FMT, TERMS) CASCMM_WAVEK_VARIANT_B(NAME, W, MB, NB, FMT, TERMS, 0)
+#define CASCMM_WAVEK_SCALED_VARIANT(NAME, W, MB, NB)                                                                       \
+  {NAME, KIND_WAVEK, CASCMM_DT_F32, CASCMM_FMT_FP16, 3, false, W * MB, W * NB, 32, 512,                                    \
+   WaveKOf<W, MB, NB, W * MB / 8, CASCMM_FMT_FP16, 3, 0>::LDS_BYTES + 32, true, true, &launch_wavek_scaled<W, MB, NB>, false, false, true, true}
 
 #define CASCMM_W512_VARIANT(NAME, BPRE)                                                                             \
   {NAME, KIND_W512, CASCMM_DT_F32, CASCMM_FMT_BF16, 2, false, W512::BM, W512::BN, 32, W512::NT, W512::LDS_BYTES, true, \

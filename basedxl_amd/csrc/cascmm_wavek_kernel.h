@@ -30,7 +30,7 @@
 #pragma once
 #include <type_traits>
 
-#include "cascmm_tile_kernel.h"
+#include "cascmm_f16k_kernel.h"
 
 namespace cascmm {
 
@@ -103,6 +103,18 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
   else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
 }
 
+// Three fp16 terms on values as they are: what the largest element of an operand has to reach.  The terms resolve 2^-46 then, 2^-33 of
+// that element; the products that are left out are 2^-33 of a product too, and the roundings of the sums 2^-24.
+constexpr short kWaveKLeast = 0x0800;   // 2^-13
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void wavek_top(s16x2& top, const u32x4& t) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) top = __builtin_elementwise_max(top, __builtin_bit_cast(s16x2, (unsigned)t[d]));
+}
+__device__ __forceinline__ bool wavek_seen(const s16x2& top) {
+  return (short)(top[0] & 0x7FFF) >= kWaveKLeast || (short)(top[1] & 0x7FFF) >= kWaveKLeast;
+}
+
 // A's rows in a stage: position pos of row r holds chunk (pos - wavek_rot(r / 2)) mod 8 (16-row blocks: the rotations of
 // cascmm_slotn_kernel.h, which explains them)
 template <int W>
@@ -136,9 +148,18 @@ using WaveKOf = WaveK<W, MB, NB, AL, BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W /
 // AL < W MB / 8: only the first 8 AL rows of A are fetched (M <= 8 AL), the lanes of the others read those again.
 // BPRE = 1: B is a prepared weight, [plane][4 ceil(K/32)][N] operand slots, a load per plane and column block (block nb: columns
 // W nb + c).  GLU = 1 (prepared, 64-wide tiles): the gated store, C has N / 2 columns, B alternates 32 value and 32 gate columns.
-template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0>
+// SCALED = 1 (three fp16 terms, raw): for the calls of the slot kernels (cascmm_f16k_kernel.h), which find the maxima of both operands and
+// scale them before they split, in launches of their own.  Here a tile is computed on the values as they are; where a value of its rows
+// of A or columns of B left fp16's range (a sum is then not finite), or all of A's or of B's lie below kWaveKLeast (the terms would be
+// coarse), the same workgroup reads its operands' maxima and computes the tile again, scaled: once more for the tiles concerned,
+// nothing but a packed maximum per two elements for the others.  Three launches and the slots' trip through memory are saved, and the
+// tiles are small (us, graph replay, before: on 64 x 160 slot tiles): 5 x 3164 x 3136 80.9, here 16.2; 33 x 1612 x 1374 47.3, 12.9; 223 x
+// 1400 x 1024 43.7, 15.3; 71 x 3800 x 3520 97.9, 57.6; with every tile computed twice 45.7, 39.2, 44.1 and 161.  Errors against 64 bits:
+// 1.1 to 7.2 1e-9 (rms, of the sum of magnitudes), 6.1e-9 to 1.2e-8 in slots.
+template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0, int SCALED = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
   static_assert(!GLU || (BPRE && W == 16 && NB == 4), "a value block and its gate block in one tile");
+  static_assert(!SCALED || (FMT == CASCMM_FMT_FP16 && TERMS == 3 && !BPRE && TAIL), "for the calls of the slot kernels");
   typedef WaveKOf<W, MB, NB, AL, FMT, TERMS, BPRE> T;
   typedef Lowp<FMT> L;
   constexpr int KM = T::KM, HALVES = T::HALVES, REGS = T::REGS;
@@ -252,8 +273,14 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       scale_out = __builtin_ldexpf(1.f, -(ea + eb));
     }
   }
-  auto step = [&](int i, auto U) {
+  // SCALED: of A, and of the columns of B, the largest leading term that a lane has seen (as 16-bit integers: the largest positive one,
+  // or the negative one of largest magnitude where there is no other)
+  s16x2 top_a = {-32768, -32768}, top_b[SCALED ? NB : 1];
+#pragma unroll
+  for (int nb = 0; nb < (SCALED ? NB : 1); ++nb) top_b[nb] = top_a;
+  auto step = [&](int i, auto U, auto again) {
     constexpr int u = decltype(U)::value;
+    constexpr bool kAgain = decltype(again)::value;
     const unsigned char* stp = ring + u * T::A_STAGE;
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
@@ -268,7 +295,12 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 #pragma unroll
           for (int e = 0; e < 8; ++e) xa[e] = e < left ? xa[e] : 0.f;
         }
+        if constexpr (kAgain) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xa[e] *= scale_a;
+        }
         split8<FMT, TERMS>(xa, ta[mb], scale_a);
+        if constexpr (SCALED && !kAgain) wavek_top(top_a, ta[mb][0]);
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -280,7 +312,12 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           float xb[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
+          if constexpr (kAgain) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xb[e] *= scale_b;
+          }
           split8<FMT, TERMS>(xb, tb, scale_b);
+          if constexpr (SCALED && !kAgain) wavek_top(top_b[nb], tb[0]);
         }
         // smallest products first
 #pragma unroll
@@ -321,7 +358,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (u + NS - 1 < S) issue(u + NS - 1, (u + NS - 1) % NS);
         wavek_wait_loads<younger * L1>();
-        step(u, std::integral_constant<int, u % NS>{});
+        step(u, std::integral_constant<int, u % NS>{}, std::false_type{});
       });
     }
   });
@@ -333,7 +370,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         constexpr int u = decltype(U)::value;
         issue(i + u + NS - 1, (u + NS - 1) % NS);
         wavek_wait_loads<(NS - 1) * L1>();
-        step(i + u, U);
+        step(i + u, U, std::false_type{});
       });
       fold();
     }
@@ -342,7 +379,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
                                constexpr int u = decltype(U)::value;
                                __builtin_amdgcn_sched_barrier(0);
                                wavek_wait_loads<(NS - 2 - u) * L1>();
-                               step(i + u, U);
+                               step(i + u, U, std::false_type{});
                              });
   }
   fold();
@@ -351,21 +388,100 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 
   // ---- the eight partial tiles meet in LDS: [wave][mb][nb][reg][lane] fp32 -------------------------
   float* part = (float*)wavek_smem;
+  // (SCALED: false where a sum of a column that exists is not finite)
+  auto leave = [&]() {
+    bool finite = true;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int e = 0; e < REGS; ++e) {
-        float v = acc[CL - 1][mb][nb][e];
-        if constexpr (CL > 1) {
+        for (int e = 0; e < REGS; ++e) {
+          float v = acc[CL - 1][mb][nb][e];
+          if constexpr (CL > 1) {
 #pragma unroll
-          for (int c = CL - 2; c >= 0; --c) v = __builtin_fmaf(v, AccClasses<FMT, TERMS, false>::kFoldScale, acc[c][mb][nb][e]);
+            for (int c = CL - 2; c >= 0; --c) v = __builtin_fmaf(v, AccClasses<FMT, TERMS, false>::kFoldScale, acc[c][mb][nb][e]);
+          }
+          if constexpr (kFold) v += master[mb][nb][e];
+          if constexpr (SCALED) finite = finite && (__builtin_fabsf(v) < __builtin_inff() || n0 + NB * lw + nb >= p.N);
+          part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
         }
-        if constexpr (kFold) v += master[mb][nb][e];
-        part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
-      }
+    return finite;
+  };
+  const bool finite = leave();
+  unsigned* word = (unsigned*)(wavek_smem + T::LDS_BYTES);   // (SCALED: eight words behind the tiles)
+  if constexpr (SCALED) {
+    bool seen_b = false;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) seen_b = seen_b || (n0 + NB * lw + nb < p.N && wavek_seen(top_b[nb]));
+    const unsigned mine = (__any(wavek_seen(top_a)) ? 1u : 0u) | (__any(seen_b) ? 2u : 0u) | (__any(!finite) ? 4u : 0u);
+    if (lane == 0) word[wave] = mine;
+  }
   __syncthreads();
+  if constexpr (SCALED) {
+    unsigned all = 0;
+#pragma unroll
+    for (int w = 0; w < T::NW; ++w) all |= word[w];
+    if (__builtin_amdgcn_readfirstlane(all) != 3) {
+      __syncthreads();
+      if (tid < 2) word[tid] = 0;
+      __syncthreads();
+      // the largest finite elements of the tile's rows of A and columns of B (rows past the last one: that one again)
+      unsigned best = 0;
+      const auto look = [&](float x) {
+        const unsigned bits = __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu;
+        best = bits < 0x7F800000u && bits > best ? bits : best;
+      };
+      for (int k = tid; k < p.K; k += T::NT) {
+        float x[T::BM];
+#pragma unroll
+        for (int r = 0; r < T::BM; ++r) x[r] = ((const float*)pa)[(int64_t)(m0 + r < p.M ? m0 + r : p.M - 1) * p.lda + k];
+#pragma unroll
+        for (int r = 0; r < T::BM; ++r) look(x[r]);
+      }
+      atomicMax(&word[0], best);
+      best = 0;
+      constexpr int ROWS = T::NT / T::BN, U = 16;
+      const float* col = (const float*)pb + (n0 + tid % T::BN < p.N ? n0 + tid % T::BN : p.N - 1);
+      for (int k = tid / T::BN; k < p.K; k += ROWS * U) {
+        float x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = col[(int64_t)(k + u * ROWS < p.K ? k + u * ROWS : p.K - 1) * p.ldb];
+#pragma unroll
+        for (int u = 0; u < U; ++u) look(x[u]);
+      }
+      atomicMax(&word[1], best);
+      __syncthreads();
+      const int ea = f16k_exp_of_amax(word[0]), eb = f16k_exp_of_amax(word[1]);
+      scale_a = __builtin_ldexpf(1.f, ea);
+      scale_b = __builtin_ldexpf(1.f, eb);
+      scale_out = __builtin_ldexpf(1.f, -(ea + eb));
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+          for (int c = 0; c < CL; ++c) acc[c][mb][nb] = zero;
+          if constexpr (kFold) master[mb][nb] = zero;
+        }
+      // (steps past the last one add products of zeros)
+      __builtin_amdgcn_sched_barrier(0);
+      wavek_each<NS - 1>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+      for (int i = 0; i < my_steps; i += NS) {
+        wavek_each<NS>([&](auto U) {
+          constexpr int u = decltype(U)::value;
+          issue(i + u + NS - 1, (u + NS - 1) % NS);
+          wavek_wait_loads<(NS - 1) * L1>();
+          step(i + u, U, std::true_type{});
+        });
+        fold();
+      }
+      wavek_wait_loads<0>();
+      __syncthreads();
+      leave();
+      __syncthreads();
+    }
+  }
   // thread -> (mb, nb, reg, lane) positions tid, tid + 512, ...; of a block a lane holds column lw, rows 4 kg + reg (of 32
   // rows: 8 (reg / 4) + 4 kg + reg % 4)
   float* C = (float*)pc;
@@ -401,7 +517,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     float sum = 0.f;
 #pragma unroll
     for (int w = 0; w < T::NW; ++w) sum += part[((w * MB * NB + blk) * REGS + e) * 64 + ln];
-    if constexpr (kScaled8) sum *= scale_out;
+    if constexpr (kScaled8 || SCALED) sum *= scale_out;
     if (row < p.M && (!TAIL || col < p.N)) C[(int64_t)row * p.ldc + col] = sum + (bias ? bias[col] : 0.f);
   }
 }

@@ -1,0 +1,74 @@
+"""Three fp16 terms of few rows whose K or N fits no whole stages: K over the eight waves, each tile scaled by its own workgroup where
+its values need it, in the place of the slot kernels, which scale both operands in launches of their own."""
+import pytest
+import torch
+
+from basedxl_amd import _lib, cascaded_lowp_matmul
+
+NAMES = [n for n in _lib.variant_names() if n.endswith("_scaled")]
+SHAPES = [(1, 33, 5), (17, 100, 47), (33, 1193, 70), (5, 2570, 129)]
+
+
+def test_few_rows_take_the_kernel_that_scales_its_own_tiles():
+    l, names = _lib.lib(), _lib.variant_names()
+
+    def kernel(M, K, N, lda=None):
+        lda = lda or K
+        return names[l.cascmm_call_variant(1 << 40, 2 << 40, M, N, K, lda, N, N, 0, 1, 3, 0, l.cascmm_workspace_bytes(M, N, K, 0, 1, 3, 0)) & 0xFFFF]
+
+    for shape in ((5, 3164, 3136), (6, 1193, 462), (33, 1612, 1374)):
+        assert kernel(*shape).endswith("_scaled"), shape
+    for shape in ((882, 899, 3968), (300, 576, 4480), (2048, 1281, 1280)):
+        assert "_wavek_" not in kernel(*shape), shape
+
+
+def _check(a, b, c, bias=None):
+    """Each of a wave's sums over K / 256 steps is rounded once per MFMA and folded in blocks, the waves' eight are added: below 16 + K / 256
+    roundings of 2^-24 of the sum of magnitudes; the terms hold an operand to 2^-36 of the largest element of its tile (tiles of 32 at most)."""
+    ad, bd = a.double(), b.double()
+    ref = ad @ bd + (0 if bias is None else bias.double())
+    K = a.shape[1]
+    mag = ad.abs() @ bd.abs()
+    tile_a = torch.cat([r.abs().amax().expand(r.shape[0]) for r in ad.split(32)])[:, None]
+    tile_b = torch.cat([r.abs().amax().expand(r.shape[1]) for r in bd.split(32, 1)])[None, :]
+    bound = (16 + K / 256) * 2.0 ** -24 * mag + 2.0 ** -36 * (tile_a * bd.abs().sum(0)[None, :] + tile_b * ad.abs().sum(1)[:, None])
+    bad = ~((c.double() - ref).abs() <= bound + ref.abs() * 2.0 ** -23)
+    assert not bad.any(), float(((c.double() - ref).abs() / bound).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_scaled_rows(M, K, N, name):
+    print(name, M, K, N, flush=True)
+    v = _lib.variant_names().index(name)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, b = (torch.randn(s, device="cuda", generator=g) for s in ((M, K), (K, N)))
+    bias = torch.randn(N, device="cuda", generator=g)
+
+    def run(x, y, **kw):
+        return cascaded_lowp_matmul(x, y, lowp="fp16", terms=3, variant=v, **kw)
+
+    # as they are; beyond fp16's range; below what its terms hold; both; rows of A that lie apart
+    _check(a, b, run(a, b, bias=bias), bias)
+    for ea, eb in ((40, -30), (0, 17), (-25, 0), (-50, 55)):
+        _check(a * 2.0 ** ea, b * 2.0 ** eb, run(a * 2.0 ** ea, b * 2.0 ** eb))
+    wide = torch.full((M, K + 3), 1.0e30, device="cuda")
+    wide[:, :K] = a
+    _check(a, b, run(wide[:, :K], b))
+    # operands without a positive element, of zeros, of whole numbers
+    _check(-a.abs(), -b.abs(), run(-a.abs(), -b.abs()))
+    assert not run(torch.zeros_like(a), b).any() and not run(a, torch.zeros_like(b)).any()
+    ia, ib = (a * 8).round(), (b * 8).round()
+    assert torch.equal(run(ia, ib).double(), ia.double() @ ib.double())
+    # one element out of range in a row of each 32, the last column of B not finite
+    big, nan = a.clone(), b.clone()
+    big[::32, K - 1] = 3.0e6
+    _check(big, b, run(big, b))
+    nan[0, N - 1] = float("nan")
+    inf = a.clone()
+    inf[M - 1, K // 2] = float("inf")
+    c = run(inf, nan)
+    assert not torch.isfinite(c[M - 1]).any() and torch.isnan(c[:, N - 1]).all()
+    if M > 1:
+        _check(inf[:M - 1], nan[:, :N - 1], c[:M - 1, :N - 1])
