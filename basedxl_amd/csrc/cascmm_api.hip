@@ -622,12 +622,14 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
 // 28.6; 788 x 659 x 818 bounds-checked 35.0, 23.0), 2 % behind the fastest of all; beyond: 391 x 384 x 1984 13.6, here 16.7; 96 x 2048 x 8192
 // 41.0, 45.3 (eager); 1136 x 3200 x 256 42.8, 44.9.
 // fp8: in the place of the slot kernels too (all scale by the same exponents), whose passes it does without, up to one tile per CU: 0.56 of the
-// time (2 x 1280 x 1280 11.7, here 6.3; 18 x 2688 x 384 20.4, 10.3); beyond, the fp8-rate instruction wins: 391 x 384 x 1984 11.8, here 17.3; 222 x 4352 x
-// 704 27.4, 28.1.
+// time (2 x 1280 x 1280 11.7, here 6.3; 18 x 2688 x 384 20.4, 10.3), for 16 rows up to 400 tiles (2 x 320 x 10240 14.8, 10.9; 16 x 1280 x 12800
+// 32.7, 23.6); beyond, the fp8-rate instruction wins: 391 x 384 x 1984 11.8, here 17.3; 222 x 4352 x 704 27.4, 28.1.  Deep K, of few tiles: 4 x
+// 4372 x 1728 50.4, 21.6; 8 x 8192 x 2048 48.0, 31.3; 40 x 6144 x 1280 39.7, 27.9; but 154 x 10240 x 640 43.5, here 52.1; 20 x 20480 x 1280 74.6,
+// 84.6; 64 x 8192 x 2560 49.6, 56.2.
 static bool wavek_three_terms(const VariantDesc& v) { return v.kind == KIND_WAVEK && v.terms == 3; }
 static bool few_tiles_three_terms(const Problem& q, int count, bool bounds_checked) {
   const int64_t tiles = (int64_t)count * ((q.M + 31) / 32) * ((q.N + 31) / 32);
-  if (q.fmt == CASCMM_FMT_FP8) return tiles <= kNumCUs && q.K <= 4096;
+  if (q.fmt == CASCMM_FMT_FP8) return q.K > 4096 ? tiles * q.K <= 640 * 1024 : tiles <= (q.M <= 16 ? 400 : kNumCUs);
   return tiles <= (bounds_checked ? 3 : q.K <= 2048 ? 2 : 1) * kNumCUs;
 }
 
