@@ -67,6 +67,7 @@ SIGNATURES = {
     "cascmm_probe_stream": (c_int, [c_void_p, c_void_p, c_size_t, c_int, c_void_p, c_size_t, c_void_p]),
     "cascmm_tensor_exp": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p]),
     "cascmm_tensor_exps": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "cascmm_gate": (c_int, [c_void_p, c_void_p] + [c_int64] * 4 + [c_int, c_void_p]),
     "cascmm_gemm_fp8_autoscale": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int64] * 6 + [c_int, c_int]
                                   + [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "cascmm_split_terms": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p]),

@@ -569,6 +569,22 @@ def gated_variant(a: torch.Tensor, b: torch.Tensor, *, lowp: Optional[str] = Non
                                                 terms, _lib.PROD_BY_NAME[products])
 
 
+def gate_product(h: torch.Tensor) -> torch.Tensor:
+    """``value * gelu(gate)`` of ``h = [value | gate]``, a product of this library, in one kernel (erf form, in fp32, rounded once)."""
+    inner = h.shape[-1] // 2
+    h2 = _rows(h.reshape(-1, h.shape[-1]))
+    out = torch.empty(*h.shape[:-1], inner, dtype=h.dtype, device=h.device)
+    if out.numel() == 0:
+        return out
+    if out.numel() >= 2 ** 32 - 4096:      # (the kernel's numbers have 32 bits)
+        value, gate = h.chunk(2, dim=-1)
+        return value * torch.nn.functional.gelu(gate)
+    with torch.cuda.device(h.device):
+        _lib.check(_lib.lib().cascmm_gate(h2.data_ptr(), out.data_ptr(), h2.shape[0], inner, h2.stride(0) if h2.shape[0] > 1 else 2 * inner, inner, _DTYPES[h.dtype],
+                                          torch.cuda.current_stream(h.device).cuda_stream), "cascmm_gate")
+    return out
+
+
 def cascaded_lowp_matmul_glu(a: torch.Tensor, b: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
                              out: Optional[torch.Tensor] = None, lowp: Optional[str] = None, terms: Optional[int] = None,
                              products: str = "tri", variant: int = -1) -> torch.Tensor:

@@ -8,6 +8,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "cascmm_gate_kernel.h"
 #include "cascmm_variants.h"
 
 namespace cascmm {
@@ -1623,6 +1624,21 @@ int cascmm_tensor_exps(const void* x, int64_t rows, int64_t cols, int64_t ld, in
   else
     CASCMM_LAUNCH(err, (amax_single_launch_kernel<CASCMM_DT_BF16>), dim3(grid), dim3(1024), 0, s, x, rows, cols, ld, second_exp,
                        exps_out, (unsigned*)scratch);
+  return err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
+}
+
+int cascmm_gate(const void* h, void* out, int64_t rows, int64_t inner, int64_t ldh, int64_t ldo, int dtype, void* stream) {
+  if (dtype != CASCMM_DT_F32 && dtype != CASCMM_DT_F16 && dtype != CASCMM_DT_BF16) return CASCMM_ERR_BAD_DTYPE;
+  if (rows < 0 || inner < 0 || ldh < 2 * inner || ldo < inner) return CASCMM_ERR_BAD_SHAPE;
+  if (rows == 0 || inner == 0) return CASCMM_OK;
+  if (!h || !out) return CASCMM_ERR_NULL_POINTER;
+  if (!aligned_to(h, dtype_size(dtype)) || !aligned_to(out, dtype_size(dtype))) return CASCMM_ERR_ALIGNMENT;
+  // (the kernel counts a row's elements, and all runs, in 32 bits, in steps of 256 past the last)
+  if (inner > INT32_MAX || rows > INT32_MAX || rows * inner > (int64_t)UINT32_MAX - 4096) return CASCMM_ERR_TOO_LARGE;
+  const hipStream_t s = (hipStream_t)stream;
+  const hipError_t err = dtype == CASCMM_DT_F32   ? launch_gate<CASCMM_DT_F32>(h, ldh, out, ldo, rows, inner, s)
+                         : dtype == CASCMM_DT_F16 ? launch_gate<CASCMM_DT_F16>(h, ldh, out, ldo, rows, inner, s)
+                                                  : launch_gate<CASCMM_DT_BF16>(h, ldh, out, ldo, rows, inner, s);
   return err == hipSuccess ? CASCMM_OK : CASCMM_ERR_LAUNCH;
 }
 

@@ -15,7 +15,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import _lib
-from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, cascaded_lowp_matmul_glu, default_cascade, gated_variant
+from ..cascaded_lowp_matmul import PreparedWeight, cascaded_lowp_matmul, cascaded_lowp_matmul_glu, default_cascade, gate_product, gated_variant
 
 
 class BasedXLLowPGEGLU(nn.Module):
@@ -27,7 +27,7 @@ class BasedXLLowPGEGLU(nn.Module):
     (pre-split, column-interleaved) copy of the weight, made on first use.  ``prepared=False`` keeps
     no such copy: the large-tile kernel applies the gate on the raw weight where it takes the problem
     (fp32, two bf16 terms, rows % 256 == 0, inner % 160 == 0).  Anything else runs the cascade GEMM on the
-    raw weight followed by torch's gate (the same arithmetic in three kernels)."""
+    raw weight followed by a kernel that applies the gate (the same arithmetic in two kernels)."""
 
     def __init__(self, proj: nn.Linear, *, lowp: Optional[str] = None, terms: Optional[int] = None,
                  products: str = "tri", prepared: Optional[bool] = None):
@@ -85,6 +85,4 @@ class BasedXLLowPGEGLU(nn.Module):
             x2 = x.reshape(-1, self.in_features)
             if self._prepared.usable_with(x2 if x2.stride(-1) == 1 else x2.contiguous(), self.products):
                 return cascaded_lowp_matmul(x, self._prepared, bias=self.bias, products=self.products)
-        h = cascaded_lowp_matmul(x, self.weight, bias=self.bias, lowp=self.lowp, terms=self.terms, products=self.products)
-        value, gate = h.chunk(2, dim=-1)
-        return value * F.gelu(gate)
+        return gate_product(cascaded_lowp_matmul(x, self.weight, bias=self.bias, lowp=self.lowp, terms=self.terms, products=self.products))

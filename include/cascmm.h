@@ -300,6 +300,11 @@ int cascmm_tensor_exp(const void* x, int64_t rows, int64_t cols, int64_t ld, int
 int cascmm_tensor_exps(const void* x, int64_t rows, int64_t cols, int64_t ld, int dtype,
                        const int32_t* second_exp, int32_t* exps_out, int32_t* scratch, void* stream);
 
+/* The gate of a gated projection as a pass of its own, where no kernel stores the product gated: out [rows, inner] =
+ * value * gelu(gate) of h [rows, 2 * inner] = [value | gate] (erf form, in fp32, rounded once), leading dimensions
+ * ldh >= 2 * inner and ldo >= inner in elements.  One kernel in place of gelu and product. */
+int cascmm_gate(const void* h, void* out, int64_t rows, int64_t inner, int64_t ldh, int64_t ldo, int dtype, void* stream);
+
 /* A three-term (or any) fp8 GEMM on fp32 tensors that finds the scale of its left operand itself:
  * the same result, bit for bit, as cascmm_tensor_exps(A, ..., b_exp, exps_out, scratch) followed by
  * cascmm_gemm (b_prepared == 0) or cascmm_gemm_prepared with count 1 (b_prepared != 0: B is a buffer
