@@ -630,7 +630,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
 static bool wavek_three_terms(const VariantDesc& v) { return v.kind == KIND_WAVEK && v.terms == 3; }
 static bool few_tiles_three_terms(const Problem& q, int count, bool bounds_checked) {
   const int64_t tiles = (int64_t)count * ((q.M + 31) / 32) * ((q.N + 31) / 32);
-  if (q.fmt == CASCMM_FMT_FP8) return q.K > 4096 ? tiles * q.K <= 640 * 1024 : tiles <= (q.M <= 16 ? 400 : kNumCUs);
+  if (q.fmt == CASCMM_FMT_FP8) return q.K > 4096 ? tiles <= 640 * 1024 / q.K : tiles <= (q.M <= 16 ? 400 : kNumCUs);
   return tiles <= (bounds_checked ? 3 : q.K <= 2048 ? 2 : 1) * kNumCUs;
 }
 
