@@ -13,13 +13,13 @@
 //
 // What bounds it: one product per element leaves three times fewer MFMA cycles per byte than the two-term
 // cascade, so a tile is as good as its bytes per multiply-add: (BM + BN) x 2 bytes per k through the CU's share
-// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared, graph replay in the steady state, two boxes;
-// in brackets the copy-only LDS kernels with producer waves that these replaced, on another one): 2048 x 1280 x 10240 on
-// 256 x 320 57.4 and 59.5 us (62.1; 52.1 here on that box), its loop at the board's power with random operands (zeros: a
-// third faster); 4096^3 on 256 x 256 115 and 119 us (135); 8192 x 2560 x 640 on 128 x 160 27.8 and 29.4 us (33.5); 2048^3 on
-// 128 x 128 18.8 and 21.2 us (23.0), its loop at 66 bytes per ns and CU from the L2s; 2048 x 1280 x 1280 11.2 us (14.0);
-// 512 x 1280 x 1280 on 64 x 64 6.5 us (9.5).  With B raw (no re-lay pass: 2048^3 20.7 and 21.8 us, 28.7 with it) the transposing
-// reads cost 3 - 16 %.  Kernel times and counters: profiles/cascmm_h16_kernel_fp16.txt.
+// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared / raw, graph replay, all on one box, others are up to a
+// tenth faster; in brackets before rows of A came in whole lines, sums stayed in place and fragments were read earlier): 2048 x 1280 x
+// 10240 on 256 x 320 52.3 / 52.8 us (62.4 / 64.4), its loop at the board's power with random operands (zeros: a third faster); 4096^3 on
+// 256 x 256 115.3 / 114.4 us (121.4 / 123.2); 8192 x 2560 x 640 33.7 / 34.3 us (33.7 / 35.0); 2048^3 on 128 x 128 22.3 / 22.6 us (22.6 /
+// 23.7), its loop at 66 bytes per ns and CU from the L2s; 2048 x 1280 x 1280 13.3 / 14.0 us (13.5 / 15.0); 512 x 1280 x 1280 on 64 x 64 8.2 /
+// 9.0 us (8.4 / 9.5); gated 2048 x 1280 x 10240 56.2 (60.2), 8192 x 640 x 5120 66.1 (69.6).  Kernel times and counters of the earlier state:
+// profiles/cascmm_h16_kernel_fp16.txt.
 //
 // The MFMAs take their operands swapped (B first): a lane then holds ONE ROW of C and four consecutive columns
 // per register quad, which are packed to 8 bytes, turned row-wise through LDS and stored 16 bytes per lane.
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
     b_frag[0] = T::B_AREA + wk * b_slice + (g * T::BN + wn0 + l31) * 16;
   }
   // How many slices ahead fragments are read: a slice of few MFMAs is over before the next one's are there.  Two on 128 x 128 (loop of 2048^3
-  // 23.7 -> 23.0 k cycles); the smaller tiles gained nothing (512 x 1280 x 1280 on 64 x 64 8.4 -> 8.6 us), the larger ones have MFMAs
+  // 23.7 -> 23.0 k cycles); the smaller tiles gained nothing, the larger ones have MFMAs
   // enough, and raw, the reads written as assembly must not be in flight where the loop closes.
   constexpr int PF = !T::PAIR && T::WK == 1 && !RAWB && T::MT * T::NTL == 4 ? 2 : 1;
   u32x4 Af[2 * PF][T::MT], Bf[2 * PF][T::NTL];
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
         __builtin_amdgcn_s_barrier();
         H16_FENCE();
       }
-      // behind the MFMAs of a slice: first the fragment reads of the next one, then this slice's share of the loads
+      // between the MFMAs of a slice: first the fragment reads of the next one, then this slice's share of the loads
       constexpr int READS = T::MT + T::NTL, MF = T::MT * T::NTL, PB = P[Before::value], WB = WIN[Before::value];
       const int l0 = late ? (x - FIRST) * P[ODD] / PF : PB + x * (WB - PB) / FIRST, l1 = late ? (x - FIRST + 1) * P[ODD] / PF : PB + (x + 1) * (WB - PB) / FIRST;
       // gaps that take the reads.  Of four, the first two: spread over all of them the last one is waited for (loop of 2048^3 on 128 x 128
@@ -282,11 +282,16 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
 #pragma unroll
       for (int mf = 0; mf < MF; ++mf) {
         const int ni = mf / T::MT, mi = mf % T::MT;
-        if (mi * T::NTL + ni < 16)
-          acc[mi][ni] = Lowp<FMT>::mfma(Lowp<FMT>::operand(Bf[buf][ni], 0), Lowp<FMT>::operand(Af[buf][mi], 0), acc[mi][ni]);
-        else
-          h16_mfma_v<FMT>(Bf[buf][ni], Af[buf][mi], acc[mi][ni]);
-        H16_FENCE();
+        auto multiply = [&]() {
+          if (mi * T::NTL + ni < 16)
+            acc[mi][ni] = Lowp<FMT>::mfma(Lowp<FMT>::operand(Bf[buf][ni], 0), Lowp<FMT>::operand(Af[buf][mi], 0), acc[mi][ni]);
+          else
+            h16_mfma_v<FMT>(Bf[buf][ni], Af[buf][mi], acc[mi][ni]);
+          H16_FENCE();
+        };
+        // (Of one or two MFMAs a slice's reads go out first: behind them the next slice waited for all of its reads.  512 x 1280 x 1280 on 64 x
+        // 64 9.1 -> 8.35 us, raw 9.6 -> 9.0; 1000 x 2560 x 1280 on 128 x 64 17.1 -> 16.9; of four, raw 128 x 128 lost 3 %)
+        if (MF > 2) multiply();
 #pragma unroll
         for (int r = 0; r < READS; ++r) {
           if (r * RG / READS != mf) continue;
@@ -300,6 +305,7 @@ __global__ __launch_bounds__(T::NT, 1) void cascmm_h16_kernel(const GroupParams 
           else issue(s - 1, before, Before(), j);
         }
         H16_FENCE();
+        if (MF <= 2) multiply();
       }
       if (RAWB) {   // (results of reads written as assembly: the compiler does not wait for them)
         __builtin_amdgcn_s_waitcnt(0xC07F);

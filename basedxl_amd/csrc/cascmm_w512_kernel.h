@@ -11,9 +11,9 @@
 // fills its SIMD).  Both operands reach LDS as raw fp32 without passing registers (wave-wide
 // `buffer_load ... lds`, 1 KB each), and every wave splits the values of its own fragments in
 // registers right after reading them:
-//   * A: 256 rows x 16 k per stage; four consecutive lanes fetch the four 16-byte chunks of one row's
-//     64 bytes (whole cache lines), rotated by row / 4 inside the row so that the fragment reads (lane
-//     l: row l%32, chunks 2 (l/32) and 2 (l/32) + 1) spread over all banks;
+//   * A: 256 rows x 32 k, two stages at once; eight consecutive lanes fetch the eight 16-byte chunks of one row's
+//     128 bytes (a whole cache line; in halves, a stage at a time, every line was fetched twice: 4096^3 329.8 us, 320.6 since), rotated
+//     inside the row so that the fragment reads (lane l: row l%32, two chunks of a stage's four) spread over all banks;
 //   * B: 16 k rows x 320 columns per stage, 256 consecutive floats per load; lane l of a fragment reads
 //     column l%32 at k = 8 (l/32) .. +7 with eight ds_read_b32 (rows of the odd k-group are rotated by
 //     32 columns, which keeps the two half waves on different banks).
@@ -21,10 +21,10 @@
 // workgroup; the split's VALU work issues in the gaps between the wave's own MFMAs, as do the LDS
 // reads and the loads of later stages, and it costs no measurable time there.
 //
-// Stages are 16 k deep (60 MFMAs per wave), four of them in LDS (144 KB).  At the barrier that opens
+// Stages are 16 k deep (60 MFMAs per wave), two pairs of A and four stages of B in LDS (144 KB).  At the barrier that opens
 // stage s, stage s + 1 has landed as well, so the first fragments of the next stage are read before
-// its barrier and no LDS latency is exposed after it; the loads of stage s + 3 are issued during
-// stage s.  Loads are issued unconditionally (past the last stage the last one is fetched again into
+// its barrier and no LDS latency is exposed after it; later loads are issued during stage s into what it has freed.
+// Loads are issued unconditionally (past the last stage the last one is fetched again into
 // a dead buffer): a wave that is alone on its SIMD pays tens of cycles for every branch.
 //
 // The order of everything between two MFMAs is pinned with scheduling fences; the four blocks held
@@ -88,13 +88,13 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // tile of the kernels with producer waves; with the weight prepared that one stays the faster, 61 against 68).
 // EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
 // costs the loop nothing, and the stores past it go beyond the descriptor's end; the last stages may hang over K.
-// Measured (graph replay, raw / prepared weight, everything on one box: others are up to 6 % slower, see
-// profiles/cascmm_w512_edge_kernels.txt; in brackets the fastest other kernel): 1976 x 1280 x 10240 on 256 x 320
-// 129.6 / 122.4 us (164.8 / 153.6), its gated form 126.1 (158.5); 7800 x 640 x 5120 139 / 134 (155 / 143); 1500 x 1280 x 10240
-// on 256 x 256 104 / 98 (134 / 110); 4096^3 316 / 297 (351 / 326) = 1.30 PFLOP/s of MFMA work, as on the wider tile: what is
-// left is the clock the board's power allows.  K off its steps (in brackets the K-over-waves kernel, the only other one that
-// takes it): 3700^3 270 / 253 us (350 / 314), 8192 x 328 x 2560 47.5 / 45.3 (84 / 82), 3000 x 1100 x 9000 175 / 165 (239 / 219);
-// the test per load of A costs whole K nothing that can be measured (2048 x 1280 x 10240 131.4 / 123.7, without EDGE 130.0 / 123.2).
+// Measured (graph replay, raw / prepared weight, all on one box, others are up to a tenth faster; in brackets before rows of A came in
+// whole lines): 1976 x 1280 x 10240 on 256 x 320 142.5 / 140.7 us (143.8 / 138.3: the board's power), its gated form 127.4 (132.9);
+// 7800 x 640 x 5120 145.7 / 137.9 (145.1 / 141.1); 1500 x 1280 x 10240 on 256 x 256 109.9 / 103.0 (111.3 / 103.4); 4096^3 323.8 / 303.8
+// (326.7 / 311.4) = 1.27 / 1.36 PFLOP/s of MFMA work, as on the wider tile: what is left is the clock the board's power allows.  K off its
+// steps 3700^3 281 / 263 us (283 / 264; the K-over-waves kernel, the only other one that takes it, 1.25 times that).  The test per load of A
+// costs whole K nothing that can be measured.  Against the kernels with producer waves see profiles/cascmm_w512_edge_kernels.txt (an
+// earlier state of this one).
 // Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, raw B: N % 4 == 0; with the gated store N % 320 == 0 on the wider
 // tile), K % 32 == 0 (EDGE: rows of A of whole 16-byte chunks, zeros between K and the last one's end), lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
 // aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets
