@@ -1367,15 +1367,17 @@ int cascmm_select_variant_glu(int64_t M, int64_t N, int64_t K, int64_t lda, int6
   const RowFit fit = row_fit(q, nullptr, nullptr);
   const int v = select_variant(q, fit, 1);
   if (v < 0) return v;
-  // worth it?  The alternative is the best plain kernel for the product plus the caller's gate, which
-  // reads M x N values and writes half as many (measured at about 3.5 TB/s, two launches); the kernel
-  // with the gated store may be a poor fit for the shape (too few tiles for the chip).
+  // worth it?  The alternative is the plain product, as a call takes it, plus cascmm_gate, which reads M x N values and writes half as many
+  // (5.8 TB/s, and a launch); the kernel with the gated store may be a poor fit for the shape (too few tiles for the chip).
+  // Over 78 shapes of 512 - 8192 rows 0.2 % behind the faster of the two on average, 1.0 % with gelu and product as two launches in mind and the
+  // selection functions' kernels: 2048 x 320 x 2560 gated 34.5 us, plain and gate 30.2; 1792 x 640 x 5120 53.8, 50.3; 3072 x 960 x 7680 165, 159.
   Problem plain = q;
   plain.glu = false;
+  plain.call = true;
   plain.ldc = N;
   const int vp = select_variant(plain, fit, 1);
   if (vp >= 0) {
-    const double gate_us = 2.0 + (double)M * (double)N * 6.0 / 3.5e6;
+    const double gate_us = 2.0 + (double)M * (double)N * 6.0 / 5.8e6;
     if (variant_cost(v, q, 1) > variant_cost(vp, plain, 1) + gate_us) return CASCMM_ERR_BAD_FORMAT;
   }
   return v;
