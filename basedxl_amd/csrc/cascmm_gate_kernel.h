@@ -3,9 +3,11 @@
 //
 // Bound by memory: h is read once and the result written once, where an elementwise gelu and a product read and write gelu(gate) besides.
 // A thread takes runs of VEC elements (16 bytes where the rows allow them) and asks for all of its own before the first is used.
-// Measured (graph replay, us, rows x inner; in brackets gelu and product as two launches): fp32 4000 x 2560 20.7 (46.4, 5.9 TB/s), 700 x 2560
-// 6.2 (11.3), 120 x 2560 4.4 (6.8), single elements 4000 x 2559 28.1 (46.1); fp16 4000 x 2560 14.5 (31.4), 120 x 2560 4.1 (8.0), in 4-byte
-// runs 4000 x 2558 18.9 (30.9), single elements 4000 x 2559 24.6 (31.1).
+// 16-bit elements take the gated stores' gelu (3.4e-6 relative at most where it matters, an element's half ulp is 4.9e-4): with erff, some 40
+// instructions an element beside half the bytes, 4000 x 2560 took 14.5 us.
+// Measured (graph replay, us, rows x inner; in brackets gelu and product as two launches): fp32 4000 x 2560 21.0 (47.1, 5.8 TB/s), 700 x 2560
+// 6.2 (11.3), 120 x 2560 4.7 (7.0), single elements 4000 x 2559 27.3 (47.0); fp16 4000 x 2560 12.5 (31.5), 120 x 2560 4.3 (8.0), in 4-byte
+// runs 4000 x 2558 16.7 (31.4), single elements 4000 x 2559 22.9 (31.3).
 #pragma once
 #include "cascmm_common.h"
 
@@ -35,11 +37,17 @@ __global__ __launch_bounds__(256) void cascmm_gate_kernel(const typename IoType<
     if (i >= total) continue;
     const unsigned row = i / per_row;
     Run r;
+    float g[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float g = IoType<IODT>::load(&gate[u].v[e]);
-      IoType<IODT>::store(&r.v[e], IoType<IODT>::load(&value[u].v[e]) * (0.5f * g * (1.f + erff(g * 0.70710678118654752f))));
+    for (int e = 0; e < VEC; ++e) g[e] = IoType<IODT>::load(&gate[u].v[e]);
+    if constexpr (sizeof(T) == 2) {
+      gelu_values(g);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) g[e] = 0.5f * g[e] * (1.f + erff(g[e] * 0.70710678118654752f));
     }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) IoType<IODT>::store(&r.v[e], IoType<IODT>::load(&value[u].v[e]) * g[e]);
     *(Run*)(out + (int64_t)row * ldo + (int64_t)(i - row * per_row) * VEC) = r;
   }
 }
