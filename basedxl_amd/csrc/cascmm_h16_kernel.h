@@ -13,7 +13,7 @@
 //
 // What bounds it: one product per element leaves three times fewer MFMA cycles per byte than the two-term
 // cascade, so a tile is as good as its bytes per multiply-add: (BM + BN) x 2 bytes per k through the CU's share
-// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared / raw, graph replay, all on one box, others are up to a
+// of the L2s against BM x BN / 2048 matrix cycles.  Measured (fp16, weight prepared / raw, graph replay, all on one card, others are up to a
 // tenth faster; in brackets before rows of A came in whole lines, sums stayed in place and fragments were read earlier): 2048 x 1280 x
 // 10240 on 256 x 320 52.3 / 52.8 us (62.4 / 64.4), its loop at the board's power with random operands (zeros: a third faster); 4096^3 on
 // 256 x 256 115.3 / 114.4 us (121.4 / 123.2); 8192 x 2560 x 640 33.7 / 34.3 us (33.7 / 35.0); 2048^3 on 128 x 128 22.3 / 22.6 us (22.6 /

@@ -132,7 +132,7 @@ __device__ void llvm_raw_buffer_store_v2f32(f32x2 v, i32x4 rsrc, int voffset, in
 __device__ void llvm_raw_buffer_store_i16(short v, i32x4 rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.i16");
 
 // Cache policy of the result stores: sc1 (agent scope) for the kernels with small tiles, the default for the
-// large ones.  A/B on one box, whole kernels: 2048x1280x1280 27.1 -> 26.4 us, 4096x640x640 18.2 -> 17.6 us,
+// large ones.  A/B on one card, whole kernels: 2048x1280x1280 27.1 -> 26.4 us, 4096x640x640 18.2 -> 17.6 us,
 // 8192x640x640 31.7 -> 30.5 us, 2048x5120x1280 83.3 -> 82.7 us with sc1; the 256x320 and the fp8-rate tiles,
 // whose workgroups store 160-320 KB each at the same moment, measured 0.0-0.4 % slower with it and keep the
 // default.  (A bare store loop of the large tile's pattern is faster with sc1, 16.5 -> 13.9 us for 84 MB, and

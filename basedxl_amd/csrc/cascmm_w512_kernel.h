@@ -88,7 +88,7 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // tile of the kernels with producer waves; with the weight prepared that one stays the faster, 61 against 68).
 // EDGE = 1: tiles may hang over the edges of C: rows and columns past the end are loaded as copies of the last one, which
 // costs the loop nothing, and the stores past it go beyond the descriptor's end; the last stages may hang over K.
-// Measured (graph replay, raw / prepared weight, all on one box, others are up to a tenth faster; in brackets before rows of A came in
+// Measured (graph replay, raw / prepared weight, all on one card, others are up to a tenth faster; in brackets before rows of A came in
 // whole lines): 1976 x 1280 x 10240 on 256 x 320 142.5 / 140.7 us (143.8 / 138.3: the board's power), its gated form 127.4 (132.9);
 // 7800 x 640 x 5120 145.7 / 137.9 (145.1 / 141.1); 1500 x 1280 x 10240 on 256 x 256 109.9 / 103.0 (111.3 / 103.4); 4096^3 323.8 / 303.8
 // (326.7 / 311.4) = 1.27 / 1.36 PFLOP/s of MFMA work, as on the wider tile: what is left is the clock the board's power allows.  K off its
