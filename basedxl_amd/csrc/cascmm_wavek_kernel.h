@@ -388,27 +388,28 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 
   // ---- the eight partial tiles meet in LDS: [wave][mb][nb][reg][lane] fp32 -------------------------
   float* part = (float*)wavek_smem;
-  // (SCALED: false where a sum of a column that exists is not finite)
-  auto leave = [&]() {
-    bool finite = true;
+  auto wave_sum = [&](int mb, int nb, int e) {
+    float v = acc[CL - 1][mb][nb][e];
+    if constexpr (CL > 1) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int e = 0; e < REGS; ++e) {
-          float v = acc[CL - 1][mb][nb][e];
-          if constexpr (CL > 1) {
-#pragma unroll
-            for (int c = CL - 2; c >= 0; --c) v = __builtin_fmaf(v, AccClasses<FMT, TERMS, false>::kFoldScale, acc[c][mb][nb][e]);
-          }
-          if constexpr (kFold) v += master[mb][nb][e];
-          if constexpr (SCALED) finite = finite && (__builtin_fabsf(v) < __builtin_inff() || n0 + NB * lw + nb >= p.N);
-          part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
-        }
-    return finite;
+      for (int c = CL - 2; c >= 0; --c) v = __builtin_fmaf(v, AccClasses<FMT, TERMS, false>::kFoldScale, acc[c][mb][nb][e]);
+    }
+    if constexpr (kFold) v += master[mb][nb][e];
+    return v;
   };
-  const bool finite = leave();
+  // (these loops stand here and not in a lambda that a scaled tile calls twice: with it the compiler ordered the straight code
+  // above otherwise, prepared 12 x 4096 x 512 7.86 -> 8.05 us)
+  bool finite = true;   // SCALED: the sums of the columns that exist
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) {
+        const float v = wave_sum(mb, nb, e);
+        if constexpr (SCALED) finite = finite && (__builtin_fabsf(v) < __builtin_inff() || n0 + NB * lw + nb >= p.N);
+        part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
+      }
   unsigned* word = (unsigned*)(wavek_smem + T::LDS_BYTES);   // (SCALED: eight words behind the tiles)
   if constexpr (SCALED) {
     bool seen_b = false;
@@ -478,7 +479,12 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       }
       wavek_wait_loads<0>();
       __syncthreads();
-      leave();
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int e = 0; e < REGS; ++e) part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = wave_sum(mb, nb, e);
       __syncthreads();
     }
   }
