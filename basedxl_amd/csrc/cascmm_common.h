@@ -313,29 +313,34 @@ struct GemmParams {
 // A group of GEMMs of one shape launched as one kernel (count == 1 for a plain GEMM).  Work
 // item i = problem i / tiles, tile i % tiles; workgroup w runs items w, w + grid, w + 2 grid ...
 constexpr int kMaxGroup = 8;
-// gelu(g) = g Phi(g), and value x gelu(gate).  With x = |g|:  t = Phi(-x) = 2^P(x), P a degree-10 fit of log2 Phi(-x) on
-// [0, 5.66], |P - log2 Phi| < 8e-8 (1 + (x / 2)^3), P(0) = -1;  Phi(g) = t for g < 0, 1 - t otherwise: no cancellation in the
-// negative tail, no branch, one v_exp_f32.  Behind 5.66 (Phi = 7.6e-9) P keeps falling, to -inf without an inf - inf, so nothing
-// is clamped.  Against 64 bits, evaluated in fp32: 1.8e-7 relative for g > 0, for g < 0 1e-6 down to -3 and 3.4e-6 down to -5.66
-// (the textbook formula on a correctly rounded erff cancels there).
-// The store of a gated tile is bound by these instructions, four cycles each with one wave per SIMD: a lane of the large tiles evaluates
-// 160 of them.  (As a fit of log2 erfc(x / sqrt 2) of degree 11, clamped at 4, with 2 - t halved: 24 instructions in place of 18.)
+// gelu(g) = g Phi(g), and value x gelu(gate).  With x = |g|:  t = 2 Phi(-x) = 2^P(x), P a degree-10 fit of log2 Phi(-x) + 1 on
+// [0, 5.66], |P - (log2 Phi + 1)| < 7.2e-8 (1 + (x / 2)^4), P(0) = 0;  gelu(g) = max(g, 0) - x t / 2 with one rounding: no cancellation in
+// the negative tail, no branch, one v_exp_f32.  Behind 5.66 (Phi = 7.6e-9) P keeps falling, to -inf without an inf - inf, so nothing
+// is clamped but an infinite gate (inf x 0).  Against 64 bits, evaluated in fp32: 1.2e-7 relative for g > 0, for g < 0 5.2e-7 down to -2, 9e-7
+// down to -3 and 3.8e-6 down to -5.66 (the textbook formula on a correctly rounded erff cancels there); rms, of the result's rms, 3.5e-8 for gates
+// of N(0, 0.3) and 2.8e-8 for N(0, 1).  (P(0) = -1 and g (1 - t) instead, as many instructions: 5.1e-8 and 3.5e-8, since P is rounded below -1 and
+// the difference once more; log2 erfc(x / sqrt 2) of degree 11, clamped at 4, 24 instructions: 4.5e-8 and 3.5e-8.)
+// The store of a gated tile is bound by these 18 instructions, four cycles each with one wave per SIMD: a lane of the large tiles evaluates
+// 160 of them.
 // Several at a time (g: gates, on return gelu of each), step by step: of one alone every instruction waits for the one before it.
+constexpr float kGeluFit[10] = {-2.498480178e-08f, 7.532745485e-07f, -9.763462913e-06f, 6.904493057e-05f, -2.528995683e-04f,
+                                -5.766478353e-05f, 7.019202691e-03f, -5.249055102e-02f, -4.592050016e-01f, -1.151105881e+00f};   // x^10 .. x
 template <int N> __device__ __forceinline__ void gelu_values(float (&g)[N]) {
-  constexpr float c[11] = {-2.313676539e-08f, 7.062524219e-07f, -9.261655578e-06f, 6.612614379e-05f, -2.428296721e-04f, -7.868819375e-05f,
-                           7.045188919e-03f, -5.250833556e-02f, -4.591991603e-01f, -1.151106477e+00f, -1.0f};
   float t[N];
 #pragma unroll
-  for (int e = 0; e < N; ++e) t[e] = c[0];
+  for (int e = 0; e < N; ++e) t[e] = kGeluFit[0];
 #pragma unroll
-  for (int i = 1; i < 11; ++i) {
+  for (int i = 1; i < 10; ++i) {
 #pragma unroll
-    for (int e = 0; e < N; ++e) t[e] = __builtin_fmaf(t[e], __builtin_fabsf(g[e]), c[i]);
+    for (int e = 0; e < N; ++e) t[e] = __builtin_fmaf(t[e], __builtin_fabsf(g[e]), kGeluFit[i]);
   }
 #pragma unroll
-  for (int e = 0; e < N; ++e) t[e] = __builtin_amdgcn_exp2f(t[e]);
+  for (int e = 0; e < N; ++e) t[e] = __builtin_amdgcn_exp2f(t[e] * __builtin_fabsf(g[e]));
 #pragma unroll
-  for (int e = 0; e < N; ++e) g[e] *= g[e] < 0.f ? t[e] : 1.f - t[e];
+  for (int e = 0; e < N; ++e) {
+    const int bits = __builtin_bit_cast(int, g[e]);   // (max(g, 0) of integers: of floats the compiler quiets g in an instruction of its own)
+    g[e] = __builtin_fmaf(-__builtin_fabsf(__builtin_fminf(0.5f * g[e], 1.0e38f)), t[e], __builtin_bit_cast(float, bits > 0 ? bits : 0));
+  }
 }
 __device__ __forceinline__ float gelu_value(float g) {
   float t[1] = {g};

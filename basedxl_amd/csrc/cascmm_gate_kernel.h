@@ -3,7 +3,7 @@
 //
 // Bound by memory: h is read once and the result written once, where an elementwise gelu and a product read and write gelu(gate) besides.
 // A thread takes runs of VEC elements (16 bytes where the rows allow them) and asks for all of its own before the first is used.
-// 16-bit elements take the gated stores' gelu (3.4e-6 relative at most where it matters, an element's half ulp is 4.9e-4): with erff, some 40
+// 16-bit elements take the gated stores' gelu (3.8e-6 relative at most where it matters, an element's half ulp is 4.9e-4): with erff, some 40
 // instructions an element beside half the bytes, 4000 x 2560 took 14.5 us.
 // Measured (graph replay, us, rows x inner; in brackets gelu and product as two launches): fp32 4000 x 2560 21.0 (47.1, 5.8 TB/s), 700 x 2560
 // 6.2 (11.3), 120 x 2560 4.7 (7.0), single elements 4000 x 2559 27.3 (47.0); fp16 4000 x 2560 12.5 (31.5), 120 x 2560 4.3 (8.0), in 4-byte
