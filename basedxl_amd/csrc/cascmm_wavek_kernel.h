@@ -103,16 +103,14 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
   else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
 }
 
-// Three fp16 terms on values as they are: what the largest element of an operand has to reach.  The terms resolve 2^-46 then, 2^-33 of
-// that element; the products that are left out are 2^-33 of a product too, and the roundings of the sums 2^-24.
-constexpr short kWaveKLeast = 0x0800;   // 2^-13
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void wavek_top(s16x2& top, const u32x4& t) {
+// Three fp16 terms on values as they are: what the largest element of an operand has to reach.  The terms resolve 2^-46 at the
+// least, 2^-33 of that element; the products that are left out are 2^-33 of a product too, and the roundings of the sums 2^-24.
+constexpr float kWaveKLeast = 0x1p-13f;
+// (in assembly: the compiler quiets values from memory, in an instruction each, before it compares them.  A NaN may end in top what
+// was in it before; where there is one, a sum is one too.)
+__device__ __forceinline__ void wavek_top(float& top, const float (&x)[8]) {
 #pragma unroll
-  for (int d = 0; d < 4; ++d) top = __builtin_elementwise_max(top, __builtin_bit_cast(s16x2, (unsigned)t[d]));
-}
-__device__ __forceinline__ bool wavek_seen(const s16x2& top) {
-  return (short)(top[0] & 0x7FFF) >= kWaveKLeast || (short)(top[1] & 0x7FFF) >= kWaveKLeast;
+  for (int e = 0; e < 8; e += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(x[e]), "v"(x[e + 1]));
 }
 
 // A's rows in a stage: position pos of row r holds chunk (pos - wavek_rot(r / 2)) mod 8 (16-row blocks: the rotations of
@@ -151,10 +149,11 @@ using WaveKOf = WaveK<W, MB, NB, AL, BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W /
 // SCALED = 1 (three fp16 terms, raw): for the calls of the slot kernels (cascmm_f16k_kernel.h), which find the maxima of both operands and
 // scale them before they split, in launches of their own.  Here a tile is computed on the values as they are; where a value of its rows
 // of A or columns of B left fp16's range (a sum is then not finite), or all of A's or of B's lie below kWaveKLeast (the terms would be
-// coarse), the same workgroup reads its operands' maxima and computes the tile again, scaled: once more for the tiles concerned,
-// nothing but a packed maximum per two elements for the others.  Three launches and the slots' trip through memory are saved, and the
-// tiles are small (us, graph replay, before: on 64 x 160 slot tiles): 5 x 3164 x 3136 80.9, here 16.2; 33 x 1612 x 1374 47.3, 12.9; 223 x
-// 1400 x 1024 43.7, 15.3; 71 x 3800 x 3520 97.9, 57.6; with every tile computed twice 45.7, 39.2, 44.1 and 161.  Errors against 64 bits:
+// coarse), the same workgroup computes the tile again, scaled by its operands' maxima, which the first pass has kept (beyond the range they are
+// read once more): nothing but a maximum of three per two elements for the other tiles, nor for those of zeros.  Three launches and the slots' trip through memory are saved, and the
+// tiles are small (us, graph replay, in slots on 64 x 160 tiles and here): 5 x 3164 x 3136 80.7, 15.9; 33 x 1612 x 1374 47.4, 14.0; 223 x
+// 1400 x 1024 43.0, 16.5; 71 x 3800 x 3520 96.5, 56.1; with every tile computed twice because its values are small 33.8, 32.8, 35.2 and 119.8,
+// because they are large 44.3, 40.5, 44.3 and 161.8, with A of zeros 19.4, 18.7, 19.6 and 63.5.  Errors against 64 bits:
 // 1.1 to 7.2 1e-9 (rms, of the sum of magnitudes), 6.1e-9 to 1.2e-8 in slots.
 template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0, int SCALED = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
@@ -273,11 +272,8 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
       scale_out = __builtin_ldexpf(1.f, -(ea + eb));
     }
   }
-  // SCALED: of A, and of the columns of B, the largest leading term that a lane has seen (as 16-bit integers: the largest positive one,
-  // or the negative one of largest magnitude where there is no other)
-  s16x2 top_a = {-32768, -32768}, top_b[SCALED ? NB : 1];
-#pragma unroll
-  for (int nb = 0; nb < (SCALED ? NB : 1); ++nb) top_b[nb] = top_a;
+  // SCALED: the largest magnitude that a lane has seen of A, and of its columns of B
+  float top_a = 0.f, top_b[SCALED ? NB : 1] = {};
   auto step = [&](int i, auto U, auto again) {
     constexpr int u = decltype(U)::value;
     constexpr bool kAgain = decltype(again)::value;
@@ -298,9 +294,10 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         if constexpr (kAgain) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) xa[e] *= scale_a;
+        } else if constexpr (SCALED) {
+          wavek_top(top_a, xa);
         }
         split8<FMT, TERMS>(xa, ta[mb], scale_a);
-        if constexpr (SCALED && !kAgain) wavek_top(top_a, ta[mb][0]);
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -315,9 +312,10 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           if constexpr (kAgain) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) xb[e] *= scale_b;
+          } else if constexpr (SCALED) {
+            wavek_top(top_b[nb], xb);
           }
           split8<FMT, TERMS>(xb, tb, scale_b);
-          if constexpr (SCALED && !kAgain) wavek_top(top_b[nb], tb[0]);
         }
         // smallest products first
 #pragma unroll
@@ -411,48 +409,61 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
       }
   unsigned* word = (unsigned*)(wavek_smem + T::LDS_BYTES);   // (SCALED: eight words behind the tiles)
+  float top = 0.f;                                           // (SCALED: of this lane's columns of B that exist)
   if constexpr (SCALED) {
-    bool seen_b = false;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) seen_b = seen_b || (n0 + NB * lw + nb < p.N && wavek_seen(top_b[nb]));
-    const unsigned mine = (__any(wavek_seen(top_a)) ? 1u : 0u) | (__any(seen_b) ? 2u : 0u) | (__any(!finite) ? 4u : 0u);
+    for (int nb = 0; nb < NB; ++nb) top = n0 + NB * lw + nb < p.N && top_b[nb] > top ? top_b[nb] : top;
+    const unsigned mine = (__any(top_a >= kWaveKLeast) ? 1u : 0u) | (__any(top >= kWaveKLeast) ? 2u : 0u) | (__any(!finite) ? 4u : 0u);
     if (lane == 0) word[wave] = mine;
   }
   __syncthreads();
+  bool again = false;
   if constexpr (SCALED) {
     unsigned all = 0;
 #pragma unroll
     for (int w = 0; w < T::NW; ++w) all |= word[w];
-    if (__builtin_amdgcn_readfirstlane(all) != 3) {
-      __syncthreads();
-      if (tid < 2) word[tid] = 0;
-      __syncthreads();
-      // the largest finite elements of the tile's rows of A and columns of B (rows past the last one: that one again)
-      unsigned best = 0;
-      const auto look = [&](float x) {
-        const unsigned bits = __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu;
-        best = bits < 0x7F800000u && bits > best ? bits : best;
+    all = __builtin_amdgcn_readfirstlane(all);
+    if (all != 3) {
+      // the largest elements of the tile's rows of A and columns of B
+      const auto most = [&](unsigned a, unsigned b) {
+        __syncthreads();
+        if (tid < 2) word[tid] = 0;
+        __syncthreads();
+        atomicMax(&word[0], a);
+        atomicMax(&word[1], b);
+        __syncthreads();
       };
-      for (int k = tid; k < p.K; k += T::NT) {
-        float x[T::BM];
+      if (all & 4) {
+        // values beyond fp16's range, infinities or NaN among them: the largest finite ones (rows past the last one: that one again)
+        unsigned best_a = 0, best_b = 0;
+        const auto look = [](unsigned& best, float x) {
+          const unsigned bits = __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu;
+          best = bits < 0x7F800000u && bits > best ? bits : best;
+        };
+        for (int k = tid; k < p.K; k += T::NT) {
+          float x[T::BM];
 #pragma unroll
-        for (int r = 0; r < T::BM; ++r) x[r] = ((const float*)pa)[(int64_t)(m0 + r < p.M ? m0 + r : p.M - 1) * p.lda + k];
+          for (int r = 0; r < T::BM; ++r) x[r] = ((const float*)pa)[(int64_t)(m0 + r < p.M ? m0 + r : p.M - 1) * p.lda + k];
 #pragma unroll
-        for (int r = 0; r < T::BM; ++r) look(x[r]);
+          for (int r = 0; r < T::BM; ++r) look(best_a, x[r]);
+        }
+        constexpr int ROWS = T::NT / T::BN, U = 16;
+        const float* col = (const float*)pb + (n0 + tid % T::BN < p.N ? n0 + tid % T::BN : p.N - 1);
+        for (int k = tid / T::BN; k < p.K; k += ROWS * U) {
+          float x[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) x[u] = col[(int64_t)(k + u * ROWS < p.K ? k + u * ROWS : p.K - 1) * p.ldb];
+#pragma unroll
+          for (int u = 0; u < U; ++u) look(best_b, x[u]);
+        }
+        most(best_a, best_b);
+      } else {
+        most(__builtin_bit_cast(unsigned, top_a), __builtin_bit_cast(unsigned, top));
       }
-      atomicMax(&word[0], best);
-      best = 0;
-      constexpr int ROWS = T::NT / T::BN, U = 16;
-      const float* col = (const float*)pb + (n0 + tid % T::BN < p.N ? n0 + tid % T::BN : p.N - 1);
-      for (int k = tid / T::BN; k < p.K; k += ROWS * U) {
-        float x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = col[(int64_t)(k + u * ROWS < p.K ? k + u * ROWS : p.K - 1) * p.ldb];
-#pragma unroll
-        for (int u = 0; u < U; ++u) look(x[u]);
-      }
-      atomicMax(&word[1], best);
-      __syncthreads();
+      // (finite sums of zeros are what they are)
+      again = __builtin_amdgcn_readfirstlane((all & 4) != 0 || (word[0] != 0 && word[1] != 0));
+    }
+    if (again) {
       const int ea = f16k_exp_of_amax(word[0]), eb = f16k_exp_of_amax(word[1]);
       scale_a = __builtin_ldexpf(1.f, ea);
       scale_b = __builtin_ldexpf(1.f, eb);

@@ -58,6 +58,10 @@ def test_scaled_rows(M, K, N, name):
     _check(a, b, run(wide[:, :K], b))
     # operands without a positive element, of zeros, of whole numbers
     _check(-a.abs(), -b.abs(), run(-a.abs(), -b.abs()))
+    # ... and computed once, with the unscaled kernel's bits (a second pass splits small elements into other terms and folds its sums elsewhere)
+    once, low = _lib.variant_names().index(name[:-len("_scaled")]), a.clamp(max=0) * torch.logspace(-5, 0, K, device="cuda")
+    for x, y in ((a, b), (low, b), (a, -b.abs())):
+        assert torch.equal(run(x, y), cascaded_lowp_matmul(x, y, lowp="fp16", terms=3, variant=once))
     assert not run(torch.zeros_like(a), b).any() and not run(a, torch.zeros_like(b)).any()
     ia, ib = (a * 8).round(), (b * 8).round()
     assert torch.equal(run(ia, ib).double(), ia.double() @ ib.double())
