@@ -103,9 +103,11 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
   else return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
 }
 
-// Three fp16 terms on values as they are: what the largest element of an operand has to reach.  The terms resolve 2^-46 at the
-// least, 2^-33 of that element; the products that are left out are 2^-33 of a product too, and the roundings of the sums 2^-24.
-constexpr float kWaveKLeast = 0x1p-13f;
+// Three fp16 terms on values as they are: what the largest element of an operand has to reach.  The terms are whole multiples of 2^-46,
+// 2^-38 of that element: what the slots hold (their smallest term is kept at 2^-35 of elements scaled to 14 at most).  The products
+// that are left out are 2^-33 of a product, and the roundings of the sums 2^-24.  (At 2^-13 a tile's elements 2^-16 below its largest one
+// were off by 2.9e-6 of themselves, in slots by 1.0e-7.)
+constexpr float kWaveKLeast = 0x1p-8f;
 // (in assembly: the compiler quiets values from memory, in an instruction each, before it compares them.  A NaN may end in top what
 // was in it before; where there is one, a sum is one too.)
 __device__ __forceinline__ void wavek_top(float& top, const float (&x)[8]) {

@@ -24,14 +24,15 @@ def test_few_rows_take_the_kernel_that_scales_its_own_tiles():
 
 def _check(a, b, c, bias=None):
     """Each of a wave's sums over K / 256 steps is rounded once per MFMA and folded in blocks, the waves' eight are added: below 16 + K / 256
-    roundings of 2^-24 of the sum of magnitudes; the terms hold an operand to 2^-36 of the largest element of its tile (tiles of 32 at most)."""
+    roundings of 2^-24 of the sum of magnitudes; the terms hold an operand to 2^-39 of the largest element of its tile (half of 2^-46 where that
+    is 2^-8, the least that is taken unscaled; tiles of 32 at most): twice that, for the products of two such roundings and the dropped ones."""
     ad, bd = a.double(), b.double()
     ref = ad @ bd + (0 if bias is None else bias.double())
     K = a.shape[1]
     mag = ad.abs() @ bd.abs()
     tile_a = torch.cat([r.abs().amax().expand(r.shape[0]) for r in ad.split(32)])[:, None]
     tile_b = torch.cat([r.abs().amax().expand(r.shape[1]) for r in bd.split(32, 1)])[None, :]
-    bound = (16 + K / 256) * 2.0 ** -24 * mag + 2.0 ** -36 * (tile_a * bd.abs().sum(0)[None, :] + tile_b * ad.abs().sum(1)[:, None])
+    bound = (16 + K / 256) * 2.0 ** -24 * mag + 2.0 ** -38 * (tile_a * bd.abs().sum(0)[None, :] + tile_b * ad.abs().sum(1)[:, None])
     bad = ~((c.double() - ref).abs() <= bound + ref.abs() * 2.0 ** -23)
     assert not bad.any(), float(((c.double() - ref).abs() / bound).max())
 
@@ -76,3 +77,24 @@ def test_scaled_rows(M, K, N, name):
     assert not torch.isfinite(c[M - 1]).any() and torch.isnan(c[:, N - 1]).all()
     if M > 1:
         _check(inf[:M - 1], nan[:, :N - 1], c[:M - 1, :N - 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("top", [2.0 ** -8 * (1 + 2.0 ** -10), 2.0 ** -8 * (1 - 2.0 ** -10), 2.0 ** -10, 2.0 ** -13 * 1.01, 2.0 ** -13 * 0.99])
+def test_scaled_rows_near_the_least_unscaled_tile(top, name):
+    """Operands whose largest element meets zeros and whose other elements are 2^-20 of it: the results' errors are what the terms resolve
+    (unscaled 2^-47 an element, against the bound 2^-38 of the largest), the roundings of the sums 2^-40 of that."""
+    print(name, top, flush=True)
+    v = _lib.variant_names().index(name)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    M, K, N = 19, 41, 45
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g)
+    a[:, 5:], b[5:] = 0, 0
+    low_a, low_b, plain_a, plain_b = a * (top * 2.0 ** -20), b * (top * 2.0 ** -20), a.clone(), b.clone()
+    low_a[:, 0], plain_b[0] = top, 0            # A's largest elements meet zeros
+    low_b[0], plain_a[:, 0] = top, 0            # B's
+    low_b2, low_a2 = low_b.clone(), low_a.clone()
+    low_b2[0], low_b2[7], low_a2[:, 7] = 0, top, 0          # both
+    for x, y in ((low_a, plain_b), (plain_a, low_b), (low_a2, low_b2)):
+        _check(x, y, cascaded_lowp_matmul(x, y, lowp="fp16", terms=3, variant=v))
