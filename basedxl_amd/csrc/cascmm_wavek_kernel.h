@@ -108,12 +108,19 @@ __device__ __forceinline__ ACC wavek_mfma(typename Lowp<FMT>::Vec a, typename Lo
 // that are left out are 2^-33 of a product, and the roundings of the sums 2^-24.  (At 2^-13 a tile's elements 2^-16 below its largest one
 // were off by 2.9e-6 of themselves, in slots by 1.0e-7.)
 constexpr float kWaveKLeast = 0x1p-8f;
-// (in assembly: the compiler quiets values from memory, in an instruction each, before it compares them.  A NaN may end in top what
-// was in it before; where there is one, a sum is one too.)
+// A wave whose first step has nothing from kWaveKLeast on, or something beyond kWaveKMost, scales: that step's largest element to 2^-6, so
+// that later ones may be 2^22 times as large
+constexpr float kWaveKMost = 0x1p15f;
+__device__ __forceinline__ int wavek_exp(unsigned bits) {
+  const int e = exp_of_amax(bits) - 14;
+  return e < -60 ? -60 : e > 60 ? 60 : e;
+}
+// (in assembly: the compiler quiets values from memory, in an instruction each, before it compares them.  A NaN stays in top.)
 __device__ __forceinline__ void wavek_top(float& top, const float (&x)[8]) {
 #pragma unroll
-  for (int e = 0; e < 8; e += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(x[e]), "v"(x[e + 1]));
+  for (int e = 0; e < 8; e += 2) asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(x[e]), "v"(x[e + 1]));
 }
+__device__ __forceinline__ unsigned wavek_bits(float top) { return __builtin_bit_cast(unsigned, top) & 0x7FFFFFFFu; }
 
 // A's rows in a stage: position pos of row r holds chunk (pos - wavek_rot(r / 2)) mod 8 (16-row blocks: the rotations of
 // cascmm_slotn_kernel.h, which explains them)
@@ -149,14 +156,15 @@ using WaveKOf = WaveK<W, MB, NB, AL, BPRE ? Lowp<FMT>::planes(TERMS) * NB * (W /
 // BPRE = 1: B is a prepared weight, [plane][4 ceil(K/32)][N] operand slots, a load per plane and column block (block nb: columns
 // W nb + c).  GLU = 1 (prepared, 64-wide tiles): the gated store, C has N / 2 columns, B alternates 32 value and 32 gate columns.
 // SCALED = 1 (three fp16 terms, raw): for the calls of the slot kernels (cascmm_f16k_kernel.h), which find the maxima of both operands and
-// scale them before they split, in launches of their own.  Here a tile is computed on the values as they are; where a value of its rows
-// of A or columns of B left fp16's range (a sum is then not finite), or all of A's or of B's lie below kWaveKLeast (the terms would be
-// coarse), the same workgroup computes the tile again, scaled by its operands' maxima, which the first pass has kept (beyond the range they are
-// read once more): nothing but a maximum of three per two elements for the other tiles, nor for those of zeros.  Three launches and the slots' trip through memory are saved, and the
-// tiles are small (us, graph replay, in slots on 64 x 160 tiles and here): 5 x 3164 x 3136 80.7, 15.9; 33 x 1612 x 1374 47.4, 14.0; 223 x
-// 1400 x 1024 43.0, 16.5; 71 x 3800 x 3520 96.5, 56.1; with every tile computed twice because its values are small 33.8, 32.8, 35.2 and 119.8,
-// because they are large 44.3, 40.5, 44.3 and 161.8, with A of zeros 19.4, 18.7, 19.6 and 63.5.  Errors against 64 bits:
-// 1.1 to 7.2 1e-9 (rms, of the sum of magnitudes), 6.1e-9 to 1.2e-8 in slots.
+// scale them before they split, in launches of their own.  Here a wave looks at its first step: values within fp16's range and not too small are
+// computed as they are, others scaled by that step's maxima, undone on the wave's sums.  Where that was not enough, a sum is not
+// finite or all of the tile's rows of A or columns of B lie below kWaveKLeast, the workgroup computes the tile again, scaled by its operands'
+// maxima, which the first pass has kept (infinities and NaN among them: the largest finite ones, read once more).  Tiles of zeros are not
+// computed again.  Three launches and the slots' trip through memory are saved, and the tiles are small (us, graph replay: in slots on 64 x 160
+// tiles; here; here with values that are scaled): 5 x 3165 x 3136 79.9, 15.0, 19.5; 33 x 1613 x 1374 46.0, 11.8, 19.4; 223 x 1401 x 1024 43.1,
+// 14.9, 21.5; 71 x 3801 x 3520 96.4, 54.8, 66.1.  A second pass is dearer: with one element of A beyond the range 33.3, 29.7, 33.0, 86.6, with A's
+// first 512 k 2^30 below the others 37.9, 37.1, 39.2, 128.9.  Errors against 64 bits: 1.1 to 7.2 1e-9 (rms, of the sum of magnitudes), 6.1e-9
+// to 1.2e-8 in slots.
 template <int W, int MB, int NB, int AL, int TAIL, int FMT, int TERMS, int BPRE = 0, int GLU = 0, int SCALED = 0>
 __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) {
   static_assert(!GLU || (BPRE && W == 16 && NB == 4), "a value block and its gate block in one tile");
@@ -265,7 +273,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 
   // fp8 terms: the tensors' scales, powers of two
   constexpr bool kScaled8 = FMT == CASCMM_FMT_FP8;
-  float scale_a = 1.f, scale_b = 1.f, scale_out = 1.f;
+  float scale_a = 1.f, scale_b = 1.f, scale_out = 1.f, scale_wave = 1.f;   // (scale_wave: of this wave's sums, SCALED)
   if constexpr (kScaled8) {
     if (p.tensor_exps) {
       const int ea = p.tensor_exps[2 * prob], eb = p.tensor_exps[2 * prob + 1];
@@ -276,9 +284,13 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   }
   // SCALED: the largest magnitude that a lane has seen of A, and of its columns of B
   float top_a = 0.f, top_b[SCALED ? NB : 1] = {};
-  auto step = [&](int i, auto U, auto again) {
+  // how a step takes its values
+  typedef std::integral_constant<int, 0> AsTheyAre;
+  typedef std::integral_constant<int, 1> Scaled;
+  typedef std::integral_constant<int, 2> ScaledAgain;   // the maxima are known
+  auto step = [&](int i, auto U, auto how) {
     constexpr int u = decltype(U)::value;
-    constexpr bool kAgain = decltype(again)::value;
+    constexpr bool kScale = decltype(how)::value != 0, kTop = SCALED && decltype(how)::value != 2;
     const unsigned char* stp = ring + u * T::A_STAGE;
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
@@ -293,11 +305,10 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
 #pragma unroll
           for (int e = 0; e < 8; ++e) xa[e] = e < left ? xa[e] : 0.f;
         }
-        if constexpr (kAgain) {
+        if constexpr (kTop) wavek_top(top_a, xa);
+        if constexpr (kScale) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) xa[e] *= scale_a;
-        } else if constexpr (SCALED) {
-          wavek_top(top_a, xa);
         }
         split8<FMT, TERMS>(xa, ta[mb], scale_a);
       }
@@ -311,11 +322,10 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           float xb[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) xb[e] = Bv[u][h][e][nb];
-          if constexpr (kAgain) {
+          if constexpr (kTop) wavek_top(top_b[nb], xb);
+          if constexpr (kScale) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) xb[e] *= scale_b;
-          } else if constexpr (SCALED) {
-            wavek_top(top_b[nb], xb);
           }
           split8<FMT, TERMS>(xb, tb, scale_b);
         }
@@ -343,6 +353,43 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         }
     }
   };
+  // SCALED: the first step's maxima, once its loads have landed; whether the wave scales, by scale_a and scale_b
+  auto scales = [&]() {
+    float first_a = 0.f, first_b = 0.f;
+    const int left = p.K - wave * T::BK - 8 * kg;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const unsigned char* src = ring + mb * (W * 128);
+      const f32x4 x0 = *(const f32x4*)(src + a_frag[0][0]), x1 = *(const f32x4*)(src + a_frag[0][1]);
+      float xa[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xa[e] = e < left ? xa[e] : 0.f;
+      wavek_top(first_a, xa);
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      float xb[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xb[e] = n0 + NB * lw + nb < p.N ? Bv[0][0][e][nb] : 0.f;
+      wavek_top(first_b, xb);
+    }
+    const bool take_a = __any(first_a >= kWaveKLeast) && !__any(first_a > kWaveKMost), take_b = __any(first_b >= kWaveKLeast) && !__any(first_b > kWaveKMost);
+    if (take_a && take_b) return false;
+    unsigned bits_a = wavek_bits(first_a), bits_b = wavek_bits(first_b);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned a = (unsigned)__shfl_xor((int)bits_a, off, 64), b = (unsigned)__shfl_xor((int)bits_b, off, 64);
+      bits_a = a > bits_a ? a : bits_a;
+      bits_b = b > bits_b ? b : bits_b;
+    }
+    // (zeros, infinities and NaN say nothing)
+    const int ea = take_a || bits_a == 0 || bits_a >= 0x7F800000u ? 0 : wavek_exp(bits_a), eb = take_b || bits_b == 0 || bits_b >= 0x7F800000u ? 0 : wavek_exp(bits_b);
+    scale_a = __builtin_ldexpf(1.f, ea);
+    scale_b = __builtin_ldexpf(1.f, eb);
+    scale_wave = __builtin_ldexpf(1.f, -(ea + eb));
+    return __builtin_amdgcn_readfirstlane(ea | eb) != 0;
+  };
+  bool scaled = false;
   // Up to T::STRAIGHT steps: straight code for their number, which issues no load that nobody needs (a step's loads past the
   // end of the buffers cost 0.25 us).  More: trips of NS steps without a branch inside, then those that are left, whose loads
   // are under way already.  In both every path into a step has issued the same loads, so the compiler knows how many are
@@ -352,25 +399,35 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   wavek_each<T::STRAIGHT>([&](auto Z) {
     constexpr int S = decltype(Z)::value + 1;
     if (my_steps == S) {
-      wavek_each<(S < NS - 1 ? S : NS - 1)>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+      constexpr int AHEAD = S < NS - 1 ? S : NS - 1;
+      wavek_each<AHEAD>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+      if constexpr (SCALED) {
+        wavek_wait_loads<(AHEAD - 1) * L1>();
+        scaled = scales();
+        if (scaled) return;
+      }
       wavek_each<S>([&](auto U) {
         constexpr int u = decltype(U)::value, younger = S - 1 - u < NS - 1 ? S - 1 - u : NS - 1;
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (u + NS - 1 < S) issue(u + NS - 1, (u + NS - 1) % NS);
         wavek_wait_loads<younger * L1>();
-        step(u, std::integral_constant<int, u % NS>{}, std::false_type{});
+        step(u, std::integral_constant<int, u % NS>{}, AsTheyAre{});
       });
     }
   });
   if (my_steps > T::STRAIGHT) {
     wavek_each<NS - 1>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
-    int i = 0;
+    if constexpr (SCALED) {
+      wavek_wait_loads<(NS - 2) * L1>();
+      scaled = scales();
+    }
+    int i = SCALED && scaled ? my_steps : 0;
     for (; i + NS <= my_steps; i += NS) {
       wavek_each<NS>([&](auto U) {
         constexpr int u = decltype(U)::value;
         issue(i + u + NS - 1, (u + NS - 1) % NS);
         wavek_wait_loads<(NS - 1) * L1>();
-        step(i + u, U, std::false_type{});
+        step(i + u, U, AsTheyAre{});
       });
       fold();
     }
@@ -379,10 +436,28 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
                                constexpr int u = decltype(U)::value;
                                __builtin_amdgcn_sched_barrier(0);
                                wavek_wait_loads<(NS - 2 - u) * L1>();
-                               step(i + u, U, std::false_type{});
+                               step(i + u, U, AsTheyAre{});
                              });
   }
   fold();
+  // all steps, scaled, from the first one on (those past the last one add products of zeros)
+  auto scaled_steps = [&](auto how) {
+    wavek_wait_loads<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    wavek_each<NS - 1>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
+    for (int i = 0; i < my_steps; i += NS) {
+      wavek_each<NS>([&](auto U) {
+        constexpr int u = decltype(U)::value;
+        issue(i + u + NS - 1, (u + NS - 1) % NS);
+        wavek_wait_loads<(NS - 1) * L1>();
+        step(i + u, U, how);
+      });
+      fold();
+    }
+  };
+  if constexpr (SCALED) {
+    if (scaled) scaled_steps(Scaled{});
+  }
   wavek_wait_loads<0>();   // the loads past the last step land before the ring is reused
   __syncthreads();
 
@@ -406,7 +481,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int e = 0; e < REGS; ++e) {
-        const float v = wave_sum(mb, nb, e);
+        const float v = SCALED ? wave_sum(mb, nb, e) * scale_wave : wave_sum(mb, nb, e);
         if constexpr (SCALED) finite = finite && (__builtin_fabsf(v) < __builtin_inff() || n0 + NB * lw + nb >= p.N);
         part[(((wave * MB + mb) * NB + nb) * REGS + e) * 64 + lane] = v;
       }
@@ -414,8 +489,11 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
   float top = 0.f;                                           // (SCALED: of this lane's columns of B that exist)
   if constexpr (SCALED) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) top = n0 + NB * lw + nb < p.N && top_b[nb] > top ? top_b[nb] : top;
-    const unsigned mine = (__any(top_a >= kWaveKLeast) ? 1u : 0u) | (__any(top >= kWaveKLeast) ? 2u : 0u) | (__any(!finite) ? 4u : 0u);
+    for (int nb = 0; nb < NB; ++nb) {
+      float xb[8] = {n0 + NB * lw + nb < p.N ? top_b[nb] : 0.f};
+      wavek_top(top, xb);
+    }
+    const unsigned mine = (__any(top_a * scale_a >= kWaveKLeast) ? 1u : 0u) | (__any(top * scale_b >= kWaveKLeast) ? 2u : 0u) | (__any(!finite) ? 4u : 0u);
     if (lane == 0) word[wave] = mine;
   }
   __syncthreads();
@@ -435,8 +513,9 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
         atomicMax(&word[1], b);
         __syncthreads();
       };
-      if (all & 4) {
-        // values beyond fp16's range, infinities or NaN among them: the largest finite ones (rows past the last one: that one again)
+      most(wavek_bits(top_a), wavek_bits(top));
+      if (__builtin_amdgcn_readfirstlane(word[0] >= 0x7F800000u || word[1] >= 0x7F800000u)) {
+        // infinities or NaN among the values: the largest finite ones (rows past the last one: that one again)
         unsigned best_a = 0, best_b = 0;
         const auto look = [](unsigned& best, float x) {
           const unsigned bits = __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu;
@@ -459,8 +538,6 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           for (int u = 0; u < U; ++u) look(best_b, x[u]);
         }
         most(best_a, best_b);
-      } else {
-        most(__builtin_bit_cast(unsigned, top_a), __builtin_bit_cast(unsigned, top));
       }
       // (finite sums of zeros are what they are)
       again = __builtin_amdgcn_readfirstlane((all & 4) != 0 || (word[0] != 0 && word[1] != 0));
@@ -478,18 +555,7 @@ __global__ __launch_bounds__(512) void cascmm_wavek_kernel(const GroupParams p) 
           for (int c = 0; c < CL; ++c) acc[c][mb][nb] = zero;
           if constexpr (kFold) master[mb][nb] = zero;
         }
-      // (steps past the last one add products of zeros)
-      __builtin_amdgcn_sched_barrier(0);
-      wavek_each<NS - 1>([&](auto U) { issue(decltype(U)::value, decltype(U)::value); });
-      for (int i = 0; i < my_steps; i += NS) {
-        wavek_each<NS>([&](auto U) {
-          constexpr int u = decltype(U)::value;
-          issue(i + u + NS - 1, (u + NS - 1) % NS);
-          wavek_wait_loads<(NS - 1) * L1>();
-          step(i + u, U, std::true_type{});
-        });
-        fold();
-      }
+      scaled_steps(ScaledAgain{});
       wavek_wait_loads<0>();
       __syncthreads();
 #pragma unroll

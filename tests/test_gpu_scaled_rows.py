@@ -59,8 +59,17 @@ def test_scaled_rows(M, K, N, name):
     _check(a, b, run(wide[:, :K], b))
     # operands without a positive element, of zeros, of whole numbers
     _check(-a.abs(), -b.abs(), run(-a.abs(), -b.abs()))
+    # waves whose first steps are small, zero, large or of another size than what follows
+    k = torch.arange(K, device="cuda") // 32
+    for first, rest in ((-30, 0), (0, -30), (-30, 30), (30, -12), (-9, 12)):
+        x = a * 2.0 ** torch.where(k < 8, first, rest)
+        _check(x, b, run(x, b))
+        y = b * 2.0 ** torch.where(k < 8, first, rest)[:, None]
+        _check(a, y, run(a, y))
+    x, y = a * 2.0 ** (10.0 * (k % 5) - 20), b * (k % 3 != 0)[:, None] * 2.0 ** -14
+    _check(x, y, run(x, y))
     # ... and computed once, with the unscaled kernel's bits (a second pass splits small elements into other terms and folds its sums elsewhere)
-    once, low = _lib.variant_names().index(name[:-len("_scaled")]), a.clamp(max=0) * torch.logspace(-5, 0, K, device="cuda")
+    once, low = _lib.variant_names().index(name[:-len("_scaled")]), a.clamp(max=0) * torch.logspace(-1.5, 0, K, device="cuda")
     for x, y in ((a, b), (low, b), (a, -b.abs())):
         assert torch.equal(run(x, y), cascaded_lowp_matmul(x, y, lowp="fp16", terms=3, variant=once))
     assert not run(torch.zeros_like(a), b).any() and not run(a, torch.zeros_like(b)).any()
