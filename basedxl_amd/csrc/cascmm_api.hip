@@ -1029,12 +1029,22 @@ static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem*
   return (fp8 ? std::max(slots + 5.0, 32.0) : slots) < 3.5 + step * rounds * (double)((q.K + 31) / 32) ? v : (int)CASCMM_ERR_BAD_FORMAT;
 }
 
-// A call that the fp16 slot kernel v would take, as e: K over eight waves on the rows as they lie, which scales its tiles itself, or -1.  (A
-// tile costs 1.15 of the unscaled kernels' time in the median of 119 shapes.)  Up to two tiles of 32 x 32 per CU: 330 tiles of 71 x 3800 x 3520
-// 97.9 us in slots, here 57.6; 286 of 341 x 3576 x 832 77.1, 55.7; beyond 389 x 1152 x 2175 41.3, 47.7; 421 x 760 x 2496 32.8, 41.3.
-static int select_scaled_rows(const Problem& q, RowFit fit, int v, const Problem& e) {
+// A call that an fp16 slot kernel would take if it had all the workspace that it wants: K over eight waves on the rows as they lie, which scales
+// its tiles itself and needs no workspace, or -1.  (A tile costs 1.15 of the unscaled kernels' time in the median of 119 shapes.)  Up to two tiles
+// of 32 x 32 per CU: 330 tiles of 71 x 3801 x 3520 96.4 us in slots, here 54.8 (66.1 where the values are scaled); 286 of 341 x 3577 x 832 75.4,
+// 53.0 (66.7); beyond 389 x 1152 x 2175 41.3, 47.7; 421 x 760 x 2496 32.8, 41.3.
+static int select_scaled_rows(const Problem& q, RowFit fit) {
   const auto& t = table();
-  if (v < 0 || t[v].kind != KIND_F16K || !q.call || ((q.M + 31) / 32) * ((q.N + 31) / 32) > 2 * kNumCUs) return -1;
+  if (!q.call || q.dtype != CASCMM_DT_F32 || q.fmt != CASCMM_FMT_FP16 || q.terms != 3 || q.bpre || q.glu || q.split_first ||
+      ((q.M + 31) / 32) * ((q.N + 31) / 32) > 2 * kNumCUs)
+    return -1;
+  Problem e;
+  int v = select_rounded_up(q, fit, (size_t)-1, &e);
+  if (v < 0) {
+    e = q;
+    v = select_variant(q, fit, 1);
+  }
+  if (v < 0 || t[v].kind != KIND_F16K) return -1;
   int best = -1;
   double best_cost = variant_cost(v, e, 1);
   for (int i = 0; i < (int)t.size(); ++i) {
@@ -1074,15 +1084,15 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
   const auto& t = table();
   int splits = 1;
   if (variant < 0) {
-    const RowFit rows_fit = fit;
-    if (count == 1 && !q.split_first) {
+    const int rows = count == 1 ? select_scaled_rows(q, fit) : -1;
+    if (count == 1 && !q.split_first && rows < 0) {
       Problem e;
       if (select_rounded_up(q, fit, workspace ? workspace_bytes : 0, &e) >= 0) {
         q = e;
         fit = FIT_FAST;
       }
     }
-    variant = select_variant(q, fit, count, workspace ? workspace_bytes : 0, &splits);
+    variant = rows >= 0 ? rows : select_variant(q, fit, count, workspace ? workspace_bytes : 0, &splits);
     if (variant < 0 && count > 1) {
       // no kernel takes these problems in one launch (the fp8-rate kernel runs one at a time): one
       // launch each, in order on the stream, sharing the workspace
@@ -1095,13 +1105,6 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
       return CASCMM_OK;
     }
     if (variant < 0) return none(variant);
-    if (count == 1) {
-      const int rows = select_scaled_rows(q0, rows_fit, variant, q);
-      if (rows >= 0) {
-        variant = rows;
-        q = q0;
-      }
-    }
   } else {
     splits = (variant >> 16) > 0 ? (variant >> 16) : 1;   // forced: kernel index | K splits << 16
     variant &= 0xFFFF;
@@ -1541,14 +1544,11 @@ int cascmm_call_variant(const void* A, const void* B, int64_t M, int64_t N, int6
     return select_variant(e, row_fit(e, r.a ? nullptr : A, r.b ? nullptr : B), 1, workspace_bytes - relay_bytes(r, 1));
   }
   const RowFit fit = row_fit(q, A, B);
+  const int rows = select_scaled_rows(q, fit);
+  if (rows >= 0) return rows;
   Problem e;
-  int v = select_rounded_up(q, fit, workspace_bytes, &e);
-  if (v < 0) {
-    e = q;
-    v = select_variant(q, fit, 1, workspace_bytes);
-  }
-  const int rows = select_scaled_rows(q, fit, v, e);
-  return rows >= 0 ? rows : v;
+  const int v = select_rounded_up(q, fit, workspace_bytes, &e);
+  return v >= 0 ? v : select_variant(q, fit, 1, workspace_bytes);
 }
 
 int cascmm_call_variant_prepared(const void* A, int glu, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldc, int dtype, int fmt,

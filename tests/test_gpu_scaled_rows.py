@@ -12,12 +12,12 @@ SHAPES = [(1, 33, 5), (17, 100, 47), (33, 1193, 70), (5, 2570, 129)]
 def test_few_rows_take_the_kernel_that_scales_its_own_tiles():
     l, names = _lib.lib(), _lib.variant_names()
 
-    def kernel(M, K, N, lda=None):
-        lda = lda or K
-        return names[l.cascmm_call_variant(1 << 40, 2 << 40, M, N, K, lda, N, N, 0, 1, 3, 0, l.cascmm_workspace_bytes(M, N, K, 0, 1, 3, 0)) & 0xFFFF]
+    def kernel(M, K, N, ws=None):
+        return names[l.cascmm_call_variant(1 << 40, 2 << 40, M, N, K, K, N, N, 0, 1, 3, 0, l.cascmm_workspace_bytes(M, N, K, 0, 1, 3, 0) if ws is None else ws) & 0xFFFF]
 
     for shape in ((5, 3164, 3136), (6, 1193, 462), (33, 1612, 1374)):
         assert kernel(*shape).endswith("_scaled"), shape
+        assert kernel(*shape, ws=0) == kernel(*shape), shape       # (it needs no room for slots)
     for shape in ((882, 899, 3968), (300, 576, 4480), (2048, 1281, 1280)):
         assert "_wavek_" not in kernel(*shape), shape
 
@@ -107,3 +107,17 @@ def test_scaled_rows_near_the_least_unscaled_tile(top, name):
     low_b2[0], low_b2[7], low_a2[:, 7] = 0, top, 0          # both
     for x, y in ((low_a, plain_b), (plain_a, low_b), (low_a2, low_b2)):
         _check(x, y, cascaded_lowp_matmul(x, y, lowp="fp16", terms=3, variant=v))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(5, 3164, 3136), (33, 1612, 1374)])
+def test_few_rows_without_a_workspace_hold_values_beyond_the_format(M, K, N):
+    print(M, K, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = torch.randn(M, K, device="cuda", generator=g) * 2.0 ** 20, torch.randn(K, N, device="cuda", generator=g)
+    c = torch.full((M, N), 7.0, device="cuda")
+    st = _lib.lib().cascmm_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), None, M, N, K, K, N, N, 0, 1, 3, 0, None, None, 0,
+                                torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    _check(a, b, c)
+    assert torch.equal(c, cascaded_lowp_matmul(a, b, lowp="fp16", terms=3))
