@@ -51,7 +51,9 @@ struct H16 {
   // tile rows an XCD walks down before moving one tile to the right: about square in bytes
   static constexpr int GROUP_M = BN >= 2 * BM ? 8 : 4;
   static_assert(WM * WN * WK == 4 && (BK == 32 || BK == 64) && SLW % 2 == 0 && NS >= 3, "layout");
-  static_assert(!PAIR || (WK == 1 && NS >= 4 && A_LOADS % 2 == 0), "pairs");
+  // (pairs: the prologue issues the first pair of A before all of B and one pair more, so the wait counts at the first stages hold for four
+  // stages only: with five, two pairs would be taken to be in flight behind stage 1's B, which is read then)
+  static_assert(!PAIR || (WK == 1 && NS == 4 && A_LOADS % 2 == 0), "pairs");
   static_assert(A_BUF % 4096 == 0 && B_STAGE % 4096 == 0, "every wave issues the same number of loads");
   static_assert((NS - 1) * LOADS <= 63, "the wait counter has six bits");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
