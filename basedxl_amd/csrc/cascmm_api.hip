@@ -360,7 +360,11 @@ static double call_estimate_us(const CallCost& t, const VariantDesc& v, const Pr
                         : (full > 0 ? 1.07 : 1.0) * ((double)q.M * (double)q.K > 5.0e6 ? 1.25 : (double)q.M * (double)q.K > 1.25e6 ? 1.1 : 1.0);
     return late * (q.N % v.BN != 0 ? us * (1.0 + t.edge) : us);
   }
-  const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * (full + 1.0) : us;
+  // (The gated 256 x 128 tile with producer waves: a wave's rows over the edge are stored one by one, which few of them do quickly: 1289 x 576 x
+  // 4608 28.1 us, 29.5 on the large tile of 128 columns; 3087 x 384 x 2304 22.3, 24.2.  The smaller tiles with less of an edge lost 14 - 22 % to
+  // the eight-wave ones: 530 x 832 x 3200, 295 x 1088 x 6528)
+  const double rows_over = q.glu && v.kind == KIND_TILE && v.BM == 256 && q.N % v.BN == 0 ? std::min(1.0, (double)(q.M % v.BM) / 64.0) : 1.0;
+  const double edged = q.N % v.BN != 0 || q.M % v.BM != 0 ? us + t.edge * rows_over * (full + 1.0) : us;
   const double power = t.deep * tiles * v.BM * v.BN * (double)k_per * 1.0e-9;
   // (the large tiles of 192 and 128 columns, prepared: with a margin; without one 3072^3 took 153 us on 192, 138 on 256 x 160)
   const double margin = count > 1 && q.bpre && v.BM == 64 && v.BN == 160 ? 1.08 : q.bpre && v.kind == KIND_W512E && v.call_only ? 1.03 : 1.0;

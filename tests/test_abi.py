@@ -267,6 +267,14 @@ def test_gated_calls_compare_their_kernels_by_one_scale(M, K, N, kernel):
     assert _lib.variant_names()[v].startswith(kernel)
 
 
+# (us: 28.1 there, 29.5 on the large tile of 128 columns; 1500 rows 34.8 and 29.2; 295 x 1088 x 6528 22.7, 28.0 on 128 x 128)
+@pytest.mark.parametrize("M,K,N,kernel", [(1289, 576, 4608, "t256x128x32_w4x1x1"), (1500, 576, 4608, "t256x128x32_w512_narrow"),
+                                          (295, 1088, 6528, "t64x64x32_wavek")])
+def test_gated_calls_count_the_rows_over_the_edge(M, K, N, kernel):
+    l = _lib.lib()
+    assert _lib.variant_names()[l.cascmm_call_variant_prepared(1 << 40, 1, M, N, K, K, N // 2, 0, 0, 2, 0, 0)].startswith(kernel)
+
+
 @pytest.mark.parametrize("M,K,N,large", [(3072, 576, 1728, False), (4928, 384, 1152, False), (6976, 320, 960, False),
                                          (1500, 1280, 10240, True), (4096, 4096, 4096, True), (7800, 640, 5120, True)])
 def test_prepared_layers_take_the_large_tile_where_it_is_faster(M, K, N, large):
