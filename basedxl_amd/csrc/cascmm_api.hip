@@ -399,7 +399,9 @@ static double skinny_estimate_us(const Problem& q) {
 // The 16-bit kernels (KIND_H16).  A workgroup's k costs s1 with every CU at work (L2 or the board's power is shared)
 // and s0 with few; a round of 256 tiles adds `end` for its store, a launch `start`.  raw: the factor on k of a right
 // operand that the LDS transposes.  Measured on the Linear shapes of a UNet and on squares (graph replay, every tile
-// forced in turn).
+// forced in turn), before the two tiles of 32-k stages loaded pairs of them: those run in 0.83 - 1.00 of what is said here, in pairs of 32 k, and
+// are left out now and then.  Looked at again with every kernel forced on 600 shapes: the one chosen is 0.3 - 1.2 % behind the fastest on average (raw,
+// few rows 1.8), 2 - 6 % in one of twenty (16); with k rounded to the pairs' 64 here two choices changed, both for the worse.
 struct H16Cost { int BM, BN; double s0, s1, start, end, raw; };
 static const H16Cost kH16Cost[] = {
     {256, 320, 0.0205, 0.0315, 3.8, 8.0, 1.06}, {256, 256, 0.0175, 0.0255, 4.0, 6.5, 1.03}, {128, 256, 0.0090, 0.0138, 3.5, 3.5, 1.04},
