@@ -278,10 +278,11 @@ static const CallCost kCallCost[] = {
     {"t16x16x32_wavek_fp16x3_tri", 2.47, 0.728, 0.176, 0.125, 28.6, 1, 0.664, 0.051, 0},
     {"t16x32x32_wavek_fp16x3_tri", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
     {"t32x32x32_wavek_fp16x3_tri", 2.79, 1.5, 0.319, 1.57, 60, 1, 1.62, 0, 0},
-    // three fp8 terms (493 shapes, hardly ever behind the fastest; without rounds 0.6 %, at most 33 %)
+    // ... tiles that scale themselves: the same, select_scaled_rows adds what the maxima take
     {"t16x16x32_wavek_fp16x3_tri_scaled", 2.47, 0.728, 0.176, 0.125, 28.6, 1, 0.664, 0.051, 0},
     {"t16x32x32_wavek_fp16x3_tri_scaled", 2.44, 1.13, 0.236, 0.804, 38.3, 1, 1.23, 0, 0},
     {"t32x32x32_wavek_fp16x3_tri_scaled", 2.79, 1.5, 0.319, 1.57, 60, 1, 1.62, 0, 0},
+    // three fp8 terms (493 shapes, hardly ever behind the fastest; without rounds 0.6 %, at most 33 %)
     {"t16x16x32_wavek_fp8x3_tri", 2.54, 0.713, 0.229, 0.147, 28.1, 1, 0.655, 0.00446, 0},
     {"t16x32x32_wavek_fp8x3_tri", 2.57, 1.1, 0.207, 1.1, 26.9, 1, 1.24, 0, 0},
     {"t32x32x32_wavek_fp8x3_tri", 2.91, 1.4, 0.425, 2.04, 60, 1, 4.23, 0.0301, 0},
@@ -624,7 +625,7 @@ static double variant_cost(int vi, const Problem& q, int count, size_t ws_bytes 
 
 // Three terms on K over eight waves, by the tiles of 32 x 32 (graph replay, 150 shapes of 2 - 1500 rows each).
 // fp16: only in the place of the tile kernels, which split the operands as they are too (the slot kernels scale both first and so take
-// values beyond fp16's range: their calls stay theirs), up to two tiles per CU, of deep K up to one, and up to three where the other kernel is
+// values beyond fp16's range: of their calls the tiles that scale themselves take some, see select_scaled_rows), up to two tiles per CU, of deep K up to one, and up to three where the other kernel is
 // the bounds-checked one.  0.47 of the tile kernels' time (2 x 1280 x 1280 12.8 us, here 6.1; 38 x 256 x 448 9.9, 3.3; 222 x 4352 x 704 32.9,
 // 28.6; 788 x 659 x 818 bounds-checked 35.0, 23.0), 2 % behind the fastest of all; beyond: 391 x 384 x 1984 13.6, here 16.7; 96 x 2048 x 8192
 // 41.0, 45.3 (eager); 1136 x 3200 x 256 42.8, 44.9.

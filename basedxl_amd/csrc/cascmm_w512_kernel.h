@@ -224,8 +224,9 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
   // ---- software pipeline ---------------------------------------------------------------------
   // Blocks are numbered t = stage * NTL + ni.  While the 12 MFMAs of block t issue, the raw B values of
   // block t + 2 are read from LDS and those of block t + 1 (read one block earlier) are split; the A
-  // values of row block ni of the next stage are read and split during block ni (0 .. 3), two loads of
-  // a later stage are issued per block.
+  // values of the next stage's row blocks are read and split during the blocks that RB_OF gives them to (five and four
+  // blocks: row block ni during block ni), and loads of later stages are issued: one per block of an even stage (B), up to SLOTS per block
+  // of an odd one (a pair of A, then B).
 #define W512_FENCE() __builtin_amdgcn_sched_barrier(0)
   u32x4 Af[2][2][T::MT];   // [buffer][hi / lo][mi]
   float R[2][8];           // raw B values of two blocks in flight
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(W512Tile<NTL>::NT) __attribute__((amdgpu_waves_per_
           }
           if (BPRE && gi == 4) read_slot_hi(nxt, stn, n1);     // seven MFMAs before the next block's first
           if (BPRE && gi == 8) read_slot_lo(nxt, stn, n1);
-          // the stage's loads: two per block, apart from each other and in gaps that hold one half-split
+          // the stage's loads, apart from each other: an even stage's one in gap 9, an odd stage's two to five in every other gap
           // (several loads in neighbouring gaps of one block cost 30 cycles each: counted)
           if (gi == 3) dl(0);
           if (gi == 9) dl(1);
