@@ -1040,11 +1040,13 @@ static int select_rounded_up(const Problem& q, RowFit fit, size_t room, Problem*
 // its tiles itself and needs no workspace, or -1.  (A tile costs 1.15 of the unscaled kernels' time in the median of 119 shapes.)  Up to two tiles
 // of 32 x 32 per CU: 330 tiles of 71 x 3801 x 3520 96.4 us in slots, here 54.8 (66.1 where the values are scaled); 286 of 341 x 3577 x 832 75.4,
 // 53.0 (66.7); beyond 389 x 1152 x 2175 41.3, 47.7; 421 x 760 x 2496 32.8, 41.3.
+static bool few_scaled_tiles(const Problem& q) {
+  return q.call && q.dtype == CASCMM_DT_F32 && q.fmt == CASCMM_FMT_FP16 && q.terms == 3 && !q.bpre && !q.glu && !q.split_first &&
+         ((q.M + 31) / 32) * ((q.N + 31) / 32) <= 2 * kNumCUs;
+}
 static int select_scaled_rows(const Problem& q, RowFit fit) {
   const auto& t = table();
-  if (!q.call || q.dtype != CASCMM_DT_F32 || q.fmt != CASCMM_FMT_FP16 || q.terms != 3 || q.bpre || q.glu || q.split_first ||
-      ((q.M + 31) / 32) * ((q.N + 31) / 32) > 2 * kNumCUs)
-    return -1;
+  if (!few_scaled_tiles(q)) return -1;
   Problem e;
   int v = select_rounded_up(q, fit, (size_t)-1, &e);
   if (v < 0) {
@@ -1091,15 +1093,23 @@ static int gemm_on_rows(int count, const void* const* A, const void* const* B, v
   const auto& t = table();
   int splits = 1;
   if (variant < 0) {
-    const int rows = count == 1 ? select_scaled_rows(q, fit) : -1;
+    // (with room for slots a call of select_scaled_rows is one that a slot kernel would take: the others do not pay for its answer)
+    const size_t room = workspace ? workspace_bytes : 0;
+    const RowFit rows_fit = fit;
+    const bool no_slots = count == 1 && few_scaled_tiles(q) && f16k_workspace_bytes(q.M, q.N, rounded_up(q, fit).K) > room;
+    int rows = no_slots ? select_scaled_rows(q, fit) : -1;
     if (count == 1 && !q.split_first && rows < 0) {
       Problem e;
-      if (select_rounded_up(q, fit, workspace ? workspace_bytes : 0, &e) >= 0) {
+      if (select_rounded_up(q, fit, room, &e) >= 0) {
         q = e;
         fit = FIT_FAST;
       }
     }
-    variant = rows >= 0 ? rows : select_variant(q, fit, count, workspace ? workspace_bytes : 0, &splits);
+    variant = rows >= 0 ? rows : select_variant(q, fit, count, room, &splits);
+    if (count == 1 && variant >= 0 && t[variant].kind == KIND_F16K && (rows = select_scaled_rows(q0, rows_fit)) >= 0) {
+      variant = rows;
+      q = q0;
+    }
     if (variant < 0 && count > 1) {
       // no kernel takes these problems in one launch (the fp8-rate kernel runs one at a time): one
       // launch each, in order on the stream, sharing the workspace
