@@ -93,8 +93,7 @@ __device__ __forceinline__ void w512_in_vec(f32x16& c) { asm volatile("" : "+v"(
 // 7800 x 640 x 5120 145.7 / 137.9 (145.1 / 141.1); 1500 x 1280 x 10240 on 256 x 256 109.9 / 103.0 (111.3 / 103.4); 4096^3 323.8 / 303.8
 // (326.7 / 311.4) = 1.27 / 1.36 PFLOP/s of MFMA work, as on the wider tile: what is left is the clock the board's power allows.  K off its
 // steps 3700^3 281 / 263 us (283 / 264; the K-over-waves kernel, the only other one that takes it, 1.25 times that).  The test per load of A
-// costs whole K nothing that can be measured.  Traces and counters: profiles/cascmm_w512_edge_kernels.txt (its
-// comparison with the kernels with producer waves is of an earlier state of this one).
+// costs whole K nothing that can be measured.  Traces and counters: profiles/cascmm_w512_edge_kernels.txt.
 // Host-checked: M % 256 == 0, N % BN == 0 (EDGE: M >= 64, N >= BN, raw B: N % 4 == 0; with the gated store N % 320 == 0 on the wider
 // tile), K % 32 == 0 (EDGE: rows of A of whole 16-byte chunks, zeros between K and the last one's end), lda % 4 == 0, ldb % 4 == 0, A and B 16-byte
 // aligned, M * lda * 4 and K * ldb * 4 below 2 GiB, C rows addressable with 32-bit byte offsets
